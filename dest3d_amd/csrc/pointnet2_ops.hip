@@ -2,10 +2,9 @@
 // gathering, 3-nearest-neighbour search and interpolation (the functions of the reference's `pointnet2._ext`,
 // pointnet2/_ext_src/src/*.cpp).  Index arithmetic is exact; all tensors fp32 / int32, contiguous.
 //
-//  * furthest point sampling: one 512-thread workgroup per sample; a thread owns points tid, tid + 512, ... and keeps
-//    their coordinates and running minimum distance in registers (up to 24576 points; beyond that coordinates are
-//    re-read and distances kept in the caller's `temp`); per sample drawn: one pass over the thread's points, an
-//    argmax over the wave with shuffles, over the 8 waves through LDS.  Ties go to the smaller index.
+//  * furthest point sampling: one workgroup per sample; up to 24576 points live in registers with their running minimum
+//    distance, sorted into groups of 64 neighbours so that a draw looks only at groups it can change; beyond that
+//    coordinates are re-read and distances kept in the caller's `temp`.  Ties go to the smaller index.
 //  * ball query: one wave per query centre; 64 points are tested per step and compacted in index order with a
 //    ballot, so the first `nsample` hits are found without a serial scan; the wave stops as soon as it has them.
 //  * 3-NN: one thread per unknown point, known points staged through LDS 256 at a time.
@@ -13,6 +12,8 @@
 //    with hardware float atomics (duplicates in idx are the rule), as the reference does -- either straight into
 //    the (b, c, n) layout, one scattered cache line per lane, or (the *_cl entry points) into a channel-last
 //    (b, n, c) buffer through an LDS transpose, 64 consecutive floats per instruction.
+#include <type_traits>
+
 #include "issm_dev.h"
 
 namespace issm {
@@ -38,9 +39,213 @@ __device__ __forceinline__ ArgMax better(ArgMax a, ArgMax b) {  // larger value,
 
 // idxs[b][0] = 0; then repeatedly the point farthest from the chosen set.  Points with |p|^2 <= 1e-3 (padding at the
 // origin) are never chosen and keep their distance, as in the reference (sampling_gpu.cu:105-106).
-// PPT > 0: the thread's PPT points -- coordinates and running distance -- live in registers for the whole kernel
-// (n <= 512 * PPT); PPT == 0: any n, coordinates re-read from memory (L2) and distances kept in `temp`.
-template <int PPT>
+
+// Wave-wide maxima with DPP: four shifts inside each row of 16 lanes, then the rows (zero, what lanes without a source
+// receive, is the identity of an unsigned maximum, so a step is one v_max_u32).
+__device__ __forceinline__ unsigned umax(unsigned a, unsigned b) { return a > b ? a : b; }
+__device__ __forceinline__ unsigned umin(unsigned a, unsigned b) { return a < b ? a : b; }
+__device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
+__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
+#define UMAX_STEP(ctrl) v = umax(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true))
+// the maximum over the first ROWS * 16 lanes (ROWS = 1, 2 or 4), in a scalar register
+template <int ROWS>
+__device__ __forceinline__ unsigned wave_max(unsigned v) {
+  UMAX_STEP(0x111); UMAX_STEP(0x112); UMAX_STEP(0x114); UMAX_STEP(0x118);
+  if (ROWS >= 2) v = umax(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));  // row 0 -> 1, 2 -> 3
+  if (ROWS == 4) v = umax(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));  // row 1 -> 2, 3
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 16 * ROWS - 1);
+}
+#undef UMAX_STEP
+__device__ __forceinline__ float wave_fmax(float v) {  // (used once per slot, not per draw)
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ float lane_f(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+// of the lanes in `cand`, the one with the smallest `key` (rare: equal distances)
+__device__ __forceinline__ int lane_of_least(unsigned long long cand, int key) {
+  int best = __builtin_ctzll(cand), bk = __builtin_amdgcn_readlane(key, best);
+  for (cand &= cand - 1; cand; cand &= cand - 1) {
+    const int l = __builtin_ctzll(cand), k = __builtin_amdgcn_readlane(key, l);
+    if (k < bk) { bk = k; best = l; }
+  }
+  return best;
+}
+
+// Up to 64 W S points: one workgroup of W waves per sample, points in registers, and only those looked at that a draw can
+// change.  The draws are a serial chain, so what counts is the time of one: passing over all points costs 40 distances
+// per lane at 20000 points (1.92 us a draw, the vector unit of one CU saturated).  Here the points are first sorted along a
+// Z-order curve over a 16^3 grid (counting sort in LDS) and cut into groups of 64 neighbours, one point per lane; group g
+// belongs to wave g % W (neighbouring groups to different waves) as its slot g / W, and lane l of the wave keeps slot l's
+// bounding box, largest running distance and the point that has it.  A draw at o compares o's distance to every box with
+// the group's largest distance -- one instruction sequence for all groups of a wave -- and goes through the points of
+// those groups only that are nearer: about 10 of 313.  One barrier per draw (the waves' bests go through LDS buffers used
+// in turn).  20000 points, 2048 draws, 8 samples: 3.93 ms -> 1.97 ms (0.96 us a
+// draw: a chain of about 100 dependent instructions, two LDS round trips and a barrier).
+//
+// The pruning is exact: fp32 rounding is monotone, so for a point q of the box each step of the box's squared distance
+// (subtract, square, add, in sqdist's order) is at most the same step for q, and where the box's distance is not below the
+// group's largest running distance, no minimum of the group changes.  A NaN anywhere makes the comparison fail, which means
+// "look".  Equal distances go to the smaller index at every level, as a pass over all points in order would decide.
+constexpr int FPS_CELLS = 4096;   // 16^3
+// f(0), f(1), ... f(N - 1) with constant arguments: register arrays indexed inside f stay in registers for every N (the
+// loop unroller left a loop over 20 or 24 slots to dynamic indexing, and the arrays to scratch)
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void for_each_slot(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    for_each_slot<N, I + 1>(static_cast<F&&>(f));
+  }
+}
+__device__ __forceinline__ unsigned spread4(unsigned v) {   // bits 0..3 -> 0, 3, 6, 9
+  return (v & 1u) | ((v & 2u) << 2) | ((v & 4u) << 4) | ((v & 8u) << 6);
+}
+
+template <int W, int S>
+__global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const float* __restrict__ xyz, int* __restrict__ idxs) {
+  constexpr int T = 64 * W, ROWS = (S + 15) / 16;
+  static_assert(S % 4 == 0 && S <= 32 && W <= 16 && (W & (W - 1)) == 0, "slots and waves sit in the lanes of one wave");
+  __shared__ int hist[FPS_CELLS];
+  __shared__ unsigned short order[T * S];
+  __shared__ float red[6][W];
+  __shared__ int wsum[W];
+  struct alignas(16) Best { unsigned d; float x, y, z; };
+  __shared__ Best best[2][W];
+  __shared__ int best_pos[2][W];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* p = xyz + (long)b * n * 3;
+  int* out = idxs + (long)b * npoint;
+  const float INFV = __builtin_huge_valf();
+
+  // bounding box of the points that take part
+  float lo[3] = {INFV, INFV, INFV}, hi[3] = {-INFV, -INFV, -INFV};
+  for (int k = tid; k < n; k += T) {
+    const float x = p[k * 3], y = p[k * 3 + 1], z = p[k * 3 + 2];
+    if (sqdist(x, y, z, 0.0f, 0.0f, 0.0f) > 1e-3f) {
+      lo[0] = fminf(lo[0], x); lo[1] = fminf(lo[1], y); lo[2] = fminf(lo[2], z);
+      hi[0] = fmaxf(hi[0], x); hi[1] = fmaxf(hi[1], y); hi[2] = fmaxf(hi[2], z);
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float l = -wave_fmax(-lo[a]), h = wave_fmax(hi[a]);
+    if (lane == 0) { red[a][wave] = l; red[3 + a][wave] = h; }
+  }
+  for (int c = tid; c < FPS_CELLS; c += T) hist[c] = 0;
+  __syncthreads();
+  float ext = 0.0f;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    for (int w = 0; w < W; ++w) { lo[a] = fminf(w ? lo[a] : INFV, red[a][w]); hi[a] = fmaxf(w ? hi[a] : -INFV, red[3 + a][w]); }
+    ext = fmaxf(ext, hi[a] - lo[a]);
+  }
+  const float inv = ext > 0.0f && ext < INFV ? 16.0f / ext : 0.0f;
+  auto cell = [&](int k) {
+    unsigned c = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      c |= spread4((unsigned)imin(imax((int)((p[k * 3 + a] - lo[a]) * inv), 0), 15)) << a;
+    return c;
+  };
+  for (int k = tid; k < n; k += T) atomicAdd(&hist[cell(k)], 1);
+  __syncthreads();
+  {  // exclusive prefix sum of the histogram: FPS_CELLS / T neighbours per thread
+    constexpr int E = FPS_CELLS / T;
+    int own = 0;
+    for (int e = 0; e < E; ++e) own += hist[tid * E + e];
+    int incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int at = incl - own;
+    for (int w = 0; w < wave; ++w) at += wsum[w];
+    for (int e = 0; e < E; ++e) { const int v = hist[tid * E + e]; hist[tid * E + e] = at; at += v; }
+  }
+  __syncthreads();
+  for (int k = tid; k < n; k += T) order[atomicAdd(&hist[cell(k)], 1)] = (unsigned short)k;
+  __syncthreads();
+
+  // the wave's slots into registers; lane l keeps what belongs to slot l.  A running distance is kept as its bit pattern
+  // plus one: distances are >= 0 and order as unsigned integers do, 0 marks a point that never takes part (or a lane
+  // without a slot), and a NaN or infinite distance is above every running one.
+  const unsigned far = __builtin_bit_cast(unsigned, 1e10f) + 1u;
+  float px[S], py[S], pz[S];
+  unsigned d[S];
+  float blx = INFV, bly = INFV, blz = INFV, bhx = -INFV, bhy = -INFV, bhz = -INFV, gx = 0.0f, gy = 0.0f, gz = 0.0f;
+  unsigned gd = 0;
+  int gpos = 0;
+  for_each_slot<S>([&](auto slot) {
+    constexpr int j = decltype(slot)::value;
+    const int pos = (j * W + wave) * 64 + lane;
+    px[j] = py[j] = pz[j] = 0.0f;
+    if (pos < n) { const int k = order[pos]; px[j] = p[k * 3]; py[j] = p[k * 3 + 1]; pz[j] = p[k * 3 + 2]; }
+    const bool in = sqdist(px[j], py[j], pz[j], 0.0f, 0.0f, 0.0f) > 1e-3f;
+    d[j] = in ? far : 0u;
+    const float lx = -wave_fmax(in ? -px[j] : -INFV), ly = -wave_fmax(in ? -py[j] : -INFV), lz = -wave_fmax(in ? -pz[j] : -INFV);
+    const float hx = wave_fmax(in ? px[j] : -INFV), hy = wave_fmax(in ? py[j] : -INFV), hz = wave_fmax(in ? pz[j] : -INFV);
+    const bool any = __ballot(in) != 0;
+    if (lane == j) {
+      blx = lx; bly = ly; blz = lz; bhx = hx; bhy = hy; bhz = hz;
+      gd = any ? far : 0u;
+    }
+  });
+  float ox = p[0], oy = p[1], oz = p[2];
+  for (int s = 1; s < npoint; ++s) {
+    // the slots whose box is nearer than their largest distance (never NaN: fmaxf drops one)
+    const float ex = fmaxf(fmaxf(blx - ox, ox - bhx), 0.0f), ey = fmaxf(fmaxf(bly - oy, oy - bhy), 0.0f),
+                ez = fmaxf(fmaxf(blz - oz, oz - bhz), 0.0f);
+    const unsigned mask = (unsigned)__ballot(__builtin_bit_cast(unsigned, sqdist(ex, ey, ez, 0.0f, 0.0f, 0.0f)) + 1u < gd);
+    for_each_slot<S / 4>([&](auto block) {
+      constexpr int j4 = 4 * decltype(block)::value;
+      if (((mask >> j4) & 15u) == 0) return;
+      for_each_slot<4>([&](auto slot) {
+        constexpr int j = j4 + decltype(slot)::value;
+        if (((mask >> j) & 1u) == 0) return;
+        d[j] = umin(d[j], __builtin_bit_cast(unsigned, sqdist(px[j], py[j], pz[j], ox, oy, oz)) + 1u);
+        const unsigned m = wave_max<4>(d[j]);
+        const unsigned long long cand = __ballot(d[j] == m);
+        const int base = (j * W + wave) * 64;
+        int l = __builtin_ctzll(cand);
+        if (cand & (cand - 1)) l = lane_of_least(cand, base + lane < n ? (int)order[base + lane] : 0x7fffffff);
+        const float x = lane_f(px[j], l), y = lane_f(py[j], l), z = lane_f(pz[j], l);
+        if (lane == j) { gd = m; gpos = base + l; gx = x; gy = y; gz = z; }
+      });
+    });
+    // the wave's best, then the workgroup's
+    {
+      const unsigned m = wave_max<(S > 16 ? 2 : 1)>(gd);
+      const unsigned long long cand = __ballot(gd == m);
+      int l = __builtin_ctzll(cand);
+      if (m && (cand & (cand - 1))) l = lane_of_least(cand, (int)order[gpos]);
+      if (lane == l) { best[s & 1][wave] = Best{gd, gx, gy, gz}; best_pos[s & 1][wave] = gpos; }
+    }
+    __syncthreads();
+    Best w = best[s & 1][lane & (W - 1)];   // repeated through the wave: the first row holds every wave's
+    const int wp = best_pos[s & 1][lane & (W - 1)];
+    const unsigned m = wave_max<1>(w.d);
+    const unsigned long long cand = __ballot(w.d == m) & ((1ull << W) - 1);
+    int l = __builtin_ctzll(cand);
+    if (m && (cand & (cand - 1))) l = lane_of_least(cand, (int)order[wp]);
+    if (m) {
+      ox = lane_f(w.x, l); oy = lane_f(w.y, l); oz = lane_f(w.z, l);
+      if (tid == l) out[s] = wp;   // a place in `order` for now: its translation would be waited for here
+    } else {  // nothing but padding points: index 0, as the reference
+      ox = p[0]; oy = p[1]; oz = p[2];
+      if (tid == 0) out[s] = -1;
+    }
+  }
+  __syncthreads();
+  for (int s = tid; s < npoint; s += T) out[s] = s && out[s] >= 0 ? (int)order[out[s]] : 0;
+}
+
+// Any number of points (used above 24576, where they no longer fit one workgroup's registers): coordinates re-read from
+// memory (L2) and distances kept in `temp`.
 __global__ __launch_bounds__(FPS_T) void k_fps(int n, int npoint, const float* __restrict__ xyz, float* __restrict__ temp,
                                                 int* __restrict__ idxs) {
   __shared__ float sv[FPS_T / 64];
@@ -49,43 +254,20 @@ __global__ __launch_bounds__(FPS_T) void k_fps(int n, int npoint, const float* _
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float* p = xyz + (long)b * n * 3;
   int* out = idxs + (long)b * npoint;
-  constexpr int R = PPT > 0 ? PPT : 1;
-  float px[R], py[R], pz[R], dreg[R];
-  float* tmp = nullptr;
-  if (PPT > 0) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const int k = tid + j * FPS_T;
-      px[j] = py[j] = pz[j] = 0.0f;  // a slot past n looks like a padding point: skipped
-      if (k < n) { px[j] = p[k * 3]; py[j] = p[k * 3 + 1]; pz[j] = p[k * 3 + 2]; }
-      // padding points get a distance that never wins; the others start at 1e10
-      dreg[j] = sqdist(px[j], py[j], pz[j], 0.0f, 0.0f, 0.0f) > 1e-3f ? 1e10f : -2.0f;
-    }
-  } else {
-    tmp = temp + (long)b * n;
-    for (int k = tid; k < n; k += FPS_T) tmp[k] = 1e10f;
-  }
+  float* tmp = temp + (long)b * n;
+  for (int k = tid; k < n; k += FPS_T) tmp[k] = 1e10f;
   if (tid == 0) out[0] = 0;
   int old = 0;
   for (int s = 1; s < npoint; ++s) {
     const float ox = p[old * 3], oy = p[old * 3 + 1], oz = p[old * 3 + 2];
     float bv = -1.0f;
     int bi = 0;
-    if (PPT > 0) {
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const float d = fminf(dreg[j], sqdist(px[j], py[j], pz[j], ox, oy, oz));
-        dreg[j] = d;
-        if (d > bv) { bv = d; bi = tid + j * FPS_T; }  // indices ascend with j: the first maximum stays
-      }
-    } else {
-      for (int k = tid; k < n; k += FPS_T) {
-        const float x = p[k * 3], y = p[k * 3 + 1], z = p[k * 3 + 2];
-        if (sqdist(x, y, z, 0.0f, 0.0f, 0.0f) > 1e-3f) {
-          const float d = fminf(tmp[k], sqdist(x, y, z, ox, oy, oz));
-          tmp[k] = d;
-          if (d > bv) { bv = d; bi = k; }
-        }
+    for (int k = tid; k < n; k += FPS_T) {
+      const float x = p[k * 3], y = p[k * 3 + 1], z = p[k * 3 + 2];
+      if (sqdist(x, y, z, 0.0f, 0.0f, 0.0f) > 1e-3f) {
+        const float d = fminf(tmp[k], sqdist(x, y, z, ox, oy, oz));
+        tmp[k] = d;
+        if (d > bv) { bv = d; bi = k; }
       }
     }
     ArgMax best = {bv, bi};
@@ -278,15 +460,18 @@ int launch_scatter_channel_last(bool k3, int b, int c, int n, int ne, const floa
 static unsigned blocks_for(long total) { return (unsigned)((total + NTHREADS - 1) / NTHREADS); }
 
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st) {
-  const dim3 g(b), t(FPS_T);
-  if (n <= FPS_T * 4) hipLaunchKernelGGL(k_fps<4>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 8) hipLaunchKernelGGL(k_fps<8>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 16) hipLaunchKernelGGL(k_fps<16>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 24) hipLaunchKernelGGL(k_fps<24>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 32) hipLaunchKernelGGL(k_fps<32>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 40) hipLaunchKernelGGL(k_fps<40>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else if (n <= FPS_T * 48) hipLaunchKernelGGL(k_fps<48>, g, t, 0, st, n, npoint, xyz, temp, idxs);
-  else hipLaunchKernelGGL(k_fps<0>, g, t, 0, st, n, npoint, xyz, temp, idxs);
+#define FPS_GROUPS(W, S) hipLaunchKernelGGL((k_fps_groups<W, S>), dim3(b), dim3(64 * W), 0, st, n, npoint, xyz, idxs)
+  // Eight waves up to 2048 points (fewer meet at the barrier: 0.73 against 0.78 us a draw at 2048), sixteen above (0.82
+  // against 0.83 at 4096, 0.86 against 0.92 at 8192); slots just enough for n, every empty one costs 5 ns a draw.
+  if (n <= 64 * 8 * 4) FPS_GROUPS(8, 4);
+  else if (n <= 64 * 16 * 4) FPS_GROUPS(16, 4);
+  else if (n <= 64 * 16 * 8) FPS_GROUPS(16, 8);
+  else if (n <= 64 * 16 * 12) FPS_GROUPS(16, 12);
+  else if (n <= 64 * 16 * 16) FPS_GROUPS(16, 16);
+  else if (n <= 64 * 16 * 20) FPS_GROUPS(16, 20);
+  else if (n <= 64 * 16 * 24) FPS_GROUPS(16, 24);
+  else hipLaunchKernelGGL(k_fps, dim3(b), dim3(FPS_T), 0, st, n, npoint, xyz, temp, idxs);
+#undef FPS_GROUPS
   return (int)hipGetLastError();
 }
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,

@@ -35,6 +35,24 @@ def test_furthest_point_sampling_beyond_the_register_path():
     assert (idx == R.furthest_point_sampling(xyz, 48)).all()
 
 
+@pytest.mark.parametrize("n", [63, 64, 65, 2048, 2049, 4096, 4097, 8193, 12289, 16385, 20481, 24576, 24577])
+def test_furthest_point_sampling_at_the_edges_of_its_variants(n):
+    """Group and slot remainders of every register variant, and the first size beyond them; sample 1 is clustered (a flat
+    sheet, duplicates, one far point), sample 2 all padding but one point, sample 3 one point repeated."""
+    from dest3d_amd.pointnet2_utils import furthest_point_sample
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(-4, 4, size=(4, n, 3)).astype(np.float32)
+    xyz[1, :, 2] = 1.0
+    xyz[1, n // 2:] = xyz[1, :n - n // 2]
+    xyz[1, 11] = (300.0, -20.0, 5.0)
+    xyz[2] = 0.0
+    xyz[2, n // 3] = 2.0
+    xyz[3] = xyz[3, 5]
+    npoint = min(n, 80)
+    idx = furthest_point_sample(_cuda(xyz), npoint).cpu().numpy()
+    assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
+
+
 @pytest.mark.parametrize("seed,npoint", [(3, 1024), (8, 1024), (54, 1024)])
 def test_furthest_point_sampling_near_ties_go_the_way_of_plain_fp32_steps(seed, npoint):
     """Clouds in which two candidates' running minimum distances come within one unit in the last place of each other
