@@ -13,6 +13,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libissm_hip.so")
+HOST_PATH = os.path.join(_HERE, "_issm_host.so")
 
 ISSM_CHUNK = 64
 ISSM_F32, ISSM_BF16 = 0, 1
@@ -222,6 +223,23 @@ def load() -> C.CDLL:
     lib.issm_box_dist_bwd_scratch_bytes.restype = C.c_int64
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The compiled host side of the operators (csrc/host_ops.cpp: checks, argument blocks, allocation, autograd nodes)."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _issm_host
+        except ImportError as e:
+            raise RuntimeError("dest3d_amd/_issm_host.so is missing or does not load: build it with "
+                               "`python -m dest3d_amd.build`.  This package has no fallback path.") from e
+        _host = _issm_host
+    return _host
 
 
 def check(rc: int, what: str) -> None:

@@ -1,14 +1,17 @@
-"""Builds libissm_hip.so (gfx950) in-tree with hipcc.  `python -m dest3d_amd.build`."""
+"""Builds libissm_hip.so (gfx950, hipcc) and _issm_host.so (the operators' host side on PyTorch tensors, g++) in-tree.
+`python -m dest3d_amd.build`."""
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libissm_hip.so")
+HOST = os.path.join(HERE, "_issm_host.so")
 SOURCES = ["issm_abi.hip", "issm_fwd.hip", "issm_fwd_tile.hip", "issm_bwd.hip", "issm_bwd_tile.hip", "rmsnorm_gated.hip", "param_gen.hip", "dwconv_silu.hip", "box_dist.hip", "box_dist_sorted.hip", "hilbert.hip", "pointnet2_ops.hip", "transpose_states.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -40,16 +43,42 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build(verbose: bool = True) -> str:
-    """Compile every HIP source for gfx950 and link the shared library; returns its path."""
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
-        objs = list(ex.map(_compile, SOURCES))
-    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB]
+def _run(cmd, what: str) -> None:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stderr}")
+        raise RuntimeError(f"{what} failed:\n{r.stderr}")
+
+
+def _compile_host() -> str:
+    import torch
+    t = os.path.dirname(torch.__file__)
+    obj = os.path.join(CSRC, "host_ops.o")
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_path("include"), "/opt/rocm/include"]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", *("-I" + i for i in inc), "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-DTORCH_EXTENSION_NAME=_issm_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          "-c", os.path.join(CSRC, "host_ops.cpp"), "-o", obj], "g++ host_ops.cpp")
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run(["g++", "-shared", obj, "-o", HOST, "-L" + HERE, "-l:libissm_hip.so", "-L" + lib, "-ltorch", "-ltorch_cpu",
+          "-ltorch_python", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], "link of _issm_host.so")
+
+
+def build(verbose: bool = True) -> str:
+    """Compile every HIP source for gfx950 and the host side, link both shared libraries; returns the HIP library's path."""
+    with ThreadPoolExecutor(max_workers=4) as ex:
+        host = ex.submit(_compile_host)
+        objs = list(ex.map(_compile, SOURCES))
+        host_obj = host.result()
+    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB]
+    _run(cmd, "link")
+    _link_host(host_obj)
     if verbose:
-        print(f"built {LIB}")
+        print(f"built {LIB} and {HOST}")
     return LIB
 
 

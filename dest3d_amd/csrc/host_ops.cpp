@@ -1,0 +1,788 @@
+// Host side of the operators on PyTorch tensors: checks, argument blocks, output and workspace allocation and the autograd
+// nodes around the entry points of libissm_hip.so.  One call of the scan takes some thirty tensor descriptors, a dozen
+// allocations and an autograd node in each direction; issued from Python that is 100 - 300 us of host time for kernels
+// that take 30 - 100 us at a single scene's size, and a decoder layer (four projections, the core, a norm) ran at the pace
+// of the interpreter.  Here the same sequence costs the tensor library's own calls only.  All arithmetic is in the HIP
+// kernels (and, for the layer's four projections, in the tensor library's matrix products).
+#include <Python.h>
+
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include "../../include/issm.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+// ---------------------------------------------------------------------------------------------------------------- helpers
+void check(int rc, const char* what) {
+  if (rc != 0)
+    throw std::runtime_error(std::string(what) + " failed (status " + std::to_string(rc) + "): " + issm_last_error());
+}
+
+// Argument errors keep the exception types a Python implementation raises (called with the interpreter lock held).
+[[noreturn]] void raise_py(PyObject* type, const std::string& msg) {
+  PyErr_SetString(type, msg.c_str());
+  throw py::error_already_set();
+}
+void require(bool ok, const char* msg) {
+  if (!ok) raise_py(PyExc_AssertionError, msg);
+}
+void require_gpu(const Tensor& t, const char* name) {
+  if (!t.is_cuda())
+    raise_py(PyExc_RuntimeError, std::string(name) + " must live on a HIP device: the ISSM operator has no CPU path");
+}
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+bool is_kernel_type(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
+at::ScalarType kernel_type(at::ScalarType t) { return is_kernel_type(t) ? t : at::kFloat; }
+int code(at::ScalarType t) { return t == at::kBFloat16 ? ISSM_BF16 : ISSM_F32; }
+
+Tensor cast(const Tensor& t, at::ScalarType type) { return !t.defined() || t.scalar_type() == type ? t : t.to(type); }
+Tensor io_cast(const Tensor& t, at::ScalarType type) {
+  if (!t.defined()) return t;
+  Tensor r = cast(t, type);
+  return r.stride(-1) == 1 ? r : r.contiguous();
+}
+Tensor f32c(const Tensor& t) { return t.defined() ? cast(t, at::kFloat).contiguous() : t; }
+Tensor fresh(at::IntArrayRef sizes, const Tensor& like, at::ScalarType type) {
+  return at::empty(sizes, like.options().dtype(type));
+}
+template <class T = void>
+T* data(const Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
+
+issm_tensor desc(const Tensor& t) {
+  issm_tensor d{};
+  if (t.defined()) {
+    TORCH_CHECK(t.dim() == 4 && t.stride(-1) == 1, "innermost dimension must be contiguous");
+    d.ptr = t.data_ptr();
+    for (int i = 0; i < 3; ++i) d.stride[i] = t.stride(i);
+  }
+  return d;
+}
+
+typedef c10::optional<Tensor> MaybeTensor;   // an absent input of a node: it takes no undefined tensors
+
+Tensor opt(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+// ------------------------------------------------------------------------------------------------------------------- scan
+// Kernel-ready operands of one call (1 or 2 directions).
+struct Scan {
+  int ndir = 1;
+  Tensor x[2], dt, A, B[2], C[2], D, z[2], dt_bias, h0, seq;
+  bool softplus = false;
+  double lo = 0, hi = 0;
+
+  static Scan make(int ndir, const Tensor (&x)[2], const Tensor& dt, const Tensor& A, const Tensor (&B)[2], const Tensor (&C)[2],
+                   const Tensor& D, const Tensor (&z)[2], const Tensor& dt_bias, const Tensor& h0, const Tensor& seq,
+                   bool softplus, double lo, double hi) {
+    Scan s;
+    s.ndir = ndir;
+    const at::ScalarType io = kernel_type(x[0].scalar_type());
+    for (int i = 0; i < ndir; ++i) {
+      s.x[i] = io_cast(x[i], io);
+      s.B[i] = io_cast(B[i], io);
+      s.C[i] = io_cast(C[i], io);
+      s.z[i] = io_cast(z[i], io);
+    }
+    s.dt = io_cast(dt, kernel_type(dt.scalar_type()));
+    s.A = f32c(A);
+    s.D = f32c(D);
+    s.dt_bias = f32c(dt_bias);
+    if (h0.defined()) s.h0 = io_cast(h0, kernel_type(h0.scalar_type()));
+    if (seq.defined()) s.seq = cast(seq, at::kInt).contiguous();
+    s.softplus = softplus;
+    s.lo = lo;
+    s.hi = hi;
+    return s;
+  }
+
+  issm_scan_args args() const {
+    issm_scan_args a{};
+    a.dims.batch = (int)x[0].size(0);
+    a.dims.seqlen = (int)x[0].size(1);
+    a.dims.nheads = (int)x[0].size(2);
+    a.dims.headdim = (int)x[0].size(3);
+    a.dims.ngroups = (int)B[0].size(2);
+    a.dims.dstate = (int)B[0].size(3);
+    a.dims.chunk_size = ISSM_CHUNK;
+    a.dims.ndir = ndir;
+    a.io_dtype = code(x[0].scalar_type());
+    a.dt_dtype = code(dt.scalar_type());
+    a.h0_dtype = h0.defined() ? code(h0.scalar_type()) : ISSM_F32;
+    a.flags = (softplus ? ISSM_FLAG_DT_SOFTPLUS : 0u) | (D.defined() && D.dim() == 2 ? ISSM_FLAG_D_HAS_HDIM : 0u);
+    if (seq.defined()) {
+      a.flags |= ISSM_FLAG_SEQ_IDX;
+      a.seq_idx = data<const int32_t>(seq);
+      a.seq_idx_stride[0] = seq.stride(0);
+      a.seq_idx_stride[1] = seq.stride(1);
+    }
+    a.dt_min = (float)lo;
+    a.dt_max = (float)std::min(hi, 3.0e38);
+    for (int i = 0; i < ndir; ++i) {
+      a.x[i] = desc(x[i]);
+      a.Bm[i] = desc(B[i]);
+      a.Cm[i] = desc(C[i]);
+      a.z[i] = desc(z[i]);
+    }
+    a.dt = desc(dt);
+    a.A = data<const float>(A);
+    a.D = data<const float>(D);
+    a.dt_bias = data<const float>(dt_bias);
+    a.h0 = desc(h0);
+    a.stream = stream_of(x[0]);
+    return a;
+  }
+
+  struct Out {
+    Tensor y[2], last[2], ws;
+  };
+  Out forward(bool want_last) const {
+    issm_scan_args a = args();
+    Out o;
+    const auto& s = x[0].sizes();
+    for (int i = 0; i < ndir; ++i) {
+      o.y[i] = fresh(s, x[0], x[0].scalar_type());
+      a.out[i] = desc(o.y[i]);
+      if (want_last) {
+        o.last[i] = fresh({s[0], s[2], s[3], B[0].size(3)}, x[0], at::kFloat);
+        a.final_states[i] = data<float>(o.last[i]);
+      }
+    }
+    size_t n = 0;
+    check(issm_fwd_workspace_bytes(&a, &n), "workspace query");
+    o.ws = fresh({(int64_t)std::max<size_t>(n, 256)}, x[0], at::kByte);
+    a.workspace = data(o.ws);
+    a.workspace_bytes = (size_t)o.ws.numel();
+    check(issm_scan_fwd(&a), "issm_scan_fwd");
+    return o;
+  }
+
+  struct Grad {
+    Tensor dx[2], ddt, dA, dB[2], dC[2], dD, dz[2], dbias, dh0;
+  };
+  // dy: one per direction; dlast may be undefined (no gradient reaches the final states)
+  Grad backward(const Tensor& ws_fwd, const Tensor (&dy_)[2], const Tensor (&dlast_)[2]) const {
+    issm_scan_args a = args();
+    const at::ScalarType io = x[0].scalar_type();
+    a.saved = data(ws_fwd);
+    Grad g;
+    Tensor dy[2], dlast[2];
+    for (int i = 0; i < ndir; ++i) {
+      dy[i] = dy_[i].defined() ? io_cast(dy_[i], io) : at::zeros(x[i].sizes(), x[i].options());
+      dlast[i] = f32c(dlast_[i]);
+      g.dx[i] = fresh(x[i].sizes(), x[i], io);
+      g.dB[i] = fresh(B[i].sizes(), x[i], io);
+      g.dC[i] = fresh(C[i].sizes(), x[i], io);
+      if (z[i].defined()) g.dz[i] = fresh(x[i].sizes(), x[i], io);
+      a.dout[i] = desc(dy[i]);
+      a.dfinal[i] = data<const float>(dlast[i]);
+      a.dx[i] = desc(g.dx[i]);
+      a.dB[i] = desc(g.dB[i]);
+      a.dC[i] = desc(g.dC[i]);
+      a.dz[i] = desc(g.dz[i]);
+    }
+    g.ddt = fresh(dt.sizes(), x[0], dt.scalar_type());
+    g.dA = fresh(A.sizes(), x[0], at::kFloat);
+    if (D.defined()) g.dD = fresh(D.sizes(), x[0], at::kFloat);
+    if (dt_bias.defined()) g.dbias = fresh(dt_bias.sizes(), x[0], at::kFloat);
+    g.dh0 = fresh({x[0].size(0), x[0].size(2), x[0].size(3), B[0].size(3)}, x[0], at::kFloat);
+    a.ddt = desc(g.ddt);
+    a.dA = data<float>(g.dA);
+    a.dD = data<float>(g.dD);
+    a.ddt_bias = data<float>(g.dbias);
+    a.dh0 = data<float>(g.dh0);
+    size_t n = 0;
+    check(issm_bwd_workspace_bytes(&a, &n), "workspace query");
+    Tensor ws = fresh({(int64_t)std::max<size_t>(n, 256)}, x[0], at::kByte);
+    a.bwd_workspace = data(ws);
+    a.bwd_workspace_bytes = (size_t)ws.numel();
+    check(issm_scan_bwd(&a), "issm_scan_bwd");
+    return g;
+  }
+
+  static constexpr int NSAVED = 14;
+  void push(variable_list& v) const {
+    for (const Tensor& t : {x[0], x[1], dt, A, B[0], B[1], C[0], C[1], D, z[0], z[1], dt_bias, h0, seq}) v.push_back(t);
+  }
+  static Scan pop(const variable_list& v, size_t at, int ndir, bool softplus, double lo, double hi) {
+    Scan s;
+    s.ndir = ndir;
+    Tensor* to[NSAVED] = {&s.x[0], &s.x[1], &s.dt, &s.A, &s.B[0], &s.B[1], &s.C[0], &s.C[1], &s.D, &s.z[0], &s.z[1], &s.dt_bias,
+                          &s.h0, &s.seq};
+    for (int i = 0; i < NSAVED; ++i) *to[i] = v[at + i];
+    s.softplus = softplus;
+    s.lo = lo;
+    s.hi = hi;
+    return s;
+  }
+};
+
+// Inputs 0 .. 11 of the node: x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, z, dt_bias, h0 (those of an absent direction undefined).
+// The caller's own tensors are among the saved ones: reading them back is what makes the autograd engine raise when one of
+// them was modified in place between forward and backward.
+struct ScanFn : public Function<ScanFn> {
+  static constexpr int NIN = 12;
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& x_f, const MaybeTensor& x_b_, const Tensor& dt, const Tensor& A,
+                               const Tensor& B_f, const MaybeTensor& B_b_, const Tensor& C_f, const MaybeTensor& C_b_,
+                               const MaybeTensor& D_, const MaybeTensor& z_, const MaybeTensor& dt_bias_, const MaybeTensor& h0_,
+                               const MaybeTensor& seq_, bool softplus, double lo, double hi, bool want_last) {
+    const c10::DeviceGuard guard(x_f.device());
+    const Tensor x_b = opt(x_b_), B_b = opt(B_b_), C_b = opt(C_b_), D = opt(D_), z = opt(z_), dt_bias = opt(dt_bias_), h0 = opt(h0_),
+                 seq = opt(seq_);
+    const int ndir = x_b.defined() ? 2 : 1;
+    const Tensor x[2] = {x_f, x_b}, B[2] = {B_f, B_b}, C[2] = {C_f, C_b}, zz[2] = {z, Tensor()};
+    const Scan s = Scan::make(ndir, x, dt, A, B, C, D, zz, dt_bias, h0, seq, softplus, lo, hi);
+    Scan::Out o = s.forward(want_last);
+    ctx->set_materialize_grads(false);
+    variable_list saved{x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, z, dt_bias, h0};
+    s.push(saved);
+    saved.push_back(o.ws);
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["ndir"] = (int64_t)ndir;
+    ctx->saved_data["softplus"] = softplus;
+    ctx->saved_data["lo"] = lo;
+    ctx->saved_data["hi"] = hi;
+    ctx->saved_data["last"] = want_last;
+    variable_list out;
+    for (int i = 0; i < ndir; ++i) out.push_back(cast(o.y[i], x[i].scalar_type()));
+    if (want_last)
+      for (int i = 0; i < ndir; ++i) out.push_back(o.last[i]);
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const int ndir = (int)ctx->saved_data["ndir"].toInt();
+    const bool last = ctx->saved_data["last"].toBool();
+    const Scan s = Scan::pop(v, NIN, ndir, ctx->saved_data["softplus"].toBool(), ctx->saved_data["lo"].toDouble(),
+                             ctx->saved_data["hi"].toDouble());
+    const c10::DeviceGuard guard(s.x[0].device());
+    Tensor dy[2], dlast[2];
+    for (int i = 0; i < ndir; ++i) {
+      dy[i] = grads[i];
+      if (last) dlast[i] = grads[ndir + i];
+    }
+    Scan::Grad g = s.backward(v[NIN + Scan::NSAVED], dy, dlast);
+    const Tensor all[NIN] = {g.dx[0], g.dx[1], g.ddt, g.dA, g.dB[0], g.dB[1], g.dC[0], g.dC[1], g.dD, g.dz[0], g.dbias, g.dh0};
+    variable_list out(NIN + 5);
+    for (int i = 0; i < NIN; ++i)
+      if (v[i].defined() && all[i].defined()) out[i] = cast(all[i], v[i].scalar_type());
+    return out;
+  }
+};
+
+std::string shape_text(const Tensor& t) {
+  std::string s = "(";
+  for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+  return s + ")";
+}
+
+// shape rules of issm_combined.py:58-83
+void check_scan(const Tensor* x, const Tensor& dt, const Tensor& A, const Tensor* B, const Tensor* C, int ndir, const Tensor& D,
+                const Tensor& z, const Tensor& dt_bias, const Tensor& h0, const Tensor& seq) {
+  require_gpu(x[0], "x");
+  if (x[0].dim() != 4) raise_py(PyExc_ValueError, "x must be (batch, seqlen, nheads, headdim), got " + shape_text(x[0]));
+  if (B[0].dim() != 4) raise_py(PyExc_ValueError, "B must be (batch, seqlen, ngroups, dstate), got " + shape_text(B[0]));
+  const int64_t b = x[0].size(0), l = x[0].size(1), h = x[0].size(2), p = x[0].size(3), g = B[0].size(2), n = B[0].size(3);
+  require(g > 0 && h % g == 0, "nheads must be divisible by ngroups");
+  for (int i = 0; i < ndir; ++i) {
+    require(x[i].sizes() == at::IntArrayRef({b, l, h, p}), "x must be (batch, seqlen, nheads, headdim)");
+    require(B[i].sizes() == at::IntArrayRef({b, l, g, n}), "B must be (batch, seqlen, ngroups, dstate)");
+    require(C[i].sizes() == B[i].sizes(), "C must have B's shape");
+  }
+  require(dt.sizes() == at::IntArrayRef({b, l, h, n}), "dt must be (batch, seqlen, nheads, dstate)");
+  require(A.sizes() == at::IntArrayRef({h, n}), "A must be (nheads, dstate)");
+  if (z.defined()) require(z.sizes() == x[0].sizes(), "z must have x's shape");
+  if (D.defined())
+    require(D.sizes() == at::IntArrayRef({h, p}) || D.sizes() == at::IntArrayRef({h}), "D must be (nheads,) or (nheads, headdim)");
+  if (dt_bias.defined()) require(dt_bias.sizes() == at::IntArrayRef({h, n}), "dt_bias must be (nheads, dstate)");
+  if (h0.defined()) require(h0.sizes() == at::IntArrayRef({b, h, p, n}), "initial_states must be (batch, nheads, headdim, dstate)");
+  if (seq.defined()) require(seq.sizes() == at::IntArrayRef({b, l}), "seq_idx must be (batch, seqlen)");
+}
+
+std::vector<Tensor> scan(const Tensor& x, const Tensor& dt, const Tensor& A, const Tensor& B, const Tensor& C,
+                         const MaybeTensor& D_, const MaybeTensor& z_, const MaybeTensor& dt_bias_,
+                         const MaybeTensor& h0_, const MaybeTensor& seq_, bool softplus, double lo, double hi,
+                         bool want_last) {
+  const Tensor D = opt(D_), z = opt(z_), dt_bias = opt(dt_bias_), h0 = opt(h0_), seq = opt(seq_);
+  check_scan(&x, dt, A, &B, &C, 1, D, z, dt_bias, h0, seq);
+  py::gil_scoped_release release;
+  return ScanFn::apply(x, MaybeTensor(), dt, A, B, MaybeTensor(), C, MaybeTensor(), D_, z_, dt_bias_, h0_, seq_, softplus, lo, hi,
+                       want_last);
+}
+
+std::vector<Tensor> biscan(const Tensor& x_f, const Tensor& x_b, const Tensor& dt, const Tensor& A, const Tensor& B_f,
+                           const Tensor& B_b, const Tensor& C_f, const Tensor& C_b, const MaybeTensor& D_,
+                           const MaybeTensor& dt_bias_, const MaybeTensor& h0_, bool softplus, double lo,
+                           double hi) {
+  const Tensor D = opt(D_), dt_bias = opt(dt_bias_), h0 = opt(h0_), none;
+  const Tensor x[2] = {x_f, x_b}, B[2] = {B_f, B_b}, C[2] = {C_f, C_b};
+  check_scan(x, dt, A, B, C, 2, D, none, dt_bias, h0, none);
+  py::gil_scoped_release release;
+  return ScanFn::apply(x_f, MaybeTensor(x_b), dt, A, B_f, MaybeTensor(B_b), C_f, MaybeTensor(C_b), D_, MaybeTensor(), dt_bias_, h0_,
+                       MaybeTensor(), softplus, lo, hi, true);
+}
+
+// ------------------------------------------------------------------------------------------------------------- gated norm
+Tensor as_rows(const Tensor& t) {
+  Tensor r = t.reshape({-1, t.size(-1)});
+  return r.stride(-1) == 1 ? r : r.contiguous();
+}
+
+issm_norm_args norm_args(const Tensor& x, const Tensor& z, const Tensor& w, const Tensor& bias, double eps, int64_t group,
+                         bool before_gate, bool layer_norm) {
+  issm_norm_args a{};
+  a.rows = x.size(0);
+  a.ncols = (int)x.size(1);
+  a.group_size = (int)group;
+  a.dtype = code(x.scalar_type());
+  a.weight_dtype = code(w.scalar_type());
+  a.norm_before_gate = before_gate;
+  a.eps = (float)eps;
+  a.x = data(x);
+  a.w = data(w);
+  a.x_row_stride = x.stride(0);
+  if (z.defined()) {
+    a.z = data(z);
+    a.z_row_stride = z.stride(0);
+  }
+  a.bias = data(bias);
+  a.layer_norm = layer_norm;
+  a.stream = stream_of(x);
+  return a;
+}
+
+struct NormFn : public Function<NormFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& z_,
+                        double eps, int64_t group, bool before_gate, bool rms) {
+    const c10::DeviceGuard guard(x.device());
+    const Tensor bias = opt(bias_), z = opt(z_);
+    const at::ScalarType k = kernel_type(x.scalar_type());
+    Tensor x2 = as_rows(cast(x, k)), z2, w = weight, b;
+    if (z.defined()) z2 = as_rows(cast(z, k));
+    if (!is_kernel_type(w.scalar_type())) w = w.to(at::kFloat);
+    if (bias.defined()) {
+      // The kernels read weight and bias in one dtype, the reference's widen each to fp32 on its own
+      // (layernorm_gated.py:77-80): where the two differ both go to fp32, so that neither is rounded.
+      if (bias.scalar_type() != w.scalar_type()) w = w.to(at::kFloat);
+      b = cast(bias, w.scalar_type()).contiguous();
+    }
+    w = w.contiguous();
+    const int64_t groups = group ? x2.size(1) / group : 1;
+    Tensor y = fresh(x2.sizes(), x2, k), stats = fresh({2, groups * x2.size(0)}, x2, at::kFloat);
+    issm_norm_args a = norm_args(x2, z2, w, b, eps, group, before_gate, !rms);
+    a.y = data(y);
+    a.y_row_stride = y.stride(0);
+    a.rstd = data<float>(stats);
+    if (!rms) a.mean = data<float>(stats) + stats.size(1);
+    check(issm_gated_rmsnorm_fwd(&a), "issm_gated_rmsnorm_fwd");
+    ctx->save_for_backward({x, weight, bias, z, x2, z2, w, b, stats});
+    ctx->saved_data["eps"] = eps;
+    ctx->saved_data["group"] = group;
+    ctx->saved_data["before"] = before_gate;
+    ctx->saved_data["rms"] = rms;
+    return cast(y.view(x.sizes()), x.scalar_type());
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const Tensor &x2 = v[4], &z2 = v[5], &w = v[6], &b = v[7], &stats = v[8];
+    const c10::DeviceGuard guard(x2.device());
+    const bool rms = ctx->saved_data["rms"].toBool();
+    Tensor dy = as_rows(cast(grads[0], x2.scalar_type()));
+    Tensor dx = fresh(x2.sizes(), x2, x2.scalar_type()), dz;
+    if (z2.defined()) dz = fresh(z2.sizes(), z2, z2.scalar_type());
+    const int64_t cols = x2.size(1), nb = issm_rmsnorm_bwd_blocks(x2.size(0)), np = b.defined() ? 2 : 1;
+    Tensor part = fresh({np, nb, cols}, x2, at::kFloat), dwb = fresh({np, cols}, x2, at::kFloat);
+    issm_norm_args a = norm_args(x2, z2, w, b, ctx->saved_data["eps"].toDouble(), ctx->saved_data["group"].toInt(),
+                                 ctx->saved_data["before"].toBool(), !rms);
+    a.rstd = data<float>(stats);
+    if (!rms) a.mean = data<float>(stats) + stats.size(1);
+    a.dy = data(dy);
+    a.dy_row_stride = dy.stride(0);
+    a.dx = data(dx);
+    a.dx_row_stride = dx.stride(0);
+    if (dz.defined()) {
+      a.dz = data(dz);
+      a.dz_row_stride = dz.stride(0);
+    }
+    a.dw_partial = data<float>(part);
+    a.dw = data<float>(dwb);
+    if (np == 2) {
+      a.db_partial = data<float>(part) + nb * cols;
+      a.db = data<float>(dwb) + cols;
+    }
+    check(issm_gated_rmsnorm_bwd(&a), "issm_gated_rmsnorm_bwd");
+    variable_list out(8);
+    out[0] = cast(dx.view(v[0].sizes()), v[0].scalar_type());
+    out[1] = cast(dwb.select(0, 0), v[1].scalar_type());
+    if (np == 2) out[2] = cast(dwb.select(0, 1), v[2].scalar_type());
+    if (dz.defined()) out[3] = cast(dz.view(v[3].sizes()), v[3].scalar_type());
+    return out;
+  }
+};
+
+// group: 0 = the whole row
+Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& z_, double eps,
+            int64_t group, bool before_gate, bool rms) {
+  const Tensor bias = opt(bias_), z = opt(z_);
+  require_gpu(x, "x");
+  if (z.defined()) require(z.sizes() == x.sizes(), "z must have x's shape");
+  require(weight.dim() == 1 && weight.size(0) == x.size(-1), "weight must have one entry per column");
+  if (bias.defined()) require(bias.dim() == 1 && bias.size(0) == x.size(-1), "bias must have one entry per column");
+  require(group >= 0 && (group == 0 || x.size(-1) % group == 0), "group_size must divide the number of columns");
+  py::gil_scoped_release release;
+  return NormFn::apply(x, weight, bias_, z_, eps, group, before_gate, rms);
+}
+
+// ------------------------------------------------------------------------------------------------ projections of the layer
+// y = x W^T for a (tokens, features) activation with thousands of tokens and a few hundred features (the four projections of
+// the layer).  Forward and input gradient are the library products nn.Linear uses; the weight gradient dW = dy^T x contracts
+// over the tokens, and as one product its (out x in) result makes only a few dozen tiles -- a fraction of the GPU, 54 us for
+// 8192 x 288 -> 586 in bf16.  Here the tokens are cut into slices that run as one batched product and the slices' results are
+// summed (24 us).
+struct LinearFn : public Function<LinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    ctx->save_for_backward({x, w});
+    return at::linear(x, w);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    // (whatever autocast says where backward() is called: the products below see operands of one type already)
+    const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
+    const variable_list v = ctx->get_saved_variables();
+    const Tensor &x = v[0], &w = v[1];
+    const Tensor dy = cast(grads[0], x.scalar_type());
+    Tensor dx, dw;
+    if (ctx->needs_input_grad(0)) dx = at::matmul(dy, w);
+    if (ctx->needs_input_grad(1)) {
+      const Tensor x2 = x.reshape({-1, x.size(-1)}), dy2 = dy.reshape({-1, dy.size(-1)});
+      const int64_t tokens = x2.size(0);
+      int64_t slices = x2.scalar_type() == at::kBFloat16 ? 4 : 2;   // fastest of 2 .. 32 on MI355X at 2048 and 8192 tokens
+      if (tokens < 1024 || tokens % slices) slices = 1;
+      if (slices > 1)
+        dw = at::bmm(dy2.view({slices, tokens / slices, -1}).transpose(1, 2), x2.view({slices, tokens / slices, -1})).sum(0);
+      else
+        dw = at::mm(dy2.t(), x2);
+    }
+    return {dx, dw};
+  }
+};
+
+Tensor linear_tokens(Tensor x, Tensor w) {
+  // under autocast the product runs in the autocast type; what is saved must be in that type too, or the backward would mix
+  // types
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) {
+    const at::ScalarType t = at::autocast::get_autocast_dtype(at::kCUDA);
+    if (x.scalar_type() != at::kDouble) x = x.to(t);
+    if (w.scalar_type() != at::kDouble) w = w.to(t);
+  }
+  const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
+  return LinearFn::apply(x, w);
+}
+
+// ------------------------------------------------------------------------------- the chain between a layer's projections
+// (B, R, C) -> (B, C, R): alpha * (in0 + in1) in `type`; in1 may be undefined (issm_transpose_states)
+Tensor transpose_states(const Tensor& in0_, const Tensor& in1_, double alpha, at::ScalarType type) {
+  const at::ScalarType k = kernel_type(in0_.scalar_type());
+  const Tensor in0 = cast(in0_, k).contiguous(), in1 = in1_.defined() ? cast(in1_, k).contiguous() : in1_;
+  Tensor out = fresh({in0.size(0), in0.size(2), in0.size(1)}, in0, type);
+  issm_transpose_args a{};
+  a.batch = (int)in0.size(0);
+  a.rows = (int)in0.size(1);
+  a.cols = (int)in0.size(2);
+  a.in_dtype = code(k);
+  a.out_dtype = code(type);
+  a.in0 = data(in0);
+  a.in1 = data(in1);
+  a.out = data(out);
+  a.alpha = (float)alpha;
+  a.stream = stream_of(in0);
+  check(issm_transpose_states(&a), "issm_transpose_states");
+  return out;
+}
+
+constexpr int TAPS = 7;   // of the depthwise convolutions
+constexpr int WIDTH = 16; // of the distance encoding
+
+issm_dwconv_args conv_args(const Tensor& u) {
+  issm_dwconv_args a{};
+  a.batch = (int)u.size(0);
+  a.seqlen = (int)u.size(1);
+  a.channels = (int)u.size(2);
+  a.nsets = 2;
+  a.taps = TAPS;
+  a.dtype = code(u.scalar_type());
+  a.u = data(u);
+  a.u_batch_stride = u.stride(0);
+  a.u_token_stride = u.stride(1);
+  a.chain = 1;   // key_conv_back reads key_conv's output
+  a.stream = stream_of(u);
+  return a;
+}
+
+issm_pgen_args pgen_args(const Tensor& dist, const float* W, int64_t H, int64_t G) {
+  issm_pgen_args a{};
+  a.tokens = dist.size(0) * dist.size(1);
+  a.K = (int)dist.size(2);
+  a.M = (int)dist.size(3);
+  a.H = (int)H;
+  a.G = (int)G;
+  a.dtype = code(dist.scalar_type());
+  a.has_back = 1;
+  a.dist = data(dist);
+  a.W = W;
+  a.stream = stream_of(dist);
+  return a;
+}
+
+// Depthwise conv + SiLU of both branches (the reversed-order branch convolves the forward-order branch's output,
+// dest_module.py:530,534), generation of dt / B / C from the distance encoding, the bidirectional scan, the average of the two
+// directions and the gated RMSNorm as one autograd node (dest_module.py:528-581): the entry points of libissm_hip.so back to
+// back, and their backward passes chained by hand.
+struct CoreFn : public Function<CoreFn> {
+  // the small parameters, in the order of their places in the flat fp32 buffer
+  enum { CW_F, CW_B, CB_F, CB_B, DT_W, BC_W, DT_BIAS, A_LOG, NSMALL };
+  // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
+  static constexpr int NIN = 14;
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
+                               const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
+                               const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
+                               const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
+                               int64_t ngroups, double lo, double hi, double eps) {
+    const c10::DeviceGuard guard(zxbcdt.device());
+    const Tensor weights = opt(weights_);
+    const int64_t Bsz = zxbcdt.size(0), Ln = zxbcdt.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
+                  K = dist.size(2);
+    const at::ScalarType k = kernel_type(zxbcdt.scalar_type());
+    Tensor zx = io_cast(zxbcdt, k);
+    const Tensor z = zx.narrow(2, 0, di), xbc = zx.narrow(2, di, Cc), dt_tok = zx.narrow(2, di + Cc, H);
+    // all small parameters in one fp32 buffer (one concatenation + one conversion instead of one per tensor); adjacent pieces
+    // form the stacked operands the kernels take
+    std::vector<Tensor> small;
+    int64_t off[NSMALL + 1] = {0};
+    for (const Tensor& t : {conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log}) {
+      off[small.size() + 1] = off[small.size()] + t.numel();
+      small.push_back(t.reshape({-1}));
+    }
+    const Tensor flat = cast(at::cat(small), at::kFloat);
+    float* const par = data<float>(flat);
+    // 1. both depthwise convolutions + SiLU; the conv writes x and the B / C biases apart
+    Tensor x = fresh({2, Bsz, Ln, H, P}, zx, k), tail = fresh({2, Bsz, Ln, 2 * G}, zx, k), pre = fresh({2, Bsz, Ln, Cc}, zx, k);
+    {
+      issm_dwconv_args a = conv_args(xbc);
+      a.w = par;
+      a.bias = par + off[CB_F];
+      a.y = data(x);
+      a.pre = data(pre);
+      a.split = (int)di;
+      a.y_tail = data(tail);
+      check(issm_dwconv_silu_fwd(&a), "issm_dwconv_silu_fwd");
+    }
+    // 2. dt / B / C (and the reversed-order B / C) from the distance encoding
+    Tensor bias = fresh({Bsz, Ln, H + 4 * G}, zx, at::kFloat);
+    {
+      Tensor b_dt = bias.narrow(2, 0, H);
+      at::add_out(b_dt, dt_tok, flat.narrow(0, off[DT_BIAS], H));
+    }
+    bias.narrow(2, H, 4 * G).unflatten(-1, {2, 2 * G}).copy_(tail.permute({1, 2, 0, 3}));
+    const Tensor d = cast(dist, k).contiguous(), wt = f32c(weights);
+    Tensor dt = fresh({Bsz, Ln, H, K}, zx, k), bc = fresh({4, Bsz, Ln, G, K}, zx, k), raw;
+    {
+      issm_pgen_args a = pgen_args(d, par + off[DT_W], H, G);
+      a.bias = data<const float>(bias);
+      a.dt = data(dt);
+      void** to[4] = {&a.Bm, &a.Cm, &a.Bm_back, &a.Cm_back};
+      for (int i = 0; i < 4; ++i) *to[i] = (char*)data(bc) + i * (bc.numel() / 4) * bc.element_size();
+      if (wt.defined()) {
+        raw = fresh(dt.sizes(), zx, k);
+        a.weights = data<const float>(wt);
+        a.dt_raw = data(raw);
+      }
+      check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
+    }
+    // 3. the bidirectional scan, queries as initial state
+    const Tensor A1 = flat.narrow(0, off[A_LOG], H).exp().neg_();
+    const Tensor h0 = transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()))
+                          .view({Bsz, H, P, K});
+    const Tensor xs[2] = {x.select(0, 0), x.select(0, 1)}, Bs[2] = {bc.select(0, 0), bc.select(0, 2)},
+                 Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
+    const Scan s = Scan::make(2, xs, dt, A1.unsqueeze(1).expand({H, K}), Bs, Cs, D, none, Tensor(), h0, Tensor(),
+                              !wt.defined(), lo, hi);
+    Scan::Out o = s.forward(true);
+    // 4. gated RMSNorm (norm(x * silu(z))) of the two directions' average: the norm of s / 2 with eps is the norm of s with
+    // 4 eps, so the sum goes in as it is and the halving never runs (nor its backward)
+    const Tensor key = at::add(o.y[0], o.y[1]).view({Bsz * Ln, di});
+    const Tensor z2 = z.as_strided({Bsz * Ln, di}, {zx.stride(1), 1});
+    const Tensor nw = cast(norm_w, kernel_type(norm_w.scalar_type())).contiguous();
+    Tensor key_n = fresh(key.sizes(), key, k), rstd = fresh({Bsz * Ln}, key, at::kFloat);
+    {
+      issm_norm_args a = norm_args(key, z2, nw, Tensor(), 4.0 * eps, 0, false, false);
+      a.y = data(key_n);
+      a.y_row_stride = key_n.stride(0);
+      a.rstd = data<float>(rstd);
+      check(issm_gated_rmsnorm_fwd(&a), "issm_gated_rmsnorm_fwd");
+    }
+    const Tensor last = transpose_states(o.last[0].view({Bsz, di, K}), o.last[1].view({Bsz, di, K}), 0.5,
+                                         kernel_type(h0_lin.scalar_type()));
+    variable_list saved{zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
+                        norm_w};
+    for (const Tensor& t : {xbc, pre, flat, d, wt, raw, key, z2, nw, rstd, A1, o.ws}) saved.push_back(t);
+    s.push(saved);
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["sizes"] = std::vector<int64_t>{H, G, di};
+    ctx->saved_data["limits"] = std::vector<double>{lo, hi, 4.0 * eps};
+    return {cast(key_n.view({Bsz, Ln, di}), zxbcdt.scalar_type()), cast(last, h0_lin.scalar_type())};
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
+    const variable_list v = ctx->get_saved_variables();
+    const Tensor &xbc = v[NIN], &pre = v[NIN + 1], &flat = v[NIN + 2], &d = v[NIN + 3], &wt = v[NIN + 4], &raw = v[NIN + 5],
+                 &key = v[NIN + 6], &z2 = v[NIN + 7], &nw = v[NIN + 8], &rstd = v[NIN + 9], &A1 = v[NIN + 10], &ws = v[NIN + 11];
+    const c10::DeviceGuard guard(key.device());
+    const std::vector<int64_t> sizes = ctx->saved_data["sizes"].toIntVector();
+    const std::vector<double> lim = ctx->saved_data["limits"].toDoubleVector();
+    const int64_t H = sizes[0], G = sizes[1], di = sizes[2], P = di / H, Cc = di + 2 * G, Bsz = d.size(0), Ln = d.size(1),
+                  K = d.size(2), R0 = H + 2 * G, R = H + 4 * G, Wd = di + Cc + H;
+    const Scan s = Scan::pop(v, NIN + 12, 2, !wt.defined(), lim[0], lim[1]);
+    const at::ScalarType k = key.scalar_type(), hdt = v[1].scalar_type();
+    float* const par = data<float>(flat);
+    const int64_t off_w = 2 * Cc * TAPS + 2 * Cc;
+    // 4'. gated RMSNorm
+    const Tensor dy = cast(grads[0], k).reshape({Bsz * Ln, di}).contiguous();
+    Tensor dkey = fresh(key.sizes(), key, k);
+    Tensor dzx = fresh({Bsz, Ln, Wd}, key, k);   // row of d zxbcdt: [dz | d xbc | d dt]; each producer writes its part
+    const int64_t nb = issm_rmsnorm_bwd_blocks(Bsz * Ln);
+    Tensor dwp = fresh({nb, di}, key, at::kFloat), dnw = fresh({di}, key, at::kFloat);
+    {
+      issm_norm_args a = norm_args(key, z2, nw, Tensor(), lim[2], 0, false, false);
+      a.rstd = data<float>(rstd);
+      a.dy = data(dy);
+      a.dy_row_stride = dy.stride(0);
+      a.dx = data(dkey);
+      a.dx_row_stride = dkey.stride(0);
+      a.dz = data(dzx);
+      a.dz_row_stride = Wd;
+      a.dw_partial = data<float>(dwp);
+      a.dw = data<float>(dnw);
+      check(issm_gated_rmsnorm_bwd(&a), "issm_gated_rmsnorm_bwd");
+    }
+    // 3'. the scan: both directions receive the gradient of their sum, and half of the averaged final states'
+    const Tensor dyh = dkey.view({Bsz, Ln, H, P});
+    const Tensor dfin = transpose_states(grads[1].reshape({Bsz, K, di}), Tensor(), 0.5, at::kFloat).view({Bsz, H, P, K});
+    const Tensor dys[2] = {dyh, dyh}, dlast[2] = {dfin, dfin};
+    const Scan::Grad g = s.backward(ws, dys, dlast);
+    // 2'. parameter generation
+    Tensor ddist, dbias = fresh({Bsz, Ln, R}, key, at::kFloat), dW = fresh({R0, WIDTH}, key, at::kFloat),
+                  dbias_sum = fresh({R}, key, at::kFloat);
+    Tensor dwpart = fresh({std::max(issm_param_gen_bwd_blocks(Bsz * Ln), 1), R0, WIDTH}, key, at::kFloat);
+    if (ctx->needs_input_grad(2)) ddist = fresh(d.sizes(), d, k);
+    {
+      issm_pgen_args a = pgen_args(d, par + off_w, H, G);
+      a.ddt = data(g.ddt);
+      a.dBm = data(g.dB[0]);
+      a.dCm = data(g.dC[0]);
+      a.dBm_back = data(g.dB[1]);
+      a.dCm_back = data(g.dC[1]);
+      a.ddist = data(ddist);
+      a.dbias = data<float>(dbias);
+      a.dw_partial = data<float>(dwpart);
+      a.dW = data<float>(dW);
+      a.dbias_sum = data<float>(dbias_sum);
+      if (wt.defined()) {
+        a.weights = data<const float>(wt);
+        a.dt_raw = data(raw);
+      }
+      check(issm_param_gen_bwd(&a), "issm_param_gen_bwd");
+    }
+    // 1'. the convolutions: gradients of (x, b-bias, c-bias) per branch
+    Tensor dtail = fresh({2, Bsz, Ln, 2 * G}, key, k);
+    dtail.copy_(dbias.narrow(2, H, 4 * G).unflatten(-1, {2, 2 * G}).permute({2, 0, 1, 3}));
+    Tensor part = fresh({std::max(issm_dwconv_partial_rows((int)Bsz, (int)Ln), 1), 2, 8, Cc}, key, at::kFloat);
+    Tensor dcw = fresh({2, Cc, TAPS}, key, at::kFloat), dcb = fresh({2, Cc}, key, at::kFloat);
+    {
+      issm_dwconv_args a = conv_args(xbc);
+      a.w = par;
+      a.pre = data(pre);
+      a.split = (int)di;
+      for (int i = 0; i < 2; ++i) {
+        a.dy[i] = data(g.dx[i]);
+        a.dy_tail[i] = (char*)data(dtail) + i * (dtail.numel() / 2) * dtail.element_size();
+      }
+      a.du = (char*)data(dzx) + di * dzx.element_size();
+      a.du_batch_stride = Ln * Wd;
+      a.du_token_stride = Wd;
+      a.partial = data<float>(part);
+      a.dw = data<float>(dcw);
+      a.dbias = data<float>(dcb);
+      check(issm_dwconv_silu_bwd(&a), "issm_dwconv_silu_bwd");
+    }
+    dzx.narrow(2, di + Cc, H).copy_(dbias.narrow(2, 0, H));
+    const Tensor dA_log = g.dA.sum(-1).mul_(A1);
+    const Tensor dh0 = transpose_states(g.dh0.view({Bsz, di, K}), Tensor(), 1.0, kernel_type(hdt));
+    // parameter gradients, inputs 4 .. 13: one buffer, one conversion to the parameters' type when they share one
+    std::vector<Tensor> pg{dcw.select(0, 0), dcb.select(0, 0), dcw.select(0, 1), dcb.select(0, 1), dW.narrow(0, 0, H),
+                           dW.narrow(0, H, 2 * G), dbias_sum.narrow(0, 0, H), dA_log, g.dD, dnw};
+    bool shared = v[4].scalar_type() != at::kFloat;
+    for (int i = 4; i < NIN; ++i) shared = shared && v[i].scalar_type() == v[4].scalar_type();
+    if (shared) {
+      std::vector<int64_t> n;
+      for (Tensor& t : pg) {
+        n.push_back(t.numel());
+        t = t.reshape({-1});
+      }
+      pg = at::split_with_sizes(at::cat(pg).to(v[4].scalar_type()), n);
+    }
+    variable_list out(NIN + 6);
+    out[0] = cast(dzx, v[0].scalar_type());
+    out[1] = cast(dh0, hdt);
+    out[2] = cast(ddist, v[2].scalar_type());
+    for (int i = 4; i < NIN; ++i) out[i] = cast(pg[i - 4], v[i].scalar_type()).view(v[i].sizes());
+    return out;
+  }
+};
+
+// MultiHeadISSMScan.forward as a whole (dest_module.py:515-585) for the configuration CoreFn is built for.
+std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, const Tensor& dist, const MaybeTensor& weights_,
+                               const Tensor& key_proj, const Tensor& query_proj, const Tensor& out_key_proj,
+                               const Tensor& out_query_proj, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
+                               const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
+                               const Tensor& A_log, const Tensor& D, const Tensor& key_norm, double key_eps,
+                               const MaybeTensor& query_w, const MaybeTensor& query_b, double query_eps,
+                               int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
+  require_gpu(in_key, "in_key");
+  require(in_key.dim() == 3 && in_query.dim() == 3 && dist.dim() == 4, "in_key (B, L, D), in_query (B, K, D), dist (B, L, K, M)");
+  require(dist.size(0) == in_key.size(0) && dist.size(1) == in_key.size(1) && in_query.size(0) == in_key.size(0) &&
+              dist.size(2) == in_query.size(1) && dist.size(3) == WIDTH, "dist must be (B, L, K, 16)");
+  const Tensor weights = opt(weights_);
+  if (weights.defined()) require(weights.sizes() == dist.sizes().slice(0, 3), "mask must be (B, L, K)");
+  py::gil_scoped_release release;
+  const Tensor zx = linear_tokens(in_key, key_proj), h0 = linear_tokens(in_query, query_proj);
+  variable_list core = CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
+                                     key_norm, d_inner, nheads, ngroups, lo, hi, key_eps);
+  const Tensor q = at::layer_norm(core[1], {d_inner}, query_w, query_b, query_eps);
+  return {linear_tokens(core[0], out_key_proj), linear_tokens(q, out_query_proj)};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("scan", &scan);
+  m.def("biscan", &biscan);
+  m.def("norm", &norm);
+  m.def("linear_tokens", [](const Tensor& x, const Tensor& w) {
+    py::gil_scoped_release release;
+    return linear_tokens(x, w);
+  });
+  m.def("scan_layer", &scan_layer);
+}

@@ -5,7 +5,8 @@ Same Python surface as the reference's issm_triton/issm_combined.py:
 initial_states=None, seq_idx=None, dt_softplus=False, dt_limit=(0, inf),
 return_final_states=False)`` (issm_combined.py:16-34) backed by
 ``ISSMChunkScanCombinedFn`` (issm_combined.py:37-54) with the same 14 backward slots.
-Host code only marshals pointers; all arithmetic runs in libissm_hip.so.
+Checks, argument blocks, allocation and the autograd nodes are compiled (csrc/host_ops.cpp);
+all arithmetic runs in libissm_hip.so.
 
 ``ISSM_biscan_combined`` additionally runs the bidirectional pair of scans that
 MultiHeadISSMScan issues (models/dest_module.py:565-575) in one call, reading the shared
@@ -15,7 +16,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
-from typing import List, Optional, Sequence, Tuple
+from typing import Optional
 
 import torch
 
@@ -43,7 +44,8 @@ def _kernel_dtype(dt: torch.dtype) -> torch.dtype:
 
 
 class _Problem:
-    """Validated, kernel-ready view of one call (1 or 2 directions)."""
+    """Validated, kernel-ready view of one call (1 or 2 directions) for callers of the C ABI from Python (the stage entry
+    points, preallocated buffers); the operators below do the same in compiled code."""
 
     def __init__(self, xs, dt, A, Bs, Cs, chunk_size, D, zs, dt_bias, h0, seq_idx, dt_softplus, dt_limit):
         x0 = xs[0]
@@ -138,100 +140,22 @@ class _Problem:
         return torch.empty(max(n.value, 256), dtype=torch.uint8, device=self.device)
 
 
-def _scan_fwd(prob: _Problem, want_final: bool):
-    lib = L.load()
-    with torch.cuda.device(prob.device):
-        a = prob.args()
-        outs = [torch.empty((prob.batch, prob.seqlen, prob.nheads, prob.headdim), dtype=prob.io_dtype,
-                            device=prob.device) for _ in range(prob.ndir)]
-        finals = [torch.empty((prob.batch, prob.nheads, prob.headdim, prob.dstate), dtype=torch.float32,
-                              device=prob.device) if want_final else None for _ in range(prob.ndir)]
-        ws = prob.workspace(a, bwd=False)
-        for i in range(prob.ndir):
-            a.out[i] = L.tensor_desc(outs[i])
-            a.final_states[i] = L.ptr(finals[i])
-        a.workspace = ws.data_ptr()
-        a.workspace_bytes = ws.numel()
-        L.check(lib.issm_scan_fwd(C.byref(a)), "issm_scan_fwd")
-    return outs, finals, ws
+def _chunk_size(chunk_size):
+    if not (isinstance(chunk_size, int) and chunk_size > 0):
+        raise ValueError(f"chunk_size must be a positive int, got {chunk_size!r}")
 
 
-def _scan_bwd(prob: _Problem, saved_ws: torch.Tensor, douts, dfinals, want_dz: bool):
-    lib = L.load()
-    dev = prob.device
-    with torch.cuda.device(dev):
-        a = prob.args()
-        a.saved = saved_ws.data_ptr()
-        douts = [_io_cast(t, prob.io_dtype) for t in douts]
-        dfinals = [_f32c(t) for t in dfinals]
-        dxs = [torch.empty_like(o, memory_format=torch.contiguous_format) for o in prob.xs]
-        dBs = [torch.empty(prob.Bs[i].shape, dtype=prob.io_dtype, device=dev) for i in range(prob.ndir)]
-        dCs = [torch.empty(prob.Cs[i].shape, dtype=prob.io_dtype, device=dev) for i in range(prob.ndir)]
-        dzs = [torch.empty(prob.xs[i].shape, dtype=prob.io_dtype, device=dev) if (want_dz and prob.zs[i] is not None)
-               else None for i in range(prob.ndir)]
-        ddt = torch.empty(prob.dt.shape, dtype=prob.dt_dtype, device=dev)
-        dA = torch.empty(prob.A.shape, dtype=torch.float32, device=dev)
-        dD = torch.empty(prob.D.shape, dtype=torch.float32, device=dev) if prob.D is not None else None
-        dbias = torch.empty(prob.dt_bias.shape, dtype=torch.float32, device=dev) if prob.dt_bias is not None else None
-        dh0 = torch.empty((prob.batch, prob.nheads, prob.headdim, prob.dstate), dtype=torch.float32, device=dev)
-        ws = prob.workspace(a, bwd=True)
-        for i in range(prob.ndir):
-            a.dout[i] = L.tensor_desc(douts[i])
-            a.dfinal[i] = L.ptr(dfinals[i])
-            a.dx[i] = L.tensor_desc(dxs[i])
-            a.dB[i] = L.tensor_desc(dBs[i])
-            a.dC[i] = L.tensor_desc(dCs[i])
-            a.dz[i] = L.tensor_desc(dzs[i])
-        a.ddt = L.tensor_desc(ddt)
-        a.dA, a.dD, a.ddt_bias, a.dh0 = L.ptr(dA), L.ptr(dD), L.ptr(dbias), L.ptr(dh0)
-        a.bwd_workspace = ws.data_ptr()
-        a.bwd_workspace_bytes = ws.numel()
-        L.check(lib.issm_scan_bwd(C.byref(a)), "issm_scan_bwd")
-    return dxs, ddt, dA, dBs, dCs, dD, dzs, dbias, dh0
-
-
-def _like(g: Optional[torch.Tensor], dtype: Optional[torch.dtype]) -> Optional[torch.Tensor]:
-    """Gradient in the dtype of the input it belongs to (None if that input was absent)."""
-    if g is None or dtype is None:
-        return None
-    return g if g.dtype == dtype else g.to(dtype)
-
-
-def _dtypes(*ts):
-    return tuple(None if t is None else t.dtype for t in ts)
-
-
-class ISSMChunkScanCombinedFn(torch.autograd.Function):
-    """Autograd contract of issm_combined.py:37-54 (14 inputs, grads for x, dt, A, B, C, D, z,
-    dt_bias, initial_states; None for chunk_size, seq_idx, dt_softplus, dt_limit,
-    return_final_states)."""
+class ISSMChunkScanCombinedFn:
+    """Autograd contract of issm_combined.py:37-54: gradients for x, dt, A, B, C, D, z, dt_bias, initial_states, none for
+    chunk_size, seq_idx, dt_softplus, dt_limit, return_final_states.  The node itself is compiled."""
 
     @staticmethod
-    def forward(ctx, x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initial_states=None, seq_idx=None,
-                dt_softplus=False, dt_limit=(0.0, INF), return_final_states=False):
-        prob = _Problem([x], dt, A, [B], [C], chunk_size, D, [z], dt_bias, initial_states, seq_idx, dt_softplus,
-                        dt_limit)
-        outs, finals, ws = _scan_fwd(prob, return_final_states)
-        # The caller's tensors go through save_for_backward (issm_combined.py:42 does the same): `prob` holds detached
-        # views of the same storage, and reading ctx.saved_tensors in backward is what makes PyTorch raise when one of
-        # them was modified in place between forward and backward instead of returning gradients of changed data.
-        ctx.save_for_backward(x, dt, A, B, C, D, z, dt_bias, initial_states)
-        ctx.prob = prob
-        ctx.ws = ws
-        ctx.return_final_states = return_final_states
-        ctx.refs = _dtypes(x, dt, A, B, C, D, z, dt_bias, initial_states)
-        out = outs[0] if outs[0].dtype == x.dtype else outs[0].to(x.dtype)
-        return out if not return_final_states else (out, finals[0])
-
-    @staticmethod
-    def backward(ctx, dout, *args):
-        ctx.saved_tensors  # version check of the inputs
-        prob = ctx.prob
-        x, dt, A, B, C, D, z, dt_bias, h0 = ctx.refs
-        dfinal = args[0] if ctx.return_final_states else None
-        dxs, ddt, dA, dBs, dCs, dD, dzs, dbias, dh0 = _scan_bwd(prob, ctx.ws, [dout], [dfinal], want_dz=z is not None)
-        return (_like(dxs[0], x), _like(ddt, dt), _like(dA, A), _like(dBs[0], B), _like(dCs[0], C), None,
-                _like(dD, D), _like(dzs[0], z), _like(dbias, dt_bias), _like(dh0, h0), None, None, None, None)
+    def apply(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initial_states=None, seq_idx=None,
+              dt_softplus=False, dt_limit=(0.0, INF), return_final_states=False):
+        _chunk_size(chunk_size)
+        res = L.host().scan(x, dt, A, B, C, D, z, dt_bias, initial_states, seq_idx, bool(dt_softplus), float(dt_limit[0]),
+                            float(dt_limit[1]), bool(return_final_states))
+        return (res[0], res[1]) if return_final_states else res[0]
 
 
 def ISSM_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bias=None, initial_states=None,
@@ -299,46 +223,19 @@ def _merge_heads(s, t, state=False):
     return t.reshape(t.shape[0], t.shape[1], t.shape[2] // s, t.shape[3] * s)
 
 
-class ISSMBiScanFn(torch.autograd.Function):
-    """Both directions of MultiHeadISSMScan's bidirectional scan in one operator call.
-    Inputs are in natural time order; direction "b" is scanned from the last token to the
-    first and its output is returned in natural order (what dest_module.py:568-573 obtains
-    with four flips and a second operator call)."""
-
-    @staticmethod
-    def forward(ctx, x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D, dt_bias, initial_states, dt_softplus,
-                dt_limit):
-        prob = _Problem([x_f, x_b], dt, A, [B_f, B_b], [C_f, C_b], chunk_size, D, [None, None], dt_bias,
-                        initial_states, None, dt_softplus, dt_limit)
-        outs, finals, ws = _scan_fwd(prob, True)
-        ctx.save_for_backward(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, initial_states)  # see ISSMChunkScanCombinedFn
-        ctx.prob = prob
-        ctx.ws = ws
-        ctx.refs = _dtypes(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, initial_states)
-        cast = lambda o, r: o if o.dtype == r.dtype else o.to(r.dtype)
-        return cast(outs[0], x_f), cast(outs[1], x_b), finals[0], finals[1]
-
-    @staticmethod
-    def backward(ctx, dy_f, dy_b, dl_f, dl_b):
-        ctx.saved_tensors  # version check of the inputs
-        prob = ctx.prob
-        x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, h0 = ctx.refs
-        dxs, ddt, dA, dBs, dCs, dD, _, dbias, dh0 = _scan_bwd(prob, ctx.ws, [dy_f, dy_b], [dl_f, dl_b], want_dz=False)
-        return (_like(dxs[0], x_f), _like(dxs[1], x_b), _like(ddt, dt), _like(dA, A), _like(dBs[0], B_f),
-                _like(dBs[1], B_b), _like(dCs[0], C_f), _like(dCs[1], C_b), None, _like(dD, D), _like(dbias, dt_bias),
-                _like(dh0, h0), None, None)
-
-
 def ISSM_biscan_combined(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D=None, dt_bias=None,
                          initial_states=None, dt_softplus=False, dt_limit=(0.0, INF)):
-    """Returns (y_f, y_b, last_f, last_b), all in natural time order; see ISSMBiScanFn."""
+    """Both directions of MultiHeadISSMScan's bidirectional scan in one operator call -> (y_f, y_b, last_f, last_b).
+    Inputs and outputs are in natural time order; direction "b" is scanned from the last token to the first (what
+    dest_module.py:568-573 obtains with four flips and a second operator call)."""
+    _chunk_size(chunk_size)
     s = _head_split(x_f.shape[-1]) if x_f.dim() == 4 else 1
     if s > 1:
         x_b = x_b.reshape(x_b.shape[0], x_b.shape[1], x_b.shape[2] * s, x_b.shape[3] // s)
         x_f, dt, A, D, _, dt_bias, initial_states = _split_heads(s, x_f, dt, A, D, None, dt_bias, initial_states)
-    res = ISSMBiScanFn.apply(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D, dt_bias, initial_states,
-                             dt_softplus, dt_limit)
+    res = L.host().biscan(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, initial_states, bool(dt_softplus),
+                          float(dt_limit[0]), float(dt_limit[1]))
     if s == 1:
-        return res
+        return tuple(res)
     return (_merge_heads(s, res[0]), _merge_heads(s, res[1]), _merge_heads(s, res[2], state=True),
             _merge_heads(s, res[3], state=True))
