@@ -231,7 +231,7 @@ static KP make_kp(const issm_scan_args* a) {
     p.seq_idx = a->seq_idx; p.seq_s0 = a->seq_idx_stride[0]; p.seq_s1 = a->seq_idx_stride[1];
   }
   p.c_lo = 0; p.ncl = p.nc;
-  if (p.N % 64 == 0 && !p.seq_idx) p.full_tiles = p.L % ISSM_CHUNK == 0 ? 1 : (p.nc > 1 ? 2 : 0);
+  p.full_tiles = p.N % 64 == 0 && p.L % ISSM_CHUNK == 0 && !p.seq_idx;
   return p;
 }
 
@@ -435,11 +435,15 @@ int issm_scan_bwd(const issm_scan_args* a) {
                        "bwd_chunk")))
       return rc;
   }
-  if (pending &&
-      (rc = launched(launch_bwd_chunk_redo(p, p.ndir, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last,
-                                           ws + bw.partA, ws + bw.partBias, redo, st),
-                     "bwd_chunk (redo)")))
-    return rc;
+  const int together = p.L % ISSM_CHUNK == 0 ? p.ndir : 1;   // directions per launch of the pass over the marks
+  for (int dir = 0; pending && dir < p.ndir; dir += together) {
+    KP pd = p;
+    pd.dir0 = dir;
+    if ((rc = launched(launch_bwd_chunk_redo(pd, together, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last,
+                                             ws + bw.partA, ws + bw.partBias, redo, st),
+                       "bwd_chunk (redo)")))
+      return rc;
+  }
   if ((rc = launched(launch_bwd_dx(p, dy, ws + bw.dstates, sv + fw.cabt, ws + bw.partD, st), "bwd_dx"))) return rc;
   return launched(launch_bwd_reduce(p, ws + bw.partA, ws + bw.partBias, ws + bw.partD, ws + bw.dh0_dir, a->dA,
                                     a->dt_bias ? a->ddt_bias : nullptr, a->D ? a->dD : nullptr, a->dh0, st),

@@ -171,28 +171,25 @@ __device__ __forceinline__ void k_bwd_dstates_body(const KP& p, const float* __r
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) acc[pt] = (f4){0, 0, 0, 0};
     rows_product_split<PT, LDT, IOB ? 0 : 1>(acc, s.dyt_hi, s.dyt_lo, [&](int k) { return ct[k]; }, cm, g4);
-    float* dst = dstates + dst_off(p, u.bt, u.c, u.h);
+    float* dst = dstates + dst_off(p, u.bt, u.c, u.h) + (4 * g4) * p.N + n_cur;
+    if (p.P == PT * 16 && (FULL || n0 + NS <= p.N)) {  // uniform: nothing to mask
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt)
+      for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int pp = pt * 16 + 4 * g4 + r;
-        if (pp < p.P && vn_cur) dst[(long)pp * p.N + n_cur] = acc[pt][r];
-      }
+        for (int r = 0; r < 4; ++r) dst[(pt * 16 + r) * p.N] = acc[pt][r];
+    } else {
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (pt * 16 + 4 * g4 + r < p.P && vn_cur) dst[(pt * 16 + r) * p.N] = acc[pt][r];
+    }
   }
 }
 template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS) void k_bwd_dstates(KP p, const float* __restrict__ dy_ws, float* __restrict__ dstates, float* __restrict__ dm) {
+__global__ __launch_bounds__(NTHREADS, (PT <= 3 && !FULL) ? 4 : 1) void k_bwd_dstates(KP p, const float* __restrict__ dy_ws, float* __restrict__ dstates, float* __restrict__ dm) {
   k_bwd_dstates_body<PT, IOB, DTB, FULL>(p, dy_ws, dstates, dm);
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool IOB, bool DTB>
-__global__ __launch_bounds__(NTHREADS) void k_bwd_dstates_mixed(KP p, const float* __restrict__ dy_ws, float* __restrict__ dstates, float* __restrict__ dm) {
-  if (decode_unit(p, xcd_remap(blockIdx.x, gridDim.x)).c == p.nc - 1) k_bwd_dstates_body<PT, IOB, DTB, false>(p, dy_ws, dstates, dm);
-  else k_bwd_dstates_body<PT, IOB, DTB, true>(p, dy_ws, dstates, dm);
-}
-
 
 // ------------------------------------------------------- reverse state passing
 // Block = (bt, h, 64 state columns); thread (pg = tid >> 4, nq = tid & 15) carries rows
@@ -313,15 +310,21 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd(KP p, const float* __res
   }
 }
 
-// The same recurrence for N a multiple of the slice width, with no conditional access anywhere: every load of the
-// loop is issued on every path, so the compiler can count the loads still in flight and the prefetched operands of
+// The same recurrence with no conditional access in its loop: every load is issued on every path, so the compiler can
+// count the loads still in flight and the prefetched operands of
 // the next chunks stay in flight across the barrier (with loads inside branches it waits for all of them before each
 // store, which exposes the full memory latency once per chunk; few workgroups walking many chunks -- batch 2, 256
 // chunks -- then run at that pace).  A thread owns KM rows, pg + PGN k; for rows past the head dimension it stands in
 // for the head's last row: it issues the same loads (so that every load of the loop is unconditional) but stores
 // nothing and adds nothing to the column sums -- what a stand-in computes is never used, so it does not matter that
 // the row's owner overwrites dH with dS while the stand-in's prefetches of that row are in flight.
-template <int NQ, int KM, int R, bool BATCH>
+// TAIL (N >= 4, not a multiple of the slice width; accesses at any float): a column quad that crosses or lies past N is
+// columns N - 4 .. N - 1 instead, once more.  The threads that own a column twice sit in one wave (the quads of a row are
+// adjacent lanes), issue their loads and stores of it in the same instructions and compute the same values, so storing
+// twice is harmless; a column's sum is formed per quad, and stored twice as well.  Columns such a quad shares with the
+// previous slice are that workgroup's alone to store.  8 x 1024 tokens, 8 heads, N = 250:
+// 53.4 us with per-element guards, N = 256 without: 17.6.
+template <int NQ, int KM, int R, bool BATCH, bool TAIL>
 __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* __restrict__ states,
                                                              const float* __restrict__ cs_last,
                                                              float* __restrict__ dstates, float* __restrict__ g_last,
@@ -341,7 +344,7 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
   static_assert(R % K == 0 && K * NCOL <= NTHREADS && (NQ == 8 || NQ == 16), "batches of K steps tile the ring");
   __shared__ __align__(16) float red2[2][BATCH ? K * NCOL * 16 : PGN * NCOL];
   int par = 0;
-  const int nsl = p.N / NCOL;
+  const int nsl = (p.N + NCOL - 1) / NCOL;
   int bid = blockIdx.x;
   const int ns = bid % nsl;
   bid /= nsl;
@@ -349,7 +352,25 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
   const int bt = bid / p.H;
   const int b = bt / p.ndir, dir = bt % p.ndir;
   const int tid = threadIdx.x, pg = tid / NQ, nq = tid % NQ;
-  const int n = ns * NCOL + nq * 4;
+  const int n = TAIL ? min(ns * NCOL + nq * 4, p.N - 4) : ns * NCOL + nq * 4;
+  // column `col` of the workgroup's slice (quad col / 4, entry col % 4), relative to the slice's first
+  auto col_at = [&](int col) { return TAIL ? min(col & ~3, p.N - 4 - ns * NCOL) + (col & 3) : col; };
+  auto ld = [](const float* a) -> f4 {
+    if constexpr (TAIL) return ld_f4_any(a);
+    else return *(const f4*)a;
+  };
+  const int foreign = TAIL ? max(ns * NCOL - n, 0) : 0;   // first columns of the quad that are another workgroup's
+  auto put = [&](float* a, f4 v) {
+    if constexpr (!TAIL) {
+      *(f4*)a = v;
+    } else if (foreign == 0) {
+      st_f4_any(a, v);
+    } else {
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (j >= foreign) a[j] = v[j];
+    }
+  };
   const int part = (tid >> 6) * 4 + ((tid & 63) >> 4);  // (wave, 16-lane row): which of a column's 16 partial sums
   const bool deposits = NQ == 16 || !(tid & 8);
   long rowk[KM];   // offsets of the thread's rows
@@ -364,7 +385,7 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
 #pragma unroll
   for (int k = 0; k < KM; ++k) {
     carry[k] = (f4){0, 0, 0, 0};
-    if (p.dfinal[dir]) carry[k] = *(const f4*)(p.dfinal[dir] + ((long)b * p.H + h) * p.P * p.N + rowk[k]);
+    if (p.dfinal[dir]) carry[k] = ld(p.dfinal[dir] + ((long)b * p.H + h) * p.P * p.N + rowk[k]);
   }
   const float* hp = states + st_off(p, bt, p.nc, h);      // H_{c+1}, c = nc - 1
   float* dd = dstates + dst_off(p, bt, p.nc - 1, h);      // dH_c in, dS_c out
@@ -376,11 +397,11 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
   f4 dec[R], hn[R][KM], dh[R][KM];
   auto request = [&](int slot, int back_chunks) {
     const long back = (long)back_chunks * cstep;
-    dec[slot] = *(const f4*)(cl - (long)back_chunks * vstep);
+    dec[slot] = ld(cl - (long)back_chunks * vstep);
 #pragma unroll
     for (int k = 0; k < KM; ++k) {
-      hn[slot][k] = *(const f4*)(hp - back + rowk[k]);
-      dh[slot][k] = *(const f4*)(dd - back + rowk[k]);
+      hn[slot][k] = ld(hp - back + rowk[k]);
+      dh[slot][k] = ld(dd - back + rowk[k]);
     }
   };
 #pragma unroll
@@ -392,7 +413,7 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
     for (int j = 0; j < 4; ++j) e[j] = __expf(dec[cur][j]);
 #pragma unroll
     for (int k = 0; k < KM; ++k) {
-      if (own[k]) *(f4*)(dd + rowk[k]) = carry[k];
+      if (own[k]) put(dd + rowk[k], carry[k]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         gp[j] += own[k] ? hn[cur][k][j] * carry[k][j] : 0.0f;
@@ -436,13 +457,14 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
         for (int k = 0; k < PGN / PARTS; ++k) sum += red[(k * PARTS + prt) * NCOL + col];
 #pragma unroll
         for (int d = NCOL; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
-        if (prt == 0) gl[col] = sum;
+        if (prt == 0 && (!TAIL || col_at(col) >= 0)) gl[col_at(col)] = sum;
       }
     } else if (tid < cnt * NCOL) {
       const f4* r = (const f4*)(red2[par] + tid * 16);
       const f4 a = r[0], b4 = r[1], c4 = r[2], d4 = r[3];
       const f4 s4 = (a + b4) + (c4 + d4);
-      gl[-(long)(tid / NCOL) * vstep + tid % NCOL] = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+      if (!TAIL || col_at(tid % NCOL) >= 0)
+        gl[-(long)(tid / NCOL) * vstep + col_at(tid % NCOL)] = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     }
     gl -= (long)cnt * vstep;
     par ^= 1;
@@ -465,7 +487,7 @@ __global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* 
   }
 #pragma unroll
   for (int k = 0; k < KM; ++k)
-    if (own[k]) *(f4*)(dh0_dir + (((long)dir * p.B + b) * p.H + h) * p.P * p.N + rowk[k]) = carry[k];
+    if (own[k]) put(dh0_dir + (((long)dir * p.B + b) * p.H + h) * p.P * p.N + rowk[k], carry[k]);
 }
 
 // -------------------------------------------------------------- chunk backward
@@ -657,9 +679,9 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
   Unit u;
   // `redo` (one word per direction, workgroup and head, written by the tile-base kernel): only the marked heads are
   // evaluated here, and their ddt / dB / dC are added to what that kernel left (zero, or the other direction's share).
-  // `mirror`: the workgroup's chunk index counts from the other end -- the chunk of this direction that covers the
-  // same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions' shares to
-  // those tokens' ddt one after the other, and no two workgroups ever update one address).
+  // `mirror` (complete chunks only): the workgroup's chunk index counts from the other end -- the chunk of this direction
+  // that covers the same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions'
+  // shares to those tokens' ddt one after the other, and no two workgroups ever update one address).
   int id = xcd_remap(blockIdx.x, gridDim.x);
   const int ns = id % nsl;
   id /= nsl;
@@ -682,10 +704,7 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
   const int n = ns * NS + wave * 16 + cm;
   const bool vn = FULL || n < p.N;
 
-  // rows past the end of the sequence and absent columns: lane_row(k) >= lim
   const RowMap rm = make_rowmap<FULL>(p, u, g4, ns * NS);
-  const int lim = vn ? rm.nvalid - 4 * g4 : 0;
-  auto rowk = [&](int k) { return 16 * (k >> 2) + (k & 3); };
   const bool pn_full = FULL && p.P == PT * 16;
 
   float Bv[16], Cv[16];
@@ -704,7 +723,7 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
     float raw[16], dsv[KP_], hv[KP_];
     lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
     const Coef cf = lane_coef(p, u.h, n, vn);
-    const float gl = (g4 == 3 && vn) ? g_last[vec_off(p, u.bt, u.c, u.h) + n] : 0.0f;
+    const float gl_any = g_last[vec_off(p, u.bt, u.c, u.h) + (vn ? n : 0)], gl = g4 == 3 ? gl_any : 0.0f;
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, dsv);
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, hv);
     f4 mkeep[SM::DM_OVER_X ? 4 : 1];  // the thread's part of the dM tile until the x tile's place is free
@@ -890,7 +909,7 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
       const float da = dcs[k];
       sumA += da * dtp[k];
       val[k] = (val[k] + da * An) * dfac[k];
-      if (rm.full || rowk(k) < lim) sumB += val[k];
+      sumB += val[k];  // (absent rows: the derivative of dt' is 0)
       if (redo || dir_here > 0) val[k] += old[k];
     }
     if (p.ddt.ptr) lane_store_ln<DTB>(p.ddt, u.b, u.h, n, vn, g4, rm, val);
@@ -931,14 +950,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk(KP p, const float* __
     k_bwd_chunk_body<PT, IOB, DTB, FULL>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, p.dir0 + d, d > 0);
   }
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool IOB, bool DTB>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_mixed(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias) {
-  if (p.c_lo + (xcd_remap(blockIdx.x, gridDim.x) / ((p.N + NS - 1) / NS) / p.G) % p.ncl == p.nc - 1) k_bwd_chunk_body<PT, IOB, DTB, false>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, nullptr, p.dir0, false);
-  else k_bwd_chunk_body<PT, IOB, DTB, true>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, nullptr, p.dir0, false);
-}
-
 
 // ------------------------------------------------- chunk backward, bf16 inputs
 // The same computation for bf16 x / B / C / dy: every matrix product runs on v_mfma_f32_16x16x32_bf16 with operands
@@ -1146,9 +1157,9 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   Unit u;
   // `redo` (one word per direction, workgroup and head, written by the tile-base kernel): only the marked heads are
   // evaluated here, and their ddt / dB / dC are added to what that kernel left (zero, or the other direction's share).
-  // `mirror`: the workgroup's chunk index counts from the other end -- the chunk of this direction that covers the
-  // same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions' shares to
-  // those tokens' ddt one after the other, and no two workgroups ever update one address).
+  // `mirror` (complete chunks only): the workgroup's chunk index counts from the other end -- the chunk of this direction
+  // that covers the same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions'
+  // shares to those tokens' ddt one after the other, and no two workgroups ever update one address).
   int id = xcd_remap(blockIdx.x, gridDim.x);
   const int ns = id % nsl;
   id /= nsl;
@@ -1171,8 +1182,6 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   const int n = ns * NS + wave * 16 + cm;
   const bool vn = FULL || n < p.N;
   const RowMap rm = make_rowmap<FULL>(p, u, g4, ns * NS);
-  const int lim = vn ? rm.nvalid - 4 * g4 : 0;
-  auto rowk = [&](int k) { return 16 * (k >> 2) + (k & 3); };
   const bool pn_full = FULL && p.P == PT * 16;
 
   float Bv[16], Cv[16];
@@ -1219,7 +1228,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
     float raw[16], dsv[KP_], hv[KP_];
     lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
     const Coef cf = lane_coef(p, u.h, n, vn);
-    const float gl = (g4 == 3 && vn) ? g_last[vec_off(p, u.bt, u.c, u.h) + n] : 0.0f;
+    const float gl_any = g_last[vec_off(p, u.bt, u.c, u.h) + (vn ? n : 0)], gl = g4 == 3 ? gl_any : 0.0f;
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, dsv);
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, hv);
     request(u.h);
@@ -1358,7 +1367,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
       const float da = dcs[k];
       sumA += da * dtp[k];
       val[k] = (val[k] + da * An) * dfac[k];
-      if (rm.full || rowk(k) < lim) sumB += val[k];
+      sumB += val[k];  // (absent rows: the derivative of dt' is 0)
     }
     if ((redo || dir_here > 0) && p.ddt.ptr) {
 #pragma unroll
@@ -1401,14 +1410,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf(KP p, const float*
     k_bwd_chunk_bf_body<PT, DTB, FULL>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, p.dir0 + d, d > 0);
   }
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool DTB>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf_mixed(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias) {
-  if (p.c_lo + (xcd_remap(blockIdx.x, gridDim.x) / ((p.N + NS - 1) / NS) / p.G) % p.ncl == p.nc - 1) k_bwd_chunk_bf_body<PT, DTB, false>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, nullptr, p.dir0, false);
-  else k_bwd_chunk_bf_body<PT, DTB, true>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, nullptr, p.dir0, false);
-}
-
 
 // ------------------------------------------------------------------------- dx
 // BF (bf16 inputs): the operands of the product over the state index are bf16 tiles read as matrix fragments of 8
@@ -1487,7 +1488,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, bv);
-  pn_load<PT>(p, ds, 0, sv);
+  pn_load<PT, FULL>(p, ds, 0, sv);
   // M^T of this wave's 16 columns goes straight into matrix-operand registers (lane (column cm, group g4) holds
   // rows 16 kb + 4 g4 .. + 3 of the blocks kb >= wave, the upper triangle of the diagonal block zeroed): no LDS tile,
   // which lets a fourth workgroup live on the CU
@@ -1545,6 +1546,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
           s.bt[lane_row(k, g4) * LDN + wave * 16 + cm] = bv[k] * dtp[k] * ex2(last - cs[k]);
       }
     }
+    if constexpr (!FULL) pn_edge<PT>(p, n0, sv);
     if constexpr (IOB) pn_store_bf16<PT, LDK>(sv, s.dss);
     else if constexpr (SM::SPL) pn_store_hl<PT, LDK>(sv, s.dss, s.dss + PT * 16 * LDK);
     else pn_store<PT>(sv, s.dss);
@@ -1555,7 +1557,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
       lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
       cf = lane_coef(p, u.h, n, vn);
       lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, bv);
-      pn_load<PT>(p, ds, n0 + NS, sv);
+      pn_load<PT, FULL>(p, ds, n0 + NS, sv);
     }
     __syncthreads();
     if constexpr (IOB) {
@@ -1639,17 +1641,9 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   }
 }
 template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, (PT <= 2 && FULL) ? 4 : 1) void k_bwd_dx(KP p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
+__global__ __launch_bounds__(NTHREADS, PT <= 2 ? 4 : 1) void k_bwd_dx(KP p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
   k_bwd_dx_body<PT, IOB, DTB, FULL>(p, dy_ws, dstates, cabt, partD);
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool IOB, bool DTB>
-__global__ __launch_bounds__(NTHREADS, (PT <= 2 && false) ? 4 : 1) void k_bwd_dx_mixed(KP p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
-  if (decode_unit(p, xcd_remap(blockIdx.x, gridDim.x)).c == p.nc - 1) k_bwd_dx_body<PT, IOB, DTB, false>(p, dy_ws, dstates, cabt, partD);
-  else k_bwd_dx_body<PT, IOB, DTB, true>(p, dy_ws, dstates, cabt, partD);
-}
-
 
 // ------------------------------------------------------------------- reductions
 // All final reductions run as ONE launch (they are independent of each other and tiny, so separate
@@ -1771,7 +1765,7 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     const size_t sm = sizeof(BwdStSmem<PT_, IOB_>);
-    constexpr auto kern = MIXED_ ? &k_bwd_dstates_mixed<PT_, IOB_, DTB_> : &k_bwd_dstates<PT_, IOB_, DTB_, FULL_>;
+    constexpr auto kern = &k_bwd_dstates<PT_, IOB_, DTB_, FULL_>;
     if (int e = set_lds(kern, sm)) return e;
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, dy_ws, dstates, dm);
   });
@@ -1783,46 +1777,41 @@ int launch_state_bwd(const KP& p, const float* states, const float* cs_last, flo
   // One workgroup walks the chunks of its columns one after the other.  Complete shapes take the variant without
   // conditional accesses; with few (batch, head) pairs narrower column slices put more workgroups on the chip.
   const int wide = p.B * p.ndir * p.H * ((p.N + 63) / 64);
-#define ISSM_STATE_BWD_FULL(NQ_, KM_, R_, BATCH_)                                                                          \
-  hipLaunchKernelGGL((k_state_bwd_full<NQ_, KM_, R_, BATCH_>), dim3(p.B * p.ndir * p.H * (p.N / (4 * NQ_))), dim3(NTHREADS), \
-                     0, st, p, states, cs_last, dstates, g_last, dh0_dir)
-  if (p.N % 32 == 0 && (wide < 256 || p.N % 64 != 0)) {
+  // (sequence of the tests: slices of 32 columns where 64 would leave the chip idle or N fits them exactly)
+#define ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, TAIL_)                                                                         \
+  hipLaunchKernelGGL((k_state_bwd_full<NQ_, KM_, R_, BATCH_, TAIL_>), dim3(p.B * p.ndir * p.H * ((p.N + 4 * NQ_ - 1) / (4 * NQ_))), \
+                     dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir)
+#define ISSM_STATE_BWD_FULL(NQ_, KM_, R_, BATCH_)                                                   \
+  do {                                                                                              \
+    if (p.N % (4 * NQ_)) ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, true);                              \
+    else ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, false);                                             \
+  } while (0)
+  if (p.N < 4) {
+    const int blocks = p.B * p.ndir * p.H * ((p.N + 15) / 16);
+    hipLaunchKernelGGL(k_state_bwd<4>, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir);
+  } else if (wide < 256 || (p.N % 64 != 0 && (p.N + 63) / 64 * 2 != (p.N + 31) / 32)) {
     // few workgroups walking many chunks: the column sums of several steps behind one barrier
-    const bool batch = p.B * p.ndir * p.H * (p.N / 32) <= 128 && p.nc >= 32;
+    const bool batch = p.B * p.ndir * p.H * ((p.N + 31) / 32) <= 128 && p.nc >= 32;
     if (p.P <= 32) { if (batch) ISSM_STATE_BWD_FULL(8, 1, 6, true); else ISSM_STATE_BWD_FULL(8, 1, 6, false); }
     else { if (batch) ISSM_STATE_BWD_FULL(8, 2, 4, true); else ISSM_STATE_BWD_FULL(8, 2, 4, false); }
-  } else if (p.N % 64 == 0) {
+  } else {
     switch ((p.P + 15) / 16) {
       case 1: ISSM_STATE_BWD_FULL(16, 1, 3, false); break;
       case 2: ISSM_STATE_BWD_FULL(16, 2, 3, false); break;
       case 3: ISSM_STATE_BWD_FULL(16, 3, 3, false); break;
       default: ISSM_STATE_BWD_FULL(16, 4, 3, false); break;
     }
-  } else if (wide < 256) {
-    const int blocks = p.B * p.ndir * p.H * ((p.N + 15) / 16);
-    hipLaunchKernelGGL(k_state_bwd<4>, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir);
-  } else {
-    hipLaunchKernelGGL(k_state_bwd<16>, dim3(wide), dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir);
   }
+#undef ISSM_STATE_BWD_T
 #undef ISSM_STATE_BWD_FULL
   return (int)hipGetLastError();
 }
 
-template <int PT, bool IOB, bool DTB, bool FULL, bool MIXED>
+template <int PT, bool IOB, bool DTB, bool FULL>
 static int launch_bwd_chunk_t(const KP& p, int blocks, const float* dy_ws, const float* states, const float* dstates,
                               const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
                               int ndirs, hipStream_t st) {
-  if constexpr (MIXED) {  // (never with `redo`: the tile-base kernel takes complete tiles only)
-    if constexpr (IOB) {
-      const size_t sm = sizeof(BwdChunkBfSmem<PT>);
-      if (int e = set_lds(&k_bwd_chunk_bf_mixed<PT, DTB>, sm)) return e;
-      hipLaunchKernelGGL((k_bwd_chunk_bf_mixed<PT, DTB>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, g_last, partA, partBias);
-    } else {
-      const size_t sm = sizeof(BwdChunkSmem<PT>);
-      if (int e = set_lds(&k_bwd_chunk_mixed<PT, false, DTB>, sm)) return e;
-      hipLaunchKernelGGL((k_bwd_chunk_mixed<PT, false, DTB>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, g_last, partA, partBias);
-    }
-  } else if constexpr (IOB) {  // bf16 inputs: every product on the bf16 matrix instructions
+  if constexpr (IOB) {  // bf16 inputs: every product on the bf16 matrix instructions
     const size_t sm = sizeof(BwdChunkBfSmem<PT>);
     if (int e = set_lds(&k_bwd_chunk_bf<PT, DTB, FULL>, sm)) return e;
     hipLaunchKernelGGL((k_bwd_chunk_bf<PT, DTB, FULL>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, ndirs);
@@ -1835,22 +1824,22 @@ static int launch_bwd_chunk_t(const KP& p, int blocks, const float* dy_ws, const
 }
 
 bool bwd_tile_available(const KP& p, const float* dy_ws);
-int launch_bwd_tile(const KP& p, const float* states, const float* dstates, const float* dm, const float* g_last,
+int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm, const float* g_last,
                     float* partA, float* partBias, int* redo, hipStream_t st);
 
 // Chunk backward of direction p.dir0.  With a `redo` buffer (issm_bwd_chunk_redo_ints words) the tile-base kernel
 // (issm_bwd_tile.hip) does the work and marks the heads outside its range; launch_bwd_chunk_redo then evaluates those
-// with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (ragged tiles, packed
-// sequences, a gate, mixed input types), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
+// with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (packed
+// sequences, a gate beside bf16 inputs, mixed input types), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
                      const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   if (redo && bwd_tile_available(p, dy_ws)) {
     if (redo_pending) *redo_pending = 1;
-    return launch_bwd_tile(p, states, dstates, dm, g_last, partA, partBias, redo, st);
+    return launch_bwd_tile(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, st);
   }
   ISSM_DISPATCH(p, {
-    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_, MIXED_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
+    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
                                                                   partBias, nullptr, 1, st))
       return e;
   });
@@ -1858,13 +1847,14 @@ int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const
 }
 
 // The level-hierarchy kernel over the heads the tile-base launches of directions p.dir0 .. p.dir0 + ndirs - 1 marked in
-// `redo` (ordinary inputs mark none, and its workgroups return at once).
+// `redo` (ordinary inputs mark none, and its workgroups return at once).  Where the sequence length is not a multiple of
+// the chunk the two directions' chunks do not cover the same tokens: the caller then launches direction by direction.
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
                           const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
                           hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   ISSM_DISPATCH(p, {
-    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_, MIXED_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
+    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
                                                                   partBias, redo, ndirs, st))
       return e;
   });
@@ -1876,7 +1866,7 @@ int launch_bwd_dx(const KP& p, const float* dy_ws, const float* dstates, const f
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     const size_t sm = sizeof(BwdDxSmem<PT_, IOB_>);
-    constexpr auto kern = MIXED_ ? &k_bwd_dx_mixed<PT_, IOB_, DTB_> : &k_bwd_dx<PT_, IOB_, DTB_, FULL_>;
+    constexpr auto kern = &k_bwd_dx<PT_, IOB_, DTB_, FULL_>;
     if (int e = set_lds(kern, sm)) return e;
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, dy_ws, dstates, cabt, partD);
   });

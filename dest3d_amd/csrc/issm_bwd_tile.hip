@@ -16,16 +16,23 @@
 // (|tt| <= 96: operands below 2^96, no overflow before the factors meet).  A head of a workgroup where some column
 // exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
 // (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands: bf16 inputs -> one bf16 instruction
-// per block, operands rounded once; fp32 inputs -> operands cut to 16 significand bits and split exactly into (hi, lo)
-// bf16 pairs, a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  d/d(cs) is formed as
-// (operand as the matrix instruction took it) x (product) on both rows of a pair, so the two entries of a pair cancel
-// to fp32 rounding in the suffix sums.
+// per block, operands rounded once; in launches with incomplete tiles the diagonal blocks take operands as (hi, lo) pairs
+// instead (the level form, which evaluated those launches before, keeps close pairs of rows in fp32: this one is not to be
+// less accurate; pairs for every block spill 300 bytes a lane and take twice the time).  fp32
+// inputs -> operands rounded to 17 significand bits and split exactly into (hi, lo) bf16 pairs, a.b = (ah.bl + al.bh) +
+// (ah.bh + al.bl), each bracket one K = 32 instruction.  d/d(cs) is formed as (operand as the matrix instruction took it) x
+// (product) on both rows of a pair, so the two entries of a pair cancel to fp32 rounding in the suffix sums.
 //
-// Built for complete tiles only (sequence length and state dimension multiples of 64, no packed sequences, x / dout
-// rows that allow 8- / 16-byte accesses, no z gate, x / B / C and dt of one type); every other call takes the
-// level-hierarchy kernel alone.  That is what lets the kernel issue every global load of a head without a branch, one
-// head ahead: the wave then knows how many requests are outstanding at every point and waits for exactly the ones it
-// needs (a load inside a branch, even a uniform one, makes the compiler wait for all outstanding loads at the join).
+// Built for x / dout rows that allow 8- / 16-byte accesses, x / B / C and dt of one type, no packed sequences, and for bf16
+// inputs no z gate; every other call takes the level-hierarchy kernel alone.  That is what lets the kernel issue every
+// global load of a head without a branch, one head ahead: the wave then knows how many requests are outstanding at every
+// point and waits for exactly the ones it needs (a load inside a branch, even a uniform one, makes the compiler wait for
+// all outstanding loads at the join).  Incomplete tiles (FULL = false) run the same code: rows past the end are read through
+// a buffer whose bounds check returns zero, columns past the end read column 0 and have dt' = 0, stores are guarded in the
+// workgroups that have such rows or columns. 8 x 1024 tokens, 8 heads
+// x 32, one direction, N = 250: 108 us fp32, 87 us bf16 (N = 256: 88 and 59 us; the difference is registers, 90 - 130 bytes a
+// lane spill in the incomplete form).  With the other kernels' edge forms the whole forward + backward went from 462 to
+// 347 us (fp32) and from 406 to 277 us (bf16).
 #include "issm_dev.h"
 
 namespace issm {
@@ -55,13 +62,15 @@ __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflev
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
-template <int PT, bool IOB, bool PNF, bool ACC, bool P32>
+// FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).
+template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL>
 __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
                                                           const float* __restrict__ dstates,
                                                           const float* __restrict__ dm,
                                                           const float* __restrict__ g_last, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo) {
   constexpr bool SPLIT = !IOB;
+  constexpr bool DIAG2 = IOB && !FULL;  // operands of the diagonal blocks as (hi, lo) pairs
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdTileSmem<PT, SPLIT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
@@ -70,7 +79,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   constexpr int KP_ = PT * 4;  // dS / H values per lane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
-  const int nsl = p.N / NS;
+  const int nsl = (p.N + NS - 1) / NS;
   Unit u;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   int id = wg;
@@ -84,15 +93,17 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   u.bt = u.b * p.ndir + u.dir;
   u.h = u.g * p.hpg;
   const int n = ns * NS + wave * 16 + cm;
-  const RowMap rm = make_rowmap<true>(p, u, g4, ns * NS);
+  const bool vn = FULL || n < p.N;
+  const int nc_ = FULL ? n : (vn ? n : 0);   // where an absent column reads its per-column values
+  const RowMap rm = make_rowmap<FULL>(p, u, g4, ns * NS);
 
 #pragma unroll
   for (int k = 0; k < 16; ++k) s.dbc[k * NTHREADS + tid] = s.dbc[(16 + k) * NTHREADS + tid] = 0.0f;
 
   if constexpr (BCL) {
     float tb[16], tc[16];
-    lane_load_ln<true>(p.Bm[u.dir], u.b, u.g, n, true, g4, rm, tb);
-    lane_load_ln<true>(p.Cm[u.dir], u.b, u.g, n, true, g4, rm, tc);
+    lane_load_ln<true>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, tb);
+    lane_load_ln<true>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, tc);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       s.bc[i * NTHREADS + tid] = pack_bf16(tb[2 * i], tb[2 * i + 1]);  // exact: the values are bf16 numbers
@@ -139,7 +150,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
       for (int i = 0; i < PT; ++i) {
         const int e4 = tq + i * NTHREADS, l = e4 / G4, p4 = (e4 % G4) * 4;
-        const bool ok = p4 < p.P;
+        const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
         const long ox = ok ? (t0 + sgn * l) * tx.s1 + p4 : 0, oy = ok ? (t0 + sgn * l) * ty.s1 + p4 : 0;
         if constexpr (SPLIT) {
           const f4 a = *(const f4*)(qy + oy), b = *(const f4*)(qx + ox);
@@ -152,19 +163,19 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       }
     }
-    lane_load_ln<IOB>(p.dt, u.b, hnext, n, true, g4, rm, l_raw);
-    l_A = p.A[hnext * p.N + n];
+    lane_load_ln<IOB>(p.dt, u.b, hnext, n, vn, g4, rm, l_raw);
+    l_A = p.A[hnext * p.N + nc_];
     {
       const float* bp = p.dt_bias ? p.dt_bias : p.A;  // no bias: any readable address, the value is dropped
-      const float b = bp[hnext * p.N + n];
+      const float b = bp[hnext * p.N + nc_];
       l_bias = p.dt_bias ? b : 0.0f;
     }
-    l_gl = g_last[vec_off(p, u.bt, u.c, hnext) + n];  // (every lane of the column; the last lane group uses it)
-    lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, hnext), p.P, p.N, n, true, g4, PNF, l_dsv);
-    lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, true, g4, PNF, l_hv);
+    l_gl = g_last[vec_off(p, u.bt, u.c, hnext) + nc_];  // (every lane of the column; the last lane group uses it)
+    lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_dsv);
+    lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
     if constexpr (!BCL) {
-      lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, true, g4, rm, l_Bv);
-      lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, true, g4, rm, l_Cv);
+      lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, l_Bv);
+      lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, l_Cv);
     }
   };
   request(head_of(0));
@@ -208,7 +219,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     cf.bias = l_bias;
     const float An = cf.A;
     float dtp[16], dfac[16], pc[16], tt[4];
-    lane_dt<true>(p, cf, true, g4, rm, l_raw, dtp, dfac);
+    lane_dt<true>(p, cf, vn, g4, rm, l_raw, dtp, dfac);
     lane_tile_sums(An * LOG2E, cm, g4, rm, dtp, pc, tt);
     {
       const float worst = fmaxf(fmaxf(fabsf(tt[0]), fabsf(tt[1])), fmaxf(fabsf(tt[2]), fabsf(tt[3])));
@@ -266,13 +277,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
             bi = half_of(s.bc[(k >> 1) * NTHREADS + tid], k) * dtp[k] * iup[k];
           }
           if (SPLIT) {
-            cu = trunc16(cu);
-            bi = trunc16(bi);
+            cu = round17(cu);
+            bi = round17(bi);
           }
           Ch[J][j] = (__bf16)cu;
           Bh[J][j] = (__bf16)bi;
           if (SPLIT) {
-            Cl[J][j] = (__bf16)(cu - (float)Ch[J][j]);  // exact: 16 bits = 8 + 8
+            Cl[J][j] = (__bf16)(cu - (float)Ch[J][j]);  // exact: 17 bits = 8 + 8 and the sign
             Bl[J][j] = (__bf16)(bi - (float)Bh[J][j]);
           }
         }
@@ -280,7 +291,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       // to a register
       unsigned bvp[8], cvp[8];
       float bvf[SPLIT ? 16 : 1];
-      if constexpr (BCL) {
+      if constexpr (BCL && DIAG2) {  // read tile by tile below
+      } else if constexpr (BCL) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           bvp[i] = s.bc[i * NTHREADS + tid];
@@ -328,7 +340,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         const bf4 a_h = __builtin_bit_cast(bf4, ah);
         if constexpr (SPLIT) {
           // (ah + al) . (bh + bl) in full: the same A fragment against (bl | bh) and (bh | bl).  All four terms, so
-          // that F and G see one and the same product dM16 . B16 . C16 for a pair of rows
+          // that F and G see one and the same product dM . B . C (as the instructions took them) for a pair of rows
           const bf8 a2 = cat_bf4(a_h, __builtin_bit_cast(bf4, al));
           acc = mfma_bf(a2, cat_bf4(bl, bh), acc);
           return mfma_bf(a2, cat_bf4(bh, bl), acc);
@@ -337,12 +349,34 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       };
 
+      auto block_pair = [&](uint2 ah, bf4 bh, bf4 bl) -> f4 {  // a . (bl + bh)
+        const f4 z = {0, 0, 0, 0};
+        const bf4 a_h = __builtin_bit_cast(bf4, ah);
+        return mfma_bf(cat_bf4(a_h, a_h), cat_bf4(bl, bh), z);
+      };
+
       // ---- tile by tile: the state terms of the lane's four rows of tile R, the blocks of F and G that end in them,
       // and their share of the column phase.  Row block R of T (rows 16 R + cm) serves the F blocks (R, c <= R) and, T
       // being symmetric, the G blocks (c >= R, R); on the diagonal block F keeps the columns <= the row and G those >= it.
 #pragma unroll
       for (int R = 0; R < 4; ++R) {
         f4 xf = {0, 0, 0, 0}, xg = {0, 0, 0, 0};  // the blocks' sums
+        f4 df = {0, 0, 0, 0}, dg = {0, 0, 0, 0};  // DIAG2: those of the diagonal block
+        bf4 cl = {}, bl = {};                     // DIAG2: what the operands of rows 16 R + 4 g4 + j lost to bf16
+        if constexpr (DIAG2) {
+          if constexpr (BCL)
+#pragma unroll
+            for (int i = 2 * R; i < 2 * R + 2; ++i) {
+              bvp[i] = s.bc[i * NTHREADS + tid];
+              cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
+            }
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int k = 4 * R + j;
+            cl[j] = (__bf16)(unpk(cvp, k) * up[k] - (float)Ch[R][j]);
+            bl[j] = (__bf16)(unpk(bvp, k) * dtp[k] * iup[k] - (float)Bh[R][j]);
+          }
+        }
         f4 sf, sg;                                // the state terms
         {
           f4 q = {0, 0, 0, 0}, r = {0, 0, 0, 0};
@@ -386,9 +420,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
               ah.x &= mf[0]; ah.y &= mf[1];
               al.x &= mf[0]; al.y &= mf[1];
             }
-            const f4 acc = block(ah, al, Bh[c], Bl[c]);
+            if (DIAG2 && c == R) {
+              df = block_pair(ah, Bh[c], bl);
+            } else {
+              const f4 acc = block(ah, al, Bh[c], Bl[c]);
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
+              for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
+            }
           }
           if (c >= R) {  // G block (c, R)
             uint2 ah = th[c], al = tl[c];
@@ -396,21 +434,25 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
               ah.x &= mg[0]; ah.y &= mg[1];
               al.x &= mg[0]; al.y &= mg[1];
             }
-            const f4 acc = block(ah, al, Ch[c], Cl[c]);
+            if (DIAG2 && c == R) {
+              dg = block_pair(ah, Ch[c], cl);
+            } else {
+              const f4 acc = block(ah, al, Ch[c], Cl[c]);
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
+              for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
+            }
           }
         }
         // The rows' share of the column phase.  d/d(cs) = C X2 - Bd E1 takes the blocks' sums times the operands as the
         // matrix instructions took them: a pair of rows then enters both of its rows as one and the same product and
         // cancels in the suffix sums to fp32 rounding.  The state terms cancel against the state pass's column sums,
         // which were formed from unrounded states: with bf16 inputs they take the unrounded operands (B and C are
-        // exact, the decays fp32); with fp32 inputs the 16-bit operands are as accurate as the split products Q and R.
+        // exact, the decays fp32); with fp32 inputs the 17-bit operands are as accurate as the split products Q and R.
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int k = 4 * R + rr;
           const float bv = SPLIT ? bvf[k] : unpk(bvp, k);
-          const float E1 = iup[k] * (sg[rr] + xg[rr]), X2 = up[k] * (sf[rr] + xf[rr]);
+          const float E1 = iup[k] * (sg[rr] + xg[rr] + dg[rr]), X2 = up[k] * (sf[rr] + xf[rr] + df[rr]);
           s.dbc[k * NTHREADS + tid] += dtp[k] * E1;
           s.dbc[(16 + k) * NTHREADS + tid] += X2;
           val[k] = bv * E1;
@@ -419,7 +461,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
             dcs[k] = c16 * (xf[rr] + sf[rr]) - b16 * (xg[rr] + sg[rr]);
           } else {
             const float c16 = (float)Ch[R][rr], b16 = (float)Bh[R][rr];
-            dcs[k] = (c16 * xf[rr] - b16 * xg[rr]) + (unpk(cvp, k) * up[k] * sf[rr] - bv * dtp[k] * iup[k] * sg[rr]);
+            float pairs = c16 * xf[rr] - b16 * xg[rr];
+            if constexpr (DIAG2) pairs += (c16 + (float)cl[rr]) * df[rr] - (b16 + (float)bl[rr]) * dg[rr];
+            dcs[k] = pairs + (unpk(cvp, k) * up[k] * sf[rr] - bv * dtp[k] * iup[k] * sg[rr]);
           }
         }
       }
@@ -432,18 +476,18 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     const float gl_keep = l_gl;
     float old[16];
     if constexpr (ACC) {
-      if constexpr (P32) lane_load_ln<false>(p.ddt_part, u.b, u.h, n, true, g4, rm, old);
-      else lane_load_ln<IOB>(p.ddt, u.b, u.h, n, true, g4, rm, old);
+      if constexpr (P32) lane_load_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, old);
+      else lane_load_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, old);
     }
     request(head_of(min(hh + 1, p.hpg - 1)));  // (unconditional: the last head is requested again and not used)
     __builtin_amdgcn_sched_barrier(0);
     if (skip) {
       // the level-hierarchy kernel adds this head's share to ddt later: it must find the other direction's, or zero
       if constexpr (!ACC) {  // (val is all zero here)
-        if constexpr (P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, true, g4, rm, val);
-        else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, true, g4, rm, val);
+        if constexpr (P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
+        else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, val);
       } else if constexpr (P32) {
-        lane_store_ln<IOB>(p.ddt, u.b, u.h, n, true, g4, rm, old);  // the other direction's share moves into ddt
+        lane_store_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, old);  // the other direction's share moves into ddt
       }
       continue;
     }
@@ -498,11 +542,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
       for (int k = 0; k < 16; ++k) val[k] += old[k];
     }
-    if constexpr (!ACC && P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, true, g4, rm, val);
-    else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, true, g4, rm, val);
+    if constexpr (!ACC && P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
+    else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, val);
     sumA = scan_g_incl(sumA, g4);
     sumB = scan_g_incl(sumB, g4);
-    if (g4 == 3) {
+    if (g4 == 3 && vn) {
       // (an opaque copy of the column: the two per-lane addresses are then formed here instead of being kept, as 64-bit
       // values, across the head loop -- a reload from scratch at this point would wait for every request in flight)
       int nq = n;
@@ -519,22 +563,23 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       vb[k] = s.dbc[k * NTHREADS + tid];
       vc[k] = s.dbc[(16 + k) * NTHREADS + tid];
     }
-    if (p.dB[u.dir].ptr) lane_store_ln<IOB>(p.dB[u.dir], u.b, u.g, n, true, g4, rm, vb);
-    if (p.dC[u.dir].ptr) lane_store_ln<IOB>(p.dC[u.dir], u.b, u.g, n, true, g4, rm, vc);
+    if (p.dB[u.dir].ptr) lane_store_ln<IOB>(p.dB[u.dir], u.b, u.g, n, vn, g4, rm, vb);
+    if (p.dC[u.dir].ptr) lane_store_ln<IOB>(p.dC[u.dir], u.b, u.g, n, vn, g4, rm, vc);
   }
 }
 
-// Whether the tile-base kernel is built for this call (otherwise the level-hierarchy kernel does all the work): complete
-// tiles, x / B / C and dt of one type, x and dout rows that allow vector accesses, no gate, ddt wanted, and -- fp32
+// Whether the tile-base kernel is built for this call (otherwise the level-hierarchy kernel does all the work): no packed
+// sequences (their cuts are outside the form's range), x / B / C and dt of one type, x and dout rows that allow vector
+// accesses, ddt wanted, a gated dy (which is fp32) only beside fp32 inputs, and -- fp32
 // inputs with four head tiles would need split x / dy tiles and T that leave one workgroup per CU -- P <= 48 for fp32.
 bool bwd_tile_available(const KP& p, const float* dy_ws) {
-  if (p.full_tiles != 1 || dy_ws || p.io_dt != p.dt_dt || !p.ddt.ptr) return false;
+  if (p.seq_idx || (dy_ws && p.io_dt) || p.io_dt != p.dt_dt || !p.ddt.ptr) return false;
   if (p.io_dt == 0 && p.P > 48) return false;
   const int es = p.io_dt ? 2 : 4;
   for (int d = 0; d < p.ndir; ++d) {
     const TensorD* ts[2] = {&p.x[d], &p.dout[d]};
     for (const TensorD* t : ts)
-      if ((p.P & 3) || ((t->s0 | t->s1 | t->s2) & 3) || (((uintptr_t)t->ptr) & (4 * es - 1))) return false;
+      if ((dy_ws && t == &p.dout[d]) ? (p.P & 3) != 0 : (p.P & 3) || ((t->s0 | t->s1 | t->s2) & 3) || (((uintptr_t)t->ptr) & (4 * es - 1))) return false;
   }
   return true;
 }
@@ -552,19 +597,28 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), sm, st, p, states, dstates, dm, g_last, partA, partBias, redo);
     return 0;
   };
-  if constexpr (IOB) {
-    if (p.ddt_part.ptr) {
-      if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, true>) : go(&k_bwd_tile<PT, IOB, true, false, true>);
-      return acc ? go(&k_bwd_tile<PT, IOB, false, true, true>) : go(&k_bwd_tile<PT, IOB, false, false, true>);
-    }
-  }
-  if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, false>) : go(&k_bwd_tile<PT, IOB, true, false, false>);
-  return acc ? go(&k_bwd_tile<PT, IOB, false, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, false>);
+  auto pick = [&](auto p32) -> int {
+    constexpr bool P32 = decltype(p32)::value;
+    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false>);
+    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true>);
+    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true>);
+  };
+  if constexpr (IOB)
+    if (p.ddt_part.ptr) return pick(std::true_type{});
+  return pick(std::false_type{});
 }
 
-int launch_bwd_tile(const KP& p, const float* states, const float* dstates, const float* dm, const float* g_last,
-                    float* partA, float* partBias, int* redo, hipStream_t st) {
-  const int blocks = p.B * p.nc * p.G * (p.N / NS);
+int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const float* dstates, const float* dm,
+                    const float* g_last, float* partA, float* partBias, int* redo, hipStream_t st) {
+  KP p = p_;
+  if (dy_ws) {  // a gated dy: fp32 (Bt, L, H, P) contiguous, batch * direction outermost
+    TensorD& t = p.dout[p.dir0];
+    t.s2 = p.P;
+    t.s1 = (long)p.H * p.P;
+    t.s0 = (long)p.ndir * p.L * p.H * p.P;
+    t.ptr = dy_ws + (long)p.dir0 * p.L * p.H * p.P;
+  }
+  const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   const int pt = (p.P + 15) / 16;
   int e = 0;
   if (p.io_dt) {

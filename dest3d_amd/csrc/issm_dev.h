@@ -66,11 +66,9 @@ struct KP {
   const int* seq_idx;   // (B, L) sequence ids of packed rows, or null
   long seq_s0, seq_s1;
   // Chunks [c_lo, c_lo + ncl) are the ones a launch of a per-chunk kernel covers (all nc of them).  full_tiles picks
-  // the kernel variants: 1 = every chunk has 64 rows and every column slice 64 columns (complete-tile code, no
-  // masks); 2 = that holds for all chunks but the last in scan order (the sequence length is not a multiple of 64):
-  // one launch whose workgroups take the complete-tile code except those of the last chunk, which take the general
-  // code -- the general code alone runs 1.5 - 2x longer; 0 = general code everywhere (ragged column slices, packed
-  // sequences, a single chunk).
+  // the kernel variants: 1 = every chunk has 64 rows and every column slice 64 columns (complete-tile code); 0 = the
+  // "edge" variants (FULL = false), the same code with clamped addresses, dt' = 0 where a row or column is absent and
+  // guarded stores in the workgroups and steps that have such rows or columns.
   int c_lo, ncl, full_tiles;
 };
 
@@ -496,10 +494,13 @@ __device__ __forceinline__ float scan_g_incl_rev(float v, int g4) {
 // i.e. physical row base + step * (16J + j): a per-lane part (base) plus a part that is the same
 // for the whole wave, so that in a full chunk the address of every element is a scalar base
 // plus ONE per-lane offset.  `full` (a compile-time constant of the kernel variant) says that all 64
-// rows and all 64 columns of every slice exist (the head dimension is checked separately at run time); otherwise rows >= nvalid and lanes with !vn read as zero.
+// rows and all 64 columns of every slice exist (the head dimension is checked separately at run time).  Otherwise
+// `edge` (uniform) says whether this chunk has fewer than 64 rows or the slice fewer than 64 columns: absent rows read
+// zero and absent columns column 0 -- finite whenever the inputs are -- and everything that would let them act is zero:
+// dt' (hence B dt' and the decays), x and dy rows, stored results.
 struct RowMap {
-  int base, step, nvalid;
-  bool full;
+  int base, step, nvalid, rows, cols;
+  bool full, edge;
   unsigned long long cut;  // bit r: the sequence id changes between rows r - 1 and r of the chunk (scan order; the initial states count as id 0); uniform
 };
 template <bool FULL>
@@ -511,6 +512,9 @@ __device__ __forceinline__ RowMap make_rowmap(const KP& p, const Unit& u, int g4
   r.nvalid = min(CS, p.L - u.c * CS);
   // FULL kernels are only launched when every chunk and every column slice is complete
   r.full = FULL;
+  r.rows = p.L;
+  r.cols = p.N;
+  r.edge = !FULL && (r.nvalid < CS || n0 + NS > p.N);
   r.cut = 0;
   if (!FULL && p.seq_idx) {  // packed sequences take the kernels' general variants
     // lane = row of the chunk in scan order; its predecessor in scan order may be the previous chunk's last row
@@ -527,48 +531,46 @@ __device__ __forceinline__ RowMap make_rowmap(const KP& p, const Unit& u, int g4
   }
   return r;
 }
+// A (b, third) slab of a (B,L,G|H,N)-shaped tensor as a raw buffer: a load whose byte offset lies at or beyond the end
+// of the slab's last row returns zero.  That covers the rows a chunk does not have at no cost
+// per access: forwards they lie past the last row; backwards they lie before the first one, and a negative 32-bit offset
+// is a very large one.  (The host keeps a slab below 2^32 bytes; within 63 rows of that an absent row's offset may wrap to
+// one of another row: still inside the slab, and the value is not used.)  Word 3: raw 32-bit data format.
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_of(const T* q, const TensorD& t, int rows, int cols) {
+  const unsigned bytes = (unsigned)((rows - 1) * (int)t.s1 + cols) * (unsigned)sizeof(T);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)const_cast<T*>(q), 0, bytes, 0x00027000);
+}
 // Lane's 16 values of column n of a (B,L,G|H,N)-shaped tensor.
 template <bool BF>
 __device__ __forceinline__ void lane_load_ln(const TensorD& t, int b, int third, int n, bool vn, int g4,
                                              const RowMap& rm, float (&out)[16]) {
   typedef typename std::conditional<BF, uint16_t, float>::type T;
   const T* q = (const T*)t.ptr + ((long)b * t.s0 + (long)third * t.s2);
-  const long ss = (long)rm.step * t.s1;  // uniform
   T r[16];
+  // 32-bit offsets (the host checks that seqlen * stride fits): address = scalar base + per-lane offset.
+  // ks is made opaque so that its multiples are formed here, next to their use, instead of being
+  // hoisted out of an enclosing loop into (scarce) scalar registers.
+  // BYTE offsets in 32 bits, so that the access is "scalar base + 32-bit per-lane offset" and costs one
+  // integer add per element.
+  const unsigned lo = (unsigned)(rm.base * (int)t.s1 + (rm.full || vn ? n : 0)) * (unsigned)sizeof(T);
+  unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
+  ISSM_OPAQUE_S(ks);
+  const char* qb = (const char*)q;
   if (rm.full) {
-    // 32-bit offsets (the host checks that seqlen * stride fits): address = scalar base + per-lane offset.
-    // ks is made opaque so that its multiples are formed here, next to their use, instead of being
-    // hoisted out of an enclosing loop into (scarce) scalar registers.
-    // BYTE offsets in 32 bits, so that the access is "scalar base + 32-bit per-lane offset" and costs one
-    // integer add per element.
-    const unsigned lo = (unsigned)(rm.base * (int)t.s1 + n) * (unsigned)sizeof(T);
-    unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
-    ISSM_OPAQUE_S(ks);
-    const char* qb = (const char*)q;
 #pragma unroll
     for (int k = 0; k < 16; ++k) r[k] = *(const T*)(qb + (lo + (unsigned)(16 * (k >> 2) + (k & 3)) * ks));
-#pragma unroll
-    for (int k = 0; k < 16; ++k) out[k] = BF ? bf16_to_f((uint16_t)r[k]) : (float)r[k];
   } else {
-    // The same 32-bit addressing with the row clamped to the chunk's last existing row and the column to 0: every
-    // lane reads an address inside the tensor, and what it read is replaced by zero where the row or column is absent
-    // (64-bit per-element offsets and a mask array held across the loads cost the general variants some forty
-    // registers per call site).
-    (void)ss;
-    const int rmax = rm.nvalid - 1 - 4 * g4;  // last existing row, relative to the lane's row 0 (may be negative)
-    const unsigned lo = (unsigned)(rm.base * (int)t.s1 + (vn ? n : 0)) * (unsigned)sizeof(T);
-    unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
-    ISSM_OPAQUE_S(ks);
-    const char* qb = (const char*)q;
+    const __amdgpu_buffer_rsrc_t rs = slab_of(q, t, rm.rows, rm.cols);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      const int rk = 16 * (k >> 2) + (k & 3);
-      r[k] = *(const T*)(qb + (lo + (unsigned)min(rk, rmax) * ks));  // a negative row wraps like the base does
+      const unsigned o = lo + (unsigned)(16 * (k >> 2) + (k & 3)) * ks;
+      if constexpr (BF) r[k] = __builtin_amdgcn_raw_buffer_load_b16(rs, o, 0, 0);
+      else r[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
     }
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-      out[k] = (vn && 16 * (k >> 2) + (k & 3) <= rmax) ? (BF ? bf16_to_f((uint16_t)r[k]) : (float)r[k]) : 0.0f;
   }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) out[k] = BF ? bf16_to_f((uint16_t)r[k]) : (float)r[k];
 }
 // Store of the lane's 16 values to column n of a (B,L,G|H,N)-shaped tensor (absent rows / columns skipped).
 template <bool BF>
@@ -576,58 +578,46 @@ __device__ __forceinline__ void lane_store_ln(const TensorD& t, int b, int third
                                               const RowMap& rm, const float (&v)[16]) {
   typedef typename std::conditional<BF, uint16_t, float>::type T;
   T* q = (T*)const_cast<void*>(t.ptr) + ((long)b * t.s0 + (long)third * t.s2);
-  const long ss = (long)rm.step * t.s1;
-  if (rm.full) {
-    const unsigned lo = (unsigned)(rm.base * (int)t.s1 + n) * (unsigned)sizeof(T);
-    unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
-    ISSM_OPAQUE_S(ks);
-    char* qb = (char*)q;
+  const unsigned lo = (unsigned)(rm.base * (int)t.s1 + n) * (unsigned)sizeof(T);
+  unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
+  ISSM_OPAQUE_S(ks);
+  char* qb = (char*)q;
+  if (rm.full || !rm.edge) {  // uniform
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       T* d = (T*)(qb + (lo + (unsigned)(16 * (k >> 2) + (k & 3)) * ks));
       if (BF) *d = (T)f_to_bf16(v[k]); else *d = (T)v[k];
     }
   } else {
-    (void)ss;
-    const int rmax = rm.nvalid - 1 - 4 * g4;
-    const unsigned lo = (unsigned)(rm.base * (int)t.s1 + n) * (unsigned)sizeof(T);
-    unsigned ks = (unsigned)(rm.step * (int)t.s1) * (unsigned)sizeof(T);
-    ISSM_OPAQUE_S(ks);
-    char* qb = (char*)q;
+    const int rmax = vn ? rm.nvalid - 1 - 4 * g4 : -1;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       const int rk = 16 * (k >> 2) + (k & 3);
-      if (vn && rk <= rmax) {
+      if (rk <= rmax) {
         T* d = (T*)(qb + (lo + (unsigned)rk * ks));
         if (BF) *d = (T)f_to_bf16(v[k]); else *d = (T)v[k];
       }
     }
   }
 }
-// Lane's values of column n of a (P x N) fp32 slab: index q <-> row 16 (q >> 2) + 4 g4 + (q & 3).
+// Lane's values of column n of a (P x N) fp32 slab: index q <-> row 16 (q >> 2) + 4 g4 + (q & 3).  `full`: every row
+// exists; otherwise rows past the head dimension read its last row (they meet zero columns of the x / dy tiles).  Absent
+// columns read column 0.
 template <int CNT>
 __device__ __forceinline__ void lane_load_pn(const float* __restrict__ src, int P, int N, int n, bool vn, int g4,
                                              bool full, float (&out)[CNT]) {
+  const int nn = vn ? n : 0;
+  const unsigned lo = (unsigned)(4 * g4 * N + nn) * 4u;
+  unsigned nb = (unsigned)N * 4u;
+  ISSM_OPAQUE_S(nb);
+  const char* sb = (const char*)src;
   if (full) {
-    const unsigned lo = (unsigned)(4 * g4 * N + n) * 4u;
-    unsigned nb = (unsigned)N * 4u;
-    ISSM_OPAQUE_S(nb);
-    const char* sb = (const char*)src;
 #pragma unroll
     for (int q = 0; q < CNT; ++q) out[q] = *(const float*)(sb + (lo + (unsigned)(16 * (q >> 2) + (q & 3)) * nb));
   } else {
-    // rows clamped to the last one of the head, the column to 0; absent values replaced by zero afterwards
-    float r[CNT];
-    const int pmax = P - 1 - 4 * g4;
-    const unsigned lo = (unsigned)(4 * g4 * N + (vn ? n : 0)) * 4u;
-    unsigned nb = (unsigned)N * 4u;
-    ISSM_OPAQUE_S(nb);
-    const char* sb = (const char*)src;
+    const unsigned last = (unsigned)((P - 1) * N + nn) * 4u;
 #pragma unroll
-    for (int q = 0; q < CNT; ++q)
-      r[q] = *(const float*)(sb + (lo + (unsigned)min(16 * (q >> 2) + (q & 3), pmax) * nb));
-#pragma unroll
-    for (int q = 0; q < CNT; ++q) out[q] = (vn && 16 * (q >> 2) + (q & 3) <= pmax) ? r[q] : 0.0f;
+    for (int q = 0; q < CNT; ++q) out[q] = *(const float*)(sb + min(lo + (unsigned)(16 * (q >> 2) + (q & 3)) * nb, last));
   }
 }
 // dt transform (bias -> softplus -> clamp) of the lane's rows and the inclusive running sum of
@@ -640,9 +630,10 @@ struct Coef {
   float A, bias;
 };
 __device__ __forceinline__ Coef lane_coef(const KP& p, int h, int n, bool vn) {
+  const int o = h * p.N + (vn ? n : 0);
   Coef c;
-  c.A = vn ? p.A[h * p.N + n] : 0.0f;
-  c.bias = (vn && p.dt_bias) ? p.dt_bias[h * p.N + n] : 0.0f;
+  c.A = p.A[o];
+  c.bias = p.dt_bias ? p.dt_bias[o] : 0.0f;
   return c;
 }
 // dt transform of CNT values that already include the bias: softplus -> clamp; dfac (if WANT_DFAC) receives
@@ -682,7 +673,7 @@ __device__ __forceinline__ void dt_transform(const KP& p, const float (&pre_)[CN
   }
 }
 // dt transform (bias -> softplus -> clamp) of the lane's 16 rows.  Rows past the end of the sequence and absent columns
-// come out as dt' = 0.
+// come out as dt' = 0 with derivative 0.
 template <bool WANT_DFAC>
 __device__ __forceinline__ void lane_dt(const KP& p, const Coef& cf, bool vn, int g4, const RowMap& rm,
                                         const float (&raw)[16], float (&dtp)[16], float (&dfac)[16]) {
@@ -690,10 +681,14 @@ __device__ __forceinline__ void lane_dt(const KP& p, const Coef& cf, bool vn, in
 #pragma unroll
   for (int k = 0; k < 16; ++k) pre[k] = raw[k] + cf.bias;
   dt_transform<WANT_DFAC, 16>(p, pre, dtp, dfac);
-  if (!rm.full) {  // rows past the end of the sequence and absent columns behave as dt' = 0
+  if (!rm.full && rm.edge) {  // uniform: rows past the end of the sequence and absent columns behave as dt' = 0
+    const int lim = vn ? rm.nvalid - 4 * g4 : 0;
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-      if (!(vn && lane_row(k, g4) < rm.nvalid)) dtp[k] = 0.0f;
+      if (16 * (k >> 2) + (k & 3) >= lim) {
+        dtp[k] = 0.0f;
+        if (WANT_DFAC) dfac[k] = 0.0f;
+      }
   }
 }
 template <bool WANT_DFAC>
@@ -807,8 +802,8 @@ typedef short sh4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f4 mfma_bf16k(bf4 a, bf4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(sh4, a), __builtin_bit_cast(sh4, b), c, 0, 0, 0);
 }
-// an fp32 value cut to 16 significand bits (towards zero): it then splits into two bf16 numbers exactly
-__device__ __forceinline__ float trunc16(float v) { return __uint_as_float(__float_as_uint(v) & 0xffffff00u); }
+// an fp32 value rounded to 17 significand bits: it then splits into a bf16 number and a signed bf16 rest exactly
+__device__ __forceinline__ float round17(float v) { return __uint_as_float((__float_as_uint(v) + 0x40u) & 0xffffff80u); }
 
 // ------------------------------------------------------------------ cooperative tile loaders
 // The unit's (64 x P) tile of a (B,L,H,P) tensor, zero padded to 16*PT columns: registers, then
@@ -977,40 +972,61 @@ __device__ __forceinline__ void tril_store(const f4 (&v)[4], float* dst, int tid
   }
 }
 
-// Columns n0..n0+63 of a (P x N) fp32 slab, zero padded to 16*PT rows and past N: registers, then
-// LDS dst[p][col] (leading dimension LDN).
+// Four adjacent fp32 values at any element offset (a type that only promises element alignment: unaligned accesses are
+// legal on this target, and rows of N floats start anywhere when N is not a multiple of 4).
+struct __attribute__((packed, aligned(4))) F4Any {
+  float x, y, z, w;
+};
+__device__ __forceinline__ f4 ld_f4_any(const float* q) {
+  const F4Any w = *(const F4Any*)q;
+  return (f4){w.x, w.y, w.z, w.w};
+}
+__device__ __forceinline__ void st_f4_any(float* q, f4 v) {
+  F4Any w;
+  w.x = v[0]; w.y = v[1]; w.z = v[2]; w.w = v[3];
+  *(F4Any*)q = w;
+}
+
+// Columns n0..n0+63 of a (P x N) fp32 slab: registers, then LDS dst[p][col] (leading dimension LDN).  Rows past P repeat
+// the last one (what they contribute to is not stored).  Columns past N read whatever follows in the slab, or zero beyond
+// its end (a raw buffer load checks every dword; it needs dword alignment only): pn_edge, called before the values are used,
+// zeroes them.
 template <int PT>
 struct PnRegs {
   static constexpr int Q = NS / 4, TOT = PT * 16 * Q, CNT = (TOT + NTHREADS - 1) / NTHREADS;
+  static_assert(TOT % NTHREADS == 0, "every thread owns CNT quads");
   f4 v[CNT];
 };
-template <int PT>
+template <int PT, bool FULL>
 __device__ __forceinline__ void pn_load(const KP& p, const float* __restrict__ src, int n0, PnRegs<PT>& r,
                                         int tid = threadIdx.x) {
   typedef PnRegs<PT> R;
-  const bool vec = (p.N & 3) == 0;
+  const int c = n0 + (tid % R::Q) * 4;
+  if constexpr (FULL) {
 #pragma unroll
-  for (int i = 0; i < R::CNT; ++i) {
-    const int e = tid + i * NTHREADS, pp = e / R::Q, c4 = (e % R::Q) * 4;
-    const bool ok = e < R::TOT && pp < p.P;
-    const long o = (long)pp * p.N + n0 + c4;
-    // absent rows / columns read the slab's first elements and count as zero: a conditional load would become a
-    // branch, and a branch per load makes each wait for the one before
-    if (vec) {
-      const bool in = ok && n0 + c4 < p.N;
-      const f4 w = *(const f4*)(src + (in ? o : 0));
-      r.v[i] = in ? w : (f4){0, 0, 0, 0};
-    } else {
-      f4 w;
+    for (int i = 0; i < R::CNT; ++i)
+      r.v[i] = *(const f4*)(src + (min((tid + i * NTHREADS) / R::Q, p.P - 1) * p.N + c));
+  } else {
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)const_cast<float*>(src), 0, (unsigned)(p.P * p.N) * 4u, 0x00027000);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const bool in = ok && n0 + c4 + j < p.N;
-        const float t = src[in ? o + j : 0];
-        w[j] = in ? t : 0.0f;
-      }
-      r.v[i] = w;
+    for (int i = 0; i < R::CNT; ++i) {
+      const u4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, (min((tid + i * NTHREADS) / R::Q, p.P - 1) * p.N + c) * 4, 0, 0);
+      r.v[i] = __builtin_bit_cast(f4, w);
     }
   }
+}
+template <int PT>
+__device__ __forceinline__ void pn_edge(const KP& p, int n0, PnRegs<PT>& r, int tid = threadIdx.x) {
+  typedef PnRegs<PT> R;
+  if (n0 + NS <= p.N) return;  // uniform
+  const int left = p.N - n0 - (tid % R::Q) * 4;   // columns of the quad that exist
+#pragma unroll
+  for (int i = 0; i < R::CNT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j >= left) r.v[i][j] = 0.0f;
 }
 template <int PT>
 __device__ __forceinline__ void pn_store(const PnRegs<PT>& r, float* dst, int tid = threadIdx.x) {
@@ -1039,12 +1055,11 @@ __device__ __forceinline__ long sq_off(const KP& p, int bt, int c, int h) {
   return (((long)bt * p.nc + c) * p.H + h) * CS * CS;
 }
 
-// Kernel dispatch on (P tiles, io dtype, dt dtype, complete / mixed tiles): the statement sees PT_, IOB_, DTB_, FULL_, MIXED_
-// as constants.
-#define ISSM_DISPATCH_FULL(full, ...)                                                                       \
-  if ((full) == 1) { constexpr bool FULL_ = true; constexpr bool MIXED_ = false; (void)MIXED_; __VA_ARGS__ }        \
-  else if ((full) == 2) { constexpr bool FULL_ = false; constexpr bool MIXED_ = true; (void)FULL_; __VA_ARGS__ }    \
-  else { constexpr bool FULL_ = false; constexpr bool MIXED_ = false; (void)MIXED_; __VA_ARGS__ }
+// Kernel dispatch on (P tiles, io dtype, dt dtype, complete tiles or not): the statement sees PT_, IOB_, DTB_, FULL_ as
+// constants.
+#define ISSM_DISPATCH_FULL(full, ...)                              \
+  if (full) { constexpr bool FULL_ = true; __VA_ARGS__ }           \
+  else { constexpr bool FULL_ = false; __VA_ARGS__ }
 #define ISSM_DISPATCH_DT(iob, dtb, full, ...)                          \
   if (iob) {                                                           \
     constexpr bool IOB_ = true;                                        \

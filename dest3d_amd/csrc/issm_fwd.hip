@@ -29,27 +29,22 @@ template <int PT, bool IOB, bool DTB, bool FULL>
 __global__ __launch_bounds__(NTHREADS, 2) void k_chunk_local(KP p, float* __restrict__ states, float* __restrict__ cs_last, float* __restrict__ cabt) {
   k_chunk_local_body<PT, IOB, DTB, FULL>(p, states, cs_last, cabt);
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool IOB, bool DTB>
-__global__ __launch_bounds__(NTHREADS, 2) void k_chunk_local_mixed(KP p, float* __restrict__ states, float* __restrict__ cs_last, float* __restrict__ cabt) {
-  if (decode_unit(p, xcd_remap(blockIdx.x, gridDim.x)).c == p.nc - 1) k_chunk_local_body<PT, IOB, DTB, false>(p, states, cs_last, cabt);
-  else k_chunk_local_body<PT, IOB, DTB, true>(p, states, cs_last, cabt);
-}
-
 
 // ---------------------------------------------------------------- state passing
 // One thread carries 4 adjacent state columns of one (bt, h, p) through all chunks.
 // Slot c of `states` holds S_c on entry and H_c (state at the start of chunk c) on exit;
 // slot nc receives the final state.
-// The recurrence for N a multiple of 4, without any conditional access: thread = 4 adjacent columns of one state row,
+// The recurrence without any conditional access in its loop: thread = 4 adjacent columns of one state row,
 // the operands of the next D chunks always requested (near the end the last chunk again: in range, unused), so the
 // compiler can count the loads in flight and never waits for all of them; with loads inside branches it did, once
 // per chunk.  D = 8 when few threads walk many chunks (memory latency sets the pace there), otherwise 4.
-template <int D>
+// TAIL (N >= 4, not a multiple of 4; accesses at any float): the last thread of a row works on columns N - 4 .. N - 1 and
+// stores only those its neighbour does not own (what it computes for the others may read the neighbour's results and is
+// dropped).  8 x 1024 tokens, N = 250: 30.3 us with per-element guards, as fast as N = 256 without.
+template <int D, bool TAIL>
 __global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __restrict__ states,
                                                              const float* __restrict__ cs_last) {
-  const int nq = p.N >> 2;
+  const int nq = (p.N + 3) >> 2;
   const long total = (long)p.B * p.ndir * p.H * p.P * nq;
   const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
   if (id >= total) return;
@@ -60,7 +55,22 @@ __global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __rest
   const int h = r % p.H;
   const int bt = r / p.H;
   const int b = bt / p.ndir, dir = bt % p.ndir;
-  const int n = q * 4;
+  const int n = TAIL ? min(q * 4, p.N - 4) : q * 4, skip = q * 4 - n;   // skip: columns of the thread that are its neighbour's
+  auto ld = [](const float* a) -> f4 {
+    if constexpr (TAIL) return ld_f4_any(a);
+    else return *(const f4*)a;
+  };
+  auto put = [&](float* a, f4 v) {
+    if constexpr (!TAIL) {
+      *(f4*)a = v;
+    } else if (skip == 0) {
+      st_f4_any(a, v);
+    } else {
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (j >= skip) a[j] = v[j];
+    }
+  };
   f4 st = {0, 0, 0, 0};
   if (p.h0.ptr) {
     const long o = (long)b * p.h0.s0 + (long)h * p.h0.s1 + (long)pp * p.h0.s2 + n;
@@ -78,8 +88,8 @@ __global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __rest
 #pragma unroll
   for (int i = 0; i < D; ++i) {
     const int ci = min(i, p.nc - 1);
-    t[i] = *(const f4*)(sp0 + ci * cstride);
-    d[i] = *(const f4*)(cl0 + ci * dstride);
+    t[i] = ld(sp0 + ci * cstride);
+    d[i] = ld(cl0 + ci * dstride);
   }
   int c = 0;
   for (; c + D <= p.nc; c += D) {
@@ -87,9 +97,9 @@ __global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __rest
     for (int i = 0; i < D; ++i) {
       const f4 tt = t[i], dd = d[i];
       const int cn = min(c + i + D, p.nc - 1);
-      t[i] = *(const f4*)(sp0 + cn * cstride);
-      d[i] = *(const f4*)(cl0 + cn * dstride);
-      *(f4*)sp = st;
+      t[i] = ld(sp0 + cn * cstride);
+      d[i] = ld(cl0 + cn * dstride);
+      put(sp, st);
 #pragma unroll
       for (int j = 0; j < 4; ++j) st[j] = __expf(dd[j]) * st[j] + tt[j];
       sp += cstride;
@@ -98,16 +108,16 @@ __global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __rest
 #pragma unroll
   for (int i = 0; i < D - 1; ++i)
     if (c + i < p.nc) {  // uniform: the last nc % D chunks
-      *(f4*)sp = st;
+      put(sp, st);
 #pragma unroll
       for (int j = 0; j < 4; ++j) st[j] = __expf(d[i][j]) * st[j] + t[i][j];
       sp += cstride;
     }
-  *(f4*)sp = st;  // slot nc keeps the final state for the backward pass
-  if (p.final_states[dir]) *(f4*)(p.final_states[dir] + (((long)b * p.H + h) * p.P + pp) * p.N + n) = st;
+  put(sp, st);  // slot nc keeps the final state for the backward pass
+  if (p.final_states[dir]) put(p.final_states[dir] + (((long)b * p.H + h) * p.P + pp) * p.N + n, st);
 }
 
-// The recurrence for any N (launched when N is not a multiple of 4): element-wise guards, scalar accesses.
+// The recurrence for N < 4: element-wise guards, scalar accesses.
 __global__ __launch_bounds__(NTHREADS) void k_state_fwd(KP p, float* __restrict__ states,
                                                         const float* __restrict__ cs_last) {
   const int nq = (p.N + 3) >> 2;
@@ -234,7 +244,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, cv);
-  pn_load<PT>(p, hsrc, 0, hv);
+  pn_load<PT, FULL>(p, hsrc, 0, hv);
   // M of this wave's 16 rows goes straight into matrix-operand registers (lane (row cm, group g4) holds columns
   // 16 kb + 4 g4 .. + 3 of the blocks kb <= wave, the upper triangle of the diagonal block zeroed): no LDS tile, which
   // lets a fourth workgroup live on the CU
@@ -277,6 +287,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
         for (int k = 0; k < 16; ++k) s.ct[lane_row(k, g4) * LDN + wave * 16 + cm] = cv[k] * ex2(cs[k]);
       }
     }
+    if constexpr (!FULL) pn_edge<PT>(p, n0, hv);
     if constexpr (IOB) pn_store_bf<PT, LDK>(hv, s.hs);
     else if constexpr (SM::SPL) pn_store_split<PT, LDK>(hv, s.hs, s.hs + PT * 16 * LDK);
     else pn_store<PT>(hv, s.hs);
@@ -287,7 +298,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
       lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
       cf = lane_coef(p, u.h, n, vn);
       lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, cv);
-      pn_load<PT>(p, hsrc, n0 + NS, hv);
+      pn_load<PT, FULL>(p, hsrc, n0 + NS, hv);
     }
     __syncthreads();
     // y[l][p] += sum_n Ct[l][n] H[p][n]; wave owns 16 rows
@@ -365,20 +376,12 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
     gstore<IOB, 4>(const_cast<void*>(to.ptr), (long)u.b * to.s0 + (long)u.h * to.s2, off, v);
   }
 }
-// fp32 inputs, two head tiles: 128 registers, so that a fourth workgroup lives on the CU (130 without the bound; the
-// nine spilled dwords cost less than the fourth workgroup gives: 52 -> 48.5 us)
+// two head tiles, fp32 inputs or edges: 128 registers, so that a fourth workgroup lives on the CU (130 - 145 without the
+// bound; the spilled dwords cost less than the fourth workgroup gives: 52 -> 48.5 us)
 template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, (PT <= 2 && FULL && !IOB) ? 4 : 1) void k_chunk_scan(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
+__global__ __launch_bounds__(NTHREADS, (PT <= 2 && (!IOB || !FULL)) ? 4 : 1) void k_chunk_scan(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
   k_chunk_scan_body<PT, IOB, DTB, FULL>(p, states, cabt, out_x);
 }
-// One launch for a sequence whose last chunk is ragged: complete-tile code for the complete chunks, the general code
-// for the last one (uniform per workgroup).
-template <int PT, bool IOB, bool DTB>
-__global__ __launch_bounds__(NTHREADS) void k_chunk_scan_mixed(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
-  if (decode_unit(p, xcd_remap(blockIdx.x, gridDim.x)).c == p.nc - 1) k_chunk_scan_body<PT, IOB, DTB, false>(p, states, cabt, out_x);
-  else k_chunk_scan_body<PT, IOB, DTB, true>(p, states, cabt, out_x);
-}
-
 
 // ------------------------------------------------------------------- launchers
 template <typename K>
@@ -389,14 +392,14 @@ static int set_lds(K kernel, size_t bytes) {
 bool local_tile_available(const KP& p, const float* states, const float* cabt);
 int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st);
 
-// Launches made of complete tiles go to the row-lane kernel (which itself falls back to the level-hierarchy body for
-// the chunks outside its range); everything else to the level-hierarchy kernel.
+// The row-lane kernel takes what it can (it falls back to the level-hierarchy body itself for the chunks outside its
+// range); packed sequences and calls that want one output only go to the level-hierarchy kernel.
 int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
   if (local_tile_available(p, states, cabt)) return launch_local_tile(p, states, cs_last, cabt, st);
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     const size_t sm = sizeof(FwdLocalSmem<PT_, !IOB_>);
-    constexpr auto kern = MIXED_ ? &k_chunk_local_mixed<PT_, IOB_, DTB_> : &k_chunk_local<PT_, IOB_, DTB_, FULL_>;
+    constexpr auto kern = &k_chunk_local<PT_, IOB_, DTB_, FULL_>;
     if (int e = set_lds(kern, sm)) return e;
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);
   });
@@ -406,14 +409,13 @@ int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, 
 int launch_state_fwd(const KP& p, float* states, const float* cs_last, hipStream_t st) {
   const long total = (long)p.B * p.ndir * p.H * p.P * ((p.N + 3) / 4);
   const int blocks = (int)((total + NTHREADS - 1) / NTHREADS);
-  if ((p.N & 3) == 0) {
-    if (total < (1L << 17) && p.nc >= 16)
-      hipLaunchKernelGGL(k_state_fwd_full<8>, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last);
-    else
-      hipLaunchKernelGGL(k_state_fwd_full<4>, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last);
-  } else {
-    hipLaunchKernelGGL(k_state_fwd, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last);
-  }
+#define ISSM_STATE_FWD(D_, TAIL_) \
+  hipLaunchKernelGGL((k_state_fwd_full<D_, TAIL_>), dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last)
+  const bool few = total < (1L << 17) && p.nc >= 16;
+  if (p.N < 4) hipLaunchKernelGGL(k_state_fwd, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last);
+  else if (p.N & 3) { if (few) ISSM_STATE_FWD(8, true); else ISSM_STATE_FWD(4, true); }
+  else { if (few) ISSM_STATE_FWD(8, false); else ISSM_STATE_FWD(4, false); }
+#undef ISSM_STATE_FWD
   return (int)hipGetLastError();
 }
 
@@ -421,7 +423,7 @@ int launch_chunk_scan(const KP& p, const float* states, const float* cabt, float
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     const size_t sm = sizeof(FwdScanSmem<PT_, IOB_>);
-    constexpr auto kern = MIXED_ ? &k_chunk_scan_mixed<PT_, IOB_, DTB_> : &k_chunk_scan<PT_, IOB_, DTB_, FULL_>;
+    constexpr auto kern = &k_chunk_scan<PT_, IOB_, DTB_, FULL_>;
     if (int e = set_lds(kern, sm)) return e;
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cabt, out_x);
   });

@@ -1,5 +1,5 @@
 // k_local_tile: the chunk-local pass of the forward (dt transform, running sums, chunk end states S_c, intra-chunk
-// matrix M_c, the chunk's total decay) for complete 64 x 64 tiles, in a ROW-lane layout.
+// matrix M_c, the chunk's total decay) in a ROW-lane layout.
 //
 // Lane (i, kg) of a wave owns row i of every 16-row tile of the chunk and four adjacent state columns
 // n = n0 + 4 kg .. + 3: exactly the operand layout of v_mfma_f32_16x16x16_bf16 for a contraction over the state
@@ -92,9 +92,13 @@ __device__ __forceinline__ f4 frag_product(const Frag<SPLIT>& a, const Frag<SPLI
   return mfma_bf16k(a.h, b.h, acc);
 }
 
+// Four adjacent elements at any element offset (one wide access: unaligned ones are legal on this target).
+struct __attribute__((packed, aligned(2))) Bf4Any {
+  unsigned x, y;
+};
 template <bool BF>
 struct RawVec {
-  typedef typename std::conditional<BF, uint2, f4>::type type;
+  typedef typename std::conditional<BF, Bf4Any, F4Any>::type type;
 };
 template <bool BF>
 __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, float* out) {
@@ -104,11 +108,15 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
     out[2] = __uint_as_float(r.y << 16);
     out[3] = __uint_as_float(r.y & 0xffff0000u);
   } else {
-    out[0] = r[0]; out[1] = r[1]; out[2] = r[2]; out[3] = r[3];
+    out[0] = r.x; out[1] = r.y; out[2] = r.z; out[3] = r.w;
   }
 }
 
-template <int PT, bool IOB, bool DTB, bool FULLP>
+// FULLP: the head dimension fills its tiles.  EDGE: chunks with fewer than 64 rows and steps with fewer than 64 columns
+// exist (N >= 4).  A lane's rows past the end read the chunk's last one and get dt' = 0, as do whole lanes past the last
+// column; a lane whose four columns cross it works on columns N - 4 .. N - 1 instead, those its neighbour owns with dt' = 0
+// and not stored.
+template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -132,36 +140,48 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   // tile J lies 16 J rows further along the scan, the step's columns 64 further along the row
   const int tl = u.dir ? p.L - 1 - u.c * CS - i : u.c * CS + i;   // the lane's token of tile 0
   const int sgn = u.dir ? -1 : 1;
+  const int nvalid = EDGE ? min(CS, p.L - u.c * CS) : CS;
   const int ncol = 16 * w + 4 * kg;                                // the lane's first column within a step
   const TDt* qdt = (const TDt*)p.dt.ptr + ((long)u.b * p.dt.s0 + (long)u.h * p.dt.s2);
   const TIo* qB = (const TIo*)p.Bm[u.dir].ptr + ((long)u.b * p.Bm[u.dir].s0 + (long)u.g * p.Bm[u.dir].s2);
   const TIo* qC = (const TIo*)p.Cm[u.dir].ptr + ((long)u.b * p.Cm[u.dir].s0 + (long)u.g * p.Cm[u.dir].s2);
-  const unsigned odt = (unsigned)(tl * (int)p.dt.s1 + ncol), oB = (unsigned)(tl * (int)p.Bm[u.dir].s1 + ncol),
-                 oC = (unsigned)(tl * (int)p.Cm[u.dir].s1 + ncol);
-  const int jdt = sgn * 16 * (int)p.dt.s1, jB = sgn * 16 * (int)p.Bm[u.dir].s1, jC = sgn * 16 * (int)p.Cm[u.dir].s1;
-  const float* qA = p.A + u.h * p.N + ncol;
-  const float* qbias = (p.dt_bias ? p.dt_bias : p.A) + u.h * p.N + ncol;  // without a bias: any valid address, scaled by 0
+  // element offsets of the lane's rows.  Complete tiles: tile J lies a uniform distance behind tile 0, so one register per
+  // tensor; otherwise a row past the end is the chunk's last one, and each tile has its own.
+  const int sdt = (int)p.dt.s1, sB = (int)p.Bm[u.dir].s1, sC = (int)p.Cm[u.dir].s1;
+  constexpr int NO = EDGE ? 4 : 1;
+  unsigned odt[NO], oB[NO], oC[NO];
+#pragma unroll
+  for (int J = 0; J < NO; ++J) {
+    const int t = EDGE ? tl + sgn * (min(16 * J + i, nvalid - 1) - i) : tl;
+    odt[J] = (unsigned)(t * sdt + (EDGE ? 0 : ncol));
+    oB[J] = (unsigned)(t * sB + (EDGE ? 0 : ncol));
+    oC[J] = (unsigned)(t * sC + (EDGE ? 0 : ncol));
+  }
+  const int jdt = EDGE ? 0 : sgn * 16 * sdt, jB = EDGE ? 0 : sgn * 16 * sB, jC = EDGE ? 0 : sgn * 16 * sC;
+  const float* qA = p.A + u.h * p.N;
+  const float* qbias = (p.dt_bias ? p.dt_bias : p.A) + u.h * p.N;  // without a bias: any valid address, scaled by 0
   const float bias_on = p.dt_bias ? 1.0f : 0.0f;
 
   RawDt rdt[4];
   RawIo rB[4], rC[4];
-  f4 rA, rbias;
+  F4Any rA, rbias;
 #define ISSM_REQUEST(n0_)                                                              \
   {                                                                                    \
+    const int c_ = EDGE ? min((n0_) + ncol, p.N - 4) : (n0_);                          \
     _Pragma("unroll") for (int J = 0; J < 4; ++J) {                                    \
-      rdt[J] = *(const RawDt*)(qdt + (int)(odt + (unsigned)(J * jdt + (n0_))));        \
-      rB[J] = *(const RawIo*)(qB + (int)(oB + (unsigned)(J * jB + (n0_))));            \
-      rC[J] = *(const RawIo*)(qC + (int)(oC + (unsigned)(J * jC + (n0_))));            \
+      rdt[J] = *(const RawDt*)(qdt + (int)(odt[J % NO] + (unsigned)(J * jdt + c_)));   \
+      rB[J] = *(const RawIo*)(qB + (int)(oB[J % NO] + (unsigned)(J * jB + c_)));       \
+      rC[J] = *(const RawIo*)(qC + (int)(oC[J % NO] + (unsigned)(J * jC + c_)));       \
     }                                                                                  \
-    rA = *(const f4*)(qA + (n0_));                                                     \
-    rbias = *(const f4*)(qbias + (n0_));                                               \
+    rA = *(const F4Any*)(qA + (EDGE ? c_ : c_ + ncol));                                \
+    rbias = *(const F4Any*)(qbias + (EDGE ? c_ : c_ + ncol));                          \
   }
   ISSM_REQUEST(0);
 
   // the unit's x tile, transposed, as bf16 (hi, lo) in LDS (its loads travel together with the first step's above)
   {
     float xv[CS * PT * 16 / NTHREADS];
-    lp_load<IOB, PT, true>(p, u, p.x[u.dir], xv);
+    lp_load<IOB, PT, !EDGE>(p, u, p.x[u.dir], xv);
     lp_store_split_t<PT, LDT, SPLIT>(xv, s.xt_hi, s.xt_lo);
   }
 
@@ -196,14 +216,23 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       unpack4<IOB>(rB[J], bv + 4 * J);
       unpack4<IOB>(rC[J], cv + 4 * J);
     }
-    float A2[4], bias[4];
+    const float A2[4] = {rA.x * LOG2E, rA.y * LOG2E, rA.z * LOG2E, rA.w * LOG2E};
+    const float bias[4] = {rbias.x * bias_on, rbias.y * bias_on, rbias.z * bias_on, rbias.w * bias_on};
+    // the lane's columns this step: c .. c + 3, of which the first `skip` are not its own
+    const int c = EDGE ? min(n0 + ncol, p.N - 4) : n0 + ncol, skip = EDGE ? n0 + ncol - c : 0;
+    auto put = [&](float* q, f4 v) {   // q: where column c goes
+      if constexpr (!EDGE) {
+        *(f4*)q = v;
+      } else if (skip == 0) {
+        st_f4_any(q, v);
+      } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      A2[r] = rA[r] * LOG2E;
-      bias[r] = rbias[r] * bias_on;
-    }
+        for (int j = 1; j < 4; ++j)
+          if (j >= skip) q[j] = v[j];
+      }
+    };
     {  // branch-free: the last step asks for its own columns once more
-      const int nn = min(n0 + NS, p.N - NS);
+      const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
       ISSM_REQUEST(nn);
     }
 
@@ -214,6 +243,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
       for (int k = 0; k < 16; ++k) pre[k] = dtv[k] + bias[k & 3];
       dt_transform<false, 16>(p, pre, dtp, dummy);
+      if constexpr (EDGE) {
+        if (nvalid < CS || n0 + NS > p.N) {  // uniform
+#pragma unroll
+          for (int k = 0; k < 16; ++k) {
+            const bool past = 16 * (k >> 2) + i >= nvalid;
+            if (past || (k & 3) < skip) dtp[k] = 0.0f;
+            if (past) cv[k] = 0.0f;   // (rows of M past the end come out as zero)
+          }
+        }
+      }
     }
     float pc[16], up[16], et[16];
 #pragma unroll
@@ -232,7 +271,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         tot[r] = __shfl((((pc[r] + pc[4 + r]) + pc[8 + r]) + pc[12 + r]) * LN2, last_lane, 64);
-      *(f4*)(cdst + n0 + ncol) = tot;
+      put(cdst + c, tot);
     }
 
     // ---- operands
@@ -306,11 +345,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     // S^T block: lane (p = i, kg) holds columns n0 + ncol .. + 3 of state row 16 pt + i
     if (FULLP) {  // every state row exists: plain stores (see the note at the chunk's total decay)
 #pragma unroll
-      for (int pt = 0; pt < PT; ++pt) *(f4*)(sdst + (16 * pt + i) * p.N + n0 + ncol) = sacc[pt];
+      for (int pt = 0; pt < PT; ++pt) put(sdst + (16 * pt + i) * p.N + c, sacc[pt]);
     } else {
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt)
-        if (16 * pt + i < p.P) *(f4*)(sdst + (16 * pt + i) * p.N + n0 + ncol) = sacc[pt];
+        if (16 * pt + i < p.P) put(sdst + (16 * pt + i) * p.N + c, sacc[pt]);
     }
   }
 #undef ISSM_REQUEST
@@ -349,23 +388,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     // such limit.  The fence orders this workgroup's stores above before the ones the other form makes to the same places.
     __threadfence();
     __syncthreads();
-    k_chunk_local_body<PT, IOB, DTB, true>(p, states, cs_last, cabt);
+    k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
   }
 }
 
-// Whether the row-lane kernel can take the launch: complete tiles everywhere, both outputs wanted, and every operand
-// addressable with 16-byte (fp32) / 8-byte (bf16) accesses.
+// Whether the row-lane kernel takes the launch: both outputs wanted, four columns to work on, no packed sequences (their
+// cuts are outside the form's range).
 bool local_tile_available(const KP& p, const float* states, const float* cabt) {
-  if (p.full_tiles != 1 || !states || !cabt) return false;
-  auto vec_ok = [](const TensorD& t, int bf) {
-    return ((t.s0 | t.s1 | t.s2) & 3) == 0 && (((uintptr_t)t.ptr) & (bf ? 7 : 15)) == 0;
-  };
-  if (!vec_ok(p.dt, p.dt_dt)) return false;
-  for (int d = 0; d < p.ndir; ++d)
-    if (!vec_ok(p.Bm[d], p.io_dt) || !vec_ok(p.Cm[d], p.io_dt)) return false;
-  if ((((uintptr_t)p.A) & 15) || (p.dt_bias && (((uintptr_t)p.dt_bias) & 15))) return false;
-  if ((((uintptr_t)states) & 15) || (p.N & 63)) return false;
-  return true;
+  return !p.seq_idx && p.N >= 4 && states && cabt;
 }
 
 template <typename K>
@@ -376,18 +406,20 @@ static int set_lds_tile(K kernel, size_t bytes) {
 int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
   const int units = p.B * p.ndir * p.nc * p.H;
   const int pt = (p.P + 15) / 16;
+  // aligned 16-byte stores of the states and decay totals need rows of a multiple of four floats: they have them where
+  // the tiles are complete
+#define ISSM_LT_ONE(PT_, IOB_, DTB_, FULLP_, EDGE_)                                                         \
+  {                                                                                                         \
+    constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, FULLP_, EDGE_>;                                    \
+    if (int e = set_lds_tile(kern, sm)) return e;                                                           \
+    hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);                \
+  }
 #define ISSM_LT(PT_, IOB_, DTB_)                                                                            \
   {                                                                                                         \
     const size_t sm = fwd_tile_lds<PT_, !IOB_>();                                                           \
-    if (p.P == 16 * PT_) {                                                                                  \
-      constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, true>;                                           \
-      if (int e = set_lds_tile(kern, sm)) return e;                                                         \
-      hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);              \
-    } else {                                                                                                \
-      constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, false>;                                          \
-      if (int e = set_lds_tile(kern, sm)) return e;                                                         \
-      hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);              \
-    }                                                                                                       \
+    if (!p.full_tiles || ((uintptr_t)states & 15) || ((uintptr_t)cs_last & 15)) ISSM_LT_ONE(PT_, IOB_, DTB_, false, true) \
+    else if (p.P == 16 * PT_) ISSM_LT_ONE(PT_, IOB_, DTB_, true, false)                                     \
+    else ISSM_LT_ONE(PT_, IOB_, DTB_, false, false)                                                         \
   }
 #define ISSM_LT_DT(PT_)                                                      \
   {                                                                          \
@@ -400,6 +432,7 @@ int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, h
   if (pt <= 2) ISSM_LT_DT(2) else if (pt == 3) ISSM_LT_DT(3) else ISSM_LT_DT(4)
 #undef ISSM_LT_DT
 #undef ISSM_LT
+#undef ISSM_LT_ONE
   return (int)hipGetLastError();
 }
 

@@ -135,6 +135,44 @@ def test_operator_fp32_matches_oracle(case):
         _check("d" + k, g[k], g_ref[k], BWD32)
 
 
+@pytest.mark.parametrize("dtype,L_,N,P,strong", [
+    (torch.float32, 63, 1, 4, False), (torch.float32, 65, 3, 16, False), (torch.float32, 5, 4, 20, False),
+    (torch.float32, 127, 5, 8, False), (torch.float32, 129, 63, 36, False), (torch.float32, 200, 66, 32, True),
+    (torch.float32, 191, 130, 64, True), (torch.bfloat16, 2, 6, 16, False), (torch.bfloat16, 100, 67, 36, True),
+    (torch.bfloat16, 129, 125, 32, False), (torch.bfloat16, 66, 191, 48, True), (torch.bfloat16, 193, 128, 24, True)])
+def test_rows_and_columns_that_fill_no_tile_in_both_directions(dtype, L_, N, P, strong):
+    """Edges of chunks, column slices and column quads, both directions (the reversed one has its absent rows before the
+    first token); `strong`: one head decays by more than the per-tile form holds."""
+    from dest3d_amd import ISSM_biscan_combined
+    _say(f"edges {dtype} L={L_} N={N} P={P} strong={strong}")
+    d = _problem(2, L_, 2, P, N, 1, seed=L_ * N + P)
+    if strong:
+        d["A"][0] *= 12.0
+    g = torch.Generator().manual_seed(L_)
+    two = {k + "_b": torch.randn(d[k].shape, generator=g) * (1.0 if k == "x" else N ** -0.5) for k in ("x", "B", "C")}
+    d.update(two)
+    lead = ("x", "x_b", "dt", "B", "B_b", "C", "C_b")
+    for k in lead:
+        d[k] = d[k].to(dtype).float()
+    w = [torch.randn(d["x"].shape, generator=g), torch.randn(d["x"].shape, generator=g), torch.randn(d["h0"].shape, generator=g),
+         torch.randn(d["h0"].shape, generator=g)]
+    names = (*lead, "A", "D", "dt_bias", "h0")
+    call = lambda f, t, **kw: f(t["x"], t["x_b"], t["dt"], t["A"], t["B"], t["B_b"], t["C"], t["C_b"], D=t["D"], dt_bias=t["dt_bias"],
+                                initial_states=t["h0"], dt_softplus=True, dt_limit=d["dt_limit"], **kw)
+    ref = {k: d[k].double().requires_grad_() for k in names}
+    o_ref = call(R.issm_biscan_ref, ref)
+    torch.autograd.backward(o_ref, [t.double() for t in w])
+    gi = {k: d[k].cuda().to(dtype if k in lead else torch.float32).requires_grad_() for k in names}
+    o = call(lambda *a, **kw: ISSM_biscan_combined(*a, 64, **kw), gi)
+    torch.autograd.backward(o, [t.cuda().to(q.dtype) for t, q in zip(w, o)])
+    torch.cuda.synchronize()
+    fwd, bwd = (FWD32, BWD32) if dtype == torch.float32 else (FWD16, BWD16)
+    for n_, a, b in zip(("y_f", "y_b", "last_f", "last_b"), o, o_ref):
+        _check(n_, a, b, fwd)
+    for k in names:
+        _check("d" + k, gi[k].grad, ref[k].grad, bwd)
+
+
 @pytest.mark.parametrize("P", [128, 96, 67])
 def test_head_dimension_above_the_tile_limit(P):
     """Heads wider than the kernels' 64 run as several narrower heads that share dt, A, dt_bias and the group's B, C
