@@ -33,7 +33,8 @@ EXPORTS = [
     "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states",
     "issm_pn2_furthest_point_sampling", "issm_pn2_ball_query", "issm_pn2_group_points", "issm_pn2_group_points_grad",
     "issm_pn2_gather_points", "issm_pn2_gather_points_grad", "issm_pn2_three_nn", "issm_pn2_three_interpolate",
-    "issm_pn2_three_interpolate_grad", "issm_pn2_group_points_grad_cl", "issm_pn2_three_interpolate_grad_cl",
+    "issm_pn2_three_interpolate_grad", "issm_pn2_group_xyz_points", "issm_pn2_group_points_grad_rows",
+    "issm_pn2_three_interpolate_grad_rows", "issm_pn2_three_interpolate_grad_rows_workspace", "issm_pn2_group_points_grad_cl", "issm_pn2_three_interpolate_grad_cl",
 ]
 
 
@@ -207,6 +208,11 @@ def load() -> C.CDLL:
     lib.issm_pn2_three_nn.argtypes = [i32, i32, i32, vp, vp, vp, vp, vp]
     lib.issm_pn2_three_interpolate.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp]
     lib.issm_pn2_three_interpolate_grad.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp]
+    lib.issm_pn2_group_xyz_points.argtypes = [i32, i32, i32, i32, i32, vp, vp, f32, vp, vp, vp, vp]
+    lib.issm_pn2_group_points_grad_rows.argtypes = [i32, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp]
+    lib.issm_pn2_three_interpolate_grad_rows.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp, vp]
+    lib.issm_pn2_three_interpolate_grad_rows_workspace.argtypes = [i32, i32, i32]
+    lib.issm_pn2_three_interpolate_grad_rows_workspace.restype = C.c_int64
     lib.issm_pn2_group_points_grad_cl.argtypes = [i32, i32, i32, i32, i32, vp, vp, vp, vp]
     lib.issm_pn2_three_interpolate_grad_cl.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp]
     lib.issm_box_dist_fwd.argtypes = [P(BoxDistArgs)]

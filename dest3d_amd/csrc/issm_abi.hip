@@ -45,7 +45,13 @@ int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
                       hipStream_t st);
-int launch_group_points(int b, int c, int n, int ms, const float* points, const int* idx, float* out, hipStream_t st);
+int launch_group_points(int b, int c, int n, int npoints, int nsample, const float* xyz, const float* centre, float scale,
+                        const float* points, const int* idx, float* out, hipStream_t st);
+int launch_group_rows_grad(int b, int c, int c0, int cdim, int n, int ms, const float* grad_out, const int* idx,
+                           float* grad_points, hipStream_t st);
+int launch_interp_rows_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight, int* ws,
+                            float* grad_points, hipStream_t st);
+long interp_rows_grad_ints(int b, int n, int m);
 int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out, const int* idx, float* grad_points,
                              hipStream_t st);
 int launch_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2, int* idx, hipStream_t st);
@@ -835,7 +841,33 @@ int issm_pn2_group_points(int32_t b, int32_t c, int32_t n, int32_t npoints, int3
   if (n == 0) return fail(ISSM_E_SHAPE, "group_points: no points to index");
   if ((int64_t)npoints * nsample > 0x7fffffff) return fail(ISSM_E_SHAPE, "group_points: too many indices per sample");
   PN2_PTRS("group_points", points, idx, out);
-  return launched(launch_group_points(b, c, n, npoints * nsample, points, idx, out, (hipStream_t)stream), "group_points");
+  return launched(launch_group_points(b, c, n, npoints, nsample, nullptr, nullptr, 0.0f, points, idx, out, (hipStream_t)stream),
+                  "group_points");
+}
+
+int issm_pn2_group_xyz_points(int32_t b, int32_t c, int32_t n, int32_t npoints, int32_t nsample, const float* xyz,
+                              const float* new_xyz, float scale, const float* points, const int32_t* idx, float* out,
+                              void* stream) {
+  PN2_SIZES("group_xyz_points", b, c, n, npoints, nsample);
+  if ((int64_t)b * npoints * nsample == 0) return ISSM_OK;
+  if (n == 0) return fail(ISSM_E_SHAPE, "group_xyz_points: no points to index");
+  if ((int64_t)npoints * nsample > 0x7fffffff) return fail(ISSM_E_SHAPE, "group_xyz_points: too many indices per sample");
+  PN2_PTRS("group_xyz_points", xyz, new_xyz, idx, out);
+  if (c > 0 && !points) return fail(ISSM_E_NULL, "group_xyz_points: points is NULL");
+  return launched(launch_group_points(b, c, n, npoints, nsample, xyz, new_xyz, scale, points, idx, out, (hipStream_t)stream),
+                  "group_xyz_points");
+}
+
+int issm_pn2_group_points_grad_rows(int32_t b, int32_t c, int32_t c0, int32_t cdim, int32_t n, int32_t npoints, int32_t nsample,
+                                    const float* grad_out, const int32_t* idx, float* grad_points, void* stream) {
+  PN2_SIZES("group_points_grad_rows", b, c, c0, cdim, n, npoints, nsample);
+  if ((int64_t)b * c * npoints * nsample == 0) return ISSM_OK;
+  if (n == 0 || (int64_t)c0 + c > cdim) return fail(ISSM_E_SHAPE, "group_points_grad_rows: no points, or channels beyond grad_out's");
+  if (n > ISSM_PN2_ROW_POINTS || (int64_t)npoints * nsample > 0x7fffffff || (int64_t)b * c > 0x7fffffff / 1024)
+    return fail(ISSM_E_UNSUPPORTED, "group_points_grad_rows: n = %d > %d, or too many indices or rows", n, ISSM_PN2_ROW_POINTS);
+  PN2_PTRS("group_points_grad_rows", grad_out, idx, grad_points);
+  return launched(launch_group_rows_grad(b, c, c0, cdim, n, npoints * nsample, grad_out, idx, grad_points, (hipStream_t)stream),
+                  "group_points_grad_rows");
 }
 
 int issm_pn2_group_points_grad(int32_t b, int32_t c, int32_t n, int32_t npoints, int32_t nsample, const float* grad_out,
@@ -886,6 +918,23 @@ int issm_pn2_three_interpolate_grad(int32_t b, int32_t c, int32_t n, int32_t m, 
   PN2_PTRS("three_interpolate_grad", grad_out, idx, weight, grad_points);
   return launched(launch_three_interpolate_grad(b, c, n, m, grad_out, idx, weight, grad_points, (hipStream_t)stream),
                   "three_interpolate_grad");
+}
+
+int64_t issm_pn2_three_interpolate_grad_rows_workspace(int32_t b, int32_t n, int32_t m) {
+  return b < 0 || n < 0 || m < 0 ? 0 : (int64_t)sizeof(int) * interp_rows_grad_ints(b, n, m);
+}
+
+int issm_pn2_three_interpolate_grad_rows(int32_t b, int32_t c, int32_t n, int32_t m, const float* grad_out, const int32_t* idx,
+                                         const float* weight, void* workspace, float* grad_points, void* stream) {
+  PN2_SIZES("three_interpolate_grad_rows", b, c, n, m);
+  if ((int64_t)b * c * n == 0) return ISSM_OK;
+  if (m == 0) return fail(ISSM_E_SHAPE, "three_interpolate_grad_rows: no points to index");
+  if (n > ISSM_PN2_ROW_POINTS || m > ISSM_PN2_ROW_POINTS || b > 65535)
+    return fail(ISSM_E_UNSUPPORTED, "three_interpolate_grad_rows: n = %d or m = %d > %d, or batch > 65535", n, m, ISSM_PN2_ROW_POINTS);
+  PN2_PTRS("three_interpolate_grad_rows", grad_out, idx, weight, workspace, grad_points);
+  if ((uintptr_t)workspace & 7) return fail(ISSM_E_STRIDE, "three_interpolate_grad_rows: workspace is not aligned to 8 bytes");
+  return launched(launch_interp_rows_grad(b, c, n, m, grad_out, idx, weight, (int*)workspace, grad_points, (hipStream_t)stream),
+                  "three_interpolate_grad_rows");
 }
 
 int issm_pn2_group_points_grad_cl(int32_t b, int32_t c, int32_t n, int32_t npoints, int32_t nsample, const float* grad_out,

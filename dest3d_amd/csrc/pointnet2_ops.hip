@@ -7,16 +7,22 @@
 //    coordinates are re-read and distances kept in the caller's `temp`.  Ties go to the smaller index.
 //  * ball query: one wave per query centre; 64 points are tested per step and compacted in index order with a
 //    ballot, so the first `nsample` hits are found without a serial scan; the wave stops as soon as it has them.
-//  * 3-NN: one thread per unknown point, known points staged through LDS 256 at a time.
-//  * group / gather / interpolate: one thread per output element, innermost index fastest; the gradients scatter
-//    with hardware float atomics (duplicates in idx are the rule), as the reference does -- either straight into
-//    the (b, c, n) layout, one scattered cache line per lane, or (the *_cl entry points) into a channel-last
+//  * 3-NN: one thread per unknown point; 256 to 8192 known points are sorted into a grid in LDS of which a thread looks at
+//    the cells around its point, fewer or more are staged through LDS 256 at a time and all looked at.
+//  * group / interpolate and their gradients: whole rows (one channel's points) live in LDS, the indices of a sample stream
+//    past them; gradients are summed there and written once.  Rows too long for LDS, and gathers of fewer entries than a
+//    row has points, take one thread per output element; their gradients scatter with hardware float atomics -- either
+//    straight into the (b, c, n) layout, one scattered cache line per lane, or (the *_cl entry points) into a channel-last
 //    (b, n, c) buffer through an LDS transpose, 64 consecutive floats per instruction.
+#include <algorithm>
 #include <type_traits>
 
 #include "issm_dev.h"
 
 namespace issm {
+
+constexpr int ROW_POINTS = 40960;     // points of a row that fit in a CU's 160 KB of LDS
+constexpr int INTERP_POINTS = 10240;  // of four rows
 
 constexpr int FPS_T = 512;    // threads of the sampling workgroup (two waves per SIMD: 256 registers each)
 
@@ -319,16 +325,176 @@ __global__ __launch_bounds__(NTHREADS) void k_ball_query(int n, int m, float rad
   for (int s = cnt + lane; s < nsample; s += 64) out[s] = first;  // first == 0 when nothing was found
 }
 
-// out[b][c][j][s] = points[b][c][idx[b][j][s]]   (one thread per output element)
-__global__ __launch_bounds__(NTHREADS) void k_group_points(long total, int c, int n, int ms, const float* __restrict__ points,
-                                                           const int* __restrict__ idx, float* __restrict__ out) {
+// Grouping.  Output channel ch < cx (cx = 0 or 3): coordinate ch of the point relative to the entry's centre, times `scale`;
+// then the c feature channels.
+struct GroupP {
+  int c, cx, n, ms, npoints, nsample, rows;   // rows: of the whole batch
+  long share;
+  const float *xyz, *centre, *points;
+  const int* idx;
+  float* out;
+  float scale;
+};
+__device__ __forceinline__ int index_of(int v, int n) { return min(max(v, 0), n - 1); }  // a stray index must not leave the tensor
+struct __attribute__((packed, aligned(4))) I4Any {
+  int v[4];
+};
+// Values read or written once, past the caches' replacement order: the indices, read again for every row, stay in L2.
+typedef float f4_stream __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f4 ld_stream(const float* q) { return __builtin_nontemporal_load((const f4_stream*)q); }
+__device__ __forceinline__ void st_stream(float* q, f4 v) { __builtin_nontemporal_store((f4_stream)v, (f4_stream*)q); }
+
+// One thread per output element.
+__global__ __launch_bounds__(NTHREADS) void k_group_points(GroupP g) {
+  const int e = blockIdx.x * NTHREADS + threadIdx.x;
+  if (e >= g.ms) return;
+  const int rows = g.cx + g.c;
+  for (int row = blockIdx.y; row < g.rows; row += gridDim.y) {
+    const int b = row / rows, ch = row % rows;
+    const int k = index_of(g.idx[(long)b * g.ms + e], g.n);
+    float v;
+    if (ch < g.cx) v = (g.xyz[((long)b * g.n + k) * 3 + ch] - g.centre[((long)b * g.npoints + e / g.nsample) * 3 + ch]) * g.scale;
+    else v = g.points[((long)b * g.c + ch - g.cx) * g.n + k];
+    g.out[(long)row * g.ms + e] = v;
+  }
+}
+
+// The output's entries, row after row, in equal shares of one workgroup each; of every row it meets, a workgroup holds the
+// n source values in LDS and streams the indices past them, four entries per thread and step.  (A workgroup per row left a
+// third of the time to the last few rows: 1048 rows on 512 places.)  Bound by writing the output: 8 samples of 20000
+// points, 131 x 131072 entries each, 240 us (549 MB written:
+// 2.3 TB/s); separate gathers, a subtraction, a product and a concatenation took 656.
+__global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
+  extern __shared__ float srow[];
+  const int T = blockDim.x, tid = threadIdx.x, rows1 = g.cx + g.c;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x);   // an XCD's workgroups: neighbouring rows, one sample's indices in its L2
+  const long end = min((long)(wg + 1) * g.share, (long)g.rows * g.ms);
+  for (long at = (long)wg * g.share; at < end;) {
+    const int row = (int)(at / g.ms), b = row / rows1, ch = row % rows1;
+    const int lo = (int)(at - (long)row * g.ms), hi = (int)min((long)g.ms, lo + (end - at));
+    at += hi - lo;
+    __syncthreads();
+    if (ch < g.cx) {
+      const float* q = g.xyz + (long)b * g.n * 3 + ch;
+      for (int k = tid; k < g.n; k += T) srow[k] = q[k * 3];
+    } else {
+      const float* q = g.points + ((long)b * g.c + ch - g.cx) * g.n;
+      for (int k = 4 * tid; k + 3 < g.n; k += 4 * T) *(f4*)(srow + k) = ld_f4_any(q + k);
+      const int k = (g.n & ~3) + tid;
+      if (k < g.n) srow[k] = q[k];
+    }
+    __syncthreads();
+    const int* q = g.idx + (long)b * g.ms;
+    float* o = g.out + (long)row * g.ms;
+    for (int e = lo + 4 * tid; e < hi; e += 4 * T) {
+      const int cnt = min(hi - e, 4);
+      I4Any i = {};
+      if (cnt == 4) i = *(const I4Any*)(q + e);
+      else for (int j = 0; j < cnt; ++j) i.v[j] = q[e + j];
+      f4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = srow[index_of(i.v[j], g.n)];
+      if (ch < g.cx) {
+        // (one division per step: what a coordinate row costs beyond a feature row decides when its workgroup ends)
+        int at_c = (int)((unsigned)e / (unsigned)g.nsample), left = (at_c + 1) * g.nsample - e;
+        const float* cq = g.centre + ((long)b * g.npoints + at_c) * 3 + ch;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = (v[j] - *cq) * g.scale;
+          if (--left == 0 && e + j + 1 < hi) { cq += 3; left = g.nsample; }
+        }
+      }
+      if (cnt == 4) st_stream(o + e, v);
+      else
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (j < cnt) o[e + j] = v[j];
+    }
+  }
+}
+
+// A value from the lane N places before (SHR) or after (SHL) within the row of 16 lanes; `old` where there is none.
+template <int CTRL>
+__device__ __forceinline__ int row_lane(int old, int v) {
+  return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float row_lane_f(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// Gradient of the grouping, all of grad_points (b, c, n) written: one workgroup per channel row (and part of its entries),
+// the row's n sums in LDS, grad_out streamed once.  A ball with fewer points than slots repeats its first point, and 64
+// lanes adding to one LDS word take 64 turns: runs of equal indices are summed first -- four consecutive entries per lane,
+// then a segmented scan over the row of 16 lanes -- and only the last entry of a run adds.  Bound by reading grad_out:
+// with the mostly repeated indices of a 0.2 m ball
+// 144 us for those 537 MB (3.7 TB/s; atomics into a channel-last buffer: 592 and 190 for copies around them), with 64
+// different ones 684 us, the rate of LDS float additions to scattered words (before: 479 and 190).  With splits > 1 (few rows) the parts meet in grad_points, which is zero before.
+__global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdim, int n, int ms, int splits, int per,
+                                                          const float* __restrict__ grad_out, const int* __restrict__ idx,
+                                                          float* __restrict__ grad_points) {
+  extern __shared__ float srow[];
+  const int T = blockDim.x, tid = threadIdx.x, lane = tid & 63;
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), row = wg / splits, part = wg % splits, b = row / c, ch = row % c;
+  for (int k = tid; k < n; k += T) srow[k] = 0.0f;
+  __syncthreads();
+  const int* q = idx + (long)b * ms;
+  const float* g = grad_out + ((long)b * cdim + c0 + ch) * ms;
+  const int hi = min((part + 1) * per, ms);
+  for (int e0 = part * per + (tid >> 6) * 256; e0 < hi; e0 += 4 * T) {   // wave-uniform
+    const int e = e0 + 4 * lane;
+    I4Any i;
+    f4 v = {0, 0, 0, 0};
+    if (e + 4 <= hi) {
+      i = *(const I4Any*)(q + e);
+      v = ld_stream(g + e);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) i.v[j] = index_of(i.v[j], n);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        i.v[j] = -1;   // not an entry
+        if (e + j < hi) {
+          i.v[j] = index_of(q[e + j], n);
+          v[j] = g[e + j];
+        }
+      }
+    }
+    const bool q1 = i.v[1] == i.v[0], q2 = i.v[2] == i.v[1], q3 = i.v[3] == i.v[2];
+    v[1] += q1 ? v[0] : 0.0f;
+    v[2] += q2 ? v[1] : 0.0f;
+    v[3] += q3 ? v[2] : 0.0f;
+    // runs across lanes: s = sum of the run that ends at the lane's last entry; `on` = that run began in an earlier lane
+    const bool link = row_lane<0x111>(-2, i.v[3]) == i.v[0];
+    int on = q1 && q2 && q3 && link ? -1 : 0;
+    float s = v[3];
+    auto step = [&](auto ctrl) {
+      constexpr int C = decltype(ctrl)::value;
+      s += __builtin_bit_cast(float, __builtin_bit_cast(int, row_lane_f<C>(s)) & on);
+      on &= row_lane<C>(0, on);
+    };
+    step(std::integral_constant<int, 0x111>{});
+    step(std::integral_constant<int, 0x112>{});
+    step(std::integral_constant<int, 0x114>{});
+    step(std::integral_constant<int, 0x118>{});
+    const float before = row_lane_f<0x111>(s), carry = link ? before : 0.0f;
+    const bool end3 = row_lane<0x101>(-2, i.v[0]) != i.v[3];
+    if (!q1 && i.v[0] >= 0) unsafeAtomicAdd(srow + i.v[0], v[0] + carry);
+    if (!q2 && i.v[1] >= 0) unsafeAtomicAdd(srow + i.v[1], v[1] + (q1 ? carry : 0.0f));
+    if (!q3 && i.v[2] >= 0) unsafeAtomicAdd(srow + i.v[2], v[2] + (q1 && q2 ? carry : 0.0f));
+    if (end3 && i.v[3] >= 0) unsafeAtomicAdd(srow + i.v[3], v[3] + (q1 && q2 && q3 ? carry : 0.0f));
+  }
+  __syncthreads();
+  float* o = grad_points + (long)row * n;
+  if (splits == 1)
+    for (int k = tid; k < n; k += T) o[k] = srow[k];
+  else
+    for (int k = tid; k < n; k += T)
+      if (srow[k] != 0.0f) unsafeAtomicAdd(o + k, srow[k]);   // (NaN != 0)
+}
+__global__ __launch_bounds__(NTHREADS) void k_zero(long total, float* __restrict__ q) {
   const long e = (long)blockIdx.x * NTHREADS + threadIdx.x;
-  if (e >= total) return;
-  const int r = (int)(e % ms);
-  const long bc = e / ms;
-  const int b = (int)(bc / c);
-  const int k = min(max(idx[(long)b * ms + r], 0), n - 1);  // a stray index must not leave the tensor
-  out[e] = points[bc * n + k];
+  if (e < total) q[e] = 0.0f;
 }
 __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int c, int n, int ms,
                                                                 const float* __restrict__ grad_out,
@@ -342,7 +508,179 @@ __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int 
   unsafeAtomicAdd(grad_points + bc * n + k, grad_out[e]);
 }
 
-// 3 nearest known points of every unknown point: squared distances ascending, ties to the smaller index
+// 3 nearest known points of every unknown point: squared distances ascending, ties to the smaller index.
+//
+// 256 to 8192 known points: every workgroup sorts them (counting sort) into a uniform grid of about two points a cell in
+// LDS, 16 bytes a point; a thread visits the 27 cells around its point, rows of neighbouring cells as one range, and then
+// whatever else lies within its third distance (which shrinks on the way; rows beyond it are skipped).  The answer is that of
+// the pass over all points: distances are evaluated the same way, ordered by (distance, index), and cells are left out only
+// if their distance, shortened by far more than the rounding of cell numbers and distances, is above the third one.  Coordinates that
+// are not finite (or above 1e18) send the workgroup to the pass over all points.  20000 x 2048 points, 8 samples:
+// 258 us looking at all, 50 us here.
+constexpr int NN_T = 512, NN_CELLS = 4096;
+struct Nearest3 {
+  float d1, d2, d3;
+  int i1, i2, i3;
+  __device__ __forceinline__ void take(float d, int k) {
+    if (d > d3) return;   // (NaN goes on and fails every test below)
+    const bool a = d < d1 || (d == d1 && k < i1), m = d < d2 || (d == d2 && k < i2), z = d < d3 || (d == d3 && k < i3);
+    if (a) { d3 = d2; i3 = i2; d2 = d1; i2 = i1; d1 = d; i1 = k; }
+    else if (m) { d3 = d2; i3 = i2; d2 = d; i2 = k; }
+    else if (z) { d3 = d; i3 = k; }
+  }
+};
+__global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const float* __restrict__ unknown,
+                                                        const float* __restrict__ known, float* __restrict__ dist2,
+                                                        int* __restrict__ idx) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  float4* pts = (float4*)smem_raw;           // [m] x, y, z, index
+  int* end = (int*)(pts + m);                // [NN_CELLS + 1]: end[c + 1] = end of cell c's points, end[0] = 0
+  __shared__ float red[7][NN_T / 64];
+  __shared__ int wsum[NN_T / 64];
+  const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float INFV = __builtin_huge_valf();
+  const float* kp = known + (long)b * m * 3;
+  float lo[3] = {INFV, INFV, INFV}, hi[3] = {-INFV, -INFV, -INFV}, odd = 0.0f;
+  for (int k = tid; k < m; k += NN_T)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float v = kp[k * 3 + a];
+      if (!(fabsf(v) < 1e18f)) odd = 1.0f;
+      lo[a] = fminf(lo[a], v);
+      hi[a] = fmaxf(hi[a], v);
+    }
+  odd = wave_fmax(odd);
+  if (lane == 0) red[6][wave] = odd;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float l = -wave_fmax(-lo[a]), h = wave_fmax(hi[a]);
+    if (lane == 0) { red[a][wave] = l; red[3 + a][wave] = h; }
+  }
+  for (int c = tid; c <= NN_CELLS; c += NN_T) end[c] = 0;
+  __syncthreads();
+  odd = red[6][0];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) { lo[a] = red[a][0]; hi[a] = red[3 + a][0]; }
+#pragma unroll
+  for (int w = 1; w < NN_T / 64; ++w) {
+    odd = fmaxf(odd, red[6][w]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) { lo[a] = fminf(lo[a], red[a][w]); hi[a] = fmaxf(hi[a], red[3 + a][w]); }
+  }
+  // cells: cubes of side `side`, at most 32 along an axis and NN_CELLS in all
+  const float ext[3] = {hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]};
+  const float longest = fmaxf(fmaxf(ext[0], ext[1]), ext[2]);
+  float side = fmaxf(cbrtf(ext[0] * ext[1] * ext[2] * 2.0f / (float)m), longest * (1.0f / 32.0f));
+  if (!(side > 1e-30f)) side = 1.0f;   // all in one place
+  int g[3];
+  auto count_cells = [&]() {
+    for (int a = 0; a < 3; ++a) g[a] = min(max((int)(ext[a] / side) + 1, 1), 33);
+    return g[0] * g[1] * g[2];
+  };
+  while (count_cells() > NN_CELLS) side *= 1.25f;
+  const float inv = 1.0f / side;
+  auto cell1 = [&](float v, int a) { return min(max((int)((v - lo[a]) * inv), 0), g[a] - 1); };
+
+  const int j = blockIdx.x * NN_T + tid;
+  const bool live = j < n;
+  float ux = 0.0f, uy = 0.0f, uz = 0.0f;
+  if (live) {
+    const float* u = unknown + ((long)b * n + j) * 3;
+    ux = u[0]; uy = u[1]; uz = u[2];
+  }
+  Nearest3 best = {INFV, INFV, INFV, 0, 0, 0};
+  if (odd == 0.0f && longest < INFV) {   // uniform
+    for (int k = tid; k < m; k += NN_T)
+      atomicAdd(&end[1 + (cell1(kp[k * 3 + 2], 2) * g[1] + cell1(kp[k * 3 + 1], 1)) * g[0] + cell1(kp[k * 3], 0)], 1);
+    __syncthreads();
+    {  // exclusive prefix sum: NN_CELLS / NN_T neighbours per thread
+      constexpr int E = NN_CELLS / NN_T;
+      int own = 0;
+      for (int e = 0; e < E; ++e) own += end[1 + tid * E + e];
+      int incl = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
+      }
+      if (lane == 63) wsum[wave] = incl;
+      __syncthreads();
+      int at = incl - own;
+      for (int w = 0; w < wave; ++w) at += wsum[w];
+      for (int e = 0; e < E; ++e) { const int v = end[1 + tid * E + e]; end[1 + tid * E + e] = at; at += v; }
+    }
+    __syncthreads();
+    for (int k = tid; k < m; k += NN_T) {
+      const float x = kp[k * 3], y = kp[k * 3 + 1], z = kp[k * 3 + 2];
+      const int at = atomicAdd(&end[1 + (cell1(z, 2) * g[1] + cell1(y, 1)) * g[0] + cell1(x, 0)], 1);
+      pts[at] = make_float4(x, y, z, __builtin_bit_cast(float, k));
+    }
+    __syncthreads();
+    if (live) {
+      const int cx = cell1(ux, 0), cy = cell1(uy, 1), cz = cell1(uz, 2);
+      auto cells = [&](int x0, int x1, int y, int z) {   // cells x0 .. x1 of a row
+        const int c = (z * g[1] + y) * g[0];
+        const int e1 = end[c + x1 + 1];
+        for (int e = end[c + x0]; e < e1; ++e) {
+          const float4 p = pts[e];
+          best.take(sqdist(ux, uy, uz, p.x, p.y, p.z), __builtin_bit_cast(int, p.w));
+        }
+      };
+      // how near a point of cell row (y, z) can be, squared (0 if it may be nearer than the margin for rounding)
+      const float du[3] = {ux - lo[0], uy - lo[1], uz - lo[2]};
+      const float margin = 1e-4f * side;
+      auto gap = [&](float d, int c) {   // distance along one axis from d to cells' interval number c
+        const float q = fmaxf((float)c * side - d, d - (float)(c + 1) * side) * (1.0f - 1e-5f) - margin;
+        return q > 0.0f ? q * q : 0.0f;
+      };
+      // cells x0 .. x1 of row (y, z), unless every point of it is farther than the third one
+      auto row = [&](int x0, int x1, int y, int z) {
+        if (x0 <= x1 && !(gap(du[1], y) + gap(du[2], z) > best.d3)) cells(x0, x1, y, z);
+      };
+      int a0[3], a1[3];   // the cells visited so far: first the block around the point's own, its row first
+      const int cc[3] = {cx, cy, cz};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) { a0[a] = max(cc[a] - 1, 0); a1[a] = min(cc[a] + 1, g[a] - 1); }
+      for (int t = 0; t < 9; ++t) {
+        const int y = cy + (t == 0 || t == 3 || t == 6 ? 0 : t == 1 || t == 4 || t == 7 ? -1 : 1), z = cz + (t < 3 ? 0 : t < 6 ? -1 : 1);
+        if (y >= a0[1] && y <= a1[1] && z >= a0[2] && z <= a1[2]) row(a0[0], a1[0], y, z);
+      }
+      for (int r = 2;; r *= 2) {
+        // everything within the third distance, if there is one: after that nothing is left to see.  Else a larger block.
+        const bool three = best.d3 < INFV;
+        const float reach = three ? sqrtf(best.d3) * (1.0f + 1e-5f) + margin : 0.0f;
+        int b0[3], b1[3];
+        bool same = true;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          b0[a] = three ? min(max((int)((du[a] - reach) * inv), 0), a0[a]) : max(cc[a] - r, 0);
+          b1[a] = three ? max(min((int)fminf((du[a] + reach) * inv, 64.0f), g[a] - 1), a1[a]) : min(cc[a] + r, g[a] - 1);
+          same = same && b0[a] == a0[a] && b1[a] == a1[a];
+        }
+        if (!same)
+          for (int z = b0[2]; z <= b1[2]; ++z)
+            for (int y = b0[1]; y <= b1[1]; ++y) {
+              const bool seen = y >= a0[1] && y <= a1[1] && z >= a0[2] && z <= a1[2];
+              row(b0[0], seen ? a0[0] - 1 : b1[0], y, z);
+              if (seen) row(a1[0] + 1, b1[0], y, z);
+            }
+        if (three || (b0[0] == 0 && b0[1] == 0 && b0[2] == 0 && b1[0] == g[0] - 1 && b1[1] == g[1] - 1 && b1[2] == g[2] - 1)) break;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) { a0[a] = b0[a]; a1[a] = b1[a]; }
+      }
+    }
+  } else if (live) {
+    for (int k = 0; k < m; ++k) best.take(sqdist(ux, uy, uz, kp[k * 3], kp[k * 3 + 1], kp[k * 3 + 2]), k);
+  }
+  if (live) {
+    float* dd = dist2 + ((long)b * n + j) * 3;
+    int* ii = idx + ((long)b * n + j) * 3;
+    dd[0] = best.d1; dd[1] = best.d2; dd[2] = best.d3;
+    ii[0] = best.i1; ii[1] = best.i2; ii[2] = best.i3;
+  }
+}
+
+// Any number of known points.
 __global__ __launch_bounds__(NTHREADS) void k_three_nn(int n, int m, const float* __restrict__ unknown,
                                                        const float* __restrict__ known, float* __restrict__ dist2,
                                                        int* __restrict__ idx) {
@@ -413,6 +751,137 @@ __global__ __launch_bounds__(NTHREADS) void k_three_interpolate_grad(long total,
   for (int k = 0; k < 3; ++k) unsafeAtomicAdd(dst + min(max(idx[o + k], 0), m - 1), g * weight[o + k]);
 }
 
+// Interpolation with CH channels of the m known points in LDS, [m][CH]: one thread per target and step reads the target's
+// indices and weights once for all of them and CH / 4 16-byte LDS reads per neighbour.  Bound by writing the output:
+// 256 channels, 2048 -> 20000 points, 8 samples: 166 us with a
+// thread per element, 45 us here (164 MB written).
+template <int CH>
+__global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int splits, int per, const float* __restrict__ points,
+                                                     const int* __restrict__ idx, const float* __restrict__ weight,
+                                                     float* __restrict__ out) {
+  extern __shared__ __align__(16) float srow[];
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), per_b = (c + CH - 1) / CH * splits;
+  const int tid = threadIdx.x, b = wg / per_b, c0 = (wg % per_b) / splits * CH, part = wg % splits;
+  for (int e = tid; e < m * CH; e += 512) {   // neighbouring lanes: neighbouring channels (no bank conflict)
+    const int ch = min(c0 + e % CH, c - 1);
+    srow[e] = points[((long)b * c + ch) * m + e / CH];
+  }
+  __syncthreads();
+  const int hi = min((part + 1) * per, n);
+  for (int j = part * per + tid; j < hi; j += 512) {
+    const long o = ((long)b * n + j) * 3;
+    f4 acc[CH / 4];
+#pragma unroll
+    for (int q = 0; q < CH / 4; ++q) acc[q] = (f4){0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float w = weight[o + k];
+      const f4* s = (const f4*)(srow + index_of(idx[o + k], m) * CH);
+#pragma unroll
+      for (int q = 0; q < CH / 4; ++q) {
+        const f4 v = s[q];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[q][r] += w * v[r];
+      }
+    }
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch)
+      if (c0 + ch < c) out[((long)b * c + c0 + ch) * n + j] = acc[ch / 4][ch % 4];
+  }
+}
+// Its gradient, all of grad_points (b, c, m) written.  Adding target by target into rows of sums in LDS takes 600 us (8
+// samples, 256 channels, 2048 <- 20000 points): an LDS float addition to scattered words runs at a third of a lane a cycle.
+// So the targets' three (point, weight) entries are sorted by point first, once for all channels -- k_inverse_rank counts
+// and gives every entry its place within its point, k_inverse_fill writes (point, target, weight) in that order, thread t's
+// share of the sorted list at [i][t] -- and k_interp_rows_grad holds R rows of grad_out in LDS, reads them by target, sums
+// runs of a point in registers and adds a run's sum to the result.  212 us and 33 for the lists, 397 with atomics into a channel-last buffer.
+constexpr int INV_T = 1024;
+__global__ __launch_bounds__(INV_T) void k_inverse_rank(int n, int m, const int* __restrict__ idx, int* __restrict__ start,
+                                                        int* __restrict__ rank) {
+  extern __shared__ int cnt[];
+  __shared__ int wsum[INV_T / 64];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int k = tid; k < m; k += INV_T) cnt[k] = 0;
+  __syncthreads();
+  const int* q = idx + (long)b * n * 3;
+  int* r = rank + (long)b * n * 3;
+#pragma unroll 4
+  for (int e = tid; e < 3 * n; e += INV_T) r[e] = atomicAdd(cnt + index_of(q[e], m), 1);
+  __syncthreads();
+  const int per = (m + INV_T - 1) / INV_T, k0 = tid * per, k1 = min(k0 + per, m);
+  int own = 0;
+  for (int k = k0; k < k1; ++k) own += cnt[k];
+  int incl = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) wsum[wave] = incl;
+  __syncthreads();
+  int at = incl - own;
+  for (int w = 0; w < wave; ++w) at += wsum[w];
+  for (int k = k0; k < k1; ++k) {
+    start[(long)b * m + k] = at;
+    at += cnt[k];
+  }
+}
+// list entry: point << 16 | target, weight.  Places behind the 3 n entries hold point 0, target 0 and weight 0.
+__global__ __launch_bounds__(NTHREADS) void k_inverse_fill(int n, int m, int per, const int* __restrict__ idx,
+                                                           const float* __restrict__ weight, const int* __restrict__ start,
+                                                           const int* __restrict__ rank, uint2* __restrict__ list) {
+  const int b = blockIdx.y, e = blockIdx.x * NTHREADS + threadIdx.x;
+  if (e >= per * INV_T) return;
+  int at = e;
+  uint2 v = make_uint2(0u, 0u);
+  if (e < 3 * n) {
+    const int k = index_of(idx[(long)b * n * 3 + e], m);
+    at = start[(long)b * m + k] + rank[(long)b * n * 3 + e];
+    v = make_uint2((unsigned)k << 16 | (unsigned)(e / 3), __builtin_bit_cast(unsigned, weight[(long)b * n * 3 + e]));
+  }
+  list[(long)b * per * INV_T + (long)(at % per) * INV_T + at / per] = v;
+}
+template <int R>
+__global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m, int per, const float* __restrict__ grad_out,
+                                                            const uint2* __restrict__ list, float* __restrict__ grad_points) {
+  extern __shared__ float srow[];
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), per_b = (c + R - 1) / R;   // an XCD's workgroups: one sample's list in its L2
+  const int tid = threadIdx.x, b = wg / per_b, c0 = (wg % per_b) * R, nch = min(R, c - c0);
+  const float* g = grad_out + ((long)b * c + c0) * n;   // R neighbouring rows
+  for (int k = 4 * tid; k + 3 < nch * n; k += 4 * INV_T) *(f4*)(srow + k) = ld_stream(g + k);
+  {
+    const int k = (nch * n & ~3) + tid;
+    if (k < nch * n) srow[k] = g[k];
+  }
+  __syncthreads();
+  const uint2* q = list + (long)b * per * INV_T + tid;
+  float* o = grad_points + ((long)b * c + c0) * m;
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  unsigned cur = per ? q[0].x >> 16 : 0u;
+  auto put = [&]() {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r < nch) unsafeAtomicAdd(o + (long)r * m + cur, acc[r]);
+  };
+#pragma unroll 4
+  for (int i = 0; i < per; ++i) {
+    const uint2 v = q[(long)i * INV_T];
+    const unsigned k = v.x >> 16, j = v.x & 0xffffu;
+    const float w = __builtin_bit_cast(float, v.y);
+    if (k != cur) {
+      put();
+      cur = k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] += w * srow[min(r, nch - 1) * n + j];
+  }
+  put();
+}
+
 // Gradients into a channel-last buffer, out_cl (b, n, c) += ...: a 64 x 64 tile of grad_out (channels x entries) is
 // read along the entries (coalesced), turned in LDS, and added with lanes running over channels, so one atomic
 // instruction covers 64 consecutive floats of one point instead of 64 scattered cache lines.
@@ -480,9 +949,50 @@ int launch_ball_query(int b, int n, int m, float radius, int nsample, const floa
                      idx);
   return (int)hipGetLastError();
 }
-int launch_group_points(int b, int c, int n, int ms, const float* points, const int* idx, float* out, hipStream_t st) {
-  const long total = (long)b * c * ms;
-  hipLaunchKernelGGL(k_group_points, dim3(blocks_for(total)), dim3(NTHREADS), 0, st, total, c, n, ms, points, idx, out);
+template <typename K>
+static int set_lds_rows(K kern, size_t bytes) {
+  return bytes > 64 * 1024 ? (int)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) : 0;
+}
+// How the entries of a row are cut: about two workgroups per CU in all, but no part shorter than what it costs to put the
+// row into LDS (or to clear it and write it back), and a multiple of `unit` entries each.
+static int parts_of(long row_blocks, int entries, int row_len, int unit, int* per) {
+  long parts = (512 + row_blocks - 1) / row_blocks;
+  parts = std::max<long>(1, std::min<long>(parts, entries / std::max(row_len, 2048)));
+  *per = (int)(((entries + parts - 1) / parts + unit - 1) / unit * unit);
+  return (entries + *per - 1) / *per;
+}
+static int row_threads(int n) { return n > 10240 ? 1024 : 512; }   // above, at most three workgroups fit a CU's LDS
+
+int launch_group_points(int b, int c, int n, int npoints, int nsample, const float* xyz, const float* centre, float scale,
+                        const float* points, const int* idx, float* out, hipStream_t st) {
+  GroupP g;
+  g.c = c; g.cx = xyz ? 3 : 0; g.n = n; g.ms = npoints * nsample; g.npoints = npoints; g.nsample = nsample;
+  g.xyz = xyz; g.centre = centre; g.points = points; g.idx = idx; g.out = out; g.scale = scale;
+  const long rows = (long)b * (g.cx + c);
+  if (rows > 0x7fffffff) return (int)hipErrorInvalidValue;
+  g.rows = (int)rows;
+  // rows in LDS where one fits and has at least as many entries as it has points to read, and there are rows for the chip
+  if (n <= ROW_POINTS && g.ms >= n) {
+    const long total = rows * g.ms, places = 256L * std::max(1, std::min(4, ROW_POINTS / n));
+    const long shares = std::max<long>(1, std::min<long>(places, total / std::max(n, 4096)));
+    g.share = (total + shares - 1) / shares;
+    if (int e = set_lds_rows(&k_group_rows, n * sizeof(float))) return e;
+    hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((total + g.share - 1) / g.share)), dim3(row_threads(n)), n * sizeof(float), st, g);
+  } else {
+    hipLaunchKernelGGL(k_group_points, dim3((g.ms + NTHREADS - 1) / NTHREADS, (unsigned)std::min<long>(rows, 65535)),
+                       dim3(NTHREADS), 0, st, g);
+  }
+  return (int)hipGetLastError();
+}
+int launch_group_rows_grad(int b, int c, int c0, int cdim, int n, int ms, const float* grad_out, const int* idx,
+                           float* grad_points, hipStream_t st) {
+  const long rows = (long)b * c;
+  int per;
+  const int splits = parts_of(rows, ms, n, 256, &per);
+  if (splits > 1) hipLaunchKernelGGL(k_zero, dim3(blocks_for(rows * n)), dim3(NTHREADS), 0, st, rows * n, grad_points);
+  if (int e = set_lds_rows(&k_group_rows_grad, n * sizeof(float))) return e;
+  hipLaunchKernelGGL(k_group_rows_grad, dim3((unsigned)(rows * splits)), dim3(row_threads(n)), n * sizeof(float), st, c, c0,
+                     cdim, n, ms, splits, per, grad_out, idx, grad_points);
   return (int)hipGetLastError();
 }
 int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out, const int* idx, float* grad_points,
@@ -493,6 +1003,12 @@ int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out,
   return (int)hipGetLastError();
 }
 int launch_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2, int* idx, hipStream_t st) {
+  if (m >= 256 && m <= 8192) {   // fewer: building the grid costs as much as looking at all; more: they do not fit in LDS
+    const size_t sm = m * sizeof(float4) + (NN_CELLS + 1) * sizeof(int);
+    if (int e = set_lds_rows(&k_three_nn_grid, sm)) return e;
+    hipLaunchKernelGGL(k_three_nn_grid, dim3((n + NN_T - 1) / NN_T, b), dim3(NN_T), sm, st, n, m, unknown, known, dist2, idx);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(k_three_nn, dim3((n + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, unknown, known, dist2,
                      idx);
   return (int)hipGetLastError();
@@ -500,9 +1016,52 @@ int launch_three_nn(int b, int n, int m, const float* unknown, const float* know
 int launch_three_interpolate(int b, int c, int m, int n, const float* points, const int* idx, const float* weight, float* out,
                              hipStream_t st) {
   const long total = (long)b * c * n;
+  // rows in LDS, see launch_group_points; below two million elements filling LDS takes longer than it saves (64 channels,
+  // 400 -> 3000 points, 2 samples: 12 us against 4)
+  if (n >= m && total >= 1 << 21 && m <= INTERP_POINTS) {
+    const int ch = m <= INTERP_POINTS / 4 ? 8 : 4, groups = (c + ch - 1) / ch;
+    const size_t sm = (size_t)m * ch * sizeof(float);
+    int per;
+    const int splits = parts_of((long)b * groups, n, m, 512, &per);
+    if (ch == 8) {
+      if (int e = set_lds_rows(&k_interp_rows<8>, sm)) return e;
+      hipLaunchKernelGGL(k_interp_rows<8>, dim3(groups * splits * b), dim3(512), sm, st, c, m, n, splits, per, points, idx, weight, out);
+    } else {
+      if (int e = set_lds_rows(&k_interp_rows<4>, sm)) return e;
+      hipLaunchKernelGGL(k_interp_rows<4>, dim3(groups * splits * b), dim3(512), sm, st, c, m, n, splits, per, points, idx, weight, out);
+    }
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(k_three_interpolate, dim3(blocks_for(total)), dim3(NTHREADS), 0, st, total, c, m, n, points, idx, weight,
                      out);
   return (int)hipGetLastError();
+}
+// ints of scratch: start (b, m), rank (b, 3 n), list (b, per * INV_T) of two
+static int inverse_per(int n) { return (3 * n + INV_T - 1) / INV_T; }
+long interp_rows_grad_ints(int b, int n, int m) { return (long)b * ((m + 3L * n + 1) / 2 * 2 + 2L * inverse_per(n) * INV_T); }
+int launch_interp_rows_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight, int* ws,
+                            float* grad_points, hipStream_t st) {
+  const int per = inverse_per(n);
+  uint2* list = (uint2*)ws;
+  int *start = ws + 2L * b * per * INV_T, *rank = start + (long)b * m;
+  if (int e = set_lds_rows(&k_inverse_rank, m * sizeof(int))) return e;
+  hipLaunchKernelGGL(k_inverse_rank, dim3(b), dim3(INV_T), m * sizeof(int), st, n, m, idx, start, rank);
+  hipLaunchKernelGGL(k_inverse_fill, dim3((per * INV_T + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, per, idx, weight,
+                     start, rank, list);
+  const long total = (long)b * c * m;
+  hipLaunchKernelGGL(k_zero, dim3(blocks_for(total)), dim3(NTHREADS), 0, st, total, grad_points);
+  auto go = [&](auto kern, int r) -> int {
+    const size_t sm = (size_t)r * n * sizeof(float);
+    if (int e = set_lds_rows(kern, sm)) return e;
+    hipLaunchKernelGGL(kern, dim3((c + r - 1) / r * b), dim3(INV_T), sm, st, c, n, m, per, grad_out, list, grad_points);
+    return 0;
+  };
+  // more rows per workgroup: the list is read less often; as many as fit, where that leaves a workgroup for every CU
+  int e;
+  if (n <= ROW_POINTS / 4 && (long)b * ((c + 3) / 4) >= 256) e = go(&k_interp_rows_grad<4>, 4);
+  else if (n <= ROW_POINTS / 2 && (long)b * ((c + 1) / 2) >= 256) e = go(&k_interp_rows_grad<2>, 2);
+  else e = go(&k_interp_rows_grad<1>, 1);
+  return e ? e : (int)hipGetLastError();
 }
 int launch_three_interpolate_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight,
                                   float* grad_points, hipStream_t st) {

@@ -6,11 +6,15 @@ from __future__ import annotations
 
 import ctypes as C
 
+import numpy as np
 import torch
 import torch.nn as nn
 from torch.autograd import Function
 
 from . import _lib as L
+
+
+_ROW_POINTS = 40960      # ISSM_PN2_ROW_POINTS: points of the longest channel row the *_rows gradients take
 
 
 def _f(t):
@@ -129,6 +133,15 @@ class ThreeInterpolate(Function):
         g = _f(grad_out)
         Bsz, c, n = g.shape
         with torch.cuda.device(g.device):
+            # (the sorted lists of the rows form pay off from two million elements: 64 channels, 400 <- 3000 points, 2 samples
+            # take 20 us with it and 13 without)
+            if g.numel() >= 1 << 21 and max(n, m) <= _ROW_POINTS and Bsz <= 65535:
+                ws = torch.empty(lib.issm_pn2_three_interpolate_grad_rows_workspace(Bsz, n, m), dtype=torch.uint8, device=g.device)
+                out = torch.empty((Bsz, c, m), dtype=torch.float32, device=g.device)
+                L.check(lib.issm_pn2_three_interpolate_grad_rows(Bsz, c, n, m, g.data_ptr(), ix.data_ptr(), w.data_ptr(),
+                                                                 ws.data_ptr(), out.data_ptr(), _st(g)),
+                        "issm_pn2_three_interpolate_grad_rows")
+                return out.to(dt), None, None
             # accumulated channel-last (coalesced atomics); the transpose is the gradient in the features' layout
             out = torch.zeros((Bsz, m, c), dtype=torch.float32, device=g.device)
             L.check(lib.issm_pn2_three_interpolate_grad_cl(Bsz, c, n, m, g.data_ptr(), ix.data_ptr(), w.data_ptr(),
@@ -157,19 +170,55 @@ class GroupingOperation(Function):
 
     @staticmethod
     def backward(ctx, grad_out):
-        lib = L.load()
         ix, N, dt = ctx.for_backwards
-        g = _f(grad_out)
-        Bsz, Cn, M, S = g.shape
-        with torch.cuda.device(g.device):
-            # accumulated channel-last (coalesced atomics); the transpose is the gradient in the features' layout
-            out = torch.zeros((Bsz, N, Cn), dtype=torch.float32, device=g.device)
-            L.check(lib.issm_pn2_group_points_grad_cl(Bsz, Cn, N, M, S, g.data_ptr(), ix.data_ptr(), out.data_ptr(), _st(g)),
-                    "issm_pn2_group_points_grad_cl")
-        return out.transpose(1, 2).to(dt), None
+        return _grouping_grad(_f(grad_out), ix, N, 0).to(dt), None
+
+
+def _grouping_grad(g, ix, N, c0):
+    """Gradient (B, C, N) of the features behind channels c0 .. of g (B, c0 + C, npoint, nsample)."""
+    lib = L.load()
+    Bsz, cdim, M, S = g.shape
+    Cn = cdim - c0
+    with torch.cuda.device(g.device):
+        if M * S and N <= _ROW_POINTS and Bsz * Cn < 1 << 20:
+            out = torch.empty((Bsz, Cn, N), dtype=torch.float32, device=g.device)
+            L.check(lib.issm_pn2_group_points_grad_rows(Bsz, Cn, c0, cdim, N, M, S, g.data_ptr(), ix.data_ptr(), out.data_ptr(),
+                                                        _st(g)), "issm_pn2_group_points_grad_rows")
+            return out
+        g = g[:, c0:].contiguous()
+        # accumulated channel-last (coalesced atomics); the transpose is the gradient in the features' layout
+        out = torch.zeros((Bsz, N, Cn), dtype=torch.float32, device=g.device)
+        L.check(lib.issm_pn2_group_points_grad_cl(Bsz, Cn, N, M, S, g.data_ptr(), ix.data_ptr(), out.data_ptr(), _st(g)),
+                "issm_pn2_group_points_grad_cl")
+    return out.transpose(1, 2)
 
 
 grouping_operation = GroupingOperation.apply
+
+
+class _GroupXyzPoints(Function):
+    """Coordinates relative to the centres times `scale`, then features, grouped in one pass; gradient to the features."""
+
+    @staticmethod
+    def forward(ctx, features, xyz, new_xyz, idx, scale):
+        if features is not None:
+            L.require_gpu(features, "features")
+        lib = L.load()
+        x, q, ix = _f(xyz), _f(new_xyz), _i(idx)
+        f = None if features is None else _f(features)
+        (Bsz, N, _), (_, M, S), Cn = x.shape, ix.shape, 0 if f is None else f.shape[1]
+        with torch.cuda.device(x.device):
+            out = torch.empty((Bsz, 3 + Cn, M, S), dtype=torch.float32, device=x.device)
+            L.check(lib.issm_pn2_group_xyz_points(Bsz, Cn, N, M, S, x.data_ptr(), q.data_ptr(), scale,
+                                                  None if f is None else f.data_ptr(), ix.data_ptr(), out.data_ptr(), _st(x)),
+                    "issm_pn2_group_xyz_points")
+        ctx.for_backwards = (ix, N)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        ix, N = ctx.for_backwards
+        return _grouping_grad(_f(grad_out), ix, N, 3), None, None, None, None
 
 
 class BallQuery(Function):
@@ -225,6 +274,11 @@ class QueryAndGroup(nn.Module):
                     pick = torch.randint(0, uniq.shape[0], (self.nsample - uniq.shape[0],), dtype=torch.long,
                                          device=uniq.device)
                     idx[b, r, :] = torch.cat((uniq, uniq[pick]))
+        if self.use_xyz and not self.ret_grouped_xyz and self._one_pass(xyz, new_xyz, features):
+            # (a division by a Python number is a product with its fp32 reciprocal)
+            scale = float(np.float32(1.0) / np.float32(self.radius)) if self.normalize_xyz else 1.0
+            new_features = _GroupXyzPoints.apply(features, xyz, new_xyz, idx, scale)
+            return (new_features, unique_cnt) if self.ret_unique_cnt else new_features
         grouped_xyz = grouping_operation(xyz.transpose(1, 2).contiguous(), idx)   # (B, 3, npoint, nsample)
         grouped_xyz = grouped_xyz - new_xyz.transpose(1, 2).unsqueeze(-1)
         if self.normalize_xyz:
@@ -241,6 +295,15 @@ class QueryAndGroup(nn.Module):
         if self.ret_unique_cnt:
             ret.append(unique_cnt)
         return ret[0] if len(ret) == 1 else tuple(ret)
+
+
+    @staticmethod
+    def _one_pass(xyz, new_xyz, features):
+        """fp32 throughout, one feature column per point, and no gradient wanted for coordinates."""
+        given = [t for t in (xyz, new_xyz, features) if t is not None]
+        return (all(t.dtype == torch.float32 and t.shape[0] == xyz.shape[0] for t in given) and xyz.shape[1] > 0
+                and (features is None or features.shape[2] == xyz.shape[1])
+                and not (torch.is_grad_enabled() and (xyz.requires_grad or new_xyz.requires_grad)))
 
 
 class GroupAll(nn.Module):

@@ -518,6 +518,21 @@ int issm_pn2_three_interpolate(int32_t b, int32_t c, int32_t m, int32_t n, const
                                const float* weight, float* out, void* stream);
 int issm_pn2_three_interpolate_grad(int32_t b, int32_t c, int32_t n, int32_t m, const float* grad_out, const int32_t* idx,
                                     const float* weight, float* grad_points, void* stream);
+/* Ball grouping with coordinates in one pass: out (b, 3 + c, npoints, nsample), channels 0 .. 2 the coordinates of the
+ * entry's point relative to its centre times `scale` (xyz (b, n, 3), new_xyz (b, npoints, 3)), then points (b, c, n). */
+int issm_pn2_group_xyz_points(int32_t b, int32_t c, int32_t n, int32_t npoints, int32_t nsample, const float* xyz,
+                              const float* new_xyz, float scale, const float* points, const int32_t* idx, float* out,
+                              void* stream);
+/* The gradients of grouping (channels c0 .. c0 + c - 1 of a grad_out (b, cdim, npoints, nsample)) and of interpolation, all
+ * of grad_points (b, c, n) resp. (b, c, m) written: up to ISSM_PN2_ROW_POINTS points a row (both rows for interpolation, which
+ * sorts its entries in a workspace of ..._workspace(b, n, m) bytes, aligned to 8).  Nothing is written when there are no
+ * entries. */
+#define ISSM_PN2_ROW_POINTS 40960
+int issm_pn2_group_points_grad_rows(int32_t b, int32_t c, int32_t c0, int32_t cdim, int32_t n, int32_t npoints, int32_t nsample,
+                                    const float* grad_out, const int32_t* idx, float* grad_points, void* stream);
+int64_t issm_pn2_three_interpolate_grad_rows_workspace(int32_t b, int32_t n, int32_t m);
+int issm_pn2_three_interpolate_grad_rows(int32_t b, int32_t c, int32_t n, int32_t m, const float* grad_out, const int32_t* idx,
+                                         const float* weight, void* workspace, float* grad_points, void* stream);
 /* The same two gradients accumulated into a channel-last buffer, grad_points_cl (b, n, c) resp. (b, m, c), zeroed by
  * the caller: its transpose is the reference's result.  No counterpart in the reference; the atomics then touch
  * 64 consecutive floats per instruction instead of 64 scattered cache lines (about 10x faster at C = 128). */

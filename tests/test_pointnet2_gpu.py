@@ -175,6 +175,78 @@ def test_query_and_group_module():
     assert GroupAll()(txyz, None, tf).shape == (B, 3 + C, 1, N)
 
 
+@pytest.mark.parametrize("B,C,N,M,S", [(1, 1, 1, 1, 1), (2, 3, 63, 16, 4), (1, 2, 257, 300, 7), (2, 5, 1023, 511, 9),
+                                       (1, 3, 4099, 640, 32), (1, 1, 40960, 5200, 16), (1, 1, 40961, 5200, 16)])
+def test_grouped_rows_and_their_gradient(B, C, N, M, S):
+    """Row remainders, entries cut over several workgroups (few channels, many entries), the longest row in LDS and the first
+    beyond it; index runs of every length, within a lane's four entries, across lanes and across the rows of a wave."""
+    from dest3d_amd.pointnet2_utils import QueryAndGroup, grouping_operation
+    rng = np.random.default_rng(N + M)
+    idx = np.repeat(rng.integers(0, N, size=B * M * S), rng.integers(1, 90, size=B * M * S))[:B * M * S]
+    idx = idx.astype(np.int32).reshape(B, M, S)
+    idx[0, M // 2:] = rng.integers(0, N, size=(M - M // 2, S))
+    feats = rng.standard_normal((B, C, N)).astype(np.float32)
+    f = _cuda(feats).requires_grad_()
+    g = grouping_operation(f, _cuda(idx))
+    assert (g.detach().cpu().numpy() == R.group_points(feats, idx)).all()
+    gy = rng.standard_normal(g.shape).astype(np.float32)
+    g.backward(_cuda(gy))
+    ref = R.group_points_grad(gy, idx, N)
+    assert np.abs(f.grad.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+    # coordinates and features in one pass: bit for bit what the separate operators give, and the same gradient
+    xyz = rng.uniform(-1, 1, size=(B, N, 3)).astype(np.float32)
+    x, q = _cuda(xyz), _cuda(xyz[:, rng.integers(0, N, size=M)])
+    one = QueryAndGroup(0.3, S, normalize_xyz=True)
+    parts = QueryAndGroup(0.3, S, normalize_xyz=True, ret_grouped_xyz=True)
+    f1, f2 = f.detach().clone().requires_grad_(), f.detach().clone().requires_grad_()
+    a, (b, _) = one(x, q, f1), parts(x, q, f2)
+    assert torch.equal(a, b)
+    w = _cuda(rng.standard_normal(a.shape).astype(np.float32))
+    a.backward(w)
+    b.backward(w)
+    assert (f1.grad - f2.grad).abs().max() <= 1e-5 * f2.grad.abs().max()
+
+
+@pytest.mark.parametrize("c,m,n", [(1, 1, 3), (3, 5, 700), (9, 2560, 2600), (8, 2561, 2700), (5, 10240, 10300), (2, 10241, 10300),
+                                   (2, 40, 20000), (512, 30, 1023), (700, 3, 5121), (3, 1000, 40960), (1, 900, 40961)])
+def test_interpolation_rows(c, m, n):
+    from dest3d_amd.pointnet2_utils import three_interpolate
+    rng = np.random.default_rng(m)
+    feats = rng.standard_normal((2, c, m)).astype(np.float32)
+    idx = rng.integers(0, m, size=(2, n, 3)).astype(np.int32)
+    w = rng.uniform(0, 1, size=(2, n, 3)).astype(np.float32)
+    f = _cuda(feats).requires_grad_()
+    y = three_interpolate(f, _cuda(idx), _cuda(w))
+    ref = R.three_interpolate(feats, idx, w)
+    assert np.abs(y.detach().cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+    gy = rng.standard_normal(ref.shape).astype(np.float32)
+    y.backward(_cuda(gy))
+    gref = R.three_interpolate_grad(gy, idx, w, m)
+    assert np.abs(f.grad.cpu().numpy() - gref).max() <= 1e-5 * np.abs(gref).max()
+
+
+@pytest.mark.parametrize("m", [255, 256, 257, 2048, 8192, 8193])
+def test_three_nn_grid(m):
+    """Both sides of the grid's range; sample 1: a flat sheet with duplicates (ties go to the smaller index), clusters and far
+    points, unknown points far outside; sample 2: one place; sample 3: coordinates the grid cannot hold."""
+    from dest3d_amd.pointnet2_utils import three_nn
+    rng = np.random.default_rng(m)
+    k = rng.uniform(-2, 2, size=(4, m, 3)).astype(np.float32)
+    u = rng.uniform(-2, 2, size=(4, 700, 3)).astype(np.float32)
+    k[1, :, 1] = 0.5
+    k[1, m // 2:] = k[1, :m - m // 2]
+    k[1, m // 4:m // 3] *= 0.01
+    k[1, 7] = (1e4, 3.0, -1e5)
+    u[1, :50] *= 1e3
+    u[1, 50:60] = k[1, :10]
+    k[2] = k[2, 0]
+    k[3, 5, 0] = np.inf
+    dist, idx = three_nn(_cuda(u), _cuda(k))
+    d2_ref, idx_ref = R.three_nn(u, k)
+    assert (idx.cpu().numpy() == idx_ref).all()
+    assert np.allclose(dist.cpu().numpy(), np.sqrt(d2_ref), rtol=1e-6, atol=0)
+
+
 def test_error_codes():
     from dest3d_amd import _lib as L
     lib = L.load()
