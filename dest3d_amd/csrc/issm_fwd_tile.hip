@@ -21,23 +21,15 @@
 //                  on the OUTPUT row n only: the accumulator is multiplied by et[J+1] between the tiles (Horner).  The
 //                  result holds four adjacent columns of a state row per lane: 16-byte stores.
 //
-// Everything but W is a product of factors <= 1.  W grows like 2^(span of a tile), and a tile whose sum of a is below
-// -FWD_SPAN_LIMIT needs another form ("deep": large dt |A|; a quarter of the chunks of a freshly initialised decoder).
-//   bf16 inputs    the wave's 16 columns of the step take the diagonal blocks and V from halves of eight rows.  A half's own
-//                  square is anchored in the middle of the half, the square between the halves at their border, where both
-//                  factors are <= 1: three products instead of one, their operands as pairs.  Steps of a row are cut at DEEP_STEP = -28 there, so
-//                  seven of them stay in range whatever the inputs: a decay below 2^-28 = 4e-9 counts as at most that,
-//                  beside a diagonal term whose dt is the large one.  Tile and chunk decays stay uncut.  A decoder layer of
-//                  8 x 1024 tokens, 256 queries, both directions: 195 us with the form below, 94 us (on average over six layers).
-//   fp32 inputs    the chunk is computed once more, by the same workgroup, with the level-hierarchy body
-//                  (k_chunk_local_body), which has no such limit and overwrites everything written for the chunk before:
-//                  the operands' (hi, lo) pairs leave no registers for the halves (100 - 200 bytes a lane spill).
+// Everything but W is a product of factors <= 1.  W grows like 2^(span of a tile): a chunk with a tile whose sum of a is
+// below -FWD_SPAN_LIMIT is computed once more, by the same workgroup, with the level-hierarchy body (k_chunk_local_body),
+// which has no such limit and overwrites everything written for the chunk before.
 #include "issm_dev.h"
 #include "issm_fwd_local.h"
 
 namespace issm {
 
-constexpr float FWD_SPAN_LIMIT = 100.0f, DEEP_STEP = -28.0f;
+constexpr float FWD_SPAN_LIMIT = 100.0f;
 
 template <int PT, bool SPLIT>
 struct FwdTileSmem {
@@ -48,8 +40,7 @@ struct FwdTileSmem {
   int bad[4];
 };
 template <int PT, bool SPLIT>
-constexpr size_t fwd_tile_lds() {     // fp32: the level-hierarchy body lays its own structure over the same memory
-  if (!SPLIT) return sizeof(FwdTileSmem<PT, SPLIT>);
+constexpr size_t fwd_tile_lds() {     // the level-hierarchy body lays its own structure over the same memory
   return sizeof(FwdTileSmem<PT, SPLIT>) > sizeof(FwdLocalSmem<PT, SPLIT>) ? sizeof(FwdTileSmem<PT, SPLIT>)
                                                                           : sizeof(FwdLocalSmem<PT, SPLIT>);
 }
@@ -62,20 +53,6 @@ __device__ __forceinline__ float row_scan16(float v) {
   ISSM_DPP_SHR(0x112);
   ISSM_DPP_SHR(0x114);
   ISSM_DPP_SHR(0x118);
-#undef ISSM_DPP_SHR
-  return v;
-}
-
-// the same over the halves of a DPP row (lanes sharing lane >> 3); i8 = lane & 7
-__device__ __forceinline__ float row_scan8(float v, int i8) {
-#define ISSM_DPP_SHR(ctrl, d)                                                                                                    \
-  {                                                                                                                              \
-    const float o = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true)); \
-    v += i8 >= d ? o : 0.0f;                                                                                                     \
-  }
-  ISSM_DPP_SHR(0x111, 1);
-  ISSM_DPP_SHR(0x112, 2);
-  ISSM_DPP_SHR(0x114, 4);
 #undef ISSM_DPP_SHR
   return v;
 }
@@ -143,7 +120,7 @@ template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr bool SPLIT = !IOB, DEEP = !SPLIT;
+  constexpr bool SPLIT = !IOB;
   typedef FwdTileSmem<PT, SPLIT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
   constexpr int LDT = SM::LDT;
@@ -286,11 +263,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     for (int k = 0; k < 16; ++k) et[k] = __shfl(up[k], last_lane, 64);  // whole-tile decay of the lane's columns
 #pragma unroll
     for (int k = 0; k < 16; k += 2) etmin = fminf(etmin, fminf(et[k], et[k + 1]));
-    bool deep = false;   // wave-uniform
-    if constexpr (DEEP) {
-      deep = __ballot(!(etmin >= thr)) != 0ull;
-      etmin = 1.0f;
-    }
     {  // the chunk's total decay (natural logarithm), four adjacent columns per lane group.  All 16 lanes of a group
        // store the same values to the same place: a store under a lane condition sits behind a branch, and the waits
        // for the requests in flight -- counted in order with the stores -- would then have to assume it away and wait
@@ -313,50 +285,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     for (int pt = 0; pt < PT; ++pt) sacc[pt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int J = 0; J < 4; ++J) {
-      float V[4];
-      if (!DEEP || !deep) {
-        float W[4];
+      float W[4], V[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int k = 4 * J + r;
-          W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
-          V[r] = W[r] * et[k];
-        }
+      for (int r = 0; r < 4; ++r) {
+        const int k = 4 * J + r;
+        W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
+        V[r] = W[r] * et[k];
+      }
+      {
         const Fr f = make_frag<SPLIT>(W[0], W[1], W[2], W[3]);
         macc[J] = frag_product<SPLIT>(U[J], f, macc[J]);
-      } else {
-        // rows in halves lo = 0 .. 7, hi = 8 .. 15; t = the half's running sum, its first value f, its total e
-        const bool lo = i < 8;
-        float ud[4], wd[4], uh[4], wl[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int k = 4 * J + r;
-          const float t = row_scan8(fmaxf(dtp[k] * A2[r], DEEP_STEP), i & 7);
-          const float e = __shfl(t, lane | 7, 64), mid = 0.5f * (__shfl(t, lane & ~7, 64) + e);
-          const float e_hi = __shfl(t, last_lane, 64), v = dtp[k] * bv[k];
-          ud[r] = cv[k] * ex2(t - mid);
-          wd[r] = v * ex2(mid - t);
-          uh[r] = lo ? 0.0f : cv[k] * ex2(t);
-          const float we = v * ex2(e - t);
-          wl[r] = lo ? we : 0.0f;
-          V[r] = lo ? we * ex2(e_hi) : we;
-        }
-        // Pairs for both operands: the level form kept the pairs of rows next to the diagonal in fp32.  (lo, lo): what it
-        // leaves in (lo, hi) lies above the diagonal and is dropped with the rest of it.
-        auto add = [&](const float (&a)[4], const float (&b)[4]) {
-          macc[J] = frag_product<true>(make_frag<true>(a[0], a[1], a[2], a[3]), make_frag<true>(b[0], b[1], b[2], b[3]), macc[J]);
-        };
-        float ul[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          ul[r] = lo ? ud[r] : 0.0f;
-          ud[r] = lo ? 0.0f : ud[r];
-        }
-        add(ul, wd);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wd[r] = lo ? 0.0f : wd[r];
-        add(ud, wd);  // (hi, hi)
-        add(uh, wl);  // (hi, lo)
       }
       // V serves the block below the diagonal one (J < 3) and the chunk state: always as a (hi, lo) pair
       const Frag<true> fv = make_frag<true>(V[0], V[1], V[2], V[3]);
@@ -445,12 +383,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       }
     }
   }
-  if (!DEEP && anybad) {
+  if (anybad) {
     // A tile of this chunk decays by more than 2^-FWD_SPAN_LIMIT: everything is computed once more in the form that has no
     // such limit.  The fence orders this workgroup's stores above before the ones the other form makes to the same places.
     __threadfence();
     __syncthreads();
-    if constexpr (!DEEP) k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
+    k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
   }
 }
 
