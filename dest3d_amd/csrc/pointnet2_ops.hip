@@ -70,14 +70,14 @@ __device__ __forceinline__ float wave_fmax(float v) {  // (used once per slot, n
 __device__ __forceinline__ float lane_f(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
-// of the lanes in `cand`, the one with the smallest `key` (rare: equal distances)
+// of the lanes in `cand`, the one with the smallest `key` (equal distances; keys differ).  One reduction however many there
+// are: on a voxelized cloud most lanes tie, and taken one by one they made a draw three times as long (8192 points on a
+// quarter-metre grid, 2048 draws, 8 samples: 6.9 -> 2.2 ms).
 __device__ __forceinline__ int lane_of_least(unsigned long long cand, int key) {
-  int best = __builtin_ctzll(cand), bk = __builtin_amdgcn_readlane(key, best);
-  for (cand &= cand - 1; cand; cand &= cand - 1) {
-    const int l = __builtin_ctzll(cand), k = __builtin_amdgcn_readlane(key, l);
-    if (k < bk) { bk = k; best = l; }
-  }
-  return best;
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const unsigned v = (cand >> lane) & 1ull ? ~(unsigned)key : 0u;   // keys are >= 0, so a candidate's v is never 0
+  const unsigned m = wave_max<4>(v);
+  return __builtin_ctzll(__ballot(v == m));
 }
 
 // Up to 64 W S points: one workgroup of W waves per sample, points in registers, and only those looked at that a draw can

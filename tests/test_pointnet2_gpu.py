@@ -53,6 +53,15 @@ def test_furthest_point_sampling_at_the_edges_of_its_variants(n):
     assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
 
 
+@pytest.mark.parametrize("n,npoint", [(700, 300), (4096, 512)])
+def test_furthest_point_sampling_on_a_voxelized_cloud(n, npoint):
+    """Coordinates on a quarter-metre grid: most running distances tie, within groups, waves and the workgroup."""
+    from dest3d_amd.pointnet2_utils import furthest_point_sample
+    xyz = (np.random.default_rng(n).integers(1, 17, size=(2, n, 3)) * 0.25).astype(np.float32)
+    idx = furthest_point_sample(_cuda(xyz), npoint).cpu().numpy()
+    assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
+
+
 @pytest.mark.parametrize("seed,npoint", [(3, 1024), (8, 1024), (54, 1024)])
 def test_furthest_point_sampling_near_ties_go_the_way_of_plain_fp32_steps(seed, npoint):
     """Clouds in which two candidates' running minimum distances come within one unit in the last place of each other
