@@ -67,19 +67,22 @@ __device__ __forceinline__ float wave_uniform(float v) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
-// dist: a wave owns one box (its corners and rotations in scalar registers) and BD_SEG key points, a lane one point
+// dist: a wave owns one box (its corners and rotations in scalar registers) and up to BD_SEG key points, a lane one point
 // at a time.  Pairs whose corners share a 3 x 3 x 3 window take the short path at once; the others (a box next to
 // or around the point: about four in ten at detector scales) are queued in LDS and then walked corner by corner in
 // full waves -- done in place, the long path would run for every wave with most lanes idle, and cost more than the
-// rest together.  The eight waves of a workgroup own adjacent boxes, so a point's eight rows are neighbours in memory.
+// rest together.  The sixteen waves of a workgroup own eight adjacent boxes, so a point's eight rows are neighbours in memory,
+// and two segments of points each: four waves per SIMD on one table (vector issue bounds it, 83 M instructions; with two
+// waves per SIMD their LDS reads were not hidden).  8 x 1024 points, 256 boxes: 219 -> 176 us; one scene, whose segments are
+// shortened to 64 points so that all CUs have one (32 workgroups before): 209 -> 40 us.
 // The table lies node-major in LDS with 20 floats from node to node: a lane reads its node's 16 channels as four
 // 16-byte pieces, and with 16 floats per node the lanes of one read would meet in the 16 banks that (node mod 4)
 // selects; 20 n mod 64 runs through all sixteen 4-bank groups as n does.
-constexpr int BD_SEG = 1024;   // points per wave
-constexpr int BD_FWD_T = 512;  // 8 waves = 8 adjacent boxes per workgroup, one workgroup (96 KB of LDS) per CU
+constexpr int BD_SEG = 512;     // points per wave at most
+constexpr int BD_FWD_T = 1024;  // 16 waves = 8 adjacent boxes x 2 segments per workgroup, one workgroup (96 KB of LDS) per CU
 constexpr int BD_NS = 20;      // floats from node to node
 template <bool BF>
-__global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p) {
+__global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_points) {
   __shared__ __attribute__((aligned(16))) float tab[BD_MAXCELLS * BD_NS];
   __shared__ unsigned short queue[BD_FWD_T / 64][BD_SEG];
   const int cells = p.D * p.H * p.W;
@@ -89,11 +92,11 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p) {
   }
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int kgroups = (p.K + 7) / 8, nseg = (p.L + BD_SEG - 1) / BD_SEG;
+  const int kgroups = (p.K + 7) / 8, npair = (p.L + 2 * seg_points - 1) / (2 * seg_points);
   const int kgroup = blockIdx.x % kgroups, bs = blockIdx.x / kgroups;
-  const int seg = bs % nseg, b = bs / nseg, k = kgroup * 8 + wave;
-  const bool live = k < p.K;  // uniform per wave
-  const int l0 = seg * BD_SEG, n = min(BD_SEG, p.L - l0);
+  const int b = bs / npair, k = kgroup * 8 + (wave & 7);
+  const int l0 = (2 * (bs % npair) + (wave >> 3)) * seg_points, n = min(seg_points, p.L - l0);
+  const bool live = k < p.K && n > 0;  // uniform per wave
   const float scale = 1.0f / (3.0f * p.max_value);
   BoxLane bx;
   int queued = 0;
@@ -297,9 +300,12 @@ int box_dist_bwd_workgroups(int B, int L, int K) {
 int launch_box_dist_fwd(const BoxDistP& p, hipStream_t st) {
   const dim3 b(NTHREADS);
   if (p.dist) {
-    const dim3 g((unsigned)((long)p.B * ((p.L + BD_SEG - 1) / BD_SEG) * ((p.K + 7) / 8)));
-    if (p.dtype) hipLaunchKernelGGL(k_box_dist_fwd<true>, g, dim3(BD_FWD_T), 0, st, p);
-    else hipLaunchKernelGGL(k_box_dist_fwd<false>, g, dim3(BD_FWD_T), 0, st, p);
+    // segments of whole waves, as long as the queue allows but no longer than leaves every CU (256) a workgroup
+    const long rows = (long)p.B * ((p.K + 7) / 8), want = (256 + rows - 1) / rows;
+    const int half = (int)((p.L + 2 * want - 1) / (2 * want)), seg = half >= BD_SEG ? BD_SEG : (half + 63) / 64 * 64;
+    const dim3 g((unsigned)(rows * ((p.L + 2 * seg - 1) / (2 * seg))));
+    if (p.dtype) hipLaunchKernelGGL(k_box_dist_fwd<true>, g, dim3(BD_FWD_T), 0, st, p, seg);
+    else hipLaunchKernelGGL(k_box_dist_fwd<false>, g, dim3(BD_FWD_T), 0, st, p, seg);
   }
   if (p.weights) hipLaunchKernelGGL(k_box_dist_weights, dim3(p.nwg), b, 0, st, p);
   return (int)hipGetLastError();

@@ -30,6 +30,19 @@ CASES = [(2, 37, 256, False, (10, 10, 10)), (1, 5, 300, True, (10, 10, 10)), (2,
          (1, 1100, 64, True, (4, 6, 7)), (1, 1500, 43, True, (10, 10, 10))]   # two point segments, ragged box group
 
 
+def test_box_dist_forward_does_not_depend_on_the_segments():
+    """Enough boxes for the longest segments, the last pair of which has a short one and an empty one, against the same
+    points in calls of few points (shortest segments): the same bits."""
+    from dest3d_amd.box_dist import box_dist, box_parametrization_to_corners
+    key, qxyz, qsize, ang = (torch.from_numpy(x).cuda() for x in _inputs(1, 1030, 2041, 5, True))
+    table = torch.randn(16, 10, 10, 10, generator=torch.Generator().manual_seed(1)).cuda()
+    corners = box_parametrization_to_corners(qxyz, qsize, ang)
+    whole = box_dist(table, key, corners)
+    for lo, hi in ((0, 65), (448, 577), (1000, 1030)):
+        part = box_dist(table, key[:, lo:hi].contiguous(), corners[:, 1980:].contiguous())
+        assert torch.equal(part, whole[:, lo:hi, 1980:])
+
+
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "B%d_P%d_Q%d_ang%d_%dx%dx%d" % (*c[:3], int(c[3]), *c[4]))
 def test_box_dist_forward_and_table_gradient(case):
     from dest3d_amd.box_dist import box_dist, box_parametrization_to_corners
