@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libissm_hip.so")
 HOST = os.path.join(HERE, "_issm_host.so")
-SOURCES = ["issm_abi.hip", "issm_fwd.hip", "issm_fwd_tile.hip", "issm_bwd.hip", "issm_bwd_tile.hip", "rmsnorm_gated.hip", "param_gen.hip", "dwconv_silu.hip", "box_dist.hip", "box_dist_sorted.hip", "hilbert.hip", "pointnet2_ops.hip", "transpose_states.hip"]
+SOURCES = ["issm_abi.hip", "issm_fwd.hip", "issm_fwd_tile.hip", "issm_bwd.hip", "issm_bwd_tile.hip", "rmsnorm_gated.hip", "param_gen.hip", "dwconv_silu.hip", "box_dist.hip", "box_dist_sorted.hip", "hilbert.hip", "pointnet2_ops.hip", "transpose_states.hip", "layer_params.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffast-math", "-fno-finite-math-only",
@@ -27,7 +27,8 @@ FLAGS = [
 #  - pointnet2_ops.hip: squared distances pick indices (furthest point, ball membership, three nearest).  Under
 #    -ffast-math the backend fuses multiply and add whatever `#pragma clang fp contract(off)` says, and a distance one
 #    unit in the last place off decides a near-tie differently from a plain fp32 evaluation.
-EXACT_ARITHMETIC = {"hilbert.hip", "pointnet2_ops.hip"}
+# and one that computes no more than a few exponentials, which are to be the accurate ones: layer_params.hip.
+EXACT_ARITHMETIC = {"hilbert.hip", "pointnet2_ops.hip", "layer_params.hip"}
 
 
 def _compile(src: str) -> str:

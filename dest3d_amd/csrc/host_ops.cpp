@@ -550,7 +550,7 @@ issm_pgen_args pgen_args(const Tensor& dist, const float* W, int64_t H, int64_t 
 // back, and their backward passes chained by hand.
 struct CoreFn : public Function<CoreFn> {
   // the small parameters, in the order of their places in the flat fp32 buffer
-  enum { CW_F, CW_B, CB_F, CB_B, DT_W, BC_W, DT_BIAS, A_LOG, NSMALL };
+  enum { CW_F, CW_B, CB_F, CB_B, DT_W, BC_W, DT_BIAS, A_LOG, D_, NSMALL };
   // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
   static constexpr int NIN = 14;
 
@@ -565,16 +565,32 @@ struct CoreFn : public Function<CoreFn> {
                   K = dist.size(2);
     const at::ScalarType k = kernel_type(zxbcdt.scalar_type());
     Tensor zx = io_cast(zxbcdt, k);
-    const Tensor z = zx.narrow(2, 0, di), xbc = zx.narrow(2, di, Cc), dt_tok = zx.narrow(2, di + Cc, H);
-    // all small parameters in one fp32 buffer (one concatenation + one conversion instead of one per tensor); adjacent pieces
-    // form the stacked operands the kernels take
-    std::vector<Tensor> small;
+    const Tensor z = zx.narrow(2, 0, di), xbc = zx.narrow(2, di, Cc);
+    // all small parameters in one fp32 buffer, and A for all state columns; adjacent pieces form the stacked operands the
+    // kernels take
+    static_assert(NSMALL == ISSM_LAYER_ARRAYS, "one array per parameter");
     int64_t off[NSMALL + 1] = {0};
-    for (const Tensor& t : {conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log}) {
-      off[small.size() + 1] = off[small.size()] + t.numel();
-      small.push_back(t.reshape({-1}));
+    Tensor flat, A1 = fresh({H, K}, zx, at::kFloat);
+    {
+      issm_layer_params_args a{};
+      std::vector<Tensor> small;
+      for (const Tensor& t : {conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log, D}) {
+        const size_t i = small.size();
+        off[i + 1] = off[i] + t.numel();
+        small.push_back(cast(t, kernel_type(t.scalar_type())).contiguous());
+        a.src[i] = data(small[i]);
+        a.n[i] = (int32_t)t.numel();
+        a.dtype[i] = code(small[i].scalar_type());
+      }
+      TORCH_CHECK(A_log.numel() == H, "A_log must have one entry per head");
+      flat = fresh({off[NSMALL]}, zx, at::kFloat);
+      a.a_log = A_LOG;
+      a.K = (int32_t)K;
+      a.out = data<float>(flat);
+      a.A = data<float>(A1);
+      a.stream = stream_of(zx);
+      check(issm_layer_params(&a), "issm_layer_params");
     }
-    const Tensor flat = cast(at::cat(small), at::kFloat);
     float* const par = data<float>(flat);
     // 1. both depthwise convolutions + SiLU; the conv writes x and the B / C biases apart
     Tensor x = fresh({2, Bsz, Ln, H, P}, zx, k), tail = fresh({2, Bsz, Ln, 2 * G}, zx, k), pre = fresh({2, Bsz, Ln, Cc}, zx, k);
@@ -589,17 +605,14 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_dwconv_silu_fwd(&a), "issm_dwconv_silu_fwd");
     }
     // 2. dt / B / C (and the reversed-order B / C) from the distance encoding
-    Tensor bias = fresh({Bsz, Ln, H + 4 * G}, zx, at::kFloat);
-    {
-      Tensor b_dt = bias.narrow(2, 0, H);
-      at::add_out(b_dt, dt_tok, flat.narrow(0, off[DT_BIAS], H));
-    }
-    bias.narrow(2, H, 4 * G).unflatten(-1, {2, 2 * G}).copy_(tail.permute({1, 2, 0, 3}));
     const Tensor d = cast(dist, k).contiguous(), wt = f32c(weights);
     Tensor dt = fresh({Bsz, Ln, H, K}, zx, k), bc = fresh({4, Bsz, Ln, G, K}, zx, k), raw;
     {
       issm_pgen_args a = pgen_args(d, par + off[DT_W], H, G);
-      a.bias = data<const float>(bias);
+      a.tok = (const char*)data(zx) + (di + Cc) * zx.element_size();
+      a.tok_stride = zx.stride(1);
+      a.tok_add = par + off[DT_BIAS];
+      a.tail = data(tail);
       a.dt = data(dt);
       void** to[4] = {&a.Bm, &a.Cm, &a.Bm_back, &a.Cm_back};
       for (int i = 0; i < 4; ++i) *to[i] = (char*)data(bc) + i * (bc.numel() / 4) * bc.element_size();
@@ -611,13 +624,12 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
     }
     // 3. the bidirectional scan, queries as initial state
-    const Tensor A1 = flat.narrow(0, off[A_LOG], H).exp().neg_();
     const Tensor h0 = transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()))
                           .view({Bsz, H, P, K});
     const Tensor xs[2] = {x.select(0, 0), x.select(0, 1)}, Bs[2] = {bc.select(0, 0), bc.select(0, 2)},
                  Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
-    const Scan s = Scan::make(2, xs, dt, A1.unsqueeze(1).expand({H, K}), Bs, Cs, D, none, Tensor(), h0, Tensor(),
-                              !wt.defined(), lo, hi);
+    const Scan s = Scan::make(2, xs, dt, A1, Bs, Cs, D.dim() == 1 ? flat.narrow(0, off[D_], H) : D, none, Tensor(), h0,
+                              Tensor(), !wt.defined(), lo, hi);
     Scan::Out o = s.forward(true);
     // 4. gated RMSNorm (norm(x * silu(z))) of the two directions' average: the norm of s / 2 with eps is the norm of s with
     // 4 eps, so the sum goes in as it is and the halving never runs (nor its backward)
@@ -728,7 +740,7 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_dwconv_silu_bwd(&a), "issm_dwconv_silu_bwd");
     }
     dzx.narrow(2, di + Cc, H).copy_(dbias.narrow(2, 0, H));
-    const Tensor dA_log = g.dA.sum(-1).mul_(A1);
+    const Tensor dA_log = g.dA.sum(-1).mul_(A1.select(1, 0));
     const Tensor dh0 = transpose_states(g.dh0.view({Bsz, di, K}), Tensor(), 1.0, kernel_type(hdt));
     // parameter gradients, inputs 4 .. 13: one buffer, one conversion to the parameters' type when they share one
     std::vector<Tensor> pg{dcw.select(0, 0), dcb.select(0, 0), dcw.select(0, 1), dcb.select(0, 1), dW.narrow(0, 0, H),

@@ -42,6 +42,7 @@ struct TrP {
   float alpha;
 };
 int launch_transpose_states(const TrP& p, hipStream_t st);
+int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
                       hipStream_t st);
@@ -602,13 +603,16 @@ static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd) {
   if (!a->dist || !a->W) return fail(ISSM_E_NULL, "param_gen: dist/W is NULL");
   if (a->weights && !a->dt_raw) return fail(ISSM_E_NULL, "param_gen: weights given but dt_raw is NULL");
   if (!bwd) {
-    if (!a->bias || !a->dt || !a->Bm || !a->Cm) return fail(ISSM_E_NULL, "param_gen: bias/dt/Bm/Cm is NULL");
+    if (!a->dt || !a->Bm || !a->Cm) return fail(ISSM_E_NULL, "param_gen: dt/Bm/Cm is NULL");
+    if (!a->bias && (!a->tok || !a->tok_add || !a->tail)) return fail(ISSM_E_NULL, "param_gen: neither bias nor tok/tok_add/tail");
+    if (!a->bias && a->tok_stride < a->H) return fail(ISSM_E_STRIDE, "param_gen: tok_stride %lld", (long long)a->tok_stride);
     if (a->has_back && (!a->Bm_back || !a->Cm_back)) return fail(ISSM_E_NULL, "param_gen: Bm_back/Cm_back is NULL");
   } else {
     if (!a->dw_partial || !a->dW) return fail(ISSM_E_NULL, "param_gen bwd: dw_partial/dW is NULL");
   }
   p->tokens = a->tokens; p->K = a->K; p->H = a->H; p->G = a->G; p->dtype = a->dtype; p->has_back = a->has_back ? 1 : 0;
   p->dist = a->dist; p->W = a->W; p->bias = a->bias;
+  p->tok = a->tok; p->tok_stride = a->tok_stride; p->tok_add = a->tok_add; p->tail = a->tail;
   p->dt = a->dt; p->Bm = a->Bm; p->Cm = a->Cm; p->Bb = a->Bm_back; p->Cb = a->Cm_back;
   p->ddt = a->ddt; p->dB = a->dBm; p->dC = a->dCm; p->dBb = a->dBm_back; p->dCb = a->dCm_back;
   p->weights = a->weights; p->dt_raw = a->dt_raw; p->dweights = a->weights ? a->dweights : nullptr;
@@ -733,6 +737,27 @@ int issm_box_dist_bwd(const issm_box_dist_args* a) {
   if (rc) return rc;
   if (p.nwg_bwd == 0) return ISSM_OK;
   return launched(launch_box_dist_bwd(p, (hipStream_t)a->stream), "box_dist_bwd");
+}
+
+int issm_layer_params(const issm_layer_params_args* a) {
+  static_assert(LAYER_ARRAYS == ISSM_LAYER_ARRAYS, "one count");
+  if (!a) return fail(ISSM_E_NULL, "layer_params: args is NULL");
+  if (a->a_log < 0 || a->a_log >= LAYER_ARRAYS || a->K < 0) return fail(ISSM_E_SHAPE, "layer_params: a_log %d, K %d", a->a_log, a->K);
+  LayerParamsP p;
+  int64_t total = 0;
+  for (int i = 0; i < LAYER_ARRAYS; ++i) {
+    if (a->n[i] < 0) return fail(ISSM_E_SHAPE, "layer_params: n[%d] = %d", i, a->n[i]);
+    if (a->dtype[i] != ISSM_F32 && a->dtype[i] != ISSM_BF16) return fail(ISSM_E_DTYPE, "layer_params: dtype[%d] = %d", i, a->dtype[i]);
+    if (a->n[i] && !a->src[i]) return fail(ISSM_E_NULL, "layer_params: src[%d] is NULL", i);
+    p.src[i] = a->src[i]; p.n[i] = a->n[i]; p.bf16[i] = a->dtype[i] == ISSM_BF16;
+    total += a->n[i];
+  }
+  p.a_log = a->a_log; p.H = a->n[a->a_log]; p.K = a->K; p.out = a->out; p.A = a->A;
+  if (total + (int64_t)p.H * p.K > ((int64_t)1 << 30)) return fail(ISSM_E_SHAPE, "layer_params: too large");
+  p.total = (int)total;
+  if (total == 0) return ISSM_OK;
+  if (!a->out || !a->A) return fail(ISSM_E_NULL, "layer_params: out/A is NULL");
+  return launched(launch_layer_params(p, (hipStream_t)a->stream), "layer_params");
 }
 
 int issm_transpose_states(const issm_transpose_args* a) {

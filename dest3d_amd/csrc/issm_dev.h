@@ -164,12 +164,26 @@ struct DwConvP {
 };
 
 // parameters of the dt / B / C generation kernels (param_gen.hip)
+// parameters of the layer-parameter kernel (layer_params.hip)
+constexpr int LAYER_ARRAYS = 9;
+struct LayerParamsP {
+  const void* src[LAYER_ARRAYS];
+  int n[LAYER_ARRAYS], bf16[LAYER_ARRAYS];
+  int total, a_log, H, K;   // sum of n; which array is A_log
+  float* out;               // (total)
+  float* A;                 // (H, K)
+};
+
 struct PGenP {
   long tokens;
   int K, H, G, dtype, has_back;
   const void* dist;      // (tokens, K, M) io dtype
   const float* W;        // (R0, M) fp32
-  const float* bias;     // (tokens, R) fp32, R = R0 + (has_back ? 2G : 0)
+  const float* bias;     // (tokens, R) fp32, R = R0 + (has_back ? 2G : 0), or NULL with the three below:
+  const void* tok;       // io dtype, row of H values per token, tok_stride elements apart
+  long tok_stride;
+  const float* tok_add;  // (H)
+  const void* tail;      // (has_back ? 2 : 1, tokens, 2G) io dtype
   void *dt, *Bm, *Cm, *Bb, *Cb;                    // (tokens, H|G, K) io dtype
   const float* weights;  // (tokens, K) fp32 or NULL: dt = softplus(raw) * weights instead of raw
   void* dt_raw;          // (tokens, H, K) io dtype: raw dt, written by the forward when weights is given

@@ -96,13 +96,29 @@ __device__ __forceinline__ void stv(void* p, long i, const float (&v)[KV]) {
 // Forward: thread = (token, KV adjacent k) -- KV = 2 whenever K is even, so that every store instruction of a wave
 // covers 256 (bf16) or 512 bytes instead of 128 / 256.  W and the token's biases are uniform across the lanes of a
 // token: scalar operands.
-template <bool BF, int KV>
+// TOK: the biases come from the tensors their producers wrote (the projection's row, the convolution's tail) instead of a
+// gathered fp32 copy, which cost two launches and a pass of its own.  The workgroup's tokens (two at 256 queries) are gathered
+// into LDS, a value per thread; each lane loading its own row in 2-byte pieces took 55 us at 8192 tokens x 256, this 36,
+// reading the gathered copy 35.
+template <bool BF, int KV, bool TOK>
 __global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
   const int R0 = p.H + 2 * p.G, R = R0 + (p.has_back ? 2 * p.G : 0);
   const int per_tok = (p.K + KV - 1) / KV;  // threads per token
   const long gid = (long)blockIdx.x * NTHREADS + threadIdx.x;
   const long t = gid / per_tok;
   const int k = (int)(gid % per_tok) * KV;
+  extern __shared__ float tok_bias[];   // TOK: (tokens of the workgroup, R), rows as in p.bias
+  const long t0 = (long)blockIdx.x * NTHREADS / per_tok;
+  if constexpr (TOK) {
+    const long t1 = min(((long)(blockIdx.x + 1) * NTHREADS - 1) / per_tok, p.tokens - 1);
+    const int n = (int)(t1 - t0 + 1) * R;
+    for (int e = threadIdx.x; e < n; e += NTHREADS) {
+      const int tl = e / R, r = e - tl * R, i = r - p.H, set = i >= 2 * p.G ? 1 : 0;
+      tok_bias[e] = r < p.H ? ld1<BF>(p.tok, (t0 + tl) * p.tok_stride + r) + p.tok_add[r]
+                            : ld1<BF>(p.tail, (set * p.tokens + t0 + tl) * (2 * p.G) + i - set * 2 * p.G);
+    }
+    __syncthreads();
+  }
   if (t >= p.tokens) return;
   float d[KV][PG_M];
 #pragma unroll
@@ -112,8 +128,8 @@ __global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
   for (int j = 0; j < KV; ++j) wk[j] = p.weights ? p.weights[t * p.K + k + j] : 1.0f;
   // the token's biases, all requested before the row loop (a load per row inside it would be waited for row by
   // row); bb: the reversed-order pair's bias of a B / C row
-  const float* bias = p.bias + t * R;
   float bv[PG_MAXR0], bb[PG_MAXR0];
+  const float* bias = TOK ? tok_bias + (int)(t - t0) * R : p.bias + t * R;
 #pragma unroll
   for (int r = 0; r < PG_MAXR0; ++r) {
     bv[r] = bias[min(r, R - 1)];
@@ -520,12 +536,15 @@ int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
   const int kv = (p.K % 2 == 0 && al) ? 2 : 1;
   const long threads = p.tokens * ((p.K + kv - 1) / kv);
   const unsigned blocks = (unsigned)((threads + NTHREADS - 1) / NTHREADS);
-  if (p.dtype) {
-    if (kv == 2) hipLaunchKernelGGL((k_pgen_fwd<true, 2>), dim3(blocks), dim3(NTHREADS), 0, st, p);
-    else hipLaunchKernelGGL((k_pgen_fwd<true, 1>), dim3(blocks), dim3(NTHREADS), 0, st, p);
+  const int per_tok = (p.K + kv - 1) / kv, R = p.H + (p.has_back ? 4 : 2) * p.G;
+  const size_t lds = p.bias ? 0 : ((NTHREADS - 1) / per_tok + 2) * (size_t)R * sizeof(float);   // at most 23 KB
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), lds, st, p); };
+  if (p.bias) {
+    if (p.dtype) kv == 2 ? go(&k_pgen_fwd<true, 2, false>) : go(&k_pgen_fwd<true, 1, false>);
+    else kv == 2 ? go(&k_pgen_fwd<false, 2, false>) : go(&k_pgen_fwd<false, 1, false>);
   } else {
-    if (kv == 2) hipLaunchKernelGGL((k_pgen_fwd<false, 2>), dim3(blocks), dim3(NTHREADS), 0, st, p);
-    else hipLaunchKernelGGL((k_pgen_fwd<false, 1>), dim3(blocks), dim3(NTHREADS), 0, st, p);
+    if (p.dtype) kv == 2 ? go(&k_pgen_fwd<true, 2, true>) : go(&k_pgen_fwd<true, 1, true>);
+    else kv == 2 ? go(&k_pgen_fwd<false, 2, true>) : go(&k_pgen_fwd<false, 1, true>);
   }
   return (int)hipGetLastError();
 }

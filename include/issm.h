@@ -332,7 +332,29 @@ typedef struct issm_pgen_args {
   float* dW;
   void* stream;
   float* dbias_sum; /* optional, (R) fp32: dbias summed over the tokens (the dt_bias parameter's gradient is its first H) */
+  /* forward with bias = NULL: the biases from where their producers left them, in `dtype`.  Row h of dt: tok[t *
+   * tok_stride + h] + tok_add[h]; rows of B, C: tail[0][t][0 .. 2G); of the reversed pair: tail[1][t][0 .. 2G). */
+  const void* tok;
+  int64_t tok_stride;
+  const float* tok_add; /* (H) fp32 */
+  const void* tail;     /* (has_back ? 2 : 1, tokens, 2G) */
 } issm_pgen_args;
+
+/* The small parameters of a layer as its kernels read them: ISSM_LAYER_ARRAYS arrays src[i] of n[i] values of dtype[i]
+ * (issm_dtype), converted to fp32 and laid one behind the other in out, and A[h][k] = -exp(src[a_log][h]) for h < n[a_log],
+ * k < K. */
+#define ISSM_LAYER_ARRAYS 9
+typedef struct issm_layer_params_args {
+  const void* src[ISSM_LAYER_ARRAYS];
+  int32_t n[ISSM_LAYER_ARRAYS];
+  int32_t dtype[ISSM_LAYER_ARRAYS];
+  int32_t a_log, K;
+  float* out;
+  float* A;
+  void* stream;
+} issm_layer_params_args;
+
+int issm_layer_params(const issm_layer_params_args* args);
 
 int issm_param_gen_bwd_blocks(int64_t tokens);
 int issm_param_gen_fwd(const issm_pgen_args* args);

@@ -300,3 +300,20 @@ def test_box_dist_weights_and_six_layers_chain_bf16_at_detector_shape():
     torch.cuda.synchronize()
     for name, a, b in zip(("out_key", "out_query", "d in_key", "d in_query", "d encoding table weights"), o16, o32):
         _check(name, a, b, 5e-2)
+
+
+@pytest.mark.parametrize("L_,K,H,G", [(70, 3, 4, 1), (33, 50, 2, 2), (5, 300, 8, 1), (9, 257, 2, 1)])
+def test_fused_layer_matches_the_separate_operators(L_, K, H, G):
+    """Token biases gathered per workgroup (one to 128 tokens in it, rows that span workgroups) and all small parameters
+    converted in one launch, against the operators one by one; fp32, both orders of the same sums."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(L_ * K)
+    m = MultiHeadISSMScan(d_model=64, d_state=K, d_dist=16, nheads=H, ngroups=G, expand=1).cuda()
+    g = torch.Generator().manual_seed(K)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    args = (r(2, L_, 64), r(2, K, 64), r(2, L_, K, 16), r(2, L_, 3))
+    with torch.no_grad():
+        fused = m(*args)
+        m.fused = False
+        for a, b in zip(fused, m(*args)):
+            assert a.shape == b.shape and ((a - b).norm() / b.norm()).item() <= 1e-5
