@@ -336,6 +336,9 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_dw(DwConvP p) {
   float a0 = 0.0f, a1 = 0.0f;
   if (col < ncol) {
     int r = g;
+    // latency: the adds are a chain in a fixed order, but the loads of eight rounds travel together (12.2 -> 5.1 us at 8 x 1024
+    // tokens, 290 channels)
+#pragma unroll 8
     for (; r + 8 < p.nrows; r += 16) {
       a0 += p.partial[(long)r * ncol + col];
       a1 += p.partial[(long)(r + 8) * ncol + col];

@@ -504,6 +504,9 @@ __global__ __launch_bounds__(NTHREADS) void k_pgen_dw(PGenP p) {
   } else {
     const int R = p.H + 2 * p.G + (p.has_back ? 2 * p.G : 0), r = c - n;
     long t = threadIdx.x;
+    // latency: the adds are a chain in a fixed order, but the loads of eight rounds travel together (8.3 -> 6.9 us at 8192
+    // tokens)
+#pragma unroll 8
     for (; t + NTHREADS < p.tokens; t += 2 * NTHREADS) {
       a0 += p.dbias[t * R + r];
       a1 += p.dbias[(t + NTHREADS) * R + r];

