@@ -195,10 +195,16 @@ __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const 
     d[j] = in ? far : 0u;
     const float lx = -wave_fmax(in ? -px[j] : -INFV), ly = -wave_fmax(in ? -py[j] : -INFV), lz = -wave_fmax(in ? -pz[j] : -INFV);
     const float hx = wave_fmax(in ? px[j] : -INFV), hy = wave_fmax(in ? py[j] : -INFV), hz = wave_fmax(in ? pz[j] : -INFV);
-    const bool any = __ballot(in) != 0;
+    const unsigned long long members = __ballot(in);
+    // the group's best until a draw changes it: all members are equally far, so the smallest index.  (A group whose box is
+    // `far` or more from every draw is never looked at -- points 1e5 apart, infinite coordinates -- and is chosen as it is.)
+    const int l = lane_of_least(members, pos < n ? (int)order[pos] : 0x7fffffff);
+    const float x = lane_f(px[j], l), y = lane_f(py[j], l), z = lane_f(pz[j], l);
     if (lane == j) {
       blx = lx; bly = ly; blz = lz; bhx = hx; bhy = hy; bhz = hz;
-      gd = any ? far : 0u;
+      gd = members ? far : 0u;
+      gpos = (j * W + wave) * 64 + l;
+      gx = x; gy = y; gz = z;
     }
   });
   float ox = p[0], oy = p[1], oz = p[2];

@@ -46,7 +46,7 @@ def furthest_point_sampling(xyz, npoint):
         old = 0
         for s in range(1, npoint):
             d = _d2(p, p[old])
-            temp = np.where(live, np.minimum(temp, d), temp)
+            temp = np.where(live, np.fmin(temp, d), temp)   # (a distance that is no number changes nothing)
             cand = np.where(live, temp, np.float32(-1.0))
             old = int(np.argmax(cand)) if cand.max() > -1.0 else 0   # argmax returns the first maximum
             out[b, s] = old

@@ -62,6 +62,31 @@ def test_furthest_point_sampling_on_a_voxelized_cloud(n, npoint):
     assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
 
 
+@pytest.mark.parametrize("n", [64, 700, 5000, 24576])
+@pytest.mark.parametrize("kind", ["extent 1e6", "metres on a map", "infinite points", "first point no number"])
+def test_furthest_point_sampling_where_running_distances_never_come_below_their_start(n, kind):
+    """Squared distances of 1e10 and more leave every running distance at its start of 1e10: the smallest index is next, also
+    of a group of points that no draw comes near."""
+    from dest3d_amd.pointnet2_utils import furthest_point_sample
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(-4, 4, size=(2, n, 3)).astype(np.float32)
+    if kind == "extent 1e6":
+        xyz *= np.float32(2e5)
+    elif kind == "metres on a map":
+        xyz = (xyz * 100 + np.array([5e5, 4.2e6, 100.0])).astype(np.float32)
+        xyz[:, 0] = 0.0                     # a padding point first
+    elif kind == "infinite points":
+        xyz[0, n // 3:n // 3 + 9] = np.inf
+        xyz[1, n // 2:, 0] = -np.inf
+    else:
+        xyz[0, 0] = np.nan
+        xyz.view(np.uint32)[1, 0] = 0xffffffff
+    npoint = min(n, 64)
+    idx = furthest_point_sample(_cuda(xyz), npoint).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
+
+
 @pytest.mark.parametrize("seed,npoint", [(3, 1024), (8, 1024), (54, 1024)])
 def test_furthest_point_sampling_near_ties_go_the_way_of_plain_fp32_steps(seed, npoint):
     """Clouds in which two candidates' running minimum distances come within one unit in the last place of each other
