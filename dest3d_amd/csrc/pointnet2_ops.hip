@@ -832,14 +832,17 @@ __global__ __launch_bounds__(INV_T) void k_inverse_rank(int n, int m, const int*
     at += cnt[k];
   }
 }
-// list entry: point << 16 | target, weight.  Places behind the 3 n entries hold point 0, target 0 and weight 0.
+// list entry: point << 16 | target, weight.  Places behind the 3 n entries hold point NO_POINT, whose sum is never written
+// (a weight of 0 alone would not do: 0 times an infinite or undefined gradient is no number).
+constexpr unsigned NO_POINT = 0xffffu;
+static_assert(ROW_POINTS < (int)NO_POINT, "no point has this number");
 __global__ __launch_bounds__(NTHREADS) void k_inverse_fill(int n, int m, int per, const int* __restrict__ idx,
                                                            const float* __restrict__ weight, const int* __restrict__ start,
                                                            const int* __restrict__ rank, uint2* __restrict__ list) {
   const int b = blockIdx.y, e = blockIdx.x * NTHREADS + threadIdx.x;
   if (e >= per * INV_T) return;
   int at = e;
-  uint2 v = make_uint2(0u, 0u);
+  uint2 v = make_uint2(NO_POINT << 16, 0u);
   if (e < 3 * n) {
     const int k = index_of(idx[(long)b * n * 3 + e], m);
     at = start[(long)b * m + k] + rank[(long)b * n * 3 + e];
@@ -865,8 +868,9 @@ __global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m,
   float acc[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-  unsigned cur = per ? q[0].x >> 16 : 0u;
+  unsigned cur = per ? q[0].x >> 16 : NO_POINT;
   auto put = [&]() {
+    if (cur == NO_POINT) return;
 #pragma unroll
     for (int r = 0; r < R; ++r)
       if (r < nch) unsafeAtomicAdd(o + (long)r * m + cur, acc[r]);

@@ -259,6 +259,29 @@ def test_interpolation_rows(c, m, n):
     assert np.abs(f.grad.cpu().numpy() - gref).max() <= 1e-5 * np.abs(gref).max()
 
 
+@pytest.mark.parametrize("c,m,n", [(300, 50, 3501), (700, 3, 5121), (220, 900, 9999), (60, 1000, 40960)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_interpolation_rows_keep_a_target_without_a_number_to_its_points(c, m, n, value):
+    """Target 0's gradient is no number (ordinary under loss scaling): its own three points get it, the others nothing of it.
+    Four, two and one row per workgroup, and list lengths that fill no workgroup's share."""
+    from dest3d_amd.pointnet2_utils import three_interpolate
+    rng = np.random.default_rng(n)
+    idx = rng.integers(0, m, size=(2, n, 3)).astype(np.int32)
+    idx[:, 0] = m - 1
+    idx[:, 1:][idx[:, 1:] == m - 1] = 0
+    w = rng.uniform(0.1, 1, size=(2, n, 3)).astype(np.float32)
+    f = _cuda(rng.standard_normal((2, c, m)).astype(np.float32)).requires_grad_()
+    y = three_interpolate(f, _cuda(idx), _cuda(w))
+    gy = rng.standard_normal(y.shape).astype(np.float32)
+    gy[:, :, 0] = value
+    y.backward(_cuda(gy))
+    g = f.grad.cpu().numpy()
+    assert (np.isnan(g[..., m - 1]) if np.isnan(value) else np.isposinf(g[..., m - 1])).all()
+    gy[:, :, 0] = 0.0
+    ref = R.three_interpolate_grad(gy, idx, w, m)[..., :m - 1]
+    assert np.abs(g[..., :m - 1] - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("m", [255, 256, 257, 2048, 8192, 8193])
 def test_three_nn_grid(m):
     """Both sides of the grid's range; sample 1: a flat sheet with duplicates (ties go to the smaller index), clusters and far
