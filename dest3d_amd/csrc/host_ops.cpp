@@ -764,6 +764,27 @@ struct CoreFn : public Function<CoreFn> {
   }
 };
 
+// What lies between the input projections and the output projections (dest_module.py:528-581): zx (B, L, 2 d_inner + 2 G + H)
+// from key_proj, h0 (B, K, d_inner) from query_proj -> the normalised key and the averaged final states.
+void check_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const Tensor& weights) {
+  require_gpu(zx, "in_key");
+  require(zx.dim() == 3 && h0.dim() == 3 && dist.dim() == 4, "in_key (B, L, D), in_query (B, K, D), dist (B, L, K, M)");
+  require(dist.size(0) == zx.size(0) && dist.size(1) == zx.size(1) && h0.size(0) == zx.size(0) && dist.size(2) == h0.size(1) &&
+              dist.size(3) == WIDTH, "dist must be (B, L, K, 16)");
+  if (weights.defined()) require(weights.sizes() == dist.sizes().slice(0, 3), "mask must be (B, L, K)");
+}
+
+std::vector<Tensor> scan_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const MaybeTensor& weights_,
+                              const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b, const Tensor& conv_b_b,
+                              const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias, const Tensor& A_log, const Tensor& D,
+                              const Tensor& key_norm, double key_eps, int64_t d_inner, int64_t nheads, int64_t ngroups, double lo,
+                              double hi) {
+  check_core(zx, h0, dist, opt(weights_));
+  py::gil_scoped_release release;
+  return CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, key_norm,
+                       d_inner, nheads, ngroups, lo, hi, key_eps);
+}
+
 // MultiHeadISSMScan.forward as a whole (dest_module.py:515-585) for the configuration CoreFn is built for.
 std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, const Tensor& dist, const MaybeTensor& weights_,
                                const Tensor& key_proj, const Tensor& query_proj, const Tensor& out_key_proj,
@@ -772,12 +793,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                const Tensor& A_log, const Tensor& D, const Tensor& key_norm, double key_eps,
                                const MaybeTensor& query_w, const MaybeTensor& query_b, double query_eps,
                                int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
-  require_gpu(in_key, "in_key");
-  require(in_key.dim() == 3 && in_query.dim() == 3 && dist.dim() == 4, "in_key (B, L, D), in_query (B, K, D), dist (B, L, K, M)");
-  require(dist.size(0) == in_key.size(0) && dist.size(1) == in_key.size(1) && in_query.size(0) == in_key.size(0) &&
-              dist.size(2) == in_query.size(1) && dist.size(3) == WIDTH, "dist must be (B, L, K, 16)");
-  const Tensor weights = opt(weights_);
-  if (weights.defined()) require(weights.sizes() == dist.sizes().slice(0, 3), "mask must be (B, L, K)");
+  check_core(in_key, in_query, dist, opt(weights_));
   py::gil_scoped_release release;
   const Tensor zx = linear_tokens(in_key, key_proj), h0 = linear_tokens(in_query, query_proj);
   variable_list core = CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
@@ -796,5 +812,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::gil_scoped_release release;
     return linear_tokens(x, w);
   });
+  m.def("scan_core", &scan_core);
   m.def("scan_layer", &scan_layer);
 }

@@ -317,3 +317,42 @@ def test_fused_layer_matches_the_separate_operators(L_, K, H, G):
         m.fused = False
         for a, b in zip(fused, m(*args)):
             assert a.shape == b.shape and ((a - b).norm() / b.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("which", ["forward pre", "forward", "backward pre", "backward", "all modules", "replaced forward"])
+@pytest.mark.parametrize("name", ["query_norm", "out_query_proj", "key_proj"])
+def test_hooks_of_the_layers_modules_act(which, name):
+    """The layer reads weights where calling a module would do nothing else; a hook is something else."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(5)
+    m = MultiHeadISSMScan(d_model=64, d_state=9, d_dist=16, nheads=2, expand=1).cuda()
+    mod, seen = getattr(m, name), []
+    note = lambda *a: seen.append(a[0])
+    if which == "forward pre":
+        h = mod.register_forward_pre_hook(note)
+    elif which == "forward":
+        h = mod.register_forward_hook(note)
+    elif which == "backward pre":
+        h = mod.register_full_backward_pre_hook(note)
+    elif which == "backward":
+        h = mod.register_full_backward_hook(note)
+    elif which == "all modules":
+        h = torch.nn.modules.module.register_module_forward_hook(note)
+    else:
+        plain = mod.forward
+        mod.forward = lambda x: (note(mod), plain(x))[1]
+        h = None
+    g = torch.Generator().manual_seed(6)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    ins = (r(1, 70, 64).requires_grad_(), r(1, 9, 64).requires_grad_(), r(1, 70, 9, 16), r(1, 70, 3))
+    try:
+        a = m(*ins)
+        (a[0].sum() + a[1].square().sum()).backward()
+    finally:
+        if h is not None:
+            h.remove()
+    assert mod in seen, "the hook was passed by"
+    if h is None:
+        mod.forward = plain
+    for x, y in zip(a, m(*ins)):
+        assert ((x - y).norm() / y.norm()).item() <= 1e-5
