@@ -116,9 +116,12 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
 }
 
 // FULLP: the head dimension fills its tiles.  EDGE: chunks with fewer than 64 rows and steps with fewer than 64 columns
-// exist (N >= 4).  A lane's rows past the end read the chunk's last one and get dt' = 0, as do whole lanes past the last
+// may exist (N >= 4).  A lane's rows past the end read the chunk's last one and get dt' = 0, as do whole lanes past the last
 // column; a lane whose four columns cross it works on columns N - 4 .. N - 1 instead, those its neighbour owns with dt' = 0
-// and not stored.
+// and not stored.  The diagonal blocks of M take fp32 matrix instructions: the level form, which evaluates such calls
+// wherever this kernel cannot, has the pairs inside groups of four rows in fp32, and what a pair is computed in is not to
+// depend on the kernel.  (Those entries of M: 2.4e-3 from float64 with operands rounded once to bf16, 4.4e-6 as bf16 pairs,
+// 2.6e-7 like this.  4 x 1000 tokens, heads of 36, 200 states, fp32, forward + backward: 221.6 us with pairs, 222.4 like this.)
 template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
@@ -302,7 +305,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
         W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
         V[r] = W[r] * et[k];
       }
-      {
+      if constexpr (EDGE) {  // fp32 matrix instructions: k-slot kg of instruction r <-> the lane's column r
+#pragma unroll
+        for (int r = 0; r < 4; ++r) macc[J] = mfma4(cv[4 * J + r] * up[4 * J + r], W[r], macc[J]);
+      } else {
         const Fr f = make_frag<SPLIT>(W[0], W[1], W[2], W[3]);
         macc[J] = frag_product<SPLIT>(U[J], f, macc[J]);
       }
@@ -413,8 +419,14 @@ static int set_lds_tile(K kernel, size_t bytes) {
 int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
   const int units = p.B * p.ndir * p.nc * p.H;
   const int pt = (p.P + 15) / 16;
-  // aligned 16-byte stores of the states and decay totals need rows of a multiple of four floats: they have them where
-  // the tiles are complete
+  // EDGE unless every tile is complete and every operand starts its rows at a multiple of four elements (16-byte stores of
+  // the states and decay totals; operands elsewhere belong to the calls the level form's precision is kept for, see EDGE)
+  auto rows_of_four = [](const TensorD& t, int bf) {
+    return ((t.s0 | t.s1 | t.s2) & 3) == 0 && ((uintptr_t)t.ptr & (bf ? 7 : 15)) == 0;
+  };
+  bool edge = !p.full_tiles || !rows_of_four(p.dt, p.dt_dt) ||
+              (((uintptr_t)states | (uintptr_t)cs_last | (uintptr_t)p.A | (uintptr_t)p.dt_bias) & 15);
+  for (int d = 0; d < p.ndir; ++d) edge = edge || !rows_of_four(p.Bm[d], p.io_dt) || !rows_of_four(p.Cm[d], p.io_dt);
 #define ISSM_LT_ONE(PT_, IOB_, DTB_, FULLP_, EDGE_)                                                         \
   {                                                                                                         \
     constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, FULLP_, EDGE_>;                                    \
@@ -424,7 +436,7 @@ int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, h
 #define ISSM_LT(PT_, IOB_, DTB_)                                                                            \
   {                                                                                                         \
     const size_t sm = fwd_tile_lds<PT_, !IOB_>();                                                           \
-    if (!p.full_tiles || ((uintptr_t)states & 15) || ((uintptr_t)cs_last & 15)) ISSM_LT_ONE(PT_, IOB_, DTB_, false, true) \
+    if (edge) ISSM_LT_ONE(PT_, IOB_, DTB_, false, true)                                                     \
     else if (p.P == 16 * PT_) ISSM_LT_ONE(PT_, IOB_, DTB_, true, false)                                     \
     else ISSM_LT_ONE(PT_, IOB_, DTB_, false, false)                                                         \
   }

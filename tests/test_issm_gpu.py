@@ -173,6 +173,40 @@ def test_rows_and_columns_that_fill_no_tile_in_both_directions(dtype, L_, N, P, 
         _check("d" + k, gi[k].grad, ref[k].grad, bwd)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,P,offset", [(100, 70, 16, 0), (130, 128, 36, 0), (128, 200, 48, 0), (67, 5, 64, 0), (128, 64, 32, 1)])
+def test_close_pairs_of_incomplete_tiles_are_evaluated_in_fp32(dtype, L_, N, P, offset):
+    """Entries of M whose rows lie in one group of four, where rows or columns are missing or (offset) operands start off a
+    multiple of four elements: no operand is rounded to 16 bits or to a pair of them.  Bound: the decay's exponent is a
+    difference of running sums of at most 16 rows, here below 16 (half a unit in the last place 4.8e-7), and every entry is a sum of
+    N fp32 products; pairs of bf16 numbers give 4e-6, single ones 2.4e-3."""
+    from dest3d_amd import _lib as L
+    from dest3d_amd.issm_combined import _Problem
+    d = _problem(2, L_, 2, P, N, 1, seed=N + P)
+    d["A"] *= 0.25
+    for k in ("x", "dt", "B", "C"):
+        d[k] = d[k].to(dtype).float()
+    ref = R.issm_bwd_closed_form(d["x"], d["dt"], d["A"], d["B"], d["C"], 64, d["dy"], D=d["D"], dt_bias=d["dt_bias"],
+                                 initial_states=d["h0"], dt_softplus=True, dt_limit=d["dt_limit"], intermediates=True)["M"]
+    shift = lambda t: torch.cat([torch.zeros(offset, dtype=t.dtype), t.flatten()]).cuda()[offset:].view(t.shape)
+    t = {k: shift(d[k].to(dtype)) for k in ("x", "dt", "B", "C")}
+    prob = _Problem([t["x"]], t["dt"], d["A"].cuda(), [t["B"]], [t["C"]], 64, d["D"].cuda(), [None], d["dt_bias"].cuda(),
+                    d["h0"].cuda(), None, True, d["dt_limit"])
+    a, nc = prob.args(), math.ceil(L_ / 64)
+    f = lambda *s: torch.full(s, float("nan"), device="cuda")
+    states, cs_last, m = f(2, nc + 1, 2, P, N), f(2, nc, 2, N), f(2, nc, 2, 64, 64)
+    L.check(L.load().issm_stage_chunk_local(C.byref(a), states.data_ptr(), cs_last.data_ptr(), m.data_ptr()), "local")
+    torch.cuda.synchronize()
+    row = torch.arange(64)
+    close = (row[:, None] // 4 == row[None] // 4) & (row[:, None] >= row[None])
+    there = torch.arange(64 * nc).view(nc, 64) < L_
+    pick = (close & there[:, :, None])[None, :, None].expand(2, nc, 2, 64, 64)
+    got, want = m.cpu().double()[pick], ref.double()[pick]
+    err = ((got - want).norm() / want.norm()).item()
+    print(f"    close pairs rel_l2={err:.3e}", flush=True)
+    assert err <= 1e-6
+
+
 @pytest.mark.parametrize("P", [128, 96, 67])
 def test_head_dimension_above_the_tile_limit(P):
     """Heads wider than the kernels' 64 run as several narrower heads that share dt, A, dt_bias and the group's B, C
