@@ -15,13 +15,15 @@
 // iup grows like 2^(decay across one tile), so the form is only used where every tile's sum stays within SPAN_LIMIT
 // (|tt| <= 96: operands below 2^96, no overflow before the factors meet).  A head of a workgroup where some column
 // exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
-// (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands: bf16 inputs -> one bf16 instruction
-// per block, operands rounded once; in launches with incomplete tiles the diagonal blocks take operands as (hi, lo) pairs
-// instead (the level form, which evaluated those launches before, keeps close pairs of rows in fp32: this one is not to be
-// less accurate; pairs for every block spill 300 bytes a lane and take twice the time).  fp32
-// inputs -> operands rounded to 17 significand bits and split exactly into (hi, lo) bf16 pairs, a.b = (ah.bl + al.bh) +
-// (ah.bh + al.bl), each bracket one K = 32 instruction.  d/d(cs) is formed as (operand as the matrix instruction took it) x
-// (product) on both rows of a pair, so the two entries of a pair cancel to fp32 rounding in the suffix sums.
+// (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands, complete tiles: bf16 inputs -> one bf16
+// instruction per block, operands rounded once; fp32 inputs -> operands rounded to 17 significand bits and split exactly into
+// (hi, lo) bf16 pairs, a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, and a
+// gated dy: the level form evaluates these calls wherever this kernel cannot, close pairs of rows (bf16 inputs) or all pairs
+// (fp32 inputs) from fp32 operands, and what a pair is computed in is not to depend on the kernel.  So the diagonal blocks
+// (bf16 inputs) or all blocks (fp32 inputs) are fp32 matrix instructions there.  That costs less than it saves: no operand is
+// split, and the 90 - 130 bytes a lane that the pairs of the incomplete form spilled are gone.  d/d(cs) is formed as (operand
+// as the matrix instruction took it) x (product) on both rows of a pair, so the two entries of a pair cancel to fp32 rounding
+// in the suffix sums.
 //
 // Built for x / dout rows that allow 8- / 16-byte accesses, x / B / C and dt of one type, no packed sequences, and for bf16
 // inputs no z gate; every other call takes the level-hierarchy kernel alone.  That is what lets the kernel issue every
@@ -29,10 +31,9 @@
 // point and waits for exactly the ones it needs (a load inside a branch, even a uniform one, makes the compiler wait for
 // all outstanding loads at the join).  Incomplete tiles (FULL = false) run the same code: rows past the end are read through
 // a buffer whose bounds check returns zero, columns past the end read column 0 and have dt' = 0, stores are guarded in the
-// workgroups that have such rows or columns. 8 x 1024 tokens, 8 heads
-// x 32, one direction, N = 250: 108 us fp32, 87 us bf16 (N = 256: 88 and 59 us; the difference is registers, 90 - 130 bytes a
-// lane spill in the incomplete form).  With the other kernels' edge forms the whole forward + backward went from 462 to
-// 347 us (fp32) and from 406 to 277 us (bf16).
+// workgroups that have such rows or columns.  8 x 1024 tokens, 8 heads x 32, one direction: N = 250 104 us fp32, 83 us bf16
+// (107 and 86 with operand pairs, 147 and 111 in the level form; N = 256: 88 and 59 us); N = 256 with a gated dy, fp32: 99 us
+// (88 with operand pairs, 122 in the level form).
 #include "issm_dev.h"
 
 namespace issm {
@@ -46,7 +47,10 @@ struct BwdTileSmem {
   static constexpr int NH = SPLIT ? 2 : 1;          // hi (and lo) copies
   uint16_t xs[NH * CS * LDP];
   uint16_t dys[NH * CS * LDP];
-  uint16_t tm[NH * CS * LDM];
+  alignas(16) uint16_t tm[NH * CS * LDM];
+  static constexpr int LDF = CS + 4;                // the same matrix in fp32 (fp32 inputs, incomplete tiles)
+  static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
+  __device__ __forceinline__ float* tf() { return reinterpret_cast<float*>(tm); }
   float dbc[32 * NTHREADS];  // per-lane dB / dC accumulators [k][tid]
   // bf16 inputs, two head tiles: the group's B and C values of every lane, packed in pairs, [i][tid] (i < 8: B, then C).
   // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
@@ -70,7 +74,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
                                                           const float* __restrict__ g_last, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo) {
   constexpr bool SPLIT = !IOB;
-  constexpr bool DIAG2 = IOB && !FULL;  // operands of the diagonal blocks as (hi, lo) pairs
+  constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && !FULL;  // fp32 products in the diagonal blocks / in all blocks
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdTileSmem<PT, SPLIT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
@@ -188,11 +192,30 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       asm volatile("" : "+v"(tq));
       const int mrow = tq >> 3, mcol = (tq & 7) * 8;
       constexpr int G4 = 4 * PT;
-      *(uint4*)(s.tm + mrow * LDM + mcol) = l_th0;
-      *(uint4*)(s.tm + (32 + mrow) * LDM + mcol) = l_th1;
+      if constexpr (ALL32) {  // T = hi + lo as fp32 numbers
+        auto put = [&](int row, uint4 h, uint4 l) {
+          const unsigned a[4] = {h.x, h.y, h.z, h.w}, b[4] = {l.x, l.y, l.z, l.w};
+          f4 v[2];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[i >> 1][(2 * i) & 3] = __uint_as_float(a[i] << 16) + __uint_as_float(b[i] << 16);
+            v[i >> 1][(2 * i + 1) & 3] = __uint_as_float(a[i] & 0xffff0000u) + __uint_as_float(b[i] & 0xffff0000u);
+          }
+          f4* d = (f4*)(s.tf() + row * SM::LDF + mcol);
+          d[0] = v[0];
+          d[1] = v[1];
+        };
+        put(mrow, l_th0, l_tl0);
+        put(32 + mrow, l_th1, l_tl1);
+      } else {
+        *(uint4*)(s.tm + mrow * LDM + mcol) = l_th0;
+        *(uint4*)(s.tm + (32 + mrow) * LDM + mcol) = l_th1;
+        if constexpr (SPLIT) {
+          *(uint4*)(s.tm + CS * LDM + mrow * LDM + mcol) = l_tl0;
+          *(uint4*)(s.tm + CS * LDM + (32 + mrow) * LDM + mcol) = l_tl1;
+        }
+      }
       if constexpr (SPLIT) {
-        *(uint4*)(s.tm + CS * LDM + mrow * LDM + mcol) = l_tl0;
-        *(uint4*)(s.tm + CS * LDM + (32 + mrow) * LDM + mcol) = l_tl1;
 #pragma unroll
         for (int i = 0; i < PT; ++i) {
           const int e4 = tq + i * NTHREADS, o = (e4 / G4) * LDP + (e4 % G4) * 4;
@@ -260,9 +283,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       auto unpk = [](const unsigned (&a)[8], int k) {
         return __uint_as_float((k & 1) ? (a[k >> 1] & 0xffff0000u) : (a[k >> 1] << 16));
       };
+      auto wide = [](uint2 a) -> f4 {  // four bf16 numbers
+        return (f4){__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u), __uint_as_float(a.y << 16),
+                    __uint_as_float(a.y & 0xffff0000u)};
+      };
       auto half_of = [](unsigned w, int k) { return __uint_as_float((k & 1) ? (w & 0xffff0000u) : (w << 16)); };
       // Cu = C up (operand of the G blocks), Bi = B dt' iup (operand of the F blocks)
       bf4 Ch[4], Bh[4], Cl[4], Bl[4];
+      float cf32[ALL32 ? 16 : 1], bf32[ALL32 ? 16 : 1];
 #pragma unroll
       for (int J = 0; J < 4; ++J)
 #pragma unroll
@@ -275,6 +303,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           } else {  // out of the workgroup's LDS copy of the group's B and C
             cu = half_of(s.bc[(8 + (k >> 1)) * NTHREADS + tid], k) * up[k];
             bi = half_of(s.bc[(k >> 1) * NTHREADS + tid], k) * dtp[k] * iup[k];
+          }
+          if constexpr (ALL32) {
+            cf32[k] = cu;
+            bf32[k] = bi;
+            continue;
           }
           if (SPLIT) {
             cu = round17(cu);
@@ -291,7 +324,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       // to a register
       unsigned bvp[8], cvp[8];
       float bvf[SPLIT ? 16 : 1];
-      if constexpr (BCL && DIAG2) {  // read tile by tile below
+      if constexpr (BCL && DIAG32) {  // read tile by tile below
       } else if constexpr (BCL) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -349,10 +382,22 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       };
 
-      auto block_pair = [&](uint2 ah, bf4 bh, bf4 bl) -> f4 {  // a . (bl + bh)
-        const f4 z = {0, 0, 0, 0};
-        const bf4 a_h = __builtin_bit_cast(bf4, ah);
-        return mfma_bf(cat_bf4(a_h, a_h), cat_bf4(bl, bh), z);
+      auto block32 = [&](f4 a, const float* op) -> f4 {  // fp32: k-slot g4 of instruction j <-> row / column 4 g4 + j
+        f4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = mfma4(a[j], op[j], acc);
+        return acc;
+      };
+      // the diagonal block's entries on or before (F) / on or after (G) the diagonal, for the lane's columns 4 g4 + j
+      auto upto = [&](f4 a) -> f4 {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = 4 * gq + j <= cq ? a[j] : 0.0f;
+        return a;
+      };
+      auto from = [&](f4 a) -> f4 {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = 4 * gq + j >= cq ? a[j] : 0.0f;
+        return a;
       };
 
       // ---- tile by tile: the state terms of the lane's four rows of tile R, the blocks of F and G that end in them,
@@ -361,9 +406,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
       for (int R = 0; R < 4; ++R) {
         f4 xf = {0, 0, 0, 0}, xg = {0, 0, 0, 0};  // the blocks' sums
-        f4 df = {0, 0, 0, 0}, dg = {0, 0, 0, 0};  // DIAG2: those of the diagonal block
-        bf4 cl = {}, bl = {};                     // DIAG2: what the operands of rows 16 R + 4 g4 + j lost to bf16
-        if constexpr (DIAG2) {
+        f4 df = {0, 0, 0, 0}, dg = {0, 0, 0, 0};  // DIAG32: those of the diagonal block
+        float cd[4], bd[4];                       // DIAG32: the operands of rows 16 R + 4 g4 + j
+        if constexpr (DIAG32) {
           if constexpr (BCL)
 #pragma unroll
             for (int i = 2 * R; i < 2 * R + 2; ++i) {
@@ -373,8 +418,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int k = 4 * R + j;
-            cl[j] = (__bf16)(unpk(cvp, k) * up[k] - (float)Ch[R][j]);
-            bl[j] = (__bf16)(unpk(bvp, k) * dtp[k] * iup[k] - (float)Bh[R][j]);
+            cd[j] = unpk(cvp, k) * up[k];
+            bd[j] = unpk(bvp, k) * dtp[k] * iup[k];
           }
         }
         f4 sf, sg;                                // the state terms
@@ -404,42 +449,62 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
             sf[rr] = R == 0 ? r[rr] : E[R][0] * r[rr];
           }
         }
-        uint2 th[4], tl[4];
-        const uint16_t* row = tm_ + (16 * R + cq) * LDM + 4 * gq;
+        if constexpr (ALL32) {
+          const float* row = s.tf() + (16 * R + cq) * SM::LDF + 4 * gq;
+          f4 t[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          th[c] = *(const uint2*)(row + 16 * c);
-          if (SPLIT) tl[c] = *(const uint2*)(row + CS * LDM + 16 * c);
-          else tl[c] = make_uint2(0u, 0u);
-        }
+          for (int c = 0; c < 4; ++c) t[c] = *(const f4*)(row + 16 * c);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          if (c <= R) {  // F block (R, c)
-            uint2 ah = th[c], al = tl[c];
-            if (c == R) {
-              ah.x &= mf[0]; ah.y &= mf[1];
-              al.x &= mf[0]; al.y &= mf[1];
-            }
-            if (DIAG2 && c == R) {
-              df = block_pair(ah, Bh[c], bl);
-            } else {
-              const f4 acc = block(ah, al, Bh[c], Bl[c]);
+          for (int c = 0; c < 4; ++c) {
+            if (c <= R) {  // F block (R, c)
+              const f4 acc = block32(c == R ? upto(t[c]) : t[c], bf32 + 4 * c);
 #pragma unroll
               for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
             }
-          }
-          if (c >= R) {  // G block (c, R)
-            uint2 ah = th[c], al = tl[c];
-            if (c == R) {
-              ah.x &= mg[0]; ah.y &= mg[1];
-              al.x &= mg[0]; al.y &= mg[1];
-            }
-            if (DIAG2 && c == R) {
-              dg = block_pair(ah, Ch[c], cl);
-            } else {
-              const f4 acc = block(ah, al, Ch[c], Cl[c]);
+            if (c >= R) {  // G block (c, R)
+              const f4 acc = block32(c == R ? from(t[c]) : t[c], cf32 + 4 * c);
 #pragma unroll
               for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
+            }
+          }
+        } else {
+          uint2 th[4], tl[4];
+          const uint16_t* row = tm_ + (16 * R + cq) * LDM + 4 * gq;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            th[c] = *(const uint2*)(row + 16 * c);
+            if (SPLIT) tl[c] = *(const uint2*)(row + CS * LDM + 16 * c);
+            else tl[c] = make_uint2(0u, 0u);
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            if (c <= R) {  // F block (R, c)
+              uint2 ah = th[c], al = tl[c];
+              if (c == R) {
+                ah.x &= mf[0]; ah.y &= mf[1];
+                al.x &= mf[0]; al.y &= mf[1];
+              }
+              if (DIAG32 && c == R) {
+                df = block32(upto(wide(th[c])), bd);
+              } else {
+                const f4 acc = block(ah, al, Bh[c], Bl[c]);
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
+              }
+            }
+            if (c >= R) {  // G block (c, R)
+              uint2 ah = th[c], al = tl[c];
+              if (c == R) {
+                ah.x &= mg[0]; ah.y &= mg[1];
+                al.x &= mg[0]; al.y &= mg[1];
+              }
+              if (DIAG32 && c == R) {
+                dg = block32(from(wide(th[c])), cd);
+              } else {
+                const f4 acc = block(ah, al, Ch[c], Cl[c]);
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
+              }
             }
           }
         }
@@ -456,13 +521,15 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           s.dbc[k * NTHREADS + tid] += dtp[k] * E1;
           s.dbc[(16 + k) * NTHREADS + tid] += X2;
           val[k] = bv * E1;
-          if constexpr (SPLIT) {
+          if constexpr (ALL32) {
+            dcs[k] = cf32[k] * (xf[rr] + sf[rr]) - bf32[k] * (xg[rr] + sg[rr]);
+          } else if constexpr (SPLIT) {
             const float c16 = (float)Ch[R][rr] + (float)Cl[R][rr], b16 = (float)Bh[R][rr] + (float)Bl[R][rr];
             dcs[k] = c16 * (xf[rr] + sf[rr]) - b16 * (xg[rr] + sg[rr]);
           } else {
             const float c16 = (float)Ch[R][rr], b16 = (float)Bh[R][rr];
             float pairs = c16 * xf[rr] - b16 * xg[rr];
-            if constexpr (DIAG2) pairs += (c16 + (float)cl[rr]) * df[rr] - (b16 + (float)bl[rr]) * dg[rr];
+            if constexpr (DIAG32) pairs += cd[rr] * df[rr] - bd[rr] * dg[rr];
             dcs[k] = pairs + (unpk(cvp, k) * up[k] * sf[rr] - bv * dtp[k] * iup[k] * sg[rr]);
           }
         }
@@ -617,6 +684,7 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
     t.s1 = (long)p.H * p.P;
     t.s0 = (long)p.ndir * p.L * p.H * p.P;
     t.ptr = dy_ws + (long)p.dir0 * p.L * p.H * p.P;
+    p.full_tiles = 0;   // the variants with fp32 products, see the head of this file
   }
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   const int pt = (p.P + 15) / 16;

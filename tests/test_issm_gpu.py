@@ -207,6 +207,43 @@ def test_close_pairs_of_incomplete_tiles_are_evaluated_in_fp32(dtype, L_, N, P, 
     assert err <= 1e-6
 
 
+@pytest.mark.parametrize("L_,N,P,gated", [(100, 70, 16, False), (130, 128, 36, False), (128, 200, 48, False), (67, 5, 24, False),
+                                           (128, 128, 32, True), (70, 66, 36, True)])
+def test_tile_and_level_form_of_the_chunk_backward_agree_to_fp32(L_, N, P, gated):
+    """fp32 inputs, incomplete tiles or a gated dy: the tile-base kernel (with a list of heads to redo) against the level
+    form (without one), both from fp32 operands on fp32 matrix instructions; pairs of rows alone (states and their gradients
+    are zero).  Exponents are differences of running sums below 32 (half a unit in the last place 9.5e-7, times ln 2, for a
+    few of the pairs); operands rounded to 17 bits give 2e-6."""
+    d = _problem(2, L_, 4, P, N, 2, seed=N + P)
+    d["A"] *= 0.25
+    L, prob, a = _stage_args(d)
+    lib, nc, B, H, G = L.load(), math.ceil(L_ / 64), 2, 4, 2
+    f = lambda *s: torch.full(s, float("nan"), device="cuda")
+    g = torch.Generator().manual_seed(P)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    dy, w = d["dy"].cuda(), r(B, nc, H, 64, 64)
+    states, dst, g_next = (torch.zeros(s, device="cuda") for s in ((B, nc + 1, H, P, N), (B, nc, H, P, N), (B, nc, H, N)))
+    a.dout[0] = L.tensor_desc(dy)
+    w = torch.tril(w) + torch.tril(w, -1).transpose(-1, -2)
+    hi = w.bfloat16()
+    dm = torch.stack([hi, (w - hi.float()).bfloat16()], dim=3).contiguous()
+    out = []
+    for redo in (None, torch.full((lib.issm_bwd_chunk_redo_ints(C.byref(a)),), -1, dtype=torch.int32, device="cuda")):
+        t = [f(B, L_, H, N), f(B, L_, G, N), f(B, L_, G, N), f(B * nc, H, N), f(B * nc, H, N)]
+        a.ddt, a.dB[0], a.dC[0] = (L.tensor_desc(q) for q in t[:3])
+        L.check(lib.issm_stage_bwd_chunk(C.byref(a), 0, dy.data_ptr() if gated else None, states.data_ptr(), dst.data_ptr(),
+                                         dm.data_ptr(), g_next.data_ptr(), t[3].data_ptr(), t[4].data_ptr(),
+                                         None if redo is None else redo.data_ptr()), "bwd_chunk")
+        torch.cuda.synchronize()
+        out.append(t)
+    assert (redo == 0).all()
+    for n_, x, y in zip(("ddt", "dB", "dC", "partA", "partBias"), out[1], out[0]):
+        l2 = ((x.double() - y.double()).norm() / y.double().norm()).item()
+        print(f"    {n_:9s} rel_l2={l2:.3e}", flush=True)
+        if n_ in ("dB", "dC"):
+            assert l2 <= 7e-7
+
+
 @pytest.mark.parametrize("P", [128, 96, 67])
 def test_head_dimension_above_the_tile_limit(P):
     """Heads wider than the kernels' 64 run as several narrower heads that share dt, A, dt_bias and the group's B, C
