@@ -102,7 +102,7 @@ struct FwdWs {
   size_t states, cs_last, cabt, out_x, total;  // offsets in floats
 };
 struct BwdWs {
-  size_t dstates, dm, g_last, dh0_dir, partA, partBias, partD, redo, dy_ws, ddt_part, total;
+  size_t dstates, dm, g_last, dh0_dir, partA, partBias, partD, redo, dy_ws, ddt_part, dbc_part, total;
 };
 
 static int nchunks(const issm_dims& d) { return (d.seqlen + ISSM_CHUNK - 1) / ISSM_CHUNK; }
@@ -119,8 +119,13 @@ static FwdWs fwd_layout(const issm_dims& d, bool has_z) {
   return w;
 }
 
-// ddt_part: with two directions and a bf16 ddt, the first direction's share of ddt in fp32 ((B, L, H, N))
-static BwdWs bwd_layout(const issm_dims& d, bool has_z, bool ddt_part) {
+static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
+// Partial sums that would be rounded to bf16 on their way between kernels: with two directions and a bf16 ddt the first
+// direction's share of ddt in fp32 ((B, L, H, N)), with bf16 inputs and incomplete
+// tiles dB and dC of workgroups two kernels share (KP::dbc_part).
+static BwdWs bwd_layout(const issm_scan_args* a) {
+  const issm_dims& d = a->dims;
+  const bool has_z = a->z[0].ptr != nullptr, ddt_part = wants_ddt_part(a);
   const size_t Bt = (size_t)d.batch * d.ndir, nc = nchunks(d), H = d.nheads, P = d.headdim, N = d.dstate;
   BwdWs w;
   size_t o = 0;
@@ -133,11 +138,12 @@ static BwdWs bwd_layout(const issm_dims& d, bool has_z, bool ddt_part) {
   w.partD = o; o += align64(Bt * nc * H * P);
   w.redo = o; o += align64(Bt * nc * H * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK));  // one int per direction, workgroup and head
   w.dy_ws = o; if (has_z) o += align64(Bt * d.seqlen * H * P);
+  w.dbc_part = o;
+  if (a->io_dtype == ISSM_BF16 && (N % 64 || d.seqlen % ISSM_CHUNK)) o += Bt * nc * d.ngroups * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK) * 2 * ISSM_CHUNK * ISSM_CHUNK;
   w.ddt_part = o; if (ddt_part) o += align64((size_t)d.batch * d.seqlen * H * N);
   w.total = o;
   return w;
 }
-static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
 
 static int check_dims(const issm_scan_args* a) {
   if (!a) return fail(ISSM_E_NULL, "args is NULL");
@@ -266,7 +272,7 @@ int issm_bwd_workspace_bytes(const issm_scan_args* a, size_t* out) {
   int rc = check_dims(a);
   if (rc) return rc;
   if (!out) return fail(ISSM_E_NULL, "out is NULL");
-  *out = bwd_layout(a->dims, a->z[0].ptr != nullptr, wants_ddt_part(a)).total * sizeof(float);
+  *out = bwd_layout(a).total * sizeof(float);
   return ISSM_OK;
 }
 
@@ -403,7 +409,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
   if (rc) return rc;
   const bool has_z = a->z[0].ptr != nullptr;
   const FwdWs fw = fwd_layout(a->dims, has_z);
-  const BwdWs bw = bwd_layout(a->dims, has_z, wants_ddt_part(a));
+  const BwdWs bw = bwd_layout(a);
   if (!a->saved) return fail(ISSM_E_WORKSPACE, "saved forward workspace is NULL");
   if (!a->bwd_workspace || a->bwd_workspace_bytes < bw.total * sizeof(float))
     return fail(ISSM_E_WORKSPACE, "backward workspace: need %zu bytes, got %zu", bw.total * sizeof(float),
@@ -434,6 +440,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
     pc.ddt_part.s1 = (long)p.H * p.N;
     pc.ddt_part.s0 = (long)p.L * p.H * p.N;
   }
+  if (p.io_dt && !p.full_tiles && bwd_tile_available(p, dy)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
   for (int dir = 0; dir < p.ndir; ++dir) {
     KP pd = pc;
     pd.dir0 = dir;

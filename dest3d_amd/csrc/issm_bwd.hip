@@ -1168,6 +1168,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   const int cj = id % p.ncl;
   u.c = p.c_lo + (mirror ? p.ncl - 1 - cj : cj);
   u.b = id / p.ncl;
+  const float* before = nullptr;   // the sums over the heads the tile-base kernel evaluated
   if (redo) {
     const int nblk = p.B * p.ncl * p.G * nsl;
     const int wg = ((u.b * p.ncl + (u.c - p.c_lo)) * p.G + u.g) * nsl + ns;  // as the tile-base kernel counts them
@@ -1175,6 +1176,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
     int any = 0;
     for (int hh = 0; hh < p.hpg; ++hh) any |= redo[hh];
     if (!any) return;
+    if (!FULL && p.dbc_part) before = p.dbc_part + ((long)dir_here * nblk + wg) * (32 * NTHREADS);
   }
   u.dir = dir_here;
   u.bt = u.b * p.ndir + u.dir;
@@ -1188,7 +1190,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   lane_load_ln<true>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, Bv);
   lane_load_ln<true>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, Cv);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) s.dbc[k * NTHREADS + tid] = s.dbc[(16 + k) * NTHREADS + tid] = 0.0f;
+  for (int k = 0; k < 32; ++k) s.dbc[k * NTHREADS + tid] = before ? before[k * NTHREADS + tid] : 0.0f;
 
   // The reversed direction's launch follows the forward one's and shares dt, x, B, C and ddt with it: it walks the
   // heads backwards, so what the first launch touched last (and the last-level cache still holds) is read first.
@@ -1389,7 +1391,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
       vb[k] = s.dbc[k * NTHREADS + tid];
       vc[k] = s.dbc[(16 + k) * NTHREADS + tid];
     }
-    if (redo) {
+    if (redo && !before) {
       float ob[16], oc[16];
       if (p.dB[u.dir].ptr) lane_load_ln<true>(p.dB[u.dir], u.b, u.g, n, vn, g4, rm, ob);
       if (p.dC[u.dir].ptr) lane_load_ln<true>(p.dC[u.dir], u.b, u.g, n, vn, g4, rm, oc);

@@ -59,6 +59,7 @@ struct BwdTileSmem {
   static constexpr bool BCL = !SPLIT && PT == 2;
   unsigned bc[BCL ? 16 * NTHREADS : 1];
   int bad[4];                // per wave: some column of the head exceeds SPAN_LIMIT
+  int shared[4];             // per wave: some head was left to the level form
 };
 
 __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
@@ -103,6 +104,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
 #pragma unroll
   for (int k = 0; k < 16; ++k) s.dbc[k * NTHREADS + tid] = s.dbc[(16 + k) * NTHREADS + tid] = 0.0f;
+
+  if (DIAG32) s.shared[wave] = 0;
 
   if constexpr (BCL) {
     float tb[16], tc[16];
@@ -254,6 +257,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     const int4 bd = *(const int4*)s.bad;
     const bool skip = (bd.x | bd.y | bd.z | bd.w) != 0;  // uniform: the whole head is left to the level-hierarchy kernel
     if (tid == 0) redo[(p.dir0 * (int)gridDim.x + wg) * p.hpg + hh] = skip ? 1 : 0;
+    if (DIAG32 && skip) s.shared[wave] = 1;
     const uint16_t* xs_ = s.xs;
     const uint16_t* dys_ = s.dys;
     const uint16_t* tm_ = s.tm;
@@ -623,7 +627,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     }
   }
 
-  {
+  if (DIAG32 && p.dbc_part && s.shared[wave]) {  // (the wave's own word)
+    float* q = p.dbc_part + ((long)p.dir0 * gridDim.x + wg) * (32 * NTHREADS) + tid;
+#pragma unroll
+    for (int k = 0; k < 32; ++k) q[k * NTHREADS] = s.dbc[k * NTHREADS + tid];
+  } else {
     float vb[16], vc[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) {

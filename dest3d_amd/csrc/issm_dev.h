@@ -58,6 +58,11 @@ struct KP {
   // Two directions with a bf16 ddt: the first direction's share of ddt travels in fp32 through this (B, L, H, N) buffer
   // instead of through ddt itself, so that the sum of the two is rounded to bf16 once (null: it travels through ddt).
   TensorD ddt_part;
+  // bf16 inputs, incomplete tiles: sums of dB and dC over the heads the tile-base chunk backward evaluated, in fp32, of the
+  // workgroups with heads it left to the level form (which goes on from them, so that dB and dC are rounded once, as where
+  // the level form evaluates all heads): per direction and workgroup the lanes' 16 + 16 values [32][NTHREADS].  Null: they
+  // travel through dB and dC themselves.  (Complete tiles do that: six decoder layers, a training step, 7.38 against 7.52 ms.)
+  float* dbc_part;
   const float* A;
   const float* D;
   const float* dt_bias;
