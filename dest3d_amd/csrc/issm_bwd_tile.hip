@@ -16,8 +16,8 @@
 // (|tt| <= 96: operands below 2^96, no overflow before the factors meet).  A head of a workgroup where some column
 // exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
 // (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands, complete tiles: bf16 inputs -> one bf16
-// instruction per block, operands rounded once; fp32 inputs -> operands rounded to 17 significand bits and split exactly into
-// (hi, lo) bf16 pairs, a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, and a
+// instruction per block, operands rounded once; fp32 inputs -> operands as (hi, lo) bf16 pairs (17 significand
+// bits and more), a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, and a
 // gated dy: the level form evaluates these calls wherever this kernel cannot, close pairs of rows (bf16 inputs) or all pairs
 // (fp32 inputs) from fp32 operands, and what a pair is computed in is not to depend on the kernel.  So the diagonal blocks
 // (bf16 inputs) or all blocks (fp32 inputs) are fp32 matrix instructions there.  That costs less than it saves: no operand is
@@ -61,6 +61,10 @@ struct BwdTileSmem {
   int bad[4];                // per wave: some column of the head exceeds SPAN_LIMIT
   int shared[4];             // per wave: some head was left to the level form
 };
+
+// An fp32 value rounded to 17 significand bits; a NaN may come out as zero.  (Where it stands below the conversion alone gives
+// the same number but for ties; without it the kernel spills 200 bytes a lane instead of 20.)
+__device__ __forceinline__ float round17(float v) { return __uint_as_float((__float_as_uint(v) + 0x40u) & 0xffffff80u); }
 
 __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
 
@@ -313,14 +317,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
             bf32[k] = bi;
             continue;
           }
-          if (SPLIT) {
-            cu = round17(cu);
-            bi = round17(bi);
-          }
-          Ch[J][j] = (__bf16)cu;
-          Bh[J][j] = (__bf16)bi;
-          if (SPLIT) {
-            Cl[J][j] = (__bf16)(cu - (float)Ch[J][j]);  // exact: 17 bits = 8 + 8 and the sign
+          Ch[J][j] = (__bf16)(SPLIT ? round17(cu) : cu);
+          Bh[J][j] = (__bf16)(SPLIT ? round17(bi) : bi);
+          if (SPLIT) {  // of the value itself, rounded to 8 bits: the pair holds it to 2^-18, and what is no number stays none
+            Cl[J][j] = (__bf16)(cu - (float)Ch[J][j]);
             Bl[J][j] = (__bf16)(bi - (float)Bh[J][j]);
           }
         }
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         // matrix instructions took them: a pair of rows then enters both of its rows as one and the same product and
         // cancels in the suffix sums to fp32 rounding.  The state terms cancel against the state pass's column sums,
         // which were formed from unrounded states: with bf16 inputs they take the unrounded operands (B and C are
-        // exact, the decays fp32); with fp32 inputs the 17-bit operands are as accurate as the split products Q and R.
+        // exact, the decays fp32); with fp32 inputs the operand pairs are as accurate as the split products Q and R.
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int k = 4 * R + rr;

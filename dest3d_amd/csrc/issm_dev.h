@@ -821,8 +821,6 @@ typedef short sh4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f4 mfma_bf16k(bf4 a, bf4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(sh4, a), __builtin_bit_cast(sh4, b), c, 0, 0, 0);
 }
-// an fp32 value rounded to 17 significand bits: it then splits into a bf16 number and a signed bf16 rest exactly
-__device__ __forceinline__ float round17(float v) { return __uint_as_float((__float_as_uint(v) + 0x40u) & 0xffffff80u); }
 
 // ------------------------------------------------------------------ cooperative tile loaders
 // The unit's (64 x P) tile of a (B,L,H,P) tensor, zero padded to 16*PT columns: registers, then

@@ -604,6 +604,23 @@ def test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel(dtyp
             "head 3 is out of range only in the chunk that holds tokens 70..109"
 
 
+@pytest.mark.parametrize("L_", [64, 60], ids=["complete tile", "ragged"])
+@pytest.mark.parametrize("bits", [0x7fc00000, 0x7fffffff, -1, 0x7f800000], ids=["nan", "nan of all bits", "-nan of all bits", "inf"])
+def test_an_operand_that_is_no_number_reaches_the_gradients(bits, L_):
+    """C (B) of one token and column is NaN or infinite: dB of all tokens up to it (dC from it on) is none in that column,
+    whatever the NaN's payload."""
+    from dest3d_amd import ISSM_chunk_scan_combined
+    for name, grad, rows in (("C", "B", slice(0, 6)), ("B", "C", slice(5, L_))):
+        g = torch.Generator().manual_seed(1)
+        r = lambda *s: torch.randn(*s, generator=g)
+        q = dict(x=r(1, L_, 1, 16), dt=torch.rand(1, L_, 1, 64, generator=g) * 0.1, A=-torch.ones(1, 64), B=r(1, L_, 1, 64), C=r(1, L_, 1, 64))
+        q[name].view(torch.int32)[0, 5, 0, 3] = bits
+        q = {k: v.cuda().requires_grad_() for k, v in q.items()}
+        ISSM_chunk_scan_combined(q["x"], q["dt"], q["A"], q["B"], q["C"], 64).backward(r(1, L_, 1, 16).cuda())
+        assert not torch.isfinite(q[grad].grad[0, rows, 0, 3]).any(), grad
+        assert torch.isfinite(q[grad].grad[0, :, 0, 4:]).all()
+
+
 @pytest.mark.parametrize("L_,N,P", [(70, 64, 32), (100, 70, 36), (256, 130, 16)])
 def test_gradients_of_bf16_heads_two_kernels_share_are_rounded_once(L_, N, P):
     """Head 0 stays in the tile-base kernel, head 1 decays by more than 2^96 over rows 48 .. 63 of the first chunk and is left
