@@ -961,8 +961,8 @@ int issm_pn2_three_interpolate_grad_rows(int32_t b, int32_t c, int32_t n, int32_
   PN2_SIZES("three_interpolate_grad_rows", b, c, n, m);
   if ((int64_t)b * c * n == 0) return ISSM_OK;
   if (m == 0) return fail(ISSM_E_SHAPE, "three_interpolate_grad_rows: no points to index");
-  if (n > ISSM_PN2_ROW_POINTS || m > ISSM_PN2_ROW_POINTS || b > 65535)
-    return fail(ISSM_E_UNSUPPORTED, "three_interpolate_grad_rows: n = %d or m = %d > %d, or batch > 65535", n, m, ISSM_PN2_ROW_POINTS);
+  if (n > ISSM_PN2_ROW_POINTS || m > ISSM_PN2_ROW_POINTS || b > 65535 || (int64_t)b * c > 0x7fffffff / 1024)
+    return fail(ISSM_E_UNSUPPORTED, "three_interpolate_grad_rows: n = %d or m = %d > %d, or too many rows", n, m, ISSM_PN2_ROW_POINTS);
   PN2_PTRS("three_interpolate_grad_rows", grad_out, idx, weight, workspace, grad_points);
   if ((uintptr_t)workspace & 7) return fail(ISSM_E_STRIDE, "three_interpolate_grad_rows: workspace is not aligned to 8 bytes");
   return launched(launch_interp_rows_grad(b, c, n, m, grad_out, idx, weight, (int*)workspace, grad_points, (hipStream_t)stream),

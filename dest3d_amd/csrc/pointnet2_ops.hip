@@ -377,7 +377,8 @@ __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
   const long end = min((long)(wg + 1) * g.share, (long)g.rows * g.ms);
   for (long at = (long)wg * g.share; at < end;) {
     const int row = (int)(at / g.ms), b = row / rows1, ch = row % rows1;
-    const int lo = (int)(at - (long)row * g.ms), hi = (int)min((long)g.ms, lo + (end - at));
+    // (entries are counted without a sign: a sample has up to 2^31 - 1, and the loop steps beyond them)
+    const unsigned lo = (unsigned)(at - (long)row * g.ms), hi = (unsigned)min((long)g.ms, lo + (end - at));
     at += hi - lo;
     __syncthreads();
     if (ch < g.cx) {
@@ -392,8 +393,8 @@ __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
     __syncthreads();
     const int* q = g.idx + (long)b * g.ms;
     float* o = g.out + (long)row * g.ms;
-    for (int e = lo + 4 * tid; e < hi; e += 4 * T) {
-      const int cnt = min(hi - e, 4);
+    for (unsigned e = lo + 4 * tid; e < hi; e += 4 * T) {
+      const int cnt = (int)min(hi - e, 4u);
       I4Any i = {};
       if (cnt == 4) i = *(const I4Any*)(q + e);
       else for (int j = 0; j < cnt; ++j) i.v[j] = q[e + j];
@@ -402,7 +403,8 @@ __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
       for (int j = 0; j < 4; ++j) v[j] = srow[index_of(i.v[j], g.n)];
       if (ch < g.cx) {
         // (one division per step: what a coordinate row costs beyond a feature row decides when its workgroup ends)
-        int at_c = (int)((unsigned)e / (unsigned)g.nsample), left = (at_c + 1) * g.nsample - e;
+        const unsigned at_c = e / (unsigned)g.nsample;
+        int left = (int)((at_c + 1) * g.nsample - e);
         const float* cq = g.centre + ((long)b * g.npoints + at_c) * 3 + ch;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -436,7 +438,7 @@ __device__ __forceinline__ float row_lane_f(float v) {
 // with the mostly repeated indices of a 0.2 m ball
 // 144 us for those 537 MB (3.7 TB/s; atomics into a channel-last buffer: 592 and 190 for copies around them), with 64
 // different ones 684 us, the rate of LDS float additions to scattered words (before: 479 and 190).  With splits > 1 (few rows) the parts meet in grad_points, which is zero before.
-__global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdim, int n, int ms, int splits, int per,
+__global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdim, int n, int ms, int splits, unsigned per,
                                                           const float* __restrict__ grad_out, const int* __restrict__ idx,
                                                           float* __restrict__ grad_points) {
   extern __shared__ float srow[];
@@ -446,9 +448,9 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
   __syncthreads();
   const int* q = idx + (long)b * ms;
   const float* g = grad_out + ((long)b * cdim + c0 + ch) * ms;
-  const int hi = min((part + 1) * per, ms);
-  for (int e0 = part * per + (tid >> 6) * 256; e0 < hi; e0 += 4 * T) {   // wave-uniform
-    const int e = e0 + 4 * lane;
+  const unsigned hi = min((part + 1) * per, (unsigned)ms);   // (without a sign, see k_group_rows)
+  for (unsigned e0 = part * per + (tid >> 6) * 256; e0 < hi; e0 += 4 * T) {   // wave-uniform
+    const unsigned e = e0 + 4 * lane;
     I4Any i;
     f4 v = {0, 0, 0, 0};
     if (e + 4 <= hi) {
@@ -499,8 +501,7 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
       if (srow[k] != 0.0f) unsafeAtomicAdd(o + k, srow[k]);   // (NaN != 0)
 }
 __global__ __launch_bounds__(NTHREADS) void k_zero(long total, float* __restrict__ q) {
-  const long e = (long)blockIdx.x * NTHREADS + threadIdx.x;
-  if (e < total) q[e] = 0.0f;
+  for (long e = (long)blockIdx.x * NTHREADS + threadIdx.x; e < total; e += (long)gridDim.x * NTHREADS) q[e] = 0.0f;
 }
 __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int c, int n, int ms,
                                                                 const float* __restrict__ grad_out,
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(NTHREADS) void k_three_interpolate_grad(long total,
 // 256 channels, 2048 -> 20000 points, 8 samples: 166 us with a
 // thread per element, 45 us here (164 MB written).
 template <int CH>
-__global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int splits, int per, const float* __restrict__ points,
+__global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int splits, unsigned per, const float* __restrict__ points,
                                                      const int* __restrict__ idx, const float* __restrict__ weight,
                                                      float* __restrict__ out) {
   extern __shared__ __align__(16) float srow[];
@@ -773,8 +774,8 @@ __global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int sp
     srow[e] = points[((long)b * c + ch) * m + e / CH];
   }
   __syncthreads();
-  const int hi = min((part + 1) * per, n);
-  for (int j = part * per + tid; j < hi; j += 512) {
+  const unsigned hi = min((part + 1) * per, (unsigned)n);
+  for (unsigned j = part * per + tid; j < hi; j += 512) {
     const long o = ((long)b * n + j) * 3;
     f4 acc[CH / 4];
 #pragma unroll
@@ -937,6 +938,7 @@ int launch_scatter_channel_last(bool k3, int b, int c, int n, int ne, const floa
 }
 
 static unsigned blocks_for(long total) { return (unsigned)((total + NTHREADS - 1) / NTHREADS); }
+static unsigned zero_blocks(long total) { return (unsigned)std::min<long>(blocks_for(std::min(total, 1L << 31)), 1 << 20); }
 
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st) {
 #define FPS_GROUPS(W, S) hipLaunchKernelGGL((k_fps_groups<W, S>), dim3(b), dim3(64 * W), 0, st, n, npoint, xyz, idxs)
@@ -965,11 +967,11 @@ static int set_lds_rows(K kern, size_t bytes) {
 }
 // How the entries of a row are cut: about two workgroups per CU in all, but no part shorter than what it costs to put the
 // row into LDS (or to clear it and write it back), and a multiple of `unit` entries each.
-static int parts_of(long row_blocks, int entries, int row_len, int unit, int* per) {
+static int parts_of(long row_blocks, long entries, int row_len, int unit, unsigned* per) {
   long parts = (512 + row_blocks - 1) / row_blocks;
   parts = std::max<long>(1, std::min<long>(parts, entries / std::max(row_len, 2048)));
-  *per = (int)(((entries + parts - 1) / parts + unit - 1) / unit * unit);
-  return (entries + *per - 1) / *per;
+  *per = (unsigned)(((entries + parts - 1) / parts + unit - 1) / unit * unit);
+  return (int)((entries + *per - 1) / *per);
 }
 static int row_threads(int n) { return n > 10240 ? 1024 : 512; }   // above, at most three workgroups fit a CU's LDS
 
@@ -989,7 +991,7 @@ int launch_group_points(int b, int c, int n, int npoints, int nsample, const flo
     if (int e = set_lds_rows(&k_group_rows, n * sizeof(float))) return e;
     hipLaunchKernelGGL(k_group_rows, dim3((unsigned)((total + g.share - 1) / g.share)), dim3(row_threads(n)), n * sizeof(float), st, g);
   } else {
-    hipLaunchKernelGGL(k_group_points, dim3((g.ms + NTHREADS - 1) / NTHREADS, (unsigned)std::min<long>(rows, 65535)),
+    hipLaunchKernelGGL(k_group_points, dim3(blocks_for(g.ms), (unsigned)std::min<long>(rows, 65535)),
                        dim3(NTHREADS), 0, st, g);
   }
   return (int)hipGetLastError();
@@ -997,9 +999,9 @@ int launch_group_points(int b, int c, int n, int npoints, int nsample, const flo
 int launch_group_rows_grad(int b, int c, int c0, int cdim, int n, int ms, const float* grad_out, const int* idx,
                            float* grad_points, hipStream_t st) {
   const long rows = (long)b * c;
-  int per;
+  unsigned per;
   const int splits = parts_of(rows, ms, n, 256, &per);
-  if (splits > 1) hipLaunchKernelGGL(k_zero, dim3(blocks_for(rows * n)), dim3(NTHREADS), 0, st, rows * n, grad_points);
+  if (splits > 1) hipLaunchKernelGGL(k_zero, dim3(zero_blocks(rows * n)), dim3(NTHREADS), 0, st, rows * n, grad_points);
   if (int e = set_lds_rows(&k_group_rows_grad, n * sizeof(float))) return e;
   hipLaunchKernelGGL(k_group_rows_grad, dim3((unsigned)(rows * splits)), dim3(row_threads(n)), n * sizeof(float), st, c, c0,
                      cdim, n, ms, splits, per, grad_out, idx, grad_points);
@@ -1031,7 +1033,7 @@ int launch_three_interpolate(int b, int c, int m, int n, const float* points, co
   if (n >= m && total >= 1 << 21 && m <= INTERP_POINTS) {
     const int ch = m <= INTERP_POINTS / 4 ? 8 : 4, groups = (c + ch - 1) / ch;
     const size_t sm = (size_t)m * ch * sizeof(float);
-    int per;
+    unsigned per;
     const int splits = parts_of((long)b * groups, n, m, 512, &per);
     if (ch == 8) {
       if (int e = set_lds_rows(&k_interp_rows<8>, sm)) return e;
@@ -1059,7 +1061,7 @@ int launch_interp_rows_grad(int b, int c, int n, int m, const float* grad_out, c
   hipLaunchKernelGGL(k_inverse_fill, dim3((per * INV_T + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, per, idx, weight,
                      start, rank, list);
   const long total = (long)b * c * m;
-  hipLaunchKernelGGL(k_zero, dim3(blocks_for(total)), dim3(NTHREADS), 0, st, total, grad_points);
+  hipLaunchKernelGGL(k_zero, dim3(zero_blocks(total)), dim3(NTHREADS), 0, st, total, grad_points);
   auto go = [&](auto kern, int r) -> int {
     const size_t sm = (size_t)r * n * sizeof(float);
     if (int e = set_lds_rows(kern, sm)) return e;

@@ -135,7 +135,7 @@ class ThreeInterpolate(Function):
         with torch.cuda.device(g.device):
             # (the sorted lists of the rows form pay off from two million elements: 64 channels, 400 <- 3000 points, 2 samples
             # take 20 us with it and 13 without)
-            if g.numel() >= 1 << 21 and max(n, m) <= _ROW_POINTS and Bsz <= 65535:
+            if g.numel() >= 1 << 21 and max(n, m) <= _ROW_POINTS and Bsz <= 65535 and Bsz * c < 1 << 20:
                 ws = torch.empty(lib.issm_pn2_three_interpolate_grad_rows_workspace(Bsz, n, m), dtype=torch.uint8, device=g.device)
                 out = torch.empty((Bsz, c, m), dtype=torch.float32, device=g.device)
                 L.check(lib.issm_pn2_three_interpolate_grad_rows(Bsz, c, n, m, g.data_ptr(), ix.data_ptr(), w.data_ptr(),

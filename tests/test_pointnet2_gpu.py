@@ -241,6 +241,32 @@ def test_grouped_rows_and_their_gradient(B, C, N, M, S):
     assert (f1.grad - f2.grad).abs().max() <= 1e-5 * f2.grad.abs().max()
 
 
+def test_grouping_up_to_the_largest_sample():
+    """2^31 - 1024 entries in a sample: counts of entries that step past the end of a row stay right.  Forward (features, and
+    coordinates relative to the centres) and gradient (ones: how often a point is grouped, exact in fp32)."""
+    from dest3d_amd.pointnet2_utils import _GroupXyzPoints, grouping_operation
+    N, M, S = 5000, (1 << 21) - 1, 1024
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 80 GB of free memory")
+    idx = torch.arange(M * S, dtype=torch.int32, device="cuda").remainder_(N).view(1, M, S)
+    feats = torch.randn(1, 1, N, device="cuda").requires_grad_()
+    out = grouping_operation(feats, idx)
+    step = 1 << 28
+    for at in range(0, M * S, step):
+        part = idx.flatten()[at:at + step]
+        assert torch.equal(out.detach().flatten()[at:at + step], feats.detach().flatten()[part.long()])
+    count, = torch.autograd.grad(out, feats, torch.ones((), device="cuda").expand_as(out))
+    want = torch.full((N,), M * S // N, dtype=torch.float32, device="cuda")
+    want[:M * S % N] += 1
+    assert torch.equal(count.flatten(), want)
+    del out
+    xyz, centres = torch.randn(1, N, 3, device="cuda"), torch.randn(1, M, 3, device="cuda")
+    out = _GroupXyzPoints.apply(None, xyz, centres, idx, 2.0)
+    for lo, hi in ((0, 3), (M // 2, M // 2 + 5), (M - 9, M)):
+        want = (xyz[0, idx[0, lo:hi].long()] - centres[0, lo:hi, None]) * 2.0
+        assert torch.equal(out[0, :, lo:hi], want.permute(2, 0, 1))
+
+
 @pytest.mark.parametrize("c,m,n", [(1, 1, 3), (3, 5, 700), (9, 2560, 2600), (8, 2561, 2700), (5, 10240, 10300), (2, 10241, 10300),
                                    (2, 40, 20000), (512, 30, 1023), (700, 3, 5121), (3, 1000, 40960), (1, 900, 40961)])
 def test_interpolation_rows(c, m, n):
