@@ -23,6 +23,7 @@ namespace issm {
 
 constexpr int ROW_POINTS = 40960;     // points of a row that fit in a CU's 160 KB of LDS
 constexpr int INTERP_POINTS = 10240;  // of four rows
+constexpr int WIDE_POINTS = 5120;     // of a row of doubles, four workgroups to a CU
 
 constexpr int FPS_T = 512;    // threads of the sampling workgroup (two waves per SIMD: 256 registers each)
 
@@ -432,19 +433,35 @@ __device__ __forceinline__ float row_lane_f(float v) {
 }
 
 // Gradient of the grouping, all of grad_points (b, c, n) written: one workgroup per channel row (and part of its entries),
-// the row's n sums in LDS, grad_out streamed once.  A ball with fewer points than slots repeats its first point, and 64
-// lanes adding to one LDS word take 64 turns: runs of equal indices are summed first -- four consecutive entries per lane,
-// then a segmented scan over the row of 16 lanes -- and only the last entry of a run adds.  Bound by reading grad_out:
-// with the mostly repeated indices of a 0.2 m ball
-// 144 us for those 537 MB (3.7 TB/s; atomics into a channel-last buffer: 592 and 190 for copies around them), with 64
-// different ones 684 us, the rate of LDS float additions to scattered words (before: 479 and 190).  With splits > 1 (few rows) the parts meet in grad_points, which is zero before.
+// the row's n sums in LDS, grad_out streamed once.  A ball with fewer points than slots repeats its first point, and lanes
+// adding to one LDS word take turns: runs of equal indices are summed first -- four consecutive entries per lane, then a
+// segmented scan over the row of 16 lanes -- and only the last entry of a run adds.  How it adds decides the rest: an LDS
+// float addition takes 3 cycles a lane however the words lie (measured: 0.77 lanes a nanosecond and CU), one of doubles a
+// fifth of a cycle (6.4), a compare-and-swap of a word just read, if it succeeds, half a cycle.  So up to 5120 points, of
+// which four workgroups still share a CU, the sums are doubles (WIDE); beyond, a lane tries one compare-and-swap and adds the
+// ordinary way where another lane was faster.  Bound by reading grad_out then: 8 samples, 128 channels of 20000 points, 2048
+// balls of 64, 152 us for those 537 MB (3.5 TB/s), whether a ball repeats one point or has 64 different ones (float
+// additions alone: 152 and 677; atomics into a channel-last buffer: 495 and 486).  2048 points, 2048 balls, 64 channels:
+// 65 - 67 us (89 - 332; 252 - 243).  The worst for it, entries that hop between two points
+// (20000 points as above): 1340 us (898; 6000).  With splits > 1 (few rows) the parts meet in grad_points, zero before.
+template <bool WIDE>
 __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdim, int n, int ms, int splits, unsigned per,
                                                           const float* __restrict__ grad_out, const int* __restrict__ idx,
                                                           float* __restrict__ grad_points) {
-  extern __shared__ float srow[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  typedef typename std::conditional<WIDE, double, float>::type Sum;
+  Sum* srow = reinterpret_cast<Sum*>(smem_raw);
+  auto add = [&](int k, float v) {
+    if constexpr (!WIDE) {
+      unsigned* u = (unsigned*)srow + k;
+      const unsigned e = *(volatile unsigned*)u;
+      if (atomicCAS(u, e, __builtin_bit_cast(unsigned, __builtin_bit_cast(float, e) + v)) == e) return;
+    }
+    unsafeAtomicAdd(srow + k, (Sum)v);
+  };
   const int T = blockDim.x, tid = threadIdx.x, lane = tid & 63;
   const int wg = xcd_remap(blockIdx.x, gridDim.x), row = wg / splits, part = wg % splits, b = row / c, ch = row % c;
-  for (int k = tid; k < n; k += T) srow[k] = 0.0f;
+  for (int k = tid; k < n; k += T) srow[k] = 0;
   __syncthreads();
   const int* q = idx + (long)b * ms;
   const float* g = grad_out + ((long)b * cdim + c0 + ch) * ms;
@@ -487,18 +504,18 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
     step(std::integral_constant<int, 0x118>{});
     const float before = row_lane_f<0x111>(s), carry = link ? before : 0.0f;
     const bool end3 = row_lane<0x101>(-2, i.v[0]) != i.v[3];
-    if (!q1 && i.v[0] >= 0) unsafeAtomicAdd(srow + i.v[0], v[0] + carry);
-    if (!q2 && i.v[1] >= 0) unsafeAtomicAdd(srow + i.v[1], v[1] + (q1 ? carry : 0.0f));
-    if (!q3 && i.v[2] >= 0) unsafeAtomicAdd(srow + i.v[2], v[2] + (q1 && q2 ? carry : 0.0f));
-    if (end3 && i.v[3] >= 0) unsafeAtomicAdd(srow + i.v[3], v[3] + (q1 && q2 && q3 ? carry : 0.0f));
+    if (!q1 && i.v[0] >= 0) add(i.v[0], v[0] + carry);
+    if (!q2 && i.v[1] >= 0) add(i.v[1], v[1] + (q1 ? carry : 0.0f));
+    if (!q3 && i.v[2] >= 0) add(i.v[2], v[2] + (q1 && q2 ? carry : 0.0f));
+    if (end3 && i.v[3] >= 0) add(i.v[3], v[3] + (q1 && q2 && q3 ? carry : 0.0f));
   }
   __syncthreads();
   float* o = grad_points + (long)row * n;
   if (splits == 1)
-    for (int k = tid; k < n; k += T) o[k] = srow[k];
+    for (int k = tid; k < n; k += T) o[k] = (float)srow[k];
   else
     for (int k = tid; k < n; k += T)
-      if (srow[k] != 0.0f) unsafeAtomicAdd(o + k, srow[k]);   // (NaN != 0)
+      if (srow[k] != 0) unsafeAtomicAdd(o + k, (float)srow[k]);   // (NaN != 0)
 }
 __global__ __launch_bounds__(NTHREADS) void k_zero(long total, float* __restrict__ q) {
   for (long e = (long)blockIdx.x * NTHREADS + threadIdx.x; e < total; e += (long)gridDim.x * NTHREADS) q[e] = 0.0f;
@@ -1002,9 +1019,15 @@ int launch_group_rows_grad(int b, int c, int c0, int cdim, int n, int ms, const 
   unsigned per;
   const int splits = parts_of(rows, ms, n, 256, &per);
   if (splits > 1) hipLaunchKernelGGL(k_zero, dim3(zero_blocks(rows * n)), dim3(NTHREADS), 0, st, rows * n, grad_points);
-  if (int e = set_lds_rows(&k_group_rows_grad, n * sizeof(float))) return e;
-  hipLaunchKernelGGL(k_group_rows_grad, dim3((unsigned)(rows * splits)), dim3(row_threads(n)), n * sizeof(float), st, c, c0,
-                     cdim, n, ms, splits, per, grad_out, idx, grad_points);
+  auto go = [&](auto kern, size_t bytes, int threads) -> int {
+    if (int e = set_lds_rows(kern, bytes)) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(rows * splits)), dim3(threads), bytes, st, c, c0, cdim, n, ms, splits, per, grad_out, idx,
+                       grad_points);
+    return 0;
+  };
+  const int e = n <= WIDE_POINTS ? go(&k_group_rows_grad<true>, n * sizeof(double), 512)
+                                 : go(&k_group_rows_grad<false>, n * sizeof(float), row_threads(n));
+  if (e) return e;
   return (int)hipGetLastError();
 }
 int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out, const int* idx, float* grad_points,

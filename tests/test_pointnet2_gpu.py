@@ -210,9 +210,10 @@ def test_query_and_group_module():
 
 
 @pytest.mark.parametrize("B,C,N,M,S", [(1, 1, 1, 1, 1), (2, 3, 63, 16, 4), (1, 2, 257, 300, 7), (2, 5, 1023, 511, 9),
-                                       (1, 3, 4099, 640, 32), (1, 1, 40960, 5200, 16), (1, 1, 40961, 5200, 16)])
+                                       (1, 3, 4099, 640, 32), (1, 2, 5120, 700, 16), (2, 3, 5121, 800, 16), (1, 1, 40960, 5200, 16),
+                                       (1, 1, 40961, 5200, 16)])
 def test_grouped_rows_and_their_gradient(B, C, N, M, S):
-    """Row remainders, entries cut over several workgroups (few channels, many entries), the longest row in LDS and the first
+    """Row remainders, sums in doubles and in floats, entries cut over several workgroups (few channels, many entries), the longest row in LDS and the first
     beyond it; index runs of every length, within a lane's four entries, across lanes and across the rows of a wave."""
     from dest3d_amd.pointnet2_utils import QueryAndGroup, grouping_operation
     rng = np.random.default_rng(N + M)
@@ -239,6 +240,24 @@ def test_grouped_rows_and_their_gradient(B, C, N, M, S):
     a.backward(w)
     b.backward(w)
     assert (f1.grad - f2.grad).abs().max() <= 1e-5 * f2.grad.abs().max()
+
+
+@pytest.mark.parametrize("N", [300, 5121])
+@pytest.mark.parametrize("few", [2, 16, 256])
+def test_grouping_gradient_where_many_entries_meet_in_few_points(N, few):
+    """Neighbouring entries go to different points, all to the same few: the additions of a wave and of the waves collide."""
+    from dest3d_amd.pointnet2_utils import grouping_operation
+    rng = np.random.default_rng(few)
+    idx = (np.arange(2 * 500 * 32) % 2 if few == 2 else rng.integers(0, few, size=2 * 500 * 32)).astype(np.int32).reshape(2, 500, 32)
+    f = torch.zeros(2, 7, N, device="cuda", requires_grad=True)
+    gy = rng.integers(-8, 9, size=(2, 7, 500, 32)).astype(np.float32)       # sums are whole numbers: exact in any order
+    gy[0, 0, 3, 5] = np.nan
+    g, = torch.autograd.grad(grouping_operation(f, _cuda(idx)), f, _cuda(gy))
+    want = np.zeros((2, 7, N))
+    for b in range(2):
+        for c in range(7):
+            np.add.at(want[b, c], idx[b].ravel(), gy[b, c].ravel().astype(np.float64))
+    assert np.array_equal(g.cpu().numpy(), want.astype(np.float32), equal_nan=True)
 
 
 def test_grouping_up_to_the_largest_sample():
