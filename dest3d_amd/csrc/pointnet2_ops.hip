@@ -96,7 +96,13 @@ __device__ __forceinline__ int lane_of_least(unsigned long long cand, int key) {
 // (subtract, square, add, in sqdist's order) is at most the same step for q, and where the box's distance is not below the
 // group's largest running distance, no minimum of the group changes.  A NaN anywhere makes the comparison fail, which means
 // "look".  Equal distances go to the smaller index at every level, as a pass over all points in order would decide.
-constexpr int FPS_CELLS = 4096;   // 16^3
+//
+// What the pruning saves depends on how small the groups' boxes are, so the grid must fit the cloud: one point 300 m away from
+// a room of 8 m would leave the room a single cell of a grid over everything, its groups in index order and every box the
+// whole room.  The grid therefore covers what most points fill -- the middle half of a sample along each axis and as much again
+// on either side -- and a second, coarser one, sorted behind it, everything.  20000 points, 2048 draws, 8 samples: uniform 1.95
+// ms; with one far point 9.5 -> 1.97, one in twenty far 5.5 -> 1.88, a third far 1.77 -> 1.73 (passing over all points: 3.9).
+constexpr int FPS_CELLS = 4096, FPS_BINS = 5120;   // 16^3 cells and 8^3 behind them, rounded up to a multiple of the threads
 // f(0), f(1), ... f(N - 1) with constant arguments: register arrays indexed inside f stay in registers for every N (the
 // loop unroller left a loop over 20 or 24 slots to dynamic indexing, and the arrays to scratch)
 template <int N, int I = 0, class F>
@@ -114,8 +120,10 @@ template <int W, int S>
 __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const float* __restrict__ xyz, int* __restrict__ idxs) {
   constexpr int T = 64 * W, ROWS = (S + 15) / 16;
   static_assert(S % 4 == 0 && S <= 32 && W <= 16 && (W & (W - 1)) == 0, "slots and waves sit in the lanes of one wave");
-  __shared__ int hist[FPS_CELLS];
+  __shared__ int hist[FPS_BINS];
   __shared__ unsigned short order[T * S];
+  __shared__ float quart[6];
+  __shared__ int sampled;
   __shared__ float red[6][W];
   __shared__ int wsum[W];
   struct alignas(16) Best { unsigned d; float x, y, z; };
@@ -126,6 +134,22 @@ __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const 
   int* out = idxs + (long)b * npoint;
   const float INFV = __builtin_huge_valf();
 
+  // quartiles of a sample of 64 points: wave a takes axis a, a lane counts the values before its own
+  if (wave < 3) {
+    const float* q = p + (long)lane * n / 64 * 3;
+    const float x = q[0], y = q[1], z = q[2], r = sqdist(x, y, z, 0.0f, 0.0f, 0.0f);
+    const float v = r > 1e-3f && r < INFV ? (wave == 0 ? x : wave == 1 ? y : z) : INFV;
+    const int m = __popcll(__ballot(v < INFV));
+    int before = 0;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const float u = lane_f(v, j);
+      before += u < v || (u == v && j < lane) ? 1 : 0;
+    }
+    if (before == m / 4) quart[wave] = v;
+    if (before == m - 1 - m / 4) quart[3 + wave] = v;
+    if (tid == 0) sampled = m;
+  }
   // bounding box of the points that take part
   float lo[3] = {INFV, INFV, INFV}, hi[3] = {-INFV, -INFV, -INFV};
   for (int k = tid; k < n; k += T) {
@@ -140,26 +164,34 @@ __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const 
     const float l = -wave_fmax(-lo[a]), h = wave_fmax(hi[a]);
     if (lane == 0) { red[a][wave] = l; red[3 + a][wave] = h; }
   }
-  for (int c = tid; c < FPS_CELLS; c += T) hist[c] = 0;
+  for (int c = tid; c < FPS_BINS; c += T) hist[c] = 0;
   __syncthreads();
-  float ext = 0.0f;
+  float ext = 0.0f, ext1 = 0.0f, lo1[3], hi1[3];   // 1: of the grid over most points
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     for (int w = 0; w < W; ++w) { lo[a] = fminf(w ? lo[a] : INFV, red[a][w]); hi[a] = fmaxf(w ? hi[a] : -INFV, red[3 + a][w]); }
     ext = fmaxf(ext, hi[a] - lo[a]);
+    const float half = quart[3 + a] - quart[a];
+    lo1[a] = sampled < 8 ? lo[a] : fmaxf(lo[a], quart[a] - half);
+    hi1[a] = sampled < 8 ? hi[a] : fminf(hi[a], quart[3 + a] + half);
+    ext1 = fmaxf(ext1, hi1[a] - lo1[a]);
   }
-  const float inv = ext > 0.0f && ext < INFV ? 16.0f / ext : 0.0f;
+  const float inv = ext > 0.0f && ext < INFV ? 8.0f / ext : 0.0f, inv1 = ext1 > 0.0f && ext1 < INFV ? 16.0f / ext1 : 0.0f;
   auto cell = [&](int k) {
-    unsigned c = 0;
+    const float v[3] = {p[k * 3], p[k * 3 + 1], p[k * 3 + 2]};
+    bool most = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) most = most && v[a] >= lo1[a] && v[a] <= hi1[a];
+    unsigned c = most ? 0 : FPS_CELLS;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
-      c |= spread4((unsigned)imin(imax((int)((p[k * 3 + a] - lo[a]) * inv), 0), 15)) << a;
+      c |= spread4((unsigned)imin(imax((int)((v[a] - (most ? lo1[a] : lo[a])) * (most ? inv1 : inv)), 0), most ? 15 : 7)) << a;
     return c;
   };
   for (int k = tid; k < n; k += T) atomicAdd(&hist[cell(k)], 1);
   __syncthreads();
-  {  // exclusive prefix sum of the histogram: FPS_CELLS / T neighbours per thread
-    constexpr int E = FPS_CELLS / T;
+  {  // exclusive prefix sum of the histogram: FPS_BINS / T neighbours per thread
+    constexpr int E = FPS_BINS / T;
     int own = 0;
     for (int e = 0; e < E; ++e) own += hist[tid * E + e];
     int incl = own;

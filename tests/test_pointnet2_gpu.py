@@ -62,6 +62,19 @@ def test_furthest_point_sampling_on_a_voxelized_cloud(n, npoint):
     assert (idx == R.furthest_point_sampling(xyz, npoint)).all()
 
 
+@pytest.mark.parametrize("n", [65, 2048, 8193])
+@pytest.mark.parametrize("every", [2, 3, 20, 1000])
+def test_furthest_point_sampling_where_some_points_lie_far_from_most(n, every):
+    """Points of either sorting grid, and on their limits: sample 1 has more than half of its points in one place."""
+    from dest3d_amd.pointnet2_utils import furthest_point_sample
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(0, 8, size=(2, n, 3)).astype(np.float32)
+    xyz[:, every // 2::every] = rng.uniform(-900, 900, size=xyz[:, every // 2::every].shape)
+    xyz[1, n // 3:] = xyz[1, n // 3]
+    idx = furthest_point_sample(_cuda(xyz), min(n, 200)).cpu().numpy()
+    assert (idx == R.furthest_point_sampling(xyz, min(n, 200))).all()
+
+
 @pytest.mark.parametrize("n", [64, 700, 5000, 24576])
 @pytest.mark.parametrize("kind", ["extent 1e6", "metres on a map", "infinite points", "first point no number"])
 def test_furthest_point_sampling_where_running_distances_never_come_below_their_start(n, kind):
