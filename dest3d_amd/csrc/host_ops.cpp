@@ -68,6 +68,24 @@ issm_tensor desc(const Tensor& t) {
   return d;
 }
 
+// What a backward pass needs to know of an input it does not read: its type and sizes.  (Such inputs are not saved: they may
+// be changed in place between forward and backward, and need not be kept alive.)
+struct Kind {
+  at::ScalarType type = at::kFloat;
+  at::DimVector sizes;
+  Kind() = default;
+  explicit Kind(const Tensor& t) {
+    if (!t.defined()) return;
+    type = t.scalar_type();
+    sizes = at::DimVector(t.sizes());
+  }
+};
+// A node's own record, beside its saved tensors
+template <class T>
+void keep(AutogradContext* ctx, c10::intrusive_ptr<T> record) { ctx->saved_data["record"] = c10::IValue::make_capsule(std::move(record)); }
+template <class T>
+c10::intrusive_ptr<T> kept(AutogradContext* ctx) { return c10::static_intrusive_pointer_cast<T>(ctx->saved_data["record"].toCapsule()); }
+
 typedef c10::optional<Tensor> MaybeTensor;   // an absent input of a node: it takes no undefined tensors
 
 Tensor opt(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
@@ -362,6 +380,13 @@ issm_norm_args norm_args(const Tensor& x, const Tensor& z, const Tensor& w, cons
 }
 
 struct NormFn : public Function<NormFn> {
+  struct Record : torch::CustomClassHolder {
+    Kind x, weight, bias, z;
+    double eps;
+    int64_t group;
+    bool before_gate, rms;
+  };
+
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& z_,
                         double eps, int64_t group, bool before_gate, bool rms) {
     const c10::DeviceGuard guard(x.device());
@@ -385,26 +410,32 @@ struct NormFn : public Function<NormFn> {
     a.rstd = data<float>(stats);
     if (!rms) a.mean = data<float>(stats) + stats.size(1);
     check(issm_gated_rmsnorm_fwd(&a), "issm_gated_rmsnorm_fwd");
-    ctx->save_for_backward({x, weight, bias, z, x2, z2, w, b, stats});
-    ctx->saved_data["eps"] = eps;
-    ctx->saved_data["group"] = group;
-    ctx->saved_data["before"] = before_gate;
-    ctx->saved_data["rms"] = rms;
+    ctx->save_for_backward({x2, z2, w, b, stats});   // (x2, z2, w, b: the inputs themselves where the kernels read those)
+    auto r = c10::make_intrusive<Record>();
+    r->x = Kind(x);
+    r->weight = Kind(weight);
+    r->bias = Kind(bias);
+    r->z = Kind(z);
+    r->eps = eps;
+    r->group = group;
+    r->before_gate = before_gate;
+    r->rms = rms;
+    keep(ctx, std::move(r));
     return cast(y.view(x.sizes()), x.scalar_type());
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const variable_list v = ctx->get_saved_variables();
-    const Tensor &x2 = v[4], &z2 = v[5], &w = v[6], &b = v[7], &stats = v[8];
+    const Tensor &x2 = v[0], &z2 = v[1], &w = v[2], &b = v[3], &stats = v[4];
+    const auto in = kept<Record>(ctx);
     const c10::DeviceGuard guard(x2.device());
-    const bool rms = ctx->saved_data["rms"].toBool();
+    const bool rms = in->rms;
     Tensor dy = as_rows(cast(grads[0], x2.scalar_type()));
     Tensor dx = fresh(x2.sizes(), x2, x2.scalar_type()), dz;
     if (z2.defined()) dz = fresh(z2.sizes(), z2, z2.scalar_type());
     const int64_t cols = x2.size(1), nb = issm_rmsnorm_bwd_blocks(x2.size(0)), np = b.defined() ? 2 : 1;
     Tensor part = fresh({np, nb, cols}, x2, at::kFloat), dwb = fresh({np, cols}, x2, at::kFloat);
-    issm_norm_args a = norm_args(x2, z2, w, b, ctx->saved_data["eps"].toDouble(), ctx->saved_data["group"].toInt(),
-                                 ctx->saved_data["before"].toBool(), !rms);
+    issm_norm_args a = norm_args(x2, z2, w, b, in->eps, in->group, in->before_gate, !rms);
     a.rstd = data<float>(stats);
     if (!rms) a.mean = data<float>(stats) + stats.size(1);
     a.dy = data(dy);
@@ -423,10 +454,10 @@ struct NormFn : public Function<NormFn> {
     }
     check(issm_gated_rmsnorm_bwd(&a), "issm_gated_rmsnorm_bwd");
     variable_list out(8);
-    out[0] = cast(dx.view(v[0].sizes()), v[0].scalar_type());
-    out[1] = cast(dwb.select(0, 0), v[1].scalar_type());
-    if (np == 2) out[2] = cast(dwb.select(0, 1), v[2].scalar_type());
-    if (dz.defined()) out[3] = cast(dz.view(v[3].sizes()), v[3].scalar_type());
+    out[0] = cast(dx.view(in->x.sizes), in->x.type);
+    out[1] = cast(dwb.select(0, 0), in->weight.type);
+    if (np == 2) out[2] = cast(dwb.select(0, 1), in->bias.type);
+    if (dz.defined()) out[3] = cast(dz.view(in->z.sizes), in->z.type);
     return out;
   }
 };
@@ -553,6 +584,11 @@ struct CoreFn : public Function<CoreFn> {
   enum { CW_F, CW_B, CB_F, CB_B, DT_W, BC_W, DT_BIAS, A_LOG, D_, NSMALL };
   // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
   static constexpr int NIN = 14;
+  struct Record : torch::CustomClassHolder {
+    Kind in[NIN];
+    int64_t H, G, di;
+    double lo, hi, eps;
+  };
 
   static variable_list forward(AutogradContext* ctx, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
                                const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
@@ -646,28 +682,35 @@ struct CoreFn : public Function<CoreFn> {
     }
     const Tensor last = transpose_states(o.last[0].view({Bsz, di, K}), o.last[1].view({Bsz, di, K}), 0.5,
                                          kernel_type(h0_lin.scalar_type()));
-    variable_list saved{zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
-                        norm_w};
-    for (const Tensor& t : {xbc, pre, flat, d, wt, raw, key, z2, nw, rstd, A1, o.ws}) saved.push_back(t);
+    variable_list saved{xbc, pre, flat, d, wt, raw, key, z2, nw, rstd, A1, o.ws};
     s.push(saved);
     ctx->save_for_backward(std::move(saved));
-    ctx->saved_data["sizes"] = std::vector<int64_t>{H, G, di};
-    ctx->saved_data["limits"] = std::vector<double>{lo, hi, 4.0 * eps};
+    auto r = c10::make_intrusive<Record>();
+    const Tensor* ins[NIN] = {&zxbcdt, &h0_lin, &dist, &weights, &conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias,
+                              &A_log, &D, &norm_w};
+    for (int i = 0; i < NIN; ++i) r->in[i] = Kind(*ins[i]);
+    r->H = H;
+    r->G = G;
+    r->di = di;
+    r->lo = lo;
+    r->hi = hi;
+    r->eps = 4.0 * eps;
+    keep(ctx, std::move(r));
     return {cast(key_n.view({Bsz, Ln, di}), zxbcdt.scalar_type()), cast(last, h0_lin.scalar_type())};
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
     const variable_list v = ctx->get_saved_variables();
-    const Tensor &xbc = v[NIN], &pre = v[NIN + 1], &flat = v[NIN + 2], &d = v[NIN + 3], &wt = v[NIN + 4], &raw = v[NIN + 5],
-                 &key = v[NIN + 6], &z2 = v[NIN + 7], &nw = v[NIN + 8], &rstd = v[NIN + 9], &A1 = v[NIN + 10], &ws = v[NIN + 11];
+    const Tensor &xbc = v[0], &pre = v[1], &flat = v[2], &d = v[3], &wt = v[4], &raw = v[5], &key = v[6], &z2 = v[7], &nw = v[8],
+                 &rstd = v[9], &A1 = v[10], &ws = v[11];
+    const auto r = kept<Record>(ctx);
+    const Kind* in = r->in;
     const c10::DeviceGuard guard(key.device());
-    const std::vector<int64_t> sizes = ctx->saved_data["sizes"].toIntVector();
-    const std::vector<double> lim = ctx->saved_data["limits"].toDoubleVector();
-    const int64_t H = sizes[0], G = sizes[1], di = sizes[2], P = di / H, Cc = di + 2 * G, Bsz = d.size(0), Ln = d.size(1),
+    const int64_t H = r->H, G = r->G, di = r->di, P = di / H, Cc = di + 2 * G, Bsz = d.size(0), Ln = d.size(1),
                   K = d.size(2), R0 = H + 2 * G, R = H + 4 * G, Wd = di + Cc + H;
-    const Scan s = Scan::pop(v, NIN + 12, 2, !wt.defined(), lim[0], lim[1]);
-    const at::ScalarType k = key.scalar_type(), hdt = v[1].scalar_type();
+    const Scan s = Scan::pop(v, 12, 2, !wt.defined(), r->lo, r->hi);
+    const at::ScalarType k = key.scalar_type(), hdt = in[1].type;
     float* const par = data<float>(flat);
     const int64_t off_w = 2 * Cc * TAPS + 2 * Cc;
     // 4'. gated RMSNorm
@@ -677,7 +720,7 @@ struct CoreFn : public Function<CoreFn> {
     const int64_t nb = issm_rmsnorm_bwd_blocks(Bsz * Ln);
     Tensor dwp = fresh({nb, di}, key, at::kFloat), dnw = fresh({di}, key, at::kFloat);
     {
-      issm_norm_args a = norm_args(key, z2, nw, Tensor(), lim[2], 0, false, false);
+      issm_norm_args a = norm_args(key, z2, nw, Tensor(), r->eps, 0, false, false);
       a.rstd = data<float>(rstd);
       a.dy = data(dy);
       a.dy_row_stride = dy.stride(0);
@@ -745,21 +788,21 @@ struct CoreFn : public Function<CoreFn> {
     // parameter gradients, inputs 4 .. 13: one buffer, one conversion to the parameters' type when they share one
     std::vector<Tensor> pg{dcw.select(0, 0), dcb.select(0, 0), dcw.select(0, 1), dcb.select(0, 1), dW.narrow(0, 0, H),
                            dW.narrow(0, H, 2 * G), dbias_sum.narrow(0, 0, H), dA_log, g.dD, dnw};
-    bool shared = v[4].scalar_type() != at::kFloat;
-    for (int i = 4; i < NIN; ++i) shared = shared && v[i].scalar_type() == v[4].scalar_type();
+    bool shared = in[4].type != at::kFloat;
+    for (int i = 4; i < NIN; ++i) shared = shared && in[i].type == in[4].type;
     if (shared) {
       std::vector<int64_t> n;
       for (Tensor& t : pg) {
         n.push_back(t.numel());
         t = t.reshape({-1});
       }
-      pg = at::split_with_sizes(at::cat(pg).to(v[4].scalar_type()), n);
+      pg = at::split_with_sizes(at::cat(pg).to(in[4].type), n);
     }
     variable_list out(NIN + 6);
-    out[0] = cast(dzx, v[0].scalar_type());
+    out[0] = cast(dzx, in[0].type);
     out[1] = cast(dh0, hdt);
-    out[2] = cast(ddist, v[2].scalar_type());
-    for (int i = 4; i < NIN; ++i) out[i] = cast(pg[i - 4], v[i].scalar_type()).view(v[i].sizes());
+    out[2] = cast(ddist, in[2].type);
+    for (int i = 4; i < NIN; ++i) out[i] = cast(pg[i - 4], in[i].type).view(in[i].sizes);
     return out;
   }
 };

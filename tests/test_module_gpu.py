@@ -356,3 +356,28 @@ def test_hooks_of_the_layers_modules_act(which, name):
         mod.forward = plain
     for x, y in zip(a, m(*ins)):
         assert ((x - y).norm() / y.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_small_parameters_may_change_between_forward_and_backward(dtype):
+    """The layer's kernels read copies of the small parameters and of the projected queries: changing the parameters in place
+    before backward (a running average, a clamp) is no error and leaves the gradients those of the forward's values."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(9)
+    m = MultiHeadISSMScan(d_model=64, d_state=9, d_dist=16, nheads=2, expand=1).cuda().to(dtype)
+    g = torch.Generator().manual_seed(10)
+    r = lambda *s: torch.randn(*s, generator=g).cuda().to(dtype)
+    ins = (r(2, 70, 64), r(2, 9, 64), r(2, 70, 9, 16), None)
+    small = [m.key_conv.dwconv.weight, m.key_conv.dwconv.bias, m.key_conv_back.dwconv.weight, m.key_conv_back.dwconv.bias,
+             m.dt_proj.weight, m.bc_proj.weight, m.dt_bias, m.A_log, m.D]
+    grads = []
+    for change in (False, True):
+        k, q = m(*ins)
+        if change:
+            with torch.no_grad():
+                for p in small:
+                    p.add_(1.0)
+        grads.append(torch.autograd.grad(k.sum() + q.square().sum(), list(m.parameters())))
+    for (n_, _), a, b in zip(m.named_parameters(), *grads):
+        # (sums over tokens in the projections' gradients need not run in one order: 1e-2 is bf16's, 1e-5 fp32's rounding)
+        assert ((a - b).float().norm() / b.float().norm()).item() <= (1e-5 if dtype == torch.float32 else 1e-2), n_

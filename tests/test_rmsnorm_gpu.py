@@ -177,3 +177,19 @@ def test_rmsnorm_rows_at_odd_element_offsets(dtype):
     _check("dx", bg.grad[:, xs], ins[0].grad, bt)
     _check("dz", bg.grad[:, zs], ins[2].grad, bt)
     _check("dw", m.weight.grad, ins[1].grad, bt)
+
+
+def test_inputs_the_kernels_read_copies_of_may_change_before_the_backward():
+    """fp16 inputs are converted for the kernels: changing the caller's tensors afterwards is no error and changes nothing."""
+    from dest3d_amd.layernorm_gated import layernorm_fn
+    g = torch.Generator().manual_seed(2)
+    x, z = (torch.randn(40, 72, generator=g).cuda().half().requires_grad_() for _ in range(2))
+    w, b = (torch.randn(72, generator=g).cuda().half().requires_grad_() for _ in range(2))
+    dy = torch.randn(40, 72, generator=g).cuda().half()
+    want = torch.autograd.grad(layernorm_fn(x, w, b, z), (x, w, b, z), dy)
+    y = layernorm_fn(x, w, b, z)
+    with torch.no_grad():
+        for t in (x, w, b, z):
+            t.mul_(2.0)
+    for a, c in zip(torch.autograd.grad(y, (x, w, b, z), dy), want):
+        assert torch.equal(a, c)
