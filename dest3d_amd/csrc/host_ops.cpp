@@ -350,6 +350,24 @@ std::vector<Tensor> biscan(const Tensor& x_f, const Tensor& x_b, const Tensor& d
                        MaybeTensor(), softplus, lo, hi, true);
 }
 
+// The checked argument block of a call, for callers of the C ABI from Python (stage entry points, preallocated buffers), and
+// the tensors it points into.
+std::pair<py::bytes, std::vector<Tensor>> scan_args(const Tensor& x_f, const MaybeTensor& x_b, const Tensor& dt, const Tensor& A,
+                                                    const Tensor& B_f, const MaybeTensor& B_b, const Tensor& C_f,
+                                                    const MaybeTensor& C_b, const MaybeTensor& D, const MaybeTensor& z_f,
+                                                    const MaybeTensor& z_b, const MaybeTensor& dt_bias, const MaybeTensor& h0,
+                                                    const MaybeTensor& seq, bool softplus, double lo, double hi) {
+  const int ndir = x_b.has_value() ? 2 : 1;
+  const Tensor x[2] = {x_f, opt(x_b)}, B[2] = {B_f, opt(B_b)}, C[2] = {C_f, opt(C_b)}, z[2] = {opt(z_f), opt(z_b)};
+  for (int i = 0; i < ndir; ++i) check_scan(x, dt, A, B, C, ndir, opt(D), z[i], opt(dt_bias), opt(h0), opt(seq));
+  const at::NoGradGuard no_grad;
+  const Scan s = Scan::make(ndir, x, dt, A, B, C, opt(D), z, opt(dt_bias), opt(h0), opt(seq), softplus, lo, hi);
+  const issm_scan_args a = s.args();
+  std::vector<Tensor> used;
+  s.push(used);
+  return {py::bytes((const char*)&a, sizeof a), used};
+}
+
 // ------------------------------------------------------------------------------------------------------------- gated norm
 Tensor as_rows(const Tensor& t) {
   Tensor r = t.reshape({-1, t.size(-1)});
@@ -850,7 +868,13 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("scan", &scan);
   m.def("biscan", &biscan);
+  m.def("scan_args", &scan_args);
   m.def("norm", &norm);
+  m.def("norm_args", [](const Tensor& x, const MaybeTensor& z, const Tensor& w, const MaybeTensor& bias, double eps, int64_t group,
+                        bool before_gate, bool layer_norm) {
+    const issm_norm_args a = norm_args(x, opt(z), w, opt(bias), eps, group, before_gate, layer_norm);
+    return py::bytes((const char*)&a, sizeof a);
+  });
   m.def("linear_tokens", [](const Tensor& x, const Tensor& w) {
     py::gil_scoped_release release;
     return linear_tokens(x, w);

@@ -15,8 +15,6 @@ dt backwards for the second direction instead of materialising flipped copies.
 from __future__ import annotations
 
 import ctypes as C
-import math
-from typing import Optional
 
 import torch
 
@@ -25,110 +23,22 @@ from . import _lib as L
 INF = float("inf")
 
 
-def _io_cast(t: Optional[torch.Tensor], dtype: torch.dtype) -> Optional[torch.Tensor]:
-    if t is None:
-        return None
-    if t.dtype != dtype:
-        t = t.to(dtype)
-    if t.stride(-1) != 1:
-        t = t.contiguous()
-    return t
-
-
-def _f32c(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    return None if t is None else t.detach().to(torch.float32).contiguous()
-
-
-def _kernel_dtype(dt: torch.dtype) -> torch.dtype:
-    return dt if dt in (torch.float32, torch.bfloat16) else torch.float32
-
-
 class _Problem:
-    """Validated, kernel-ready view of one call (1 or 2 directions) for callers of the C ABI from Python (the stage entry
-    points, preallocated buffers); the operators below do the same in compiled code."""
+    """Kernel-ready argument block of one call (1 or 2 directions) for callers of the C ABI from Python (the stage entry
+    points, preallocated buffers): checks, conversions and the block itself are those of the operators below."""
 
     def __init__(self, xs, dt, A, Bs, Cs, chunk_size, D, zs, dt_bias, h0, seq_idx, dt_softplus, dt_limit):
-        x0 = xs[0]
-        L.require_gpu(x0, "x")
-        if x0.dim() != 4:
-            raise ValueError(f"x must be (batch, seqlen, nheads, headdim), got {tuple(x0.shape)}")
-        self.batch, self.seqlen, self.nheads, self.headdim = x0.shape
-        if Bs[0].dim() != 4:
-            raise ValueError(f"B must be (batch, seqlen, ngroups, dstate), got {tuple(Bs[0].shape)}")
-        self.ngroups, self.dstate = Bs[0].shape[2], Bs[0].shape[3]
-        b, l, h, p, g, n = self.batch, self.seqlen, self.nheads, self.headdim, self.ngroups, self.dstate
-        # shape rules of issm_combined.py:58-83
-        assert h % g == 0, "nheads must be divisible by ngroups"
-        for x_, B_, C_ in zip(xs, Bs, Cs):
-            assert x_.shape == (b, l, h, p)
-            assert B_.shape == (b, l, g, n)
-            assert C_.shape == B_.shape
-        assert dt.shape == (b, l, h, n)
-        assert A.shape == (h, n)
-        for z_ in zs:
-            if z_ is not None:
-                assert z_.shape == (b, l, h, p)
-        if D is not None:
-            assert D.shape == (h, p) or D.shape == (h,)
-        if dt_bias is not None:
-            assert dt_bias.shape == (h, n)
-        if h0 is not None:
-            assert h0.shape == (b, h, p, n)
-        self.seq_idx = None
-        if seq_idx is not None:
-            assert seq_idx.shape == (b, l)                      # issm_combined.py:70-71
-            if len(xs) != 1:
-                raise NotImplementedError("seq_idx with the fused bidirectional scan")
-            self.seq_idx = seq_idx.detach().to(torch.int32).contiguous()
-        if not (isinstance(chunk_size, int) and chunk_size > 0):
-            raise ValueError(f"chunk_size must be a positive int, got {chunk_size!r}")
-        self.ndir = len(xs)
-        self.chunk_size = chunk_size
-        self.io_dtype = _kernel_dtype(x0.dtype)
-        self.dt_dtype = _kernel_dtype(dt.dtype)
-        self.xs = [_io_cast(t.detach(), self.io_dtype) for t in xs]
-        self.Bs = [_io_cast(t.detach(), self.io_dtype) for t in Bs]
-        self.Cs = [_io_cast(t.detach(), self.io_dtype) for t in Cs]
-        self.zs = [_io_cast(None if t is None else t.detach(), self.io_dtype) for t in zs]
-        self.dt = _io_cast(dt.detach(), self.dt_dtype)
-        self.A = _f32c(A)
-        self.D = _f32c(D)
-        self.dt_bias = _f32c(dt_bias)
-        if h0 is not None:
-            self.h0 = _io_cast(h0.detach(), _kernel_dtype(h0.dtype))
-        else:
-            self.h0 = None
-        self.dt_softplus = bool(dt_softplus)
-        self.dt_limit = (float(dt_limit[0]), float(dt_limit[1]))
-        self.device = x0.device
-        self.nchunks = math.ceil(l / L.ISSM_CHUNK)
+        _chunk_size(chunk_size)
+        if seq_idx is not None and len(xs) != 1:
+            raise NotImplementedError("seq_idx with the fused bidirectional scan")
+        two = lambda v: (v[0], v[1] if len(v) > 1 else None)
+        self.device = xs[0].device
+        self._block, self._tensors = L.host().scan_args(
+            *two(xs), dt, A, *two(Bs), *two(Cs), D, *two(zs), dt_bias, h0, seq_idx, bool(dt_softplus), float(dt_limit[0]),
+            float(dt_limit[1]))
 
     def args(self) -> L.ScanArgs:
-        a = L.ScanArgs()
-        d = a.dims
-        d.batch, d.seqlen, d.nheads, d.headdim = self.batch, self.seqlen, self.nheads, self.headdim
-        d.dstate, d.ngroups, d.chunk_size, d.ndir = self.dstate, self.ngroups, self.chunk_size, self.ndir
-        a.io_dtype = L.dtype_code(self.io_dtype)
-        a.dt_dtype = L.dtype_code(self.dt_dtype)
-        a.h0_dtype = L.dtype_code(self.h0.dtype) if self.h0 is not None else L.ISSM_F32
-        a.flags = (L.FLAG_DT_SOFTPLUS if self.dt_softplus else 0) | \
-                  (L.FLAG_D_HAS_HDIM if (self.D is not None and self.D.dim() == 2) else 0)
-        if self.seq_idx is not None:
-            a.flags |= L.FLAG_SEQ_IDX
-            a.seq_idx = self.seq_idx.data_ptr()
-            a.seq_idx_stride[0], a.seq_idx_stride[1] = self.seq_idx.stride(0), self.seq_idx.stride(1)
-        a.dt_min = self.dt_limit[0]
-        a.dt_max = min(self.dt_limit[1], 3.0e38)
-        for i in range(self.ndir):
-            a.x[i] = L.tensor_desc(self.xs[i])
-            a.Bm[i] = L.tensor_desc(self.Bs[i])
-            a.Cm[i] = L.tensor_desc(self.Cs[i])
-            a.z[i] = L.tensor_desc(self.zs[i])
-        a.dt = L.tensor_desc(self.dt)
-        a.A = L.ptr(self.A)
-        a.D = L.ptr(self.D)
-        a.dt_bias = L.ptr(self.dt_bias)
-        a.h0 = L.tensor_desc(self.h0)
+        a = L.ScanArgs.from_buffer_copy(self._block)
         a.stream = L.current_stream_ptr(self.device)
         return a
 
@@ -223,19 +133,27 @@ def _merge_heads(s, t, state=False):
     return t.reshape(t.shape[0], t.shape[1], t.shape[2] // s, t.shape[3] * s)
 
 
+class ISSMBiScanFn:
+    """ISSM_biscan_combined for heads of up to 64; gradients for all tensor arguments.  The node itself is compiled."""
+
+    @staticmethod
+    def apply(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D, dt_bias, initial_states, dt_softplus, dt_limit):
+        _chunk_size(chunk_size)
+        return tuple(L.host().biscan(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, initial_states, bool(dt_softplus),
+                                     float(dt_limit[0]), float(dt_limit[1])))
+
+
 def ISSM_biscan_combined(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D=None, dt_bias=None,
                          initial_states=None, dt_softplus=False, dt_limit=(0.0, INF)):
     """Both directions of MultiHeadISSMScan's bidirectional scan in one operator call -> (y_f, y_b, last_f, last_b).
     Inputs and outputs are in natural time order; direction "b" is scanned from the last token to the first (what
     dest_module.py:568-573 obtains with four flips and a second operator call)."""
-    _chunk_size(chunk_size)
     s = _head_split(x_f.shape[-1]) if x_f.dim() == 4 else 1
     if s > 1:
         x_b = x_b.reshape(x_b.shape[0], x_b.shape[1], x_b.shape[2] * s, x_b.shape[3] // s)
         x_f, dt, A, D, _, dt_bias, initial_states = _split_heads(s, x_f, dt, A, D, None, dt_bias, initial_states)
-    res = L.host().biscan(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, D, dt_bias, initial_states, bool(dt_softplus),
-                          float(dt_limit[0]), float(dt_limit[1]))
+    res = ISSMBiScanFn.apply(x_f, x_b, dt, A, B_f, B_b, C_f, C_b, chunk_size, D, dt_bias, initial_states, dt_softplus, dt_limit)
     if s == 1:
-        return tuple(res)
+        return res
     return (_merge_heads(s, res[0]), _merge_heads(s, res[1]), _merge_heads(s, res[2], state=True),
             _merge_heads(s, res[3], state=True))

@@ -10,24 +10,9 @@ from . import _lib as L
 
 
 def _norm_args(x2, z2, w, eps, group_size, norm_before_gate, bias=None, layer_norm=False) -> L.NormArgs:
-    """The C ABI's argument block for callers from Python (preallocated buffers, graph capture)."""
-    a = L.NormArgs()
-    a.rows, a.ncols = x2.shape
-    a.group_size = 0 if group_size is None else int(group_size)
-    a.dtype = L.dtype_code(x2.dtype)
-    a.weight_dtype = L.dtype_code(w.dtype)
-    a.norm_before_gate = int(bool(norm_before_gate))
-    a.eps = float(eps)
-    a.x, a.w = x2.data_ptr(), w.data_ptr()
-    a.x_row_stride = x2.stride(0)
-    if z2 is not None:
-        a.z = z2.data_ptr()
-        a.z_row_stride = z2.stride(0)
-    if bias is not None:
-        a.bias = bias.data_ptr()
-    a.layer_norm = int(bool(layer_norm))
-    a.stream = L.current_stream_ptr(x2.device)
-    return a
+    """The C ABI's argument block for callers from Python (preallocated buffers, graph capture), as the operator fills it."""
+    return L.NormArgs.from_buffer_copy(L.host().norm_args(x2, z2, w, bias, float(eps), 0 if group_size is None else int(group_size),
+                                                          bool(norm_before_gate), bool(layer_norm)))
 
 
 class LayerNormFn:

@@ -537,6 +537,30 @@ def test_biscan_matches_two_flipped_scans_and_oracle():
     assert torch.equal(fl(y2), o[1]) and torch.equal(l2, o[3])
 
 
+def test_function_classes_take_their_arguments_in_place():
+    """``ISSMBiScanFn.apply`` and ``ISSMChunkScanCombinedFn.apply`` with positional arguments, and the argument block that
+    callers of the C ABI get from the same checks."""
+    from dest3d_amd import _lib as L
+    from dest3d_amd.issm_combined import ISSM_biscan_combined, ISSM_chunk_scan_combined, ISSMBiScanFn, ISSMChunkScanCombinedFn, _Problem
+    d = {k: v.cuda() if torch.is_tensor(v) else v for k, v in _problem(2, 70, 2, 16, 24, 1, seed=3).items()}
+    lim = d["dt_limit"]
+    a = ISSMBiScanFn.apply(d["x"], d["x"], d["dt"], d["A"], d["B"], d["B"], d["C"], d["C"], 64, d["D"], d["dt_bias"], d["h0"], True, lim)
+    b = ISSM_biscan_combined(d["x"], d["x"], d["dt"], d["A"], d["B"], d["B"], d["C"], d["C"], 64, D=d["D"], dt_bias=d["dt_bias"],
+                             initial_states=d["h0"], dt_softplus=True, dt_limit=lim)
+    assert isinstance(a, tuple) and all(torch.equal(p, q) for p, q in zip(a, b))
+    a = ISSMChunkScanCombinedFn.apply(d["x"], d["dt"], d["A"], d["B"], d["C"], 64, d["D"], None, d["dt_bias"], d["h0"], None, True, lim, True)
+    b = ISSM_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], 64, D=d["D"], dt_bias=d["dt_bias"], initial_states=d["h0"],
+                                 dt_softplus=True, dt_limit=lim, return_final_states=True)
+    assert all(torch.equal(p, q) for p, q in zip(a, b))
+    block = _Problem([d["x"]], d["dt"], d["A"], [d["B"]], [d["C"]], 64, d["D"], [None], d["dt_bias"], d["h0"], None, True, lim).args()
+    assert (block.dims.batch, block.dims.seqlen, block.dims.nheads, block.dims.headdim, block.dims.dstate, block.dims.ndir) == (2, 70, 2, 16, 24, 1)
+    assert block.x[0].ptr == d["x"].data_ptr() and (block.stream or 0) == L.current_stream_ptr(d["x"].device)
+    for bad in (dict(dt=d["dt"][:, :-1]), dict(A=d["A"].T), dict(h0=d["h0"][:1])):
+        t = dict(d, **bad)
+        with pytest.raises(AssertionError):
+            _Problem([t["x"]], t["dt"], t["A"], [t["B"]], [t["C"]], 64, t["D"], [None], t["dt_bias"], t["h0"], None, True, lim)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel(dtype):
     """Complete tiles, both directions, four heads in two groups: head 1 decays by far more than 2^96 per 16 rows
