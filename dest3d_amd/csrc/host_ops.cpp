@@ -618,6 +618,21 @@ struct CoreFn : public Function<CoreFn> {
     const int64_t Bsz = zxbcdt.size(0), Ln = zxbcdt.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
                   K = dist.size(2);
     const at::ScalarType k = kernel_type(zxbcdt.scalar_type());
+    // (the kernels address the parameters by the layer's sizes: none may be smaller than its place)
+    auto has = [](const Tensor& t, int64_t n, const char* name) {
+      TORCH_CHECK(t.numel() == n, name, " must have ", n, " entries, got ", t.numel());
+    };
+    TORCH_CHECK(zxbcdt.size(2) == di + Cc + H, "key_proj must give ", di + Cc + H, " features, got ", zxbcdt.size(2));
+    has(conv_w_f, Cc * TAPS, "key_conv.weight");
+    has(conv_w_b, Cc * TAPS, "key_conv_back.weight");
+    has(conv_b_f, Cc, "key_conv.bias");
+    has(conv_b_b, Cc, "key_conv_back.bias");
+    has(dt_w, H * WIDTH, "dt_proj.weight");
+    has(bc_w, 2 * G * WIDTH, "bc_proj.weight");
+    has(dt_bias, H, "dt_bias");
+    has(A_log, H, "A_log");
+    has(D, D.dim() == 1 ? H : H * P, "D");
+    has(norm_w, di, "key_norm.weight");
     Tensor zx = io_cast(zxbcdt, k);
     const Tensor z = zx.narrow(2, 0, di), xbc = zx.narrow(2, di, Cc);
     // all small parameters in one fp32 buffer, and A for all state columns; adjacent pieces form the stacked operands the
@@ -636,7 +651,6 @@ struct CoreFn : public Function<CoreFn> {
         a.n[i] = (int32_t)t.numel();
         a.dtype[i] = code(small[i].scalar_type());
       }
-      TORCH_CHECK(A_log.numel() == H, "A_log must have one entry per head");
       flat = fresh({off[NSMALL]}, zx, at::kFloat);
       a.a_log = A_LOG;
       a.K = (int32_t)K;

@@ -381,3 +381,20 @@ def test_small_parameters_may_change_between_forward_and_backward(dtype):
     for (n_, _), a, b in zip(m.named_parameters(), *grads):
         # (sums over tokens in the projections' gradients need not run in one order: 1e-2 is bf16's, 1e-5 fp32's rounding)
         assert ((a - b).float().norm() / b.float().norm()).item() <= (1e-5 if dtype == torch.float32 else 1e-2), n_
+
+
+@pytest.mark.parametrize("name,shape", [("dt_proj.weight", (1, 16)), ("bc_proj.weight", (1, 16)), ("dt_bias", (1,)), ("A_log", (1,)),
+                                        ("D", (1,)), ("D", (3,)), ("key_norm.weight", (32,)), ("key_conv.dwconv.weight", (65, 1, 7)),
+                                        ("key_conv_back.dwconv.bias", (60,)), ("key_proj.weight", (100, 64))])
+def test_parameters_of_another_size_are_refused(name, shape):
+    """A parameter that is not of the layer's size raises before any kernel is given its address."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    m = MultiHeadISSMScan(d_model=64, d_state=9, d_dist=16, nheads=2, expand=1).cuda()
+    *path, last = name.split(".")
+    mod = m
+    for part in path:
+        mod = getattr(mod, part)
+    setattr(mod, last, torch.nn.Parameter(torch.randn(shape, device="cuda")))
+    r = lambda *s: torch.randn(*s, device="cuda")
+    with pytest.raises(RuntimeError):
+        m(r(1, 70, 64), r(1, 9, 64), r(1, 70, 9, 16), None)
