@@ -121,7 +121,7 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
 // and not stored.  The diagonal blocks of M take fp32 matrix instructions: the level form, which evaluates such calls
 // wherever this kernel cannot, has the pairs inside groups of four rows in fp32, and what a pair is computed in is not to
 // depend on the kernel.  (Those entries of M: 2.4e-3 from float64 with operands rounded once to bf16, 4.4e-6 as bf16 pairs,
-// 2.6e-7 like this.  4 x 1000 tokens, heads of 36, 200 states, fp32, forward + backward: 221.6 us with pairs, 222.4 like this.)
+// 2.6e-7 like this.  8 x 1024 tokens, 8 heads x 32, N = 250: fp32 55.4 us with pairs, 55.8 like this; bf16 43.4 and 46.9.)
 template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
@@ -288,11 +288,24 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     }
 
     // ---- operands
+    float w16[EDGE ? 16 : 1];
+    if constexpr (EDGE) {
+      // diagonal blocks, before anything else needs registers: W takes the place of B and dt', C up that of C.  fp32 matrix
+      // instructions: k-slot kg of instruction r <-> the lane's column r; the blocks' chains are interleaved.
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        w16[k] = dtp[k] * bv[k] * ex2(-pc[k]);
+        cv[k] *= up[k];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int J = 0; J < 4; ++J) macc[J] = mfma4(cv[4 * J + r], w16[4 * J + r], macc[J]);
+    }
+    auto cu = [&](int k) { return EDGE ? cv[k] : cv[k] * up[k]; };
     Fr U[4];
 #pragma unroll
-    for (int J = 0; J < 4; ++J)
-      U[J] = make_frag<SPLIT>(cv[4 * J] * up[4 * J], cv[4 * J + 1] * up[4 * J + 1], cv[4 * J + 2] * up[4 * J + 2],
-                              cv[4 * J + 3] * up[4 * J + 3]);
+    for (int J = 0; J < 4; ++J) U[J] = make_frag<SPLIT>(cu(4 * J), cu(4 * J + 1), cu(4 * J + 2), cu(4 * J + 3));
     f4 sacc[PT];
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) sacc[pt] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
@@ -302,13 +315,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int k = 4 * J + r;
-        W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
+        if constexpr (EDGE) W[r] = w16[k];
+        else W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
         V[r] = W[r] * et[k];
       }
-      if constexpr (EDGE) {  // fp32 matrix instructions: k-slot kg of instruction r <-> the lane's column r
-#pragma unroll
-        for (int r = 0; r < 4; ++r) macc[J] = mfma4(cv[4 * J + r] * up[4 * J + r], W[r], macc[J]);
-      } else {
+      if constexpr (!EDGE) {
         const Fr f = make_frag<SPLIT>(W[0], W[1], W[2], W[3]);
         macc[J] = frag_product<SPLIT>(U[J], f, macc[J]);
       }
