@@ -121,8 +121,8 @@ static FwdWs fwd_layout(const issm_dims& d, bool has_z) {
 
 static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
 // Partial sums that would be rounded to bf16 on their way between kernels: with two directions and a bf16 ddt the first
-// direction's share of ddt in fp32 ((B, L, H, N)), with bf16 inputs and incomplete
-// tiles dB and dC of workgroups two kernels share (KP::dbc_part).
+// direction's share of ddt in fp32 ((B, L, H, N)), with bf16 inputs and incomplete tiles dB and dC of workgroups two
+// kernels share (KP::dbc_part).
 static BwdWs bwd_layout(const issm_scan_args* a) {
   const issm_dims& d = a->dims;
   const bool has_z = a->z[0].ptr != nullptr, ddt_part = wants_ddt_part(a);

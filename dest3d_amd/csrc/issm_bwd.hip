@@ -4,7 +4,8 @@
 //   k_bwd_dstates   dH_c = dy^T (C*exp(cs))  and  dM = tril(dy x^T)
 //   k_state_bwd_full / k_state_bwd   reverse inter-chunk recurrence (HBM streaming)
 //   k_bwd_chunk     per (chunk, group, 64-column slice), looping over the heads of the
-//                   group: ddt, dB, dC and the per-unit partial sums of dA / ddt_bias
+//                   group: ddt, dB, dC and the per-unit partial sums of dA / ddt_bias; for the
+//                   calls and heads that k_bwd_tile (issm_bwd_tile.hip) does not take
 //   k_bwd_dx        dx and the per-unit partial sums of dD
 //   k_bwd_reduce    fixed-order sums of the partials (bit-reproducible, no atomics), one launch
 //
@@ -1776,8 +1777,8 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
 
 int launch_state_bwd(const KP& p, const float* states, const float* cs_last, float* dstates, float* g_last,
                      float* dh0_dir, hipStream_t st) {
-  // One workgroup walks the chunks of its columns one after the other.  Complete shapes take the variant without
-  // conditional accesses; with few (batch, head) pairs narrower column slices put more workgroups on the chip.
+  // One workgroup walks the chunks of its columns one after the other.  From four columns on the accesses are
+  // unconditional (TAIL: the last slice is not full); with few (batch, head) pairs narrower column slices put more workgroups on the chip.
   const int wide = p.B * p.ndir * p.H * ((p.N + 63) / 64);
   // (sequence of the tests: slices of 32 columns where 64 would leave the chip idle or N fits them exactly)
 #define ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, TAIL_)                                                                         \
@@ -1831,8 +1832,9 @@ int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const 
 
 // Chunk backward of direction p.dir0.  With a `redo` buffer (issm_bwd_chunk_redo_ints words) the tile-base kernel
 // (issm_bwd_tile.hip) does the work and marks the heads outside its range; launch_bwd_chunk_redo then evaluates those
-// with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (packed
-// sequences, a gate beside bf16 inputs, mixed input types), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
+// with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (bwd_tile_available:
+// packed sequences, a gate beside bf16 inputs, mixed input types, fp32 heads of more than 48, heads or rows of x and dout
+// that are no multiple of four elements), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
                      const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);

@@ -1,7 +1,8 @@
 // Forward kernels of the ISSM chunked scan for gfx950.
 //
 //   k_chunk_local   dt transform + cumsum, chunk-local end states S_c and the intra-chunk
-//                   matrix M_c = "C.A.B^T" in one pass over dt
+//                   matrix M_c = "C.A.B^T" in one pass over dt, in the form below; calls without
+//                   packed sequences take k_local_tile (issm_fwd_tile.hip) from four state columns on
 //   k_state_fwd_full / k_state_fwd   inter-chunk recurrence (HBM streaming)
 //   k_chunk_scan    y = (C*exp(cs)) H^T + tril(M) x + D x, optional gate
 //

@@ -1,6 +1,7 @@
 // The chunk-local pass of the forward in its level-hierarchy form (any tile shape, any decay): shared memory, helpers and
-// the kernel body.  Included by the file that launches it as k_chunk_local and by the row-lane kernel for complete tiles,
-// which calls the same body for the chunks outside its own range.
+// the kernel body.  Included by the file that launches it as k_chunk_local (packed sequences, fewer than four state columns,
+// stage calls that want one output only) and by the row-lane kernel k_local_tile, which takes every other call and runs this
+// body for the chunks outside its own range.
 #pragma once
 #include "issm_dev.h"
 

@@ -29,11 +29,13 @@
  *    one call: direction 1 walks the same dt / A / D / h0 backwards in time with its
  *    own x / Bm / Cm and writes its outputs back in natural (un-flipped) time order.
  *  - Numerics: cumulative sums, decays, dt', states and all accumulation are fp32 for every
- *    I/O dtype.  With io_dtype = ISSM_F32 the products x^T.(B dt' decay), dy^T.(C decay),
- *    x.dS, dy.H and the within-chunk matrix M of the forward are evaluated as three bf16
- *    matrix products with fp32 accumulation on operands split into bf16 high and low parts
- *    (16 significand bits per operand; relative error of a product <= 2^-16); every other
- *    product is fp32.  With io_dtype = ISSM_BF16 every matrix product takes its operands
+ *    I/O dtype.  With io_dtype = ISSM_F32 matrix products are evaluated as three bf16 matrix
+ *    products with fp32 accumulation on operands split into bf16 high and low parts (16
+ *    significand bits per operand; relative error of a product <= 2^-16; four products and
+ *    <= 2^-18 per operand in the chunk backward of complete tiles).  fp32 products: pairs of
+ *    rows of one 16-row tile in M, and the sums over pairs of rows of the chunk backward,
+ *    where L or N is no multiple of 64 (the latter also with a z gate); the sums over pairs of
+ *    rows of the chunk backward for heads wider than 48 and decays beyond 2^-96 a tile.  With io_dtype = ISSM_BF16 every matrix product takes its operands
  *    rounded once to bf16 (as the reference's kernels cast their dot operands to the input
  *    dtype, issm_triton/issm_cabt_bmm.py:42-43), except x.dS, dy.H and the chunk state
  *    x^T.(B dt' decay), whose fp32 operands enter as high and low parts; the gradient of
