@@ -847,26 +847,58 @@ __global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int sp
 }
 // Its gradient, all of grad_points (b, c, m) written.  Adding target by target into rows of sums in LDS takes 600 us (8
 // samples, 256 channels, 2048 <- 20000 points): an LDS float addition to scattered words runs at a third of a lane a cycle.
-// So the targets' three (point, weight) entries are sorted by point first, once for all channels -- k_inverse_rank counts
-// and gives every entry its place within its point, k_inverse_fill writes (point, target, weight) in that order, thread t's
-// share of the sorted list at [i][t] -- and k_interp_rows_grad holds R rows of grad_out in LDS, reads them by target, sums
-// runs of a point in registers and adds a run's sum to the result.  212 us and 33 for the lists, 397 with atomics into a channel-last buffer.
-constexpr int INV_T = 1024;
-__global__ __launch_bounds__(INV_T) void k_inverse_rank(int n, int m, const int* __restrict__ idx, int* __restrict__ start,
-                                                        int* __restrict__ rank) {
+// So the targets' three (point, weight) entries are sorted by point first, once for all channels: k_inverse_rank counts and
+// gives every entry its place within its point, k_inverse_fill writes the list.  A point's entries fill whole blocks of
+// INV_E, so that a lane of k_interp_rows_grad sums a block without asking where a point ends; neighbouring lanes with one
+// point add up by row-lane moves, and the last of them writes the sum; what a wave's share of the list has of its first and
+// last point meets in LDS.  No atomics: a thread per 59 entries that added every run it finished to the result took 211 us,
+// the waits for its list behind those additions in the one counter both have, and one addition at either end of 64 blocks
+// still cost 70 of 147 us.  81 us here, one row or two a workgroup alike (164 MB read: 36 at the copy's rate; 49 without
+// reading them), 11 + 12 for the list; longer blocks or more of the list in flight gave nothing.  397 with atomics into a
+// channel-last buffer.
+constexpr int INV_T = 1024, INV_E = 8;
+struct InvList {              // per sample `blocks` places
+  unsigned* target;           // [place][INV_E / 2] two targets each
+  float* weight;              // [INV_E / 4][place][4]
+  unsigned* point;            // entries << 16 | point
+  int *count, *first, *rank;  // [m] entries of a point, [m + 1] its first block (last: all blocks), [3 n] places in the point
+  int blocks;
+  // most blocks that 3 n entries of m points can take
+  static long most(long n, long m) { return (3 * n + (INV_E - 1) * std::min(3 * n, m)) / INV_E + 1; }
+  static long ints(long b, long n, long m) { return b * (most(n, m) * (INV_E / 2 + INV_E + 1) + 2 * m + 1 + 3 * n); }
+  InvList(int* ws, long b, long n, long m) : blocks((int)most(n, m)) {
+    target = (unsigned*)ws;
+    weight = (float*)(target + b * blocks * (INV_E / 2));
+    point = (unsigned*)(weight + b * blocks * INV_E);
+    count = (int*)(point + b * blocks);
+    first = count + b * m;
+    rank = first + b * (m + 1);
+  }
+};
+__global__ __launch_bounds__(INV_T) void k_inverse_rank(int n, int m, const int* __restrict__ idx, InvList l) {
   extern __shared__ int cnt[];
   __shared__ int wsum[INV_T / 64];
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int k = tid; k < m; k += INV_T) cnt[k] = 0;
   __syncthreads();
   const int* q = idx + (long)b * n * 3;
-  int* r = rank + (long)b * n * 3;
-#pragma unroll 4
-  for (int e = tid; e < 3 * n; e += INV_T) r[e] = atomicAdd(cnt + index_of(q[e], m), 1);
+  int* r = l.rank + (long)b * n * 3;
+  constexpr int U = 16;   // entries of a thread in flight: one workgroup a sample, so latency is all there is (20 us with four)
+  for (int e0 = tid; e0 < 3 * n; e0 += INV_T * U) {
+    int k[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) k[u] = index_of(q[min(e0 + INV_T * u, 3 * n - 1)], m);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + INV_T * u < 3 * n) k[u] = atomicAdd(cnt + k[u], 1);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + INV_T * u < 3 * n) r[e0 + INV_T * u] = k[u];
+  }
   __syncthreads();
   const int per = (m + INV_T - 1) / INV_T, k0 = tid * per, k1 = min(k0 + per, m);
   int own = 0;
-  for (int k = k0; k < k1; ++k) own += cnt[k];
+  for (int k = k0; k < k1; ++k) own += (cnt[k] + INV_E - 1) / INV_E;
   int incl = own;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -877,69 +909,185 @@ __global__ __launch_bounds__(INV_T) void k_inverse_rank(int n, int m, const int*
   __syncthreads();
   int at = incl - own;
   for (int w = 0; w < wave; ++w) at += wsum[w];
+  int* first = l.first + (long)b * (m + 1);
   for (int k = k0; k < k1; ++k) {
-    start[(long)b * m + k] = at;
-    at += cnt[k];
+    first[k] = at;
+    l.count[(long)b * m + k] = cnt[k];
+    at += (cnt[k] + INV_E - 1) / INV_E;
   }
+  if (tid == INV_T - 1) first[m] = at;
 }
-// list entry: point << 16 | target, weight.  Places behind the 3 n entries hold point NO_POINT, whose sum is never written
-// (a weight of 0 alone would not do: 0 times an infinite or undefined gradient is no number).
-constexpr unsigned NO_POINT = 0xffffu;
-static_assert(ROW_POINTS < (int)NO_POINT, "no point has this number");
-__global__ __launch_bounds__(NTHREADS) void k_inverse_fill(int n, int m, int per, const int* __restrict__ idx,
-                                                           const float* __restrict__ weight, const int* __restrict__ start,
-                                                           const int* __restrict__ rank, uint2* __restrict__ list) {
+// Writes the list and clears the result (the sums of points that two waves meet at are added to it).
+__global__ __launch_bounds__(NTHREADS) void k_inverse_fill(int n, int m, const int* __restrict__ idx, const float* __restrict__ weight,
+                                                           InvList l, int pad, long total, float* __restrict__ grad_points) {
   const int b = blockIdx.y, e = blockIdx.x * NTHREADS + threadIdx.x;
-  if (e >= per * INV_T) return;
-  int at = e;
-  uint2 v = make_uint2(NO_POINT << 16, 0u);
-  if (e < 3 * n) {
-    const int k = index_of(idx[(long)b * n * 3 + e], m);
-    at = start[(long)b * m + k] + rank[(long)b * n * 3 + e];
-    v = make_uint2((unsigned)k << 16 | (unsigned)(e / 3), __builtin_bit_cast(unsigned, weight[(long)b * n * 3 + e]));
-  }
-  list[(long)b * per * INV_T + (long)(at % per) * INV_T + at / per] = v;
+  const long threads = (long)gridDim.x * gridDim.y * NTHREADS;
+  for (long z = ((long)b * gridDim.x + blockIdx.x) * NTHREADS + threadIdx.x; z < total; z += threads) grad_points[z] = 0.0f;
+  if (e >= 3 * n) return;
+  const int k = index_of(idx[(long)b * n * 3 + e], m), r = l.rank[(long)b * n * 3 + e], cnt = l.count[(long)b * m + k];
+  const long base = (long)b * l.blocks, at = base + l.first[(long)b * (m + 1) + k] + r / INV_E;
+  unsigned short* t = (unsigned short*)(l.target + at * (INV_E / 2));
+  auto put = [&](int i, int target, float w) {
+    t[i] = (unsigned short)target;
+    l.weight[((base * (INV_E / 4)) + (long)(i / 4) * l.blocks + (at - base)) * 4 + i % 4] = w;
+  };
+  put(r % INV_E, e / 3, weight[(long)b * n * 3 + e]);
+  if (r % INV_E == 0) l.point[at] = (unsigned)min(cnt - r, INV_E) << 16 | (unsigned)k;
+  if (r == cnt - 1)
+    for (int i = r % INV_E + 1; i < INV_E; ++i) put(i, pad, 0.0f);
 }
-template <int R>
-__global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m, int per, const float* __restrict__ grad_out,
-                                                            const uint2* __restrict__ list, float* __restrict__ grad_points) {
-  extern __shared__ float srow[];
+constexpr unsigned NO_POINT = 0xffffu;
+static_assert(ROW_POINTS < (int)NO_POINT, "no point has this number, and a target fits in 16 bits");
+// R rows of grad_out in LDS, a target's R values side by side, and behind them the value zero that the entries filling up a
+// block read (a weight of zero alone would not do: zero times a gradient that is no number is none); where the row itself
+// takes all of the LDS (ZERO = false) such entries are told by the block's count.
+template <int R, bool ZERO>
+__global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m, const float* __restrict__ grad_out, InvList l,
+                                                           float* __restrict__ grad_points) {
+  extern __shared__ __align__(16) float srow[];
+  typedef float Vals __attribute__((ext_vector_type(R)));
+  typedef unsigned u4_any __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int T = INV_T;
   const int wg = xcd_remap(blockIdx.x, gridDim.x), per_b = (c + R - 1) / R;   // an XCD's workgroups: one sample's list in its L2
-  const int tid = threadIdx.x, b = wg / per_b, c0 = (wg % per_b) * R, nch = min(R, c - c0);
+  const int tid = threadIdx.x, lane = tid & 63, b = wg / per_b, c0 = (wg % per_b) * R, nch = min(R, c - c0);
   const float* g = grad_out + ((long)b * c + c0) * n;   // R neighbouring rows
-  for (int k = 4 * tid; k + 3 < nch * n; k += 4 * INV_T) *(f4*)(srow + k) = ld_stream(g + k);
-  {
-    const int k = (nch * n & ~3) + tid;
-    if (k < nch * n) srow[k] = g[k];
-  }
-  __syncthreads();
-  const uint2* q = list + (long)b * per * INV_T + tid;
+  const int blocks = l.first[(long)b * (m + 1) + m];
+  const long base = (long)b * l.blocks;
+  const unsigned* pt = l.point + base;
+  const u4_any* tg = (const u4_any*)(l.target + base * (INV_E / 2));
+  const f4_stream *w0 = (const f4_stream*)(l.weight + base * INV_E), *w1 = w0 + l.blocks;
   float* o = grad_points + ((long)b * c + c0) * m;
-  float acc[R];
+  if (blocks == 0) return;
+  // sums of a point over the lanes before (a point's lanes lie side by side); on: one point from the row's first lane, or from
+  // as far back as the step looks, to here
+  auto scan = [&](unsigned k, float (&s)[R]) {
+    int on = __builtin_amdgcn_update_dpp(-1, (int)k, 0x138, 0xf, 0xf, false) == (int)k ? -1 : 0;
+    auto step = [&](auto ctrl, auto rows) {
+      constexpr int C = decltype(ctrl)::value, M = decltype(rows)::value;
 #pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-  unsigned cur = per ? q[0].x >> 16 : NO_POINT;
-  auto put = [&]() {
-    if (cur == NO_POINT) return;
+      for (int r = 0; r < R; ++r)
+        s[r] += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s[r]), C, M, 0xf, false) & on);
+      on &= __builtin_amdgcn_update_dpp(-1, on, C, M, 0xf, false);
+    };
+    typedef std::integral_constant<int, 0xf> All;
+    step(std::integral_constant<int, 0x111>{}, All{});
+    step(std::integral_constant<int, 0x112>{}, All{});
+    step(std::integral_constant<int, 0x114>{}, All{});
+    step(std::integral_constant<int, 0x118>{}, All{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+  };
+  auto after = [&](unsigned k) {   // the next lane's
+    return (unsigned)__builtin_amdgcn_update_dpp(-1, (int)k, 0x130, 0xf, 0xf, false);
+  };
+  auto put = [&](unsigned k, const float (&s)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      if (r < nch) unsafeAtomicAdd(o + (long)r * m + cur, acc[r]);
+      if (r < nch) o[(long)r * m + k] = s[r];
   };
-#pragma unroll 4
-  for (int i = 0; i < per; ++i) {
-    const uint2 v = q[(long)i * INV_T];
-    const unsigned k = v.x >> 16, j = v.x & 0xffffu;
-    const float w = __builtin_bit_cast(float, v.y);
-    if (k != cur) {
-      put();
-      cur = k;
+  // a wave's share of the list, 64 blocks a step.  first: the share's first point, to which earlier waves may have something
+  // to add, and its sum (head) once it has ended; open, carry: the point of the step's last block and its sum so far
+  const int share = (blocks + T / 64 - 1) / (T / 64), end = min(blocks, ((tid >> 6) + 1) * share);
+  int at = (tid >> 6) * share + lane;
+  struct Block { unsigned p; u4_any t; f4 wa, wb; };
+  auto load = [&](int i) {
+    i = min(i, blocks - 1);
+    return Block{pt[i], tg[i], w0[i], w1[i]};
+  };
+  Block q0 = load(at);
+  constexpr int U = R == 1 ? 5 : 2;   // steps in flight (more registers would cost the second workgroup on a CU)
+  for (int k0 = 4 * tid; k0 + 3 < n; k0 += 4 * T * U) {
+    f4 v[U][R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[u][r] = ld_stream(g + (long)min(r, nch - 1) * n + min(k0 + 4 * T * u, n - 4));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 4 * T * u;
+      if (k + 3 < n) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < R; ++r) srow[(k + j) * R + r] = v[u][r][j];
+      }
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] += w * srow[min(r, nch - 1) * n + j];
   }
-  put();
+  {
+    const int k = (n & ~3) + tid;
+    if (k < n)
+#pragma unroll
+      for (int r = 0; r < R; ++r) srow[k * R + r] = g[(long)min(r, nch - 1) * n + k];
+  }
+  if (ZERO && tid < R) srow[n * R + tid] = 0.0f;
+  __syncthreads();
+  unsigned open = NO_POINT;
+  bool ended = false;
+  float carry[R], head[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) carry[r] = head[r] = 0.0f;
+  const unsigned first = __builtin_amdgcn_readfirstlane(q0.p & 0xffffu);
+  auto take = [&](const Block& q, int at) {
+    const unsigned k = at < end ? q.p & 0xffffu : NO_POINT;
+    float s[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < INV_E; ++e) {
+      const unsigned j = e & 1 ? q.t[e / 2] >> 16 : q.t[e / 2] & 0xffffu;
+      const Vals v = *(const Vals*)(srow + j * R);
+      const float w = e < 4 ? q.wa[e & 3] : q.wb[e & 3];
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] += w * (ZERO || e < (int)(q.p >> 16) ? v[r] : 0.0f);
+    }
+    scan(k, s);
+    const int last = __builtin_amdgcn_readfirstlane(min(63, end - 1 - at));   // of the step's blocks
+    const unsigned k0 = (unsigned)__builtin_amdgcn_readlane((int)k, 0), k_last = (unsigned)__builtin_amdgcn_readlane((int)k, last);
+    if (k0 == open) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] += k == k0 ? carry[r] : 0.0f;
+    } else if (open != NO_POINT) {   // it ended with the last step
+      if (open == first) {
+        ended = true;
+#pragma unroll
+        for (int r = 0; r < R; ++r) head[r] = carry[r];
+      } else if (lane == 0) put(open, carry);
+    }
+    if (k0 == first && k_last != first) {
+      ended = true;
+      const int l = __popcll(__ballot(k == first)) - 1;
+#pragma unroll
+      for (int r = 0; r < R; ++r) head[r] = lane_f(s[r], l);
+    }
+    if (lane < last && after(k) != k && k != first) put(k, s);
+    open = k_last;
+#pragma unroll
+    for (int r = 0; r < R; ++r) carry[r] = lane_f(s[r], last);
+  };
+  for (; at - lane < end; at += 64) {   // uniform
+    const Block n0 = load(at + 64);
+    take(q0, at);
+    q0 = n0;
+  }
+  // the waves' first and last points, in order
+  __syncthreads();
+  if (lane < 2) {
+    float* e = srow + ((tid >> 6) * 2 + lane) * (R + 1);
+    e[0] = __builtin_bit_cast(float, lane == 0 && ended ? first : open);
+#pragma unroll
+    for (int r = 0; r < R; ++r) e[1 + r] = lane ? carry[r] : ended ? head[r] : 0.0f;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const bool in = lane < T / 32;
+    const float* e = srow + (in ? lane : 0) * (R + 1);
+    const unsigned k = in ? __builtin_bit_cast(unsigned, e[0]) : NO_POINT;
+    float s[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = e[1 + r];
+    scan(k, s);
+    if (after(k) != k && k != NO_POINT) put(k, s);
+  }
 }
 
 // Gradients into a channel-last buffer, out_cl (b, n, c) += ...: a 64 x 64 tile of grad_out (channels x entries) is
@@ -1103,31 +1251,25 @@ int launch_three_interpolate(int b, int c, int m, int n, const float* points, co
                      out);
   return (int)hipGetLastError();
 }
-// ints of scratch: start (b, m), rank (b, 3 n), list (b, per * INV_T) of two
-static int inverse_per(int n) { return (3 * n + INV_T - 1) / INV_T; }
-long interp_rows_grad_ints(int b, int n, int m) { return (long)b * ((m + 3L * n + 1) / 2 * 2 + 2L * inverse_per(n) * INV_T); }
+long interp_rows_grad_ints(int b, int n, int m) { return InvList::ints(b, n, m); }
 int launch_interp_rows_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight, int* ws,
                             float* grad_points, hipStream_t st) {
-  const int per = inverse_per(n);
-  uint2* list = (uint2*)ws;
-  int *start = ws + 2L * b * per * INV_T, *rank = start + (long)b * m;
-  if (int e = set_lds_rows(&k_inverse_rank, m * sizeof(int))) return e;
-  hipLaunchKernelGGL(k_inverse_rank, dim3(b), dim3(INV_T), m * sizeof(int), st, n, m, idx, start, rank);
-  hipLaunchKernelGGL(k_inverse_fill, dim3((per * INV_T + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, per, idx, weight,
-                     start, rank, list);
+  const InvList l(ws, b, n, m);
   const long total = (long)b * c * m;
-  hipLaunchKernelGGL(k_zero, dim3(zero_blocks(total)), dim3(NTHREADS), 0, st, total, grad_points);
+  const int zero = n < ROW_POINTS ? 1 : 0;
+  if (int e = set_lds_rows(&k_inverse_rank, m * sizeof(int))) return e;
+  hipLaunchKernelGGL(k_inverse_rank, dim3(b), dim3(INV_T), m * sizeof(int), st, n, m, idx, l);
+  hipLaunchKernelGGL(k_inverse_fill, dim3(blocks_for(std::max(3L * n, 1L)), b), dim3(NTHREADS), 0, st, n, m, idx, weight, l, zero ? n : 0, total, grad_points);
   auto go = [&](auto kern, int r) -> int {
-    const size_t sm = (size_t)r * n * sizeof(float);
+    const size_t sm = std::max((size_t)r * (n + zero), (size_t)INV_T / 32 * (r + 1)) * sizeof(float);
     if (int e = set_lds_rows(kern, sm)) return e;
-    hipLaunchKernelGGL(kern, dim3((c + r - 1) / r * b), dim3(INV_T), sm, st, c, n, m, per, grad_out, list, grad_points);
+    hipLaunchKernelGGL(kern, dim3((c + r - 1) / r * b), dim3(INV_T), sm, st, c, n, m, grad_out, l, grad_points);
     return 0;
   };
-  // more rows per workgroup: the list is read less often; as many as fit, where that leaves a workgroup for every CU
   int e;
-  if (n <= ROW_POINTS / 4 && (long)b * ((c + 3) / 4) >= 256) e = go(&k_interp_rows_grad<4>, 4);
-  else if (n <= ROW_POINTS / 2 && (long)b * ((c + 1) / 2) >= 256) e = go(&k_interp_rows_grad<2>, 2);
-  else e = go(&k_interp_rows_grad<1>, 1);
+  if (n < ROW_POINTS / 4 && (long)b * ((c + 3) / 4) >= 256) e = go(&k_interp_rows_grad<4, true>, 4);
+  else if (n < ROW_POINTS / 2 && (long)b * ((c + 1) / 2) >= 256) e = go(&k_interp_rows_grad<2, true>, 2);
+  else e = zero ? go(&k_interp_rows_grad<1, true>, 1) : go(&k_interp_rows_grad<1, false>, 1);
   return e ? e : (int)hipGetLastError();
 }
 int launch_three_interpolate_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight,

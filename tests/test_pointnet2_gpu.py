@@ -317,6 +317,42 @@ def test_interpolation_rows(c, m, n):
     assert np.abs(f.grad.cpu().numpy() - gref).max() <= 1e-5 * np.abs(gref).max()
 
 
+@pytest.mark.parametrize("b,c", [(1, 1), (2, 5), (2, 515), (3, 1027)])
+@pytest.mark.parametrize("n,m,kind", [(1, 1, "any"), (21, 4, "eights"), (22, 70, "any"), (171, 1, "any"), (1366, 3, "sorted"),
+                                      (1366, 300, "one has most"), (4000, 900, "eights"), (9000, 4000, "any")])
+def test_interpolation_gradient_lists(b, c, n, m, kind):
+    """The sorted lists at their remainders, one, two and four rows a workgroup (the last one short): points whose entries
+    fill blocks of eight, fill several waves' shares, or are none; called through the C ABI at every size.  A point's sum of
+    k products carries at most k + 1 roundings of 2^-24 of the sum of their magnitudes."""
+    from dest3d_amd import _lib as L
+    lib = L.load()
+    rng = np.random.default_rng(n + c)
+    idx = rng.integers(0, m, size=(b, n * 3))
+    if kind == "eights":
+        idx = np.repeat(rng.integers(0, m, size=(b, n)), 8, axis=1)[:, :n * 3]
+    elif kind == "one has most":
+        idx[:, 20:n * 3 - 20] = m // 2
+    elif kind == "sorted":
+        idx.sort(axis=1)
+    idx = idx.reshape(b, n, 3).astype(np.int32)
+    w = rng.uniform(0, 1, size=(b, n, 3)).astype(np.float32)
+    gy = rng.standard_normal((b, c, n)).astype(np.float32)
+    tg, ti, tw = _cuda(gy), _cuda(idx), _cuda(w)
+    ws = torch.empty(lib.issm_pn2_three_interpolate_grad_rows_workspace(b, n, m), dtype=torch.uint8, device="cuda")
+    out = torch.full((b, c, m), float("nan"), device="cuda")
+    L.check(lib.issm_pn2_three_interpolate_grad_rows(b, c, n, m, tg.data_ptr(), ti.data_ptr(), tw.data_ptr(), ws.data_ptr(),
+                                                     out.data_ptr(), L.current_stream_ptr(out.device)), "interp grad rows")
+    got = out.cpu().numpy()
+    for i in range(b):
+        ref, size = np.zeros((m, c)), np.zeros((m, c))
+        for k in range(3):
+            term = gy[i].T.astype(np.float64) * w[i, :, k:k + 1]
+            np.add.at(ref, idx[i, :, k], term)
+            np.add.at(size, idx[i, :, k], np.abs(term))
+        count = np.bincount(idx[i].ravel(), minlength=m)[:, None]
+        assert (np.abs(got[i].T - ref) <= (count + 1) * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("c,m,n", [(300, 50, 3501), (700, 3, 5121), (220, 900, 9999), (60, 1000, 40960)])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 def test_interpolation_rows_keep_a_target_without_a_number_to_its_points(c, m, n, value):
