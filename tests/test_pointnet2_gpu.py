@@ -125,6 +125,32 @@ def test_ball_query(shape):
     assert (idx.cpu().numpy() == R.ball_query(radius, nsample, xyz, q.astype(np.float32))).all()
 
 
+@pytest.mark.parametrize("b,n,m", [(1, 1025, 17), (2, 5121, 40), (1, 9300, 64), (5, 1500, 3300)])
+@pytest.mark.parametrize("kind", ["spread", "in order along an axis", "heaps", "no numbers"])
+def test_ball_query_looks_in_order_and_masks(b, n, m, kind):
+    """Behind the first 1024 points a centre either goes on looking in order or takes the masks, leaves them when it has enough,
+    or overflows its list in the middle of a chunk of 4096 points; one and four centres a wave, more slots than a list holds."""
+    from dest3d_amd.pointnet2_utils import ball_query
+    rng = np.random.default_rng(n + m)
+    xyz = rng.uniform(0, 8, size=(b, n, 3)).astype(np.float32)
+    if kind == "in order along an axis":
+        xyz[..., 1].sort(axis=1)
+    elif kind == "heaps":                  # 300 points in one place, behind the first chunk where there is one
+        at = max(n - 300, 1024)
+        xyz[:, at:at + 300] = xyz[:, 5:6] + rng.normal(0, 0.01, size=xyz[:, at:at + 300].shape).astype(np.float32)
+    q = xyz[:, rng.integers(0, n, size=m)] + rng.normal(0, 0.05, size=(b, m, 3)).astype(np.float32)
+    q[:, 0] = xyz[:, 5]
+    if kind == "no numbers":
+        xyz[:, n // 2, 0] = np.nan
+        xyz[:, n // 3] = np.inf
+        q[0, 1, 2] = np.nan
+        q[-1, 2, 1] = -np.inf
+    for radius, nsample in ((0.3, 16), (0.8, 64), (1.1, 200), (-0.5, 3), (0.0, 4), (30.0, 5)):
+        idx = ball_query(radius, nsample, _cuda(xyz), _cuda(q)).cpu().numpy()
+        with np.errstate(invalid="ignore"):
+            assert (idx == R.ball_query(radius, nsample, xyz, q)).all(), (radius, nsample)
+
+
 def test_three_nn_and_interpolate():
     from dest3d_amd.pointnet2_utils import three_interpolate, three_nn
     rng = np.random.default_rng(5)
