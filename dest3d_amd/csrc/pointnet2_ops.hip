@@ -561,9 +561,10 @@ __global__ __launch_bounds__(NTHREADS) void k_group_points(GroupP g) {
 
 // The output's entries, row after row, in equal shares of one workgroup each; of every row it meets, a workgroup holds the
 // n source values in LDS and streams the indices past them, four entries per thread and step.  (A workgroup per row left a
-// third of the time to the last few rows: 1048 rows on 512 places.)  Bound by writing the output: 8 samples of 20000
-// points, 131 x 131072 entries each, 240 us (549 MB written:
-// 2.3 TB/s); separate gathers, a subtraction, a product and a concatenation took 656.
+// third of the time to the last few rows: 1048 rows on 512 places.)  The next indices are in flight while values are read and
+// stored, and a row's pieces all at once: with each step waiting for its own it was latency that counted.  8 samples of 20000
+// points, 131 x 131072 entries each: 243 -> 118 us, bound by writing the output (549 MB, 4.7 TB/s; 146 us with stores that
+// displace the indices in L2); separate gathers, a subtraction, a product and a concatenation took 656.
 __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
   extern __shared__ float srow[];
   const int T = blockDim.x, tid = threadIdx.x, rows1 = g.cx + g.c;
@@ -580,18 +581,23 @@ __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
       for (int k = tid; k < g.n; k += T) srow[k] = q[k * 3];
     } else {
       const float* q = g.points + ((long)b * g.c + ch - g.cx) * g.n;
-      for (int k = 4 * tid; k + 3 < g.n; k += 4 * T) *(f4*)(srow + k) = ld_f4_any(q + k);
+      constexpr int F = 5;   // pieces in flight
+      for (int k0 = 4 * tid; k0 + 3 < g.n; k0 += 4 * T * F) {
+        f4 v[F];
+#pragma unroll
+        for (int u = 0; u < F; ++u) v[u] = ld_f4_any(q + min(k0 + 4 * T * u, g.n - 4));
+#pragma unroll
+        for (int u = 0; u < F; ++u)
+          if (k0 + 4 * T * u + 3 < g.n) *(f4*)(srow + k0 + 4 * T * u) = v[u];
+      }
       const int k = (g.n & ~3) + tid;
       if (k < g.n) srow[k] = q[k];
     }
     __syncthreads();
     const int* q = g.idx + (long)b * g.ms;
     float* o = g.out + (long)row * g.ms;
-    for (unsigned e = lo + 4 * tid; e < hi; e += 4 * T) {
-      const int cnt = (int)min(hi - e, 4u);
-      I4Any i = {};
-      if (cnt == 4) i = *(const I4Any*)(q + e);
-      else for (int j = 0; j < cnt; ++j) i.v[j] = q[e + j];
+    const unsigned full = lo + ((hi - lo) & ~3u);   // four entries a thread up to here
+    auto values = [&](unsigned e, const I4Any& i) {
       f4 v;
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = srow[index_of(i.v[j], g.n)];
@@ -606,11 +612,29 @@ __global__ __launch_bounds__(1024) void k_group_rows(GroupP g) {
           if (--left == 0 && e + j + 1 < hi) { cq += 3; left = g.nsample; }
         }
       }
-      if (cnt == 4) st_stream(o + e, v);
-      else
+      return v;
+    };
+    // the next step's indices are asked for before this step's values are read
+    constexpr int U = 2;
+    I4Any cur[U], nxt[U];
+    unsigned e = lo + 4 * tid;
+    if (e < full) {
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-          if (j < cnt) o[e + j] = v[j];
+      for (int u = 0; u < U; ++u) cur[u] = *(const I4Any*)(q + min(e + 4 * T * u, full - 4));
+    }
+    for (; e < full; e += 4 * T * U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) nxt[u] = *(const I4Any*)(q + min(e + 4 * T * (U + u), full - 4));
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (e + 4 * T * u < full) st_stream(o + e + 4 * T * u, values(e + 4 * T * u, cur[u]));
+#pragma unroll
+      for (int u = 0; u < U; ++u) cur[u] = nxt[u];
+    }
+    if (full + tid < hi) {
+      I4Any i = {};
+      i.v[0] = q[full + tid];
+      o[full + tid] = values(full + tid, i)[0];
     }
   }
 }
