@@ -88,9 +88,11 @@ __device__ __forceinline__ int lane_of_least(unsigned long long cand, int key) {
 // belongs to wave g % W (neighbouring groups to different waves) as its slot g / W, and lane l of the wave keeps slot l's
 // bounding box, largest running distance and the point that has it.  A draw at o compares o's distance to every box with
 // the group's largest distance -- one instruction sequence for all groups of a wave -- and goes through the points of
-// those groups only that are nearer: about 10 of 313.  One barrier per draw (the waves' bests go through LDS buffers used
-// in turn).  20000 points, 2048 draws, 8 samples: 3.93 ms -> 1.97 ms (0.96 us a
-// draw: a chain of about 100 dependent instructions, two LDS round trips and a barrier).
+// those groups only that are nearer: about 15 of 313.  Few of these lose their farthest point: where that one is as far as
+// before, the group's best is what it was, and a wave none of whose groups has another best hands over the same one again.
+// One barrier per draw (the waves' bests go through LDS buffers used in turn).  20000 points, 2048 draws, 8 samples: 3.93 ms
+// looking at all points, 1.94 looking for the best of every group gone through, 1.55 here (0.57 us a draw of a chain through
+// a reduction over a group, one over a wave's groups, LDS, a barrier and one over the waves, the rest the groups looked at).
 //
 // The pruning is exact: fp32 rounding is monotone, so for a point q of the box each step of the box's squared distance
 // (subtract, square, add, in sqdist's order) is at most the same step for q, and where the box's distance is not below the
@@ -101,7 +103,8 @@ __device__ __forceinline__ int lane_of_least(unsigned long long cand, int key) {
 // a room of 8 m would leave the room a single cell of a grid over everything, its groups in index order and every box the
 // whole room.  The grid therefore covers what most points fill -- the middle half of a sample along each axis and as much again
 // on either side -- and a second, coarser one, sorted behind it, everything.  20000 points, 2048 draws, 8 samples: uniform 1.95
-// ms; with one far point 9.5 -> 1.97, one in twenty far 5.5 -> 1.88, a third far 1.77 -> 1.73 (passing over all points: 3.9).
+// ms; with one far point 9.5 -> 1.97, one in twenty far 5.5 -> 1.88, a third far 1.77 -> 1.73 (passing over all points: 3.9), all
+// before bests were kept: 1.56, 1.67, 1.53 and 1.41 with that.
 constexpr int FPS_CELLS = 4096, FPS_BINS = 5120;   // 16^3 cells and 8^3 behind them, rounded up to a multiple of the threads
 // f(0), f(1), ... f(N - 1) with constant arguments: register arrays indexed inside f stay in registers for every N (the
 // loop unroller left a loop over 20 or 24 slots to dynamic indexing, and the arrays to scratch)
@@ -241,6 +244,8 @@ __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const 
     }
   });
   float ox = p[0], oy = p[1], oz = p[2];
+  bool changed = true;   // (uniform) one of the wave's groups has another best since the wave's best was looked for
+  int mine = 0;          // the slot with the wave's best
   for (int s = 1; s < npoint; ++s) {
     // the slots whose box is nearer than their largest distance (never NaN: fmaxf drops one)
     const float ex = fmaxf(fmaxf(blx - ox, ox - bhx), 0.0f), ey = fmaxf(fmaxf(bly - oy, oy - bhy), 0.0f),
@@ -252,38 +257,43 @@ __global__ __launch_bounds__(64 * W) void k_fps_groups(int n, int npoint, const 
       for_each_slot<4>([&](auto slot) {
         constexpr int j = j4 + decltype(slot)::value;
         if (((mask >> j) & 1u) == 0) return;
+        const unsigned before = (unsigned)__builtin_amdgcn_readlane((int)gd, j);
+        const int at = __builtin_amdgcn_readlane(gpos, j) & 63;
         d[j] = umin(d[j], __builtin_bit_cast(unsigned, sqdist(px[j], py[j], pz[j], ox, oy, oz)) + 1u);
+        if ((__ballot(d[j] == before) >> at) & 1ull) return;   // its best is as far as before, and no other point is farther
         const unsigned m = wave_max<4>(d[j]);
         const unsigned long long cand = __ballot(d[j] == m);
         const int base = (j * W + wave) * 64;
         int l = __builtin_ctzll(cand);
-        if (cand & (cand - 1)) l = lane_of_least(cand, base + lane < n ? (int)order[base + lane] : 0x7fffffff);
+        if (__builtin_expect(__popcll(cand) > 1, 0)) l = lane_of_least(cand, base + lane < n ? (int)order[base + lane] : 0x7fffffff);
         const float x = lane_f(px[j], l), y = lane_f(py[j], l), z = lane_f(pz[j], l);
         if (lane == j) { gd = m; gpos = base + l; gx = x; gy = y; gz = z; }
+        changed = true;
       });
     });
     // the wave's best, then the workgroup's
-    {
+    if (changed) {
       const unsigned m = wave_max<(S > 16 ? 2 : 1)>(gd);
       const unsigned long long cand = __ballot(gd == m);
-      int l = __builtin_ctzll(cand);
-      if (m && (cand & (cand - 1))) l = lane_of_least(cand, (int)order[gpos]);
-      if (lane == l) { best[s & 1][wave] = Best{gd, gx, gy, gz}; best_pos[s & 1][wave] = gpos; }
+      mine = __builtin_ctzll(cand);
+      if (__builtin_expect(__popcll(cand) > 1, 0) && m) mine = lane_of_least(cand, (int)order[gpos]);
+      changed = false;
     }
+    if (lane == mine) { best[s & 1][wave] = Best{gd, gx, gy, gz}; best_pos[s & 1][wave] = gpos; }
     __syncthreads();
     Best w = best[s & 1][lane & (W - 1)];   // repeated through the wave: the first row holds every wave's
     const int wp = best_pos[s & 1][lane & (W - 1)];
     const unsigned m = wave_max<1>(w.d);
-    const unsigned long long cand = __ballot(w.d == m) & ((1ull << W) - 1);
-    int l = __builtin_ctzll(cand);
-    if (m && (cand & (cand - 1))) l = lane_of_least(cand, (int)order[wp]);
-    if (m) {
-      ox = lane_f(w.x, l); oy = lane_f(w.y, l); oz = lane_f(w.z, l);
-      if (tid == l) out[s] = wp;   // a place in `order` for now: its translation would be waited for here
-    } else {  // nothing but padding points: index 0, as the reference
-      ox = p[0]; oy = p[1]; oz = p[2];
-      if (tid == 0) out[s] = -1;
+    const unsigned cand = (unsigned)__ballot(w.d == m) & ((1u << W) - 1);
+    int l = __builtin_ctz(cand);
+    bool none = false;
+    if (__builtin_expect(__popc(cand) > 1, 0)) {   // (all waves, if nothing but padding points is left)
+      none = m == 0;
+      if (!none) l = lane_of_least(cand, (int)order[wp]);
     }
+    ox = lane_f(w.x, l); oy = lane_f(w.y, l); oz = lane_f(w.z, l);
+    if (__builtin_expect(none, 0)) { ox = p[0]; oy = p[1]; oz = p[2]; }   // index 0, as the reference
+    if (tid == l) out[s] = none ? -1 : wp;   // a place in `order` for now: its translation would be waited for here
   }
   __syncthreads();
   for (int s = tid; s < npoint; s += T) out[s] = s && out[s] >= 0 ? (int)order[out[s]] : 0;
@@ -1324,8 +1334,8 @@ static unsigned zero_blocks(long total) { return (unsigned)std::min<long>(blocks
 
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st) {
 #define FPS_GROUPS(W, S) hipLaunchKernelGGL((k_fps_groups<W, S>), dim3(b), dim3(64 * W), 0, st, n, npoint, xyz, idxs)
-  // Eight waves up to 2048 points (fewer meet at the barrier: 0.73 against 0.78 us a draw at 2048), sixteen above (0.82
-  // against 0.83 at 4096, 0.86 against 0.92 at 8192); slots just enough for n, every empty one costs 5 ns a draw.
+  // Eight waves up to 2048 points (fewer meet at the barrier: 0.565 against 0.58 us a draw at 2048), sixteen above (0.590
+  // against 0.593 at 4096, 0.65 against 0.67 at 8192, 0.76 against 0.94 at 20000); slots just enough for n.
   if (n <= 64 * 8 * 4) FPS_GROUPS(8, 4);
   else if (n <= 64 * 16 * 4) FPS_GROUPS(16, 4);
   else if (n <= 64 * 16 * 8) FPS_GROUPS(16, 8);
