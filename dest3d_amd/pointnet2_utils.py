@@ -38,7 +38,7 @@ class FurthestPointSampling(Function):
         x = _f(xyz)
         Bsz, N, _ = x.shape
         with torch.cuda.device(x.device):
-            out = torch.zeros((Bsz, npoint), dtype=torch.int32, device=x.device)
+            out = torch.empty((Bsz, npoint), dtype=torch.int32, device=x.device)   # (written whole)
             temp = torch.empty((Bsz, N), dtype=torch.float32, device=x.device) if N > 24576 else None
             L.check(lib.issm_pn2_furthest_point_sampling(Bsz, N, npoint, x.data_ptr(), None if temp is None else temp.data_ptr(),
                                                          out.data_ptr(), _st(x)), "issm_pn2_furthest_point_sampling")
@@ -232,7 +232,7 @@ class BallQuery(Function):
         Bsz, N, _ = x.shape
         M = q.shape[1]
         with torch.cuda.device(x.device):
-            idx = torch.zeros((Bsz, M, nsample), dtype=torch.int32, device=x.device)
+            idx = torch.empty((Bsz, M, nsample), dtype=torch.int32, device=x.device)   # (written whole)
             L.check(lib.issm_pn2_ball_query(Bsz, N, M, float(radius), nsample, q.data_ptr(), x.data_ptr(), idx.data_ptr(),
                                             _st(x)), "issm_pn2_ball_query")
         ctx.mark_non_differentiable(idx)
