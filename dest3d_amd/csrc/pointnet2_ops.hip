@@ -666,11 +666,13 @@ __device__ __forceinline__ float row_lane_f(float v) {
 // float addition takes 3 cycles a lane however the words lie (measured: 0.77 lanes a nanosecond and CU), one of doubles a
 // fifth of a cycle (6.4), a compare-and-swap of a word just read, if it succeeds, half a cycle.  So up to 5120 points, of
 // which four workgroups still share a CU, the sums are doubles (WIDE); beyond, a lane tries one compare-and-swap and adds the
-// ordinary way where another lane was faster.  Bound by reading grad_out then: 8 samples, 128 channels of 20000 points, 2048
-// balls of 64, 152 us for those 537 MB (3.5 TB/s), whether a ball repeats one point or has 64 different ones (float
-// additions alone: 152 and 677; atomics into a channel-last buffer: 495 and 486).  2048 points, 2048 balls, 64 channels:
-// 65 - 67 us (89 - 332; 252 - 243).  The worst for it, entries that hop between two points
-// (20000 points as above): 1340 us (898; 6000).  With splits > 1 (few rows) the parts meet in grad_points, zero before.
+// ordinary way where another lane was faster.  A row of 2^17 entries is 2^19 bytes, and rows read from their beginnings at one
+// pace ask the same memory channels at any time: every row begins at another step.  Then it is the instructions for the runs
+// that count: 8 samples, 128 channels of 20000 points, 2048 balls of 64, 144 -> 126 us for those 537 MB (4.3 TB/s), whether a
+// ball repeats one point or has 64 different ones (float additions alone: 152 and 677; atomics into a channel-last buffer: 495
+// and 486).  2048 points, 2048 balls, 64 channels, where the next step's loads in flight count: 69 -> 53 us.  The worst for it,
+// entries that hop between two points (20000 points as above): 1260 us (898; 6000).  Eight entries a lane: 159 us, the lanes'
+// pieces of 32 bytes.  With splits > 1 (few rows) the parts meet in grad_points, zero before.
 template <bool WIDE>
 __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdim, int n, int ms, int splits, unsigned per,
                                                           const float* __restrict__ grad_out, const int* __restrict__ idx,
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
   auto add = [&](int k, float v) {
     if constexpr (!WIDE) {
       unsigned* u = (unsigned*)srow + k;
-      const unsigned e = *(volatile unsigned*)u;
+      const unsigned e = __hip_atomic_load(u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (a volatile one is a flat load)
       if (atomicCAS(u, e, __builtin_bit_cast(unsigned, __builtin_bit_cast(float, e) + v)) == e) return;
     }
     unsafeAtomicAdd(srow + k, (Sum)v);
@@ -693,25 +695,7 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
   const int* q = idx + (long)b * ms;
   const float* g = grad_out + ((long)b * cdim + c0 + ch) * ms;
   const unsigned hi = min((part + 1) * per, (unsigned)ms);   // (without a sign, see k_group_rows)
-  for (unsigned e0 = part * per + (tid >> 6) * 256; e0 < hi; e0 += 4 * T) {   // wave-uniform
-    const unsigned e = e0 + 4 * lane;
-    I4Any i;
-    f4 v = {0, 0, 0, 0};
-    if (e + 4 <= hi) {
-      i = *(const I4Any*)(q + e);
-      v = ld_stream(g + e);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) i.v[j] = index_of(i.v[j], n);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        i.v[j] = -1;   // not an entry
-        if (e + j < hi) {
-          i.v[j] = index_of(q[e + j], n);
-          v[j] = g[e + j];
-        }
-      }
-    }
+  auto take = [&](const I4Any& i, f4 v) {
     const bool q1 = i.v[1] == i.v[0], q2 = i.v[2] == i.v[1], q3 = i.v[3] == i.v[2];
     v[1] += q1 ? v[0] : 0.0f;
     v[2] += q2 ? v[1] : 0.0f;
@@ -735,6 +719,39 @@ __global__ __launch_bounds__(1024) void k_group_rows_grad(int c, int c0, int cdi
     if (!q2 && i.v[1] >= 0) add(i.v[1], v[1] + (q1 ? carry : 0.0f));
     if (!q3 && i.v[2] >= 0) add(i.v[2], v[2] + (q1 && q2 ? carry : 0.0f));
     if (end3 && i.v[3] >= 0) add(i.v[3], v[3] + (q1 && q2 && q3 ? carry : 0.0f));
+  };
+  // a wave's steps of 256 entries, the next one's in flight, from another step on for every row; what fills no step at last
+  const unsigned lo = part * per, own = lo + (tid >> 6) * 256;   // wave-uniform
+  const unsigned steps = own + 256 <= hi ? (hi - own - 256) / (4 * T) + 1 : 0;
+  if (steps) {
+    unsigned at = row * 7u % steps;
+    auto entries = [&](unsigned at) { return own + at * (4 * T) + 4 * lane; };
+    I4Any i = *(const I4Any*)(q + entries(at));
+    f4 v = ld_stream(g + entries(at));
+    for (unsigned s = 0; s < steps; ++s) {
+      at = at + 1 < steps ? at + 1 : 0;
+      const I4Any i1 = *(const I4Any*)(q + entries(at));
+      const f4 v1 = ld_stream(g + entries(at));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) i.v[j] = index_of(i.v[j], n);
+      take(i, v);
+      i = i1;
+      v = v1;
+    }
+  }
+  const unsigned e0 = own + steps * (4 * T);
+  if (e0 < hi) {
+    I4Any i;
+    f4 v = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      i.v[j] = -1;   // not an entry
+      if (e0 + 4 * lane + j < hi) {
+        i.v[j] = index_of(q[e0 + 4 * lane + j], n);
+        v[j] = g[e0 + 4 * lane + j];
+      }
+    }
+    take(i, v);
   }
   __syncthreads();
   float* o = grad_points + (long)row * n;
