@@ -499,9 +499,41 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
 // over the tokens, and as one product its (out x in) result makes only a few dozen tiles -- a fraction of the GPU, 54 us for
 // 8192 x 288 -> 586 in bf16.  Here the tokens are cut into slices that run as one batched product and the slices' results are
 // summed (24 us).
+//
+// The forward products of few tokens are issm_linear_fwd's: 4.6 us to issue where the library's take 19, and the kernels are
+// equally long up to about this many multiply-adds (2048 x 288 -> 586: 8.5 us against 7.4; 4096: 12.3 against 9.3, 512 -> 512:
+// 24 against 9; above, and where training keeps the GPU busy, the kernel counts).
+constexpr double FEW_PRODUCTS = 3.5e8;
+bool few_tokens(const Tensor& x, const Tensor& w) {
+  if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
+  if (w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || w.size(1) == 0 || w.size(1) % 32 || x.numel() == 0) return false;
+  return (double)x.numel() * (double)w.size(0) <= FEW_PRODUCTS && x.is_contiguous() && w.is_contiguous() &&
+         (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
+}
+// y = x w^T of one or two such pairs
+template <size_t N>
+std::array<Tensor, N> linear_few(const std::array<std::pair<Tensor, Tensor>, N>& xw) {
+  const c10::DeviceGuard guard(xw[0].first.device());
+  issm_linear_args a{};
+  std::array<Tensor, N> y;
+  for (size_t i = 0; i < N; ++i) {
+    const Tensor &x = xw[i].first, &w = xw[i].second;
+    at::DimVector sizes(x.sizes());
+    sizes.back() = w.size(0);
+    y[i] = fresh(sizes, x, at::kBFloat16);
+    a.job[i] = issm_linear_job{data(x), data(w), data(y[i]), x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0)};
+  }
+  a.njobs = (int32_t)N;
+  a.dtype = ISSM_BF16;
+  a.stream = stream_of(xw[0].first);
+  check(issm_linear_fwd(&a), "issm_linear_fwd");
+  return y;
+}
+
 struct LinearFn : public Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
     ctx->save_for_backward({x, w});
+    if (few_tokens(x, w)) return linear_few<1>({{{x, w}}})[0];
     return at::linear(x, w);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {

@@ -43,6 +43,7 @@ struct TrP {
 };
 int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
+int launch_linear(LinearP& p, int njobs, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
                       hipStream_t st);
@@ -765,6 +766,27 @@ int issm_layer_params(const issm_layer_params_args* a) {
   if (total == 0) return ISSM_OK;
   if (!a->out || !a->A) return fail(ISSM_E_NULL, "layer_params: out/A is NULL");
   return launched(launch_layer_params(p, (hipStream_t)a->stream), "layer_params");
+}
+
+int issm_linear_fwd(const issm_linear_args* a) {
+  if (!a) return fail(ISSM_E_NULL, "linear: args is NULL");
+  if (a->njobs < 0 || a->njobs > ISSM_LINEAR_JOBS) return fail(ISSM_E_SHAPE, "linear: %d products (0..%d)", a->njobs, ISSM_LINEAR_JOBS);
+  if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "linear: dtype %d (bf16 only)", a->dtype);
+  LinearP p{};
+  int n = 0;
+  for (int i = 0; i < a->njobs; ++i) {
+    const issm_linear_job& j = a->job[i];
+    if (j.tokens < 0 || j.in < 0 || j.out < 0 || j.tokens > 0x7fffffff - 64 || j.out > 0x7fffffff - 64)
+      return fail(ISSM_E_SHAPE, "linear: (%lld, %d) -> %d", (long long)j.tokens, j.in, j.out);
+    if (j.in == 0 || j.in % 32) return fail(ISSM_E_UNSUPPORTED, "linear: %d features (a multiple of 32)", j.in);
+    if (j.tokens == 0 || j.out == 0) continue;
+    if (!j.x || !j.w || !j.y) return fail(ISSM_E_NULL, "linear: x/w/y is NULL");
+    if (((uintptr_t)j.x | (uintptr_t)j.w) & 15) return fail(ISSM_E_STRIDE, "linear: x and w must be aligned to 16 bytes");
+    if ((uintptr_t)j.y & 1) return fail(ISSM_E_STRIDE, "linear: y must be aligned to its elements");
+    p.job[n++] = LinearJob{(const uint16_t*)j.x, (const uint16_t*)j.w, (uint16_t*)j.y, (int)j.tokens, j.out, j.in / 32, 0};
+  }
+  if (n == 0) return ISSM_OK;
+  return launched(launch_linear(p, n, (hipStream_t)a->stream), "linear_fwd");
 }
 
 int issm_transpose_states(const issm_transpose_args* a) {

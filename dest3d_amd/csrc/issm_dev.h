@@ -171,6 +171,15 @@ struct DwConvP {
 // parameters of the dt / B / C generation kernels (param_gen.hip)
 // parameters of the layer-parameter kernel (layer_params.hip)
 constexpr int LAYER_ARRAYS = 9;
+struct LinearJob {
+  const uint16_t *x, *w;
+  uint16_t* y;
+  int tokens, out, steps, oblocks;   // steps of 32 along the contraction
+};
+struct LinearP {
+  LinearJob job[2];
+  int blocks0;   // of the first
+};
 struct LayerParamsP {
   const void* src[LAYER_ARRAYS];
   int n[LAYER_ARRAYS], bf16[LAYER_ARRAYS];

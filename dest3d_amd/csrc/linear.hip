@@ -1,0 +1,77 @@
+// y = x W^T of a decoder layer's projections where a scene or two of tokens meet a few hundred features (gfx950), bf16 operands,
+// fp32 accumulation: x (tokens, in), W (out, in), y (tokens, out).  Up to two such products share a launch.
+//
+// At these sizes a product is a few microseconds whoever computes it, and what counts is what it costs to launch: a library
+// product takes 19 us of host time to issue, 4.6 here; a decoder layer has four, and six layers on one scene (1024 tokens, 256
+// queries) ran at the pace of the host: 1240 -> 858 us.  Both operands have the contraction index contiguous, which is the operand layout of
+// v_mfma_f32_16x16x32_bf16 as it lies in memory: a wave asks for all fragments of its 16 tokens and 32 outputs at once (27 loads
+// of 16 bytes a lane at 288 features) and multiplies as they arrive; there is nothing to share through LDS that L1 does not
+// share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens or features the fragments' 64-byte pieces
+// of 16 rows a load are what it pays for, and staging tiles through LDS wins: 8192 x 288 -> 586 21 us (13.5).
+#include "issm_dev.h"
+
+namespace issm {
+
+struct __attribute__((packed, aligned(2))) LinearOut {   // four outputs; rows of an odd number of them promise no alignment
+  bf4 v;
+};
+
+// N: fragments in flight
+template <int N>
+__global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
+  const bool second = (int)blockIdx.x >= p.blocks0;
+  const LinearJob& j = p.job[second ? 1 : 0];
+  const int bid = (int)blockIdx.x - (second ? p.blocks0 : 0), lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const int t = (bid / j.oblocks) * 64 + (threadIdx.x >> 6) * 16 + i, o0 = (bid % j.oblocks) * 32;
+  const long in = 32L * j.steps;
+  const bf8* x = (const bf8*)(j.x + (long)min(t, j.tokens - 1) * in) + g;
+  const bf8 *wa = (const bf8*)(j.w + (long)min(o0 + i, j.out - 1) * in) + g,
+            *wb = (const bf8*)(j.w + (long)min(o0 + 16 + i, j.out - 1) * in) + g;
+  f4 ya = {0, 0, 0, 0}, yb = {0, 0, 0, 0};
+  for (int s0 = 0; s0 < j.steps; s0 += N) {
+    bf8 fx[N], fa[N], fb[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int s = 4 * min(s0 + u, j.steps - 1);
+      fx[u] = x[s];
+      fa[u] = wa[s];
+      fb[u] = wb[s];
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (s0 + u < j.steps) {   // uniform
+        ya = mfma_bf(fa[u], fx[u], ya);
+        yb = mfma_bf(fb[u], fx[u], yb);
+      }
+  }
+  if (t >= j.tokens) return;
+  uint16_t* y = j.y + (long)t * j.out;
+  auto put = [&](int o, f4 v) {
+    if (o + 4 <= j.out) {
+      ((LinearOut*)(y + o))->v = __builtin_convertvector(v, bf4);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+        if (o + r < j.out) y[o + r] = f_to_bf16(v[r]);
+    }
+  };
+  put(o0 + 4 * g, ya);
+  put(o0 + 16 + 4 * g, yb);
+}
+
+int launch_linear(LinearP& p, int njobs, hipStream_t st) {
+  long blocks[2] = {0, 0};
+  for (int k = 0; k < njobs; ++k) {
+    p.job[k].oblocks = (p.job[k].out + 31) / 32;
+    blocks[k] = (long)((p.job[k].tokens + 63) / 64) * p.job[k].oblocks;
+  }
+  if (blocks[0] + blocks[1] > 0x7fffffff) return (int)hipErrorInvalidValue;
+  p.blocks0 = (int)blocks[0];
+  const dim3 grid((unsigned)(blocks[0] + blocks[1])), block(NTHREADS);
+  // nine fragments where they come out even (288 features), eight otherwise
+  if (p.job[0].steps % 9 == 0) hipLaunchKernelGGL(k_linear<9>, grid, block, 0, st, p);
+  else hipLaunchKernelGGL(k_linear<8>, grid, block, 0, st, p);
+  return (int)hipGetLastError();
+}
+
+}  // namespace issm

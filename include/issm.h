@@ -407,6 +407,27 @@ int issm_dwconv_partial_rows(int32_t batch, int32_t seqlen);
 int issm_dwconv_silu_fwd(const issm_dwconv_args* args);
 int issm_dwconv_silu_bwd(const issm_dwconv_args* args);
 
+/* ---- projections of a scene or two of tokens -------------------------------------------------
+ * y = x w^T (the layer's nn.Linear without bias, models/dest_module.py:471-503) for one or two independent products in one
+ * launch: x (tokens, in), w (out, in), y (tokens, out), contiguous, dtype ISSM_BF16, sums in fp32.  in a multiple of 32
+ * (ISSM_E_UNSUPPORTED otherwise), x and w aligned to 16 bytes (ISSM_E_STRIDE). */
+#define ISSM_LINEAR_JOBS 2
+typedef struct issm_linear_job {
+  const void* x;
+  const void* w;
+  void* y;
+  int64_t tokens;
+  int32_t in, out;
+} issm_linear_job;
+typedef struct issm_linear_args {
+  issm_linear_job job[ISSM_LINEAR_JOBS];
+  int32_t njobs;
+  int32_t dtype;
+  void* stream;
+} issm_linear_args;
+
+int issm_linear_fwd(const issm_linear_args* args);
+
 /* ---- queries <-> scan states -----------------------------------------------------------------
  * The rearrangements around the scan in MultiHeadISSMScan.forward: queries become initial states
  * ("b l (h hd) -> b h hd l", models/dest_module.py:537-538) and the two directions' final states become the query
