@@ -1,5 +1,6 @@
 // C ABI of libissm_hip.so: argument validation, workspace carving and stage sequencing.
 // All device work lives in issm_fwd.hip / issm_bwd.hip / rmsnorm_gated.hip.
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -21,7 +22,8 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
 int launch_state_bwd(const KP& p, const float* states, const float* cs_last, float* dstates, float* g_last,
                      float* dh0_dir, hipStream_t st);
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, hipStream_t st);
+                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st);
+int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st);
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
                           const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
                           hipStream_t st);
@@ -120,6 +122,21 @@ static FwdWs fwd_layout(const issm_dims& d, bool has_z) {
   return w;
 }
 
+// How many workgroups of the chunk backward share the heads of a (chunk, group, 64 state columns): as many as fit the 512 places
+// of the chip (two workgroups a CU).  A part's sums of dB and dC are 32 KB, which one more launch adds up: 4 us, and as much
+// of host time, against 8 us a head and direction; worth it from four of those on (of 4 heads of 2 x 160 tokens, where the host
+// sets the pace, it is not).  Where one workgroup each fills the chip, halves only cost that, also where a last round would
+// be nearly empty (its workgroups have the CUs to themselves): 9 x 1024 tokens, 8 heads x 32, 256 states, bf16, 576 workgroups,
+// a training step 278 us, in halves 281; 320 workgroups, two directions, fp32: 376 and 389.  128 workgroups, 2 x 1024 tokens of
+// 8 heads x 36, two directions, bf16: 215 us with one part, 186, 176 and 191 with 2, 4 and 8; 64, 1 x 1024 tokens, fp32: 209
+// and 171, 152, 152.
+static int bwd_head_parts(const issm_dims& d) {
+  const long blocks = (long)d.batch * nchunks(d) * d.ngroups * ((d.dstate + ISSM_CHUNK - 1) / ISSM_CHUNK);
+  const long heads = d.nheads / d.ngroups, most = std::max<long>(1, std::min<long>(heads, 512 / blocks));
+  const long each = (heads + most - 1) / most;
+  return (heads - each) * d.ndir < 4 ? 1 : (int)((heads + each - 1) / each);   // (no part without a head)
+}
+
 static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
 // Partial sums that would be rounded to bf16 on their way between kernels: with two directions and a bf16 ddt the first
 // direction's share of ddt in fp32 ((B, L, H, N)), with bf16 inputs and incomplete tiles dB and dC of workgroups two
@@ -140,7 +157,9 @@ static BwdWs bwd_layout(const issm_scan_args* a) {
   w.redo = o; o += align64(Bt * nc * H * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK));  // one int per direction, workgroup and head
   w.dy_ws = o; if (has_z) o += align64(Bt * d.seqlen * H * P);
   w.dbc_part = o;
-  if (a->io_dtype == ISSM_BF16 && (N % 64 || d.seqlen % ISSM_CHUNK)) o += Bt * nc * d.ngroups * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK) * 2 * ISSM_CHUNK * ISSM_CHUNK;
+  const int parts = bwd_head_parts(d);
+  if (parts > 1) o += Bt * nc * d.ngroups * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK) * parts * 2 * ISSM_CHUNK * ISSM_CHUNK;
+  else if (a->io_dtype == ISSM_BF16 && (N % 64 || d.seqlen % ISSM_CHUNK)) o += Bt * nc * d.ngroups * ((N + ISSM_CHUNK - 1) / ISSM_CHUNK) * 2 * ISSM_CHUNK * ISSM_CHUNK;
   w.ddt_part = o; if (ddt_part) o += align64((size_t)d.batch * d.seqlen * H * N);
   w.total = o;
   return w;
@@ -372,7 +391,7 @@ int issm_stage_bwd_chunk(const issm_scan_args* a, int dir, const float* dy_gated
   KP p = make_kp(a);
   p.dir0 = dir;
   int pending = 0;
-  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, g_last, part_a, part_bias, redo, &pending,
+  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, g_last, part_a, part_bias, redo, &pending, 1,
                                       (hipStream_t)a->stream),
                      "bwd_chunk")))
     return rc;
@@ -441,15 +460,20 @@ int issm_scan_bwd(const issm_scan_args* a) {
     pc.ddt_part.s1 = (long)p.H * p.N;
     pc.ddt_part.s0 = (long)p.L * p.H * p.N;
   }
-  if (p.io_dt && !p.full_tiles && bwd_tile_available(p, dy)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
+  int parts = 1;
+  if (bwd_tile_available(p, dy)) {
+    parts = bwd_head_parts(a->dims);
+    if (parts > 1 || (p.io_dt && !p.full_tiles)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
+  }
   for (int dir = 0; dir < p.ndir; ++dir) {
     KP pd = pc;
     pd.dir0 = dir;
     if ((rc = launched(launch_bwd_chunk(pd, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last,
-                                        ws + bw.partA, ws + bw.partBias, redo, &pending, st),
+                                        ws + bw.partA, ws + bw.partBias, redo, &pending, parts, st),
                        "bwd_chunk")))
       return rc;
   }
+  if (parts > 1 && (rc = launched(launch_bwd_parts_sum(p, redo, parts, st), "bwd_chunk (parts)"))) return rc;
   const int together = p.L % ISSM_CHUNK == 0 ? p.ndir : 1;   // directions per launch of the pass over the marks
   for (int dir = 0; pending && dir < p.ndir; dir += together) {
     KP pd = p;

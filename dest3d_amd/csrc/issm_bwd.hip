@@ -1751,6 +1751,60 @@ __global__ __launch_bounds__(NTHREADS) void k_bwd_reduce(ReduceJobs j) {
   }
 }
 
+// dB and dC where `parts` workgroups of the tile-base kernel share the heads of a (chunk, group, 64 state columns).  Workgroup
+// = that place and direction and a quarter of the rows: a lane's rows k = 4 q .. 4 q + 3 of dB and of dC.  Where the pass over
+// the marks goes on from the sums of the heads before (bf16 inputs, incomplete tiles), they become the first part's.
+template <bool IOB>
+__global__ __launch_bounds__(NTHREADS) void k_bwd_parts_sum(KP p, const int* __restrict__ redo, int parts) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cm = lane & 15, g4 = lane >> 4;
+  const int nsl = (p.N + NS - 1) / NS, wg = blockIdx.x, q = blockIdx.y;
+  Unit u;
+  u.dir = blockIdx.z;
+  int id = wg;
+  const int ns = id % nsl;
+  id /= nsl;
+  u.g = id % p.G;
+  id /= p.G;
+  u.c = p.c_lo + id % p.ncl;
+  u.b = id / p.ncl;
+  u.bt = u.b * p.ndir + u.dir;
+  u.h = u.g * p.hpg;
+  const long at = (long)u.dir * gridDim.x + wg;
+  int any = 0;
+  for (int hh = 0; hh < p.hpg; ++hh) any |= redo[at * p.hpg + hh];
+  const long stride = (long)p.ndir * gridDim.x * (32 * NTHREADS);
+  float* part = p.dbc_part + at * (32 * NTHREADS) + 4 * q * NTHREADS + tid;
+  float vb[4] = {0, 0, 0, 0}, vc[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int i = 0; i < parts; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      vb[j] += part[i * stride + j * NTHREADS];
+      vc[j] += part[i * stride + (16 + j) * NTHREADS];
+    }
+  if (IOB && !p.full_tiles && any) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      part[j * NTHREADS] = vb[j];
+      part[(16 + j) * NTHREADS] = vc[j];
+    }
+    return;
+  }
+  const int n = ns * NS + wave * 16 + cm;
+  if (n >= p.N) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int l = 16 * q + 4 * g4 + j, t = u.c * CS + l;
+    if (t >= p.L) break;
+    const long row = u.dir ? p.L - 1 - t : t;
+    auto put = [&](const TensorD& d, float v) {
+      if (d.ptr) stv((void*)d.ptr, (long)u.b * d.s0 + row * d.s1 + (long)u.g * d.s2 + n, IOB ? 1 : 0, v);
+    };
+    put(p.dB[u.dir], vb[j]);
+    put(p.dC[u.dir], vc[j]);
+  }
+}
+
 // -------------------------------------------------------------------- launchers
 template <typename K>
 static int set_lds(K kernel, size_t bytes) {
@@ -1828,19 +1882,20 @@ static int launch_bwd_chunk_t(const KP& p, int blocks, const float* dy_ws, const
 
 bool bwd_tile_available(const KP& p, const float* dy_ws);
 int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm, const float* g_last,
-                    float* partA, float* partBias, int* redo, hipStream_t st);
+                    float* partA, float* partBias, int* redo, int parts, hipStream_t st);
 
 // Chunk backward of direction p.dir0.  With a `redo` buffer (issm_bwd_chunk_redo_ints words) the tile-base kernel
 // (issm_bwd_tile.hip) does the work and marks the heads outside its range; launch_bwd_chunk_redo then evaluates those
 // with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (bwd_tile_available:
 // packed sequences, a gate beside bf16 inputs, mixed input types, fp32 heads of more than 48, heads or rows of x and dout
 // that are no multiple of four elements), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
+// parts: workgroups of the tile-base kernel that share a group's heads (1 without p.dbc_part).
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, hipStream_t st) {
+                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   if (redo && bwd_tile_available(p, dy_ws)) {
     if (redo_pending) *redo_pending = 1;
-    return launch_bwd_tile(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, st);
+    return launch_bwd_tile(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
   }
   ISSM_DISPATCH(p, {
     if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
@@ -1862,6 +1917,13 @@ int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const floa
                                                                   partBias, redo, ndirs, st))
       return e;
   });
+  return (int)hipGetLastError();
+}
+
+int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st) {
+  const dim3 g(p.B * p.nc * p.G * ((p.N + NS - 1) / NS), 4, p.ndir), t(NTHREADS);
+  if (p.io_dt) hipLaunchKernelGGL(k_bwd_parts_sum<true>, g, t, 0, st, p, redo, parts);
+  else hipLaunchKernelGGL(k_bwd_parts_sum<false>, g, t, 0, st, p, redo, parts);
   return (int)hipGetLastError();
 }
 

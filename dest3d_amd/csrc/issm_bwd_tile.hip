@@ -71,13 +71,15 @@ __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflev
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
-// FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).
-template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL>
+// FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).  PARTS: gridDim.y workgroups
+// share the group's heads, heads_each each (a variant of its own: the two loop bounds more cost the others 25 - 50 scalar
+// registers spilled and 1 - 2 % of a training step).
+template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
 __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
                                                           const float* __restrict__ dstates,
                                                           const float* __restrict__ dm,
                                                           const float* __restrict__ g_last, float* __restrict__ partA,
-                                                          float* __restrict__ partBias, int* __restrict__ redo) {
+                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
   constexpr bool SPLIT = !IOB;
   constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && !FULL;  // fp32 products in the diagonal blocks / in all blocks
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -189,9 +191,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, l_Cv);
     }
   };
-  request(head_of(0));
+  const int hh0 = PARTS ? (int)blockIdx.y * heads_each : 0;
+  request(head_of(hh0));
 
-  for (int hh = 0; hh < p.hpg; ++hh) {
+  for (int hh = hh0; hh < (PARTS ? min(p.hpg, hh0 + heads_each) : p.hpg); ++hh) {
     u.h = head_of(hh);
     __syncthreads();  // the previous head no longer reads the tiles
     {
@@ -550,7 +553,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       if constexpr (P32) lane_load_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, old);
       else lane_load_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, old);
     }
-    request(head_of(min(hh + 1, p.hpg - 1)));  // (unconditional: the last head is requested again and not used)
+    request(head_of(min(hh + 1, (PARTS ? min(p.hpg, hh0 + heads_each) : p.hpg) - 1)));  // (unconditional: the last head is requested again and not used)
     __builtin_amdgcn_sched_barrier(0);
     if (skip) {
       // the level-hierarchy kernel adds this head's share to ddt later: it must find the other direction's, or zero
@@ -627,8 +630,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     }
   }
 
-  if (DIAG32 && p.dbc_part && s.shared[wave]) {  // (the wave's own word)
-    float* q = p.dbc_part + ((long)p.dir0 * gridDim.x + wg) * (32 * NTHREADS) + tid;
+  if (PARTS || (DIAG32 && p.dbc_part && s.shared[wave])) {  // (the wave's own word)
+    const long at = (long)p.dir0 * gridDim.x + wg;
+    float* q = p.dbc_part + (PARTS ? (long)blockIdx.y * p.ndir * gridDim.x + at : at) * (32 * NTHREADS) + tid;
 #pragma unroll
     for (int k = 0; k < 32; ++k) q[k * NTHREADS] = s.dbc[k * NTHREADS + tid];
   } else {
@@ -661,7 +665,7 @@ bool bwd_tile_available(const KP& p, const float* dy_ws) {
 
 template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
-                             const float* g_last, float* partA, float* partBias, int* redo, hipStream_t st) {
+                             const float* g_last, float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
   const size_t sm = sizeof(BwdTileSmem<PT, !IOB>);
   const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0;
   auto go = [&](auto kern) -> int {
@@ -669,14 +673,19 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
       if (int e = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm))
         return e;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), sm, st, p, states, dstates, dm, g_last, partA, partBias, redo);
+    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(NTHREADS), sm, st, p, states, dstates, dm, g_last, partA, partBias, redo,
+                       (p.hpg + parts - 1) / parts);
     return 0;
   };
   auto pick = [&](auto p32) -> int {
     constexpr bool P32 = decltype(p32)::value;
-    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false>);
-    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true>);
-    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true>);
+    if (parts > 1) {
+      if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, true>);
+      return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, true>);
+    }
+    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, false>);
+    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true, false>);
+    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, false>);
   };
   if constexpr (IOB)
     if (p.ddt_part.ptr) return pick(std::true_type{});
@@ -684,7 +693,7 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
 }
 
 int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                    const float* g_last, float* partA, float* partBias, int* redo, hipStream_t st) {
+                    const float* g_last, float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
   KP p = p_;
   if (dy_ws) {  // a gated dy: fp32 (Bt, L, H, P) contiguous, batch * direction outermost
     TensorD& t = p.dout[p.dir0];
@@ -698,12 +707,12 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
   const int pt = (p.P + 15) / 16;
   int e = 0;
   if (p.io_dt) {
-    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, st);
-    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
   } else {
-    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, st);
-    else e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    else e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
   }
   if (e) return e;
   return (int)hipGetLastError();

@@ -62,6 +62,8 @@ struct KP {
   // workgroups with heads it left to the level form (which goes on from them, so that dB and dC are rounded once, as where
   // the level form evaluates all heads): per direction and workgroup the lanes' 16 + 16 values [32][NTHREADS].  Null: they
   // travel through dB and dC themselves.  (Complete tiles do that: six decoder layers, a training step, 7.38 against 7.52 ms.)
+  // Where several workgroups of the tile-base kernel share the heads of a group (bwd_head_parts), the sums of all workgroups in
+  // all cases, one such array per part, which k_bwd_parts_sum adds up.
   float* dbc_part;
   const float* A;
   const float* D;

@@ -628,6 +628,51 @@ def test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel(dtyp
             "head 3 is out of range only in the chunk that holds tokens 70..109"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,H,ndir", [(128, 128, 6, 1), (100, 70, 5, 2), (256, 64, 3, 2), (1600, 256, 7, 1), (130, 8, 5, 1)])
+@pytest.mark.parametrize("marked", [False, True])
+def test_heads_shared_by_several_workgroups(dtype, L_, N, H, ndir, marked):
+    """Few chunks and states: several workgroups of the chunk backward share the heads of a group (7 heads at 1600 tokens and
+    256 states: parts of 2, 2, 2 and 1), some heads with decays that the level-hierarchy kernel adds afterwards.  Against calls
+    of one head each: a head's own gradients bit for bit, those of B and C to the rounding of the sum (and, bf16, of the single
+    heads' results)."""
+    from dest3d_amd import ISSM_biscan_combined, ISSM_chunk_scan_combined
+    _say(f"shared heads L={L_} N={N} H={H} ndir={ndir} {dtype} marked={marked}")
+    d = _problem(2 if L_ < 1000 else 1, L_, H, 24, N, 1, seed=L_ + H, softplus=False)
+    d["dt"] = d["dt"].abs()
+    if marked:
+        d["A"][1] = -80.0 * (1.0 + torch.rand(N, generator=torch.Generator().manual_seed(1)))
+        d["A"][H - 1] = d["A"][1]
+    io = ("x", "dt", "B", "C")
+    q = {k: d[k].cuda().to(dtype if k in io else torch.float32) for k in ("x", "dt", "B", "C", "A", "D", "h0")}
+    dy, dl = d["dy"].cuda(), d["dfinal"].cuda()
+
+    def run(heads):
+        v = {k: (t if k in ("B", "C") else t[heads] if k in ("A", "D") else t[:, heads] if k == "h0" else t[:, :, heads]).contiguous()
+             .clone().requires_grad_() for k, t in q.items()}
+        if ndir == 2:
+            x2 = v["x"].detach().flip(1).requires_grad_()
+            v["B_b"], v["C_b"] = ((2 * v[k]).detach().requires_grad_() for k in ("B", "C"))
+            o = ISSM_biscan_combined(v["x"], x2, v["dt"], v["A"], v["B"], v["B_b"], v["C"], v["C_b"], 64, D=v["D"],
+                                     initial_states=v["h0"])
+        else:
+            o = ISSM_chunk_scan_combined(v["x"], v["dt"], v["A"], v["B"], v["C"], 64, D=v["D"], initial_states=v["h0"],
+                                         return_final_states=True)
+        loss = sum((y.float() * dy[:, :, heads]).sum() for y in o[:ndir]) + sum((f * dl[:, heads]).sum() for f in o[ndir:])
+        loss.backward()
+        return {k: t.grad for k, t in v.items()}
+
+    got, each = run(slice(0, H)), [run(slice(h, h + 1)) for h in range(H)]
+    for k in ("x", "dt", "A", "D", "h0"):
+        want = torch.cat([e[k] for e in each], dim=0 if k in ("A", "D") else 1 if k == "h0" else 2)
+        assert torch.equal(got[k], want), k
+    for k in ("B", "C") + (("B_b", "C_b") if ndir == 2 else ()):
+        terms = torch.stack([e[k].double() for e in each])
+        eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24   # of a result's rounding; the marked heads are added to one
+        err = (got[k].double() - terms.sum(0)).abs()
+        assert (err <= (3 + H * 2.0 ** -24 / eps) * eps * terms.abs().sum(0)).all(), k
+
+
 @pytest.mark.parametrize("L_", [64, 60], ids=["complete tile", "ragged"])
 @pytest.mark.parametrize("bits", [0x7fc00000, 0x7fffffff, -1, 0x7f800000], ids=["nan", "nan of all bits", "-nan of all bits", "inf"])
 def test_an_operand_that_is_no_number_reaches_the_gradients(bits, L_):
