@@ -1807,8 +1807,8 @@ __global__ __launch_bounds__(NTHREADS) void k_bwd_parts_sum(KP p, const int* __r
 
 // -------------------------------------------------------------------- launchers
 template <typename K>
-static int set_lds(K kernel, size_t bytes) {
-  return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+static int set_lds(K kernel, size_t bytes) {   // (up to 64 KB needs no asking)
+  return bytes > 64 * 1024 ? (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) : 0;
 }
 
 int launch_bwd_gate(const KP& p, const float* out_x, float* dy_ws, hipStream_t st) {

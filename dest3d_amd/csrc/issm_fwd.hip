@@ -386,8 +386,8 @@ __global__ __launch_bounds__(NTHREADS, (PT <= 2 && (!IOB || !FULL)) ? 4 : 1) voi
 
 // ------------------------------------------------------------------- launchers
 template <typename K>
-static int set_lds(K kernel, size_t bytes) {
-  return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+static int set_lds(K kernel, size_t bytes) {   // (up to 64 KB needs no asking)
+  return bytes > 64 * 1024 ? (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) : 0;
 }
 
 bool local_tile_available(const KP& p, const float* states, const float* cabt);

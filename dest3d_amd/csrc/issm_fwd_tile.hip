@@ -423,8 +423,8 @@ bool local_tile_available(const KP& p, const float* states, const float* cabt) {
 }
 
 template <typename K>
-static int set_lds_tile(K kernel, size_t bytes) {
-  return (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+static int set_lds_tile(K kernel, size_t bytes) {   // (up to 64 KB needs no asking)
+  return bytes > 64 * 1024 ? (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) : 0;
 }
 
 int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
