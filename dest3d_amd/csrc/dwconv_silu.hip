@@ -20,7 +20,11 @@
 namespace issm {
 
 constexpr int DW_TAPS = 7;
-constexpr int DW_TL = 16;     // tokens per thread
+// Tokens per thread, DW_TL.  Backward: 16, but 8 for the chained one, which holds 61 values of its rows and halo per 8 tokens and
+// at 16 needed 272 registers, one wave a SIMD: 8 x 1024 tokens, 290 channels, bf16: 39 us with 16, 25 with 8, 32 with 4 (more
+// halo read twice).  Forward: the most of 16, 8 and 4 that makes two waves a SIMD: one scene of 1024 tokens makes 290 waves of 16
+// (9.4, 7.7 and 5.5 us with 16, 8 and 4), 16 x 4096 tokens pay for the halo (73 us chained with 16, 102 with 4).
+constexpr int DW_BWD = 16, DW_CHAIN_BWD = 8;
 
 template <bool BF>
 __device__ __forceinline__ float dw_ld(const void* p, long i) {
@@ -32,6 +36,7 @@ __device__ __forceinline__ void dw_st(void* p, long i, float v) {
 }
 
 // thread -> (b, tile, c), c fastest
+template <int DW_TL>
 __device__ __forceinline__ bool dw_item(const DwConvP& p, int& b, int& l0, int& c) {
   const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
   const int ntile = (p.L + DW_TL - 1) / DW_TL;
@@ -43,10 +48,10 @@ __device__ __forceinline__ bool dw_item(const DwConvP& p, int& b, int& l0, int& 
   return true;
 }
 
-template <bool BF, int S>
+template <bool BF, int S, int DW_TL>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_fwd(DwConvP p) {
   int b, l0, c;
-  if (!dw_item(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, b, l0, c)) return;
   float w[S][DW_TAPS], bias[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
@@ -91,8 +96,9 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_fwd(DwConvP p) {
 // partial layout: [(b * ntile + tile)][s][j (0..6: taps, 7: bias)][c]
 template <bool BF, int S>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_bwd(DwConvP p) {
+  constexpr int DW_TL = DW_BWD;
   int b, l0, c;
-  if (!dw_item(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, b, l0, c)) return;
   float w[S][DW_TAPS];
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -181,10 +187,10 @@ __device__ __forceinline__ long dw_out_off(const DwConvP& p, long row, int c, bo
   return head ? row * p.split + c : row * (p.C - p.split) + (c - p.split);
 }
 
-template <bool BF>
+template <bool BF, int DW_TL>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd(DwConvP p) {
   int b, l0, c;
-  if (!dw_item(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, b, l0, c)) return;
   float w[2][DW_TAPS], bias[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -235,8 +241,9 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd(DwConvP p) {
 
 template <bool BF>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_bwd(DwConvP p) {
+  constexpr int DW_TL = DW_CHAIN_BWD;
   int b, l0, c;
-  if (!dw_item(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, b, l0, c)) return;
   float w[2][DW_TAPS];
 #pragma unroll
   for (int s = 0; s < 2; ++s)
@@ -357,30 +364,39 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_dw(DwConvP p) {
   }
 }
 
-int dwconv_partial_rows(int B, int L) { return B * ((L + DW_TL - 1) / DW_TL); }
+// (the most that either backward writes)
+int dwconv_partial_rows(int B, int L) { return B * ((L + DW_CHAIN_BWD - 1) / DW_CHAIN_BWD); }
 
-static unsigned dw_blocks(const DwConvP& p) {
-  const long items = (long)p.B * ((p.L + DW_TL - 1) / DW_TL) * p.C;
-  return (unsigned)((items + NTHREADS - 1) / NTHREADS);
-}
+static long dw_items(const DwConvP& p, int tokens) { return (long)p.B * ((p.L + tokens - 1) / tokens) * p.C; }
+static unsigned dw_blocks(const DwConvP& p, int tokens) { return (unsigned)((dw_items(p, tokens) + NTHREADS - 1) / NTHREADS); }
 
-int launch_dwconv_fwd(const DwConvP& p, hipStream_t st) {
-  const dim3 g(dw_blocks(p)), b(NTHREADS);
+template <int TL>
+static int launch_dwconv_fwd_t(const DwConvP& p, hipStream_t st) {
+  const dim3 g(dw_blocks(p, TL)), b(NTHREADS);
   if (p.chain) {
-    if (p.dtype) hipLaunchKernelGGL(k_dwconv_chain_fwd<true>, g, b, 0, st, p);
-    else hipLaunchKernelGGL(k_dwconv_chain_fwd<false>, g, b, 0, st, p);
+    if (p.dtype) hipLaunchKernelGGL((k_dwconv_chain_fwd<true, TL>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((k_dwconv_chain_fwd<false, TL>), g, b, 0, st, p);
   } else if (p.dtype) {
-    if (p.nsets == 1) hipLaunchKernelGGL((k_dwconv_fwd<true, 1>), g, b, 0, st, p);
-    else hipLaunchKernelGGL((k_dwconv_fwd<true, 2>), g, b, 0, st, p);
+    if (p.nsets == 1) hipLaunchKernelGGL((k_dwconv_fwd<true, 1, TL>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((k_dwconv_fwd<true, 2, TL>), g, b, 0, st, p);
   } else {
-    if (p.nsets == 1) hipLaunchKernelGGL((k_dwconv_fwd<false, 1>), g, b, 0, st, p);
-    else hipLaunchKernelGGL((k_dwconv_fwd<false, 2>), g, b, 0, st, p);
+    if (p.nsets == 1) hipLaunchKernelGGL((k_dwconv_fwd<false, 1, TL>), g, b, 0, st, p);
+    else hipLaunchKernelGGL((k_dwconv_fwd<false, 2, TL>), g, b, 0, st, p);
   }
   return (int)hipGetLastError();
 }
+int launch_dwconv_fwd(const DwConvP& p, hipStream_t st) {
+  constexpr long waves = 2048 * 64;   // lanes of two waves a SIMD
+  if (dw_items(p, 16) >= waves) return launch_dwconv_fwd_t<16>(p, st);
+  if (dw_items(p, 8) >= waves) return launch_dwconv_fwd_t<8>(p, st);
+  return launch_dwconv_fwd_t<4>(p, st);
+}
 
-int launch_dwconv_bwd(const DwConvP& p, hipStream_t st) {
-  const dim3 g(dw_blocks(p)), b(NTHREADS);
+int launch_dwconv_bwd(const DwConvP& p_, hipStream_t st) {
+  DwConvP p = p_;
+  const int tokens = p.chain ? DW_CHAIN_BWD : DW_BWD;
+  p.nrows = p.B * ((p.L + tokens - 1) / tokens);
+  const dim3 g(dw_blocks(p, tokens)), b(NTHREADS);
   if (p.chain) {
     if (p.dtype) hipLaunchKernelGGL(k_dwconv_chain_bwd<true>, g, b, 0, st, p);
     else hipLaunchKernelGGL(k_dwconv_chain_bwd<false>, g, b, 0, st, p);

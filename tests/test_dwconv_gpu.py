@@ -26,6 +26,8 @@ CASES = [
     (2, 1, 8, 2, torch.float32, False),
     (2, 257, 290, 2, torch.bfloat16, True),
     (1, 40, 130, 1, torch.bfloat16, False),
+    (2, 1030, 520, 1, torch.bfloat16, False),   # 8 and 16 tokens a thread (few tokens, as above: 4)
+    (2, 2051, 520, 2, torch.float32, True),
 ]
 
 
@@ -68,6 +70,8 @@ CHAIN_CASES = [
     (1, 5, 33, torch.float32, False),
     (1, 23, 40, torch.float32, False),
     (2, 257, 290, torch.bfloat16, True),
+    (2, 1030, 520, torch.float32, False),
+    (2, 2051, 520, torch.bfloat16, True),
 ]
 
 
