@@ -21,12 +21,18 @@
 //                  on the OUTPUT row n only: the accumulator is multiplied by et[J+1] between the tiles (Horner).  The
 //                  result holds four adjacent columns of a state row per lane: 16-byte stores.
 //
-// Everything but W is a product of factors <= 1.  W grows like 2^(span of a tile): a chunk with a tile whose sum of a is
-// below -FWD_SPAN_LIMIT is computed once more, by the same workgroup, with the level-hierarchy body (k_chunk_local_body),
-// which has no such limit and overwrites everything written for the chunk before.  bf16 inputs: the wave that meets
-// such a tile raises a flag that all look at once a step, and the rest of the steps is left out (a quarter of the chunks of a
-// freshly initialised decoder, 8 x 1024 tokens, 256 queries: 195 -> 179 us a layer).  fp32 inputs, whose operand pairs leave no
-// registers to spare, pay for the look: 1505 -> 1575 us at 16 x 2048 tokens, 16 heads x 64, 512 states, nothing out of range.
+// Everything but W is a product of factors <= 1.  W grows like 2^(span of a tile) and is taken where every tile of the wave's
+// columns decays by less than 2^FWD_SPAN_LIMIT.
+//   bf16 inputs: a step with another tile is left by the loop over the steps and evaluated, by its wave alone, with the diagonal
+//   blocks in parts whose factors are all <= 1 (far_diagonal) and V from its own exponential; the loop then goes on.  Outside
+//   the loop, for what the usual step keeps in flight leaves that form no registers.  A freshly initialised decoder has such
+//   tiles in 16 % of its chunks and heads, there mostly in all steps, and those workgroups decide when the launch ends: 1024
+//   tokens, 256 queries 27 us a layer (36 with the chunk computed once more by the level-hierarchy body, 19 where no tile is
+//   out of range), 8 x 1024 110 us (155).
+//   fp32 inputs: the operand pairs leave no registers for a second form.  A chunk with such a tile is computed once more, by the
+//   same workgroup, with the level-hierarchy body (k_chunk_local_body), which has no such limit and overwrites everything
+//   written for the chunk before.
+// A tile's whole decay reaches the tile's 16 lanes by DPP, not through LDS (4 to 7 registers fewer; as fast).
 #include "issm_dev.h"
 #include "issm_fwd_local.h"
 
@@ -40,12 +46,12 @@ struct FwdTileSmem {
   uint16_t xt_hi[PT * 16 * LDT];       // x tile transposed, [p][l]
   uint16_t xt_lo[SPLIT ? PT * 16 * LDT : 8];
   f4 red[4 * 10 * 64];                 // the four waves' partial sums of the ten blocks of M
-  int bad;                             // some tile is out of range
+  int bad;                             // fp32: some tile is out of range
 };
 template <int PT, bool SPLIT>
-constexpr size_t fwd_tile_lds() {     // the level-hierarchy body lays its own structure over the same memory
-  return sizeof(FwdTileSmem<PT, SPLIT>) > sizeof(FwdLocalSmem<PT, SPLIT>) ? sizeof(FwdTileSmem<PT, SPLIT>)
-                                                                          : sizeof(FwdLocalSmem<PT, SPLIT>);
+constexpr size_t fwd_tile_lds() {     // fp32: the level-hierarchy body lays its own structure over the same memory
+  return SPLIT && sizeof(FwdTileSmem<PT, SPLIT>) < sizeof(FwdLocalSmem<PT, SPLIT>) ? sizeof(FwdLocalSmem<PT, SPLIT>)
+                                                                                   : sizeof(FwdTileSmem<PT, SPLIT>);
 }
 
 // inclusive running sum over the 16 lanes of a DPP row (lanes sharing lane >> 4)
@@ -58,6 +64,18 @@ __device__ __forceinline__ float row_scan16(float v) {
   ISSM_DPP_SHR(0x118);
 #undef ISSM_DPP_SHR
   return v;
+}
+
+// the value of lane J of a DPP row, on its 16 lanes
+template <int J>
+__device__ __forceinline__ float row_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + J, 0xf, 0xf, true));
+}
+
+// one of each four lanes' values (a DPP quad permutation)
+template <int PERM>
+__device__ __forceinline__ float quad_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), PERM, 0xf, 0xf, true));
 }
 
 // four fp32 accumulator values that are exact bf16 numbers -> a bf16 fragment
@@ -200,8 +218,74 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     const uint2 idr = make_uint2((r1 == 0 ? one : 0u) | (r1 == 1 ? one << 16 : 0u), (r1 == 2 ? one : 0u) | (r1 == 3 ? one << 16 : 0u));
     ident = __builtin_bit_cast(bf4, idr);
   }
-  const int last_lane = lane | 15;
   const float thr = ex2(-FWD_SPAN_LIMIT);
+
+  // Diagonal block of a tile whose decays may be out of range: pairs of rows in different halves, then in different quarters
+  // of a half, each with the row between the two as the reference -- both factors of every pair are <= 1 -- and in fp32 those
+  // inside a quarter (four rows), with its second row as the reference or, where that is out of range too, in three parts.
+  auto far_diagonal = [&](const float* c4, const float* w4, const float* pc4, f4& m) __attribute__((always_inline)) {
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    float uu[4], ww[4];
+    {
+      const bool up8 = i & 8;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float d = pc4[r] - row_lane<7>(pc4[r]), e = ex2(up8 ? d : -d);
+        uu[r] = up8 ? c4[r] * e : 0.0f;
+        ww[r] = up8 ? 0.0f : w4[r] * e;
+      }
+      m = frag_product<SPLIT>(make_frag<SPLIT>(uu[0], uu[1], uu[2], uu[3]), make_frag<SPLIT>(ww[0], ww[1], ww[2], ww[3]), m);
+    }
+    {
+      const bool up4 = i & 4;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float lo = row_lane<3>(pc4[r]), hi = row_lane<11>(pc4[r]);
+        const float d = pc4[r] - (i & 8 ? hi : lo), e = ex2(up4 ? d : -d);
+        uu[r] = up4 ? c4[r] * e : 0.0f;
+        ww[r] = up4 ? 0.0f : w4[r] * e;
+      }
+      const f4 t = frag_product<SPLIT>(make_frag<SPLIT>(uu[0], uu[1], uu[2], uu[3]), make_frag<SPLIT>(ww[0], ww[1], ww[2], ww[3]), zero);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] += kg == 3 && i < 4 ? 0.0f : t[r];   // (rows of different halves: not from here)
+    }
+    float d[4], dmin = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      d[r] = pc4[r] - quad_lane<0x55>(pc4[r]);   // lane 1 of four
+      dmin = fminf(dmin, -fabsf(d[r]));
+    }
+    if (__ballot(!(dmin >= -FWD_SPAN_LIMIT)) == 0ull) {
+      f4 t = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = mfma4(c4[r] * ex2(d[r]), w4[r] * ex2(-d[r]), t);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] += kg == i >> 2 ? t[r] : 0.0f;
+    } else {
+      f4 t = zero;   // rows 2, 3 with rows 0, 1
+      const bool up2 = i & 2, up1 = i & 1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = ex2(up2 ? d[r] : -d[r]);
+        t = mfma4(up2 ? c4[r] * e : 0.0f, up2 ? 0.0f : w4[r] * e, t);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] += kg == i >> 2 ? t[r] : 0.0f;
+      t = zero;      // 1 with 0, 3 with 2
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = ex2(quad_lane<0xf5>(pc4[r]) - pc4[r]);   // lanes 1, 1, 3, 3
+        t = mfma4(up1 ? c4[r] : 0.0f, up1 ? 0.0f : w4[r] * e, t);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] += 4 * kg + r == i + 1 ? t[r] : 0.0f;
+      t = zero;      // a row with itself
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = mfma4(c4[r], w4[r], t);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] += 4 * kg + r == i ? t[r] : 0.0f;
+    }
+  };
 
   f4 macc[10];
 #pragma unroll
@@ -213,9 +297,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   float* sdst = states + st_off(p, u.bt, u.c, u.h);
   float* cdst = cs_last + vec_off(p, u.bt, u.c, u.h);
 
-#pragma unroll 1
-  for (int n0 = 0; n0 < p.N; n0 += NS) {
-    const int bad_seen = IOB ? __hip_atomic_load(&s.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0;
+  // one step; the usual form (not DEEP) of bf16 inputs returns true, with nothing stored, where some tile of the wave's columns is out of range
+  auto step = [&](int n0, auto deep) __attribute__((always_inline)) {
+    constexpr bool DEEP = decltype(deep)::value;
     // ---- this step's values out of the request registers; the next step's request follows at once
     float dtv[16], bv[16], cv[16];
 #pragma unroll
@@ -239,7 +323,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
           if (j >= skip) q[j] = v[j];
       }
     };
-    {  // branch-free: the last step asks for its own columns once more
+    if (!DEEP) {  // branch-free: the last step asks for its own columns once more
       const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
       ISSM_REQUEST(nn);
     }
@@ -268,14 +352,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
     for (int k = 0; k < 16; ++k) up[k] = ex2(pc[k]);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) et[k] = __shfl(up[k], last_lane, 64);  // whole-tile decay of the lane's columns
+    for (int k = 0; k < 16; ++k) et[k] = row_lane<15>(up[k]);  // whole-tile decay of the lane's columns
+    if (!DEEP) {
 #pragma unroll
-    for (int k = 0; k < 16; k += 2) etmin = fminf(etmin, fminf(et[k], et[k + 1]));
-    if constexpr (IOB) {
-      const bool out = __ballot(!(etmin >= thr)) != 0ull;
-      if (out) s.bad = 1;
-      if (out || __builtin_amdgcn_readfirstlane(bad_seen)) break;  // wave-uniform; no barrier in the loop
+      for (int k = 0; k < 16; k += 2) etmin = fminf(etmin, fminf(et[k], et[k + 1]));
     }
+    if (IOB && !DEEP && __ballot(!(etmin >= thr)) != 0ull) return true;
     {  // the chunk's total decay (natural logarithm), four adjacent columns per lane group.  All 16 lanes of a group
        // store the same values to the same place: a store under a lane condition sits behind a branch, and the waits
        // for the requests in flight -- counted in order with the stores -- would then have to assume it away and wait
@@ -283,13 +365,22 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       f4 tot;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        tot[r] = __shfl((((pc[r] + pc[4 + r]) + pc[8 + r]) + pc[12 + r]) * LN2, last_lane, 64);
+        tot[r] = row_lane<15>((((pc[r] + pc[4 + r]) + pc[8 + r]) + pc[12 + r]) * LN2);
       put(cdst + c, tot);
     }
 
     // ---- operands
-    float w16[EDGE ? 16 : 1];
-    if constexpr (EDGE) {
+    float w16[EDGE || DEEP ? 16 : 1];
+    if constexpr (DEEP) {
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+#pragma unroll
+        for (int k = 4 * J; k < 4 * J + 4; ++k) w16[k] = dtp[k] * bv[k];
+        far_diagonal(cv + 4 * J, w16 + 4 * J, pc + 4 * J, macc[J]);
+#pragma unroll
+        for (int k = 4 * J; k < 4 * J + 4; ++k) cv[k] *= up[k];
+      }
+    } else if constexpr (EDGE) {
       // diagonal blocks, before anything else needs registers: W takes the place of B and dt', C up that of C.  fp32 matrix
       // instructions: k-slot kg of instruction r <-> the lane's column r; the blocks' chains are interleaved.
 #pragma unroll
@@ -302,7 +393,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
         for (int J = 0; J < 4; ++J) macc[J] = mfma4(cv[4 * J + r], w16[4 * J + r], macc[J]);
     }
-    auto cu = [&](int k) { return EDGE ? cv[k] : cv[k] * up[k]; };
+    auto cu = [&](int k) { return EDGE || DEEP ? cv[k] : cv[k] * up[k]; };
     Fr U[4];
 #pragma unroll
     for (int J = 0; J < 4; ++J) U[J] = make_frag<SPLIT>(cu(4 * J), cu(4 * J + 1), cu(4 * J + 2), cu(4 * J + 3));
@@ -315,11 +406,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int k = 4 * J + r;
-        if constexpr (EDGE) W[r] = w16[k];
+        if constexpr (EDGE || DEEP) W[r] = w16[k];
         else W[r] = dtp[k] * bv[k] * ex2(-pc[k]);
-        V[r] = W[r] * et[k];
+        V[r] = W[r] * (DEEP ? ex2(row_lane<15>(pc[k]) - pc[k]) : et[k]);
       }
-      if constexpr (!EDGE) {
+      if constexpr (!EDGE && !DEEP) {
         const Fr f = make_frag<SPLIT>(W[0], W[1], W[2], W[3]);
         macc[J] = frag_product<SPLIT>(U[J], f, macc[J]);
       }
@@ -353,7 +444,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
         }
         // (wider head dimensions: keep the scheduler from fetching every tile's x fragments ahead of time, which
         // costs more registers than there are)
-        if (PT > 2) __builtin_amdgcn_sched_barrier(0);
+        if (PT > 2 || DEEP) __builtin_amdgcn_sched_barrier(0);
         const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
         const bf4 th = exact_bf4(mfma_bf16k(fv.h, ident, zero)), tlo = exact_bf4(mfma_bf16k(fv.l, ident, zero));
 #pragma unroll
@@ -378,6 +469,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       for (int pt = 0; pt < PT; ++pt)
         if (16 * pt + i < p.P) put(sdst + (16 * pt + i) * p.N + c, sacc[pt]);
     }
+    return false;
+  };
+  for (int n0 = 0;;) {
+    asm volatile("");   // keeps the two loops apart
+#pragma unroll 1
+    for (; n0 < p.N; n0 += NS)
+      if (step(n0, std::false_type{})) break;   // wave-uniform; no barrier in the loop
+    if (!IOB || n0 >= p.N) break;
+    ISSM_REQUEST(n0);
+    step(n0, std::true_type{});
+    etmin = 1.0f;
+    n0 += NS;
+    if (n0 >= p.N) break;
+    ISSM_REQUEST(n0);
   }
 #undef ISSM_REQUEST
 
@@ -386,7 +491,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   for (int q = 0; q < 10; ++q) s.red[(w * 10 + q) * 64 + lane] = macc[q];
   if (!IOB && __ballot(!(etmin >= thr)) != 0ull) s.bad = 1;
   __syncthreads();
-  const int anybad = s.bad;  // uniform
+  const int anybad = IOB ? 0 : s.bad;  // uniform
   float* m = cabt + sq_off(p, u.bt, u.c, u.h);
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
@@ -407,12 +512,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       }
     }
   }
-  if (anybad) {
+  if (!IOB && anybad) {
     // A tile of this chunk decays by more than 2^-FWD_SPAN_LIMIT: everything is computed once more in the form that has no
     // such limit.  The fence orders this workgroup's stores above before the ones the other form makes to the same places.
     __threadfence();
     __syncthreads();
-    k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
+    if constexpr (!IOB) k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
   }
 }
 

@@ -628,6 +628,42 @@ def test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel(dtyp
             "head 3 is out of range only in the chunk that holds tokens 70..109"
 
 
+@pytest.mark.parametrize("L_,P,N", [(128, 32, 128), (128, 36, 192), (64, 64, 64), (150, 20, 100), (70, 48, 68)])
+def test_bf16_forward_of_any_decay(L_, P, N):
+    """The bf16 chunk pass holds a tile's decays to any power of two, per step and wave: heads whose tiles are in range, beyond
+    2^100, beyond that inside four rows, with single rows of 2^-300 between flat ones (in all columns, or in a quarter of a
+    step), and with every row beyond 2^-200.  Bound: four roundings to 8 bits (both operands of M, M, the result) of the sum
+    of the magnitudes, and the running sums' 2^-24 of an exponent in the thousands, an eighth of that."""
+    from dest3d_amd import ISSM_chunk_scan_combined
+    _say(f"bf16 forward of any decay, L={L_} P={P} N={N}")
+    H = 6
+    d = _problem(2, L_, H, P, N, 2, seed=L_ + N, softplus=False, D=None)
+    d["A"] = torch.full((H, N), -1.0)
+    g = torch.Generator().manual_seed(5)
+    dt = torch.rand(2, L_, H, N, generator=g)
+    dt[:, :, 1] *= 14.0
+    dt[:, :, 2] *= 60.0
+    spike = (torch.rand(2, L_, generator=g) < 0.15).float() * 208.0
+    dt[:, :, 3] = 0.1 * dt[:, :, 3] + spike[..., None]
+    dt[:, :, 4] = 0.1 * dt[:, :, 4]
+    dt[:, :, 4, 16:32] += spike[..., None]
+    dt[:, :, 5] = 140.0 + 20.0 * dt[:, :, 5]
+    d["dt"] = dt
+    q = {k: d[k].bfloat16() for k in ("x", "dt", "B", "C")}
+    ref = [R.issm_scan_sequential(f(q["x"].double()), q["dt"].double(), d["A"].double(), f(q["B"].double()), f(q["C"].double()),
+                                  initial_states=f(d["h0"].double())) for f in (lambda t: t, torch.abs)]
+    c = {k: v.cuda() for k, v in q.items()}
+    y, last = ISSM_chunk_scan_combined(c["x"], c["dt"], d["A"].cuda(), c["B"], c["C"], 64, initial_states=d["h0"].cuda(),
+                                       return_final_states=True)
+    bound = 4 * 2.0 ** -9 * 1.125
+    for name, got, want, size in (("y", y, ref[0][0], ref[1][0]), ("last", last, ref[0][1], ref[1][1])):
+        got = got.double().cpu()
+        assert torch.isfinite(got).all(), name
+        worst = ((got - want).abs() / size.clamp_min(1e-30)).transpose(0, 2 if name == "y" else 1).flatten(1).amax(1) / bound
+        print(f"    {name}: worst error by head, of the bound: {[round(w, 3) for w in worst.tolist()]}", flush=True)
+        assert ((got - want).abs() <= bound * size + 1e-30).all(), name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("L_,N,H,ndir", [(128, 128, 6, 1), (100, 70, 5, 2), (256, 64, 3, 2), (1600, 256, 7, 1), (130, 8, 5, 1)])
 @pytest.mark.parametrize("marked", [False, True])
