@@ -573,7 +573,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     asm volatile("" : "+v"(cm2), "+v"(g42));
     dcs[15] += g42 == 3 ? gl_keep : 0.0f;
     {
-      // suffix sums up the 64 rows; the cross-lane steps of the four tiles are issued together
+      // suffix sums up the 64 rows
       float c[4], v[4], t[4];
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
@@ -586,19 +586,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         c[J] = a;
       }
 #pragma unroll
-      for (int J = 0; J < 4; ++J) t[J] = __shfl_down(c[J], 16, 64);
-#pragma unroll
-      for (int J = 0; J < 4; ++J) v[J] = g42 <= 2 ? c[J] + t[J] : c[J];
-#pragma unroll
-      for (int J = 0; J < 4; ++J) t[J] = __shfl_down(v[J], 32, 64);
-#pragma unroll
-      for (int J = 0; J < 4; ++J) v[J] = g42 <= 1 ? v[J] + t[J] : v[J];  // inclusive from the last lane group down
-#pragma unroll
-      for (int J = 0; J < 4; ++J) t[J] = __shfl(v[J], cm2, 64);           // tile totals
+      for (int J = 0; J < 4; ++J) {
+        float before;
+        group_sums(c[J], g42, before, v[J], t[J]);   // of the rows behind, of the tile
+      }
       float carry = 0.0f;  // sum over all rows after the current tile
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
-        const float add = carry + (v[J] - c[J]);
+        const float add = carry + v[J];
 #pragma unroll
         for (int j = 0; j < 4; ++j) dcs[4 * J + j] += add;
         carry += t[J];
