@@ -504,15 +504,24 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
 // equally long up to about this many multiply-adds (2048 x 288 -> 586: 8.5 us against 7.4; 4096: 12.3 against 9.3, 512 -> 512:
 // 24 against 9; above, and where training keeps the GPU busy, the kernel counts).
 constexpr double FEW_PRODUCTS = 3.5e8;
+// (tensors that stand for something else than their memory, under vmap, functionalization, a tensor subclass or a lazy
+// negation, go to the library's product, which knows them)
+bool own_memory(const Tensor& t) {
+  using K = c10::DispatchKey;
+  return t.has_storage() &&
+         !t.key_set().has_any(c10::DispatchKeySet({K::Python, K::Functionalize, K::FuncTorchBatched, K::FuncTorchGradWrapper,
+                                                   K::Batched, K::Negative, K::ZeroTensor}));
+}
 bool few_tokens(const Tensor& x, const Tensor& w) {
+  if (!own_memory(x) || !own_memory(w)) return false;
   if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
   if (w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || w.size(1) == 0 || w.size(1) % 32 || x.numel() == 0) return false;
   return (double)x.numel() * (double)w.size(0) <= FEW_PRODUCTS && x.is_contiguous() && w.is_contiguous() &&
          (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
 }
-// y = x w^T of one or two such pairs
+// y = x w^T of one or two such pairs; the last of two, x (batch, n, in), gives (batch, out, n) where `turn` is set
 template <size_t N>
-std::array<Tensor, N> linear_few(const std::array<std::pair<Tensor, Tensor>, N>& xw) {
+std::array<Tensor, N> linear_few(const std::array<std::pair<Tensor, Tensor>, N>& xw, bool turn = false) {
   const c10::DeviceGuard guard(xw[0].first.device());
   issm_linear_args a{};
   std::array<Tensor, N> y;
@@ -520,8 +529,11 @@ std::array<Tensor, N> linear_few(const std::array<std::pair<Tensor, Tensor>, N>&
     const Tensor &x = xw[i].first, &w = xw[i].second;
     at::DimVector sizes(x.sizes());
     sizes.back() = w.size(0);
+    const bool turned = turn && i == N - 1;
+    if (turned) std::swap(sizes[1], sizes[2]);
     y[i] = fresh(sizes, x, at::kBFloat16);
-    a.job[i] = issm_linear_job{data(x), data(w), data(y[i]), x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0)};
+    a.job[i] = issm_linear_job{data(x), data(w), data(y[i]), x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0),
+                               turned ? (int32_t)x.size(1) : 0};
   }
   a.njobs = (int32_t)N;
   a.dtype = ISSM_BF16;
@@ -640,11 +652,28 @@ struct CoreFn : public Function<CoreFn> {
     double lo, hi, eps;
   };
 
+  // Without a gradient (scan_layer): h0_lin is (B, d_inner, K) already, and query_norm belongs to what one launch makes of the
+  // scan's results (issm_layer_out).
+  struct Plain {
+    Tensor query_w, query_b;
+    double query_eps;
+  };
+
   static variable_list forward(AutogradContext* ctx, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
                                const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
                                const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
                                const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
                                int64_t ngroups, double lo, double hi, double eps) {
+    return run(ctx, nullptr, zxbcdt, h0_lin, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
+               norm_w, d_inner, nheads, ngroups, lo, hi, eps);
+  }
+
+  // one of ctx and plain
+  static variable_list run(AutogradContext* ctx, const Plain* plain, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
+                           const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
+                           const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
+                           const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
+                           int64_t ngroups, double lo, double hi, double eps) {
     const c10::DeviceGuard guard(zxbcdt.device());
     const Tensor weights = opt(weights_);
     const int64_t Bsz = zxbcdt.size(0), Ln = zxbcdt.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
@@ -724,13 +753,38 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
     }
     // 3. the bidirectional scan, queries as initial state
-    const Tensor h0 = transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()))
-                          .view({Bsz, H, P, K});
+    const Tensor h0 = (plain ? h0_lin : transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0,
+                                                         kernel_type(h0_lin.scalar_type()))).view({Bsz, H, P, K});
     const Tensor xs[2] = {x.select(0, 0), x.select(0, 1)}, Bs[2] = {bc.select(0, 0), bc.select(0, 2)},
                  Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
     const Scan s = Scan::make(2, xs, dt, A1, Bs, Cs, D.dim() == 1 ? flat.narrow(0, off[D_], H) : D, none, Tensor(), h0,
                               Tensor(), !wt.defined(), lo, hi);
     Scan::Out o = s.forward(true);
+    if (plain) {
+      Tensor key = fresh({Bsz, Ln, di}, zx, k), query = fresh({Bsz, K, di}, zx, k);
+      issm_layer_out_args a{};
+      a.batch = (int32_t)Bsz;
+      a.seqlen = (int32_t)Ln;
+      a.queries = (int32_t)K;
+      a.d_inner = (int32_t)di;
+      a.dtype = ISSM_BF16;
+      for (int i = 0; i < 2; ++i) {
+        a.y[i] = data(o.y[i]);
+        a.last[i] = data<const float>(o.last[i]);
+      }
+      a.z = data(z);
+      a.z_row_stride = zx.stride(1);
+      a.key_weight = data(norm_w);
+      a.key_eps = (float)(4.0 * eps);
+      a.key = data(key);
+      a.query_weight = data(plain->query_w);
+      a.query_bias = data(plain->query_b);
+      a.query_eps = (float)plain->query_eps;
+      a.query = data(query);
+      a.stream = stream_of(zx);
+      check(issm_layer_out(&a), "issm_layer_out");
+      return {key, query};
+    }
     // 4. gated RMSNorm (norm(x * silu(z))) of the two directions' average: the norm of s / 2 with eps is the norm of s with
     // 4 eps, so the sum goes in as it is and the halving never runs (nor its backward)
     const Tensor key = at::add(o.y[0], o.y[1]).view({Bsz * Ln, di});
@@ -902,6 +956,35 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
   check_core(in_key, in_query, dist, opt(weights_));
   py::gil_scoped_release release;
+  // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, nine
+  // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 ->
+  // 659 us).
+  // With many tokens the products are the library's, and the launches are not what counts.
+  const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
+  auto plain_bf16 = [&](const Tensor& t) {
+    return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.device() == in_key.device() &&
+                            t.dim() == 1 && t.size(0) == d_inner && own_memory(t));
+  };
+  // (functorch's transforms refuse autograd functions, and so this path too)
+  bool plain = !at::autocast::is_autocast_enabled(at::kCUDA) &&
+               !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) && few_tokens(in_key, key_proj) && few_tokens(in_query, query_proj) &&
+               few_tokens(in_key, out_key_proj) && few_tokens(in_query, out_query_proj) && in_query.device() == in_key.device() &&
+               in_key.size(-1) == d_inner && in_query.size(-1) == d_inner && query_proj.size(0) == d_inner && d_inner % 4 == 0 &&
+               d_inner <= 1024 && plain_bf16(key_norm) && plain_bf16(query_wt) && plain_bf16(query_bt);
+  for (const Tensor* t : std::initializer_list<const Tensor*>{&in_key, &in_query, &dist, &key_proj, &query_proj, &out_key_proj,
+                                                              &out_query_proj, &conv_w_f, &conv_w_b, &conv_b_f, &conv_b_b, &dt_w,
+                                                              &bc_w, &dt_bias, &A_log, &D, &key_norm, &query_wt, &query_bt, &wts}) {
+    if (!plain) break;
+    plain = !t->defined() || (own_memory(*t) && !(at::GradMode::is_enabled() && t->requires_grad()) && !t->_fw_grad(0).defined());
+  }
+  if (plain) {
+    auto [zx, h0] = linear_few<2>({{{in_key, key_proj}, {in_query, query_proj}}}, true);
+    const CoreFn::Plain p{query_wt, query_bt, query_eps};
+    variable_list core = CoreFn::run(nullptr, &p, zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias,
+                                     A_log, D, key_norm, d_inner, nheads, ngroups, lo, hi, key_eps);
+    auto [key, query] = linear_few<2>({{{core[0], out_key_proj}, {core[1], out_query_proj}}});
+    return {key, query};
+  }
   const Tensor zx = linear_tokens(in_key, key_proj), h0 = linear_tokens(in_query, query_proj);
   variable_list core = CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
                                      key_norm, d_inner, nheads, ngroups, lo, hi, key_eps);

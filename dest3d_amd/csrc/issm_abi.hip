@@ -46,6 +46,7 @@ struct TrP {
 int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 int launch_linear(LinearP& p, int njobs, hipStream_t st);
+int launch_layer_out(LayerOutP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
                       hipStream_t st);
@@ -807,10 +808,33 @@ int issm_linear_fwd(const issm_linear_args* a) {
     if (!j.x || !j.w || !j.y) return fail(ISSM_E_NULL, "linear: x/w/y is NULL");
     if (((uintptr_t)j.x | (uintptr_t)j.w) & 15) return fail(ISSM_E_STRIDE, "linear: x and w must be aligned to 16 bytes");
     if ((uintptr_t)j.y & 1) return fail(ISSM_E_STRIDE, "linear: y must be aligned to its elements");
-    p.job[n++] = LinearJob{(const uint16_t*)j.x, (const uint16_t*)j.w, (uint16_t*)j.y, (int)j.tokens, j.out, j.in / 32, 0};
+    if (j.turn < 0 || (j.turn && j.tokens % j.turn)) return fail(ISSM_E_SHAPE, "linear: %lld tokens, turned by %d", (long long)j.tokens, j.turn);
+    p.job[n++] = LinearJob{(const uint16_t*)j.x, (const uint16_t*)j.w, (uint16_t*)j.y, (int)j.tokens, j.out, j.in / 32, 0, j.turn};
   }
   if (n == 0) return ISSM_OK;
   return launched(launch_linear(p, n, (hipStream_t)a->stream), "linear_fwd");
+}
+
+int issm_layer_out(const issm_layer_out_args* a) {
+  if (!a) return fail(ISSM_E_NULL, "layer_out: args is NULL");
+  if (a->batch < 0 || a->seqlen < 0 || a->queries < 0 || a->d_inner < 1) return fail(ISSM_E_SHAPE, "layer_out: bad shape");
+  if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "layer_out: dtype %d (bf16 only)", a->dtype);
+  if (a->d_inner % 4 || a->d_inner > 1024)
+    return fail(ISSM_E_UNSUPPORTED, "layer_out: %d features (a multiple of 4, at most 1024)", a->d_inner);
+  LayerOutP p{};
+  p.rows = (long)a->batch * a->seqlen;
+  p.B = a->queries ? a->batch : 0;
+  p.K = a->queries ? a->queries : 1;
+  if (p.rows == 0 && p.B == 0) return ISSM_OK;
+  if (p.rows && (!a->y[0] || !a->y[1] || !a->z || !a->key_weight || !a->key)) return fail(ISSM_E_NULL, "layer_out: y/z/key_weight/key is NULL");
+  if (p.rows && a->z_row_stride < a->d_inner) return fail(ISSM_E_STRIDE, "layer_out: z_row_stride %lld", (long long)a->z_row_stride);
+  if (p.B && (!a->last[0] || !a->last[1] || !a->query)) return fail(ISSM_E_NULL, "layer_out: last/query is NULL");
+  p.y0 = (const uint16_t*)a->y[0]; p.y1 = (const uint16_t*)a->y[1]; p.z = (const uint16_t*)a->z; p.zs = a->z_row_stride;
+  p.kw = (const uint16_t*)a->key_weight; p.qw = (const uint16_t*)a->query_weight; p.qb = (const uint16_t*)a->query_bias;
+  p.key = (uint16_t*)a->key; p.query = (uint16_t*)a->query;
+  p.last0 = a->last[0]; p.last1 = a->last[1];
+  p.di = a->d_inner; p.keps = a->key_eps; p.qeps = a->query_eps;
+  return launched(launch_layer_out(p, (hipStream_t)a->stream), "layer_out");
 }
 
 int issm_transpose_states(const issm_transpose_args* a) {

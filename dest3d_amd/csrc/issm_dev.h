@@ -177,10 +177,20 @@ struct LinearJob {
   const uint16_t *x, *w;
   uint16_t* y;
   int tokens, out, steps, oblocks;   // steps of 32 along the contraction
+  int turn;                          // 0: y (tokens, out); else y (tokens / turn, out, turn)
 };
 struct LinearP {
   LinearJob job[2];
   int blocks0;   // of the first
+};
+// parameters of the kernel behind the scan (layer_out.hip)
+struct LayerOutP {
+  const uint16_t *y0, *y1, *z, *kw, *qw, *qb;   // qw, qb may be NULL
+  uint16_t *key, *query;
+  const float *last0, *last1;
+  long rows, zs;   // rows of y, row stride of z
+  int B, K, di, key_blocks;
+  float keps, qeps;
 };
 struct LayerParamsP {
   const void* src[LAYER_ARRAYS];

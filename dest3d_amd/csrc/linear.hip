@@ -3,7 +3,8 @@
 //
 // At these sizes a product is a few microseconds whoever computes it, and what counts is what it costs to launch: a library
 // product takes 19 us of host time to issue, 4.6 here; a decoder layer has four, and six layers on one scene (1024 tokens, 256
-// queries) ran at the pace of the host: 1240 -> 858 us.  Both operands have the contraction index contiguous, which is the operand layout of
+// queries) ran at the pace of the host: 1240 -> 858 us.  Without a gradient a layer needs two such launches, the queries turned into
+// the layout of the scan's states on the way.  Both operands have the contraction index contiguous, which is the operand layout of
 // v_mfma_f32_16x16x32_bf16 as it lies in memory: a wave asks for all fragments of its 16 tokens and 32 outputs at once (27 loads
 // of 16 bytes a lane at 288 features) and multiplies as they arrive; there is nothing to share through LDS that L1 does not
 // share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens or features the fragments' 64-byte pieces
@@ -16,12 +17,11 @@ struct __attribute__((packed, aligned(2))) LinearOut {   // four outputs; rows o
   bf4 v;
 };
 
-// N: fragments in flight
-template <int N>
-__global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
-  const bool second = (int)blockIdx.x >= p.blocks0;
-  const LinearJob& j = p.job[second ? 1 : 0];
-  const int bid = (int)blockIdx.x - (second ? p.blocks0 : 0), lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+// N: fragments in flight.  TURN: the product is stored transposed within each j.turn tokens (queries as the scan's initial
+// states); the operands change places, and a lane holds four tokens of an output instead of four outputs of a token.
+template <int N, bool TURN>
+__device__ __forceinline__ void linear_block(const LinearJob& j, int bid) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
   const int t = (bid / j.oblocks) * 64 + (threadIdx.x >> 6) * 16 + i, o0 = (bid % j.oblocks) * 32;
   const long in = 32L * j.steps;
   const bf8* x = (const bf8*)(j.x + (long)min(t, j.tokens - 1) * in) + g;
@@ -40,9 +40,26 @@ __global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
 #pragma unroll
     for (int u = 0; u < N; ++u)
       if (s0 + u < j.steps) {   // uniform
-        ya = mfma_bf(fa[u], fx[u], ya);
-        yb = mfma_bf(fb[u], fx[u], yb);
+        ya = TURN ? mfma_bf(fx[u], fa[u], ya) : mfma_bf(fa[u], fx[u], ya);
+        yb = TURN ? mfma_bf(fx[u], fb[u], yb) : mfma_bf(fb[u], fx[u], yb);
       }
+  }
+  if constexpr (TURN) {
+    const int t4 = t - i + 4 * g, row = t4 / j.turn, col = t4 % j.turn;
+    auto put = [&](int o, f4 v) {
+      if (o >= j.out) return;
+      uint16_t* y = j.y + ((long)row * j.out + o) * j.turn + col;
+      if (col + 4 <= j.turn && t4 + 4 <= j.tokens) {
+        ((LinearOut*)y)->v = __builtin_convertvector(v, bf4);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (t4 + r < j.tokens) j.y[((long)((t4 + r) / j.turn) * j.out + o) * j.turn + (t4 + r) % j.turn] = f_to_bf16(v[r]);
+      }
+    };
+    put(o0 + i, ya);
+    put(o0 + 16 + i, yb);
+    return;
   }
   if (t >= j.tokens) return;
   uint16_t* y = j.y + (long)t * j.out;
@@ -57,6 +74,15 @@ __global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
   };
   put(o0 + 4 * g, ya);
   put(o0 + 16 + 4 * g, yb);
+}
+
+template <int N>
+__global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
+  const bool second = (int)blockIdx.x >= p.blocks0;
+  const LinearJob& j = p.job[second ? 1 : 0];
+  const int bid = (int)blockIdx.x - (second ? p.blocks0 : 0);
+  if (j.turn) linear_block<N, true>(j, bid);
+  else linear_block<N, false>(j, bid);
 }
 
 int launch_linear(LinearP& p, int njobs, hipStream_t st) {

@@ -418,6 +418,7 @@ typedef struct issm_linear_job {
   void* y;
   int64_t tokens;
   int32_t in, out;
+  int32_t turn; /* 0, or a divisor n of tokens: y is (tokens / n, out, n), each n tokens' outputs transposed */
 } issm_linear_job;
 typedef struct issm_linear_args {
   issm_linear_job job[ISSM_LINEAR_JOBS];
@@ -427,6 +428,31 @@ typedef struct issm_linear_args {
 } issm_linear_args;
 
 int issm_linear_fwd(const issm_linear_args* args);
+
+/* ---- behind the scan of a layer, without a gradient ------------------------------------------
+ * models/dest_module.py:574-585 up to the output projections, ISSM_BF16, one launch:
+ *   key   (batch, seqlen, d_inner)  = RMSNorm(bf16(y[0] + y[1]) * silu(z), key_eps) * key_weight   (the norm of the average of
+ *                                     the two directions with eps is that of their sum with 4 eps)
+ *   query (batch, queries, d_inner) = LayerNorm over d_inner of bf16((last[0] + last[1]) / 2) transposed
+ * y, key, query contiguous; z rows of d_inner at z_row_stride elements; last (batch, d_inner, queries) fp32; query_weight and
+ * query_bias (d_inner) may be NULL.  d_inner a multiple of 4 and at most 1024 (ISSM_E_UNSUPPORTED otherwise). */
+typedef struct issm_layer_out_args {
+  int32_t batch, seqlen, queries, d_inner, dtype;
+  const void* y[2];
+  const void* z;
+  int64_t z_row_stride;
+  const void* key_weight;
+  float key_eps;
+  void* key;
+  const float* last[2];
+  const void* query_weight;
+  const void* query_bias;
+  float query_eps;
+  void* query;
+  void* stream;
+} issm_layer_out_args;
+
+int issm_layer_out(const issm_layer_out_args* args);
 
 /* ---- queries <-> scan states -----------------------------------------------------------------
  * The rearrangements around the scan in MultiHeadISSMScan.forward: queries become initial states

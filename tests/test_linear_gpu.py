@@ -26,7 +26,7 @@ def _close(y, x, w, ref):
 
 class Job(C.Structure):
     _fields_ = [("x", C.c_void_p), ("w", C.c_void_p), ("y", C.c_void_p), ("tokens", C.c_int64), ("nin", C.c_int32),
-                ("nout", C.c_int32)]
+                ("nout", C.c_int32), ("turn", C.c_int32)]
 
 
 class Args(C.Structure):
@@ -34,22 +34,27 @@ class Args(C.Structure):
 
 
 @pytest.mark.parametrize("shapes", [[(1, 32, 1)], [(64, 288, 32)], [(65, 288, 33), (16, 288, 586)], [(17, 256, 31), (130, 544, 35)],
-                                    [(1023, 320, 64)], [(3, 96, 7), (0, 32, 5)]])
+                                    [(1023, 320, 64)], [(3, 96, 7), (0, 32, 5)], [(64, 288, 33), (512, 288, 288, 256)],
+                                    [(15, 64, 5, 5), (130, 96, 35, 13)], [(70, 32, 17, 70), (66, 32, 3, 1)]])
 def test_linear_at_its_remainders(shapes):
-    """Rows, outputs and steps that fill no tile, batch of fragments or aligned store; one and two products a launch."""
+    """Rows, outputs and steps that fill no tile, batch of fragments or aligned store; one and two products a launch; results
+    transposed within every fourth number of tokens."""
     lib = L.load()
     a, kept = Args(), []
-    for i, (t, nin, nout) in enumerate(shapes):
+    for i, (t, nin, nout, *turn) in enumerate(shapes):
         x, w, ref = _operands(t, nin, nout, 7 * i + t)
         xd, wd = x.cuda(), w.cuda()
         y = torch.full((t + 1, nout), 3.0, dtype=torch.bfloat16, device="cuda")     # a row behind the result
-        a.job[i] = Job(xd.data_ptr(), wd.data_ptr(), y.data_ptr(), t, nin, nout)
-        kept.append((x, w, ref, xd, wd, y))
+        a.job[i] = Job(xd.data_ptr(), wd.data_ptr(), y.data_ptr(), t, nin, nout, *turn)
+        kept.append((x, w, ref, xd, wd, y, turn))
     a.njobs, a.dtype, a.stream = len(shapes), L.ISSM_BF16, L.current_stream_ptr(torch.device("cuda", 0))
     assert lib.issm_linear_fwd(C.byref(a)) == 0
     torch.cuda.synchronize()
-    for x, w, ref, _, _, y in kept:
-        _close(y[:-1], x, w, ref)
+    for x, w, ref, _, _, y, turn in kept:
+        got = y[:-1]
+        if turn:
+            got = got.reshape(-1, y.shape[1], turn[0]).transpose(1, 2).reshape(got.shape)
+        _close(got, x, w, ref)
         assert (y[-1] == 3.0).all()
 
 
@@ -58,7 +63,8 @@ def test_linear_refuses_what_it_does_not_take():
     x = torch.zeros(64, 64, dtype=torch.bfloat16, device="cuda")
     good = (x.data_ptr(), x.data_ptr(), x.data_ptr(), 8, 32, 8)
     for job, n, dtype in ((good, 3, L.ISSM_BF16), (good, 1, L.ISSM_F32), ((*good[:4], 33, 8), 1, L.ISSM_BF16), ((*good[:4], 0, 8), 1, L.ISSM_BF16),
-                          ((x.data_ptr() + 2, *good[1:]), 1, L.ISSM_BF16), ((None, *good[1:]), 1, L.ISSM_BF16), ((*good[:3], -1, 32, 8), 1, L.ISSM_BF16)):
+                          ((x.data_ptr() + 2, *good[1:]), 1, L.ISSM_BF16), ((None, *good[1:]), 1, L.ISSM_BF16), ((*good[:3], -1, 32, 8), 1, L.ISSM_BF16),
+                          ((*good, 3), 1, L.ISSM_BF16), ((*good, -1), 1, L.ISSM_BF16)):
         a = Args()
         a.job[0] = Job(*job)
         a.njobs, a.dtype = n, dtype
@@ -92,3 +98,83 @@ def test_projections_of_every_form(kind):
     y.backward(dy)
     want = torch.ones(y.shape, dtype=torch.double) @ w.detach().double().cpu()
     assert ((x.grad.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+
+
+def test_projections_under_transforms():
+    """functorch's transforms are refused, as they are by the autograd function the kernel is reached through."""
+    from dest3d_amd.scan_module import _LinearTokens
+    x, w, _ = _operands(40, 96, 50, 4)
+    x, w = x.cuda(), w.cuda()
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        torch.vmap(lambda t: _LinearTokens.apply(t, w))(x.view(4, 10, 96))
+
+
+class OutArgs(C.Structure):
+    _fields_ = [("batch", C.c_int32), ("seqlen", C.c_int32), ("queries", C.c_int32), ("d_inner", C.c_int32), ("dtype", C.c_int32),
+                ("y", C.c_void_p * 2), ("z", C.c_void_p), ("z_row_stride", C.c_int64), ("key_weight", C.c_void_p),
+                ("key_eps", C.c_float), ("key", C.c_void_p), ("last", C.c_void_p * 2), ("query_weight", C.c_void_p),
+                ("query_bias", C.c_void_p), ("query_eps", C.c_float), ("query", C.c_void_p), ("stream", C.c_void_p)]
+
+
+@pytest.mark.parametrize("B,Ln,K,di,affine", [(1, 1, 1, 4, True), (2, 5, 9, 256, False), (3, 7, 16, 288, True), (1, 3, 7, 516, True),
+                                              (2, 0, 3, 1024, False), (2, 6, 0, 260, True)])
+def test_behind_the_scan(B, Ln, K, di, affine):
+    """Rows, queries and features that fill no workgroup, wave or vector, against fp64 on the sums and averages rounded to bf16.
+    Bound: the rounding of the result to 8 bits, and 2^-20 of the magnitudes for fp32 statistics and the fast exponential."""
+    g = torch.Generator().manual_seed(di + K)
+    r = lambda *s: torch.randn(*s, generator=g)
+    bf = lambda t: t.bfloat16().cuda()
+    y, zx, kw = [bf(r(B, Ln, di)) for _ in range(2)], bf(r(B, Ln, di + 3)), bf(r(di))
+    last, qw, qb = [r(B, di, K).cuda() for _ in range(2)], bf(r(di)), bf(r(di))
+    key, query = bf(torch.zeros(B * Ln + 1, di)), bf(torch.zeros(B * K + 1, di))
+    ptr = lambda t: t.data_ptr() if t.numel() else None
+    a = OutArgs(B, Ln, K, di, L.ISSM_BF16, (C.c_void_p * 2)(*map(ptr, y)), ptr(zx), di + 3, kw.data_ptr(), 4e-5, key.data_ptr(),
+                (C.c_void_p * 2)(*map(ptr, last)), qw.data_ptr() if affine else None, qb.data_ptr() if affine else None, 1e-5,
+                query.data_ptr(), L.current_stream_ptr(torch.device("cuda", 0)))
+    assert L.load().issm_layer_out(C.byref(a)) == 0
+    torch.cuda.synchronize()
+    c = lambda t: t.double().cpu()
+    z = c(zx)[..., :di]
+    v = c((y[0].float() + y[1].float()).bfloat16()) * z * torch.sigmoid(z)
+    v = (v * (v.pow(2).mean(-1, keepdim=True) + 4e-5).rsqrt() * c(kw)).reshape(-1, di)
+    assert ((c(key[:-1]) - v).abs() <= 2.0 ** -8 * v.abs() + 2.0 ** -20).all() and (key[-1] == 0).all()
+    s = c(((last[0] + last[1]) * 0.5).bfloat16()).transpose(1, 2).reshape(-1, di)
+    s = (s - s.mean(-1, keepdim=True)) * (s.var(-1, unbiased=False, keepdim=True) + 1e-5).rsqrt()
+    size = s.abs()
+    if affine:
+        s, size = s * c(qw) + c(qb), size * c(qw).abs() + c(qb).abs()
+    assert ((c(query[:-1]) - s).abs() <= 2.0 ** -8 * s.abs() + 2.0 ** -20 * (1 + size)).all() and (query[-1] == 0).all()
+    for field, bad in (("dtype", L.ISSM_F32), ("d_inner", 2), ("d_inner", 1028), ("batch", -1), ("z_row_stride", 1)):
+        if field == "z_row_stride" and B * Ln == 0:
+            continue
+        was = getattr(a, field)
+        setattr(a, field, bad)
+        assert L.load().issm_layer_out(C.byref(a)) != 0, field
+        setattr(a, field, was)
+
+
+@pytest.mark.parametrize("B,Ln,K", [(1, 130, 40), (2, 64, 256), (3, 1, 1)])
+@pytest.mark.parametrize("mask", [None, "weights", "drop"])
+def test_layer_without_a_gradient(B, Ln, K, mask):
+    """The layer's shorter chain against the one that is differentiated: up to the output projections the same kernels on the
+    same operands, except for the two norms, whose results may round to the neighbouring bf16 number; through the projection that
+    is 2^-7 of its terms' magnitudes (8 bits, and the result's own rounding)."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(B * Ln + K)
+    layer = MultiHeadISSMScan(d_model=288, d_state=K, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    key, query = torch.randn(B, Ln, 288).cuda().bfloat16(), torch.randn(B, K, 288).cuda().bfloat16()
+    dist = torch.randn(B, Ln, K, 16).cuda().bfloat16()
+    m = None if mask is None else torch.rand(B, Ln, K).cuda() if mask == "weights" else torch.rand(B, Ln, K).cuda() < 0.3
+    want = layer(key, query, dist, None, m)
+    with torch.no_grad():
+        got = layer(key, query, dist, None, m)
+    assert want[0].requires_grad and not got[0].requires_grad
+    with torch.no_grad():
+        for a, b, w in zip(got, want, (layer.out_key_proj.weight, layer.out_query_proj.weight)):
+            assert a.shape == b.shape and torch.isfinite(a).all()
+            # rows of the normed operand have unit mean square (times the norm's weight, 1 at initialisation)
+            size = w.float().abs().sum(1) * 1.0
+            assert ((a - b).float().abs() <= 2.0 ** -7 * size + 2.0 ** -7 * b.float().abs()).all()
+    layer.requires_grad_(False)
+    frozen = layer(key, query, dist, None, m)
+    assert all(torch.equal(a, b) for a, b in zip(frozen, got))
