@@ -46,6 +46,8 @@ struct TrP {
 int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 int launch_linear(LinearP& p, int njobs, hipStream_t st);
+int linear_dw_splits(long tokens, int in, int out);
+int launch_linear_dw(LinearDwP& p, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
@@ -813,6 +815,30 @@ int issm_linear_fwd(const issm_linear_args* a) {
   }
   if (n == 0) return ISSM_OK;
   return launched(launch_linear(p, n, (hipStream_t)a->stream), "linear_fwd");
+}
+
+static bool linear_dw_sizes(int64_t tokens, int32_t in, int32_t out) {
+  return tokens >= 0 && tokens <= 0x7fffffff / 2 && in >= 6 && out >= 4 && (int64_t)in * out < ((int64_t)1 << 31);
+}
+
+size_t issm_linear_dw_scratch_bytes(int64_t tokens, int32_t in, int32_t out) {
+  return linear_dw_sizes(tokens, in, out) ? (size_t)linear_dw_splits(tokens, in, out) * in * out * sizeof(float) : 0;
+}
+
+int issm_linear_dw(const issm_linear_dw_args* a) {
+  if (!a) return fail(ISSM_E_NULL, "linear_dw: args is NULL");
+  if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "linear_dw: dtype %d (bf16 only)", a->dtype);
+  if (!linear_dw_sizes(a->tokens, a->in, a->out)) return fail(ISSM_E_SHAPE, "linear_dw: %lld tokens, (%d, %d)", (long long)a->tokens, a->out, a->in);
+  if (a->tokens == 0) return fail(ISSM_E_SHAPE, "linear_dw: no tokens");
+  if (!a->dy || !a->x || !a->dw || !a->scratch) return fail(ISSM_E_NULL, "linear_dw: dy/x/dw/scratch is NULL");
+  if (a->scratch_bytes < issm_linear_dw_scratch_bytes(a->tokens, a->in, a->out)) return fail(ISSM_E_WORKSPACE, "linear_dw: scratch too small");
+  if ((uintptr_t)a->scratch & 15) return fail(ISSM_E_STRIDE, "linear_dw: scratch must be aligned to 16 bytes");
+  if (((uintptr_t)a->dy | (uintptr_t)a->x | (uintptr_t)a->dw) & 1) return fail(ISSM_E_STRIDE, "linear_dw: operands must be aligned to their elements");
+  LinearDwP p{};
+  p.dy = (const uint16_t*)a->dy; p.x = (const uint16_t*)a->x; p.dw = (uint16_t*)a->dw; p.partial = (float*)a->scratch;
+  p.tokens = (int)a->tokens; p.in = a->in; p.out = a->out;
+  p.splits = linear_dw_splits(a->tokens, a->in, a->out);
+  return launched(launch_linear_dw(p, (hipStream_t)a->stream), "linear_dw");
 }
 
 int issm_layer_out(const issm_layer_out_args* a) {

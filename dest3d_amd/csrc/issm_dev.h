@@ -183,6 +183,13 @@ struct LinearP {
   LinearJob job[2];
   int blocks0;   // of the first
 };
+// parameters of the projections' weight gradient (linear_dw.hip)
+struct LinearDwP {
+  const uint16_t *dy, *x;   // (tokens, out), (tokens, in)
+  float* partial;           // (splits, out, in)
+  uint16_t* dw;             // (out, in)
+  int tokens, in, out, splits, btiles, per;
+};
 // parameters of the kernel behind the scan (layer_out.hip)
 struct LayerOutP {
   const uint16_t *y0, *y1, *z, *kw, *qw, *qb;   // qw, qb may be NULL

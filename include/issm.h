@@ -429,6 +429,23 @@ typedef struct issm_linear_args {
 
 int issm_linear_fwd(const issm_linear_args* args);
 
+/* dw = dy^T x: dy (tokens, out), x (tokens, in), dw (out, in), contiguous, ISSM_BF16, sums in fp32 in an order that depends on
+ * the sizes alone; in >= 6, out >= 4.  scratch: issm_linear_dw_scratch_bytes, aligned to 16 bytes. */
+typedef struct issm_linear_dw_args {
+  const void* dy;
+  const void* x;
+  void* dw;
+  int64_t tokens;
+  int32_t in, out;
+  int32_t dtype;
+  void* scratch;
+  size_t scratch_bytes;
+  void* stream;
+} issm_linear_dw_args;
+
+size_t issm_linear_dw_scratch_bytes(int64_t tokens, int32_t in, int32_t out);
+int issm_linear_dw(const issm_linear_dw_args* args);
+
 /* ---- behind the scan of a layer, without a gradient ------------------------------------------
  * models/dest_module.py:574-585 up to the output projections, ISSM_BF16, one launch:
  *   key   (batch, seqlen, d_inner)  = RMSNorm(bf16(y[0] + y[1]) * silu(z), key_eps) * key_weight   (the norm of the average of

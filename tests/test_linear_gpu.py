@@ -109,6 +109,67 @@ def test_projections_under_transforms():
         torch.vmap(lambda t: _LinearTokens.apply(t, w))(x.view(4, 10, 96))
 
 
+class DwArgs(C.Structure):
+    _fields_ = [("dy", C.c_void_p), ("x", C.c_void_p), ("dw", C.c_void_p), ("tokens", C.c_int64), ("nin", C.c_int32),
+                ("nout", C.c_int32), ("dtype", C.c_int32), ("scratch", C.c_void_p), ("bytes", C.c_size_t), ("stream", C.c_void_p)]
+
+
+@pytest.mark.parametrize("tokens,nin,nout", [(1, 6, 4), (33, 7, 5), (64, 96, 64), (257, 98, 65), (1000, 288, 586), (8200, 97, 130)])
+def test_weight_gradient_at_its_remainders(tokens, nin, nout):
+    """Rows that fill no step, columns that fill no tile, one part and many; what is behind the operands is NaN, the scratch
+    starts as NaN.  One bf16 rounding of the result and an fp32 sum over the tokens."""
+    lib = L.load()
+    g = torch.Generator().manual_seed(tokens)
+    x, dy = torch.randn(tokens, nin, generator=g).bfloat16(), torch.randn(tokens, nout, generator=g).bfloat16()
+    pad = lambda t: torch.cat([t, torch.full_like(t[:1], float("nan"))]).cuda()
+    xd, dyd = pad(x), pad(dy)
+    dw = torch.full((nout + 1, nin), 3.0, dtype=torch.bfloat16, device="cuda")
+    size = lib.issm_linear_dw_scratch_bytes(tokens, nin, nout)
+    scratch = torch.full((size // 4 + 1,), float("nan"), device="cuda")
+    a = DwArgs(dyd.data_ptr(), xd.data_ptr(), dw.data_ptr(), tokens, nin, nout, L.ISSM_BF16, scratch.data_ptr(), size,
+               L.current_stream_ptr(torch.device("cuda", 0)))
+    assert lib.issm_linear_dw(C.byref(a)) == 0
+    torch.cuda.synchronize()
+    ref, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
+    assert ((dw[:-1].double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + tokens * 2.0 ** -24 * mag).all()
+    assert (dw[-1] == 3.0).all() and scratch[-1].isnan()
+    for field, bad in (("bytes", size - 1), ("dtype", L.ISSM_F32), ("nin", 5), ("nout", 3), ("tokens", 0), ("scratch", None)):
+        was = getattr(a, field)
+        setattr(a, field, bad)
+        assert lib.issm_linear_dw(C.byref(a)) != 0, field
+        setattr(a, field, was)
+
+
+@pytest.mark.parametrize("form", ["plain", "rows apart", "expanded gradient", "wide"])
+def test_weight_gradient_of_every_form(form):
+    from dest3d_amd.scan_module import _LinearTokens
+    nin, nout = (512, 512) if form == "wide" else (96, 50)
+    x, w, _ = _operands(300, nin, nout, 6)
+    x, w = x.cuda(), w.cuda().requires_grad_()
+    if form == "rows apart":
+        x = torch.cat([x, x], dim=1)[:, :nin]
+    dy = torch.randn(300, nout).cuda().bfloat16()
+    if form == "expanded gradient":
+        dy = dy[:1].expand(300, nout)
+    _LinearTokens.apply(x, w).backward(dy)
+    x, dy = x.double().cpu(), dy.double().cpu()
+    ref, mag = dy.t() @ x, dy.abs().t() @ x.abs()
+    # (the library may add in bf16 pieces: a rounding of the result each, four at most)
+    assert ((w.grad.double().cpu() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -9 * mag.sqrt() + 300 * 2.0 ** -24 * mag).all()
+
+
+def test_weight_gradient_differentiated_again():
+    """d/d dy of sum(dW * v) = x v^T: a backward pass under create_graph stays differentiable."""
+    from dest3d_amd.scan_module import _LinearTokens
+    x, w, _ = _operands(40, 96, 50, 8)
+    x, w = x.cuda(), w.cuda().requires_grad_()
+    dy = torch.randn(40, 50).cuda().bfloat16().requires_grad_()
+    v = torch.randn(50, 96).cuda().bfloat16()
+    dw, = torch.autograd.grad(_LinearTokens.apply(x, w), w, dy, create_graph=True)
+    got, = torch.autograd.grad(dw, dy, v)
+    _close(got, x.cpu(), v.cpu(), x.double().cpu() @ v.double().cpu().t())
+
+
 class OutArgs(C.Structure):
     _fields_ = [("batch", C.c_int32), ("seqlen", C.c_int32), ("queries", C.c_int32), ("d_inner", C.c_int32), ("dtype", C.c_int32),
                 ("y", C.c_void_p * 2), ("z", C.c_void_p), ("z_row_stride", C.c_int64), ("key_weight", C.c_void_p),
