@@ -21,7 +21,7 @@ FLAG_DT_SOFTPLUS, FLAG_D_HAS_HDIM, FLAG_SEQ_IDX = 1, 2, 4
 
 EXPORTS = [
     "issm_abi_version", "issm_last_error", "issm_fwd_workspace_bytes", "issm_bwd_workspace_bytes",
-    "issm_scan_fwd", "issm_scan_bwd", "issm_stage_chunk_local", "issm_stage_state_passing_fwd",
+    "issm_scan_fwd", "issm_scan_fwd_only", "issm_scan_bwd", "issm_stage_chunk_local", "issm_stage_state_passing_fwd",
     "issm_stage_chunk_scan", "issm_stage_bwd_gate", "issm_stage_bwd_dstates",
     "issm_stage_state_passing_bwd", "issm_stage_bwd_chunk", "issm_bwd_chunk_redo_ints", "issm_stage_bwd_dx",
     "issm_stage_bwd_reduce",
@@ -228,6 +228,7 @@ def load() -> C.CDLL:
         if name != "issm_last_error" and not name.endswith("_redo_ints"):
             getattr(lib, name).restype = C.c_int
     lib.issm_box_dist_bwd_scratch_bytes.restype = C.c_int64
+    lib.issm_scan_fwd_only.argtypes = [P(ScanArgs)]
     lib.issm_linear_dw_scratch_bytes.argtypes = [C.c_int64, C.c_int32, C.c_int32]
     lib.issm_linear_dw_scratch_bytes.restype = C.c_size_t
     _lib = lib

@@ -162,7 +162,7 @@ struct Scan {
   struct Out {
     Tensor y[2], last[2], ws;
   };
-  Out forward(bool want_last) const {
+  Out forward(bool want_last, bool forward_only = false) const {
     issm_scan_args a = args();
     Out o;
     const auto& s = x[0].sizes();
@@ -179,7 +179,7 @@ struct Scan {
     o.ws = fresh({(int64_t)std::max<size_t>(n, 256)}, x[0], at::kByte);
     a.workspace = data(o.ws);
     a.workspace_bytes = (size_t)o.ws.numel();
-    check(issm_scan_fwd(&a), "issm_scan_fwd");
+    check(forward_only ? issm_scan_fwd_only(&a) : issm_scan_fwd(&a), "issm_scan_fwd");
     return o;
   }
 
@@ -789,7 +789,7 @@ struct CoreFn : public Function<CoreFn> {
                  Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
     const Scan s = Scan::make(2, xs, dt, A1, Bs, Cs, D.dim() == 1 ? flat.narrow(0, off[D_], H) : D, none, Tensor(), h0,
                               Tensor(), !wt.defined(), lo, hi);
-    Scan::Out o = s.forward(true);
+    Scan::Out o = s.forward(true, plain != nullptr);
     if (plain) {
       Tensor key = fresh({Bsz, Ln, di}, zx, k), query = fresh({Bsz, K, di}, zx, k);
       issm_layer_out_args a{};

@@ -13,7 +13,7 @@
 #include "issm_dev.h"
 
 namespace issm {
-int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st);
+int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, bool any, hipStream_t st);
 bool bwd_tile_available(const KP& p, const float* dy_ws);
 int launch_state_fwd(const KP& p, float* states, const float* cs_last, hipStream_t st);
 int launch_chunk_scan(const KP& p, const float* states, const float* cabt, float* out_x, hipStream_t st);
@@ -304,7 +304,7 @@ int issm_stage_chunk_local(const issm_scan_args* a, float* states, float* cs_las
   if (rc) return rc;
   if (!cs_last) return fail(ISSM_E_NULL, "cs_last is NULL");
   KP p = make_kp(a);
-  return launched(launch_chunk_local(p, states, cs_last, cabt, (hipStream_t)a->stream), "chunk_local");
+  return launched(launch_chunk_local(p, states, cs_last, cabt, false, (hipStream_t)a->stream), "chunk_local");
 }
 
 int issm_stage_state_passing_fwd(const issm_scan_args* a, float* states, const float* cs_last) {
@@ -326,7 +326,7 @@ int issm_stage_chunk_scan(const issm_scan_args* a, const float* states, const fl
   return launched(launch_chunk_scan(p, states, cabt, out_x, (hipStream_t)a->stream), "chunk_scan");
 }
 
-int issm_scan_fwd(const issm_scan_args* a) {
+static int scan_fwd(const issm_scan_args* a, bool forward_only) {
   int rc = check_common(a);
   if (rc) return rc;
   const bool has_z = a->z[0].ptr != nullptr;
@@ -339,10 +339,13 @@ int issm_scan_fwd(const issm_scan_args* a) {
   float* ws = (float*)a->workspace;
   KP p = make_kp(a);
   hipStream_t st = (hipStream_t)a->stream;
-  if ((rc = launched(launch_chunk_local(p, ws + w.states, ws + w.cs_last, ws + w.cabt, st), "chunk_local"))) return rc;
+  if ((rc = launched(launch_chunk_local(p, ws + w.states, ws + w.cs_last, ws + w.cabt, forward_only, st), "chunk_local"))) return rc;
   if ((rc = launched(launch_state_fwd(p, ws + w.states, ws + w.cs_last, st), "state_passing_fwd"))) return rc;
   return launched(launch_chunk_scan(p, ws + w.states, ws + w.cabt, has_z ? ws + w.out_x : nullptr, st), "chunk_scan");
 }
+
+int issm_scan_fwd(const issm_scan_args* a) { return scan_fwd(a, false); }
+int issm_scan_fwd_only(const issm_scan_args* a) { return scan_fwd(a, true); }
 
 int issm_stage_bwd_gate(const issm_scan_args* a, const float* out_x, float* dy_gated) {
   int rc = check_common(a);

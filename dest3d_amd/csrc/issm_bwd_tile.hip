@@ -253,7 +253,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     const float An = cf.A;
     float dtp[16], dfac[16], pc[16], tt[4];
     lane_dt<true>(p, cf, vn, g4, rm, l_raw, dtp, dfac);
-    lane_tile_sums(An * LOG2E, cm, g4, rm, dtp, pc, tt);
+    lane_tile_sums<IOB>(An * LOG2E, cm, g4, rm, dtp, pc, tt);
     {
       const float worst = fmaxf(fmaxf(fabsf(tt[0]), fabsf(tt[1])), fmaxf(fabsf(tt[2]), fabsf(tt[3])));
       const bool bad = !(worst <= SPAN_LIMIT);  // also true for NaN
@@ -585,15 +585,28 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
         c[J] = a;
       }
+      if constexpr (IOB) {
 #pragma unroll
-      for (int J = 0; J < 4; ++J) {
-        float before;
-        group_sums(c[J], g42, before, v[J], t[J]);   // of the rows behind, of the tile
+        for (int J = 0; J < 4; ++J) t[J] = __shfl_down(c[J], 16, 64);
+#pragma unroll
+        for (int J = 0; J < 4; ++J) v[J] = g42 <= 2 ? c[J] + t[J] : c[J];
+#pragma unroll
+        for (int J = 0; J < 4; ++J) t[J] = __shfl_down(v[J], 32, 64);
+#pragma unroll
+        for (int J = 0; J < 4; ++J) v[J] = g42 <= 1 ? v[J] + t[J] : v[J];  // inclusive from the last lane group down
+#pragma unroll
+        for (int J = 0; J < 4; ++J) t[J] = __shfl(v[J], cm2, 64);           // tile totals
+      } else {
+#pragma unroll
+        for (int J = 0; J < 4; ++J) {
+          float before;
+          group_sums(c[J], g42, before, v[J], t[J]);   // of the rows behind, of the tile
+        }
       }
       float carry = 0.0f;  // sum over all rows after the current tile
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
-        const float add = carry + v[J];
+        const float add = carry + (IOB ? v[J] - c[J] : v[J]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) dcs[4 * J + j] += add;
         carry += t[J];

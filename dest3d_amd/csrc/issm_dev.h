@@ -524,8 +524,8 @@ __device__ __forceinline__ int lane_row(int k, int g4) { return 16 * (k >> 2) + 
 // One value per lane group: the sums of the groups before and after the lane's own, and of all four, without LDS
 // (v_permlane16_swap and v_permlane32_swap of a value with its own copy leave the even / odd rows of 16 lanes, the lower /
 // upper half, on both).  The chunk backward's running and suffix sums: six trips through LDS a head fewer, fp32, both directions,
-// 8 x 1024 tokens, 8 heads x 32, 256 states 205 -> 196 us; 4 x 1000, 36, 200 states 56.9 -> 55.4; bf16 as fast (151).  Kernels
-// that call lane_prep and take single sums gained nothing by it and keep the LDS form.
+// 8 x 1024 tokens, 8 heads x 32, 256 states 205 -> 196 us; 4 x 1000, 36, 200 states 56.9 -> 55.4.  bf16 inputs (151 us either way) and
+// the kernels that call lane_prep or take single sums gained nothing by it and keep the LDS form and its rounding.
 __device__ __forceinline__ void group_sums(float c, int g4, float& before, float& after, float& all) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(c), __float_as_uint(c), false, false);
   const float even = __uint_as_float(r[0]), odd = __uint_as_float(r[1]), pair = even + odd;
@@ -814,6 +814,8 @@ __device__ __forceinline__ float lane_prep(const KP& p, const Coef& cf, bool vn,
 // including k's row, tt[J] = the whole tile's sum (the same on the four lanes of a column).  Used by the kernels that
 // write a decay exp2(cs[l] - cs[s]) as  exp2(pc[l]) . exp2(base(tile of l) - base(tile of s)) . exp2(-pc[s])  with
 // base(J) = tt[0] + .. + tt[J-1]: two exponentials per element and ten per column serve every pair of rows of the chunk.
+// LDS: the cross-lane steps through LDS (see group_sums).
+template <bool LDS>
 __device__ __forceinline__ void lane_tile_sums(float A2, int cm, int g4, const RowMap& rm, const float (&dtp)[16],
                                                float (&pc)[16], float (&tt)[4]) {
   float c[4];
@@ -841,12 +843,32 @@ __device__ __forceinline__ void lane_tile_sums(float A2, int cm, int g4, const R
       c[J] = a;
     }
   }
+  if constexpr (LDS) {
+    float v[4], t[4];
 #pragma unroll
-  for (int J = 0; J < 4; ++J) {
-    float add, after;
-    group_sums(c[J], g4, add, after, tt[J]);
+    for (int J = 0; J < 4; ++J) t[J] = __shfl_up(c[J], 16, 64);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) pc[4 * J + j] += add;
+    for (int J = 0; J < 4; ++J) v[J] = g4 >= 1 ? c[J] + t[J] : c[J];
+#pragma unroll
+    for (int J = 0; J < 4; ++J) t[J] = __shfl_up(v[J], 32, 64);
+#pragma unroll
+    for (int J = 0; J < 4; ++J) v[J] = g4 >= 2 ? v[J] + t[J] : v[J];  // inclusive over the lane groups
+#pragma unroll
+    for (int J = 0; J < 4; ++J) tt[J] = __shfl(v[J], cm + 48, 64);    // tile totals
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+      const float add = v[J] - c[J];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pc[4 * J + j] += add;
+    }
+  } else {
+#pragma unroll
+    for (int J = 0; J < 4; ++J) {
+      float add, after;
+      group_sums(c[J], g4, add, after, tt[J]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pc[4 * J + j] += add;
+    }
   }
 }
 

@@ -391,12 +391,12 @@ static int set_lds(K kernel, size_t bytes) {   // (up to 64 KB needs no asking)
 }
 
 bool local_tile_available(const KP& p, const float* states, const float* cabt);
-int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st);
+int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, bool any, hipStream_t st);
 
 // The row-lane kernel takes what it can (it falls back to the level-hierarchy body itself for the chunks outside its
-// range); packed sequences and calls that want one output only go to the level-hierarchy kernel.
-int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
-  if (local_tile_available(p, states, cabt)) return launch_local_tile(p, states, cs_last, cabt, st);
+// range or, any, evaluates their bf16 tiles in place); packed sequences and calls that want one output only go to the level-hierarchy kernel.
+int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, bool any, hipStream_t st) {
+  if (local_tile_available(p, states, cabt)) return launch_local_tile(p, states, cs_last, cabt, any, st);
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     const size_t sm = sizeof(FwdLocalSmem<PT_, !IOB_>);

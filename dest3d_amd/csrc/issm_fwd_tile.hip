@@ -23,15 +23,18 @@
 //
 // Everything but W is a product of factors <= 1.  W grows like 2^(span of a tile) and is taken where every tile of the wave's
 // columns decays by less than 2^FWD_SPAN_LIMIT.
-//   bf16 inputs: a step with another tile is left by the loop over the steps and evaluated, by its wave alone, with the diagonal
-//   blocks in parts whose factors are all <= 1 (far_diagonal) and V from its own exponential; the loop then goes on.  Outside
-//   the loop, for what the usual step keeps in flight leaves that form no registers.  A freshly initialised decoder has such
-//   tiles in 16 % of its chunks and heads, there mostly in all steps, and those workgroups decide when the launch ends: 1024
-//   tokens, 256 queries 27 us a layer (36 with the chunk computed once more by the level-hierarchy body, 19 where no tile is
-//   out of range), 8 x 1024 110 us (155).
-//   fp32 inputs: the operand pairs leave no registers for a second form.  A chunk with such a tile is computed once more, by the
-//   same workgroup, with the level-hierarchy body (k_chunk_local_body), which has no such limit and overwrites everything
-//   written for the chunk before.
+//   A chunk with another tile is computed once more, by the same workgroup, with the level-hierarchy body (k_chunk_local_body),
+//   which has no such limit and overwrites everything written for the chunk before.  bf16 inputs: the wave that meets such a
+//   tile raises a flag that all look at once a step, and the rest of the steps is left out (a quarter of the chunks of a freshly
+//   initialised decoder, 8 x 1024 tokens, 256 queries: 195 -> 179 us a layer).  fp32 inputs, whose operand pairs leave no
+//   registers to spare, pay for the look: 1505 -> 1575 us at 16 x 2048 tokens, 16 heads x 64, 512 states, nothing out of range.
+//   ANY, bf16 inputs of calls that nothing is differentiated through: a step with such a tile is left by the loop over the steps
+//   and evaluated, by its wave alone, with the diagonal blocks in parts whose factors are all <= 1 (far_diagonal) and V from its
+//   own exponential; the loop then goes on.  Outside the loop, for what the usual step keeps in flight leaves that form no
+//   registers.  A freshly initialised decoder has such tiles in 16 % of its chunks and heads, there mostly in all steps, and those
+//   workgroups decide when the launch ends: 1024 tokens, 256 queries 27 us a layer (36 with the chunk computed once more, 19 where
+//   no tile is out of range).  As accurate as the level form, but rounded elsewhere, and through six layers the gradients move by
+//   up to 0.8 of their mean square between the two: training keeps the level form (8 x 1024 tokens: 155 us, 110 with this one).
 // bf16 inputs: a tile's whole decay reaches the tile's 16 lanes by DPP, not through LDS (both directions, 8 x 1024 tokens, 8 heads
 // x 36, 256 states 93 -> 91 us; fp32 1 to 2 % slower so).
 #include "issm_dev.h"
@@ -47,11 +50,11 @@ struct FwdTileSmem {
   uint16_t xt_hi[PT * 16 * LDT];       // x tile transposed, [p][l]
   uint16_t xt_lo[SPLIT ? PT * 16 * LDT : 8];
   f4 red[4 * 10 * 64];                 // the four waves' partial sums of the ten blocks of M
-  int bad;                             // fp32: some tile is out of range
+  int bad;                             // not ANY: some tile is out of range
 };
-template <int PT, bool SPLIT>
-constexpr size_t fwd_tile_lds() {     // fp32: the level-hierarchy body lays its own structure over the same memory
-  return SPLIT && sizeof(FwdTileSmem<PT, SPLIT>) < sizeof(FwdLocalSmem<PT, SPLIT>) ? sizeof(FwdLocalSmem<PT, SPLIT>)
+template <int PT, bool SPLIT, bool ANY>
+constexpr size_t fwd_tile_lds() {     // not ANY: the level-hierarchy body lays its own structure over the same memory
+  return !ANY && sizeof(FwdTileSmem<PT, SPLIT>) < sizeof(FwdLocalSmem<PT, SPLIT>) ? sizeof(FwdLocalSmem<PT, SPLIT>)
                                                                                    : sizeof(FwdTileSmem<PT, SPLIT>);
 }
 
@@ -141,7 +144,8 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
 // wherever this kernel cannot, has the pairs inside groups of four rows in fp32, and what a pair is computed in is not to
 // depend on the kernel.  (Those entries of M: 2.4e-3 from float64 with operands rounded once to bf16, 4.4e-6 as bf16 pairs,
 // 2.6e-7 like this.  8 x 1024 tokens, 8 heads x 32, N = 250: fp32 55.4 us with pairs, 55.8 like this; bf16 43.4 and 46.9.)
-template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE>
+// ANY (bf16 inputs): tiles of any decay within the loop's own pass.
+template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE, bool ANY>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -299,7 +303,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   float* sdst = states + st_off(p, u.bt, u.c, u.h);
   float* cdst = cs_last + vec_off(p, u.bt, u.c, u.h);
 
-  if constexpr (!IOB) {
+  if constexpr (!ANY) {
     constexpr bool DEEP = false;
 #pragma unroll 1
     for (int n0 = 0; n0 < p.N; n0 += NS) {
@@ -332,7 +336,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   for (int q = 0; q < 10; ++q) s.red[(w * 10 + q) * 64 + lane] = macc[q];
   if (!IOB && __ballot(!(etmin >= thr)) != 0ull) s.bad = 1;
   __syncthreads();
-  const int anybad = IOB ? 0 : s.bad;  // uniform
+  const int anybad = ANY ? 0 : s.bad;  // uniform
   float* m = cabt + sq_off(p, u.bt, u.c, u.h);
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
@@ -353,12 +357,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
       }
     }
   }
-  if (!IOB && anybad) {
+  if (!ANY && anybad) {
     // A tile of this chunk decays by more than 2^-FWD_SPAN_LIMIT: everything is computed once more in the form that has no
     // such limit.  The fence orders this workgroup's stores above before the ones the other form makes to the same places.
     __threadfence();
     __syncthreads();
-    if constexpr (!IOB) k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
+    if constexpr (!ANY) k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
   }
 }
 
@@ -373,7 +377,7 @@ static int set_lds_tile(K kernel, size_t bytes) {   // (up to 64 KB needs no ask
   return bytes > 64 * 1024 ? (int)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) : 0;
 }
 
-int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, hipStream_t st) {
+int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, bool any, hipStream_t st) {
   const int units = p.B * p.ndir * p.nc * p.H;
   const int pt = (p.P + 15) / 16;
   // EDGE unless every tile is complete and every operand starts its rows at a multiple of four elements (16-byte stores of
@@ -384,15 +388,20 @@ int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, h
   bool edge = !p.full_tiles || !rows_of_four(p.dt, p.dt_dt) ||
               (((uintptr_t)states | (uintptr_t)cs_last | (uintptr_t)p.A | (uintptr_t)p.dt_bias) & 15);
   for (int d = 0; d < p.ndir; ++d) edge = edge || !rows_of_four(p.Bm[d], p.io_dt) || !rows_of_four(p.Cm[d], p.io_dt);
-#define ISSM_LT_ONE(PT_, IOB_, DTB_, FULLP_, EDGE_)                                                         \
+#define ISSM_LT_FORM(PT_, IOB_, DTB_, FULLP_, EDGE_, ANY_)                                                  \
   {                                                                                                         \
-    constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, FULLP_, EDGE_>;                                    \
+    constexpr auto kern = &k_local_tile<PT_, IOB_, DTB_, FULLP_, EDGE_, ANY_>;                              \
+    constexpr size_t sm = fwd_tile_lds<PT_, !IOB_, ANY_>();                                                 \
     if (int e = set_lds_tile(kern, sm)) return e;                                                           \
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);                \
   }
+#define ISSM_LT_ONE(PT_, IOB_, DTB_, FULLP_, EDGE_)                                                         \
+  {                                                                                                         \
+    if (IOB_ && any) ISSM_LT_FORM(PT_, IOB_, DTB_, FULLP_, EDGE_, IOB_)                                     \
+    else ISSM_LT_FORM(PT_, IOB_, DTB_, FULLP_, EDGE_, false)                                                \
+  }
 #define ISSM_LT(PT_, IOB_, DTB_)                                                                            \
   {                                                                                                         \
-    const size_t sm = fwd_tile_lds<PT_, !IOB_>();                                                           \
     if (edge) ISSM_LT_ONE(PT_, IOB_, DTB_, false, true)                                                     \
     else if (p.P == 16 * PT_) ISSM_LT_ONE(PT_, IOB_, DTB_, true, false)                                     \
     else ISSM_LT_ONE(PT_, IOB_, DTB_, false, false)                                                         \
@@ -409,6 +418,7 @@ int launch_local_tile(const KP& p, float* states, float* cs_last, float* cabt, h
 #undef ISSM_LT_DT
 #undef ISSM_LT
 #undef ISSM_LT_ONE
+#undef ISSM_LT_FORM
   return (int)hipGetLastError();
 }
 

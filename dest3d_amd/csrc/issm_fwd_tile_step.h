@@ -1,7 +1,8 @@
 // One step of k_local_tile (issm_fwd_tile.hip): 64 state columns, 16 of them the wave's.  Included where it runs, inside a loop
 // over n0 and with DEEP defined: the usual form (false), which breaks off with nothing stored where some tile of the wave's
-// columns is out of range (bf16 inputs), and the form that has no range (true).  (Text and not a function: as an inlined lambda
+// columns is out of range (bf16 inputs), and, ANY only, the form that has no range (true).  (Text and not a function: as an inlined lambda
 // the usual form is allocated differently, fp32 1 to 4 % slower.)
+    const int bad_seen = IOB && !ANY ? __hip_atomic_load(&s.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0;
     // ---- this step's values out of the request registers; the next step's request follows at once
     float dtv[16], bv[16], cv[16];
 #pragma unroll
@@ -59,7 +60,11 @@
 #pragma unroll
       for (int k = 0; k < 16; k += 2) etmin = fminf(etmin, fminf(et[k], et[k + 1]));
     }
-    if (IOB && !DEEP && __ballot(!(etmin >= thr)) != 0ull) break;   // wave-uniform; no barrier in the loop
+    if constexpr (IOB && !DEEP) {
+      const bool out = __ballot(!(etmin >= thr)) != 0ull;
+      if (!ANY && out) s.bad = 1;
+      if (out || (!ANY && __builtin_amdgcn_readfirstlane(bad_seen))) break;  // wave-uniform; no barrier in the loop
+    }
     {  // the chunk's total decay (natural logarithm), four adjacent columns per lane group.  All 16 lanes of a group
        // store the same values to the same place: a store under a lane condition sits behind a branch, and the waits
        // for the requests in flight -- counted in order with the stores -- would then have to assume it away and wait

@@ -161,6 +161,9 @@ int issm_bwd_workspace_bytes(const issm_scan_args* args, size_t* out);
  *                called from ISSMChunkScanCombinedFn.backward (issm_combined.py:49-54).
  *                Unlike the reference it does not recompute the forward: it reads `saved`. */
 int issm_scan_fwd(const issm_scan_args* args);
+/* The same for a call that no backward follows: the workspace's contents are then not meant for issm_scan_bwd.  bf16 chunks with
+ * 16-row tiles that decay by more than 2^100 are evaluated in one pass (equally accurate, rounded elsewhere). */
+int issm_scan_fwd_only(const issm_scan_args* args);
 int issm_scan_bwd(const issm_scan_args* args);
 
 /* Stage entry points (used by the operator above; exported for tests and profiling).

@@ -629,13 +629,14 @@ def test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel(dtyp
 
 
 @pytest.mark.parametrize("L_,P,N", [(128, 32, 128), (128, 36, 192), (64, 64, 64), (150, 20, 100), (70, 48, 68)])
-def test_bf16_forward_of_any_decay(L_, P, N):
-    """The bf16 chunk pass holds a tile's decays to any power of two, per step and wave: heads whose tiles are in range, beyond
+@pytest.mark.parametrize("only", [False, True])
+def test_bf16_forward_of_any_decay(L_, P, N, only):
+    """issm_scan_fwd_only's chunk pass holds a tile's decays to any power of two, per step and wave (issm_scan_fwd computes such
+    chunks once more): heads whose tiles are in range, beyond
     2^100, beyond that inside four rows, with single rows of 2^-300 between flat ones (in all columns, or in a quarter of a
     step), and with every row beyond 2^-200.  Bound: four roundings to 8 bits (both operands of M, M, the result) of the sum
     of the magnitudes, and the running sums' 2^-24 of an exponent in the thousands, an eighth of that."""
-    from dest3d_amd import ISSM_chunk_scan_combined
-    _say(f"bf16 forward of any decay, L={L_} P={P} N={N}")
+    _say(f"bf16 forward of any decay, L={L_} P={P} N={N} forward only: {only}")
     H = 6
     d = _problem(2, L_, H, P, N, 2, seed=L_ + N, softplus=False, D=None)
     d["A"] = torch.full((H, N), -1.0)
@@ -653,8 +654,17 @@ def test_bf16_forward_of_any_decay(L_, P, N):
     ref = [R.issm_scan_sequential(f(q["x"].double()), q["dt"].double(), d["A"].double(), f(q["B"].double()), f(q["C"].double()),
                                   initial_states=f(d["h0"].double())) for f in (lambda t: t, torch.abs)]
     c = {k: v.cuda() for k, v in q.items()}
-    y, last = ISSM_chunk_scan_combined(c["x"], c["dt"], d["A"].cuda(), c["B"], c["C"], 64, initial_states=d["h0"].cuda(),
-                                       return_final_states=True)
+    L, prob, a = _stage_args(dict(c, A=d["A"], h0=d["h0"], D=None, z=None, dt_bias=None, softplus=False,
+                                  dt_limit=(0.0, float("inf"))))
+    lib = L.load()
+    y, last = torch.empty_like(c["x"]), torch.empty(2, H, P, N, device="cuda")
+    a.out[0], a.final_states[0] = L.tensor_desc(y), last.data_ptr()
+    n = C.c_size_t()
+    L.check(lib.issm_fwd_workspace_bytes(C.byref(a), C.byref(n)), "workspace")
+    ws = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n.value
+    L.check((lib.issm_scan_fwd_only if only else lib.issm_scan_fwd)(C.byref(a)), "scan")
+    torch.cuda.synchronize()
     bound = 4 * 2.0 ** -9 * 1.125
     for name, got, want, size in (("y", y, ref[0][0], ref[1][0]), ("last", last, ref[0][1], ref[1][1])):
         got = got.double().cpu()
