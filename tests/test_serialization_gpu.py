@@ -108,6 +108,22 @@ def test_one_launch_order_equals_codes_and_stable_sorts(n):
         assert torch.equal(inv[j], torch.argsort(want, dim=-1)), o
 
 
+@pytest.mark.parametrize("B,n", [(25, 300), (40, 500), (90, 130), (1, 65)])
+def test_order_of_many_samples(B, n):
+    """Six orders of B samples: a point's place counted by several workgroups a sample, some with more points than others, or, with
+    many samples, one workgroup's sorting network."""
+    from dest3d_amd.serialization import ORDERS, hilbert_codes, hilbert_order
+    print(f"[case] hilbert order of {B} samples of {n}", flush=True)
+    pts = torch.rand(B, n, 3, generator=torch.Generator().manual_seed(B))
+    pts[:, n // 2:] = torch.round(pts[:, n // 2:] * 4) / 4
+    pts = pts.cuda()
+    orders = list(ORDERS)
+    idx, inv = hilbert_order(pts, orders, 9)
+    for j, o in enumerate(orders):
+        want = torch.argsort(hilbert_codes(pts, o, 9), dim=-1, stable=True)
+        assert torch.equal(idx[j], want) and torch.equal(inv[j], torch.argsort(want, dim=-1)), o
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
 def test_non_finite_coordinates_sort_alike_in_the_one_launch_kernel_and_in_the_separate_steps(bad):
     """A NaN or infinite coordinate (a corrupt point): no conversion of NaN to an integer, and the one-launch kernel
