@@ -31,6 +31,7 @@ EXPORTS = [
     "issm_dwconv_partial_rows", "issm_dwconv_silu_fwd", "issm_dwconv_silu_bwd",
     "issm_box_dist_bwd_scratch_bytes", "issm_box_dist_fwd", "issm_box_dist_bwd",
     "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states", "issm_layer_params", "issm_linear_fwd", "issm_linear_dw", "issm_linear_dw_scratch_bytes", "issm_layer_out",
+    "issm_box_table",
     "issm_pn2_furthest_point_sampling", "issm_pn2_ball_query", "issm_pn2_group_points", "issm_pn2_group_points_grad",
     "issm_pn2_gather_points", "issm_pn2_gather_points_grad", "issm_pn2_three_nn", "issm_pn2_three_interpolate",
     "issm_pn2_three_interpolate_grad", "issm_pn2_group_xyz_points", "issm_pn2_group_points_grad_rows",
@@ -133,6 +134,14 @@ class BoxDistArgs(C.Structure):
     ]
 
 
+class BoxTableArgs(C.Structure):
+    _fields_ = [
+        ("nodes", C.c_int32), ("hidden", C.c_int32), ("dtype", C.c_int32), ("coords_dtype", C.c_int32),
+        ("coords", C.c_void_p), ("w1", C.c_void_p), ("b1", C.c_void_p), ("w2", C.c_void_p),
+        ("table", C.c_void_p), ("stream", C.c_void_p),
+    ]
+
+
 class TransposeArgs(C.Structure):
     _fields_ = [
         ("batch", C.c_int32), ("rows", C.c_int32), ("cols", C.c_int32),
@@ -229,6 +238,7 @@ def load() -> C.CDLL:
             getattr(lib, name).restype = C.c_int
     lib.issm_box_dist_bwd_scratch_bytes.restype = C.c_int64
     lib.issm_scan_fwd_only.argtypes = [P(ScanArgs)]
+    lib.issm_box_table.argtypes = [P(BoxTableArgs)]
     lib.issm_linear_dw_scratch_bytes.argtypes = [C.c_int64, C.c_int32, C.c_int32]
     lib.issm_linear_dw_scratch_bytes.restype = C.c_size_t
     _lib = lib

@@ -16,7 +16,10 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
+import torch.autograd.forward_ad as _forward_ad
+
 from . import _lib as L
+from .scan_module import _hooked
 
 CHANNELS = 16      # table channels the kernels are built for (DEST's decoder: BoxDistFun(out_dim=16))
 MAX_NODES = 1024   # table nodes that fit the LDS copy
@@ -161,13 +164,48 @@ class BoxDistFun(nn.Module):
         """(out_dim, n, n, n): the MLP evaluated on the coordinate lattice (dest_module.py:191)."""
         return self.cpb_mlps(self.relative_coords_table.to(self.cpb_mlps[0].weight.dtype))[0].permute(3, 0, 1, 2)
 
+    def _plain_table(self):
+        """The same table, (out_dim, n, n, n) fp32, from one kernel where nothing is to be differentiated and the modules are
+        what this class made them (calling them would do nothing else); None otherwise."""
+        if type(self.cpb_mlps) is not nn.Sequential or len(self.cpb_mlps) != 3:
+            return None
+        lin1, act, lin2 = self.cpb_mlps
+        if type(lin1) is not nn.Linear or type(act) is not nn.ReLU or type(lin2) is not nn.Linear:
+            return None
+        ps, coords = (lin1.weight, lin1.bias, lin2.weight), self.relative_coords_table
+        w = ps[0]
+        if type(self).rpe_table is not BoxDistFun.rpe_table or "rpe_table" in self.__dict__ or lin2.bias is not None or \
+                lin1.bias is None or any(_hooked(m) for m in (self.cpb_mlps, lin1, act, lin2)):
+            return None
+        if torch.is_autocast_enabled("cuda") or _forward_ad._current_level >= 0 or not w.is_cuda or \
+                w.dtype not in (torch.float32, torch.bfloat16) or coords.dtype not in (torch.float32, torch.bfloat16) or \
+                w.shape[0] > 256 or w.shape != (w.shape[0], 3) or ps[1].shape != w.shape[:1] or \
+                ps[2].shape != (CHANNELS, w.shape[0]) or not coords.is_contiguous() or coords.device != w.device or \
+                (torch.is_grad_enabled() and (coords.requires_grad or any(p.requires_grad for p in ps))) or \
+                any(p.dtype != w.dtype or p.device != w.device or not p.is_contiguous() or
+                    type(p) not in (nn.Parameter, torch.Tensor) for p in ps):
+            return None
+        n = coords.shape[1:4]
+        a = L.BoxTableArgs()
+        a.nodes, a.hidden = coords.numel() // 3, w.shape[0]
+        a.dtype, a.coords_dtype = L.dtype_code(w.dtype), L.dtype_code(coords.dtype)
+        a.coords, a.w1, a.b1, a.w2 = coords.data_ptr(), w.data_ptr(), ps[1].data_ptr(), ps[2].data_ptr()
+        table = torch.empty((CHANNELS, *n), dtype=torch.float32, device=w.device)
+        a.table, a.stream = table.data_ptr(), L.current_stream_ptr(w.device)
+        with torch.cuda.device(w.device):
+            L.check(L.load().issm_box_table(C.byref(a)), "issm_box_table")
+        return table
+
     def forward(self, key_xyz, query_xyz, query_size, query_angle, weight_query_pos=None, weight_dist=15.0):
         """-> dist (B, nP, nQ, out_dim).  With ``weight_query_pos`` (B, nQ, 6) the locality weights (B, nP, nQ)
         of ``local_weight`` are computed in the same pass and returned as a second value."""
         # the kernel derives the corners (and, for the weights, centre and radius) from the boxes themselves
         boxes = torch.cat([query_xyz, query_size, query_angle.unsqueeze(-1)], dim=-1).detach()
-        table = self.rpe_table()
-        out_dtype = table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
+        table = self._plain_table()
+        plain = table is not None
+        if not plain:
+            table = self.rpe_table()
+        out_dtype = self.cpb_mlps[0].weight.dtype if plain else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
         if weight_query_pos is None:
             return BoxDistFn.apply(table, key_xyz, boxes, query_angle, None, None, 0.0, self.log_scale, self.max_value,
                                    out_dtype, True, False)[0]

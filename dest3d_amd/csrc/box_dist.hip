@@ -160,6 +160,52 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
   }
 }
 
+// The learned table without a gradient: Linear(3, hidden), ReLU, Linear(hidden, 16) at the nodes of the lattice (dest_module.py:191),
+// rounded where the modules round (bf16: the hidden values and the results; fp32 sums).  16 nodes a workgroup, a (node, channel)
+// pair a thread; the hidden values and the second weights lie in LDS.  2.4 M products at 1000 nodes and 128 hidden: bound by the
+// launch and one trip to memory.  As modules it is seven launches, 28 us and 70 us of host time; this takes 5 us.
+template <bool BF>
+__global__ __launch_bounds__(NTHREADS) void k_box_table(BoxTableP p) {
+  extern __shared__ float box_table_lds[];
+  const int R = p.hidden, ld = R + 1, node0 = blockIdx.x * 16;
+  float *h = box_table_lds, *w2 = box_table_lds + 16 * ld;
+  constexpr int io = BF ? 1 : 0;
+  __shared__ float xyz[16][3];
+  if (threadIdx.x < 48) {
+    const int i = threadIdx.x / 3, c = threadIdx.x - 3 * i;
+    const float x = ldv(p.coords, 3L * min(node0 + i, p.nodes - 1) + c, p.coords_dtype);
+    xyz[i][c] = BF ? bf16_to_f(f_to_bf16(x)) : x;
+  }
+  // a thread takes every 16th hidden value of its row: of W2 (channels), then of the hidden values (nodes)
+  const int row = threadIdx.x >> 4;
+#pragma unroll 8
+  for (int r = threadIdx.x & 15; r < R; r += 16) w2[row * ld + r] = ldv(p.w2, (long)row * R + r, io);
+  __syncthreads();
+#pragma unroll 8
+  for (int r = threadIdx.x & 15; r < R; r += 16) {
+    float v = xyz[row][0] * ldv(p.w1, 3L * r, io);
+    v = fmaf(xyz[row][1], ldv(p.w1, 3L * r + 1, io), v);
+    v = fmaf(xyz[row][2], ldv(p.w1, 3L * r + 2, io), v) + ldv(p.b1, r, io);
+    if (BF) v = bf16_to_f(f_to_bf16(v));
+    h[row * ld + r] = v < 0.0f ? 0.0f : v;   // (NaN stays)
+  }
+  __syncthreads();
+  const int i = threadIdx.x & 15, ch = threadIdx.x >> 4;
+  float v = 0.0f;
+#pragma unroll 8
+  for (int r = 0; r < R; ++r) v = fmaf(h[i * ld + r], w2[ch * ld + r], v);
+  if (BF) v = bf16_to_f(f_to_bf16(v));
+  if (node0 + i < p.nodes) p.table[(long)ch * p.nodes + node0 + i] = v;
+}
+
+int launch_box_table(const BoxTableP& p, hipStream_t st) {
+  const dim3 g((unsigned)((p.nodes + 15) / 16)), b(NTHREADS);
+  const size_t lds = (size_t)2 * 16 * (p.hidden + 1) * sizeof(float);
+  if (p.dtype) hipLaunchKernelGGL(k_box_table<true>, g, b, lds, st, p);
+  else hipLaunchKernelGGL(k_box_table<false>, g, b, lds, st, p);
+  return (int)hipGetLastError();
+}
+
 __global__ void k_box_dist_clear(unsigned* scal) { scal[0] = 0u; }
 
 // max |ddist| (bit pattern of a non-negative float orders like the unsigned integer)

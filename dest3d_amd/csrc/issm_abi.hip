@@ -49,6 +49,7 @@ int launch_linear(LinearP& p, int njobs, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwP& p, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
+int launch_box_table(const BoxTableP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
                       hipStream_t st);
@@ -759,6 +760,17 @@ static int box_dist_params(const issm_box_dist_args* a, BoxDistP* p, bool bwd) {
 int64_t issm_box_dist_bwd_scratch_bytes(int32_t batch, int32_t seqlen, int32_t nquery, int32_t D, int32_t H, int32_t W) {
   if (batch <= 0 || seqlen <= 0 || nquery <= 0 || D <= 0 || H <= 0 || W <= 0) return 16;
   return box_dist_bwd_scratch_bytes(batch, seqlen, nquery, D, H, W);
+}
+
+int issm_box_table(const issm_box_table_args* a) {
+  if (!a) return fail(ISSM_E_NULL, "box_table: args is NULL");
+  if (a->nodes < 1 || a->hidden < 1 || a->nodes > (1 << 26)) return fail(ISSM_E_SHAPE, "box_table: %d nodes, %d hidden", a->nodes, a->hidden);
+  if (a->hidden > 256) return fail(ISSM_E_UNSUPPORTED, "box_table: %d hidden values (at most 256)", a->hidden);
+  for (int t : {a->dtype, a->coords_dtype})
+    if (t != ISSM_F32 && t != ISSM_BF16) return fail(ISSM_E_DTYPE, "box_table: dtype %d", t);
+  if (!a->coords || !a->w1 || !a->b1 || !a->w2 || !a->table) return fail(ISSM_E_NULL, "box_table: coords/w1/b1/w2/table is NULL");
+  const BoxTableP p{a->nodes, a->hidden, a->dtype, a->coords_dtype, a->coords, a->w1, a->b1, a->w2, a->table};
+  return launched(launch_box_table(p, (hipStream_t)a->stream), "box_table");
 }
 
 int issm_box_dist_fwd(const issm_box_dist_args* a) {

@@ -128,6 +128,12 @@ struct HilbertOrderP {
   long* inverse;  // may be null
 };
 
+// parameters of the encoding's table (box_dist.hip)
+struct BoxTableP {
+  int nodes, hidden, dtype, coords_dtype;
+  const void *coords, *w1, *b1, *w2;
+  float* table;
+};
 // parameters of the box-to-point distance encoding kernels (box_dist.hip)
 struct BoxDistP {
   int B, L, K, D, H, W, dtype, nwg, nwg_bwd;

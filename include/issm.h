@@ -536,6 +536,21 @@ typedef struct issm_box_dist_args {
 
 int64_t issm_box_dist_bwd_scratch_bytes(int32_t batch, int32_t seqlen, int32_t nquery, int32_t D, int32_t H, int32_t W);
 int issm_box_dist_fwd(const issm_box_dist_args* args);
+
+/* The encoding's table (dest_module.py:160-166,191): table[16][nodes] fp32 = W2 relu(W1 coords + b1) at every node, coords
+ * (nodes, 3) of coords_dtype, w1 (hidden, 3), b1 (hidden), w2 (16, hidden) of dtype, all contiguous; coords, hidden values and
+ * results are rounded to dtype.  nodes >= 1, hidden 1 .. 256 (ISSM_E_UNSUPPORTED beyond). */
+typedef struct issm_box_table_args {
+  int32_t nodes, hidden, dtype, coords_dtype;
+  const void* coords;
+  const void* w1;
+  const void* b1;
+  const void* w2;
+  float* table;
+  void* stream;
+} issm_box_table_args;
+
+int issm_box_table(const issm_box_table_args* args);
 int issm_box_dist_bwd(const issm_box_dist_args* args);
 
 /* ---- serialization codes of the key points ------------------------------------------------

@@ -135,6 +135,32 @@ def test_table_gradient_is_bit_reproducible():
                 assert t.grad.abs().max().item() <= 1e-30
 
 
+@pytest.mark.parametrize("quant,rpe_dim", [("bilinear_4_10", 128), ("bilinear_4_3", 7), ("bilinear_2_1", 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_table_without_a_gradient(quant, rpe_dim, dtype):
+    """One kernel for the table's MLP, at node and hidden counts that fill no workgroup, against fp64 with the roundings of the
+    modules: coordinates, hidden values, results.  A hidden value may round the other way (2^-8 of it, through |W2|); sums of
+    hidden products in fp32.  What the kernel is not for goes through the modules: wide MLPs, hooks, gradients."""
+    from dest3d_amd.box_dist import BoxDistFun
+    torch.manual_seed(rpe_dim)
+    m = BoxDistFun(out_dim=16, rpe_quant=quant, rpe_dim=rpe_dim).cuda().to(dtype)
+    assert m._plain_table() is None                      # parameters that want a gradient
+    with torch.no_grad():
+        got = m._plain_table()
+        hook = m.cpb_mlps[1].register_forward_hook(lambda *_: None)
+        assert m._plain_table() is None
+        hook.remove()
+        assert BoxDistFun(out_dim=16, rpe_dim=257).cuda()._plain_table() is None
+        want = m.rpe_table()
+    lin1, _, lin2 = m.cpb_mlps
+    h = (m.relative_coords_table.to(dtype).double() @ lin1.weight.double().t() + lin1.bias.double()).to(dtype).double().relu()
+    ref, mag = (f(h) @ f(lin2.weight.double()).t() for f in (lambda t: t, torch.abs))
+    ref, mag = (t[0].permute(3, 0, 1, 2).cpu() for t in (ref, mag))
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20
+    assert got.shape == want.shape and got.dtype == torch.float32 and got.is_contiguous()
+    assert ((got.double().cpu() - ref).abs() <= u * (mag + ref.abs())).all()
+
+
 def test_box_dist_rejects_unbuilt_shapes():
     import ctypes as C
     from dest3d_amd import _lib as L
