@@ -162,7 +162,7 @@ struct Scan {
   struct Out {
     Tensor y[2], last[2], ws;
   };
-  Out forward(bool want_last, bool forward_only = false) const {
+  Out forward(bool want_last) const {
     issm_scan_args a = args();
     Out o;
     const auto& s = x[0].sizes();
@@ -179,7 +179,7 @@ struct Scan {
     o.ws = fresh({(int64_t)std::max<size_t>(n, 256)}, x[0], at::kByte);
     a.workspace = data(o.ws);
     a.workspace_bytes = (size_t)o.ws.numel();
-    check(forward_only ? issm_scan_fwd_only(&a) : issm_scan_fwd(&a), "issm_scan_fwd");
+    check(issm_scan_fwd(&a), "issm_scan_fwd");
     return o;
   }
 
@@ -519,25 +519,16 @@ bool few_tokens(const Tensor& x, const Tensor& w) {
   return (double)x.numel() * (double)w.size(0) <= FEW_PRODUCTS && x.is_contiguous() && w.is_contiguous() &&
          (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
 }
-// y = x w^T of one or two such pairs; the last of two, x (batch, n, in), gives (batch, out, n) where `turn` is set
-template <size_t N>
-std::array<Tensor, N> linear_few(const std::array<std::pair<Tensor, Tensor>, N>& xw, bool turn = false) {
-  const c10::DeviceGuard guard(xw[0].first.device());
+Tensor linear_few(const Tensor& x, const Tensor& w) {
+  const c10::DeviceGuard guard(x.device());
+  at::DimVector sizes(x.sizes());
+  sizes.back() = w.size(0);
+  Tensor y = fresh(sizes, x, at::kBFloat16);
   issm_linear_args a{};
-  std::array<Tensor, N> y;
-  for (size_t i = 0; i < N; ++i) {
-    const Tensor &x = xw[i].first, &w = xw[i].second;
-    at::DimVector sizes(x.sizes());
-    sizes.back() = w.size(0);
-    const bool turned = turn && i == N - 1;
-    if (turned) std::swap(sizes[1], sizes[2]);
-    y[i] = fresh(sizes, x, at::kBFloat16);
-    a.job[i] = issm_linear_job{data(x), data(w), data(y[i]), x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0),
-                               turned ? (int32_t)x.size(1) : 0};
-  }
-  a.njobs = (int32_t)N;
+  a.job[0] = issm_linear_job{data(x), data(w), data(y), x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0), 0};
+  a.njobs = 1;
   a.dtype = ISSM_BF16;
-  a.stream = stream_of(xw[0].first);
+  a.stream = stream_of(x);
   check(issm_linear_fwd(&a), "issm_linear_fwd");
   return y;
 }
@@ -574,7 +565,7 @@ Tensor linear_dw(const Tensor& x, const Tensor& dy) {
 struct LinearFn : public Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
     ctx->save_for_backward({x, w});
-    if (few_tokens(x, w)) return linear_few<1>({{{x, w}}})[0];
+    if (few_tokens(x, w)) return linear_few(x, w);
     return at::linear(x, w);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
@@ -674,46 +665,15 @@ issm_pgen_args pgen_args(const Tensor& dist, const float* W, int64_t H, int64_t 
 struct CoreFn : public Function<CoreFn> {
   // the small parameters, in the order of their places in the flat fp32 buffer
   enum { CW_F, CW_B, CB_F, CB_B, DT_W, BC_W, DT_BIAS, A_LOG, D_, NSMALL };
-  // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
-  static constexpr int NIN = 14;
-  struct Record : torch::CustomClassHolder {
-    Kind in[NIN];
-    int64_t H, G, di;
-    double lo, hi, eps;
-  };
-
-  // Without a gradient (scan_layer): h0_lin is (B, d_inner, K) already, and query_norm belongs to what one launch makes of the
-  // scan's results (issm_layer_out).
-  struct Plain {
-    Tensor query_w, query_b;
-    double query_eps;
-  };
-
-  static variable_list forward(AutogradContext* ctx, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
-                               const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
-                               const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
-                               const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
-                               int64_t ngroups, double lo, double hi, double eps) {
-    return run(ctx, nullptr, zxbcdt, h0_lin, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
-               norm_w, d_inner, nheads, ngroups, lo, hi, eps);
-  }
-
-  // one of ctx and plain
-  static variable_list run(AutogradContext* ctx, const Plain* plain, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
-                           const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
-                           const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
-                           const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
-                           int64_t ngroups, double lo, double hi, double eps) {
-    const c10::DeviceGuard guard(zxbcdt.device());
-    const Tensor weights = opt(weights_);
-    const int64_t Bsz = zxbcdt.size(0), Ln = zxbcdt.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
-                  K = dist.size(2);
-    const at::ScalarType k = kernel_type(zxbcdt.scalar_type());
-    // (the kernels address the parameters by the layer's sizes: none may be smaller than its place)
+  // (the kernels address the parameters by the layer's sizes: none may be smaller than its place)
+  static void check_sizes(int64_t features, const Tensor& conv_w_f, const Tensor& conv_w_b, const Tensor& conv_b_f,
+                          const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias, const Tensor& A_log,
+                          const Tensor& D, const Tensor& norm_w, int64_t di, int64_t H, int64_t G) {
+    const int64_t Cc = di + 2 * G;
     auto has = [](const Tensor& t, int64_t n, const char* name) {
       TORCH_CHECK(t.numel() == n, name, " must have ", n, " entries, got ", t.numel());
     };
-    TORCH_CHECK(zxbcdt.size(2) == di + Cc + H, "key_proj must give ", di + Cc + H, " features, got ", zxbcdt.size(2));
+    TORCH_CHECK(features == di + Cc + H, "key_proj must give ", di + Cc + H, " features, got ", features);
     has(conv_w_f, Cc * TAPS, "key_conv.weight");
     has(conv_w_b, Cc * TAPS, "key_conv_back.weight");
     has(conv_b_f, Cc, "key_conv.bias");
@@ -722,34 +682,60 @@ struct CoreFn : public Function<CoreFn> {
     has(bc_w, 2 * G * WIDTH, "bc_proj.weight");
     has(dt_bias, H, "dt_bias");
     has(A_log, H, "A_log");
-    has(D, D.dim() == 1 ? H : H * P, "D");
+    has(D, D.dim() == 1 ? H : di, "D");
     has(norm_w, di, "key_norm.weight");
+  }
+  // places of the arrays in the flat buffer; its length
+  static int64_t offsets(const std::array<const Tensor*, NSMALL>& arrays, int64_t (&off)[NSMALL + 1]) {
+    off[0] = 0;
+    for (int i = 0; i < NSMALL; ++i) off[i + 1] = off[i] + arrays[i]->numel();
+    return off[NSMALL];
+  }
+  static void small_parameters(const std::array<const Tensor*, NSMALL>& arrays, int64_t K, float* flat, float* A, void* stream) {
+    static_assert(NSMALL == ISSM_LAYER_ARRAYS, "one array per parameter");
+    issm_layer_params_args a{};
+    Tensor kept[NSMALL];
+    for (int i = 0; i < NSMALL; ++i) {
+      kept[i] = cast(*arrays[i], kernel_type(arrays[i]->scalar_type())).contiguous();
+      a.src[i] = data(kept[i]);
+      a.n[i] = (int32_t)kept[i].numel();
+      a.dtype[i] = code(kept[i].scalar_type());
+    }
+    a.a_log = A_LOG;
+    a.K = (int32_t)K;
+    a.out = flat;
+    a.A = A;
+    a.stream = stream;
+    check(issm_layer_params(&a), "issm_layer_params");
+  }
+
+  // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
+  static constexpr int NIN = 14;
+  struct Record : torch::CustomClassHolder {
+    Kind in[NIN];
+    int64_t H, G, di;
+    double lo, hi, eps;
+  };
+
+  static variable_list forward(AutogradContext* ctx, const Tensor& zxbcdt, const Tensor& h0_lin, const Tensor& dist,
+                               const MaybeTensor& weights_, const Tensor& conv_w_f, const Tensor& conv_b_f, const Tensor& conv_w_b,
+                               const Tensor& conv_b_b, const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias,
+                               const Tensor& A_log, const Tensor& D, const Tensor& norm_w, int64_t d_inner, int64_t nheads,
+                               int64_t ngroups, double lo, double hi, double eps) {
+    const c10::DeviceGuard guard(zxbcdt.device());
+    const Tensor weights = opt(weights_);
+    const int64_t Bsz = zxbcdt.size(0), Ln = zxbcdt.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
+                  K = dist.size(2);
+    const at::ScalarType k = kernel_type(zxbcdt.scalar_type());
+    check_sizes(zxbcdt.size(2), conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w, di, H, G);
     Tensor zx = io_cast(zxbcdt, k);
     const Tensor z = zx.narrow(2, 0, di), xbc = zx.narrow(2, di, Cc);
     // all small parameters in one fp32 buffer, and A for all state columns; adjacent pieces form the stacked operands the
     // kernels take
-    static_assert(NSMALL == ISSM_LAYER_ARRAYS, "one array per parameter");
-    int64_t off[NSMALL + 1] = {0};
-    Tensor flat, A1 = fresh({H, K}, zx, at::kFloat);
-    {
-      issm_layer_params_args a{};
-      std::vector<Tensor> small;
-      for (const Tensor& t : {conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log, D}) {
-        const size_t i = small.size();
-        off[i + 1] = off[i] + t.numel();
-        small.push_back(cast(t, kernel_type(t.scalar_type())).contiguous());
-        a.src[i] = data(small[i]);
-        a.n[i] = (int32_t)t.numel();
-        a.dtype[i] = code(small[i].scalar_type());
-      }
-      flat = fresh({off[NSMALL]}, zx, at::kFloat);
-      a.a_log = A_LOG;
-      a.K = (int32_t)K;
-      a.out = data<float>(flat);
-      a.A = data<float>(A1);
-      a.stream = stream_of(zx);
-      check(issm_layer_params(&a), "issm_layer_params");
-    }
+    int64_t off[NSMALL + 1];
+    const std::array<const Tensor*, NSMALL> arrays{&conv_w_f, &conv_w_b, &conv_b_f, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D};
+    Tensor flat = fresh({offsets(arrays, off)}, zx, at::kFloat), A1 = fresh({H, K}, zx, at::kFloat);
+    small_parameters(arrays, K, data<float>(flat), data<float>(A1), stream_of(zx));
     float* const par = data<float>(flat);
     // 1. both depthwise convolutions + SiLU; the conv writes x and the B / C biases apart
     Tensor x = fresh({2, Bsz, Ln, H, P}, zx, k), tail = fresh({2, Bsz, Ln, 2 * G}, zx, k), pre = fresh({2, Bsz, Ln, Cc}, zx, k);
@@ -783,38 +769,13 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
     }
     // 3. the bidirectional scan, queries as initial state
-    const Tensor h0 = (plain ? h0_lin : transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0,
-                                                         kernel_type(h0_lin.scalar_type()))).view({Bsz, H, P, K});
+    const Tensor h0 = transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()))
+                          .view({Bsz, H, P, K});
     const Tensor xs[2] = {x.select(0, 0), x.select(0, 1)}, Bs[2] = {bc.select(0, 0), bc.select(0, 2)},
                  Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
     const Scan s = Scan::make(2, xs, dt, A1, Bs, Cs, D.dim() == 1 ? flat.narrow(0, off[D_], H) : D, none, Tensor(), h0,
                               Tensor(), !wt.defined(), lo, hi);
-    Scan::Out o = s.forward(true, plain != nullptr);
-    if (plain) {
-      Tensor key = fresh({Bsz, Ln, di}, zx, k), query = fresh({Bsz, K, di}, zx, k);
-      issm_layer_out_args a{};
-      a.batch = (int32_t)Bsz;
-      a.seqlen = (int32_t)Ln;
-      a.queries = (int32_t)K;
-      a.d_inner = (int32_t)di;
-      a.dtype = ISSM_BF16;
-      for (int i = 0; i < 2; ++i) {
-        a.y[i] = data(o.y[i]);
-        a.last[i] = data<const float>(o.last[i]);
-      }
-      a.z = data(z);
-      a.z_row_stride = zx.stride(1);
-      a.key_weight = data(norm_w);
-      a.key_eps = (float)(4.0 * eps);
-      a.key = data(key);
-      a.query_weight = data(plain->query_w);
-      a.query_bias = data(plain->query_b);
-      a.query_eps = (float)plain->query_eps;
-      a.query = data(query);
-      a.stream = stream_of(zx);
-      check(issm_layer_out(&a), "issm_layer_out");
-      return {key, query};
-    }
+    Scan::Out o = s.forward(true);
     // 4. gated RMSNorm (norm(x * silu(z))) of the two directions' average: the norm of s / 2 with eps is the norm of s with
     // 4 eps, so the sum goes in as it is and the halving never runs (nor its backward)
     const Tensor key = at::add(o.y[0], o.y[1]).view({Bsz * Ln, di});
@@ -1008,12 +969,131 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     plain = !t->defined() || (own_memory(*t) && !(at::GradMode::is_enabled() && t->requires_grad()) && !t->_fw_grad(0).defined());
   }
   if (plain) {
-    auto [zx, h0] = linear_few<2>({{{in_key, key_proj}, {in_query, query_proj}}}, true);
-    const CoreFn::Plain p{query_wt, query_bt, query_eps};
-    variable_list core = CoreFn::run(nullptr, &p, zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias,
-                                     A_log, D, key_norm, d_inner, nheads, ngroups, lo, hi, key_eps);
-    auto [key, query] = linear_few<2>({{{core[0], out_key_proj}, {core[1], out_query_proj}}});
-    return {key, query};
+    const c10::DeviceGuard guard(in_key.device());
+    const int64_t B = in_key.size(0), Ln = in_key.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,
+                  K = dist.size(2), W = key_proj.size(0);
+    CoreFn::check_sizes(W, conv_w_f, conv_w_b, conv_b_f, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, key_norm, di, H, G);
+    void* const stream = stream_of(in_key);
+    issm_scan_args s{};
+    s.dims = issm_dims{(int32_t)B, (int32_t)Ln, (int32_t)H, (int32_t)P, (int32_t)K, (int32_t)G, ISSM_CHUNK, 2};
+    s.io_dtype = s.dt_dtype = s.h0_dtype = ISSM_BF16;
+    size_t ws_bytes = 0;
+    check(issm_fwd_workspace_bytes(&s, &ws_bytes), "workspace query");
+    // one allocation for all that lies between the inputs and the outputs (seventeen were 24 us of host time)
+    int64_t off[CoreFn::NSMALL + 1];
+    const std::array<const Tensor*, CoreFn::NSMALL> arrays{&conv_w_f, &conv_w_b, &conv_b_f, &conv_b_b, &dt_w, &bc_w, &dt_bias,
+                                                           &A_log, &D};
+    const int64_t nflat = CoreFn::offsets(arrays, off);
+    const Tensor d = cast(dist, at::kBFloat16).contiguous(), wt = f32c(wts);
+    enum { ZX, H0, FLAT, A1, X, TAIL, PRE, DT, BC, RAW, Y, LAST, KEY, QUERY, WS, PARTS };
+    const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di, 8 * B * Ln * G, 4 * B * Ln * Cc,
+                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, wt.defined() ? 2 * B * Ln * H * K : 0, 4 * B * Ln * di,
+                                  8 * B * di * K, 2 * B * Ln * di, 2 * B * K * di, (int64_t)ws_bytes};
+    int64_t at_[PARTS + 1] = {0};
+    for (int i = 0; i < PARTS; ++i) at_[i + 1] = at_[i] + (bytes[i] + 255) / 256 * 256;
+    const Tensor arena = fresh({at_[PARTS]}, in_key, at::kByte);
+    char* const base = data<char>(arena);
+    auto part = [&](int i, int64_t byte = 0) -> void* { return base + at_[i] + byte; };
+    float *const par = (float*)part(FLAT), *const last = (float*)part(LAST);
+    // the projections, the queries' into the layout of the scan's states
+    auto product = [&](const Tensor& x, const void* px, const Tensor& w, void* y, int64_t turn) {
+      return issm_linear_job{px, data(w), y, x.numel() / x.size(-1), (int32_t)w.size(1), (int32_t)w.size(0), (int32_t)turn};
+    };
+    issm_linear_args lin{};
+    lin.njobs = 2;
+    lin.dtype = ISSM_BF16;
+    lin.stream = stream;
+    lin.job[0] = product(in_key, data(in_key), key_proj, part(ZX), 0);
+    lin.job[1] = product(in_query, data(in_query), query_proj, part(H0), K);
+    check(issm_linear_fwd(&lin), "issm_linear_fwd");
+    CoreFn::small_parameters(arrays, K, par, (float*)part(A1), stream);
+    {
+      issm_dwconv_args a{};
+      a.batch = (int32_t)B;
+      a.seqlen = (int32_t)Ln;
+      a.channels = (int32_t)Cc;
+      a.nsets = 2;
+      a.taps = TAPS;
+      a.dtype = ISSM_BF16;
+      a.u = part(ZX, 2 * di);
+      a.u_batch_stride = Ln * W;
+      a.u_token_stride = W;
+      a.chain = 1;
+      a.stream = stream;
+      a.w = par;
+      a.bias = par + off[CoreFn::CB_F];
+      a.y = part(X);
+      a.pre = part(PRE);
+      a.split = (int32_t)di;
+      a.y_tail = part(TAIL);
+      check(issm_dwconv_silu_fwd(&a), "issm_dwconv_silu_fwd");
+    }
+    void* bc[4];
+    for (int i = 0; i < 4; ++i) bc[i] = part(BC, i * 2 * B * Ln * G * K);
+    {
+      issm_pgen_args a = pgen_args(d, par + off[CoreFn::DT_W], H, G);
+      a.tok = part(ZX, 2 * (di + Cc));
+      a.tok_stride = W;
+      a.tok_add = par + off[CoreFn::DT_BIAS];
+      a.tail = part(TAIL);
+      a.dt = part(DT);
+      a.Bm = bc[0];
+      a.Cm = bc[1];
+      a.Bm_back = bc[2];
+      a.Cm_back = bc[3];
+      if (wt.defined()) {
+        a.weights = data<const float>(wt);
+        a.dt_raw = part(RAW);
+      }
+      check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
+    }
+    s.flags = (wt.defined() ? 0u : ISSM_FLAG_DT_SOFTPLUS) | (D.dim() == 2 ? ISSM_FLAG_D_HAS_HDIM : 0u);
+    s.dt_min = (float)lo;
+    s.dt_max = (float)std::min(hi, 3.0e38);
+    for (int i = 0; i < 2; ++i) {
+      s.x[i] = issm_tensor{part(X, i * 2 * B * Ln * di), {Ln * di, di, P}};
+      s.Bm[i] = issm_tensor{bc[2 * i], {Ln * G * K, G * K, K}};
+      s.Cm[i] = issm_tensor{bc[2 * i + 1], {Ln * G * K, G * K, K}};
+      s.out[i] = issm_tensor{part(Y, i * 2 * B * Ln * di), {Ln * di, di, P}};
+      s.final_states[i] = last + i * B * di * K;
+    }
+    s.dt = issm_tensor{part(DT), {Ln * H * K, H * K, K}};
+    s.h0 = issm_tensor{part(H0), {di * K, P * K, K}};
+    s.A = (const float*)part(A1);
+    s.D = par + off[CoreFn::D_];
+    s.workspace = part(WS);
+    s.workspace_bytes = ws_bytes;
+    s.stream = stream;
+    check(issm_scan_fwd_only(&s), "issm_scan_fwd_only");
+    {
+      issm_layer_out_args a{};
+      a.batch = (int32_t)B;
+      a.seqlen = (int32_t)Ln;
+      a.queries = (int32_t)K;
+      a.d_inner = (int32_t)di;
+      a.dtype = ISSM_BF16;
+      for (int i = 0; i < 2; ++i) {
+        a.y[i] = s.out[i].ptr;
+        a.last[i] = s.final_states[i];
+      }
+      a.z = part(ZX);
+      a.z_row_stride = W;
+      a.key_weight = data(key_norm);
+      a.key_eps = (float)(4.0 * key_eps);
+      a.key = part(KEY);
+      a.query_weight = data(query_wt);
+      a.query_bias = data(query_bt);
+      a.query_eps = (float)query_eps;
+      a.query = part(QUERY);
+      a.stream = stream;
+      check(issm_layer_out(&a), "issm_layer_out");
+    }
+    const Tensor out_key = fresh({B, Ln, out_key_proj.size(0)}, in_key, at::kBFloat16),
+                 out_query = fresh({B, K, out_query_proj.size(0)}, in_key, at::kBFloat16);
+    lin.job[0] = product(in_key, part(KEY), out_key_proj, data(out_key), 0);
+    lin.job[1] = product(in_query, part(QUERY), out_query_proj, data(out_query), 0);
+    check(issm_linear_fwd(&lin), "issm_linear_fwd");
+    return {out_key, out_query};
   }
   const Tensor zx = linear_tokens(in_key, key_proj), h0 = linear_tokens(in_query, query_proj);
   variable_list core = CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D,
