@@ -28,7 +28,7 @@ FLAGS = [
 #    -ffast-math the backend fuses multiply and add whatever `#pragma clang fp contract(off)` says, and a distance one
 #    unit in the last place off decides a near-tie differently from a plain fp32 evaluation.
 # and one that computes no more than a few exponentials, which are to be the accurate ones: layer_params.hip.
-EXACT_ARITHMETIC = {"hilbert.hip", "pointnet2_ops.hip", "layer_params.hip"}
+EXACT_ARITHMETIC = {"hilbert.hip", "pointnet2_ops.hip", "layer_params.hip", "linear.hip"}
 
 
 def _compile(src: str) -> str:

@@ -691,7 +691,8 @@ struct CoreFn : public Function<CoreFn> {
     for (int i = 0; i < NSMALL; ++i) off[i + 1] = off[i] + arrays[i]->numel();
     return off[NSMALL];
   }
-  static void small_parameters(const std::array<const Tensor*, NSMALL>& arrays, int64_t K, float* flat, float* A, void* stream) {
+  static void small_parameters(const std::array<const Tensor*, NSMALL>& arrays, int64_t K, float* flat, float* A, void* stream,
+                               const issm_linear_args* with = nullptr) {   // with: in the products' launch
     static_assert(NSMALL == ISSM_LAYER_ARRAYS, "one array per parameter");
     issm_layer_params_args a{};
     Tensor kept[NSMALL];
@@ -706,7 +707,7 @@ struct CoreFn : public Function<CoreFn> {
     a.out = flat;
     a.A = A;
     a.stream = stream;
-    check(issm_layer_params(&a), "issm_layer_params");
+    check(with ? issm_layer_in(with, &a) : issm_layer_params(&a), "issm_layer_params");
   }
 
   // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
@@ -947,9 +948,9 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
   check_core(in_key, in_query, dist, opt(weights_));
   py::gil_scoped_release release;
-  // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, nine
-  // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 ->
-  // 659 us).
+  // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, eight
+  // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us ->
+  // 576).
   // With many tokens the products are the library's, and the launches are not what counts.
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
   auto plain_bf16 = [&](const Tensor& t) {
@@ -985,9 +986,9 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                                            &A_log, &D};
     const int64_t nflat = CoreFn::offsets(arrays, off);
     const Tensor d = cast(dist, at::kBFloat16).contiguous(), wt = f32c(wts);
-    enum { ZX, H0, FLAT, A1, X, TAIL, PRE, DT, BC, RAW, Y, LAST, KEY, QUERY, WS, PARTS };
+    enum { ZX, H0, FLAT, A1, X, TAIL, PRE, DT, BC, Y, LAST, KEY, QUERY, WS, PARTS };
     const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di, 8 * B * Ln * G, 4 * B * Ln * Cc,
-                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, wt.defined() ? 2 * B * Ln * H * K : 0, 4 * B * Ln * di,
+                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di,
                                   8 * B * di * K, 2 * B * Ln * di, 2 * B * K * di, (int64_t)ws_bytes};
     int64_t at_[PARTS + 1] = {0};
     for (int i = 0; i < PARTS; ++i) at_[i + 1] = at_[i] + (bytes[i] + 255) / 256 * 256;
@@ -1005,8 +1006,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     lin.stream = stream;
     lin.job[0] = product(in_key, data(in_key), key_proj, part(ZX), 0);
     lin.job[1] = product(in_query, data(in_query), query_proj, part(H0), K);
-    check(issm_linear_fwd(&lin), "issm_linear_fwd");
-    CoreFn::small_parameters(arrays, K, par, (float*)part(A1), stream);
+    CoreFn::small_parameters(arrays, K, par, (float*)part(A1), stream, &lin);
     {
       issm_dwconv_args a{};
       a.batch = (int32_t)B;
@@ -1041,11 +1041,8 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
       a.Cm = bc[1];
       a.Bm_back = bc[2];
       a.Cm_back = bc[3];
-      if (wt.defined()) {
-        a.weights = data<const float>(wt);
-        a.dt_raw = part(RAW);
-      }
-      check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
+      a.weights = data<const float>(wt);
+      check(issm_param_gen_fwd_only(&a), "issm_param_gen_fwd_only");
     }
     s.flags = (wt.defined() ? 0u : ISSM_FLAG_DT_SOFTPLUS) | (D.dim() == 2 ? ISSM_FLAG_D_HAS_HDIM : 0u);
     s.dt_min = (float)lo;

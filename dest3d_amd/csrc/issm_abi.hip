@@ -45,7 +45,7 @@ struct TrP {
 };
 int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
-int launch_linear(LinearP& p, int njobs, hipStream_t st);
+int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwP& p, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
@@ -632,7 +632,7 @@ int issm_gated_rmsnorm_bwd_noalloc(const issm_norm_args* a) {
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_noalloc");
 }
 
-static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd) {
+static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward_only = false) {
   if (!a) return fail(ISSM_E_NULL, "param_gen: args is NULL");
   if (a->tokens < 0 || a->K < 0 || a->H < 1 || a->G < 1) return fail(ISSM_E_SHAPE, "param_gen: bad shape");
   if (a->M != 16) return fail(ISSM_E_UNSUPPORTED, "param_gen: M = %d (only 16 is built)", a->M);
@@ -640,7 +640,7 @@ static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd) {
   if (a->dtype != ISSM_F32 && a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "param_gen: dtype %d", a->dtype);
   if (a->tokens * (int64_t)a->K * 16 >= ((int64_t)1 << 40)) return fail(ISSM_E_SHAPE, "param_gen: too large");
   if (!a->dist || !a->W) return fail(ISSM_E_NULL, "param_gen: dist/W is NULL");
-  if (a->weights && !a->dt_raw) return fail(ISSM_E_NULL, "param_gen: weights given but dt_raw is NULL");
+  if (a->weights && !a->dt_raw && !forward_only) return fail(ISSM_E_NULL, "param_gen: weights given but dt_raw is NULL");
   if (!bwd) {
     if (!a->dt || !a->Bm || !a->Cm) return fail(ISSM_E_NULL, "param_gen: dt/Bm/Cm is NULL");
     if (!a->bias && (!a->tok || !a->tok_add || !a->tail)) return fail(ISSM_E_NULL, "param_gen: neither bias nor tok/tok_add/tail");
@@ -670,6 +670,15 @@ int issm_param_gen_fwd(const issm_pgen_args* a) {
   if (rc) return rc;
   if (p.tokens == 0 || p.K == 0) return ISSM_OK;
   return launched(launch_pgen_fwd(p, (hipStream_t)a->stream), "param_gen_fwd");
+}
+
+int issm_param_gen_fwd_only(const issm_pgen_args* a) {
+  PGenP p;
+  int rc = pgen_params(a, &p, false, true);
+  if (rc) return rc;
+  if (p.tokens == 0 || p.K == 0) return ISSM_OK;
+  p.dt_raw = nullptr;
+  return launched(launch_pgen_fwd(p, (hipStream_t)a->stream), "param_gen_fwd_only");
 }
 
 int issm_param_gen_bwd(const issm_pgen_args* a) {
@@ -789,11 +798,10 @@ int issm_box_dist_bwd(const issm_box_dist_args* a) {
   return launched(launch_box_dist_bwd(p, (hipStream_t)a->stream), "box_dist_bwd");
 }
 
-int issm_layer_params(const issm_layer_params_args* a) {
+static int layer_params(const issm_layer_params_args* a, LayerParamsP& p) {
   static_assert(LAYER_ARRAYS == ISSM_LAYER_ARRAYS, "one count");
   if (!a) return fail(ISSM_E_NULL, "layer_params: args is NULL");
   if (a->a_log < 0 || a->a_log >= LAYER_ARRAYS || a->K < 0) return fail(ISSM_E_SHAPE, "layer_params: a_log %d, K %d", a->a_log, a->K);
-  LayerParamsP p;
   int64_t total = 0;
   for (int i = 0; i < LAYER_ARRAYS; ++i) {
     if (a->n[i] < 0) return fail(ISSM_E_SHAPE, "layer_params: n[%d] = %d", i, a->n[i]);
@@ -805,17 +813,22 @@ int issm_layer_params(const issm_layer_params_args* a) {
   p.a_log = a->a_log; p.H = a->n[a->a_log]; p.K = a->K; p.out = a->out; p.A = a->A;
   if (total + (int64_t)p.H * p.K > ((int64_t)1 << 30)) return fail(ISSM_E_SHAPE, "layer_params: too large");
   p.total = (int)total;
-  if (total == 0) return ISSM_OK;
-  if (!a->out || !a->A) return fail(ISSM_E_NULL, "layer_params: out/A is NULL");
+  if (total && (!a->out || !a->A)) return fail(ISSM_E_NULL, "layer_params: out/A is NULL");
+  return ISSM_OK;
+}
+
+int issm_layer_params(const issm_layer_params_args* a) {
+  LayerParamsP p;
+  const int rc = layer_params(a, p);
+  if (rc || p.total == 0) return rc;
   return launched(launch_layer_params(p, (hipStream_t)a->stream), "layer_params");
 }
 
-int issm_linear_fwd(const issm_linear_args* a) {
+static int linear_params(const issm_linear_args* a, LinearP& p, int& n) {
   if (!a) return fail(ISSM_E_NULL, "linear: args is NULL");
   if (a->njobs < 0 || a->njobs > ISSM_LINEAR_JOBS) return fail(ISSM_E_SHAPE, "linear: %d products (0..%d)", a->njobs, ISSM_LINEAR_JOBS);
   if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "linear: dtype %d (bf16 only)", a->dtype);
-  LinearP p{};
-  int n = 0;
+  n = 0;
   for (int i = 0; i < a->njobs; ++i) {
     const issm_linear_job& j = a->job[i];
     if (j.tokens < 0 || j.in < 0 || j.out < 0 || j.tokens > 0x7fffffff - 64 || j.out > 0x7fffffff - 64)
@@ -828,8 +841,27 @@ int issm_linear_fwd(const issm_linear_args* a) {
     if (j.turn < 0 || (j.turn && j.tokens % j.turn)) return fail(ISSM_E_SHAPE, "linear: %lld tokens, turned by %d", (long long)j.tokens, j.turn);
     p.job[n++] = LinearJob{(const uint16_t*)j.x, (const uint16_t*)j.w, (uint16_t*)j.y, (int)j.tokens, j.out, j.in / 32, 0, j.turn};
   }
-  if (n == 0) return ISSM_OK;
-  return launched(launch_linear(p, n, (hipStream_t)a->stream), "linear_fwd");
+  return ISSM_OK;
+}
+
+int issm_linear_fwd(const issm_linear_args* a) {
+  LinearP p{};
+  int n;
+  const int rc = linear_params(a, p, n);
+  if (rc || n == 0) return rc;
+  return launched(launch_linear(p, n, nullptr, (hipStream_t)a->stream), "linear_fwd");
+}
+
+int issm_layer_in(const issm_linear_args* a, const issm_layer_params_args* b) {
+  LinearP p{};
+  LayerParamsP q;
+  int n, rc = linear_params(a, p, n);
+  if (rc || (rc = layer_params(b, q))) return rc;
+  if (n == 0 || q.total == 0) {   // (nothing to join)
+    if (n && (rc = issm_linear_fwd(a))) return rc;
+    return q.total ? issm_layer_params(b) : ISSM_OK;
+  }
+  return launched(launch_linear(p, n, &q, (hipStream_t)a->stream), "layer_in");
 }
 
 static bool linear_dw_sizes(int64_t tokens, int32_t in, int32_t out) {

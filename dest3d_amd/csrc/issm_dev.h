@@ -187,7 +187,7 @@ struct LinearJob {
 };
 struct LinearP {
   LinearJob job[2];
-  int blocks0;   // of the first
+  int blocks0, blocks1;   // of the first, of both
 };
 // parameters of the projections' weight gradient (linear_dw.hip)
 struct LinearDwP {

@@ -9,7 +9,7 @@
 // of 16 bytes a lane at 288 features) and multiplies as they arrive; there is nothing to share through LDS that L1 does not
 // share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens or features the fragments' 64-byte pieces
 // of 16 rows a load are what it pays for, and staging tiles through LDS wins: 8192 x 288 -> 586 21 us (13.5).
-#include "issm_dev.h"
+#include "layer_params.h"
 
 namespace issm {
 
@@ -85,15 +85,35 @@ __global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
   else linear_block<N, false>(j, bid);
 }
 
-int launch_linear(LinearP& p, int njobs, hipStream_t st) {
+// The products and, in the blocks behind theirs, the layer's small parameters (issm_layer_in): 7.6 us where the two launches
+// took 6.8 and 3.1.
+// (Compiled without -ffast-math for its exp.)
+template <int N>
+__global__ __launch_bounds__(NTHREADS) void k_layer_in(LinearP p, LayerParamsP q) {
+  if ((int)blockIdx.x >= p.blocks1) return layer_params_entry(q, ((int)blockIdx.x - p.blocks1) * NTHREADS + threadIdx.x);
+  const bool second = (int)blockIdx.x >= p.blocks0;
+  const LinearJob& j = p.job[second ? 1 : 0];
+  const int bid = (int)blockIdx.x - (second ? p.blocks0 : 0);
+  if (j.turn) linear_block<N, true>(j, bid);
+  else linear_block<N, false>(j, bid);
+}
+
+int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st) {
   long blocks[2] = {0, 0};
   for (int k = 0; k < njobs; ++k) {
     p.job[k].oblocks = (p.job[k].out + 31) / 32;
     blocks[k] = (long)((p.job[k].tokens + 63) / 64) * p.job[k].oblocks;
   }
-  if (blocks[0] + blocks[1] > 0x7fffffff) return (int)hipErrorInvalidValue;
+  const long params = q ? ((long)q->total + q->H * q->K + NTHREADS - 1) / NTHREADS : 0;
+  if (blocks[0] + blocks[1] + params > 0x7fffffff) return (int)hipErrorInvalidValue;
   p.blocks0 = (int)blocks[0];
-  const dim3 grid((unsigned)(blocks[0] + blocks[1])), block(NTHREADS);
+  p.blocks1 = (int)(blocks[0] + blocks[1]);
+  const dim3 grid((unsigned)(blocks[0] + blocks[1] + params)), block(NTHREADS);
+  if (q) {
+    if (p.job[0].steps % 9 == 0) hipLaunchKernelGGL(k_layer_in<9>, grid, block, 0, st, p, *q);
+    else hipLaunchKernelGGL(k_layer_in<8>, grid, block, 0, st, p, *q);
+    return (int)hipGetLastError();
+  }
   // nine fragments where they come out even (288 features), eight otherwise
   if (p.job[0].steps % 9 == 0) hipLaunchKernelGGL(k_linear<9>, grid, block, 0, st, p);
   else hipLaunchKernelGGL(k_linear<8>, grid, block, 0, st, p);

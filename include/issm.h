@@ -363,6 +363,8 @@ int issm_layer_params(const issm_layer_params_args* args);
 
 int issm_param_gen_bwd_blocks(int64_t tokens);
 int issm_param_gen_fwd(const issm_pgen_args* args);
+/* The same for a call that no backward follows: dt_raw is neither needed nor written. */
+int issm_param_gen_fwd_only(const issm_pgen_args* args);
 int issm_param_gen_bwd(const issm_pgen_args* args);
 
 /* ---- depthwise 7-tap convolution along the token order + SiLU -------------------------
@@ -431,6 +433,8 @@ typedef struct issm_linear_args {
 } issm_linear_args;
 
 int issm_linear_fwd(const issm_linear_args* args);
+/* issm_linear_fwd and issm_layer_params in one launch, on the products' stream; neither may read what the other writes. */
+int issm_layer_in(const issm_linear_args* products, const issm_layer_params_args* params);
 
 /* dw = dy^T x: dy (tokens, out), x (tokens, in), dw (out, in), contiguous, ISSM_BF16, sums in fp32 in an order that depends on
  * the sizes alone; in >= 6, out >= 4.  scratch: issm_linear_dw_scratch_bytes, aligned to 16 bytes. */
