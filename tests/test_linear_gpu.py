@@ -239,3 +239,28 @@ def test_layer_without_a_gradient(B, Ln, K, mask):
     layer.requires_grad_(False)
     frozen = layer(key, query, dist, None, m)
     assert all(torch.equal(a, b) for a, b in zip(frozen, got))
+
+
+def test_layer_without_a_gradient_in_a_graph():
+    """The shorter chain recorded into a HIP graph: every replay, with eager work and other inputs between, gives the eager result."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(3)
+    layer = MultiHeadISSMScan(d_model=288, d_state=64, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    x = [bf(1, 200, 288), bf(1, 64, 288), bf(1, 200, 64, 16)]
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            layer(*x, None, None)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = layer(*x, None, None)
+        for _ in range(4):
+            for t in x:
+                t.copy_(bf(*t.shape))
+            want = layer(*x, None, None)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(out, want))
