@@ -85,6 +85,7 @@ template <bool BF>
 __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_points) {
   __shared__ __attribute__((aligned(16))) float tab[BD_MAXCELLS * BD_NS];
   __shared__ unsigned short queue[BD_FWD_T / 64][BD_SEG];
+  __shared__ int queue_len[BD_FWD_T / 64];
   const int cells = p.D * p.H * p.W;
   for (int e = threadIdx.x; e < cells * BD_C; e += BD_FWD_T) {
     const int ch = e / cells, cell = e - ch * cells;
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
   const int kgroup = blockIdx.x % kgroups, bs = blockIdx.x / kgroups;
   const int b = bs / npair, k = kgroup * 8 + (wave & 7);
   const int l0 = (2 * (bs % npair) + (wave >> 3)) * seg_points, n = min(seg_points, p.L - l0);
-  const bool live = k < p.K && n > 0;  // uniform per wave
+  const bool live = k < p.K;  // uniform per wave (n may be 0 or less)
   const float scale = 1.0f / (3.0f * p.max_value);
   BoxLane bx;
   int queued = 0;
@@ -130,11 +131,15 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       queued += __popcll(rest);
     }
   }
+  if (lane == 0) queue_len[wave] = queued;
   __syncthreads();
   if (!live) return;
-  for (int i = lane; i < queued; i += 64) {
-    const int li = queue[wave][i];
-    const float* key = p.key + ((long)b * p.L + l0 + li) * 3;
+  // the box's two waves take the points both have queued in turn, 64 at a time: where the segments are short neither queue fills
+  // a wave (one scene 39 -> BD_ONE us, eight 176 -> BD_EIGHT)
+  const int qa = queue_len[wave & 7], all = qa + queue_len[(wave & 7) + 8], la = 2 * (bs % npair) * seg_points;
+  for (int i = (wave >> 3) * 64 + lane; i < all; i += 128) {
+    const int l = i < qa ? la + queue[wave & 7][i] : la + seg_points + queue[(wave & 7) + 8][i - qa];
+    const float* key = p.key + ((long)b * p.L + l) * 3;
     const float kx = key[0], ky = key[1], kz = key[2];
     f4 acc[4];
 #pragma unroll
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       }
       rotate_box(bx);
     }
-    store_dist<BF>(p, ((long)b * p.L + l0 + li) * p.K + k, acc);
+    store_dist<BF>(p, ((long)b * p.L + l) * p.K + k, acc);
   }
 }
 
