@@ -24,20 +24,24 @@ typedef int i4 __attribute__((ext_vector_type(4)));
 
 constexpr int BDS_SEG = 2048;      // entries per work item
 constexpr int BDS_MAXBINS = 9280;  // (D + 2)(H + 2)(W + 2) for D*H*W <= 1024 is at most 1026 * 3 * 3
-constexpr int BDS_NWG = 512;       // workgroups of the count and fill passes (they must walk identically)
+// Workgroups of the count and fill passes (they must walk identically): four a CU, which the 37 KB of their bins allow, where
+// each has four rows of pairs to walk (8 x 1024 points, 256 boxes: count 66 -> 57 us, fill 73 -> 62), two otherwise: with fewer rows
+// they spend their time on the bins (one scene, count 25 us with two a CU, 36 with four, both still adding up the bins' totals with
+// atomics; without those 53 and 15).
+constexpr int BDS_NWG = 1024;
 constexpr int BDS_OUT = 27 * BD_C; // results per work item
 
 struct SortP {
   unsigned* scal;               // [0] bits of max|ddist|, [1] number of work items
   int* counts;                  // [nbins] entries per bin
   int* binoff;                  // [nbins] first entry of each bin
-  int* wgbase;                  // [BDS_NWG][nbins] counts per workgroup, turned into base positions by the plan
+  int* wgbase;                  // [nwg][nbins] counts per workgroup, turned into base positions within the bin
   int* items;                   // [maxitems][3] bin, first entry, one past the last entry
   unsigned long long* records;  // [maxrecords] pair index | corner mask << 32
   long long* item_out;          // [maxitems][BDS_OUT]
   float* boxtab;                // [B * K][40] corners x, y, z and rotations cos, sin of every box, 8 values each
   long long* dtab;              // [2][cells][16]: sums of the low 32 bits of the items' results, sums of the rest
-  int nbins, maxitems;
+  int nbins, maxitems, nwg;   // nwg: BDS_NWG or half of it
   long maxrecords;
 };
 
@@ -59,7 +63,6 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_clear(BoxDistP p, SortP s) {
   const int cells = p.D * p.H * p.W;
   const int i = blockIdx.x * NTHREADS + threadIdx.x;
   if (i < 4) s.scal[i] = 0u;
-  if (i < s.nbins) s.counts[i] = 0;
   if (i < cells * BD_C) s.dtab[i] = s.dtab[cells * BD_C + i] = 0;
 }
 
@@ -110,11 +113,7 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_count(BoxDistP p, SortP s) {
   __syncthreads();
   bds_walk(p, [&](int bin, unsigned, unsigned) { atomicAdd(&hist[bin], 1); });
   __syncthreads();
-  for (int e = threadIdx.x; e < s.nbins; e += NTHREADS) {
-    const int c = hist[e];
-    s.wgbase[(long)blockIdx.x * s.nbins + e] = c;
-    if (c) atomicAdd(&s.counts[e], c);
-  }
+  for (int e = threadIdx.x; e < s.nbins; e += NTHREADS) s.wgbase[(long)blockIdx.x * s.nbins + e] = hist[e];
 }
 
 // exclusive scan of v[0..n) into out (one workgroup; v and out may alias); returns the total to every thread
@@ -177,19 +176,40 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_plan(SortP s) {
   if (threadIdx.x == 0) s.scal[1] = (unsigned)min(nitems, s.maxitems);
 }
 
-// Base position of every counting workgroup inside every bin: a running sum over the workgroups, in order (thread
-// = bin; 64 loads in flight at a time).
-__global__ __launch_bounds__(64) void k_bds_wgbase(SortP s) {
-  const int e = blockIdx.x * 64 + threadIdx.x;
+// Base position of every counting workgroup inside every bin, and the bins' counts: a running sum over the workgroups, in
+// order.  Lane = bin, wave = a sixteenth of the workgroups, 16 counts in flight; the waves' sums meet in LDS and the counts are
+// read once more (L2).  512 workgroups, 1728 bins: 7.6 us, one wave for all of a bin's 11.3; 1024 workgroups: 13 and 20.
+__global__ __launch_bounds__(1024) void k_bds_wgbase(SortP s) {
+  __shared__ int sums[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = blockIdx.x * 64 + lane, per = s.nwg / 16;
+  unsigned at = (unsigned)(wave * per * s.nbins + min(e, s.nbins - 1));   // (at most 1024 x 9280)
+  const unsigned at0 = at, nb = (unsigned)s.nbins;
+  int sum = 0;
+#pragma unroll 1
+  for (int j0 = 0; j0 < per; j0 += 16) {
+    int c[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j, at += nb) c[j] = s.wgbase[at];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sum += c[j];
+  }
+  sums[wave][lane] = sum;
+  __syncthreads();
   if (e >= s.nbins) return;
-  int run = s.binoff[e];
-  for (int w0 = 0; w0 < BDS_NWG; w0 += 64) {
-    int c[64];
+  int run = 0;
+  for (int w = 0; w < wave; ++w) run += sums[w][lane];
+  if (wave == 15) s.counts[e] = run + sum;
+  at = at0;
+#pragma unroll 1
+  for (int j0 = 0; j0 < per; j0 += 16) {
+    int c[16];
+    const unsigned from = at;
 #pragma unroll
-    for (int j = 0; j < 64; ++j) c[j] = s.wgbase[(long)(w0 + j) * s.nbins + e];
+    for (int j = 0; j < 16; ++j, at += nb) c[j] = s.wgbase[at];
+    at = from;
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      s.wgbase[(long)(w0 + j) * s.nbins + e] = run;
+    for (int j = 0; j < 16; ++j, at += nb) {
+      s.wgbase[at] = run;
       run += c[j];
     }
   }
@@ -197,7 +217,7 @@ __global__ __launch_bounds__(64) void k_bds_wgbase(SortP s) {
 
 __global__ __launch_bounds__(NTHREADS) void k_bds_fill(BoxDistP p, SortP s) {
   __shared__ int cur[BDS_MAXBINS];
-  for (int e = threadIdx.x; e < s.nbins; e += NTHREADS) cur[e] = s.wgbase[(long)blockIdx.x * s.nbins + e];
+  for (int e = threadIdx.x; e < s.nbins; e += NTHREADS) cur[e] = s.binoff[e] + s.wgbase[(long)blockIdx.x * s.nbins + e];
   __syncthreads();
   bds_walk(p, [&](int bin, unsigned pid, unsigned mask) {
     const int pos = atomicAdd(&cur[bin], 1);
@@ -449,7 +469,7 @@ static long bds_align(long v) { return (v + 15) & ~15L; }
 
 struct BdsLayout {
   long scal, counts, binoff, wgbase, items, records, item_out, dtab, boxtab, total;
-  int nbins, maxitems;
+  int nbins, maxitems, nwg;
   long maxrecords;
 };
 static BdsLayout bds_layout(int B, int L, int K, int D, int H, int W) {
@@ -457,11 +477,12 @@ static BdsLayout bds_layout(int B, int L, int K, int D, int H, int W) {
   const long pairs = (long)B * L * K, maxrec = pairs * 8;
   y.nbins = (D + 2) * (H + 2) * (W + 2);
   y.maxitems = (int)(y.nbins + maxrec / BDS_SEG + 1);
+  y.nwg = (long)B * ((K + NTHREADS - 1) / NTHREADS) * L >= 4 * BDS_NWG ? BDS_NWG : BDS_NWG / 2;
   long o = 0;
   y.scal = o; o = bds_align(o + 16);
   y.counts = o; o = bds_align(o + (long)y.nbins * 4);
   y.binoff = o; o = bds_align(o + (long)y.nbins * 4);
-  y.wgbase = o; o = bds_align(o + (long)BDS_NWG * y.nbins * 4);
+  y.wgbase = o; o = bds_align(o + (long)y.nwg * y.nbins * 4);
   y.items = o; o = bds_align(o + (long)y.maxitems * 12);
   y.records = o; o = bds_align(o + maxrec * 8);
   y.item_out = o; o = bds_align(o + (long)y.maxitems * BDS_OUT * 8);
@@ -489,6 +510,7 @@ int launch_box_dist_bwd_sorted(const BoxDistP& p, hipStream_t st) {
   s.boxtab = (float*)(base + y.boxtab);
   s.nbins = y.nbins;
   s.maxitems = y.maxitems;
+  s.nwg = y.nwg;
   s.maxrecords = (long)p.B * p.L * p.K * 8;
   const dim3 b(NTHREADS);
   const int cells16 = p.D * p.H * p.W * BD_C;
@@ -497,10 +519,10 @@ int launch_box_dist_bwd_sorted(const BoxDistP& p, hipStream_t st) {
   if (p.dtype) hipLaunchKernelGGL(k_bds_gmax<true>, dim3(512), b, 0, st, p, s.scal);
   else hipLaunchKernelGGL(k_bds_gmax<false>, dim3(512), b, 0, st, p, s.scal);
   hipLaunchKernelGGL(k_bds_boxes, dim3((p.B * p.K + NTHREADS - 1) / NTHREADS), b, 0, st, p, s);
-  hipLaunchKernelGGL(k_bds_count, dim3(BDS_NWG), b, 0, st, p, s);
+  hipLaunchKernelGGL(k_bds_count, dim3(s.nwg), b, 0, st, p, s);
+  hipLaunchKernelGGL(k_bds_wgbase, dim3((y.nbins + 63) / 64), dim3(1024), 0, st, s);
   hipLaunchKernelGGL(k_bds_plan, dim3(1), b, 0, st, s);
-  hipLaunchKernelGGL(k_bds_wgbase, dim3((y.nbins + 63) / 64), dim3(64), 0, st, s);
-  hipLaunchKernelGGL(k_bds_fill, dim3(BDS_NWG), b, 0, st, p, s);
+  hipLaunchKernelGGL(k_bds_fill, dim3(s.nwg), b, 0, st, p, s);
   int e = (int)hipGetLastError();
   if (e) return e;
   if (p.dtype) hipLaunchKernelGGL(k_bds_accum<true>, dim3(y.maxitems), b, 0, st, p, s);

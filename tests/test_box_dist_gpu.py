@@ -27,7 +27,8 @@ def _inputs(B, nP, nQ, seed, angles):
 # the table gradient scatters with LDS atomics below 65536 (point, box) pairs and sorts by window above: both sizes
 CASES = [(2, 37, 256, False, (10, 10, 10)), (1, 5, 300, True, (10, 10, 10)), (2, 64, 19, True, (4, 6, 7)),
          (1, 1, 1, False, (10, 10, 10)), (2, 160, 256, False, (10, 10, 10)), (1, 230, 300, True, (10, 10, 10)),
-         (1, 1100, 64, True, (4, 6, 7)), (1, 1500, 43, True, (10, 10, 10))]   # two point segments, ragged box group
+         (1, 1100, 64, True, (4, 6, 7)), (1, 1500, 43, True, (10, 10, 10)),   # two point segments, ragged box group
+         (1, 4200, 16, True, (5, 4, 3)), (3, 1400, 16, False, (1, 30, 30))]     # four workgroups a CU in the gradient, 3072 bins
 
 
 def test_box_dist_forward_does_not_depend_on_the_segments():
