@@ -46,6 +46,12 @@ def _f32c(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return None if t is None else t.detach().float().contiguous()
 
 
+def _lattice(coords: torch.Tensor) -> Optional[tuple]:
+    """(n0, n1, n2) of a (1, n0, n1, n2, 3) table of coordinates; None for any other shape.  (The kernel writes 16 values for
+    every three of the coordinates, so their number has to be that of the table's nodes.)"""
+    return tuple(coords.shape[1:4]) if coords.dim() == 5 and coords.shape[0] == 1 and coords.shape[4] == 3 else None
+
+
 class BoxDistFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, table, key_xyz, corners, angle, qcenter, radius, weight_dist, log_scale, max_value, out_dtype,
@@ -185,9 +191,11 @@ class BoxDistFun(nn.Module):
                 any(p.dtype != w.dtype or p.device != w.device or not p.is_contiguous() or
                     type(p) not in (nn.Parameter, torch.Tensor) for p in ps):
             return None
-        n = coords.shape[1:4]
+        n = _lattice(coords)
+        if n is None:
+            return None
         a = L.BoxTableArgs()
-        a.nodes, a.hidden = coords.numel() // 3, w.shape[0]
+        a.nodes, a.hidden = math.prod(n), w.shape[0]
         a.dtype, a.coords_dtype = L.dtype_code(w.dtype), L.dtype_code(coords.dtype)
         a.coords, a.w1, a.b1, a.w2 = coords.data_ptr(), w.data_ptr(), ps[1].data_ptr(), ps[2].data_ptr()
         table = torch.empty((CHANNELS, *n), dtype=torch.float32, device=w.device)

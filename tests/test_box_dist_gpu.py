@@ -162,6 +162,28 @@ def test_table_without_a_gradient(quant, rpe_dim, dtype):
     assert ((got.double().cpu() - ref).abs() <= u * (mag + ref.abs())).all()
 
 
+@pytest.mark.parametrize("shape", [(4, 4, 4, 3), (2, 4, 4, 4, 3), (1, 4, 4, 4, 6), (1, 2, 4, 4, 4, 3)])
+def test_table_of_a_replaced_lattice(shape):
+    """Without a gradient a lattice of another form does what it does with one: the modules take it or refuse it."""
+    from dest3d_amd.box_dist import BoxDistFun
+    m = BoxDistFun(out_dim=16).cuda()
+    m.relative_coords_table = torch.randn(shape, device="cuda")
+    args = (torch.rand(1, 5, 3).cuda(), torch.rand(1, 3, 3).cuda(), torch.rand(1, 3, 3).cuda(), torch.zeros(1, 3).cuda())
+
+    def call():
+        try:
+            return m(*args)
+        except RuntimeError:
+            return None
+
+    want = call()
+    assert (want is not None) == (shape == (2, 4, 4, 4, 3))
+    with torch.no_grad():
+        assert m._plain_table() is None
+        got = call()
+    assert want is None and got is None or torch.equal(got, want)
+
+
 def test_box_dist_rejects_unbuilt_shapes():
     import ctypes as C
     from dest3d_amd import _lib as L

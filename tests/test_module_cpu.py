@@ -69,3 +69,14 @@ def test_reversed_branch_sees_zero_padding_of_the_convolved_tensor():
     # all-ones taps over a 5-token sequence with padding 3: every output is the plain sum of y0 over the tokens in reach
     want = torch.stack([y0[0, max(0, l - 3):l + 4].sum(0) for l in range(5)])
     assert torch.allclose(y1[0], F.silu(want), atol=1e-13)
+
+
+def test_lattice_of_the_distance_table_is_checked_before_a_kernel_writes_it():
+    """The kernel that fills the distance table writes 16 values per coordinate triple into a table sized from the lattice's
+    shape: only a (1, n0, n1, n2, 3) buffer has as many triples as the table has nodes."""
+    import torch
+    from dest3d_amd.box_dist import BoxDistFun, _lattice
+    assert _lattice(BoxDistFun(out_dim=16).relative_coords_table) == (10, 10, 10)
+    assert _lattice(torch.zeros(1, 4, 5, 6, 3)) == (4, 5, 6)
+    for shape in ((10, 10, 10, 3), (2, 4, 5, 6, 3), (1, 4, 5, 6, 6), (1, 1, 4, 5, 6, 3), (1, 4, 5, 3), (8, 3), (3,)):
+        assert _lattice(torch.zeros(shape)) is None, shape
