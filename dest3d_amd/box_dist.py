@@ -17,6 +17,8 @@ import torch
 import torch.nn as nn
 
 import torch.autograd.forward_ad as _forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib as L
 from .scan_module import _hooked
@@ -50,6 +52,13 @@ def _lattice(coords: torch.Tensor) -> Optional[tuple]:
     """(n0, n1, n2) of a (1, n0, n1, n2, 3) table of coordinates; None for any other shape.  (The kernel writes 16 values for
     every three of the coordinates, so their number has to be that of the table's nodes.)"""
     return tuple(coords.shape[1:4]) if coords.dim() == 5 and coords.shape[0] == 1 and coords.shape[4] == 3 else None
+
+
+def _watched() -> bool:
+    """Whether a dispatch or function mode, a tracer or a compiler sees the operations that are called here.  (A default device
+    is a function mode as well, and asks for nothing but new tensors.)"""
+    return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
+                or any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
 
 
 class BoxDistFn(torch.autograd.Function):
@@ -172,7 +181,9 @@ class BoxDistFun(nn.Module):
 
     def _plain_table(self):
         """The same table, (out_dim, n, n, n) fp32, from one kernel where nothing is to be differentiated and the modules are
-        what this class made them (calling them would do nothing else); None otherwise."""
+        what this class made them (calling them would do nothing else, and nobody watches); None otherwise."""
+        if _watched():
+            return None
         if type(self.cpb_mlps) is not nn.Sequential or len(self.cpb_mlps) != 3:
             return None
         lin1, act, lin2 = self.cpb_mlps
@@ -184,7 +195,8 @@ class BoxDistFun(nn.Module):
                 lin1.bias is None or any(_hooked(m) for m in (self.cpb_mlps, lin1, act, lin2)):
             return None
         if torch.is_autocast_enabled("cuda") or _forward_ad._current_level >= 0 or not w.is_cuda or \
-                w.dtype not in (torch.float32, torch.bfloat16) or coords.dtype not in (torch.float32, torch.bfloat16) or \
+                w.dtype not in (torch.float32, torch.bfloat16) or type(coords) is not torch.Tensor or \
+                coords.dtype not in (torch.float32, torch.bfloat16) or \
                 w.shape[0] > 256 or w.shape != (w.shape[0], 3) or ps[1].shape != w.shape[:1] or \
                 ps[2].shape != (CHANNELS, w.shape[0]) or not coords.is_contiguous() or coords.device != w.device or \
                 (torch.is_grad_enabled() and (coords.requires_grad or any(p.requires_grad for p in ps))) or \

@@ -8,6 +8,7 @@
 
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
@@ -512,8 +513,12 @@ bool own_memory(const Tensor& t) {
          !t.key_set().has_any(c10::DispatchKeySet({K::Python, K::Functionalize, K::FuncTorchBatched, K::FuncTorchGradWrapper,
                                                    K::Batched, K::Negative, K::ZeroTensor}));
 }
+// a dispatch mode (one that counts or records operations, say) or a tracer sees the library's products, and none of the kernels here
+bool watched() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
+}
 bool few_tokens(const Tensor& x, const Tensor& w) {
-  if (!own_memory(x) || !own_memory(w)) return false;
+  if (watched() || !own_memory(x) || !own_memory(w)) return false;
   if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
   if (w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || w.size(1) == 0 || w.size(1) % 32 || x.numel() == 0) return false;
   return (double)x.numel() * (double)w.size(0) <= FEW_PRODUCTS && x.is_contiguous() && w.is_contiguous() &&
@@ -538,7 +543,7 @@ Tensor linear_few(const Tensor& x, const Tensor& w) {
 // backward pass that is itself differentiated takes the library's products, which autograd knows.
 constexpr int64_t DW_WEIGHTS = 200000;
 bool narrow_result(const Tensor& x, const Tensor& dy) {
-  return !at::GradMode::is_enabled() && own_memory(x) && own_memory(dy) && x.is_cuda() && dy.device() == x.device() &&
+  return !at::GradMode::is_enabled() && !watched() && own_memory(x) && own_memory(dy) && x.is_cuda() && dy.device() == x.device() &&
          x.scalar_type() == at::kBFloat16 && dy.scalar_type() == at::kBFloat16 && x.is_contiguous() && dy.is_contiguous() &&
          x.size(0) > 0 && x.size(0) == dy.size(0) && x.size(0) < (1 << 30) && x.size(1) >= 6 && dy.size(1) >= 4 &&
          x.size(1) <= DW_WEIGHTS / dy.size(1);

@@ -162,6 +162,40 @@ def test_table_without_a_gradient(quant, rpe_dim, dtype):
     assert ((got.double().cpu() - ref).abs() <= u * (mag + ref.abs())).all()
 
 
+def test_modes_see_the_tables_mlp():
+    """Who counts or records operations or functions sees the two products of the table's MLP; a default device does not ask."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._device import DeviceContext
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from dest3d_amd.box_dist import BoxDistFun
+    m = BoxDistFun(out_dim=16).cuda()
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func is torch.nn.functional.linear)
+            return func(*args, **(kwargs or {}))
+
+    class Operations(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func in (torch.ops.aten.mm.default, torch.ops.aten.addmm.default))
+            return func(*args, **(kwargs or {}))
+
+    args = (torch.rand(1, 5, 3).cuda(), torch.rand(1, 3, 3).cuda(), torch.rand(1, 3, 3).cuda(), torch.zeros(1, 3).cuda())
+    with torch.no_grad():
+        want = m(*args)
+        with DeviceContext("cuda"):
+            assert m._plain_table() is not None
+        for mode in (Functions, Operations):
+            seen.clear()
+            with mode():
+                got = m(*args)
+            assert sum(seen) == 2
+            assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
+        compiled = torch.compile(m.rpe_table, backend="eager")()
+        assert torch.allclose(compiled, m._plain_table(), rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("shape", [(4, 4, 4, 3), (2, 4, 4, 4, 3), (1, 4, 4, 4, 6), (1, 2, 4, 4, 4, 3)])
 def test_table_of_a_replaced_lattice(shape):
     """Without a gradient a lattice of another form does what it does with one: the modules take it or refuse it."""

@@ -4,6 +4,7 @@ import ctypes as C
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from dest3d_amd import _lib as L
 
@@ -107,6 +108,41 @@ def test_projections_under_transforms():
     x, w = x.cuda(), w.cuda()
     with torch.no_grad(), pytest.raises(RuntimeError):
         torch.vmap(lambda t: _LinearTokens.apply(t, w))(x.view(4, 10, 96))
+
+
+class Products(TorchDispatchMode):
+    """Multiply-adds of the matrix products it sees."""
+
+    def __init__(self):
+        super().__init__()
+        self.seen = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if func in (torch.ops.aten.mm.default, torch.ops.aten.bmm.default, torch.ops.aten.addmm.default):
+            a, b = args[-2:]
+            self.seen += a.numel() * b.shape[-1]
+        return func(*args, **(kwargs or {}))
+
+
+def test_a_dispatch_mode_sees_the_projections():
+    """A mode that counts operations sees the four projections, and their gradients, of a layer as the library's products."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(5)
+    B, Ln, K, D = 2, 70, 40, 288
+    layer = MultiHeadISSMScan(d_model=D, d_state=K, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    x = [bf(B, Ln, D).requires_grad_(), bf(B, K, D).requires_grad_(), bf(B, Ln, K, 16)]
+    size = B * (Ln * D * (layer.key_proj.out_features + D) + K * 2 * D * D)
+    with torch.no_grad(), Products() as forward:
+        got = layer(*x, None, None)
+    assert forward.seen == size
+    with torch.no_grad():
+        for a, b in zip(got, layer(*x, None, None)):
+            assert ((a - b).float().norm() <= 2.0 ** -7 * b.float().norm())
+    with Products() as training:
+        out = layer(*x, None, None)
+        torch.autograd.backward(out, [torch.ones_like(t) for t in out])
+    assert training.seen == 3 * size
 
 
 class DwArgs(C.Structure):
