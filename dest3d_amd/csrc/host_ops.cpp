@@ -974,6 +974,9 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     if (!plain) break;
     plain = !t->defined() || (own_memory(*t) && !(at::GradMode::is_enabled() && t->requires_grad()) && !t->_fw_grad(0).defined());
   }
+  // Activations that want a gradient while none is recorded: the first run of a checkpointed segment (reentrant checkpointing),
+  // which a second one with gradients is to repeat.  Both take the same kernels.
+  plain = plain && !(in_key.requires_grad() || in_query.requires_grad() || dist.requires_grad());
   if (plain) {
     const c10::DeviceGuard guard(in_key.device());
     const int64_t B = in_key.size(0), Ln = in_key.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,

@@ -300,3 +300,31 @@ def test_layer_without_a_gradient_in_a_graph():
             graph.replay()
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(out, want))
+
+
+def test_layers_under_reentrant_checkpointing():
+    """A checkpointed layer runs without gradients first and with them afterwards: the same kernels, hence the outputs and
+    gradients of the layers that are not checkpointed, bit for bit.  Steps long enough for chunks out of a tile's range, where the
+    kernels for either case round differently."""
+    from torch.utils.checkpoint import checkpoint
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(9)
+    layers = [MultiHeadISSMScan(d_model=288, d_state=40, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16() for _ in range(3)]
+    for layer in layers:
+        layer.dt_bias.data += 6.0
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    key, query, dist, dkey, dquery = bf(2, 130, 288), bf(2, 40, 288), bf(2, 130, 40, 16), bf(2, 130, 288), bf(2, 40, 288)
+
+    def step(run):
+        k, q = key.clone().requires_grad_(), query.clone().requires_grad_()
+        hk, hq = k, q
+        for layer in layers:
+            layer.zero_grad(set_to_none=True)
+            ok, oq = run(layer, hk, hq)
+            hk, hq = hk + ok, hq + oq
+        torch.autograd.backward((hk, hq), (dkey, dquery))
+        return hk, hq, k.grad, q.grad, *(p.grad for layer in layers for p in layer.parameters())
+
+    want = step(lambda layer, k, q: layer(k, q, dist, None))
+    got = step(lambda layer, k, q: checkpoint(layer, k, q, dist, None, use_reentrant=True))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
