@@ -39,6 +39,12 @@ void require_gpu(const Tensor& t, const char* name) {
   if (!t.is_cuda())
     raise_py(PyExc_RuntimeError, std::string(name) + " must live on a HIP device: the ISSM operator has no CPU path");
 }
+// The kernels take addresses: an operand on the host or on another device is refused before its address is used.
+void require_beside(const Tensor& x, std::initializer_list<const Tensor*> operands) {
+  for (const Tensor* t : operands)
+    if (t->defined() && t->device() != x.device())
+      raise_py(PyExc_RuntimeError, "all operands must be on " + x.device().str() + ", one is on " + t->device().str());
+}
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
@@ -309,6 +315,8 @@ std::string shape_text(const Tensor& t) {
 void check_scan(const Tensor* x, const Tensor& dt, const Tensor& A, const Tensor* B, const Tensor* C, int ndir, const Tensor& D,
                 const Tensor& z, const Tensor& dt_bias, const Tensor& h0, const Tensor& seq) {
   require_gpu(x[0], "x");
+  for (int i = 0; i < ndir; ++i) require_beside(x[0], {&x[i], &B[i], &C[i]});
+  require_beside(x[0], {&dt, &A, &D, &z, &dt_bias, &h0, &seq});
   if (x[0].dim() != 4) raise_py(PyExc_ValueError, "x must be (batch, seqlen, nheads, headdim), got " + shape_text(x[0]));
   if (B[0].dim() != 4) raise_py(PyExc_ValueError, "B must be (batch, seqlen, ngroups, dstate), got " + shape_text(B[0]));
   const int64_t b = x[0].size(0), l = x[0].size(1), h = x[0].size(2), p = x[0].size(3), g = B[0].size(2), n = B[0].size(3);
@@ -486,6 +494,7 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
             int64_t group, bool before_gate, bool rms) {
   const Tensor bias = opt(bias_), z = opt(z_);
   require_gpu(x, "x");
+  require_beside(x, {&weight, &bias, &z});
   if (z.defined()) require(z.sizes() == x.sizes(), "z must have x's shape");
   require(weight.dim() == 1 && weight.size(0) == x.size(-1), "weight must have one entry per column");
   if (bias.defined()) require(bias.dim() == 1 && bias.size(0) == x.size(-1), "bias must have one entry per column");
@@ -924,8 +933,11 @@ struct CoreFn : public Function<CoreFn> {
 
 // What lies between the input projections and the output projections (dest_module.py:528-581): zx (B, L, 2 d_inner + 2 G + H)
 // from key_proj, h0 (B, K, d_inner) from query_proj -> the normalised key and the averaged final states.
-void check_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const Tensor& weights) {
+void check_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const Tensor& weights,
+                std::initializer_list<const Tensor*> parameters) {
   require_gpu(zx, "in_key");
+  require_beside(zx, {&h0, &dist, &weights});
+  require_beside(zx, parameters);
   require(zx.dim() == 3 && h0.dim() == 3 && dist.dim() == 4, "in_key (B, L, D), in_query (B, K, D), dist (B, L, K, M)");
   require(dist.size(0) == zx.size(0) && dist.size(1) == zx.size(1) && h0.size(0) == zx.size(0) && dist.size(2) == h0.size(1) &&
               dist.size(3) == WIDTH, "dist must be (B, L, K, 16)");
@@ -937,7 +949,8 @@ std::vector<Tensor> scan_core(const Tensor& zx, const Tensor& h0, const Tensor& 
                               const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias, const Tensor& A_log, const Tensor& D,
                               const Tensor& key_norm, double key_eps, int64_t d_inner, int64_t nheads, int64_t ngroups, double lo,
                               double hi) {
-  check_core(zx, h0, dist, opt(weights_));
+  check_core(zx, h0, dist, opt(weights_),
+             {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
   return CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, key_norm,
                        d_inner, nheads, ngroups, lo, hi, key_eps);
@@ -951,7 +964,8 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                const Tensor& A_log, const Tensor& D, const Tensor& key_norm, double key_eps,
                                const MaybeTensor& query_w, const MaybeTensor& query_b, double query_eps,
                                int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
-  check_core(in_key, in_query, dist, opt(weights_));
+  check_core(in_key, in_query, dist, opt(weights_),
+             {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
   // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, eight
   // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us ->

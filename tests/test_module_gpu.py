@@ -398,3 +398,41 @@ def test_parameters_of_another_size_are_refused(name, shape):
     r = lambda *s: torch.randn(*s, device="cuda")
     with pytest.raises(RuntimeError):
         m(r(1, 70, 64), r(1, 9, 64), r(1, 70, 9, 16), None)
+
+
+def test_operands_on_the_host_are_refused():
+    """Beside an input on the GPU every other operand has to be there too: refused before a kernel is given its address."""
+    from dest3d_amd import ISSM_biscan_combined, ISSM_chunk_scan_combined
+    from dest3d_amd.layernorm_gated import RMSNorm
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    r = lambda *s: torch.randn(*s, device="cuda")
+    x, dt, A, B, D, h0 = r(1, 64, 2, 8), r(1, 64, 2, 9), -r(2, 9).exp(), r(1, 64, 1, 9), r(2), r(1, 2, 8, 9)
+    one = dict(x=x, dt=dt, A=A, B=B, C=B, chunk_size=64, D=D, z=x, dt_bias=A, initial_states=h0,
+               seq_idx=torch.zeros(1, 64, dtype=torch.int32, device="cuda"))
+    two = dict(x_f=x, x_b=x, dt=dt, A=A, B_f=B, B_b=B, C_f=B, C_b=B, chunk_size=64, D=D, dt_bias=A, initial_states=h0)
+    for call, kw in ((ISSM_chunk_scan_combined, one), (ISSM_biscan_combined, two)):
+        call(**kw)
+        for name, t in kw.items():
+            if torch.is_tensor(t):
+                with pytest.raises(RuntimeError):
+                    call(**{**kw, name: t.cpu()})
+    with pytest.raises(RuntimeError):
+        RMSNorm(8).cuda()(x, x.cpu())
+    with pytest.raises(RuntimeError):
+        RMSNorm(8)(x)
+    m = MultiHeadISSMScan(d_model=64, d_state=9, d_dist=16, nheads=2, expand=1).cuda()
+    ins = [r(1, 70, 64), r(1, 9, 64), r(1, 70, 9, 16), None, torch.rand(1, 70, 9, device="cuda")]
+    for dtype in (torch.float32, torch.bfloat16):
+        m, ins[:3] = m.to(dtype), [t.to(dtype) for t in ins[:3]]
+        for grad in (True, False):
+            with torch.set_grad_enabled(grad):
+                m(*ins)
+                for i in (0, 1, 4):
+                    with pytest.raises(RuntimeError):
+                        m(*[t.cpu() if j == i else t for j, t in enumerate(ins)])
+                for name, p in m.named_parameters():
+                    gpu = p.data
+                    p.data = gpu.cpu()
+                    with pytest.raises(RuntimeError):
+                        m(*ins)
+                    p.data = gpu
