@@ -933,11 +933,13 @@ struct CoreFn : public Function<CoreFn> {
 
 // What lies between the input projections and the output projections (dest_module.py:528-581): zx (B, L, 2 d_inner + 2 G + H)
 // from key_proj, h0 (B, K, d_inner) from query_proj -> the normalised key and the averaged final states.
-void check_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const Tensor& weights,
-                std::initializer_list<const Tensor*> parameters) {
+void check_core(const Tensor& zx, const Tensor& h0, const Tensor& dist, const Tensor& weights, int64_t d_inner, int64_t nheads,
+                int64_t ngroups, std::initializer_list<const Tensor*> parameters) {
   require_gpu(zx, "in_key");
   require_beside(zx, {&h0, &dist, &weights});
   require_beside(zx, parameters);
+  require(nheads > 0 && ngroups > 0 && d_inner % nheads == 0 && nheads % ngroups == 0,
+          "d_inner must be divisible by nheads, and nheads by ngroups");
   require(zx.dim() == 3 && h0.dim() == 3 && dist.dim() == 4, "in_key (B, L, D), in_query (B, K, D), dist (B, L, K, M)");
   require(dist.size(0) == zx.size(0) && dist.size(1) == zx.size(1) && h0.size(0) == zx.size(0) && dist.size(2) == h0.size(1) &&
               dist.size(3) == WIDTH, "dist must be (B, L, K, 16)");
@@ -949,7 +951,7 @@ std::vector<Tensor> scan_core(const Tensor& zx, const Tensor& h0, const Tensor& 
                               const Tensor& dt_w, const Tensor& bc_w, const Tensor& dt_bias, const Tensor& A_log, const Tensor& D,
                               const Tensor& key_norm, double key_eps, int64_t d_inner, int64_t nheads, int64_t ngroups, double lo,
                               double hi) {
-  check_core(zx, h0, dist, opt(weights_),
+  check_core(zx, h0, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
   return CoreFn::apply(zx, h0, dist, weights_, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, key_norm,
@@ -964,7 +966,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                const Tensor& A_log, const Tensor& D, const Tensor& key_norm, double key_eps,
                                const MaybeTensor& query_w, const MaybeTensor& query_b, double query_eps,
                                int64_t d_inner, int64_t nheads, int64_t ngroups, double lo, double hi) {
-  check_core(in_key, in_query, dist, opt(weights_),
+  check_core(in_key, in_query, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
   // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, eight

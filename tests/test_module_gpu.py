@@ -436,3 +436,13 @@ def test_operands_on_the_host_are_refused():
                     with pytest.raises(RuntimeError):
                         m(*ins)
                     p.data = gpu
+
+
+@pytest.mark.parametrize("nheads,ngroups", [(3, 1), (4, 3)])
+@pytest.mark.parametrize("grad", [True, False])
+def test_heads_that_do_not_divide_the_features_are_refused(nheads, ngroups, grad):
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    m = MultiHeadISSMScan(d_model=64, d_state=32, d_dist=16, nheads=nheads, ngroups=ngroups, expand=1).cuda().bfloat16()
+    r = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    with torch.set_grad_enabled(grad), pytest.raises(AssertionError):
+        m(r(1, 70, 64), r(1, 32, 64), r(1, 70, 32, 16), None)
