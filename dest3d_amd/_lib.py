@@ -6,6 +6,7 @@ loudly -- there is no PyTorch fallback.
 from __future__ import annotations
 
 import ctypes as C
+import math
 import os
 from typing import Optional, Sequence
 
@@ -301,3 +302,14 @@ def current_stream_ptr(device) -> int:
 def require_gpu(t: torch.Tensor, name: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(f"{name} must live on a HIP device: the ISSM operator has no CPU path")
+
+
+def require_operand(t: Optional[torch.Tensor], name: str, beside: torch.Tensor, *sizes: int) -> None:
+    """The kernels take an address and the sizes of the call: an operand on another device than `beside`, or one that does not
+    have the `sizes`' number of values (no sizes: any), is refused before its address is used."""
+    if t is None:
+        return
+    if t.device != beside.device:
+        raise RuntimeError(f"{name} is on {t.device}, the other operands are on {beside.device}")
+    if sizes and t.numel() != math.prod(sizes):
+        raise ValueError(f"{name} must be {sizes}, got {tuple(t.shape)}")

@@ -72,6 +72,9 @@ class BoxDistFn(torch.autograd.Function):
         key, cor, ang = _f32c(key_xyz), _f32c(corners), _f32c(angle)
         as_boxes = cor.dim() == 3          # (B, nQ, 7) boxes instead of (B, nQ, 8, 3) corners
         assert cor.shape[2:] == ((7,) if as_boxes else (8, 3))
+        L.require_operand(key, "key_xyz", key, Bsz, nP, 3)
+        L.require_operand(cor, "the boxes", key, Bsz, nQ, *cor.shape[2:])
+        L.require_operand(ang, "angle", key, Bsz, nQ)
         a = L.BoxDistArgs()
         a.batch, a.seqlen, a.nquery = Bsz, nP, nQ
         a.dtype = L.dtype_code(out_dtype)
@@ -89,6 +92,7 @@ class BoxDistFn(torch.autograd.Function):
             if want_dist:
                 assert table.dim() == 4 and table.shape[0] == CHANNELS, "table must be (16, D, H, W)"
                 tab = _f32c(table)
+                L.require_operand(tab, "table", key)
                 a.D, a.H, a.W = tab.shape[1:]
                 a.table = tab.data_ptr()
                 dist = torch.empty((Bsz, nP, nQ, CHANNELS), dtype=out_dtype, device=key.device)
@@ -98,6 +102,8 @@ class BoxDistFn(torch.autograd.Function):
                 a.weight_dist = float(weight_dist)
                 if qcenter is not None:
                     qc, rad = _f32c(qcenter), _f32c(radius)
+                    L.require_operand(qc, "the weights' centres", key, Bsz, nQ, 3)
+                    L.require_operand(rad, "the weights' radii", key, Bsz, nQ)
                     a.qcenter, a.radius = qc.data_ptr(), rad.data_ptr()
                 else:
                     assert as_boxes, "weights need (qcenter, radius) or boxes"

@@ -35,6 +35,8 @@ class DwConvSiLUFn(torch.autograd.Function):
         L.require_gpu(u, "u")
         lib = L.load()
         Bsz, Ln, Cn = u.shape
+        for i, t in enumerate(wb):
+            L.require_operand(t, "bias" if i & 1 else "weight", u, Cn, 1 if i & 1 else TAPS)
         ud = u.detach()
         if ud.dtype not in (torch.float32, torch.bfloat16):
             ud = ud.float()

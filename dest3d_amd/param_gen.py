@@ -43,6 +43,8 @@ class ScanParamsFn(torch.autograd.Function):
         R0 = H + 2 * G
         R = R0 + (2 * G if has_back else 0)
         assert W.shape == (R0, M) and bias.shape == (Bsz, Ln, R)
+        for t, name in ((W, "W"), (bias, "bias"), (weights, "weights")):
+            L.require_operand(t, name, dist)
         d = dist.detach().contiguous()
         w = W.detach().float().contiguous()
         b = bias.detach().float().contiguous()

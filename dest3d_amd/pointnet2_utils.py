@@ -37,6 +37,7 @@ class FurthestPointSampling(Function):
         lib = L.load()
         x = _f(xyz)
         Bsz, N, _ = x.shape
+        L.require_operand(x, "xyz", x, Bsz, N, 3)
         with torch.cuda.device(x.device):
             out = torch.empty((Bsz, npoint), dtype=torch.int32, device=x.device)   # (written whole)
             temp = torch.empty((Bsz, N), dtype=torch.float32, device=x.device) if N > 24576 else None
@@ -62,6 +63,7 @@ class GatherOperation(Function):
         f, ix = _f(features), _i(idx)
         Bsz, Cn, N = f.shape
         M = ix.shape[1]
+        L.require_operand(ix, "idx", f, Bsz, M)
         with torch.cuda.device(f.device):
             out = torch.empty((Bsz, Cn, M), dtype=torch.float32, device=f.device)
             L.check(lib.issm_pn2_gather_points(Bsz, Cn, N, M, f.data_ptr(), ix.data_ptr(), out.data_ptr(), _st(f)),
@@ -94,6 +96,8 @@ class ThreeNN(Function):
         u, k = _f(unknown), _f(known)
         Bsz, n, _ = u.shape
         m = k.shape[1]
+        L.require_operand(u, "unknown", u, Bsz, n, 3)
+        L.require_operand(k, "known", u, Bsz, m, 3)
         with torch.cuda.device(u.device):
             dist2 = torch.empty((Bsz, n, 3), dtype=torch.float32, device=u.device)
             idx = torch.empty((Bsz, n, 3), dtype=torch.int32, device=u.device)
@@ -119,6 +123,8 @@ class ThreeInterpolate(Function):
         f, ix, w = _f(features), _i(idx), _f(weight)
         Bsz, c, m = f.shape
         n = ix.shape[1]
+        L.require_operand(ix, "idx", f, Bsz, n, 3)
+        L.require_operand(w, "weight", f, Bsz, n, 3)
         with torch.cuda.device(f.device):
             out = torch.empty((Bsz, c, n), dtype=torch.float32, device=f.device)
             L.check(lib.issm_pn2_three_interpolate(Bsz, c, m, n, f.data_ptr(), ix.data_ptr(), w.data_ptr(), out.data_ptr(),
@@ -161,6 +167,7 @@ class GroupingOperation(Function):
         f, ix = _f(features), _i(idx)
         Bsz, Cn, N = f.shape
         _, M, S = ix.shape
+        L.require_operand(ix, "idx", f, Bsz, M, S)
         with torch.cuda.device(f.device):
             out = torch.empty((Bsz, Cn, M, S), dtype=torch.float32, device=f.device)
             L.check(lib.issm_pn2_group_points(Bsz, Cn, N, M, S, f.data_ptr(), ix.data_ptr(), out.data_ptr(), _st(f)),
@@ -207,6 +214,8 @@ class _GroupXyzPoints(Function):
         x, q, ix = _f(xyz), _f(new_xyz), _i(idx)
         f = None if features is None else _f(features)
         (Bsz, N, _), (_, M, S), Cn = x.shape, ix.shape, 0 if f is None else f.shape[1]
+        for t, name, sizes in ((x, "xyz", (Bsz, N, 3)), (q, "new_xyz", (Bsz, M, 3)), (f, "features", (Bsz, Cn, N)), (ix, "idx", (Bsz, M, S))):
+            L.require_operand(t, name, x, *sizes)
         with torch.cuda.device(x.device):
             out = torch.empty((Bsz, 3 + Cn, M, S), dtype=torch.float32, device=x.device)
             L.check(lib.issm_pn2_group_xyz_points(Bsz, Cn, N, M, S, x.data_ptr(), q.data_ptr(), scale,
@@ -231,6 +240,8 @@ class BallQuery(Function):
         x, q = _f(xyz), _f(new_xyz)
         Bsz, N, _ = x.shape
         M = q.shape[1]
+        L.require_operand(x, "xyz", x, Bsz, N, 3)
+        L.require_operand(q, "new_xyz", x, Bsz, M, 3)
         with torch.cuda.device(x.device):
             idx = torch.empty((Bsz, M, nsample), dtype=torch.int32, device=x.device)   # (written whole)
             L.check(lib.issm_pn2_ball_query(Bsz, N, M, float(radius), nsample, q.data_ptr(), x.data_ptr(), idx.data_ptr(),

@@ -142,3 +142,17 @@ def test_bench_refuses_more_than_one_gpu_and_a_missing_gpu():
     if not torch.cuda.is_available():
         r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py")], capture_output=True, text=True, timeout=300)
         assert r.returncode == 2 and "needs a GPU" in r.stderr
+
+
+def test_operands_of_another_size_or_device_are_refused():
+    import torch
+    from dest3d_amd import _lib as L
+    x = torch.zeros(2, 5, 3)
+    L.require_operand(None, "absent", x, 7)
+    L.require_operand(x, "x", x)
+    L.require_operand(x, "x", x, 2, 5, 3)
+    for sizes in ((2, 5, 4), (1, 5, 3), (4, 5, 3)):
+        with pytest.raises(ValueError):
+            L.require_operand(x, "x", x, *sizes)
+    with pytest.raises(RuntimeError):
+        L.require_operand(x.to("meta"), "x", x)

@@ -218,6 +218,34 @@ def test_table_of_a_replaced_lattice(shape):
     assert want is None and got is None or torch.equal(got, want)
 
 
+def test_operands_of_another_size_or_device_are_refused():
+    """Refused before a kernel is given their address."""
+    from dest3d_amd.box_dist import box_dist, box_parametrization_to_corners, local_weight
+    from dest3d_amd.dwconv import dwconv_silu
+    from dest3d_amd.param_gen import scan_params
+    key, qxyz, qsize, ang = (torch.from_numpy(x).cuda() for x in _inputs(2, 9, 5, 1, True))
+    table = torch.randn(16, 4, 4, 4).cuda()
+    corners, query = box_parametrization_to_corners(qxyz, qsize, ang), torch.cat([qxyz, qsize], -1)
+    box_dist(table, key, corners, ang)
+    for args in ((table, key, corners[:1], ang), (table, key, corners, ang[:1]), (table, key[..., :2], corners, ang),
+                 (table.cpu(), key, corners, ang), (table, key, corners.cpu(), ang), (table, key, corners, ang.cpu())):
+        with pytest.raises((RuntimeError, ValueError)):
+            box_dist(*args)
+    for bad in (query[:1], query.cpu()):
+        with pytest.raises((RuntimeError, ValueError)):
+            local_weight(key, bad)
+    u, w, b = torch.randn(1, 9, 4).cuda(), torch.randn(4, 1, 7).cuda(), torch.randn(4).cuda()
+    dwconv_silu(u, [w], [b])
+    for ww, bb in ((w.cpu(), b), (w, b.cpu()), (w, b[:3]), (w[:3], b)):
+        with pytest.raises((RuntimeError, ValueError)):
+            dwconv_silu(u, [ww], [bb])
+    d, W, bias, wts = torch.randn(1, 9, 5, 16).cuda(), torch.randn(4, 16).cuda(), torch.randn(1, 9, 4).cuda(), torch.rand(1, 9, 5).cuda()
+    scan_params(d, W, bias, 2, 1, weights=wts)
+    for args in ((W.cpu(), bias, wts), (W, bias.cpu(), wts), (W, bias, wts.cpu())):
+        with pytest.raises(RuntimeError):
+            scan_params(d, *args[:2], 2, 1, weights=args[2])
+
+
 def test_box_dist_rejects_unbuilt_shapes():
     import ctypes as C
     from dest3d_amd import _lib as L

@@ -432,3 +432,25 @@ def test_error_codes():
     assert lib.issm_pn2_ball_query(-1, 10, 4, 0.5, 8, None, None, None, None) == -2
     assert lib.issm_pn2_group_points(1, 2, 0, 4, 4, None, None, None, None) == -2
     assert lib.issm_pn2_three_nn(0, 5, 5, None, None, None, None, None) == 0
+
+
+def test_operands_of_another_batch_or_device_are_refused():
+    """Refused before a kernel is given their address: a batch smaller than the first operand's, and tensors on the host."""
+    from dest3d_amd import pointnet2_utils as P
+    xyz, feat, centres = torch.rand(2, 40, 3).cuda(), torch.rand(2, 5, 40).cuda(), torch.rand(2, 8, 3).cuda()
+    idx, idx3 = torch.zeros(2, 8, 4, dtype=torch.int32).cuda(), torch.zeros(2, 30, 3, dtype=torch.int32).cuda()
+    weight = torch.rand(2, 30, 3).cuda()
+    calls = [(P.furthest_point_sample, (torch.rand(2, 40, 2).cuda(), 8), ()), (P.gather_operation, (feat, idx[:, :, 0]), (1,)),
+             (P.three_nn, (xyz, centres), (1,)), (P.three_interpolate, (feat, idx3, weight), (1, 2)),
+             (P.grouping_operation, (feat, idx), (1,)), (P.ball_query, (0.3, 4, xyz, centres), (3,)),
+             (P.QueryAndGroup(0.3, 4), (xyz, centres, feat), (1, 2))]
+    for call, args, at in calls:
+        if not at:
+            with pytest.raises(ValueError):
+                call(*args)
+            continue
+        call(*args)
+        for i in at:
+            for bad, error in ((args[i][:1], (ValueError, RuntimeError)), (args[i].cpu(), RuntimeError)):
+                with pytest.raises(error):
+                    call(*(bad if j == i else t for j, t in enumerate(args)))
