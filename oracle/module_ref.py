@@ -24,7 +24,8 @@ def point_lite_conv(sd, prefix, t):
 
 
 def multi_head_issm_scan_ref(sd, cfg, in_key, in_query, dist, mask, intermediates=None):
-    """sd: state_dict of the module (reference parameter names); cfg: nheads, ngroups, d_inner, d_state, use_biscan.
+    """sd: state_dict of the module (reference parameter names); cfg: nheads, ngroups, d_inner, d_state, use_biscan;
+    key_eps, query_eps of the two norms (1e-5 where absent).
     Returns (out_key, out_query).  If `intermediates` is a dict it receives x, x_back, B, C, B_back, C_back, dt."""
     H, G, d_inner = cfg["nheads"], cfg["ngroups"], cfg["d_inner"]
     P, K = d_inner // H, cfg["d_state"]
@@ -62,8 +63,9 @@ def multi_head_issm_scan_ref(sd, cfg, in_key, in_query, dist, mask, intermediate
         key_b, last_b = scan(fl(x_b), fl(dt), fl(B_back), fl(C_back))                  # :568-572
         key = (key + fl(key_b)) / 2                                                    # :573-575
         last = (last + last_b) / 2
-    key = R.gated_rmsnorm_ref(key.flatten(-2), sd["key_norm.weight"], z=z, eps=1e-5, norm_before_gate=False)  # :578-579
+    key = R.gated_rmsnorm_ref(key.flatten(-2), sd["key_norm.weight"], z=z, eps=cfg.get("key_eps", 1e-5),
+                             norm_before_gate=False)                                       # :578-579
     out_key = key @ sd["out_key_proj.weight"].T
     last = last.permute(0, 3, 1, 2).flatten(-2)                                        # :582
-    last = F.layer_norm(last, (d_inner,), sd["query_norm.weight"], sd["query_norm.bias"], 1e-5)
+    last = F.layer_norm(last, (d_inner,), sd["query_norm.weight"], sd["query_norm.bias"], cfg.get("query_eps", 1e-5))
     return out_key, last @ sd["out_query_proj.weight"].T

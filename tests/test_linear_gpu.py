@@ -277,6 +277,46 @@ def test_layer_without_a_gradient(B, Ln, K, mask):
     assert all(torch.equal(a, b) for a, b in zip(frozen, got))
 
 
+@pytest.mark.parametrize("D,H,G,per_head_d,B,Ln,K,mask", [(288, 8, 1, True, 1, 130, 40, "weights"), (288, 8, 1, False, 2, 70, 33, None),
+                                                          (64, 4, 2, False, 3, 65, 20, "drop"), (96, 6, 3, True, 2, 1, 1, None),
+                                                          (160, 8, 2, False, 1, 200, 64, "weights"), (512, 8, 1, True, 1, 77, 130, None)])
+def test_layer_without_a_gradient_against_fp64(D, H, G, per_head_d, B, Ln, K, mask):
+    """The layer's shorter chain, row by row of its results, against an fp64 evaluation on the same bf16 parameters and inputs:
+    several widths, groups and forms of D, norms whose eps counts.  A rounding to bf16 is 2^-8 / sqrt 12 of a value on average; a
+    dozen to sixteen of them lie on the way from an input to a result (projection, two convolutions, dt, B, C, the scan's operands,
+    its two outputs and their sum, the norm, the result), together 3.9e-3 to 4.5e-3 of a row (measured: 3.0e-3 to 4.9e-3, single
+    rows of 64 features up to 1.5e-2).  A quarter of an eps, another head's D or A, another norm's eps move the rows by 0.05 to 1.
+    """
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    from oracle.module_ref import multi_head_issm_scan_ref
+    torch.manual_seed(D + Ln)
+    layer = MultiHeadISSMScan(d_model=D, d_state=K, d_dist=16, chunk_size=256, nheads=H, ngroups=G, expand=1)
+    if not per_head_d:
+        layer.D = torch.nn.Parameter(torch.empty(H, D // H))
+    with torch.no_grad():
+        layer.D.normal_()
+        for p in (layer.key_norm.weight, layer.query_norm.weight, layer.query_norm.bias):
+            p.add_(0.3 * torch.randn_like(p))
+    layer.key_norm.eps, layer.query_norm.eps = 0.02, 0.1
+    layer = layer.cuda().bfloat16()
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    x = bf(B, Ln, D), bf(B, K, D), 0.5 * bf(B, Ln, K, 16)
+    m = None if mask is None else torch.rand(B, Ln, K).cuda() if mask == "weights" else torch.rand(B, Ln, K).cuda() < 0.3
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    with torch.no_grad():
+        before = count()
+        got = layer(*x, None, m)
+        assert count() - before <= (5 if mask == "drop" else 3)     # one buffer between inputs and outputs: this is the shorter chain
+    want = layer(*x, None, m)
+    sd = {k: v.detach().double().cpu() for k, v in layer.state_dict().items()}
+    cfg = dict(nheads=H, ngroups=G, d_inner=D, d_state=K, use_biscan=True, key_eps=0.02, query_eps=0.1)
+    ref = multi_head_issm_scan_ref(sd, cfg, *(t.double().cpu() for t in x), None if m is None else m.cpu())
+    for out in (got, want):
+        for a, r in zip(out, ref):
+            off = (a.detach().double().cpu() - r).norm(dim=-1) / r.norm(dim=-1)
+            assert off.mean() <= 2.0 ** -7 and off.max() <= 2.0 ** -5
+
+
 def test_layer_without_a_gradient_in_a_graph():
     """The shorter chain recorded into a HIP graph: every replay, with eager work and other inputs between, gives the eager result."""
     from dest3d_amd.scan_module import MultiHeadISSMScan
