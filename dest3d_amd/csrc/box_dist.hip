@@ -73,7 +73,7 @@ __device__ __forceinline__ float wave_uniform(float v) {
 // full waves -- done in place, the long path would run for every wave with most lanes idle, and cost more than the
 // rest together.  The sixteen waves of a workgroup own eight adjacent boxes, so a point's eight rows are neighbours in memory,
 // and two segments of points each: four waves per SIMD on one table (vector issue bounds it, 83 M instructions; with two
-// waves per SIMD their LDS reads were not hidden).  8 x 1024 points, 256 boxes: 219 -> 176 us (162 with shared queues); one scene, whose segments are
+// waves per SIMD their LDS reads were not hidden).  8 x 1024 points, 256 boxes: 219 -> 176 us; one scene, whose segments are
 // shortened to 64 points so that all CUs have one (32 workgroups before): 209 -> 40 us.
 // The table lies node-major in LDS with 20 floats from node to node: a lane reads its node's 16 channels as four
 // 16-byte pieces, and with 16 floats per node the lanes of one read would meet in the 16 banks that (node mod 4)
@@ -135,7 +135,8 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
   __syncthreads();
   if (!live) return;
   // the box's two waves take the points both have queued in turn, 64 at a time: one wave that is not full instead of two, and both
-  // end together (eight scenes 176 -> 162 us; one scene, 26 points a queue, 39 either way)
+  // end together (eight scenes, points in the order of a Hilbert curve, bf16: 176 -> 163 us; in random order 178 either way, fp32
+  // 193 -> 186; one scene, 26 points a queue, 39.5 either way)
   const int qa = queue_len[wave & 7], all = qa + queue_len[(wave & 7) + 8], la = 2 * (bs % npair) * seg_points;
   for (int i = (wave >> 3) * 64 + lane; i < all; i += 128) {
     const int l = i < qa ? la + queue[wave & 7][i] : la + seg_points + queue[(wave & 7) + 8][i - qa];

@@ -971,8 +971,9 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
   py::gil_scoped_release release;
   // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, eight
   // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us ->
-  // 576).
-  // With many tokens the products are the library's, and the launches are not what counts.
+  // 571; two scenes 768).  The chain's products are issm_linear_fwd's, so it ends where those do (FEW_PRODUCTS: between two and
+  // three such scenes) and the separate steps take over -- not because they are faster there: three, four and eight scenes take
+  // 1252, 1494 and 2486 us with them, and 980, 1175 and 1942 with the chain and issm_linear_fwd at those sizes too.
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
   auto plain_bf16 = [&](const Tensor& t) {
     return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.device() == in_key.device() &&
