@@ -342,10 +342,11 @@ def test_layer_without_a_gradient_in_a_graph():
             assert all(torch.equal(a, b) for a, b in zip(out, want))
 
 
-def test_layers_under_reentrant_checkpointing():
-    """A checkpointed layer runs without gradients first and with them afterwards: the same kernels, hence the outputs and
-    gradients of the layers that are not checkpointed, bit for bit.  Steps long enough for chunks out of a tile's range, where the
-    kernels for either case round differently."""
+@pytest.mark.parametrize("reentrant", [True, False])
+def test_checkpointed_layers(reentrant):
+    """A layer under reentrant checkpointing runs without gradients first and with them afterwards, one under the other kind with
+    them twice: the same kernels, hence the outputs and gradients of the layers that are not checkpointed, bit for bit.  Steps long
+    enough for chunks out of a tile's range, where the kernels for either case round differently."""
     from torch.utils.checkpoint import checkpoint
     from dest3d_amd.scan_module import MultiHeadISSMScan
     torch.manual_seed(9)
@@ -366,5 +367,5 @@ def test_layers_under_reentrant_checkpointing():
         return hk, hq, k.grad, q.grad, *(p.grad for layer in layers for p in layer.parameters())
 
     want = step(lambda layer, k, q: layer(k, q, dist, None))
-    got = step(lambda layer, k, q: checkpoint(layer, k, q, dist, None, use_reentrant=True))
+    got = step(lambda layer, k, q: checkpoint(layer, k, q, dist, None, use_reentrant=reentrant))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
