@@ -132,8 +132,8 @@ static FwdWs fwd_layout(const issm_dims& d, bool has_z) {
 // sets the pace, it is not).  Where one workgroup each fills the chip, halves only cost that, also where a last round would
 // be nearly empty (its workgroups have the CUs to themselves): 9 x 1024 tokens, 8 heads x 32, 256 states, bf16, 576 workgroups,
 // a training step 278 us, in halves 281; 320 workgroups, two directions, fp32: 376 and 389.  128 workgroups, 2 x 1024 tokens of
-// 8 heads x 36, two directions, bf16: 215 us with one part, 186, 176 and 191 with 2, 4 and 8; 64, 1 x 1024 tokens, fp32: 209
-// and 171, 152, 152.
+// 8 heads x 36, two directions, bf16: 200 us with one part, 171 - 185, 160 - 169 and 173 with 2, 4 and 8 (three processes each in
+// turn; the host sets the pace from two parts on); 64, 1 x 1024 tokens, fp32: 194 and 170 - 184, 158 - 169, 167 - 172.
 static int bwd_head_parts(const issm_dims& d) {
   const long blocks = (long)d.batch * nchunks(d) * d.ngroups * ((d.dstate + ISSM_CHUNK - 1) / ISSM_CHUNK);
   const long heads = d.nheads / d.ngroups, most = std::max<long>(1, std::min<long>(heads, 512 / blocks));
