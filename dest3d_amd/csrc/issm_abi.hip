@@ -27,6 +27,9 @@ int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
                           const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
                           hipStream_t st);
+bool bwd_walk_available(const KP& p, const float* dy_ws);
+int launch_bwd_walk(const KP& p, const float* dy_ws, const float* states, float* dstates, float* dm, float* g_last, float* dh0_dir,
+                    hipStream_t st);
 int launch_bwd_dx(const KP& p, const float* dy_ws, const float* dstates, const float* cabt, float* partD,
                   hipStream_t st);
 int launch_bwd_reduce(const KP& p, const float* partA, const float* partBias, const float* partD,
@@ -139,6 +142,16 @@ static int bwd_head_parts(const issm_dims& d) {
   const long heads = d.nheads / d.ngroups, most = std::max<long>(1, std::min<long>(heads, 512 / blocks));
   const long each = (heads + most - 1) / most;
   return (heads - each) * d.ndir < 4 ? 1 : (int)((heads + each - 1) / each);   // (no part without a head)
+}
+
+// Whether the backward's states take one kernel (issm_bwd_walk.hip) or two.  A walk takes 2 - 3 us a chunk whatever the grid, until the
+// chip is full of them; two kernels take 13 - 25 us and then what the chip's share of the chunks costs.  So: every CU has a walk
+// (256: 8 x 4096 tokens, 8 heads x 32, 256 states fp32 190 against 230 us, 4 x 1024, two directions 41 against 43; bf16 147 and 167,
+// 33 and 38), or few chunks (7 chunks of 32 - 128 walks: 16 - 17 against 19 - 23 us; 8 of 32 with 200 states: 25 against 24;
+// 16 of 64: 35 against 27), or in between (192 walks: 16 chunks 39 against 40 us; 64 chunks would be about 140 against 117).
+static bool bwd_walks(const KP& p, const float* dy) {
+  const int walks = p.B * p.ndir * p.H * ((p.N + 63) / 64);
+  return (walks >= 256 || p.nc <= 7 || (walks >= 192 && p.nc <= 16)) && bwd_walk_available(p, dy);
 }
 
 static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
@@ -381,6 +394,17 @@ int issm_stage_state_passing_bwd(const issm_scan_args* a, const float* states, c
                   "state_passing_bwd");
 }
 
+int issm_stage_bwd_states(const issm_scan_args* a, const float* dy_gated, const float* states, float* dstates, float* dm,
+                          float* g_last, float* dh0_dir) {
+  int rc = check_common(a);
+  if (rc) return rc;
+  if ((rc = check_dout(a, dy_gated))) return rc;
+  if (!states || !dstates || !dm || !g_last || !dh0_dir) return fail(ISSM_E_NULL, "bwd_states: NULL buffer");
+  KP p = make_kp(a);
+  if (!bwd_walk_available(p, dy_gated)) return fail(ISSM_E_UNSUPPORTED, "bwd_states: packed sequences, mixed types, or rows of x or dy that are no multiple of four elements");
+  return launched(launch_bwd_walk(p, dy_gated, states, dstates, dm, g_last, dh0_dir, (hipStream_t)a->stream), "bwd_states");
+}
+
 size_t issm_bwd_chunk_redo_ints(const issm_scan_args* a) {
   if (check_dims(a)) return 0;
   const issm_dims& d = a->dims;
@@ -452,11 +476,17 @@ int issm_scan_bwd(const issm_scan_args* a) {
     if ((rc = launched(launch_bwd_gate(p, sv + fw.out_x, ws + bw.dy_ws, st), "bwd_gate"))) return rc;
     dy = ws + bw.dy_ws;
   }
-  if ((rc = launched(launch_bwd_dstates(p, dy, ws + bw.dstates, ws + bw.dm, st), "bwd_dstates"))) return rc;
-  if ((rc = launched(launch_state_bwd(p, sv + fw.states, sv + fw.cs_last, ws + bw.dstates, ws + bw.g_last,
-                                      ws + bw.dh0_dir, st),
-                     "state_passing_bwd")))
-    return rc;
+  if (bwd_walks(p, dy)) {
+    if ((rc = launched(launch_bwd_walk(p, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last, ws + bw.dh0_dir, st),
+                       "bwd_states")))
+      return rc;
+  } else {
+    if ((rc = launched(launch_bwd_dstates(p, dy, ws + bw.dstates, ws + bw.dm, st), "bwd_dstates"))) return rc;
+    if ((rc = launched(launch_state_bwd(p, sv + fw.states, sv + fw.cs_last, ws + bw.dstates, ws + bw.g_last,
+                                        ws + bw.dh0_dir, st),
+                       "state_passing_bwd")))
+      return rc;
+  }
   int* redo = reinterpret_cast<int*>(ws + bw.redo);
   int pending = 0;
   KP pc = p;

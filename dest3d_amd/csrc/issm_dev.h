@@ -610,13 +610,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_of(const T* q, const Tens
   const unsigned bytes = (unsigned)((rows - 1) * (int)t.s1 + cols) * (unsigned)sizeof(T);
   return __builtin_amdgcn_make_buffer_rsrc((void*)const_cast<T*>(q), 0, bytes, 0x00027000);
 }
-// Lane's 16 values of column n of a (B,L,G|H,N)-shaped tensor.
-template <bool BF>
-__device__ __forceinline__ void lane_load_ln(const TensorD& t, int b, int third, int n, bool vn, int g4,
-                                             const RowMap& rm, float (&out)[16]) {
-  typedef typename std::conditional<BF, uint16_t, float>::type T;
+// Lane's 16 values of column n of a (B,L,G|H,N)-shaped tensor, in the type they are stored in.
+template <bool BF, typename T = typename std::conditional<BF, uint16_t, float>::type>
+__device__ __forceinline__ void lane_load_raw(const TensorD& t, int b, int third, int n, bool vn, const RowMap& rm, T (&r)[16]) {
   const T* q = (const T*)t.ptr + ((long)b * t.s0 + (long)third * t.s2);
-  T r[16];
   // 32-bit offsets (the host checks that seqlen * stride fits): address = scalar base + per-lane offset.
   // ks is made opaque so that its multiples are formed here, next to their use, instead of being
   // hoisted out of an enclosing loop into (scarce) scalar registers.
@@ -638,6 +635,12 @@ __device__ __forceinline__ void lane_load_ln(const TensorD& t, int b, int third,
       else r[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
     }
   }
+}
+template <bool BF>
+__device__ __forceinline__ void lane_load_ln(const TensorD& t, int b, int third, int n, bool vn, int g4,
+                                             const RowMap& rm, float (&out)[16]) {
+  typename std::conditional<BF, uint16_t, float>::type r[16];
+  lane_load_raw<BF>(t, b, third, n, vn, rm, r);
 #pragma unroll
   for (int k = 0; k < 16; ++k) out[k] = BF ? bf16_to_f((uint16_t)r[k]) : (float)r[k];
 }

@@ -210,6 +210,12 @@ int issm_stage_bwd_dstates(const issm_scan_args* args, const float* dy_gated, fl
 int issm_stage_state_passing_bwd(const issm_scan_args* args, const float* states,
                                  const float* cs_last, float* dstates, float* g_last,
                                  float* dh0_dir);
+/* issm_stage_bwd_states: the two stages above in one kernel, which walks a head's chunks from the last to the first with
+ *   64 columns of the carried gradient in registers: dS_c into dstates, dM into dm, g_last and dh0_dir, as they leave them.
+ *   x / B / C and dt of one type, rows of x and dy in multiples of four elements, no packed sequences, no gate beside bf16
+ *   inputs (ISSM_E_UNSUPPORTED otherwise).  issm_scan_bwd takes it where the walks fill the chip. */
+int issm_stage_bwd_states(const issm_scan_args* args, const float* dy_gated, const float* states, float* dstates, float* dm,
+                          float* g_last, float* dh0_dir);
 /* issm_stage_bwd_chunk: ddt, dB, dC of direction `dir` and the per-unit partial sums
  *   part_a / part_bias (Bt*nc,H,N) of dA / ddt_bias.  ddt accumulates into args->ddt when
  *   dir > 0.  Replaces _chunk_state_bwd_db (issm_chunk_state.py:493-652), _chunk_scan_bwd_dc

@@ -853,6 +853,58 @@ def test_stage_entry_points_match_oracle_intermediates(shape):
         _check(name, t, ref[k], BWD32)
 
 
+@pytest.mark.parametrize("Bsz,L_,H,P,N,G,nd,bf,dfinal", [
+    (1, 64, 1, 32, 64, 1, 1, False, True),       # one complete chunk, one slice
+    (1, 1, 1, 4, 5, 1, 1, False, True),          # one token, a few columns
+    (2, 1000, 4, 48, 200, 2, 1, False, True),    # incomplete last chunk and slice, three full head tiles
+    (1, 65, 3, 64, 17, 1, 2, True, False),       # one row in the second chunk, both directions, no final gradient
+    (1, 192, 2, 20, 512, 1, 2, True, True),      # eight slices, a head tile partly filled
+    (2, 256, 2, 36, 128, 1, 2, False, True),
+    (2, 256, 2, 36, 128, 1, 2, True, True),
+])
+def test_states_of_the_backward_in_one_kernel(Bsz, L_, H, P, N, G, nd, bf, dfinal):
+    """issm_stage_bwd_states against the two stages it stands for: the same products in the same order, sums of the recurrence and
+    of the rows in another one (fp32: 1e-6 of the norm), dM bit for bit."""
+    print("[case] one-kernel states", Bsz, L_, H, P, N, G, nd, bf, dfinal, flush=True)
+    import dest3d_amd._lib as L
+    lib = L.load()
+    g = torch.Generator(device="cuda").manual_seed(L_ + P)
+    io = torch.bfloat16 if bf else torch.float32
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    nc = math.ceil(L_ / 64)
+    x, dy = [[r(Bsz, L_, H, P).to(io) for _ in range(nd)] for _ in range(2)]
+    B, Cm = [[(r(Bsz, L_, G, N) * N ** -0.5).to(io) for _ in range(nd)] for _ in range(2)]
+    dt = (torch.rand(Bsz, L_, H, N, generator=g, device="cuda") * 3 - 4).to(io)
+    A, bias, states = -torch.exp(torch.rand(H, N, generator=g, device="cuda") * 2.7), r(H, N) * 0.1, r(Bsz * nd, nc + 1, H, P, N)
+    fin = [r(Bsz, H, P, N) for _ in range(nd)]
+    a = L.ScanArgs()
+    d = a.dims
+    d.batch, d.seqlen, d.nheads, d.headdim, d.dstate, d.ngroups, d.chunk_size, d.ndir = Bsz, L_, H, P, N, G, 64, nd
+    a.io_dtype = a.dt_dtype = int(bf)
+    a.flags, a.dt_min, a.dt_max = L.FLAG_DT_SOFTPLUS, 0.0, float("inf")
+    for i in range(nd):
+        a.x[i], a.dout[i], a.Bm[i], a.Cm[i] = (L.tensor_desc(t[i]) for t in (x, dy, B, Cm))
+        if dfinal:
+            a.dfinal[i] = fin[i].data_ptr()
+    a.dt, a.A, a.dt_bias, a.stream = L.tensor_desc(dt), A.data_ptr(), bias.data_ptr(), torch.cuda.current_stream().cuda_stream
+    f = lambda *s: torch.full(s, float("nan"), device="cuda")
+    cs = f(Bsz * nd, nc, H, N)
+    L.check(lib.issm_stage_chunk_local(C.byref(a), f(Bsz * nd, nc + 1, H, P, N).data_ptr(), cs.data_ptr(), f(Bsz * nd, nc, H, 64, 64).data_ptr()), "local")
+    outs = []
+    for one in (False, True):
+        dst, dm, gl, dh0 = f(Bsz * nd, nc, H, P, N), torch.zeros(Bsz * nd, nc, H, 64, 64, device="cuda"), f(Bsz * nd, nc, H, N), f(nd, Bsz, H, P, N)
+        if one:
+            L.check(lib.issm_stage_bwd_states(C.byref(a), None, *(t.data_ptr() for t in (states, dst, dm, gl, dh0))), "states")
+        else:
+            L.check(lib.issm_stage_bwd_dstates(C.byref(a), None, dst.data_ptr(), dm.data_ptr()), "dstates")
+            L.check(lib.issm_stage_state_passing_bwd(C.byref(a), *(t.data_ptr() for t in (states, cs, dst, gl, dh0))), "passing")
+        torch.cuda.synchronize()
+        outs.append((dst, gl, dh0, dm.view(torch.int32)))
+    for name, p, q in zip(("dS", "g", "dh0"), *outs):
+        assert torch.isfinite(q).all() and (p.double() - q.double()).norm() <= 1e-6 * p.double().norm(), name
+    assert torch.equal(outs[0][3], outs[1][3])
+
+
 def test_inplace_edit_between_forward_and_backward_raises():
     """The operator saves its inputs for the backward as the reference does (issm_combined.py:42): changing one of them
     in place before backward must raise PyTorch's version-counter error, not return gradients of other data."""
