@@ -230,7 +230,7 @@ class Runner:
         Bt = B_ * nd
         f = lambda *s: torch.zeros(*s, device="cuda")
         st, csl, cabt = f(Bt, nc + 1, H, P, N), f(Bt, nc, H, N), f(Bt, nc, H, 64, 64)
-        dst, dm, gn, dh0d = f(Bt, nc, H, P, N), f(Bt, nc, H, 64, 64), f(Bt, nc, H, N), f(nd, B_, H, P, N)
+        dst, dm, dh0d = f(Bt, nc, H, P, N), f(Bt, nc, H, 64, 64), f(nd, B_, H, P, N)
         pa, pb, pd = f(Bt * nc, H, N), f(Bt * nc, H, N), f(Bt * nc * H, P)
         redo = torch.zeros(lib.issm_bwd_chunk_redo_ints(C.byref(a)), dtype=torch.int32, device="cuda")
         p = lambda t: t.data_ptr()
@@ -239,8 +239,8 @@ class Runner:
             ("state_passing_fwd", lambda: lib.issm_stage_state_passing_fwd(C.byref(a), p(st), p(csl))),
             ("chunk_scan", lambda: lib.issm_stage_chunk_scan(C.byref(a), p(st), p(cabt), None)),
             ("bwd_dstates", lambda: lib.issm_stage_bwd_dstates(C.byref(a), None, p(dst), p(dm))),
-            ("state_passing_bwd", lambda: lib.issm_stage_state_passing_bwd(C.byref(a), p(st), p(csl), p(dst), p(gn), p(dh0d))),
-            ("bwd_chunk", lambda: [lib.issm_stage_bwd_chunk(C.byref(a), d, None, p(st), p(dst), p(dm), p(gn), p(pa), p(pb), p(redo))
+            ("state_passing_bwd", lambda: lib.issm_stage_state_passing_bwd(C.byref(a), None, p(csl), p(dst), None, p(dh0d))),
+            ("bwd_chunk", lambda: [lib.issm_stage_bwd_chunk(C.byref(a), d, None, p(st), p(dst), p(dm), None, p(pa), p(pb), p(redo))
                                    for d in range(nd)][-1]),
             ("bwd_dx", lambda: lib.issm_stage_bwd_dx(C.byref(a), None, p(dst), p(cabt), p(pd))),
             ("bwd_reduce", lambda: lib.issm_stage_bwd_reduce(C.byref(a), p(pa), p(pb), p(pd), p(dh0d))),
@@ -269,8 +269,8 @@ class Runner:
         return res
 
 
-KERNEL_OF_STAGE = {"chunk_local": "k_local_tile", "state_passing_fwd": "k_state_fwd_full", "chunk_scan": "k_chunk_scan",
-                   "bwd_dstates": "k_bwd_dstates", "state_passing_bwd": "k_state_bwd_full", "bwd_chunk": "k_bwd_tile",
+KERNEL_OF_STAGE = {"chunk_local": "k_local_tile", "state_passing_fwd": "k_state_pass", "chunk_scan": "k_chunk_scan",
+                   "bwd_dstates": "k_bwd_dstates", "state_passing_bwd": "k_state_pass", "bwd_chunk": "k_bwd_tile",
                    "bwd_dx": "k_bwd_dx", "bwd_reduce": "k_bwd_reduce"}
 
 
@@ -315,13 +315,13 @@ def stage_work(ndir, shape=None, elt=4):
         "chunk_scan": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m)),
         # reads dt, C, dy, x; writes dH, dM
         "bwd_dstates": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m)),
-        # all launches: read dt, x, dy, B, C, H, dS, dM, g_last; write ddt, dB, dC, the dA / ddt_bias partials
+        # all launches: read dt, x, dy, B, C, H, dS, dM; write ddt, dB, dC, the dA / ddt_bias partials
         "bwd_chunk": (2 * U * (2 * cs * P * N + 2 * tri * N),
-                      s * (2 * E_dt + 2 * E_x + 4 * E_bc) + 4 * (2 * E_cs + E_m + 3 * E_v)),
+                      s * (2 * E_dt + 2 * E_x + 4 * E_bc) + 4 * (2 * E_cs + E_m + 2 * E_v)),
         # reads dt, B, dy, x, dS, M; writes dx
         "bwd_dx": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 3 * E_x) + 4 * (E_cs + E_m)),
         "state_passing_fwd": (0, 4 * (2 * E_cs + U * N + 2 * E_st)),
-        "state_passing_bwd": (0, 4 * (3 * E_cs + 2 * U * N + 2 * E_st)),
+        "state_passing_bwd": (0, 4 * (2 * E_cs + U * N + 2 * E_st)),
     }
     # whole step, compulsory traffic only: every caller tensor read once per pass, every output and gradient written
     # once, each direction counted with its own read of dt and initial states (a lower bound would share them)

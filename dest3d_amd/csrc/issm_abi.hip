@@ -19,17 +19,16 @@ int launch_state_fwd(const KP& p, float* states, const float* cs_last, hipStream
 int launch_chunk_scan(const KP& p, const float* states, const float* cabt, float* out_x, hipStream_t st);
 int launch_bwd_gate(const KP& p, const float* out_x, float* dy_ws, hipStream_t st);
 int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* dm, hipStream_t st);
-int launch_state_bwd(const KP& p, const float* states, const float* cs_last, float* dstates, float* g_last,
-                     float* dh0_dir, hipStream_t st);
+int launch_state_bwd(const KP& p, const float* cs_last, float* dstates, float* dh0_dir, hipStream_t st);
+int launch_state_sums(const KP& p, const float* states, const float* dstates, float* g_last, hipStream_t st);
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st);
+                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st);
 int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st);
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
-                          const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
+                          const float* dm, float* partA, float* partBias, const int* redo,
                           hipStream_t st);
 bool bwd_walk_available(const KP& p, const float* dy_ws);
-int launch_bwd_walk(const KP& p, const float* dy_ws, const float* states, float* dstates, float* dm, float* g_last, float* dh0_dir,
-                    hipStream_t st);
+int launch_bwd_walk(const KP& p, const float* dy_ws, float* dstates, float* dm, float* dh0_dir, hipStream_t st);
 int launch_bwd_dx(const KP& p, const float* dy_ws, const float* dstates, const float* cabt, float* partD,
                   hipStream_t st);
 int launch_bwd_reduce(const KP& p, const float* partA, const float* partBias, const float* partD,
@@ -112,7 +111,7 @@ struct FwdWs {
   size_t states, cs_last, cabt, out_x, total;  // offsets in floats
 };
 struct BwdWs {
-  size_t dstates, dm, g_last, dh0_dir, partA, partBias, partD, redo, dy_ws, ddt_part, dbc_part, total;
+  size_t dstates, dm, dh0_dir, partA, partBias, partD, redo, dy_ws, ddt_part, dbc_part, total;
 };
 
 static int nchunks(const issm_dims& d) { return (d.seqlen + ISSM_CHUNK - 1) / ISSM_CHUNK; }
@@ -144,14 +143,15 @@ static int bwd_head_parts(const issm_dims& d) {
   return (heads - each) * d.ndir < 4 ? 1 : (int)((heads + each - 1) / each);   // (no part without a head)
 }
 
-// Whether the backward's states take one kernel (issm_bwd_walk.hip) or two.  A walk takes 2 - 3 us a chunk whatever the grid, until the
-// chip is full of them; two kernels take 13 - 25 us and then what the chip's share of the chunks costs.  So: every CU has a walk
-// (256: 8 x 4096 tokens, 8 heads x 32, 256 states fp32 190 against 230 us, 4 x 1024, two directions 41 against 43; bf16 147 and 167,
-// 33 and 38), or few chunks (7 chunks of 32 - 128 walks: 16 - 17 against 19 - 23 us; 8 of 32 with 200 states: 25 against 24;
-// 16 of 64: 35 against 27), or in between (192 walks: 16 chunks 39 against 40 us; 64 chunks would be about 140 against 117).
+// Whether the backward's states take one kernel (issm_bwd_walk.hip) or two.  A walk takes 2 us a chunk whatever the grid, until the
+// chip is full of them; two kernels take 12 - 20 us and then what the chip's share of the chunks costs.  So: every CU has a walk
+// (256: 8 x 4096 tokens, 8 heads x 32, 256 states fp32 174 against 208 us, 4 x 1024, two directions 39 against 40; bf16 119 and 152,
+// 30 and 35), or few chunks (8 chunks of 32, 128, 192 walks: 17.4, 19, 20 against 17.6, 21, 25 us fp32, 15, 16, 17 against 16, 20, 24
+// bf16; 16 of 64: 33 against 22), or in between (192 walks: 16 chunks 35.6 against 34.3 - 35.9 us fp32, 29 against 31 bf16; 64 chunks
+// 144 against 138, 100 against 95).
 static bool bwd_walks(const KP& p, const float* dy) {
   const int walks = p.B * p.ndir * p.H * ((p.N + 63) / 64);
-  return (walks >= 256 || p.nc <= 7 || (walks >= 192 && p.nc <= 16)) && bwd_walk_available(p, dy);
+  return (walks >= 256 || p.nc <= 8 || (walks >= 192 && p.nc <= 16)) && bwd_walk_available(p, dy);
 }
 
 static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
@@ -166,7 +166,6 @@ static BwdWs bwd_layout(const issm_scan_args* a) {
   size_t o = 0;
   w.dstates = o; o += align64(Bt * nc * H * P * N);
   w.dm = o; o += align64(Bt * nc * H * ISSM_CHUNK * ISSM_CHUNK);
-  w.g_last = o; o += align64(Bt * nc * H * N);
   w.dh0_dir = o; o += align64((size_t)d.ndir * d.batch * H * P * N);
   w.partA = o; o += align64(Bt * nc * H * N);
   w.partBias = o; o += align64(Bt * nc * H * N);
@@ -388,10 +387,11 @@ int issm_stage_state_passing_bwd(const issm_scan_args* a, const float* states, c
                                  float* g_last, float* dh0_dir) {
   int rc = check_dims(a);
   if (rc) return rc;
-  if (!states || !cs_last || !dstates || !g_last || !dh0_dir) return fail(ISSM_E_NULL, "state_passing_bwd: NULL buffer");
+  if (!cs_last || !dstates || !dh0_dir || (g_last && !states)) return fail(ISSM_E_NULL, "state_passing_bwd: NULL buffer");
   KP p = make_kp(a);
-  return launched(launch_state_bwd(p, states, cs_last, dstates, g_last, dh0_dir, (hipStream_t)a->stream),
-                  "state_passing_bwd");
+  hipStream_t st = (hipStream_t)a->stream;
+  if ((rc = launched(launch_state_bwd(p, cs_last, dstates, dh0_dir, st), "state_passing_bwd")) || !g_last) return rc;
+  return launched(launch_state_sums(p, states, dstates, g_last, st), "state_passing_bwd (sums)");
 }
 
 int issm_stage_bwd_states(const issm_scan_args* a, const float* dy_gated, const float* states, float* dstates, float* dm,
@@ -399,10 +399,12 @@ int issm_stage_bwd_states(const issm_scan_args* a, const float* dy_gated, const 
   int rc = check_common(a);
   if (rc) return rc;
   if ((rc = check_dout(a, dy_gated))) return rc;
-  if (!states || !dstates || !dm || !g_last || !dh0_dir) return fail(ISSM_E_NULL, "bwd_states: NULL buffer");
+  if (!dstates || !dm || !dh0_dir || (g_last && !states)) return fail(ISSM_E_NULL, "bwd_states: NULL buffer");
   KP p = make_kp(a);
   if (!bwd_walk_available(p, dy_gated)) return fail(ISSM_E_UNSUPPORTED, "bwd_states: packed sequences, mixed types, or rows of x or dy that are no multiple of four elements");
-  return launched(launch_bwd_walk(p, dy_gated, states, dstates, dm, g_last, dh0_dir, (hipStream_t)a->stream), "bwd_states");
+  hipStream_t st = (hipStream_t)a->stream;
+  if ((rc = launched(launch_bwd_walk(p, dy_gated, dstates, dm, dh0_dir, st), "bwd_states")) || !g_last) return rc;
+  return launched(launch_state_sums(p, states, dstates, g_last, st), "bwd_states (sums)");
 }
 
 size_t issm_bwd_chunk_redo_ints(const issm_scan_args* a) {
@@ -412,22 +414,22 @@ size_t issm_bwd_chunk_redo_ints(const issm_scan_args* a) {
 }
 
 int issm_stage_bwd_chunk(const issm_scan_args* a, int dir, const float* dy_gated, const float* states,
-                         const float* dstates, const float* dm, const float* g_last, float* part_a,
+                         const float* dstates, const float* dm, const float* /*g_last*/, float* part_a,
                          float* part_bias, int32_t* redo) {
   int rc = check_common(a);
   if (rc) return rc;
   if ((rc = check_dout(a, dy_gated))) return rc;
   if (dir < 0 || dir >= a->dims.ndir) return fail(ISSM_E_SHAPE, "dir %d out of range", dir);
-  if (!states || !dstates || !dm || !g_last || !part_a || !part_bias) return fail(ISSM_E_NULL, "bwd_chunk: NULL buffer");
+  if (!states || !dstates || !dm || !part_a || !part_bias) return fail(ISSM_E_NULL, "bwd_chunk: NULL buffer");
   KP p = make_kp(a);
   p.dir0 = dir;
   int pending = 0;
-  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, g_last, part_a, part_bias, redo, &pending, 1,
+  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1,
                                       (hipStream_t)a->stream),
                      "bwd_chunk")))
     return rc;
   if (!pending) return ISSM_OK;
-  return launched(launch_bwd_chunk_redo(p, 1, dy_gated, states, dstates, dm, g_last, part_a, part_bias, redo,
+  return launched(launch_bwd_chunk_redo(p, 1, dy_gated, states, dstates, dm, part_a, part_bias, redo,
                                         (hipStream_t)a->stream),
                   "bwd_chunk (redo)");
 }
@@ -477,15 +479,10 @@ int issm_scan_bwd(const issm_scan_args* a) {
     dy = ws + bw.dy_ws;
   }
   if (bwd_walks(p, dy)) {
-    if ((rc = launched(launch_bwd_walk(p, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last, ws + bw.dh0_dir, st),
-                       "bwd_states")))
-      return rc;
+    if ((rc = launched(launch_bwd_walk(p, dy, ws + bw.dstates, ws + bw.dm, ws + bw.dh0_dir, st), "bwd_states"))) return rc;
   } else {
     if ((rc = launched(launch_bwd_dstates(p, dy, ws + bw.dstates, ws + bw.dm, st), "bwd_dstates"))) return rc;
-    if ((rc = launched(launch_state_bwd(p, sv + fw.states, sv + fw.cs_last, ws + bw.dstates, ws + bw.g_last,
-                                        ws + bw.dh0_dir, st),
-                       "state_passing_bwd")))
-      return rc;
+    if ((rc = launched(launch_state_bwd(p, sv + fw.cs_last, ws + bw.dstates, ws + bw.dh0_dir, st), "state_passing_bwd"))) return rc;
   }
   int* redo = reinterpret_cast<int*>(ws + bw.redo);
   int pending = 0;
@@ -505,7 +502,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
   for (int dir = 0; dir < p.ndir; ++dir) {
     KP pd = pc;
     pd.dir0 = dir;
-    if ((rc = launched(launch_bwd_chunk(pd, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last,
+    if ((rc = launched(launch_bwd_chunk(pd, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm,
                                         ws + bw.partA, ws + bw.partBias, redo, &pending, parts, st),
                        "bwd_chunk")))
       return rc;
@@ -515,7 +512,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
   for (int dir = 0; pending && dir < p.ndir; dir += together) {
     KP pd = p;
     pd.dir0 = dir;
-    if ((rc = launched(launch_bwd_chunk_redo(pd, together, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm, ws + bw.g_last,
+    if ((rc = launched(launch_bwd_chunk_redo(pd, together, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm,
                                              ws + bw.partA, ws + bw.partBias, redo, st),
                        "bwd_chunk (redo)")))
       return rc;

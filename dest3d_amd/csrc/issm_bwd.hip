@@ -2,7 +2,6 @@
 //
 //   k_bwd_gate      z-gate backward (elementwise)
 //   k_bwd_dstates   dH_c = dy^T (C*exp(cs))  and  dM = tril(dy x^T)
-//   k_state_bwd_full / k_state_bwd   reverse inter-chunk recurrence (HBM streaming)
 //   k_bwd_chunk     per (chunk, group, 64-column slice), looping over the heads of the
 //                   group: ddt, dB, dC and the per-unit partial sums of dA / ddt_bias; for the
 //                   calls and heads that k_bwd_tile (issm_bwd_tile.hip) does not take
@@ -14,8 +13,8 @@
 //   G[m] = sum_{l>=m} dM[l,m] C[l] E(l,m),  F[l] = sum_{s<=l} dM[l,s] Bd[s] E(l,s),
 //   E1 = exp(cs_last-cs) Q + G,   X2 = exp(cs) R + F
 // the gradients are dB = sum_heads dt' E1, dC = sum_heads X2, ddt' = B E1 + A da,
-// da[k] = sum_{l>=k} (C X2 - Bd E1)[l] + (sum_p dS[p] H_next[p]), the last term entering at
-// the chunk's last row.  G and F carry the decay inside the contraction; they use the same
+// da[k] = sum_{l>=k} (C X2 - Bd E1)[l] + (sum_p dS[p] H_next[p]), the last term, the states' gradient to the
+// chunk's total, being exp(cs_last) sum_p dS[p] H[p] + sum_l (Bd exp(cs_last-cs) Q)[l].  G and F carry the decay inside the contraction; they use the same
 // binary row hierarchy as the forward intra-chunk matrix (see issm_fwd.hip).
 #include "issm_dev.h"
 
@@ -190,305 +189,6 @@ __device__ __forceinline__ void k_bwd_dstates_body(const KP& p, const float* __r
 template <int PT, bool IOB, bool DTB, bool FULL>
 __global__ __launch_bounds__(NTHREADS, (PT <= 3 && !FULL) ? 4 : 1) void k_bwd_dstates(KP p, const float* __restrict__ dy_ws, float* __restrict__ dstates, float* __restrict__ dm) {
   k_bwd_dstates_body<PT, IOB, DTB, FULL>(p, dy_ws, dstates, dm);
-}
-
-// ------------------------------------------------------- reverse state passing
-// Block = (bt, h, 64 state columns); thread (pg = tid >> 4, nq = tid & 15) carries rows
-// p = pg, pg+16, ... of 4 adjacent columns.  dstates[c] holds dH_c on entry and dS_c (gradient
-// of the chunk-local end state) on exit.  g_last[c][n] = sum_p dS_c[p,n] * H_{c+1}[p,n].
-template <int NQ>
-__global__ __launch_bounds__(NTHREADS) void k_state_bwd(KP p, const float* __restrict__ states,
-                                                        const float* __restrict__ cs_last,
-                                                        float* __restrict__ dstates, float* __restrict__ g_last,
-                                                        float* __restrict__ dh0_dir) {
-  // NQ column quads per workgroup: NCOL columns, PGN row groups, a thread carries rows pg, pg + PGN, ...
-  constexpr int NCOL = NQ * 4, PGN = NTHREADS / NQ, KR = (MAXP + PGN - 1) / PGN;
-  __shared__ float red[PGN * NCOL];
-  const int nsl = (p.N + NCOL - 1) / NCOL;
-  int bid = blockIdx.x;
-  const int ns = bid % nsl;
-  bid /= nsl;
-  const int h = bid % p.H;
-  const int bt = bid / p.H;
-  const int b = bt / p.ndir, dir = bt % p.ndir;
-  const int tid = threadIdx.x, pg = tid / NQ, nq = tid % NQ;
-  const int n = ns * NCOL + nq * 4;
-  const bool vec = ((p.N & 3) == 0) && (n + 3 < p.N);
-  float carry[KR][4];
-#pragma unroll
-  for (int k = 0; k < KR; ++k) {
-    const int pp = pg + PGN * k;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool v = pp < p.P && n + j < p.N && p.dfinal[dir];
-      carry[k][j] = v ? p.dfinal[dir][(((long)b * p.H + h) * p.P + pp) * p.N + n + j] : 0.0f;
-    }
-  }
-  // operands of one chunk: decay exponent, H_{c+1} and dH_c of the thread's rows
-  auto load_chunk = [&](int c, float (&dec)[4], float (&hn)[KR][4], float (&dh)[KR][4]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dec[j] = n + j < p.N ? cs_last[vec_off(p, bt, c, h) + n + j] : 0.0f;
-#pragma unroll
-    for (int k = 0; k < KR; ++k) {
-      const int pp = pg + PGN * k;
-      const float* hp = states + st_off(p, bt, c + 1, h) + (long)pp * p.N + n;
-      const float* dd = dstates + dst_off(p, bt, c, h) + (long)pp * p.N + n;
-      if (vec && pp < p.P) {
-        const f4 a = *(const f4*)hp, d = *(const f4*)dd;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { hn[k][j] = a[j]; dh[k][j] = d[j]; }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const bool v = pp < p.P && n + j < p.N;
-          hn[k][j] = v ? hp[j] : 0.0f;
-          dh[k][j] = v ? dd[j] : 0.0f;
-        }
-      }
-    }
-  };
-  // The operands of the next two chunks are always in flight (the loads do not depend on the carry), so the
-  // recurrence never waits for memory and enough bytes are outstanding to keep HBM busy.
-  float dec[4], hn[KR][4], dh[KR][4], dec_1[4], hn_1[KR][4], dh_1[KR][4];
-  load_chunk(p.nc - 1, dec, hn, dh);
-  if (p.nc > 1) load_chunk(p.nc - 2, dec_1, hn_1, dh_1);
-  for (int c = p.nc - 1; c >= 0; --c) {
-    float gp[4] = {0, 0, 0, 0};
-    float dec_n[4], hn_n[KR][4], dh_n[KR][4];
-    if (c > 1) load_chunk(c - 2, dec_n, hn_n, dh_n);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dec[j] = __expf(dec[j]);
-#pragma unroll
-    for (int k = 0; k < KR; ++k) {
-      const int pp = pg + PGN * k;
-      float* dd = dstates + dst_off(p, bt, c, h) + (long)pp * p.N + n;
-      if (vec && pp < p.P) {
-        *(f4*)dd = (f4){carry[k][0], carry[k][1], carry[k][2], carry[k][3]};
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (pp < p.P && n + j < p.N) dd[j] = carry[k][j];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        gp[j] += hn[k][j] * carry[k][j];
-        carry[k][j] = dec[j] * carry[k][j] + dh[k][j];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) red[pg * NCOL + nq * 4 + j] = gp[j];
-    __syncthreads();
-    if (tid < 64) {
-      // 64 lanes over NCOL columns: a lane sums every (64 / NCOL)-th row group of its column, then the lanes of a
-      // column (NCOL apart) are added
-      constexpr int PARTS = 64 / NCOL;
-      const int col = tid % NCOL, part = tid / NCOL;
-      float sum = 0.0f;
-#pragma unroll
-      for (int k = 0; k < PGN / PARTS; ++k) sum += red[(k * PARTS + part) * NCOL + col];
-#pragma unroll
-      for (int d = NCOL; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
-      if (part == 0 && ns * NCOL + col < p.N) g_last[vec_off(p, bt, c, h) + ns * NCOL + col] = sum;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { dec[j] = dec_1[j]; dec_1[j] = dec_n[j]; }
-#pragma unroll
-    for (int k = 0; k < KR; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        hn[k][j] = hn_1[k][j]; dh[k][j] = dh_1[k][j];
-        hn_1[k][j] = hn_n[k][j]; dh_1[k][j] = dh_n[k][j];
-      }
-  }
-#pragma unroll
-  for (int k = 0; k < KR; ++k) {
-    const int pp = pg + PGN * k;
-    if (pp >= p.P) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (n + j < p.N) dh0_dir[((((long)dir * p.B + b) * p.H + h) * p.P + pp) * p.N + n + j] = carry[k][j];
-  }
-}
-
-// The same recurrence with no conditional access in its loop: every load is issued on every path, so the compiler can
-// count the loads still in flight and the prefetched operands of
-// the next chunks stay in flight across the barrier (with loads inside branches it waits for all of them before each
-// store, which exposes the full memory latency once per chunk; few workgroups walking many chunks -- batch 2, 256
-// chunks -- then run at that pace).  A thread owns KM rows, pg + PGN k; for rows past the head dimension it stands in
-// for the head's last row: it issues the same loads (so that every load of the loop is unconditional) but stores
-// nothing and adds nothing to the column sums -- what a stand-in computes is never used, so it does not matter that
-// the row's owner overwrites dH with dS while the stand-in's prefetches of that row are in flight.
-// TAIL (N >= 4, not a multiple of the slice width; accesses at any float): a column quad that crosses or lies past N is
-// columns N - 4 .. N - 1 instead, once more.  The threads that own a column twice sit in one wave (the quads of a row are
-// adjacent lanes), issue their loads and stores of it in the same instructions and compute the same values, so storing
-// twice is harmless; a column's sum is formed per quad, and stored twice as well.  Columns such a quad shares with the
-// previous slice are that workgroup's alone to store.  8 x 1024 tokens, 8 heads, N = 250:
-// 53.4 us with per-element guards, N = 256 without: 17.6.
-template <int NQ, int KM, int R, bool BATCH, bool TAIL>
-__global__ __launch_bounds__(NTHREADS) void k_state_bwd_full(KP p, const float* __restrict__ states,
-                                                             const float* __restrict__ cs_last,
-                                                             float* __restrict__ dstates, float* __restrict__ g_last,
-                                                             float* __restrict__ dh0_dir) {
-  constexpr int NCOL = NQ * 4, PGN = NTHREADS / NQ;
-  // The column sums g = sum_p H dS need the rows of all four waves.  Two ways to add them up:
-  //  - per step (BATCH = false): every thread leaves its partial sums in local memory and, behind the step's barrier,
-  //    the first wave adds each column's PGN of them.  That exchange (local-memory round trips one after the other)
-  //    lies on the path from one chunk to the next, which a chip full of workgroups hides: from 256 workgroups on
-  //    this form is as fast as the other or up to 10 % faster;
-  //  - K steps at once (BATCH = true): the steps only deposit partial sums -- 16 per column: a wave's lanes of one
-  //    16-lane row share a column quad, after one in-row rotation for NQ = 8 -- and one thread per (step, column)
-  //    adds them behind one barrier per K steps.  With few workgroups walking hundreds of chunks the pace of the
-  //    exchange is the run time: 1.3-1.6x faster up to 128 workgroups (batch 2, 256 chunks: 145 -> 110 us).
-  // Two buffers, used in turn, either way.
-  constexpr int K = !BATCH ? 1 : R * NCOL <= NTHREADS ? R : R / 2;
-  static_assert(R % K == 0 && K * NCOL <= NTHREADS && (NQ == 8 || NQ == 16), "batches of K steps tile the ring");
-  __shared__ __align__(16) float red2[2][BATCH ? K * NCOL * 16 : PGN * NCOL];
-  int par = 0;
-  const int nsl = (p.N + NCOL - 1) / NCOL;
-  int bid = blockIdx.x;
-  const int ns = bid % nsl;
-  bid /= nsl;
-  const int h = bid % p.H;
-  const int bt = bid / p.H;
-  const int b = bt / p.ndir, dir = bt % p.ndir;
-  const int tid = threadIdx.x, pg = tid / NQ, nq = tid % NQ;
-  const int n = TAIL ? min(ns * NCOL + nq * 4, p.N - 4) : ns * NCOL + nq * 4;
-  // column `col` of the workgroup's slice (quad col / 4, entry col % 4), relative to the slice's first
-  auto col_at = [&](int col) { return TAIL ? min(col & ~3, p.N - 4 - ns * NCOL) + (col & 3) : col; };
-  auto ld = [](const float* a) -> f4 {
-    if constexpr (TAIL) return ld_f4_any(a);
-    else return *(const f4*)a;
-  };
-  const int foreign = TAIL ? max(ns * NCOL - n, 0) : 0;   // first columns of the quad that are another workgroup's
-  auto put = [&](float* a, f4 v) {
-    if constexpr (!TAIL) {
-      *(f4*)a = v;
-    } else if (foreign == 0) {
-      st_f4_any(a, v);
-    } else {
-#pragma unroll
-      for (int j = 1; j < 4; ++j)
-        if (j >= foreign) a[j] = v[j];
-    }
-  };
-  const int part = (tid >> 6) * 4 + ((tid & 63) >> 4);  // (wave, 16-lane row): which of a column's 16 partial sums
-  const bool deposits = NQ == 16 || !(tid & 8);
-  long rowk[KM];   // offsets of the thread's rows
-  bool own[KM];    // a row of its own (stores, takes part in the column sums) or a stand-in (loads only)
-#pragma unroll
-  for (int k = 0; k < KM; ++k) {
-    rowk[k] = (long)min(pg + PGN * k, p.P - 1) * p.N + n;
-    own[k] = pg + PGN * k < p.P;
-  }
-  const long cstep = (long)p.H * p.P * p.N, vstep = (long)p.H * p.N;  // from chunk to chunk
-  f4 carry[KM];
-#pragma unroll
-  for (int k = 0; k < KM; ++k) {
-    carry[k] = (f4){0, 0, 0, 0};
-    if (p.dfinal[dir]) carry[k] = ld(p.dfinal[dir] + ((long)b * p.H + h) * p.P * p.N + rowk[k]);
-  }
-  const float* hp = states + st_off(p, bt, p.nc, h);      // H_{c+1}, c = nc - 1
-  float* dd = dstates + dst_off(p, bt, p.nc - 1, h);      // dH_c in, dS_c out
-  const float* cl = cs_last + vec_off(p, bt, p.nc - 1, h) + n;
-  float* gl = g_last + vec_off(p, bt, p.nc - 1, h) + ns * NCOL;  // of the first step of the current batch
-  // Operands of R chunks in R register slots: the one being used and the next R - 1, the last of which is requested
-  // at the top of a step (the final steps request chunk 0 again: in range, unused).  Step j = nc-1-c uses slot
-  // j % R; the loop is unrolled over the slots so that none is ever copied (a copy would wait for its load).
-  f4 dec[R], hn[R][KM], dh[R][KM];
-  auto request = [&](int slot, int back_chunks) {
-    const long back = (long)back_chunks * cstep;
-    dec[slot] = ld(cl - (long)back_chunks * vstep);
-#pragma unroll
-    for (int k = 0; k < KM; ++k) {
-      hn[slot][k] = ld(hp - back + rowk[k]);
-      dh[slot][k] = ld(dd - back + rowk[k]);
-    }
-  };
-#pragma unroll
-  for (int i = 0; i < R - 1; ++i) request(i, min(i, p.nc - 1));
-  auto step = [&](int cur, int pre, int c) {
-    request(pre, min(c, R - 1));
-    f4 gp = {0, 0, 0, 0}, e;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) e[j] = __expf(dec[cur][j]);
-#pragma unroll
-    for (int k = 0; k < KM; ++k) {
-      if (own[k]) put(dd + rowk[k], carry[k]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        gp[j] += own[k] ? hn[cur][k][j] * carry[k][j] : 0.0f;
-        carry[k][j] = e[j] * carry[k][j] + dh[cur][k][j];
-      }
-    }
-    if (!BATCH) {
-      *(f4*)(red2[par] + pg * NCOL + nq * 4) = gp;
-    } else {
-      if (NQ == 8) {
-        // lanes l and l ^ 8 of a 16-lane row hold the same column quad: rotate the row by 8 and add
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float own_sum = gp[j];  // a scalar copy: the bit cast below must not be applied to a vector element
-          gp[j] = own_sum + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                                          0, __builtin_bit_cast(int, own_sum), 0x128, 0xf, 0xf, false));
-        }
-      }
-      if (deposits) {
-        // the 16 partial sums of a column are added in the order of their places, whatever lane filled them: the
-        // place is rotated by the column so that a wave's stores spread over the banks
-        float* red = red2[par] + ((cur % K) * NCOL + nq * 4) * 16;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) red[j * 16 + ((part + nq * 4 + j) & 15)] = gp[j];
-      }
-    }
-    hp -= cstep; dd -= cstep; cl -= vstep;
-  };
-  // The column sums of the batch's first cnt steps: thread = (step, column).
-  auto add_up = [&](int cnt) {
-    __syncthreads();  // the other buffer is filled next; this one again after the next barrier
-    if (!BATCH) {
-      if (tid < 64) {
-        // 64 lanes over NCOL columns: a lane sums every (64 / NCOL)-th row group of its column, then the lanes of a
-        // column (NCOL apart) are added
-        constexpr int PARTS = 64 / NCOL;
-        const int col = tid % NCOL, prt = tid / NCOL;
-        const float* red = red2[par];
-        float sum = 0.0f;
-#pragma unroll
-        for (int k = 0; k < PGN / PARTS; ++k) sum += red[(k * PARTS + prt) * NCOL + col];
-#pragma unroll
-        for (int d = NCOL; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
-        if (prt == 0 && (!TAIL || col_at(col) >= 0)) gl[col_at(col)] = sum;
-      }
-    } else if (tid < cnt * NCOL) {
-      const f4* r = (const f4*)(red2[par] + tid * 16);
-      const f4 a = r[0], b4 = r[1], c4 = r[2], d4 = r[3];
-      const f4 s4 = (a + b4) + (c4 + d4);
-      if (!TAIL || col_at(tid % NCOL) >= 0)
-        gl[-(long)(tid / NCOL) * vstep + col_at(tid % NCOL)] = (s4[0] + s4[1]) + (s4[2] + s4[3]);
-    }
-    gl -= (long)cnt * vstep;
-    par ^= 1;
-  };
-  int c = p.nc - 1;
-  for (; c >= R - 1; c -= R) {
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      step(i, (i + R - 1) % R, c - i);
-      if ((i + 1) % K == 0) add_up(K);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < R - 1; ++i) {  // uniform: the last nc % R chunks
-    if (c - i >= 0) {
-      step(i, (i + R - 1) % R, c - i);
-      if ((i + 1) % K == 0) add_up(K);
-      else if (c - i == 0) add_up(i % K + 1);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < KM; ++k)
-    if (own[k]) put(dh0_dir + (((long)dir * p.B + b) * p.H + h) * p.P * p.N + rowk[k], carry[k]);
 }
 
 // -------------------------------------------------------------- chunk backward
@@ -668,7 +368,7 @@ __device__ __forceinline__ void bwd_small_levels(const float (&cs)[16], const fl
 
 // partA, partBias: (Bt*nc, H, N) per-unit partial sums of dA and ddt_bias
 template <int PT, bool IOB, bool DTB, bool FULL>
-__device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, const int dir_here, const bool mirror) {
+__device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, const int dir_here, const bool mirror) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdChunkSmem<PT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
@@ -724,7 +424,6 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
     float raw[16], dsv[KP_], hv[KP_];
     lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
     const Coef cf = lane_coef(p, u.h, n, vn);
-    const float gl_any = g_last[vec_off(p, u.bt, u.c, u.h) + (vn ? n : 0)], gl = g4 == 3 ? gl_any : 0.0f;
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, dsv);
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, hv);
     f4 mkeep[SM::DM_OVER_X ? 4 : 1];  // the thread's part of the dM tile until the x tile's place is free
@@ -765,6 +464,10 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
     int cq = cm, gq = g4;
     asm volatile("" : "+v"(cq), "+v"(gq));
     float e1[16], x2[16];
+    // the states' gradient to the chunk's total (see k_bwd_tile): the lane's share
+    float gsum = ex2(last) * lane_dot_pn<KP_>(dsv, hv, p.P, g4, pn_full);
+    asm volatile("" : "+v"(gsum));
+    __builtin_amdgcn_sched_barrier(0);
     {
       // Q = x . dS and R = dy . H contract over the head dimension: split-bf16 products, K = 32 per step.
       // k-slot s of step t <-> lane value q = 8 t + s <-> p = 16 (q >> 2) + 4 g4 + (q & 3).
@@ -826,6 +529,10 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
       }
     }
 
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gsum += Bd[k] * e1[k];
+    asm volatile("" : "+v"(gsum));
     if constexpr (SM::DM_OVER_X) {
       __syncthreads();  // every wave is done with the x tile
       int tq = tid;
@@ -871,7 +578,8 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
       val[k] = Bv[k] * E1;
       dcs[k] = Cv[k] * X2 - Bd[k] * E1;
     }
-    dcs[15] += gl;
+    gsum += __shfl_xor(gsum, 16, 64);
+    gsum += __shfl_xor(gsum, 32, 64);
     {
       // suffix sums up the 64 rows; the cross-lane steps of the four tiles are issued together (see lane_prep)
       float c[4], v[4], t[4];
@@ -895,7 +603,7 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
       for (int J = 0; J < 4; ++J) v[J] = g4 <= 1 ? v[J] + t[J] : v[J];  // inclusive from the last lane group down
 #pragma unroll
       for (int J = 0; J < 4; ++J) t[J] = __shfl(v[J], cm, 64);           // tile totals
-      float carry = 0.0f;  // sum over all rows after the current tile
+      float carry = gsum;  // sum over all rows after the current tile, and the gradient to the chunk's total
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
         const float add = carry + (v[J] - c[J]);
@@ -944,11 +652,11 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
   }
 }
 template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, int ndirs) {
+__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, int ndirs) {
   // (ndirs > 1 only with `redo`: the marked heads of directions p.dir0, p.dir0 + 1, .. one after the other)
   for (int d = 0; d < ndirs; ++d) {
     if (d) __syncthreads();
-    k_bwd_chunk_body<PT, IOB, DTB, FULL>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, p.dir0 + d, d > 0);
+    k_bwd_chunk_body<PT, IOB, DTB, FULL>(p, dy_ws, states, dstates, dm, partA, partBias, redo, p.dir0 + d, d > 0);
   }
 }
 
@@ -1146,7 +854,7 @@ __device__ __forceinline__ void bwd_small_levels_bf(const float (&cs)[16], const
 }
 
 template <int PT, bool DTB, bool FULL>
-__device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, const int dir_here, const bool mirror) {
+__device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, const int dir_here, const bool mirror) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdChunkBfSmem<PT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
@@ -1231,7 +939,6 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
     float raw[16], dsv[KP_], hv[KP_];
     lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
     const Coef cf = lane_coef(p, u.h, n, vn);
-    const float gl_any = g_last[vec_off(p, u.bt, u.c, u.h) + (vn ? n : 0)], gl = g4 == 3 ? gl_any : 0.0f;
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, dsv);
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, u.h), p.P, p.N, n, vn, g4, pn_full, hv);
     request(u.h);
@@ -1250,11 +957,13 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
     int cq = cm, gq = g4;
     asm volatile("" : "+v"(cq), "+v"(gq));
     float e1[16], x2[16];
+    // the states' gradient to the chunk's total (see k_bwd_tile): the lane's share
+    float gsum = ex2(last) * lane_dot_pn<KP_>(dsv, hv, p.P, g4, pn_full);
+    asm volatile("" : "+v"(gsum));
+    __builtin_amdgcn_sched_barrier(0);
     {
       // Q = x . dS and R = dy . H over the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s.
-      // x and dy are exact in bf16; dS and H are fp32 states and enter as (hi, lo) pairs -- two instructions per step:
-      // the last row's Bd . E1 cancels against the state term g = sum_p dS H_next in d/d(cs), and a dS rounded to 8
-      // bits would leave that difference with a relative error far above the bf16 level.
+      // x and dy are exact in bf16; dS and H are fp32 states and enter as (hi, lo) pairs -- two instructions per step.
       bf8 dsh[KT], dsl[KT], hh_[KT], hl_[KT];
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
@@ -1289,6 +998,9 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
     }
 
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gsum += Bv[k] * dtp[k] * e1[k];
+    asm volatile("" : "+v"(gsum));
     asm volatile("" : "+v"(cq), "+v"(gq));
     pin16(cs); pin16(e1); pin16(x2);
     bwd_small_levels_bf<LDM>(cs, Bv, dtp, Cv, dm_, e1, x2, gq);
@@ -1332,7 +1044,8 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
       s.dbc[(16 + k) * NTHREADS + tid] += X2;
       val[k] = Bv[k] * E1;
     }
-    dcs[15] += gl;
+    gsum += __shfl_xor(gsum, 16, 64);
+    gsum += __shfl_xor(gsum, 32, 64);
     {
       float c[4], v[4], t[4];
 #pragma unroll
@@ -1355,7 +1068,7 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
       for (int J = 0; J < 4; ++J) v[J] = g4 <= 1 ? v[J] + t[J] : v[J];
 #pragma unroll
       for (int J = 0; J < 4; ++J) t[J] = __shfl(v[J], cm, 64);
-      float carry = 0.0f;
+      float carry = gsum;
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
         const float add = carry + (v[J] - c[J]);
@@ -1407,10 +1120,10 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   }
 }
 template <int PT, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, const float* __restrict__ g_last, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, int ndirs) {
+__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states, const float* __restrict__ dstates, const float* __restrict__ dm, float* __restrict__ partA, float* __restrict__ partBias, const int* __restrict__ redo, int ndirs) {
   for (int d = 0; d < ndirs; ++d) {
     if (d) __syncthreads();
-    k_bwd_chunk_bf_body<PT, DTB, FULL>(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, p.dir0 + d, d > 0);
+    k_bwd_chunk_bf_body<PT, DTB, FULL>(p, dy_ws, states, dstates, dm, partA, partBias, redo, p.dir0 + d, d > 0);
   }
 }
 
@@ -1829,59 +1542,24 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
   return (int)hipGetLastError();
 }
 
-int launch_state_bwd(const KP& p, const float* states, const float* cs_last, float* dstates, float* g_last,
-                     float* dh0_dir, hipStream_t st) {
-  // One workgroup walks the chunks of its columns one after the other.  From four columns on the accesses are
-  // unconditional (TAIL: the last slice is not full); with few (batch, head) pairs narrower column slices put more workgroups on the chip.
-  const int wide = p.B * p.ndir * p.H * ((p.N + 63) / 64);
-  // (sequence of the tests: slices of 32 columns where 64 would leave the chip idle or N fits them exactly)
-#define ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, TAIL_)                                                                         \
-  hipLaunchKernelGGL((k_state_bwd_full<NQ_, KM_, R_, BATCH_, TAIL_>), dim3(p.B * p.ndir * p.H * ((p.N + 4 * NQ_ - 1) / (4 * NQ_))), \
-                     dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir)
-#define ISSM_STATE_BWD_FULL(NQ_, KM_, R_, BATCH_)                                                   \
-  do {                                                                                              \
-    if (p.N % (4 * NQ_)) ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, true);                              \
-    else ISSM_STATE_BWD_T(NQ_, KM_, R_, BATCH_, false);                                             \
-  } while (0)
-  if (p.N < 4) {
-    const int blocks = p.B * p.ndir * p.H * ((p.N + 15) / 16);
-    hipLaunchKernelGGL(k_state_bwd<4>, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last, dstates, g_last, dh0_dir);
-  } else if (wide < 256 || (p.N % 64 != 0 && (p.N + 63) / 64 * 2 != (p.N + 31) / 32)) {
-    // few workgroups walking many chunks: the column sums of several steps behind one barrier
-    const bool batch = p.B * p.ndir * p.H * ((p.N + 31) / 32) <= 128 && p.nc >= 32;
-    if (p.P <= 32) { if (batch) ISSM_STATE_BWD_FULL(8, 1, 6, true); else ISSM_STATE_BWD_FULL(8, 1, 6, false); }
-    else { if (batch) ISSM_STATE_BWD_FULL(8, 2, 4, true); else ISSM_STATE_BWD_FULL(8, 2, 4, false); }
-  } else {
-    switch ((p.P + 15) / 16) {
-      case 1: ISSM_STATE_BWD_FULL(16, 1, 3, false); break;
-      case 2: ISSM_STATE_BWD_FULL(16, 2, 3, false); break;
-      case 3: ISSM_STATE_BWD_FULL(16, 3, 3, false); break;
-      default: ISSM_STATE_BWD_FULL(16, 4, 3, false); break;
-    }
-  }
-#undef ISSM_STATE_BWD_T
-#undef ISSM_STATE_BWD_FULL
-  return (int)hipGetLastError();
-}
-
 template <int PT, bool IOB, bool DTB, bool FULL>
 static int launch_bwd_chunk_t(const KP& p, int blocks, const float* dy_ws, const float* states, const float* dstates,
-                              const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
+                              const float* dm, float* partA, float* partBias, const int* redo,
                               int ndirs, hipStream_t st) {
   if constexpr (IOB) {  // bf16 inputs: every product on the bf16 matrix instructions
     const size_t sm = sizeof(BwdChunkBfSmem<PT>);
     if (int e = set_lds(&k_bwd_chunk_bf<PT, DTB, FULL>, sm)) return e;
-    hipLaunchKernelGGL((k_bwd_chunk_bf<PT, DTB, FULL>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, ndirs);
+    hipLaunchKernelGGL((k_bwd_chunk_bf<PT, DTB, FULL>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, partA, partBias, redo, ndirs);
   } else {
     const size_t sm = sizeof(BwdChunkSmem<PT>);
     if (int e = set_lds(&k_bwd_chunk<PT, false, DTB, FULL>, sm)) return e;
-    hipLaunchKernelGGL((k_bwd_chunk<PT, false, DTB, FULL>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, ndirs);
+    hipLaunchKernelGGL((k_bwd_chunk<PT, false, DTB, FULL>), dim3(blocks), dim3(NTHREADS), sm, st, p, dy_ws, states, dstates, dm, partA, partBias, redo, ndirs);
   }
   return 0;
 }
 
 bool bwd_tile_available(const KP& p, const float* dy_ws);
-int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm, const float* g_last,
+int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
                     float* partA, float* partBias, int* redo, int parts, hipStream_t st);
 
 // Chunk backward of direction p.dir0.  With a `redo` buffer (issm_bwd_chunk_redo_ints words) the tile-base kernel
@@ -1891,14 +1569,14 @@ int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const 
 // that are no multiple of four elements), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
 // parts: workgroups of the tile-base kernel that share a group's heads (1 without p.dbc_part).
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     const float* g_last, float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st) {
+                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   if (redo && bwd_tile_available(p, dy_ws)) {
     if (redo_pending) *redo_pending = 1;
-    return launch_bwd_tile(p, dy_ws, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    return launch_bwd_tile(p, dy_ws, states, dstates, dm, partA, partBias, redo, parts, st);
   }
   ISSM_DISPATCH(p, {
-    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
+    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, partA,
                                                                   partBias, nullptr, 1, st))
       return e;
   });
@@ -1909,11 +1587,11 @@ int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const
 // `redo` (ordinary inputs mark none, and its workgroups return at once).  Where the sequence length is not a multiple of
 // the chunk the two directions' chunks do not cover the same tokens: the caller then launches direction by direction.
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
-                          const float* dm, const float* g_last, float* partA, float* partBias, const int* redo,
+                          const float* dm, float* partA, float* partBias, const int* redo,
                           hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   ISSM_DISPATCH(p, {
-    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, g_last, partA,
+    if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, partA,
                                                                   partBias, redo, ndirs, st))
       return e;
   });

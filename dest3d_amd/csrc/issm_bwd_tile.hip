@@ -34,6 +34,11 @@
 // workgroups that have such rows or columns.  8 x 1024 tokens, 8 heads x 32, one direction: N = 250 104 us fp32, 83 us bf16
 // (107 and 86 with operand pairs, 147 and 111 in the level form; N = 256: 88 and 59 us); N = 256 with a gated dy, fp32: 99 us
 // (88 with operand pairs, 122 in the level form).
+//
+// What reaches the chunk's total decay through the states is formed here as well (see `gsum`), from dS, H and the state terms'
+// products: the recurrences need not read the states for it (33 - 60 % of their bytes), and what cancels does so exactly: ddt_bias
+// and dA of 2 x 512 tokens, 8 heads x 32, 256 states, fp32, 1.7e-4 and 8e-5 -> 6e-6 of their norm from float64; with A a hundred
+// times larger 9e-2 and 0.4 -> 2e-4 and 8e-4.
 #include "issm_dev.h"
 
 namespace issm {
@@ -77,8 +82,7 @@ __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflev
 template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
 __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
                                                           const float* __restrict__ dstates,
-                                                          const float* __restrict__ dm,
-                                                          const float* __restrict__ g_last, float* __restrict__ partA,
+                                                          const float* __restrict__ dm, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
   constexpr bool SPLIT = !IOB;
   constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && !FULL;  // fp32 products in the diagonal blocks / in all blocks
@@ -140,7 +144,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   uint4 l_th0, l_th1, l_tl0, l_tl1;
   f4 l_xv[SPLIT ? PT : 1], l_dv[SPLIT ? PT : 1];
   uint2 l_nx[SPLIT ? 1 : PT], l_ny[SPLIT ? 1 : PT];
-  float l_raw[16], l_A, l_bias, l_gl, l_dsv[KP_], l_hv[KP_], l_Bv[BCL ? 1 : 16], l_Cv[BCL ? 1 : 16];
+  float l_raw[16], l_A, l_bias, l_dsv[KP_], l_hv[KP_], l_Bv[BCL ? 1 : 16], l_Cv[BCL ? 1 : 16];
   auto request = [&](int hnext) {
     constexpr int G4 = 4 * PT;
     int tq = tid;
@@ -183,7 +187,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       const float b = bp[hnext * p.N + nc_];
       l_bias = p.dt_bias ? b : 0.0f;
     }
-    l_gl = g_last[vec_off(p, u.bt, u.c, hnext) + nc_];  // (every lane of the column; the last lane group uses it)
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_dsv);
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
     if constexpr (!BCL) {
@@ -269,7 +272,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     const uint16_t* dys_ = s.dys;
     const uint16_t* tm_ = s.tm;
 
-    float dcs[16], val[16];
+    float dcs[16], val[16], gsum = 0.0f;   // gsum: the lane's share of the states' gradient to the chunk's total, see below
 #pragma unroll
     for (int k = 0; k < 16; ++k) dcs[k] = val[k] = 0.0f;
     if (!skip) {
@@ -353,9 +356,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       int cq = cm, gq = g4;
       asm volatile("" : "+v"(cq), "+v"(gq));
       // dS and H of the lane's column as (hi, lo) bf16 pairs: the B operands of Q = x . dS and R = dy . H (products over
-      // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states: the last
-      // row's Bd . E1 cancels against the state term g = sum_p dS H_next in d/d(cs), and a dS rounded to 8 bits would
-      // leave that difference far above the input rounding.
+      // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states, whose rounding to
+      // 8 bits would be far above that of the inputs.
+      // The chunk's total decay acts on the states alone, with the gradient sum_p dS H_next = exp2(total) sum_p dS H +
+      // sum_l (Bd exp2(total - cs))[l] Q[l]: the second sum is the state terms of the column phase, which cancel against it
+      // exactly in the suffix sums, so the next chunk's H is not read and nothing has to be summed over p elsewhere.
+      gsum = E[4][0] * lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+      if constexpr (SPLIT) asm volatile("" : "+v"(gsum));   // (8 - 20 bytes a lane of scratch less; bf16 inputs: more)
       bf8 dsh[KT], dsl[KT], hh_[KT], hl_[KT];
 #pragma unroll
       for (int t = 0; t < KT; ++t) {
@@ -517,9 +524,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
         // The rows' share of the column phase.  d/d(cs) = C X2 - Bd E1 takes the blocks' sums times the operands as the
         // matrix instructions took them: a pair of rows then enters both of its rows as one and the same product and
-        // cancels in the suffix sums to fp32 rounding.  The state terms cancel against the state pass's column sums,
-        // which were formed from unrounded states: with bf16 inputs they take the unrounded operands (B and C are
-        // exact, the decays fp32); with fp32 inputs the operand pairs are as accurate as the split products Q and R.
+        // cancels in the suffix sums to fp32 rounding.  The state terms take, with bf16 inputs, the unrounded operands (B and
+        // C are exact, the decays fp32); with fp32 inputs the operand pairs are as accurate as the split products Q and R.
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int k = 4 * R + rr;
@@ -530,14 +536,18 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           val[k] = bv * E1;
           if constexpr (ALL32) {
             dcs[k] = cf32[k] * (xf[rr] + sf[rr]) - bf32[k] * (xg[rr] + sg[rr]);
+            gsum += bf32[k] * sg[rr];
           } else if constexpr (SPLIT) {
             const float c16 = (float)Ch[R][rr] + (float)Cl[R][rr], b16 = (float)Bh[R][rr] + (float)Bl[R][rr];
             dcs[k] = c16 * (xf[rr] + sf[rr]) - b16 * (xg[rr] + sg[rr]);
+            gsum += b16 * sg[rr];
           } else {
             const float c16 = (float)Ch[R][rr], b16 = (float)Bh[R][rr];
             float pairs = c16 * xf[rr] - b16 * xg[rr];
             if constexpr (DIAG32) pairs += cd[rr] * df[rr] - bd[rr] * dg[rr];
-            dcs[k] = pairs + (unpk(cvp, k) * up[k] * sf[rr] - bv * dtp[k] * iup[k] * sg[rr]);
+            const float own = bv * dtp[k] * iup[k] * sg[rr];
+            dcs[k] = pairs + (unpk(cvp, k) * up[k] * sf[rr] - own);
+            gsum += own;
           }
         }
       }
@@ -547,7 +557,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
     // ---- this direction's predecessor in ddt, then the next head's requests: all of them stay in flight through the
     // rest of this head, which only waits for the predecessor's values (requested before them)
-    const float gl_keep = l_gl;
     float old[16];
     if constexpr (ACC) {
       if constexpr (P32) lane_load_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, old);
@@ -571,10 +580,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     // reloaded from scratch behind the requests in flight)
     int cm2 = cm, g42 = g4;
     asm volatile("" : "+v"(cm2), "+v"(g42));
-    dcs[15] += g42 == 3 ? gl_keep : 0.0f;
     {
-      // suffix sums up the 64 rows
-      float c[4], v[4], t[4];
+      // suffix sums up the 64 rows, from the gradient to the chunk's total on
+      float c[4], v[4], t[4], carry;   // carry: sum over all rows after the current tile
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
         float a = 0.0f;
@@ -588,6 +596,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       if constexpr (IOB) {
 #pragma unroll
         for (int J = 0; J < 4; ++J) t[J] = __shfl_down(c[J], 16, 64);
+        gsum += __shfl_xor(gsum, 16, 64);
 #pragma unroll
         for (int J = 0; J < 4; ++J) v[J] = g42 <= 2 ? c[J] + t[J] : c[J];
 #pragma unroll
@@ -596,14 +605,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         for (int J = 0; J < 4; ++J) v[J] = g42 <= 1 ? v[J] + t[J] : v[J];  // inclusive from the last lane group down
 #pragma unroll
         for (int J = 0; J < 4; ++J) t[J] = __shfl(v[J], cm2, 64);           // tile totals
+        carry = gsum + __shfl_xor(gsum, 32, 64);
       } else {
 #pragma unroll
         for (int J = 0; J < 4; ++J) {
           float before;
           group_sums(c[J], g42, before, v[J], t[J]);   // of the rows behind, of the tile
         }
+        float before, after;
+        group_sums(gsum, g42, before, after, carry);
       }
-      float carry = 0.0f;  // sum over all rows after the current tile
 #pragma unroll
       for (int J = 3; J >= 0; --J) {
         const float add = carry + (IOB ? v[J] - c[J] : v[J]);
@@ -673,7 +684,7 @@ bool bwd_tile_available(const KP& p, const float* dy_ws) {
 
 template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
-                             const float* g_last, float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
+                             float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
   const size_t sm = sizeof(BwdTileSmem<PT, !IOB>);
   const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0;
   auto go = [&](auto kern) -> int {
@@ -681,7 +692,7 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
       if (int e = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm))
         return e;
-    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(NTHREADS), sm, st, p, states, dstates, dm, g_last, partA, partBias, redo,
+    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
                        (p.hpg + parts - 1) / parts);
     return 0;
   };
@@ -701,7 +712,7 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
 }
 
 int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                    const float* g_last, float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
+                    float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
   KP p = p_;
   if (dy_ws) {  // a gated dy: fp32 (Bt, L, H, P) contiguous, batch * direction outermost
     TensorD& t = p.dout[p.dir0];
@@ -715,12 +726,12 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
   const int pt = (p.P + 15) / 16;
   int e = 0;
   if (p.io_dt) {
-    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
-    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
   } else {
-    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
-    else e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, g_last, partA, partBias, redo, parts, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    else e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
   }
   if (e) return e;
   return (int)hipGetLastError();

@@ -1,22 +1,22 @@
-// Backward pass over the chunk states in one kernel (gfx950): dH_c = dy^T (C exp(cs)), the reverse recurrence over the chunks,
-// the column sums g and the matrix dM, for calls whose sequences and column slices fill the chip.
+// Backward pass over the chunk states in one kernel (gfx950): dH_c = dy^T (C exp(cs)), the reverse recurrence over the chunks
+// and the matrix dM, for calls whose sequences and column slices fill the chip.
 //
 // Workgroup = (batch and direction, head, 64 state columns), walking the chunks from the last to the first.  dH contracts over
 // the rows of a chunk and the recurrence is element-wise, so neither needs another workgroup's columns: the lane that owns
 // column n and rows p = 16 pt + 4 g4 + r of the state keeps them in the accumulator of the matrix instruction that adds the next
 // dH,
-//     dS_c = carry (stored),   g_c[n] = sum_p dS_c H_(c+1),   carry = exp(chunk total) carry + dy^T (C exp(cs)).
-// As two kernels (k_bwd_dstates, k_state_bwd_full) the same work writes dH and reads it back, 8 P N bytes a chunk and head.
+//     dS_c = carry (stored),   carry = exp(chunk total) carry + dy^T (C exp(cs)).
+// As two kernels (k_bwd_dstates, k_state_pass) the same work writes dH and reads it back, 8 P N bytes a chunk and head.
 // Every operand of chunk c - 1 is requested while chunk c is computed; dy's tile, which the four waves share, is staged
 // transposed in two LDS buffers used in turn: one barrier a chunk.
 //
 // dM = tril(dy x^T) needs no state column: workgroups behind the walks in the same launch take it, one a chunk and head, and run
 // where the walks leave room on the CUs (the walks wait for one another's latencies: dealt to their waves instead, dM's ten blocks
-// held every chunk up, 97 us for 83 at the first size below).  It leaves as the symmetric bf16 matrix (and, fp32 inputs, the
+// held every chunk up, by 14 us at the first size below).  It leaves as the symmetric bf16 matrix (and, fp32 inputs, the
 // second one with what the first left) that k_bwd_dstates describes: the same products in the same order.
 //
-// Both kernels -> this one: 8 x 1024 tokens, both directions, 8 heads x 32, 256 states 109 -> 83 us fp32, 68 -> 49 bf16 (350 MB
-// fp32: 4.2 TB/s); heads of 36, bf16 90 -> 55; 4 x 2048, 16 heads x 64, 512 states fp32 674 -> 440, bf16 620 -> 344.
+// Both kernels -> this one: 8 x 1024 tokens, both directions, 8 heads x 32, 256 states 74 -> 61 us fp32, 62 -> 46 bf16 (285 MB
+// fp32: 4.7 TB/s); heads of 36, bf16 68 -> 51; 4 x 2048, 16 heads x 64, 512 states fp32 540 -> 350, bf16 485 -> 271.
 #include "issm_dev.h"
 
 namespace issm {
@@ -135,9 +135,8 @@ __device__ __forceinline__ void dm_unit(const KP& p, const float* dy_ws, float* 
 // PT, BF, FULL as in the other kernels; x / B / C / dt of one type, rows of x and dy in accesses of four elements (the host checks).
 // The first `walks` workgroups walk, the others are dM's.
 template <int PT, bool BF, bool FULL>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __restrict__ dy_ws, const float* __restrict__ states,
-                                                          float* __restrict__ dstates, float* __restrict__ dm,
-                                                          float* __restrict__ g_last, float* __restrict__ dh0_dir, int walks) {
+__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __restrict__ dy_ws, float* __restrict__ dstates,
+                                                          float* __restrict__ dm, float* __restrict__ dh0_dir, int walks) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdWalkSmem<PT, BF> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
@@ -191,7 +190,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
   RowMap rm;
   T r_dt[16], r_c[16];
   V r_dy[PT];
-  float hn[ROWS];
   auto request = [&](int c) {
     u.c = c;
     rm = make_rowmap<FULL>(p, u, g4, ns * NS);
@@ -202,7 +200,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
       const int e4 = tid + i * NTHREADS, l = e4 / G4, p4 = (e4 % G4) * 4;
       r_dy[i] = ry.get(c, l, p4);
     }
-    slab_load(states + st_off(p, u.bt, c + 1, u.h), hn);
   };
 
   f4 carry[PT];
@@ -240,10 +237,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
         }
       }
     }
-    // ---- dS of the chunk and its column sums with the next chunk's entry state
-    float g = 0.0f;
-#pragma unroll
-    for (int k = 0; k < ROWS; ++k) g += hn[k] * carry[k >> 2][k & 3];
+    // ---- dS of the chunk
     slab_store(dstates + dst_off(p, u.bt, c, u.h), carry);
     // ---- the registers the requests went to are free now: the next chunk's leave (at the end chunk 0 once more: in range, unused)
     float raw[16], ct[16];
@@ -254,9 +248,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
     }
     const RowMap rc = rm;
     request(max(c - 1, 0));
-    g += __shfl_xor(g, 16, 64);
-    g += __shfl_xor(g, 32, 64);
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(g), buffer(g_last + vec_off(p, u.bt, c, u.h), nb), (unsigned)n * 4u, 0, 0);
     // ---- C exp(cs) and the chunk's decay
     float total;
     {
@@ -286,14 +277,13 @@ bool bwd_walk_available(const KP& p, const float* dy_ws) {
   return true;
 }
 
-int launch_bwd_walk(const KP& p, const float* dy_ws, const float* states, float* dstates, float* dm, float* g_last, float* dh0_dir,
-                    hipStream_t st) {
+int launch_bwd_walk(const KP& p, const float* dy_ws, float* dstates, float* dm, float* dh0_dir, hipStream_t st) {
   const int walks = p.B * p.ndir * p.H * ((p.N + NS - 1) / NS), blocks = walks + p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
     if constexpr (IOB_ == DTB_) {
       constexpr auto kern = &k_bwd_walk<PT_, IOB_, FULL_>;
-      hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), sizeof(BwdWalkSmem<PT_, IOB_>), st, p, dy_ws, states, dstates, dm,
-                         g_last, dh0_dir, walks);
+      hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), sizeof(BwdWalkSmem<PT_, IOB_>), st, p, dy_ws, dstates, dm, dh0_dir,
+                         walks);
     }
   });
   return (int)hipGetLastError();

@@ -692,6 +692,14 @@ __device__ __forceinline__ void lane_load_pn(const float* __restrict__ src, int 
     for (int q = 0; q < CNT; ++q) out[q] = *(const float*)(sb + min(lo + (unsigned)(16 * (q >> 2) + (q & 3)) * nb, last));
   }
 }
+// The lane's share of sum_p a[p] b[p] of two arrays as lane_load_pn leaves them (`full`: no row past the head dimension).
+template <int CNT>
+__device__ __forceinline__ float lane_dot_pn(const float (&a)[CNT], const float (&b)[CNT], int P, int g4, bool full) {
+  float s = 0.0f;
+#pragma unroll
+  for (int q = 0; q < CNT; ++q) s += full || 16 * (q >> 2) + 4 * g4 + (q & 3) < P ? a[q] * b[q] : 0.0f;
+  return s;
+}
 // dt transform (bias -> softplus -> clamp) of the lane's rows and the inclusive running sum of
 // dt' * A * log2(e) down the chunk (so decays are exp2 of differences).  `raw` holds the loaded
 // dt values.  dfac (if WANT_DFAC) receives d dt' / d dt: the softplus derivative times the clamp

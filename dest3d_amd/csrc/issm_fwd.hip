@@ -3,7 +3,6 @@
 //   k_chunk_local   dt transform + cumsum, chunk-local end states S_c and the intra-chunk
 //                   matrix M_c = "C.A.B^T" in one pass over dt, in the form below; calls without
 //                   packed sequences take k_local_tile (issm_fwd_tile.hip) from four state columns on
-//   k_state_fwd_full / k_state_fwd   inter-chunk recurrence (HBM streaming)
 //   k_chunk_scan    y = (C*exp(cs)) H^T + tril(M) x + D x, optional gate
 //
 // The decay exp(cs[l]-cs[s]) sits inside the contraction over the state index n, so
@@ -29,140 +28,6 @@ namespace issm {
 template <int PT, bool IOB, bool DTB, bool FULL>
 __global__ __launch_bounds__(NTHREADS, 2) void k_chunk_local(KP p, float* __restrict__ states, float* __restrict__ cs_last, float* __restrict__ cabt) {
   k_chunk_local_body<PT, IOB, DTB, FULL>(p, states, cs_last, cabt);
-}
-
-// ---------------------------------------------------------------- state passing
-// One thread carries 4 adjacent state columns of one (bt, h, p) through all chunks.
-// Slot c of `states` holds S_c on entry and H_c (state at the start of chunk c) on exit;
-// slot nc receives the final state.
-// The recurrence without any conditional access in its loop: thread = 4 adjacent columns of one state row,
-// the operands of the next D chunks always requested (near the end the last chunk again: in range, unused), so the
-// compiler can count the loads in flight and never waits for all of them; with loads inside branches it did, once
-// per chunk.  D = 8 when few threads walk many chunks (memory latency sets the pace there), otherwise 4.
-// TAIL (N >= 4, not a multiple of 4; accesses at any float): the last thread of a row works on columns N - 4 .. N - 1 and
-// stores only those its neighbour does not own (what it computes for the others may read the neighbour's results and is
-// dropped).  8 x 1024 tokens, N = 250: 30.3 us with per-element guards, as fast as N = 256 without.
-template <int D, bool TAIL>
-__global__ __launch_bounds__(NTHREADS) void k_state_fwd_full(KP p, float* __restrict__ states,
-                                                             const float* __restrict__ cs_last) {
-  const int nq = (p.N + 3) >> 2;
-  const long total = (long)p.B * p.ndir * p.H * p.P * nq;
-  const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
-  if (id >= total) return;
-  const int q = id % nq;
-  long r = id / nq;
-  const int pp = r % p.P;
-  r /= p.P;
-  const int h = r % p.H;
-  const int bt = r / p.H;
-  const int b = bt / p.ndir, dir = bt % p.ndir;
-  const int n = TAIL ? min(q * 4, p.N - 4) : q * 4, skip = q * 4 - n;   // skip: columns of the thread that are its neighbour's
-  auto ld = [](const float* a) -> f4 {
-    if constexpr (TAIL) return ld_f4_any(a);
-    else return *(const f4*)a;
-  };
-  auto put = [&](float* a, f4 v) {
-    if constexpr (!TAIL) {
-      *(f4*)a = v;
-    } else if (skip == 0) {
-      st_f4_any(a, v);
-    } else {
-#pragma unroll
-      for (int j = 1; j < 4; ++j)
-        if (j >= skip) a[j] = v[j];
-    }
-  };
-  f4 st = {0, 0, 0, 0};
-  if (p.h0.ptr) {
-    const long o = (long)b * p.h0.s0 + (long)h * p.h0.s1 + (long)pp * p.h0.s2 + n;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) st[j] = ldv(p.h0.ptr, o + j, p.h0_dt);
-  }
-  const long cstride = (long)p.H * p.P * p.N, dstride = (long)p.H * p.N;
-  float* sp = states + st_off(p, bt, 0, h) + (long)pp * p.N + n;
-  const float* cl = cs_last + vec_off(p, bt, 0, h) + n;
-  // chunk c lives in slot c % D; the loop is unrolled over the D slots so that none is ever moved (a register copy
-  // would have to wait for the load that fills it)
-  const float* sp0 = sp;
-  const float* cl0 = cl;
-  f4 t[D], d[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    const int ci = min(i, p.nc - 1);
-    t[i] = ld(sp0 + ci * cstride);
-    d[i] = ld(cl0 + ci * dstride);
-  }
-  int c = 0;
-  for (; c + D <= p.nc; c += D) {
-#pragma unroll
-    for (int i = 0; i < D; ++i) {
-      const f4 tt = t[i], dd = d[i];
-      const int cn = min(c + i + D, p.nc - 1);
-      t[i] = ld(sp0 + cn * cstride);
-      d[i] = ld(cl0 + cn * dstride);
-      put(sp, st);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) st[j] = __expf(dd[j]) * st[j] + tt[j];
-      sp += cstride;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < D - 1; ++i)
-    if (c + i < p.nc) {  // uniform: the last nc % D chunks
-      put(sp, st);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) st[j] = __expf(d[i][j]) * st[j] + t[i][j];
-      sp += cstride;
-    }
-  put(sp, st);  // slot nc keeps the final state for the backward pass
-  if (p.final_states[dir]) put(p.final_states[dir] + (((long)b * p.H + h) * p.P + pp) * p.N + n, st);
-}
-
-// The recurrence for N < 4: element-wise guards, scalar accesses.
-__global__ __launch_bounds__(NTHREADS) void k_state_fwd(KP p, float* __restrict__ states,
-                                                        const float* __restrict__ cs_last) {
-  const int nq = (p.N + 3) >> 2;
-  const long total = (long)p.B * p.ndir * p.H * p.P * nq;
-  const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
-  if (id >= total) return;
-  const int q = id % nq;
-  long r = id / nq;
-  const int pp = r % p.P;
-  r /= p.P;
-  const int h = r % p.H;
-  const int bt = r / p.H;
-  const int b = bt / p.ndir, dir = bt % p.ndir;
-  const int n = q * 4;
-  float st[4] = {0, 0, 0, 0};
-  if (p.h0.ptr) {
-    const long o = (long)b * p.h0.s0 + (long)h * p.h0.s1 + (long)pp * p.h0.s2 + n;
-    for (int j = 0; j < 4; ++j)
-      if (n + j < p.N) st[j] = ldv(p.h0.ptr, o + j, p.h0_dt);
-  }
-  const long cstride = (long)p.H * p.P * p.N;
-  float* sp = states + st_off(p, bt, 0, h) + (long)pp * p.N + n;
-  const float* cl = cs_last + vec_off(p, bt, 0, h) + n;
-  for (int c = 0; c < p.nc; ++c) {
-    float sv[4], dv[4];
-    for (int j = 0; j < 4; ++j) {
-      const bool v = n + j < p.N;
-      sv[j] = v ? sp[j] : 0.0f;
-      dv[j] = v ? cl[j] : 0.0f;
-      if (v) sp[j] = st[j];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) st[j] = __expf(dv[j]) * st[j] + sv[j];
-    sp += cstride;
-    cl += (long)p.H * p.N;
-  }
-  // slot nc keeps the final state for the backward pass
-  for (int j = 0; j < 4; ++j)
-    if (n + j < p.N) sp[j] = st[j];
-  if (p.final_states[dir]) {
-    float* f = p.final_states[dir] + (((long)b * p.H + h) * p.P + pp) * p.N + n;
-    for (int j = 0; j < 4; ++j)
-      if (n + j < p.N) f[j] = st[j];
-  }
 }
 
 // ------------------------------------------------------------------ chunk scan
@@ -404,19 +269,6 @@ int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, 
     if (int e = set_lds(kern, sm)) return e;
     hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cs_last, cabt);
   });
-  return (int)hipGetLastError();
-}
-
-int launch_state_fwd(const KP& p, float* states, const float* cs_last, hipStream_t st) {
-  const long total = (long)p.B * p.ndir * p.H * p.P * ((p.N + 3) / 4);
-  const int blocks = (int)((total + NTHREADS - 1) / NTHREADS);
-#define ISSM_STATE_FWD(D_, TAIL_) \
-  hipLaunchKernelGGL((k_state_fwd_full<D_, TAIL_>), dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last)
-  const bool few = total < (1L << 17) && p.nc >= 16;
-  if (p.N < 4) hipLaunchKernelGGL(k_state_fwd, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last);
-  else if (p.N & 3) { if (few) ISSM_STATE_FWD(8, true); else ISSM_STATE_FWD(4, true); }
-  else { if (few) ISSM_STATE_FWD(8, false); else ISSM_STATE_FWD(4, false); }
-#undef ISSM_STATE_FWD
   return (int)hipGetLastError();
 }
 

@@ -203,21 +203,22 @@ int issm_stage_bwd_gate(const issm_scan_args* args, const float* out_x, float* d
  *   _chunk_scan_bwd_dcb (issm_chunk_scan.py:790-900). */
 int issm_stage_bwd_dstates(const issm_scan_args* args, const float* dy_gated, float* dstates, float* dm);
 /* issm_stage_state_passing_bwd: reverse recurrence in place (dstates[c] becomes dS_c, the gradient
- *   of the chunk-local end state), g_last (Bt,nc,H,N) = sum_p dS_c * H_{c+1} (the total gradient
- *   reaching the chunk's last cumulative sum through the states), and dh0_dir (ndir,B,H,P,N).
- *   `states` is (Bt,nc+1,H,P,N) as left by issm_stage_state_passing_fwd.  Replaces
+ *   of the chunk-local end state), and dh0_dir (ndir,B,H,P,N).  Where g_last is not NULL, one more kernel fills
+ *   it: (Bt,nc,H,N) = sum_p dS_c * H_{c+1} (the total gradient reaching the chunk's last cumulative sum through the
+ *   states) from `states`, (Bt,nc+1,H,P,N) as left by issm_stage_state_passing_fwd; nothing in the library reads it.  Replaces
  *   _state_passing_bwd (issm_state_passing.py:110-278) and the sum over P at issm_combined.py:159. */
 int issm_stage_state_passing_bwd(const issm_scan_args* args, const float* states,
                                  const float* cs_last, float* dstates, float* g_last,
                                  float* dh0_dir);
 /* issm_stage_bwd_states: the two stages above in one kernel, which walks a head's chunks from the last to the first with
- *   64 columns of the carried gradient in registers: dS_c into dstates, dM into dm, g_last and dh0_dir, as they leave them.
+ *   64 columns of the carried gradient in registers: dS_c into dstates, dM into dm, dh0_dir and (unless NULL) g_last, as they leave them.
  *   x / B / C and dt of one type, rows of x and dy in multiples of four elements, no packed sequences, no gate beside bf16
  *   inputs (ISSM_E_UNSUPPORTED otherwise).  issm_scan_bwd takes it where the walks fill the chip. */
 int issm_stage_bwd_states(const issm_scan_args* args, const float* dy_gated, const float* states, float* dstates, float* dm,
                           float* g_last, float* dh0_dir);
 /* issm_stage_bwd_chunk: ddt, dB, dC of direction `dir` and the per-unit partial sums
- *   part_a / part_bias (Bt*nc,H,N) of dA / ddt_bias.  ddt accumulates into args->ddt when
+ *   part_a / part_bias (Bt*nc,H,N) of dA / ddt_bias.  g_last is not read (the kernels form it from states, dstates and
+ *   their own products) and may be NULL.  ddt accumulates into args->ddt when
  *   dir > 0.  Replaces _chunk_state_bwd_db (issm_chunk_state.py:493-652), _chunk_scan_bwd_dc
  *   (issm_chunk_scan.py:515-657), _chunk_scan_chunk_state_bwd_dt (issm_combined.py:398-557),
  *   _bmm_CABT_dbc_chunk_bwd (issm_cabt_bmm.py:454-673), _chunk_scan_bwd_ddAcs_stable

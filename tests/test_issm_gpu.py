@@ -905,6 +905,29 @@ def test_states_of_the_backward_in_one_kernel(Bsz, L_, H, P, N, G, nd, bf, dfina
     assert torch.equal(outs[0][3], outs[1][3])
 
 
+@pytest.mark.parametrize("L_,H,P,N,G,scale", [
+    (256, 2, 32, 64, 1, 1.0),     # tile-base form, complete tiles
+    (200, 2, 36, 70, 1, 1.0),     # incomplete tiles, rows past the head dimension
+    (128, 2, 64, 64, 1, 1.0),     # level form
+    (130, 2, 6, 20, 2, 1.0),      # level form, a head that is no multiple of four wide
+    (130, 2, 8, 3, 1, 1.0),       # fewer than four states
+    (256, 2, 32, 64, 1, 100.0),   # tiles out of the tile-base form's range
+])
+def test_sums_over_tokens_of_the_decays_gradient(L_, H, P, N, G, scale):
+    """ddt_bias and dA are sums over all tokens of suffix sums in which what a row adds to a chunk's state is met by the state's
+    gradient to the chunk's total.  The two have to be one number: operands hold 16 bits or more (1.5e-5, less in the mean), and with
+    A a hundred times larger running sums in the thousands have half a unit of 1.2e-4 or more in the last place."""
+    _say(f"sums of the decays' gradient L={L_} P={P} N={N} scale={scale}")
+    d = _problem(2, L_, H, P, N, G, seed=5, D="h")
+    d["A"] = d["A"] * scale
+    _, _, ref = _oracle(d, GRAD_NAMES)
+    _, _, g, _ = _run_operator(d, torch.float32)
+    for k in ("dt_bias", "A"):
+        e = ((g[k].double().cpu() - ref[k].double()).norm() / ref[k].double().norm()).item()
+        print(f"    d{k:9s} rel_l2={e:.3e}", flush=True)
+        assert e <= (2e-5 if scale == 1.0 else 2e-3), (k, e)
+
+
 def test_inplace_edit_between_forward_and_backward_raises():
     """The operator saves its inputs for the backward as the reference does (issm_combined.py:42): changing one of them
     in place before backward must raise PyTorch's version-counter error, not return gradients of other data."""
