@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(NTHREADS) void k_three_interpolate_grad(long total,
 // Interpolation with CH channels of the m known points in LDS, [m][CH]: one thread per target and step reads the target's
 // indices and weights once for all of them and CH / 4 16-byte LDS reads per neighbour.  Bound by writing the output:
 // 256 channels, 2048 -> 20000 points, 8 samples: 166 us with a
-// thread per element, 45 us here (164 MB written).
+// thread per element, 53 us with stores that pass through L2, 45 us here (164 MB written, 3.6 TB/s; under the profiler).
 template <int CH>
 __global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int splits, unsigned per, const float* __restrict__ points,
                                                      const int* __restrict__ idx, const float* __restrict__ weight,
@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int sp
     }
 #pragma unroll
     for (int ch = 0; ch < CH; ++ch)
-      if (c0 + ch < c) out[((long)b * c + c0 + ch) * n + j] = acc[ch / 4][ch % 4];
+      if (c0 + ch < c) __builtin_nontemporal_store(acc[ch / 4][ch % 4], out + ((long)b * c + c0 + ch) * n + j);
   }
 }
 // Its gradient, all of grad_points (b, c, m) written.  Adding target by target into rows of sums in LDS takes 600 us (8
@@ -1065,9 +1065,9 @@ __global__ __launch_bounds__(512) void k_interp_rows(int c, int m, int n, int sp
 // point add up by row-lane moves, and the last of them writes the sum; what a wave's share of the list has of its first and
 // last point meets in LDS.  No atomics: a thread per 59 entries that added every run it finished to the result took 211 us,
 // the waits for its list behind those additions in the one counter both have, and one addition at either end of 64 blocks
-// still cost 70 of 147 us.  81 us here, one row or two a workgroup alike (164 MB read: 36 at the copy's rate; 49 without
-// reading them), 11 + 12 for the list; longer blocks or more of the list in flight gave nothing.  397 with atomics into a
-// channel-last buffer.
+// still cost 70 of 147 us.  68 us here (164 MB read: 36 at the copy's rate; 52 without reading more than the first rows, 53 with
+// one step's part of the list in place of all of it, 78 with row reads that displace the list in L2), 11 + 12 for the list;
+// longer blocks or more of the list in flight gave nothing.  397 with atomics into a channel-last buffer.
 constexpr int INV_T = 1024, INV_E = 8;
 struct InvList {              // per sample `blocks` places
   unsigned* target;           // [place][INV_E / 2] two targets each
@@ -1153,152 +1153,203 @@ static_assert(ROW_POINTS < (int)NO_POINT, "no point has this number, and a targe
 // R rows of grad_out in LDS, a target's R values side by side, and behind them the value zero that the entries filling up a
 // block read (a weight of zero alone would not do: zero times a gradient that is no number is none); where the row itself
 // takes all of the LDS (ZERO = false) such entries are told by the block's count.
-template <int R, bool ZERO>
+// PIPE: a workgroup takes `per` of the `sets` of R rows one after the other and asks for the next one's while it sums.  The rows
+// fill the CU's LDS, so no other workgroup's requests are in flight meanwhile, and reading and summing added up.  They are asked for
+// a piece a step, each behind the step's part of the list: what a wave asks for arrives in order, and the list is not to wait for
+// rows that are not needed yet.  8 samples, 256 channels, 2048 <- 20000
+// points: 84 -> 82 us so, 69 with the rows put into LDS 16 bytes at a time and read from there 8, 68 with fewer instructions.
+template <int R, bool ZERO, bool PIPE>
 __global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m, const float* __restrict__ grad_out, InvList l,
-                                                           float* __restrict__ grad_points) {
-  extern __shared__ __align__(16) float srow[];
+                                                           float* __restrict__ grad_points, int sets, int per) {
+  extern __shared__ __align__(16) float lds[];
+  float* srow = (float*)__builtin_assume_aligned(lds, 16);   // (the declaration's alignment alone gives accesses of two single words)
   typedef float Vals __attribute__((ext_vector_type(R)));
   typedef unsigned u4_any __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int T = INV_T;
   const int wg = xcd_remap(blockIdx.x, gridDim.x), per_b = (c + R - 1) / R;   // an XCD's workgroups: one sample's list in its L2
-  const int tid = threadIdx.x, lane = tid & 63, b = wg / per_b, c0 = (wg % per_b) * R, nch = min(R, c - c0);
-  const float* g = grad_out + ((long)b * c + c0) * n;   // R neighbouring rows
-  const int blocks = l.first[(long)b * (m + 1) + m];
-  const long base = (long)b * l.blocks;
-  const unsigned* pt = l.point + base;
-  const u4_any* tg = (const u4_any*)(l.target + base * (INV_E / 2));
-  const f4_stream *w0 = (const f4_stream*)(l.weight + base * INV_E), *w1 = w0 + l.blocks;
-  float* o = grad_points + ((long)b * c + c0) * m;
-  if (blocks == 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // sums of a point over the lanes before (a point's lanes lie side by side); on: one point from the row's first lane, or from
   // as far back as the step looks, to here
   auto scan = [&](unsigned k, float (&s)[R]) {
-    int on = __builtin_amdgcn_update_dpp(-1, (int)k, 0x138, 0xf, 0xf, false) == (int)k ? -1 : 0;
-    auto step = [&](auto ctrl, auto rows) {
-      constexpr int C = decltype(ctrl)::value, M = decltype(rows)::value;
+    const bool begins = __builtin_amdgcn_update_dpp(-1, (int)k, 0x138, 0xf, 0xf, false) != (int)k || lane == 0;
+    const int back = __builtin_clzll(__ballot(begins) << (63 - lane));   // lanes before it with its point
+    // a lane whose run reaches back `far` lanes or more takes what `ctrl` moves to it (by mask: zero times no number is none)
+    auto step = [&](auto ctrl, int far) {
+      int on = (far - 1 - back) >> 31;
+      asm("" : "+v"(on));
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        s[r] += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s[r]), C, M, 0xf, false) & on);
-      on &= __builtin_amdgcn_update_dpp(-1, on, C, M, 0xf, false);
+        s[r] += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s[r]), decltype(ctrl)::value, 0xf, 0xf, true) & on);
     };
-    typedef std::integral_constant<int, 0xf> All;
-    step(std::integral_constant<int, 0x111>{}, All{});
-    step(std::integral_constant<int, 0x112>{}, All{});
-    step(std::integral_constant<int, 0x114>{}, All{});
-    step(std::integral_constant<int, 0x118>{}, All{});
-    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
-    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    step(std::integral_constant<int, 0x111>{}, 1);   // from one, two, four, eight lanes before, inside a row of 16
+    step(std::integral_constant<int, 0x112>{}, 2);
+    step(std::integral_constant<int, 0x114>{}, 4);
+    step(std::integral_constant<int, 0x118>{}, 8);
+    step(std::integral_constant<int, 0x142>{}, lane & 16 ? (lane & 15) + 1 : 64);   // from the last lane of the row before
+    step(std::integral_constant<int, 0x143>{}, lane & 32 ? lane - 31 : 64);         // from lane 31
   };
   auto after = [&](unsigned k) {   // the next lane's
     return (unsigned)__builtin_amdgcn_update_dpp(-1, (int)k, 0x130, 0xf, 0xf, false);
   };
-  auto put = [&](unsigned k, const float (&s)[R]) {
+  // a set's rows in registers, a piece of 4 T of each at a time: U pieces, then the rows' last elements
+  constexpr int PIECES = (ROW_POINTS / R + 4 * T - 1) / (4 * T), U = PIPE ? PIECES : R == 1 ? 5 : 2;   // (not PIPE: more would cost the second workgroup on a CU)
+  f4 v[U][R];
+  float vt[R];
+  // piece `at` of set q into v[u]; where there is none, or with n < 4, anything that can be read
+  auto ask = [&](int u, int q, int at, bool real) {
+    const int c0 = (q % per_b) * R;
+    const float* row = real ? grad_out + ((long)(q / per_b) * c + c0) * n : l.weight;
+    const int k = real ? min(4 * (tid + T * at), n - 4) : 0, hop = real ? n : 0;
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (r < nch) o[(long)r * m + k] = s[r];
+    for (int r = 0; r < R; ++r) v[u][r] = ld_stream(row + (long)min(r, c - c0 - 1) * hop + k);
   };
-  // a wave's share of the list, 64 blocks a step.  first: the share's first point, to which earlier waves may have something
-  // to add, and its sum (head) once it has ended; open, carry: the point of the step's last block and its sum so far
-  const int share = (blocks + T / 64 - 1) / (T / 64), end = min(blocks, ((tid >> 6) + 1) * share);
-  int at = (tid >> 6) * share + lane;
-  struct Block { unsigned p; u4_any t; f4 wa, wb; };
-  auto load = [&](int i) {
-    i = min(i, blocks - 1);
-    return Block{pt[i], tg[i], w0[i], w1[i]};
+  auto ask_tail = [&](int q) {
+    const int c0 = (q % per_b) * R;
+    const float* row = grad_out + ((long)(q / per_b) * c + c0) * n;
+#pragma unroll
+    for (int r = 0; r < R; ++r) vt[r] = row[(long)min(r, c - c0 - 1) * n + min((n & ~3) + tid, n - 1)];
   };
-  Block q0 = load(at);
-  constexpr int U = R == 1 ? 5 : 2;   // steps in flight (more registers would cost the second workgroup on a CU)
-  for (int k0 = 4 * tid; k0 + 3 < n; k0 += 4 * T * U) {
-    f4 v[U][R];
+  auto keep = [&](int u, int at) {
+    const int k = 4 * (tid + T * at);
+    if (k + 3 < n) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int i = 0; i < R; ++i) {   // 16 bytes at a time: lane addresses are 16 R apart, and narrower accesses met in as many banks
+        f4 w;
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[u][r] = ld_stream(g + (long)min(r, nch - 1) * n + min(k0 + 4 * T * u, n - 4));
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + 4 * T * u;
-      if (k + 3 < n) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int r = 0; r < R; ++r) srow[(k + j) * R + r] = v[u][r][j];
+        for (int e = 0; e < 4; ++e) w[e] = v[u][(4 * i + e) % R][(4 * i + e) / R];
+        *(f4*)(srow + k * R + 4 * i) = w;
       }
     }
-  }
-  {
-    const int k = (n & ~3) + tid;
-    if (k < n)
-#pragma unroll
-      for (int r = 0; r < R; ++r) srow[k * R + r] = g[(long)min(r, nch - 1) * n + k];
-  }
-  if (ZERO && tid < R) srow[n * R + tid] = 0.0f;
-  __syncthreads();
-  unsigned open = NO_POINT;
-  bool ended = false;
-  float carry[R], head[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) carry[r] = head[r] = 0.0f;
-  const unsigned first = __builtin_amdgcn_readfirstlane(q0.p & 0xffffu);
-  auto take = [&](const Block& q, int at) {
-    const unsigned k = at < end ? q.p & 0xffffu : NO_POINT;
-    float s[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) s[r] = 0.0f;
-#pragma unroll
-    for (int e = 0; e < INV_E; ++e) {
-      const unsigned j = e & 1 ? q.t[e / 2] >> 16 : q.t[e / 2] & 0xffffu;
-      const Vals v = *(const Vals*)(srow + j * R);
-      const float w = e < 4 ? q.wa[e & 3] : q.wb[e & 3];
-#pragma unroll
-      for (int r = 0; r < R; ++r) s[r] += w * (ZERO || e < (int)(q.p >> 16) ? v[r] : 0.0f);
-    }
-    scan(k, s);
-    const int last = __builtin_amdgcn_readfirstlane(min(63, end - 1 - at));   // of the step's blocks
-    const unsigned k0 = (unsigned)__builtin_amdgcn_readlane((int)k, 0), k_last = (unsigned)__builtin_amdgcn_readlane((int)k, last);
-    if (k0 == open) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) s[r] += k == k0 ? carry[r] : 0.0f;
-    } else if (open != NO_POINT) {   // it ended with the last step
-      if (open == first) {
-        ended = true;
-#pragma unroll
-        for (int r = 0; r < R; ++r) head[r] = carry[r];
-      } else if (lane == 0) put(open, carry);
-    }
-    if (k0 == first && k_last != first) {
-      ended = true;
-      const int l = __popcll(__ballot(k == first)) - 1;
-#pragma unroll
-      for (int r = 0; r < R; ++r) head[r] = lane_f(s[r], l);
-    }
-    if (lane < last && after(k) != k && k != first) put(k, s);
-    open = k_last;
-#pragma unroll
-    for (int r = 0; r < R; ++r) carry[r] = lane_f(s[r], last);
   };
-  for (; at - lane < end; at += 64) {   // uniform
-    const Block n0 = load(at + 64);
-    take(q0, at);
-    q0 = n0;
-  }
-  // the waves' first and last points, in order
-  __syncthreads();
-  if (lane < 2) {
-    float* e = srow + ((tid >> 6) * 2 + lane) * (R + 1);
-    e[0] = __builtin_bit_cast(float, lane == 0 && ended ? first : open);
+  if (n == 0) return;
+  const int set0 = PIPE ? wg * per : wg, set1 = PIPE ? min(set0 + per, sets) : wg + 1;
+  if (PIPE && set0 < set1) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) e[1 + r] = lane ? carry[r] : ended ? head[r] : 0.0f;
+    for (int u = 0; u < U; ++u) ask(u, set0, u, n >= 4);
+    ask_tail(set0);
   }
-  __syncthreads();
-  if (tid < 64) {
-    const bool in = lane < T / 32;
-    const float* e = srow + (in ? lane : 0) * (R + 1);
-    const unsigned k = in ? __builtin_bit_cast(unsigned, e[0]) : NO_POINT;
-    float s[R];
+  for (int set = set0; set < set1; ++set) {
+    const int b = set / per_b, c0 = (set % per_b) * R, nch = min(R, c - c0);
+    const int blocks = l.first[(long)b * (m + 1) + m];
+    const long base = (long)b * l.blocks;
+    const unsigned* pt = l.point + base;
+    const u4_any* tg = (const u4_any*)(l.target + base * (INV_E / 2));
+    const f4_stream *w0 = (const f4_stream*)(l.weight + base * INV_E), *w1 = w0 + l.blocks;
+    float* o = grad_points + ((long)b * c + c0) * m;
+    auto put = [&](unsigned k, const float (&s)[R]) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) s[r] = e[1 + r];
-    scan(k, s);
-    if (after(k) != k && k != NO_POINT) put(k, s);
+      for (int r = 0; r < R; ++r)
+        if (r < nch) *(float*)((char*)(o + (long)r * m) + 4 * k) = s[r];
+    };
+    // a wave's share of the list, 64 blocks a step.  first: the share's first point, to which earlier waves may have something
+    // to add, and its sum (head) once it has ended; open, carry: the point of the step's last block and its sum so far
+    const int share = (blocks + T / 64 - 1) / (T / 64), end = min(blocks, (wave + 1) * share);
+    int at = wave * share;   // uniform
+    struct Block { unsigned p; u4_any t; f4 wa, wb; };
+    auto load = [&](int at) {
+      const unsigned i = min(at + lane, blocks - 1), i4 = i * 4, i16 = i * 16;   // (a list has less than 2^26 places)
+      return Block{*(const unsigned*)((const char*)pt + i4), *(const u4_any*)((const char*)tg + i16),
+                   *(const f4_stream*)((const char*)w0 + i16), *(const f4_stream*)((const char*)w1 + i16)};
+    };
+    Block q0 = load(at);
+    if constexpr (PIPE) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) keep(u, u);
+    } else {
+      for (int p0 = 0; 4 * T * p0 + 3 < n; p0 += U) {   // uniform
+#pragma unroll
+        for (int u = 0; u < U; ++u) ask(u, set, p0 + u, true);
+#pragma unroll
+        for (int u = 0; u < U; ++u) keep(u, p0 + u);
+      }
+      ask_tail(set);
+    }
+    if ((n & ~3) + tid < n)
+#pragma unroll
+      for (int r = 0; r < R; ++r) srow[((n & ~3) + tid) * R + r] = vt[r];
+    if (ZERO && tid < R) srow[n * R + tid] = 0.0f;
+    __syncthreads();
+    unsigned open = NO_POINT;
+    bool ended = false;
+    float carry[R], head[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) carry[r] = head[r] = 0.0f;
+    const unsigned first = __builtin_amdgcn_readfirstlane(q0.p & 0xffffu);
+    auto take = [&](const Block& q, int at) {
+      const unsigned k = at + lane < end ? q.p & 0xffffu : NO_POINT;
+      float s[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < INV_E; ++e) {
+        unsigned j = e & 1 ? q.t[e / 2] >> 16 : q.t[e / 2] & 0xffffu;
+        asm("" : "+v"(j));   // (else the masking moves behind the scaling and takes an instruction more)
+        const Vals x = *(const Vals*)(srow + j * R);
+        const float w = e < 4 ? q.wa[e & 3] : q.wb[e & 3];
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r] += w * (ZERO || e < (int)(q.p >> 16) ? x[r] : 0.0f);
+      }
+      scan(k, s);
+      const int last = min(63, end - 1 - at);   // of the step's blocks
+      const unsigned k0 = (unsigned)__builtin_amdgcn_readlane((int)k, 0), k_last = (unsigned)__builtin_amdgcn_readlane((int)k, last);
+      if (k0 == open) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) s[r] += k == k0 ? carry[r] : 0.0f;
+      } else if (open != NO_POINT) {   // it ended with the last step
+        if (open == first) {
+          ended = true;
+#pragma unroll
+          for (int r = 0; r < R; ++r) head[r] = carry[r];
+        } else if (lane == 0) put(open, carry);
+      }
+      if (k0 == first && k_last != first) {
+        ended = true;
+        const int l = __popcll(__ballot(k == first)) - 1;
+#pragma unroll
+        for (int r = 0; r < R; ++r) head[r] = lane_f(s[r], l);
+      }
+      if (lane < last && after(k) != k && k != first) put(k, s);
+      open = k_last;
+#pragma unroll
+      for (int r = 0; r < R; ++r) carry[r] = lane_f(s[r], last);
+    };
+    if constexpr (PIPE) {
+      const int next = min(set + 1, set1 - 1);
+      const bool real = set + 1 < set1 && n >= 4;
+      for_each_slot<U>([&](auto piece) {
+        const Block n0 = load(at + 64);
+        ask(decltype(piece)::value, next, decltype(piece)::value, real);
+        if (at < end) take(q0, at);   // uniform
+        q0 = n0;
+        at += 64;
+      });
+      ask_tail(next);
+    }
+    for (; at < end; at += 64) {   // uniform
+      const Block n0 = load(at + 64);
+      take(q0, at);
+      q0 = n0;
+    }
+    // the waves' first and last points, in order
+    __syncthreads();
+    if (lane < 2) {
+      float* e = srow + (wave * 2 + lane) * (R + 1);
+      e[0] = __builtin_bit_cast(float, lane == 0 && ended ? first : open);
+#pragma unroll
+      for (int r = 0; r < R; ++r) e[1 + r] = lane ? carry[r] : ended ? head[r] : 0.0f;
+    }
+    __syncthreads();
+    if (tid < 64) {
+      const bool in = lane < T / 32;
+      const float* e = srow + (in ? lane : 0) * (R + 1);
+      const unsigned k = in ? __builtin_bit_cast(unsigned, e[0]) : NO_POINT;
+      float s[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) s[r] = e[1 + r];
+      scan(k, s);
+      if (after(k) != k && k != NO_POINT) put(k, s);
+    }
+    if (PIPE) __syncthreads();   // the next set's rows take the place of these sums
   }
 }
 
@@ -1475,16 +1526,24 @@ int launch_interp_rows_grad(int b, int c, int n, int m, const float* grad_out, c
   if (int e = set_lds_rows(&k_inverse_rank, m * sizeof(int))) return e;
   hipLaunchKernelGGL(k_inverse_rank, dim3(b), dim3(INV_T), m * sizeof(int), st, n, m, idx, l);
   hipLaunchKernelGGL(k_inverse_fill, dim3(blocks_for(std::max(3L * n, 1L)), b), dim3(NTHREADS), 0, st, n, m, idx, weight, l, zero ? n : 0, total, grad_points);
-  auto go = [&](auto kern, int r) -> int {
-    const size_t sm = std::max((size_t)r * (n + zero), (size_t)INV_T / 32 * (r + 1)) * sizeof(float);
-    if (int e = set_lds_rows(kern, sm)) return e;
-    hipLaunchKernelGGL(kern, dim3((c + r - 1) / r * b), dim3(INV_T), sm, st, c, n, m, grad_out, l, grad_points);
-    return 0;
+  const auto lds = [&](int r) { return std::max((size_t)r * (n + zero), (size_t)INV_T / 32 * (r + 1)) * sizeof(float); };
+  // Sets of rows one after the other in a workgroup (PIPE): where one workgroup's rows leave no room on a CU for a second and there
+  // is more than one set for each CU.
+  auto go = [&](auto kern, auto pipe, int r) -> int {
+    const int sets = (c + r - 1) / r * b;
+    const bool one = lds(r) > 80 * 1024 && sets > 256;
+    const int per = one ? (sets + 255) / 256 : 1;
+    auto launch = [&](auto k) -> int {
+      if (int e = set_lds_rows(k, lds(r))) return e;
+      hipLaunchKernelGGL(k, dim3((sets + per - 1) / per), dim3(INV_T), lds(r), st, c, n, m, grad_out, l, grad_points, sets, per);
+      return 0;
+    };
+    return one ? launch(pipe) : launch(kern);
   };
   int e;
-  if (n < ROW_POINTS / 4 && (long)b * ((c + 3) / 4) >= 256) e = go(&k_interp_rows_grad<4, true>, 4);
-  else if (n < ROW_POINTS / 2 && (long)b * ((c + 1) / 2) >= 256) e = go(&k_interp_rows_grad<2, true>, 2);
-  else e = zero ? go(&k_interp_rows_grad<1, true>, 1) : go(&k_interp_rows_grad<1, false>, 1);
+  if (n < ROW_POINTS / 4 && (long)b * ((c + 3) / 4) >= 256) e = go(&k_interp_rows_grad<4, true, false>, &k_interp_rows_grad<4, true, true>, 4);
+  else if (n < ROW_POINTS / 2 && (long)b * ((c + 1) / 2) >= 256) e = go(&k_interp_rows_grad<2, true, false>, &k_interp_rows_grad<2, true, true>, 2);
+  else e = zero ? go(&k_interp_rows_grad<1, true, false>, &k_interp_rows_grad<1, true, true>, 1) : go(&k_interp_rows_grad<1, false, false>, &k_interp_rows_grad<1, false, true>, 1);
   return e ? e : (int)hipGetLastError();
 }
 int launch_three_interpolate_grad(int b, int c, int n, int m, const float* grad_out, const int* idx, const float* weight,

@@ -379,6 +379,13 @@ def test_interpolation_gradient_lists(b, c, n, m, kind):
         assert (np.abs(got[i].T - ref) <= (count + 1) * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("b,c,n,m", [(3, 343, 5123, 700), (2, 301, 10243, 40), (2, 151, 20483, 2048), (1, 259, 40960, 3000)])
+def test_interpolation_gradient_of_rows_that_fill_the_lds(b, c, n, m):
+    """Four, two, one row a set, and one without the zero behind it, more sets than CUs: a workgroup takes several, some of them of
+    two samples, and the last workgroup fewer."""
+    test_interpolation_gradient_lists(b, c, n, m, "any")
+
+
 @pytest.mark.parametrize("c,m,n", [(300, 50, 3501), (700, 3, 5121), (220, 900, 9999), (60, 1000, 40960)])
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 def test_interpolation_rows_keep_a_target_without_a_number_to_its_points(c, m, n, value):
