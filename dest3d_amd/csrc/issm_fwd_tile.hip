@@ -26,7 +26,7 @@
 //   A chunk with another tile is computed once more, by the same workgroup, with the level-hierarchy body (k_chunk_local_body),
 //   which has no such limit and overwrites everything written for the chunk before.  bf16 inputs: the wave that meets such a
 //   tile raises a flag that all look at once a step, and the rest of the steps is left out (a quarter of the chunks of a freshly
-//   initialised decoder, 8 x 1024 tokens, 256 queries: 195 -> 179 us a layer).  fp32 inputs, whose operand pairs leave no
+//   initialised decoder, 8 x 1024 tokens, 256 queries: 195 -> 179 us a layer, 118 without a device-wide fence).  fp32 inputs, whose operand pairs leave no
 //   registers to spare, pay for the look: 1505 -> 1575 us at 16 x 2048 tokens, 16 heads x 64, 512 states, nothing out of range.
 //   ANY, bf16 inputs of calls that nothing is differentiated through: a step with such a tile is left by the loop over the steps
 //   and evaluated, by its wave alone, with the diagonal blocks in parts whose factors are all <= 1 (far_diagonal) and V from its
@@ -359,8 +359,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   }
   if (!ANY && anybad) {
     // A tile of this chunk decays by more than 2^-FWD_SPAN_LIMIT: everything is computed once more in the form that has no
-    // such limit.  The fence orders this workgroup's stores above before the ones the other form makes to the same places.
-    __threadfence();
+    // such limit.  Its stores go to places that other waves of this workgroup have stored to above: those stores have reached the
+    // L2, which all of the workgroup's waves share, before the barrier.  (A device-wide fence in its place writes back and
+    // invalidates the XCD's L2 once a wave of every such chunk, under all the other workgroups: layers of 8 x 1024 tokens, 8 heads
+    // x 36, 256 states, bf16 with 5, 12, 16, 35 and 48 % of their chunks out of range took 119, 146, 163, 205 and 236 us, and
+    // take 104, 108, 119, 118 and 126.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if constexpr (!ANY) k_chunk_local_body<PT, IOB, DTB, !EDGE>(p, states, cs_last, cabt);
   }
