@@ -4,17 +4,21 @@
 // of one direction, looping over the heads of the group; lane (cm, g4) of a wave owns state column cm and the 16 chunk
 // rows {16J + 4 g4 + j}.  What differs is how the decay exp2(cs[l] - cs[s]) inside the sums
 //   F[l] = sum_{s<=l} dM[l,s] Bd[s] exp2(cs[l]-cs[s]),   G[s] = sum_{l>=s} dM[l,s] C[l] exp2(cs[l]-cs[s])
-// is taken apart.  With pc = running sum of a = dt' A log2(e) restarted at every 16-row tile and base(J) = sum of the
-// tiles before J,
-//   exp2(cs[l] - cs[s]) = up[l] . E(I,J) . iup[s],   up = exp2(pc), iup = exp2(-pc), E(I,J) = exp2(base(I) - base(J))
-// for l in tile I >= tile J of s.  up and iup are two exponentials per element, E ten per column, and then every block
-// (I, J) of F and G is a plain 16x16x16 product of the dM block with the tile's operand rows (Bd iup for F, C up for G)
-// whose result is scaled by E(I,J): no per-level operands, no pairs evaluated in the vector ALU.  The state terms fit the
-// same form: exp2(cs[l]) = up[l] E(I,0) and exp2(cs_last - cs[s]) = E(4,J) iup[s].
+// is taken apart.  With pc = running sum of a = dt' A log2(e) from the middle of the row's half of the chunk (32 rows; the middle
+// of its sum: pc runs from minus half of the half's sum to half of it),
+//   exp2(cs[l] - cs[s]) = up[l] . iup[s],  up = exp2(pc), iup = exp2(-pc), for rows of one half, and with
+//   across = exp2(half the halves' sums added up) between the two for rows of both.
+// up and iup are two exponentials per element, and a row tile's F or G is two chains of plain 16x16x16 products of dM blocks with
+// the tiles' operand rows (Bd iup for F, C up for G): the other half's blocks, times across, then those of its own half, all in
+// one accumulator -- no per-level operands, no pairs evaluated in the vector ALU.  The state terms fit the same form: exp2(cs[l])
+// = up[l] from_start, exp2(cs_last - cs[s]) = to_end iup[s].  (With a reference per tile a block was scaled by its own factor,
+// ten exponentials and 20 scaled blocks a head: 5 % more vector instructions, and a wait for every block's result before the next.
+// Training steps, 8 x 1024 tokens, 8 heads x 32, 256 states, both directions, fp32 502 -> 496 us; 2 x 16384, bf16, 843 -> 838; heads
+// of 36, both directions, bf16, 427 either way; 4 x 1000, 200 states, fp32 203.4 and 203.9.)
 //
-// iup grows like 2^(decay across one tile), so the form is only used where every tile's sum stays within SPAN_LIMIT
-// (|tt| <= 96: operands below 2^96, no overflow before the factors meet).  A head of a workgroup where some column
-// exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
+// up and iup reach 2^(half of the decay across a half), so the form is only used where every 16-row tile's sum stays within
+// SPAN_LIMIT (|tt| <= 96, a half's then within twice that: operands below 2^96, no overflow before the factors meet).  A head of a
+// workgroup where some column exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
 // (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands, complete tiles: bf16 inputs -> one bf16
 // instruction per block, operands rounded once; fp32 inputs -> operands as (hi, lo) bf16 pairs (17 significand
 // bits and more), a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, and a
@@ -72,6 +76,19 @@ struct BwdTileSmem {
 __device__ __forceinline__ float round17(float v) { return __uint_as_float((__float_as_uint(v) + 0x40u) & 0xffffff80u); }
 
 __device__ __forceinline__ bf8 cat_bf4(bf4 a, bf4 b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+
+// (v a) b: from one half's scale, up to 2^96, to the other's, down to 2^-96, by two decays whose product may lie below the type's
+// range -- where the decay between the rows on either side of the border does not -- and which -ffast-math would form.
+__device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
+#pragma clang fp reassociate(off)
+  f4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float t = v[i] * a;
+    r[i] = t * b;
+  }
+  return r;
+}
 
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
@@ -256,7 +273,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     const float An = cf.A;
     float dtp[16], dfac[16], pc[16], tt[4];
     lane_dt<true>(p, cf, vn, g4, rm, l_raw, dtp, dfac);
-    lane_tile_sums<IOB>(An * LOG2E, cm, g4, rm, dtp, pc, tt);
+    float half0, half1;
+    lane_half_sums<IOB>(An * LOG2E, cm, g4, rm, dtp, pc, tt, half0, half1);
     {
       const float worst = fmaxf(fmaxf(fabsf(tt[0]), fabsf(tt[1])), fmaxf(fabsf(tt[2]), fabsf(tt[3])));
       const bool bad = !(worst <= SPAN_LIMIT);  // also true for NaN
@@ -284,16 +302,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         up[k] = ex2(pc[k]);
         iup[k] = ex2(-pc[k]);
       }
-      // E(I,J) = exp2(base(I) - base(J)), 0 <= J < I <= 4 (base(0) = 0, base(4) = the chunk's total)
-      float bs[5];
-      bs[0] = 0.0f;
-#pragma unroll
-      for (int J = 0; J < 4; ++J) bs[J + 1] = bs[J] + tt[J];
-      float E[5][4];
-#pragma unroll
-      for (int I = 1; I < 5; ++I)
-#pragma unroll
-        for (int J = 0; J < I; ++J) E[I][J] = ex2(bs[I] - bs[J]);
+      // decays of half a half; from a half's middle to its end, or from its start to its middle
+      const float e0 = ex2(half0), e1 = ex2(half1);
+      const float across = e0 * e1;                        // from the middle of the first half to that of the second
+      const float from_start[2] = {e0, e0 * across};       // from the chunk's start to the middles
+      const float to_end[2] = {across * e1, e1};           // from the middles to the chunk's end
       auto unpk = [](const unsigned (&a)[8], int k) {
         return __uint_as_float((k & 1) ? (a[k >> 1] & 0xffff0000u) : (a[k >> 1] << 16));
       };
@@ -361,7 +374,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       // The chunk's total decay acts on the states alone, with the gradient sum_p dS H_next = exp2(total) sum_p dS H +
       // sum_l (Bd exp2(total - cs))[l] Q[l]: the second sum is the state terms of the column phase, which cancel against it
       // exactly in the suffix sums, so the next chunk's H is not read and nothing has to be summed over p elsewhere.
-      gsum = E[4][0] * lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+      gsum = across * across * lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
       if constexpr (SPLIT) asm volatile("" : "+v"(gsum));   // (8 - 20 bytes a lane of scratch less; bf16 inputs: more)
       bf8 dsh[KT], dsl[KT], hh_[KT], hl_[KT];
 #pragma unroll
@@ -382,8 +395,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         mf[w] = (c0 <= cq ? 0xffffu : 0u) | (c0 + 1 <= cq ? 0xffff0000u : 0u);
         mg[w] = (c0 >= cq ? 0xffffu : 0u) | (c0 + 1 >= cq ? 0xffff0000u : 0u);
       }
-      auto block = [&](uint2 ah, uint2 al, bf4 bh, bf4 bl) -> f4 {
-        f4 acc = {0, 0, 0, 0};
+      auto block = [&](uint2 ah, uint2 al, bf4 bh, bf4 bl, f4 acc) -> f4 {
         const bf4 a_h = __builtin_bit_cast(bf4, ah);
         if constexpr (SPLIT) {
           // (ah + al) . (bh + bl) in full: the same A fragment against (bl | bh) and (bh | bl).  All four terms, so
@@ -395,9 +407,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           return mfma_bf16k(a_h, bh, acc);
         }
       };
+      // the blocks of two tiles
+      auto block2 = [&](const uint2 (&ah)[4], const uint2 (&al)[4], const bf4 (&bh)[4], const bf4 (&bl)[4], int c, f4 acc) -> f4 {
+        return block(ah[c + 1], al[c + 1], bh[c + 1], bl[c + 1], block(ah[c], al[c], bh[c], bl[c], acc));
+      };
 
-      auto block32 = [&](f4 a, const float* op) -> f4 {  // fp32: k-slot g4 of instruction j <-> row / column 4 g4 + j
-        f4 acc = {0, 0, 0, 0};
+      auto block32 = [&](f4 a, const float* op, f4 acc) -> f4 {  // fp32: k-slot g4 of instruction j <-> row / column 4 g4 + j
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc = mfma4(a[j], op[j], acc);
         return acc;
@@ -459,8 +474,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           }
 #pragma unroll
           for (int rr = 0; rr < 4; ++rr) {
-            sg[rr] = E[4][R] * q[rr];
-            sf[rr] = R == 0 ? r[rr] : E[R][0] * r[rr];
+            sg[rr] = to_end[R >> 1] * q[rr];
+            sf[rr] = from_start[R >> 1] * r[rr];
           }
         }
         if constexpr (ALL32) {
@@ -468,19 +483,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           f4 t[4];
 #pragma unroll
           for (int c = 0; c < 4; ++c) t[c] = *(const f4*)(row + 16 * c);
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            if (c <= R) {  // F block (R, c)
-              const f4 acc = block32(c == R ? upto(t[c]) : t[c], bf32 + 4 * c);
-#pragma unroll
-              for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
-            }
-            if (c >= R) {  // G block (c, R)
-              const f4 acc = block32(c == R ? from(t[c]) : t[c], cf32 + 4 * c);
-#pragma unroll
-              for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
-            }
-          }
+          // (as below)
+          if (R >= 2) xf = scaled_twice(block32(t[1], bf32 + 4, block32(t[0], bf32, xf)), e0, e1);
+          if (R < 2) xg = scaled_twice(block32(t[3], cf32 + 12, block32(t[2], cf32 + 8, xg)), e1, e0);
+          const int O = R ^ 1;
+          if (R & 1) xf = block32(t[O], bf32 + 4 * O, xf);
+          else xg = block32(t[O], cf32 + 4 * O, xg);
+          xf = block32(upto(t[R]), bf32 + 4 * R, xf);
+          xg = block32(from(t[R]), cf32 + 4 * R, xg);
         } else {
           uint2 th[4], tl[4];
           const uint16_t* row = tm_ + (16 * R + cq) * LDM + 4 * gq;
@@ -490,36 +500,23 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
             if (SPLIT) tl[c] = *(const uint2*)(row + CS * LDM + 16 * c);
             else tl[c] = make_uint2(0u, 0u);
           }
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            if (c <= R) {  // F block (R, c)
-              uint2 ah = th[c], al = tl[c];
-              if (c == R) {
-                ah.x &= mf[0]; ah.y &= mf[1];
-                al.x &= mf[0]; al.y &= mf[1];
-              }
-              if (DIAG32 && c == R) {
-                df = block32(upto(wide(th[c])), bd);
-              } else {
-                const f4 acc = block(ah, al, Bh[c], Bl[c]);
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) xf[rr] = c == R ? xf[rr] + acc[rr] : fmaf(E[R][c < R ? c : 0], acc[rr], xf[rr]);
-              }
-            }
-            if (c >= R) {  // G block (c, R)
-              uint2 ah = th[c], al = tl[c];
-              if (c == R) {
-                ah.x &= mg[0]; ah.y &= mg[1];
-                al.x &= mg[0]; al.y &= mg[1];
-              }
-              if (DIAG32 && c == R) {
-                dg = block32(from(wide(th[c])), cd);
-              } else {
-                const f4 acc = block(ah, al, Ch[c], Cl[c]);
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) xg[rr] = c == R ? xg[rr] + acc[rr] : fmaf(E[c > R ? c : 4][R], acc[rr], xg[rr]);
-              }
-            }
+          // the other half's blocks first: their sum decays across the middles; then those of the rows' own half
+          if (R >= 2) xf = scaled_twice(block2(th, tl, Bh, Bl, 0, xf), e0, e1);
+          if (R < 2) xg = scaled_twice(block2(th, tl, Ch, Cl, 2, xg), e1, e0);
+          const int O = R ^ 1;   // the half's other tile
+          const uint2 dh = th[R], dl = tl[R];
+          if constexpr (DIAG32) {
+            if (R & 1) xf = block(th[O], tl[O], Bh[O], Bl[O], xf);
+            else xg = block(th[O], tl[O], Ch[O], Cl[O], xg);
+            df = block32(upto(wide(dh)), bd, df);
+            dg = block32(from(wide(dh)), cd, dg);
+          } else {
+            th[R] = make_uint2(dh.x & mf[0], dh.y & mf[1]);
+            tl[R] = make_uint2(dl.x & mf[0], dl.y & mf[1]);
+            xf = (R & 1) ? block2(th, tl, Bh, Bl, R & 2, xf) : block(th[R], tl[R], Bh[R], Bl[R], xf);
+            th[R] = make_uint2(dh.x & mg[0], dh.y & mg[1]);
+            tl[R] = make_uint2(dl.x & mg[0], dl.y & mg[1]);
+            xg = (R & 1) ? block(th[R], tl[R], Ch[R], Cl[R], xg) : block2(th, tl, Ch, Cl, R & 2, xg);
           }
         }
         // The rows' share of the column phase.  d/d(cs) = C X2 - Bd E1 takes the blocks' sums times the operands as the

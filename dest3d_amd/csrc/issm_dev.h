@@ -827,14 +827,15 @@ __device__ __forceinline__ float lane_prep(const KP& p, const Coef& cf, bool vn,
   return carry;
 }
 
-// Running sums of a = dt' A log2(e) restarted at every 16-row tile: pc[k] = sum of a over the rows of k's tile up to and
-// including k's row, tt[J] = the whole tile's sum (the same on the four lanes of a column).  Used by the kernels that
-// write a decay exp2(cs[l] - cs[s]) as  exp2(pc[l]) . exp2(base(tile of l) - base(tile of s)) . exp2(-pc[s])  with
-// base(J) = tt[0] + .. + tt[J-1]: two exponentials per element and ten per column serve every pair of rows of the chunk.
+// Running sums of a = dt' A log2(e) from the middle of the row's 32-row half of the chunk: pc[k] = sum of a over the rows of the
+// half up to and including k's row, less half of the half's sum; half0, half1 = half of the halves' sums, tt[J] = a 16-row tile's
+// (these the same on the four lanes of a column).  Used by the kernel that writes a decay exp2(cs[l] - cs[s]) as
+// exp2(pc[l]) . exp2(-pc[s]) for rows of one half and with exp2(half0 + half1) between the two for rows of both: two exponentials
+// per element and two per column serve every pair of rows of the chunk.
 // LDS: the cross-lane steps through LDS (see group_sums).
 template <bool LDS>
-__device__ __forceinline__ void lane_tile_sums(float A2, int cm, int g4, const RowMap& rm, const float (&dtp)[16],
-                                               float (&pc)[16], float (&tt)[4]) {
+__device__ __forceinline__ void lane_half_sums(float A2, int cm, int g4, const RowMap& rm, const float (&dtp)[16],
+                                               float (&pc)[16], float (&tt)[4], float& half0, float& half1) {
   float c[4];
   if (rm.full || rm.cut == 0) {
 #pragma unroll
@@ -860,6 +861,7 @@ __device__ __forceinline__ void lane_tile_sums(float A2, int cm, int g4, const R
       c[J] = a;
     }
   }
+  float add[4];
   if constexpr (LDS) {
     float v[4], t[4];
 #pragma unroll
@@ -873,19 +875,21 @@ __device__ __forceinline__ void lane_tile_sums(float A2, int cm, int g4, const R
 #pragma unroll
     for (int J = 0; J < 4; ++J) tt[J] = __shfl(v[J], cm + 48, 64);    // tile totals
 #pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const float add = v[J] - c[J];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pc[4 * J + j] += add;
-    }
+    for (int J = 0; J < 4; ++J) add[J] = v[J] - c[J];
   } else {
 #pragma unroll
     for (int J = 0; J < 4; ++J) {
-      float add, after;
-      group_sums(c[J], g4, add, after, tt[J]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pc[4 * J + j] += add;
+      float after;
+      group_sums(c[J], g4, add[J], after, tt[J]);
     }
+  }
+  half0 = 0.5f * (tt[0] + tt[1]);
+  half1 = 0.5f * (tt[2] + tt[3]);
+#pragma unroll
+  for (int J = 0; J < 4; ++J) {
+    add[J] += ((J & 1) ? tt[J & 2] : 0.0f) - ((J & 2) ? half1 : half0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pc[4 * J + j] += add[J];
   }
 }
 

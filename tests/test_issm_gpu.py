@@ -928,6 +928,29 @@ def test_sums_over_tokens_of_the_decays_gradient(L_, H, P, N, G, scale):
         assert e <= (2e-5 if scale == 1.0 else 2e-3), (k, e)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,P", [(128, 64, 32), (128, 64, 36), (100, 70, 32)])
+@pytest.mark.parametrize("spans", [(95, 95, 95, 95), (95, 0.1, 0.1, 95), (0.1, 95, 95, 0.1), (0, 0, 95, 0)], ids=str)
+def test_tiles_that_decay_as_far_as_the_tile_base_form_reaches(dtype, L_, N, P, spans):
+    """Every 16 rows of a chunk decay by 2^-span: the halves' middles lie up to 95 from their ends, and the factors between a
+    row and its half's middle up to 2^95 either way.  Running sums up to 380 keep 1.5e-5 of a row's exponent, which the parameters' sums of
+    a hundred rows may see several times (1e-4, four times that at the largest entry); bf16 as everywhere 2e-2 and, for sums, 5e-2."""
+    _say(f"tiles of 2^-{spans} L={L_} N={N} P={P} {dtype}")
+    d = _problem(2, L_, 2, P, N, 1, seed=17, softplus=False)
+    d["A"] = -torch.linspace(0.5, 1.0, N).repeat(2, 1)
+    rows = torch.tensor(spans, dtype=torch.float32).repeat_interleave(16).repeat(L_ // 64 + 1)[:L_] / (16 * 1.4427)
+    d["dt"] = rows[None, :, None, None].expand(2, L_, 2, N).contiguous()
+    for k in ("x", "dt", "B", "C"):
+        d[k] = d[k].to(dtype).float()
+    y, fin, ref = _oracle(d, GRAD_NAMES)
+    yg, fg, g, _ = _run_operator(d, dtype)
+    fp32 = dtype == torch.float32
+    _check("y", yg, y, 1e-4 if fp32 else 2e-2)
+    _check("final", fg, fin, 1e-4 if fp32 else 2e-2)
+    for k, v in ref.items():
+        _check("d" + k, g[k], v, 4e-4 if fp32 else (5e-2 if k == "A" else 2e-2))
+
+
 def test_inplace_edit_between_forward_and_backward_raises():
     """The operator saves its inputs for the backward as the reference does (issm_combined.py:42): changing one of them
     in place before backward must raise PyTorch's version-counter error, not return gradients of other data."""
