@@ -1136,7 +1136,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf(KP p, const float*
 #endif
 template <int PT, bool BF>
 struct BwdDxSmem {
-  static constexpr int LDPT = PT * 16 + 4;
   static constexpr int LDK = NS + 8;
   // fp32 inputs: the product over the state index on (hi, lo) bf16 tiles, hi.hi + hi.lo + lo.hi, instead of fp32
   // matrix instructions, which take the vector ALU's issue slots (28 - 45 % of this kernel's cycles, never beside its
@@ -1144,13 +1143,13 @@ struct BwdDxSmem {
   static constexpr bool SPL = !BF && PT >= DX_SPLIT_FROM;
   static constexpr bool B16 = BF || SPL;
   static constexpr int NH = SPL ? 2 : 1;
-  float dys[CS * LDPT];
+  float dys[RowTile<PT>::SIZE];
   typename std::conditional<B16, uint16_t, float>::type bt[NH * CS * (B16 ? LDK : LDN)];        // B dt' exp2(last - cs) [m][n]
   typename std::conditional<B16, uint16_t, float>::type dss[NH * PT * 16 * (B16 ? LDK : LDN)];  // dS [p][n]
-  float prod_own[BF ? CS * LDPT : 4];  // dy * x; with fp32 inputs it takes the place of `bt`
-  __device__ __forceinline__ float* prod() { return BF ? prod_own : reinterpret_cast<float*>(bt); }
-  static constexpr int LDPROD = B16 ? LDPT : LDN;
-  static_assert(!SPL || sizeof(uint16_t) * NH * CS * LDK >= sizeof(float) * CS * LDPT, "dy * x fits in the place of bt");
+  // dy * x, in the place of `bt` and `dss` once their product is done
+  static constexpr int LDPROD = B16 ? PT * 16 + 4 : LDN;
+  __device__ __forceinline__ float* prod() { return reinterpret_cast<float*>(bt); }
+  static_assert(sizeof(bt) % 16 == 0 && sizeof(bt) + sizeof(dss) >= sizeof(float) * CS * LDPROD, "dy * x fits");
 };
 // a (16 PT x 64) slab of fp32 values as (hi, lo) bf16 pairs into LDS hi / lo [p][col], row stride LD
 template <int PT, int LD>
@@ -1188,7 +1187,8 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdDxSmem<PT, IOB> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
-  constexpr int LDPT = SM::LDPT, LDK = SM::LDK, LDPR = SM::LDPROD;
+  typedef RowTile<PT> YT;
+  constexpr int LDY = YT::LD, LDK = SM::LDK, LDPR = SM::LDPROD;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
@@ -1224,7 +1224,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   {
     float dv[CS * PT * 16 / NTHREADS];
     dy_load<IOB, PT, FULL>(p, u, dy_ws, dv);
-    lp_store<PT>(dv, s.dys, LDPT);
+    lp_store<PT>(dv, s.dys);
   }
   f4 acc[PT];
 #pragma unroll
@@ -1310,8 +1310,8 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
       split4(mf[kb], ah, al);
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt) {
-        const float* bp = s.dys + (16 * kb + 4 * g4) * LDPT + pt * 16 + cm;
-        const float yw[4] = {bp[0], bp[LDPT], bp[2 * LDPT], bp[3 * LDPT]};
+        const float* bp = s.dys + YT::at(16 * kb + 4 * g4, pt * 16 + cm);
+        const float yw[4] = {bp[0], bp[LDY], bp[2 * LDY], bp[3 * LDY]};
         bf4 bh, bl;
         split4(yw, bh, bl);
         acc[pt] = mfma_bf16k(al, bh, acc[pt]);
@@ -1341,7 +1341,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int l = wave * 16 + 4 * g4 + r, pp = pt * 16 + cm;
-      const float dyv = s.dys[l * LDPT + pp];
+      const float dyv = s.dys[YT::at(l, pp)];
       v[r] = fmaf(dcoef, dyv, acc[pt][r]);
       prod[l * LDPR + pp] = dyv * xv[r];
     }

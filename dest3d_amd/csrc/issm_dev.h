@@ -958,14 +958,22 @@ __device__ __forceinline__ void lp_load(const KP& p, const Unit& u, const Tensor
     for (int e = 0; e < 4 * PT; ++e) v[e] = ok[e] ? (BF ? bf16_to_f((uint16_t)r[e]) : (float)r[e]) : 0.0f;
   }
 }
+// The tile in LDS as fp32, for reads of a column over four adjacent rows that differ from lane group to lane group: the groups'
+// rows lie 16 banks apart, by four columns of padding or, four head tiles, by exchanging the row's 16-column pieces -- the 1 KB of
+// padding would leave the kernels with (hi, lo) operand tiles beside it two workgroups a CU instead of three (16 x 2048 tokens, 16
+// heads x 64, 512 states, both directions, fp32: k_chunk_scan 1030 -> 936 us, k_bwd_dx 1068 -> 960).
 template <int PT>
-__device__ __forceinline__ void lp_store(const float (&v)[CS * PT * 16 / NTHREADS], float* dst, int ld,
-                                         int tid = threadIdx.x) {
+struct RowTile {
+  static constexpr int LD = PT == 4 ? 64 : PT * 16 + 4, SIZE = CS * LD;
+  static __device__ __forceinline__ int at(int l, int p) { return l * LD + (PT == 4 ? p ^ ((l & 12) << 2) : p); }
+};
+template <int PT>
+__device__ __forceinline__ void lp_store(const float (&v)[CS * PT * 16 / NTHREADS], float* dst, int tid = threadIdx.x) {
   constexpr int G4 = 4 * PT;
 #pragma unroll
   for (int i = 0; i < PT; ++i) {
     const int e4 = tid + i * NTHREADS;
-    *(f4*)(dst + (e4 / G4) * ld + (e4 % G4) * 4) = (f4){v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+    *(f4*)(dst + RowTile<PT>::at(e4 / G4, (e4 % G4) * 4)) = (f4){v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
   }
 }
 // dy tile: from the caller's dout (io dtype) or from the gated fp32 (Bt,L,H,P) workspace copy.

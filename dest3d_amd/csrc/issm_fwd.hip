@@ -38,7 +38,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_chunk_local(KP p, float* __rest
 #endif
 template <int PT, bool BF>
 struct FwdScanSmem {
-  static constexpr int LDPT = PT * 16 + 4;
   static constexpr int LDK = NS + 8;  // row stride of the bf16 tiles
   // fp32 inputs: the product over the state index on (hi, lo) bf16 tiles, hi.hi + hi.lo + lo.hi, instead of fp32
   // matrix instructions.  An fp32 matrix instruction takes the vector ALU's issue slots (the two never overlap on this
@@ -48,7 +47,7 @@ struct FwdScanSmem {
   static constexpr bool SPL = !BF && PT >= SCAN_SPLIT_FROM;
   static constexpr bool B16 = BF || SPL;
   static constexpr int NH = SPL ? 2 : 1;
-  float xs[CS * LDPT];                                          // x [s][p]
+  float xs[RowTile<PT>::SIZE];                                  // x [s][p]
   typename std::conditional<B16, uint16_t, float>::type ct[NH * CS * (B16 ? LDK : LDN)];       // C * exp2(cs) [l][n]
   typename std::conditional<B16, uint16_t, float>::type hs[NH * PT * 16 * (B16 ? LDK : LDN)];  // H [p][n]
 };
@@ -94,7 +93,8 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef FwdScanSmem<PT, IOB> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
-  constexpr int LDPT = SM::LDPT, LDK = SM::LDK;
+  typedef RowTile<PT> XT;
+  constexpr int LDX = XT::LD, LDK = SM::LDK;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
@@ -128,7 +128,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   {
     float xv[CS * PT * 16 / NTHREADS];
     lp_load<IOB, PT, FULL>(p, u, p.x[u.dir], xv);
-    lp_store<PT>(xv, s.xs, LDPT);
+    lp_store<PT>(xv, s.xs);
   }
   f4 acc[PT];
 #pragma unroll
@@ -205,8 +205,8 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
       split4(mw, ah, al);
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt) {
-        const float* bp = s.xs + (16 * kb + 4 * g4) * LDPT + pt * 16 + cm;
-        const float xw[4] = {bp[0], bp[LDPT], bp[2 * LDPT], bp[3 * LDPT]};
+        const float* bp = s.xs + XT::at(16 * kb + 4 * g4, pt * 16 + cm);
+        const float xw[4] = {bp[0], bp[LDX], bp[2 * LDX], bp[3 * LDX]};
         bf4 bh, bl;
         split4(xw, bh, bl);
         acc[pt] = mfma_bf16k(al, bh, acc[pt]);
@@ -231,7 +231,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
       const int tt = u.c * CS + l;
       const bool ok = tt < p.L && pp < p.P;
       const int pr = ok ? phys_row(p, u.dir, tt) : 0;
-      v[r] = fmaf(dcoef, s.xs[l * LDPT + pp], acc[pt][r]);
+      v[r] = fmaf(dcoef, s.xs[XT::at(l, pp)], acc[pt][r]);
       if (tz.ptr && ok) {
         if (out_x) out_x[(((long)u.bt * p.L + pr) * p.H + u.h) * p.P + pp] = v[r];
         const float zz = ldv(tz.ptr, (long)u.b * tz.s0 + (long)pr * tz.s1 + (long)u.h * tz.s2 + pp, p.io_dt);
