@@ -21,8 +21,8 @@
 // workgroup where some column exceeds it -- very large dt' |A| -- is left out here, marked in `redo`, and evaluated by the level-hierarchy kernel
 // (k_bwd_chunk / k_bwd_chunk_bf with `redo`), which has no such limit.  Operands, complete tiles: bf16 inputs -> one bf16
 // instruction per block, operands rounded once; fp32 inputs -> operands as (hi, lo) bf16 pairs (17 significand
-// bits and more), a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, and a
-// gated dy: the level form evaluates these calls wherever this kernel cannot, close pairs of rows (bf16 inputs) or all pairs
+// bits and more), a.b = (ah.bl + al.bh) + (ah.bh + al.bl), each bracket one K = 32 instruction.  Incomplete tiles, four fp32 head
+// tiles, and a gated dy: the level form evaluates these calls wherever this kernel cannot, close pairs of rows (bf16 inputs) or all pairs
 // (fp32 inputs) from fp32 operands, and what a pair is computed in is not to depend on the kernel.  So the diagonal blocks
 // (bf16 inputs) or all blocks (fp32 inputs) are fp32 matrix instructions there.  That costs less than it saves: no operand is
 // split, and the 90 - 130 bytes a lane that the pairs of the incomplete form spilled are gone.  d/d(cs) is formed as (operand
@@ -54,8 +54,11 @@ struct BwdTileSmem {
   static constexpr int KW = 16 * PT, LDP = KW + 8;  // x / dy tiles [l][p]
   static constexpr int LDM = CS + 8;                // T[i][j] = dM[max(i,j)][min(i,j)]
   static constexpr int NH = SPLIT ? 2 : 1;          // hi (and lo) copies
+  // Wide fp32 heads: x and dy one after the other in one place (see TURNS in the kernel).
+  static constexpr bool TURNS = SPLIT && PT >= 3;
   uint16_t xs[NH * CS * LDP];
-  uint16_t dys[NH * CS * LDP];
+  uint16_t dys_own[TURNS ? 8 : NH * CS * LDP];
+  __device__ __forceinline__ uint16_t* dys() { return TURNS ? xs : dys_own; }
   alignas(16) uint16_t tm[NH * CS * LDM];
   static constexpr int LDF = CS + 4;                // the same matrix in fp32 (fp32 inputs, incomplete tiles)
   static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
@@ -102,12 +105,21 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
                                                           const float* __restrict__ dm, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
   constexpr bool SPLIT = !IOB;
-  constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && !FULL;  // fp32 products in the diagonal blocks / in all blocks
+  // fp32 products in the diagonal blocks / in all blocks.  (Four head tiles, complete: as the level form, which took these calls
+  // before, has the closest pairs in fp32.  Operand pairs would leave ddt, dB, dC 5.0 -> 5.4e-6 of their norm from float64, fp32 products
+  // 4.9e-6; of 9.55 ms of training step with the level form, 16 x 2048 tokens, 16 heads x 64, 512 states, 9.09 and 9.2 are left.)
+  constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && (!FULL || PT >= 4);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdTileSmem<PT, SPLIT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
   constexpr int LDP = SM::LDP, LDM = SM::LDM, KT = (PT + 1) / 2;
   constexpr bool BCL = SM::BCL;
+  // Three or four head tiles of fp32 inputs: x and dS make Q, then dy and H, which are requested at the head's start and not a head
+  // ahead, make R in the same place: two barriers a head more.  With all four at once the prefetch spills 76 bytes a lane at three
+  // head tiles, each reload waiting for every request before it, and at four the tiles leave one workgroup a CU.  8 x 1024 tokens, 8
+  // heads, 256 states, both directions, per direction: heads of 48 128 and 137 -> 104 and 112 us; of 64, which took the level form, 135
+  // -> 114 and 121.
+  constexpr bool TURNS = SM::TURNS;
   constexpr int KP_ = PT * 4;  // dS / H values per lane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
@@ -162,6 +174,22 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   f4 l_xv[SPLIT ? PT : 1], l_dv[SPLIT ? PT : 1];
   uint2 l_nx[SPLIT ? 1 : PT], l_ny[SPLIT ? 1 : PT];
   float l_raw[16], l_A, l_bias, l_dsv[KP_], l_hv[KP_], l_Bv[BCL ? 1 : 16], l_Cv[BCL ? 1 : 16];
+  auto request_dy_h = [&](int h) {   // TURNS: the operands of R
+    constexpr int G4 = 4 * PT;
+    int tq = tid;
+    asm volatile("" : "+v"(tq));
+    const TensorD& ty = p.dout[u.dir];
+    const float* qy = (const float*)ty.ptr + ((long)u.b * ty.s0 + (long)h * ty.s2);
+    const long t0 = u.dir ? p.L - 1 - u.c * CS : u.c * CS, sgn = u.dir ? -1 : 1;
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      const int e4 = tq + i * NTHREADS, l = e4 / G4, p4 = (e4 % G4) * 4;
+      const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
+      const f4 a = *(const f4*)(qy + (ok ? (t0 + sgn * l) * ty.s1 + p4 : 0));
+      l_dv[i] = ok ? a : (f4){0, 0, 0, 0};
+    }
+    lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, h), p.P, p.N, n, vn, g4, PNF, l_hv);
+  };
   auto request = [&](int hnext) {
     constexpr int G4 = 4 * PT;
     int tq = tid;
@@ -187,8 +215,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
         const long ox = ok ? (t0 + sgn * l) * tx.s1 + p4 : 0, oy = ok ? (t0 + sgn * l) * ty.s1 + p4 : 0;
         if constexpr (SPLIT) {
-          const f4 a = *(const f4*)(qy + oy), b = *(const f4*)(qx + ox);
-          l_dv[i] = ok ? a : (f4){0, 0, 0, 0};
+          if constexpr (!TURNS) {
+            const f4 a = *(const f4*)(qy + oy);
+            l_dv[i] = ok ? a : (f4){0, 0, 0, 0};
+          }
+          const f4 b = *(const f4*)(qx + ox);
           l_xv[i] = ok ? b : (f4){0, 0, 0, 0};
         } else {
           const uint2 a = *(const uint2*)(qy + oy), b = *(const uint2*)(qx + ox);
@@ -205,10 +236,24 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       l_bias = p.dt_bias ? b : 0.0f;
     }
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_dsv);
-    lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
+    if constexpr (!TURNS) lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
     if constexpr (!BCL) {
       lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, l_Bv);
       lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, l_Cv);
+    }
+  };
+  // the thread's share of a (64 x 16 PT) tile as (hi, lo) pairs into LDS
+  auto put_split = [&](const f4 (&v)[SPLIT ? PT : 1], uint16_t* dst, int tq) {
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        const int e4 = tq + i * NTHREADS, o = (e4 / (4 * PT)) * LDP + (e4 % (4 * PT)) * 4;
+        const float w[4] = {v[i][0], v[i][1], v[i][2], v[i][3]};
+        bf4 h, l;
+        split4(w, h, l);
+        *(bf4*)(dst + o) = h;
+        *(bf4*)(dst + CS * LDP + o) = l;
+      }
     }
   };
   const int hh0 = PARTS ? (int)blockIdx.y * heads_each : 0;
@@ -246,24 +291,14 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       }
       if constexpr (SPLIT) {
-#pragma unroll
-        for (int i = 0; i < PT; ++i) {
-          const int e4 = tq + i * NTHREADS, o = (e4 / G4) * LDP + (e4 % G4) * 4;
-          const float wy[4] = {l_dv[i][0], l_dv[i][1], l_dv[i][2], l_dv[i][3]};
-          const float wx[4] = {l_xv[i][0], l_xv[i][1], l_xv[i][2], l_xv[i][3]};
-          bf4 h, l;
-          split4(wy, h, l);
-          *(bf4*)(s.dys + o) = h;
-          *(bf4*)(s.dys + CS * LDP + o) = l;
-          split4(wx, h, l);
-          *(bf4*)(s.xs + o) = h;
-          *(bf4*)(s.xs + CS * LDP + o) = l;
-        }
+        if constexpr (!TURNS) put_split(l_dv, s.dys(), tq);
+        put_split(l_xv, s.xs, tq);
       } else {
-        lp_store_raw<PT, LDP>(l_ny, s.dys, tq);
+        lp_store_raw<PT, LDP>(l_ny, s.dys(), tq);
         lp_store_raw<PT, LDP>(l_nx, s.xs, tq);
       }
     }
+    if constexpr (TURNS) request_dy_h(u.h);
 
     // ---- dt transform and the per-tile running sums, before the barrier that publishes the tiles: the same barrier
     // then also publishes whether any column of the workgroup is out of the form's range
@@ -287,13 +322,56 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     if (tid == 0) redo[(p.dir0 * (int)gridDim.x + wg) * p.hpg + hh] = skip ? 1 : 0;
     if (DIAG32 && skip) s.shared[wave] = 1;
     const uint16_t* xs_ = s.xs;
-    const uint16_t* dys_ = s.dys;
+    const uint16_t* dys_ = s.dys();
     const uint16_t* tm_ = s.tm;
 
     float dcs[16], val[16], gsum = 0.0f;   // gsum: the lane's share of the states' gradient to the chunk's total, see below
 #pragma unroll
     for (int k = 0; k < 16; ++k) dcs[k] = val[k] = 0.0f;
     if (!skip) {
+      // dS and H of the lane's column as (hi, lo) bf16 pairs: the B operands of Q = x . dS and R = dy . H (products over
+      // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states, whose rounding to
+      // 8 bits would be far above that of the inputs.
+      auto state_pairs = [&](const float (&v)[KP_], bf8 (&hi)[KT], bf8 (&lo)[KT]) {
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+          float a[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) a[j] = 8 * t + j < KP_ ? v[(8 * t + j) % KP_] : 0.0f;
+          split8(a, hi[t], lo[t]);
+        }
+      };
+      f4 qs[TURNS ? 4 : 1], rs[TURNS ? 4 : 1];
+      if constexpr (TURNS) {
+        int cq = cm, gq = g4, tq = tid;
+        asm volatile("" : "+v"(cq), "+v"(gq), "+v"(tq));
+        auto rows_times = [&](const bf8 (&hi)[KT], const bf8 (&lo)[KT], f4 (&out)[TURNS ? 4 : 1]) {
+#pragma unroll
+          for (int R = 0; R < 4; ++R) {
+            f4 q = {0, 0, 0, 0};
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+              const bool half = (PT & 1) && t == KT - 1;
+              const uint16_t* lo_tile = xs_ + CS * LDP;
+              const bf8 xh = half ? split_frag<LDP, true>(xs_, R * 16 + cq, gq, t) : split_frag<LDP>(xs_, R * 16 + cq, gq, t);
+              const bf8 xl = half ? split_frag<LDP, true>(lo_tile, R * 16 + cq, gq, t) : split_frag<LDP>(lo_tile, R * 16 + cq, gq, t);
+              q = mfma_bf(xh, lo[t], q);
+              q = mfma_bf(xl, hi[t], q);
+              q = mfma_bf(xh, hi[t], q);
+            }
+            out[R] = q;
+          }
+        };
+        bf8 hi[KT], lo[KT];
+        state_pairs(l_dsv, hi, lo);
+        rows_times(hi, lo, qs);
+        __syncthreads();   // (skip is the workgroup's)
+        put_split(l_dv, s.dys(), tq);
+        gsum = lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+        state_pairs(l_hv, hi, lo);
+        __syncthreads();
+        rows_times(hi, lo, rs);
+      }
       // ---- decay factors and the operand rows
       __builtin_amdgcn_sched_barrier(0);
       float up[16], iup[16];
@@ -368,25 +446,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
       int cq = cm, gq = g4;
       asm volatile("" : "+v"(cq), "+v"(gq));
-      // dS and H of the lane's column as (hi, lo) bf16 pairs: the B operands of Q = x . dS and R = dy . H (products over
-      // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states, whose rounding to
-      // 8 bits would be far above that of the inputs.
       // The chunk's total decay acts on the states alone, with the gradient sum_p dS H_next = exp2(total) sum_p dS H +
       // sum_l (Bd exp2(total - cs))[l] Q[l]: the second sum is the state terms of the column phase, which cancel against it
       // exactly in the suffix sums, so the next chunk's H is not read and nothing has to be summed over p elsewhere.
-      gsum = across * across * lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+      if constexpr (!TURNS) gsum = lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+      gsum *= across * across;
       if constexpr (SPLIT) asm volatile("" : "+v"(gsum));   // (8 - 20 bytes a lane of scratch less; bf16 inputs: more)
       bf8 dsh[KT], dsl[KT], hh_[KT], hl_[KT];
-#pragma unroll
-      for (int t = 0; t < KT; ++t) {
-        float a[8], b[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          a[j] = 8 * t + j < KP_ ? l_dsv[(8 * t + j) % KP_] : 0.0f;
-          b[j] = 8 * t + j < KP_ ? l_hv[(8 * t + j) % KP_] : 0.0f;
-        }
-        split8(a, dsh[t], dsl[t]);
-        split8(b, hh_[t], hl_[t]);
+      if constexpr (!TURNS) {
+        state_pairs(l_dsv, dsh, dsl);
+        state_pairs(l_hv, hh_, hl_);
       }
       unsigned mf[2], mg[2];  // bf16-pair masks of the diagonal block for this lane's four columns 4 g4 + j
 #pragma unroll
@@ -454,8 +523,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         f4 sf, sg;                                // the state terms
         {
           f4 q = {0, 0, 0, 0}, r = {0, 0, 0, 0};
+          if constexpr (TURNS) {
+            q = qs[R];
+            r = rs[R];
+          }
 #pragma unroll
-          for (int t = 0; t < KT; ++t) {
+          for (int t = 0; t < (TURNS ? 0 : KT); ++t) {
             const bool half = (PT & 1) && t == KT - 1;
             const bf8 xfr = half ? split_frag<LDP, true>(xs_, R * 16 + cq, gq, t) : split_frag<LDP>(xs_, R * 16 + cq, gq, t);
             const bf8 yfr = half ? split_frag<LDP, true>(dys_, R * 16 + cq, gq, t) : split_frag<LDP>(dys_, R * 16 + cq, gq, t);
@@ -665,11 +738,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
 // Whether the tile-base kernel is built for this call (otherwise the level-hierarchy kernel does all the work): no packed
 // sequences (their cuts are outside the form's range), x / B / C and dt of one type, x and dout rows that allow vector
-// accesses, ddt wanted, a gated dy (which is fp32) only beside fp32 inputs, and -- fp32
-// inputs with four head tiles would need split x / dy tiles and T that leave one workgroup per CU -- P <= 48 for fp32.
+// accesses, ddt wanted, a gated dy (which is fp32) only beside fp32 inputs.
 bool bwd_tile_available(const KP& p, const float* dy_ws) {
   if (p.seq_idx || (dy_ws && p.io_dt) || p.io_dt != p.dt_dt || !p.ddt.ptr) return false;
-  if (p.io_dt == 0 && p.P > 48) return false;
   const int es = p.io_dt ? 2 : 4;
   for (int d = 0; d < p.ndir; ++d) {
     const TensorD* ts[2] = {&p.x[d], &p.dout[d]};
@@ -728,7 +799,8 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
     else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
   } else {
     if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
-    else e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    else e = launch_bwd_tile_t<4, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
   }
   if (e) return e;
   return (int)hipGetLastError();

@@ -951,6 +951,26 @@ def test_tiles_that_decay_as_far_as_the_tile_base_form_reaches(dtype, L_, N, P, 
         _check("d" + k, g[k], v, 4e-4 if fp32 else (5e-2 if k == "A" else 2e-2))
 
 
+@pytest.mark.parametrize("far", [False, True], ids=["", "a head out of range"])
+@pytest.mark.parametrize("L_,N,P,H,G,gated", [(128, 64, 36, 2, 1, False), (192, 128, 48, 4, 2, False), (128, 64, 52, 3, 1, False),
+                                              (128, 64, 64, 5, 1, False), (100, 70, 64, 2, 1, False), (67, 5, 40, 2, 1, False),
+                                              (128, 64, 64, 2, 2, True)])
+def test_chunk_backward_of_wide_fp32_heads(L_, N, P, H, G, gated, far):
+    """Heads of three and four tiles, fp32: x with dS and dy with H take turns in one place of the workgroup's memory, also where a
+    head in between is left to the level form.  Operands hold 16 bits or more (1.5e-5, less in the mean; four times that and the
+    sums' order: 1e-4); running sums in the thousands as in test_heads_outside_the_tile_kernel_range_are_redone_by_the_level_kernel."""
+    _say(f"wide fp32 heads L={L_} N={N} P={P} H={H} G={G} gated={gated} far={far}")
+    d = _problem(2, L_, H, P, N, G, seed=P + N, z=gated)
+    if far:
+        d["A"][1] *= 100.0
+    y, fin, ref = _oracle(d, GRAD_NAMES)
+    yg, fg, g, _ = _run_operator(d, torch.float32)
+    _check("y", yg, y, 1e-3 if far else 1e-4)
+    _check("final", fg, fin, 1e-3 if far else 1e-4)
+    for k, v in ref.items():
+        _check("d" + k, g[k], v, (5e-2 if k == "A" else 1e-2) if far else 1e-4)
+
+
 def test_inplace_edit_between_forward_and_backward_raises():
     """The operator saves its inputs for the backward as the reference does (issm_combined.py:42): changing one of them
     in place before backward must raise PyTorch's version-counter error, not return gradients of other data."""
