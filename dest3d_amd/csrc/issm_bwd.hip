@@ -1205,22 +1205,6 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, bv);
   pn_load<PT, FULL>(p, ds, 0, sv);
-  // M^T of this wave's 16 columns goes straight into matrix-operand registers (lane (column cm, group g4) holds
-  // rows 16 kb + 4 g4 .. + 3 of the blocks kb >= wave, the upper triangle of the diagonal block zeroed): no LDS tile,
-  // which lets a fourth workgroup live on the CU
-  float mf[4][4];
-  {
-    const float* mcol = cabt + sq_off(p, u.bt, u.c, u.h) + (4 * g4) * CS + wave * 16 + cm;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) mf[kb][j] = mcol[(16 * max(kb, wave) + j) * CS];  // no branch between the loads
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (kb < wave || (kb == wave && cm > 4 * g4 + j)) mf[kb][j] = 0.0f;
-  }
   {
     float dv[CS * PT * 16 / NTHREADS];
     dy_load<IOB, PT, FULL>(p, u, dy_ws, dv);
@@ -1299,6 +1283,23 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
         for (int pt = 0; pt < PT; ++pt) mma16_mm(acc[pt], s.bt, LDN, wave * 16, s.dss, LDN, pt * 16, kb, lane);
     }
     __syncthreads();
+  }
+  // (requested behind the loop, as in k_chunk_scan: 44 bytes a lane of scratch at 128 registers otherwise)
+  // M^T of this wave's 16 columns goes straight into matrix-operand registers (lane (column cm, group g4) holds
+  // rows 16 kb + 4 g4 .. + 3 of the blocks kb >= wave, the upper triangle of the diagonal block zeroed): no LDS tile,
+  // which lets a fourth workgroup live on the CU
+  float mf[4][4];
+  {
+    const float* mcol = cabt + sq_off(p, u.bt, u.c, u.h) + (4 * g4) * CS + wave * 16 + cm;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mf[kb][j] = mcol[(16 * max(kb, wave) + j) * CS];  // no branch between the loads
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (kb < wave || (kb == wave && cm > 4 * g4 + j)) mf[kb][j] = 0.0f;
   }
   // dx[m][p] += sum_{l>=m} M[l][m] dy[l][p]
 #pragma unroll

@@ -111,20 +111,6 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, cv);
   pn_load<PT, FULL>(p, hsrc, 0, hv);
-  // M of this wave's 16 rows goes straight into matrix-operand registers (lane (row cm, group g4) holds columns
-  // 16 kb + 4 g4 .. + 3 of the blocks kb <= wave, the upper triangle of the diagonal block zeroed): no LDS tile, which
-  // lets a fourth workgroup live on the CU
-  f4 mf[4];
-  {
-    const float* mrow = cabt + sq_off(p, u.bt, u.c, u.h) + (wave * 16 + cm) * CS + 4 * g4;
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) mf[kb] = *(const f4*)(mrow + 16 * min(kb, wave));  // no branch between the loads
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (kb > wave || (kb == wave && 4 * g4 + j > cm)) mf[kb][j] = 0.0f;
-  }
   {
     float xv[CS * PT * 16 / NTHREADS];
     lp_load<IOB, PT, FULL>(p, u, p.x[u.dir], xv);
@@ -194,6 +180,22 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
     }
     __syncthreads();
   }
+  // Requested here and not with the first step's operands: over the loop its 16 registers pushed 8 dwords a lane to scratch at 128
+  // registers, or kept a fourth workgroup off the CU.
+  // M of this wave's 16 rows goes straight into matrix-operand registers (lane (row cm, group g4) holds columns
+  // 16 kb + 4 g4 .. + 3 of the blocks kb <= wave, the upper triangle of the diagonal block zeroed): no LDS tile, which
+  // lets a fourth workgroup live on the CU
+  f4 mf[4];
+  {
+    const float* mrow = cabt + sq_off(p, u.bt, u.c, u.h) + (wave * 16 + cm) * CS + 4 * g4;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) mf[kb] = *(const f4*)(mrow + 16 * min(kb, wave));  // no branch between the loads
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (kb > wave || (kb == wave && 4 * g4 + j > cm)) mf[kb][j] = 0.0f;
+  }
   // y[l][p] += sum_{s<=l} M[l][s] x[s][p]; rows of this wave only need s < 16(wave+1)
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
@@ -242,8 +244,7 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
     gstore<IOB, 4>(const_cast<void*>(to.ptr), (long)u.b * to.s0 + (long)u.h * to.s2, off, v);
   }
 }
-// two head tiles, fp32 inputs or edges: 128 registers, so that a fourth workgroup lives on the CU (130 - 145 without the
-// bound; the spilled dwords cost less than the fourth workgroup gives: 52 -> 48.5 us)
+// two head tiles, fp32 inputs or edges: 128 registers, so that a fourth workgroup lives on the CU (52 -> 48.5 us)
 template <int PT, bool IOB, bool DTB, bool FULL>
 __global__ __launch_bounds__(NTHREADS, (PT <= 2 && (!IOB || !FULL)) ? 4 : 1) void k_chunk_scan(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
   k_chunk_scan_body<PT, IOB, DTB, FULL>(p, states, cabt, out_x);
