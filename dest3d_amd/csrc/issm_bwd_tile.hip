@@ -64,11 +64,12 @@ struct BwdTileSmem {
   static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
   __device__ __forceinline__ float* tf() { return reinterpret_cast<float*>(tm); }
   float dbc[32 * NTHREADS];  // per-lane dB / dC accumulators [k][tid]
-  // bf16 inputs, two head tiles: the group's B and C values of every lane, packed in pairs, [i][tid] (i < 8: B, then C).
+  // bf16 inputs: the group's B and C values of every lane, packed in pairs, [i][tid] (i < 8: B, then C).
   // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
-  // streams have been through it in between) and were a third of the kernel's reads.  fp32 inputs have no room for them
-  // at two workgroups per CU, wider heads no registers to spare for the change (they spill and lose what it gains).
-  static constexpr bool BCL = !SPLIT && PT == 2;
+  // streams have been through it in between) and were a third of the kernel's reads; of three and four head tiles, 8 x 1024 tokens,
+  // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 250 states, three 98 and 107:
+  // 93 and 103).  fp32 inputs have no room for them at two workgroups per CU.
+  static constexpr bool BCL = !SPLIT;
   unsigned bc[BCL ? 16 * NTHREADS : 1];
   int bad[4];                // per wave: some column of the head exceeds SPAN_LIMIT
   int shared[4];             // per wave: some head was left to the level form
