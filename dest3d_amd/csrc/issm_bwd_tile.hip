@@ -54,12 +54,12 @@ struct BwdTileSmem {
   static constexpr int KW = 16 * PT, LDP = KW + 8;  // x / dy tiles [l][p]
   static constexpr int LDM = CS + 8;                // T[i][j] = dM[max(i,j)][min(i,j)]
   static constexpr int NH = SPLIT ? 2 : 1;          // hi (and lo) copies
-  // Wide fp32 heads: x and dy one after the other in one place (see TURNS in the kernel).
-  static constexpr bool TURNS = SPLIT && PT >= 3;
-  uint16_t xs[NH * CS * LDP];
-  uint16_t dys_own[TURNS ? 8 : NH * CS * LDP];
-  __device__ __forceinline__ uint16_t* dys() { return TURNS ? xs : dys_own; }
-  alignas(16) uint16_t tm[NH * CS * LDM];
+  // fp32 inputs: x and dy one after the other in one place.  (The last rows of the arrays go without
+  // padding, and three head tiles then take exactly half of a CU's 160 KB.)
+  uint16_t xs[NH * CS * LDP - (SPLIT ? 8 : 0)];
+  uint16_t dys_own[SPLIT ? 0 : NH * CS * LDP];
+  __device__ __forceinline__ uint16_t* dys() { return SPLIT ? xs : dys_own; }
+  alignas(16) uint16_t tm[NH * CS * LDM - (SPLIT ? 8 : 0)];
   static constexpr int LDF = CS + 4;                // the same matrix in fp32 (fp32 inputs, incomplete tiles)
   static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
   __device__ __forceinline__ float* tf() { return reinterpret_cast<float*>(tm); }
@@ -68,9 +68,14 @@ struct BwdTileSmem {
   // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
   // streams have been through it in between) and were a third of the kernel's reads; of three and four head tiles, 8 x 1024 tokens,
   // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 250 states, three 98 and 107:
-  // 93 and 103).  fp32 inputs have no room for them at two workgroups per CU.
+  // 93 and 103).
   static constexpr bool BCL = !SPLIT;
-  unsigned bc[BCL ? 16 * NTHREADS : 1];
+  unsigned bc[BCL ? 16 * NTHREADS : 0];
+  // fp32 inputs of up to three head tiles: the B values, [k][tid]; C has no room (8 x 1024 tokens, 8 heads x 32, 256 states, both
+  // directions, training step 480 -> 466 us, per direction 90 and 100 -> 85 and 94; heads of 48 105 and 112 -> 94 and 104.  It is the
+  // 32 registers that B takes neither ahead of a head nor through it, and the loads).
+  static constexpr bool BL = SPLIT && PT <= 3;
+  float bl[BL ? 16 * NTHREADS : 0];
   int bad[4];                // per wave: some column of the head exceeds SPAN_LIMIT
   int shared[4];             // per wave: some head was left to the level form
 };
@@ -114,13 +119,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   typedef BwdTileSmem<PT, SPLIT> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
   constexpr int LDP = SM::LDP, LDM = SM::LDM, KT = (PT + 1) / 2;
-  constexpr bool BCL = SM::BCL;
-  // Three or four head tiles of fp32 inputs: x and dS make Q, then dy and H, which are requested at the head's start and not a head
+  constexpr bool BCL = SM::BCL, BL = SM::BL;
+  // fp32 inputs take turns: x and dS make Q, then dy and H, which are requested at the head's start and not a head
   // ahead, make R in the same place: two barriers a head more.  With all four at once the prefetch spills 76 bytes a lane at three
   // head tiles, each reload waiting for every request before it, and at four the tiles leave one workgroup a CU.  8 x 1024 tokens, 8
   // heads, 256 states, both directions, per direction: heads of 48 128 and 137 -> 104 and 112 us; of 64, which took the level form, 135
-  // -> 114 and 121.
-  constexpr bool TURNS = SM::TURNS;
+  // -> 114 and 121; of 32 the same as before, but it makes room for B (SM::BL).
   constexpr int KP_ = PT * 4;  // dS / H values per lane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
@@ -147,6 +151,12 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
   if (DIAG32) s.shared[wave] = 0;
 
+  if constexpr (BL) {
+    float tb[16];
+    lane_load_ln<false>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, tb);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s.bl[k * NTHREADS + tid] = tb[k];
+  }
   if constexpr (BCL) {
     float tb[16], tc[16];
     lane_load_ln<true>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, tb);
@@ -174,8 +184,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   uint4 l_th0, l_th1, l_tl0, l_tl1;
   f4 l_xv[SPLIT ? PT : 1], l_dv[SPLIT ? PT : 1];
   uint2 l_nx[SPLIT ? 1 : PT], l_ny[SPLIT ? 1 : PT];
-  float l_raw[16], l_A, l_bias, l_dsv[KP_], l_hv[KP_], l_Bv[BCL ? 1 : 16], l_Cv[BCL ? 1 : 16];
-  auto request_dy_h = [&](int h) {   // TURNS: the operands of R
+  float l_raw[16], l_A, l_bias, l_dsv[KP_], l_hv[KP_], l_Bv[BCL || BL ? 1 : 16], l_Cv[BCL ? 1 : 16];
+  auto request_dy_h = [&](int h) {   // fp32 inputs: the operands of R
     constexpr int G4 = 4 * PT;
     int tq = tid;
     asm volatile("" : "+v"(tq));
@@ -216,10 +226,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
         const long ox = ok ? (t0 + sgn * l) * tx.s1 + p4 : 0, oy = ok ? (t0 + sgn * l) * ty.s1 + p4 : 0;
         if constexpr (SPLIT) {
-          if constexpr (!TURNS) {
-            const f4 a = *(const f4*)(qy + oy);
-            l_dv[i] = ok ? a : (f4){0, 0, 0, 0};
-          }
           const f4 b = *(const f4*)(qx + ox);
           l_xv[i] = ok ? b : (f4){0, 0, 0, 0};
         } else {
@@ -237,9 +243,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       l_bias = p.dt_bias ? b : 0.0f;
     }
     lane_load_pn<KP_>(dstates + dst_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_dsv);
-    if constexpr (!TURNS) lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
+    if constexpr (!SPLIT) lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, hnext), p.P, p.N, n, vn, g4, PNF, l_hv);
     if constexpr (!BCL) {
-      lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, l_Bv);
+      if constexpr (!BL) lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, l_Bv);
       lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, l_Cv);
     }
   };
@@ -292,14 +298,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       }
       if constexpr (SPLIT) {
-        if constexpr (!TURNS) put_split(l_dv, s.dys(), tq);
         put_split(l_xv, s.xs, tq);
       } else {
         lp_store_raw<PT, LDP>(l_ny, s.dys(), tq);
         lp_store_raw<PT, LDP>(l_nx, s.xs, tq);
       }
     }
-    if constexpr (TURNS) request_dy_h(u.h);
+    if constexpr (SPLIT) request_dy_h(u.h);
 
     // ---- dt transform and the per-tile running sums, before the barrier that publishes the tiles: the same barrier
     // then also publishes whether any column of the workgroup is out of the form's range
@@ -342,11 +347,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           split8(a, hi[t], lo[t]);
         }
       };
-      f4 qs[TURNS ? 4 : 1], rs[TURNS ? 4 : 1];
-      if constexpr (TURNS) {
+      f4 qs[SPLIT ? 4 : 1], rs[SPLIT ? 4 : 1];
+      if constexpr (SPLIT) {
         int cq = cm, gq = g4, tq = tid;
         asm volatile("" : "+v"(cq), "+v"(gq), "+v"(tq));
-        auto rows_times = [&](const bf8 (&hi)[KT], const bf8 (&lo)[KT], f4 (&out)[TURNS ? 4 : 1]) {
+        auto rows_times = [&](const bf8 (&hi)[KT], const bf8 (&lo)[KT], f4 (&out)[SPLIT ? 4 : 1]) {
 #pragma unroll
           for (int R = 0; R < 4; ++R) {
             f4 q = {0, 0, 0, 0};
@@ -393,6 +398,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         return (f4){__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u), __uint_as_float(a.y << 16),
                     __uint_as_float(a.y & 0xffff0000u)};
       };
+      auto b_of = [&](int k) { return BL ? s.bl[k * NTHREADS + tid] : l_Bv[BCL || BL ? 0 : k]; };
       auto half_of = [](unsigned w, int k) { return __uint_as_float((k & 1) ? (w & 0xffff0000u) : (w << 16)); };
       // Cu = C up (operand of the G blocks), Bi = B dt' iup (operand of the F blocks)
       bf4 Ch[4], Bh[4], Cl[4], Bl[4];
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           float cu, bi;
           if constexpr (!BCL) {
             cu = l_Cv[k] * up[k];
-            bi = l_Bv[k] * dtp[k] * iup[k];
+            bi = b_of(k) * dtp[k] * iup[k];
           } else {  // out of the workgroup's LDS copy of the group's B and C
             cu = half_of(s.bc[(8 + (k >> 1)) * NTHREADS + tid], k) * up[k];
             bi = half_of(s.bc[(k >> 1) * NTHREADS + tid], k) * dtp[k] * iup[k];
@@ -425,7 +431,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       // B (and, for bf16 inputs, C) as the column phase needs them: bf16 inputs are bf16 numbers and stay packed, two
       // to a register
       unsigned bvp[8], cvp[8];
-      float bvf[SPLIT ? 16 : 1];
+      float bvf[SPLIT && !BL ? 16 : 1];
       if constexpr (BCL && DIAG32) {  // read tile by tile below
       } else if constexpr (BCL) {
 #pragma unroll
@@ -441,7 +447,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         }
       } else {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) bvf[k] = l_Bv[k];
+        for (int k = 0; k < (BL ? 0 : 16); ++k) bvf[k] = l_Bv[k];
       }
       __builtin_amdgcn_sched_barrier(0);
 
@@ -450,11 +456,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
       // The chunk's total decay acts on the states alone, with the gradient sum_p dS H_next = exp2(total) sum_p dS H +
       // sum_l (Bd exp2(total - cs))[l] Q[l]: the second sum is the state terms of the column phase, which cancel against it
       // exactly in the suffix sums, so the next chunk's H is not read and nothing has to be summed over p elsewhere.
-      if constexpr (!TURNS) gsum = lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
+      if constexpr (!SPLIT) gsum = lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
       gsum *= across * across;
       if constexpr (SPLIT) asm volatile("" : "+v"(gsum));   // (8 - 20 bytes a lane of scratch less; bf16 inputs: more)
       bf8 dsh[KT], dsl[KT], hh_[KT], hl_[KT];
-      if constexpr (!TURNS) {
+      if constexpr (!SPLIT) {
         state_pairs(l_dsv, dsh, dsl);
         state_pairs(l_hv, hh_, hl_);
       }
@@ -524,25 +530,17 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         f4 sf, sg;                                // the state terms
         {
           f4 q = {0, 0, 0, 0}, r = {0, 0, 0, 0};
-          if constexpr (TURNS) {
+          if constexpr (SPLIT) {
             q = qs[R];
             r = rs[R];
           }
 #pragma unroll
-          for (int t = 0; t < (TURNS ? 0 : KT); ++t) {
+          for (int t = 0; t < (SPLIT ? 0 : KT); ++t) {
             const bool half = (PT & 1) && t == KT - 1;
             const bf8 xfr = half ? split_frag<LDP, true>(xs_, R * 16 + cq, gq, t) : split_frag<LDP>(xs_, R * 16 + cq, gq, t);
             const bf8 yfr = half ? split_frag<LDP, true>(dys_, R * 16 + cq, gq, t) : split_frag<LDP>(dys_, R * 16 + cq, gq, t);
             q = mfma_bf(xfr, dsl[t], q);
             r = mfma_bf(yfr, hl_[t], r);
-            if constexpr (SPLIT) {
-              const uint16_t* xl_ = xs_ + CS * LDP;
-              const uint16_t* yl_ = dys_ + CS * LDP;
-              const bf8 xg_ = half ? split_frag<LDP, true>(xl_, R * 16 + cq, gq, t) : split_frag<LDP>(xl_, R * 16 + cq, gq, t);
-              const bf8 yg_ = half ? split_frag<LDP, true>(yl_, R * 16 + cq, gq, t) : split_frag<LDP>(yl_, R * 16 + cq, gq, t);
-              q = mfma_bf(xg_, dsh[t], q);
-              r = mfma_bf(yg_, hh_[t], r);
-            }
             q = mfma_bf(xfr, dsh[t], q);
             r = mfma_bf(yfr, hh_[t], r);
           }
@@ -600,7 +598,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int k = 4 * R + rr;
-          const float bv = SPLIT ? bvf[k] : unpk(bvp, k);
+          const float bv = SPLIT ? (BL ? b_of(k) : bvf[SPLIT && !BL ? k : 0]) : unpk(bvp, k);
           const float E1 = iup[k] * (sg[rr] + xg[rr] + dg[rr]), X2 = up[k] * (sf[rr] + xf[rr] + df[rr]);
           s.dbc[k * NTHREADS + tid] += dtp[k] * E1;
           s.dbc[(16 + k) * NTHREADS + tid] += X2;
@@ -755,6 +753,7 @@ template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
                              float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
   const size_t sm = sizeof(BwdTileSmem<PT, !IOB>);
+  static_assert(sizeof(BwdTileSmem<PT, !IOB>) <= 80 * 1024, "two workgroups a CU");
   const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0;
   auto go = [&](auto kern) -> int {
     if (sm > 64 * 1024)
