@@ -191,17 +191,26 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   const float* qbias = (p.dt_bias ? p.dt_bias : p.A) + u.h * p.N;  // without a bias: any valid address, scaled by 0
   const float bias_on = p.dt_bias ? 1.0f : 0.0f;
 
+  // fp32 inputs, incomplete tiles, two head tiles: C is requested at the step's start and not a step ahead (it is used last, and its 16
+  // registers made the kernel spill 56 bytes a lane: 8 x 1000 tokens, 8 heads x 32, 250 states 60.6 -> 54.3 us, 2 x 160, 4 heads, 128 states
+  // 14.5 -> 13.7; three and four head tiles have the registers)
+  constexpr bool LATE_C = EDGE && !IOB && PT <= 2;
   RawDt rdt[4];
   RawIo rB[4], rC[4];
   F4Any rA, rbias;
+#define ISSM_REQUEST_C(c_)                                                             \
+  {                                                                                    \
+    _Pragma("unroll") for (int J = 0; J < 4; ++J)                                      \
+      rC[J] = *(const RawIo*)(qC + (int)(oC[J % NO] + (unsigned)(J * jC + (c_))));     \
+  }
 #define ISSM_REQUEST(n0_)                                                              \
   {                                                                                    \
     const int c_ = EDGE ? min((n0_) + ncol, p.N - 4) : (n0_);                          \
     _Pragma("unroll") for (int J = 0; J < 4; ++J) {                                    \
       rdt[J] = *(const RawDt*)(qdt + (int)(odt[J % NO] + (unsigned)(J * jdt + c_)));   \
       rB[J] = *(const RawIo*)(qB + (int)(oB[J % NO] + (unsigned)(J * jB + c_)));       \
-      rC[J] = *(const RawIo*)(qC + (int)(oC[J % NO] + (unsigned)(J * jC + c_)));       \
     }                                                                                  \
+    if constexpr (!LATE_C) ISSM_REQUEST_C(c_)                                          \
     rA = *(const F4Any*)(qA + (EDGE ? c_ : c_ + ncol));                                \
     rbias = *(const F4Any*)(qbias + (EDGE ? c_ : c_ + ncol));                          \
   }
@@ -330,6 +339,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     }
   }
 #undef ISSM_REQUEST
+#undef ISSM_REQUEST_C
 
   // ---- M: the waves' partial sums meet in LDS; wave w then finishes blocks w, w + 4, w + 8
 #pragma unroll

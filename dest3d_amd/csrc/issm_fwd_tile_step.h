@@ -9,7 +9,7 @@
     for (int J = 0; J < 4; ++J) {
       unpack4<DTB>(rdt[J], dtv + 4 * J);
       unpack4<IOB>(rB[J], bv + 4 * J);
-      unpack4<IOB>(rC[J], cv + 4 * J);
+      if constexpr (!LATE_C) unpack4<IOB>(rC[J], cv + 4 * J);
     }
     const float A2[4] = {rA.x * LOG2E, rA.y * LOG2E, rA.z * LOG2E, rA.w * LOG2E};
     const float bias[4] = {rbias.x * bias_on, rbias.y * bias_on, rbias.z * bias_on, rbias.w * bias_on};
@@ -26,6 +26,7 @@
           if (j >= skip) q[j] = v[j];
       }
     };
+    if constexpr (LATE_C) ISSM_REQUEST_C(c)
     if (!DEEP) {  // branch-free: the last step asks for its own columns once more
       const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
       ISSM_REQUEST(nn);
@@ -44,7 +45,7 @@
           for (int k = 0; k < 16; ++k) {
             const bool past = 16 * (k >> 2) + i >= nvalid;
             if (past || (k & 3) < skip) dtp[k] = 0.0f;
-            if (past) cv[k] = 0.0f;   // (rows of M past the end come out as zero)
+            if (!LATE_C && past) cv[k] = 0.0f;   // (rows of M past the end come out as zero)
           }
         }
       }
@@ -90,6 +91,15 @@
         for (int k = 4 * J; k < 4 * J + 4; ++k) cv[k] *= up[k];
       }
     } else if constexpr (EDGE) {
+      if constexpr (LATE_C) {
+#pragma unroll
+        for (int J = 0; J < 4; ++J) unpack4<IOB>(rC[J], cv + 4 * J);
+        if (nvalid < CS) {  // uniform
+#pragma unroll
+          for (int k = 0; k < 16; ++k)
+            if (16 * (k >> 2) + i >= nvalid) cv[k] = 0.0f;
+        }
+      }
       // diagonal blocks, before anything else needs registers: W takes the place of B and dt', C up that of C.  fp32 matrix
       // instructions: k-slot kg of instruction r <-> the lane's column r; the blocks' chains are interleaved.
 #pragma unroll
