@@ -143,15 +143,21 @@ static int bwd_head_parts(const issm_dims& d) {
   return (heads - each) * d.ndir < 4 ? 1 : (int)((heads + each - 1) / each);   // (no part without a head)
 }
 
-// Whether the backward's states take one kernel (issm_bwd_walk.hip) or two.  A walk takes 2 us a chunk whatever the grid, until the
-// chip is full of them; two kernels take 12 - 20 us and then what the chip's share of the chunks costs.  So: every CU has a walk
-// (256: 8 x 4096 tokens, 8 heads x 32, 256 states fp32 174 against 208 us, 4 x 1024, two directions 39 against 40; bf16 119 and 152,
-// 30 and 35), or few chunks (8 chunks of 32, 128, 192 walks: 17.4, 19, 20 against 17.6, 21, 25 us fp32, 15, 16, 17 against 16, 20, 24
-// bf16; 16 of 64: 33 against 22), or in between (192 walks: 16 chunks 35.6 against 34.3 - 35.9 us fp32, 29 against 31 bf16; 64 chunks
-// 144 against 138, 100 against 95).
+// Whether the backward's states take one kernel (issm_bwd_walk.hip) or two (k_bwd_dstates, k_state_pass).  Every CU has a walk (256
+// of them): one, which saves the states' way through HBM (8 x 4096 tokens, 8 heads x 32, 256 states fp32 174 against 208 us, bf16
+// 119 and 152; heads of up to 15, whose walks cost what those of 32 do, go by what follows: 4 x 1536 tokens, 8 heads x 8, 512 states
+// 48.5 against 41.2).  Fewer walks wait for latencies one chunk after the other, 3 us and `chunk` for each, while two kernels cost 8 us, 1.3
+// more for each 64 columns that k_bwd_dstates loops over, and the chip's share of what the heads and the states of all chunks take.
+// Both, us: 2 walks of 64 columns, 4 chunks: heads of 32 9.8 and 11.7 (fp32), 8.7 and 10.6 (bf16), of 64 13.4 and 13.2, 10.8 and 11.6;
+// 8 chunks: 16.7 and 12.5, 14.3 and 11.4, 23.6 and 14.0, 18.5 and 12.4.  64 walks of 256 columns, heads of 32, 8 chunks 17.5 and 18.8,
+// 15.2 and 16.7; 12 chunks 24.4 and 21.4, 20.9 and 19.2.  192 walks, heads of 64, 8 chunks 29.6 and 32.4; 16 chunks 54.8 and 48.0, bf16 37.9 and
+// 40.9.  (Of 5760 sizes the line takes the slower side by more than 8 % in 44, by at most 25 %; a walk for all of up to 8 chunks took
+// up to 1.9 times the other side's time.)
 static bool bwd_walks(const KP& p, const float* dy) {
-  const int walks = p.B * p.ndir * p.H * ((p.N + 63) / 64);
-  return (walks >= 256 || p.nc <= 8 || (walks >= 192 && p.nc <= 16)) && bwd_walk_available(p, dy);
+  const int heads = p.B * p.ndir * p.H, slices = (p.N + 63) / 64, walks = heads * slices, pt = p.P <= 32 ? 0 : (p.P - 17) / 16;
+  static const float chunks_us[2][3] = {{1.35f, 1.55f, 1.9f}, {1.1f, 1.25f, 1.45f}};   // (fp32, bf16; heads of up to 32, 48, 64)
+  const float chunk = chunks_us[p.io_dt][pt] + (p.full_tiles ? 0.0f : 0.25f), share = heads * (p.io_dt ? 3e-3f : 4.5e-3f) + (float)walks * p.P * 8e-5f;
+  return ((walks >= 256 && p.P >= 16) || p.nc * (chunk - share) <= 4.6f + 1.27f * slices) && bwd_walk_available(p, dy);
 }
 
 static bool wants_ddt_part(const issm_scan_args* a) { return a->dims.ndir == 2 && a->dt_dtype == ISSM_BF16; }
@@ -455,6 +461,13 @@ int issm_stage_bwd_reduce(const issm_scan_args* a, const float* part_a, const fl
                                     (part_d && a->D) ? a->dD : nullptr, dh0_dir ? a->dh0 : nullptr,
                                     (hipStream_t)a->stream),
                   "bwd_reduce");
+}
+
+int issm_bwd_walks(const issm_scan_args* a) {
+  if (check_common(a)) return 0;
+  const KP p = make_kp(a);
+  // a gated dy is the workspace's; whatever its address, its rows are whole
+  return bwd_walks(p, a->z[0].ptr ? reinterpret_cast<const float*>(a->z[0].ptr) : nullptr) ? 1 : 0;
 }
 
 int issm_scan_bwd(const issm_scan_args* a) {

@@ -1,5 +1,5 @@
 // Backward pass over the chunk states in one kernel (gfx950): dH_c = dy^T (C exp(cs)), the reverse recurrence over the chunks
-// and the matrix dM, for calls whose sequences and column slices fill the chip.
+// and the matrix dM, for calls whose sequences and column slices fill the chip or that have few chunks (bwd_walks, issm_abi.hip).
 //
 // Workgroup = (batch and direction, head, 64 state columns), walking the chunks from the last to the first.  dH contracts over
 // the rows of a chunk and the recurrence is element-wise, so neither needs another workgroup's columns: the lane that owns

@@ -213,9 +213,11 @@ int issm_stage_state_passing_bwd(const issm_scan_args* args, const float* states
 /* issm_stage_bwd_states: the two stages above in one kernel, which walks a head's chunks from the last to the first with
  *   64 columns of the carried gradient in registers: dS_c into dstates, dM into dm, dh0_dir and (unless NULL) g_last, as they leave them.
  *   x / B / C and dt of one type, rows of x and dy in multiples of four elements, no packed sequences, no gate beside bf16
- *   inputs (ISSM_E_UNSUPPORTED otherwise).  issm_scan_bwd takes it where the walks fill the chip. */
+ *   inputs (ISSM_E_UNSUPPORTED otherwise).  issm_scan_bwd takes it where issm_bwd_walks says so: the walks fill the chip, or
+ *   are short (a rule on sizes and types).  issm_bwd_walks launches nothing and reads no tensor; 0 too for arguments that are refused. */
 int issm_stage_bwd_states(const issm_scan_args* args, const float* dy_gated, const float* states, float* dstates, float* dm,
                           float* g_last, float* dh0_dir);
+int issm_bwd_walks(const issm_scan_args* args);
 /* issm_stage_bwd_chunk: ddt, dB, dC of direction `dir` and the per-unit partial sums
  *   part_a / part_bias (Bt*nc,H,N) of dA / ddt_bias.  g_last is not read (the kernels form it from states, dstates and
  *   their own products) and may be NULL.  ddt accumulates into args->ddt when

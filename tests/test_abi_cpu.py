@@ -57,6 +57,46 @@ def test_struct_layout_matches_header(lib):
     assert n.value > 2 * 4 * 8 * nc * 8 * 32 * 256
 
 
+@pytest.mark.parametrize("B,L_,H,P,N,nd,bf,walks", [
+    (1, 512, 2, 64, 64, 1, False, 0),      # 23.6 us as one kernel, 14.0 as two
+    (1, 512, 2, 64, 64, 1, True, 0),       # 18.5 and 12.4
+    (1, 492, 2, 64, 58, 1, False, 0),      # incomplete tiles: 27.7 and 14.9
+    (2, 512, 8, 64, 64, 1, False, 0),      # 24.5 and 14.9
+    (1, 512, 2, 16, 64, 1, False, 0),      # 16.6 and 12.5
+    (1, 128, 2, 64, 64, 1, False, 1),      # 8.5 and 12.2
+    (2, 160, 4, 32, 128, 1, False, 1),
+    (4, 512, 8, 32, 256, 1, False, 1),     # 19.1 and 21.1
+    (4, 512, 8, 32, 256, 1, True, 1),      # 15.9 and 20.5
+    (4, 1024, 8, 32, 256, 1, False, 0),    # 34.8 and 27.9
+    (6, 1024, 8, 64, 256, 1, False, 0),    # 54.8 and 48.0
+    (6, 1024, 8, 64, 256, 1, True, 1),     # 37.9 and 40.9
+    (8, 1024, 8, 32, 256, 2, False, 1),    # a walk a CU and more
+    (1, 16384, 8, 32, 512, 4, False, None),
+    (4, 1536, 8, 8, 512, 1, False, 0),     # 48.5 and 41.2
+])
+def test_backward_states_in_one_kernel_or_two(lib, B, L_, H, P, N, nd, bf, walks):
+    """issm_scan_bwd's choice follows the kernels' times (in us, above, where the two were measured)."""
+    from dest3d_amd import _lib as L
+    a = L.ScanArgs()
+    d = a.dims
+    d.batch, d.seqlen, d.nheads, d.headdim, d.dstate, d.ngroups, d.chunk_size, d.ndir = B, L_, H, P, N, 1, 64, min(nd, 2)
+    if walks is None:   # refused: no direction count of four
+        d.ndir = nd
+    a.io_dtype = a.dt_dtype = int(bf)
+    a.dt_min, a.dt_max = 0.0, float("inf")
+    at = iter(range(1 << 20, 1 << 30, 1 << 20))   # (addresses nothing reads)
+    for i in range(min(nd, 2)):
+        for t, h, w in ((a.x, H, P), (a.dout, H, P), (a.Bm, 1, N), (a.Cm, 1, N)):
+            t[i].ptr = next(at)
+            t[i].stride[0], t[i].stride[1], t[i].stride[2] = L_ * h * w, h * w, w
+    a.dt.ptr, a.A = next(at), next(at)
+    a.dt.stride[0], a.dt.stride[1], a.dt.stride[2] = L_ * H * N, H * N, N
+    assert lib.issm_bwd_walks(C.byref(a)) == (walks or 0)
+    if walks:   # what the kernel cannot take it is not given: rows of dout that are not whole
+        a.dout[0].ptr += 2
+        assert lib.issm_bwd_walks(C.byref(a)) == 0
+
+
 def test_status_codes(lib):
     from dest3d_amd import _lib as L
     a = L.ScanArgs()
