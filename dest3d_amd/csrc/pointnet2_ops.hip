@@ -1159,7 +1159,7 @@ static_assert(ROW_POINTS < (int)NO_POINT, "no point has this number, and a targe
 // rows that are not needed yet.  8 samples, 256 channels, 2048 <- 20000
 // points: 84 -> 82 us so, 69 with the rows put into LDS 16 bytes at a time and read from there 8, 68 with fewer instructions.
 template <int R, bool ZERO, bool PIPE>
-__global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m, const float* __restrict__ grad_out, InvList l,
+__global__ __launch_bounds__(INV_T, PIPE ? 4 : 8) void k_interp_rows_grad(int c, int n, int m, const float* __restrict__ grad_out, InvList l,
                                                            float* __restrict__ grad_points, int sets, int per) {
   extern __shared__ __align__(16) float lds[];
   float* srow = (float*)__builtin_assume_aligned(lds, 16);   // (the declaration's alignment alone gives accesses of two single words)
@@ -1192,7 +1192,10 @@ __global__ __launch_bounds__(INV_T) void k_interp_rows_grad(int c, int n, int m,
     return (unsigned)__builtin_amdgcn_update_dpp(-1, (int)k, 0x130, 0xf, 0xf, false);
   };
   // a set's rows in registers, a piece of 4 T of each at a time: U pieces, then the rows' last elements
-  constexpr int PIECES = (ROW_POINTS / R + 4 * T - 1) / (4 * T), U = PIPE ? PIECES : R == 1 ? 5 : 2;   // (not PIPE: more would cost the second workgroup on a CU)
+  constexpr int PIECES = (ROW_POINTS / R + 4 * T - 1) / (4 * T), U = PIPE ? PIECES : R == 1 ? 5 : R == 2 ? 2 : 1;
+  // (not PIPE: two workgroups of 16 waves a CU, so 64 registers.  Two pieces of four rows took 66, and were one too many for the rows
+  // of up to 4095 that all are in one; 8 samples, 256 channels, 512 <- 3000 points 14.8 -> 11.7 us, 1024 <- 5000 20.3 -> 17.5; 16 samples,
+  // 256 <- 1024 17.4 -> 12.7)
   f4 v[U][R];
   float vt[R];
   // piece `at` of set q into v[u]; where there is none, or with n < 4, anything that can be read

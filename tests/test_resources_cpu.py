@@ -1,0 +1,61 @@
+"""What the built kernels take of a CU, read from the library's own code objects: kernels that are laid out for a number of workgroups
+a CU have to keep within the registers that leaves them, and a compiler that spills to do so undoes what it was for."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+msgpack = pytest.importorskip("msgpack")
+
+
+def _notes(elf):
+    at, = struct.unpack_from("<Q", elf, 0x28)
+    size, count = struct.unpack_from("<HH", elf, 0x3A)
+    for s in range(count):
+        kind, = struct.unpack_from("<I", elf, at + s * size + 4)
+        if kind != 7:
+            continue
+        p, length = struct.unpack_from("<QQ", elf, at + s * size + 0x18)
+        end = p + length
+        while p < end:
+            name, desc, note = struct.unpack_from("<III", elf, p)
+            p += 12 + (name + 3 & ~3)
+            if note == 32:
+                yield msgpack.unpackb(elf[p:p + desc], strict_map_key=False)
+            p += desc + 3 & ~3
+
+
+@pytest.fixture(scope="module")
+def kernels():
+    """{name with template arguments: (registers, bytes of scratch a lane)}"""
+    from dest3d_amd import _lib as L
+    if not os.path.exists(L.LIB_PATH):
+        from dest3d_amd.build import build
+        build(verbose=False)
+    lib, magic, found = open(L.LIB_PATH, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    for m in re.finditer(magic, lib):
+        o = m.start() + len(magic)
+        entries, = struct.unpack_from("<Q", lib, o)
+        o += 8
+        for _ in range(entries if entries < 8 else 0):
+            at, size, n = struct.unpack_from("<QQQ", lib, o)
+            target, o = lib[o + 24:o + 24 + n], o + 24 + n
+            if b"gfx950" in target and lib[m.start() + at:m.start() + at + 4] == b"\x7fELF":
+                for note in _notes(lib[m.start() + at:m.start() + at + size]):
+                    for k in note["amdhsa.kernels"]:
+                        found[k[".name"]] = (k[".vgpr_count"], k[".private_segment_fixed_size"])
+    plain = subprocess.run(["c++filt"], input="\n".join(found), capture_output=True, text=True, check=True).stdout.split("\n")
+    return {re.sub(r"^void |issm::|\(.*", "", p): found[n] for n, p in zip(found, plain)}
+
+
+@pytest.mark.parametrize("name,variants,registers", [
+    # rows' gradient, one set a workgroup of 16 waves: two workgroups a CU
+    (r"k_interp_rows_grad<[124], (true|false), false>", 4, 64),
+])
+def test_registers_leave_room_for_the_workgroups(kernels, name, variants, registers):
+    hit = {k: v for k, v in kernels.items() if re.fullmatch(name, k)}
+    assert len(hit) == variants
+    for k, (r, scratch) in hit.items():
+        assert r <= registers and scratch == 0, (k, r, scratch)
