@@ -244,6 +244,31 @@ def test_tile_and_level_form_of_the_chunk_backward_agree_to_fp32(L_, N, P, gated
             assert l2 <= 7e-7
 
 
+@pytest.mark.parametrize("H,G,P,tile", [(2, 2, 64, False), (1, 1, 52, False), (4, 2, 64, True), (2, 2, 48, True)])
+def test_one_wide_fp32_head_a_group_takes_the_level_form(H, G, P, tile):
+    """The tile-base kernel writes the list of heads to redo, the level form alone does not.  One head of more than 48 a group and one
+    direction: the level form; both against the oracle."""
+    _say(f"one wide fp32 head a group H={H} G={G} P={P}")
+    d = _problem(2, 128, H, P, 64, G, seed=H + P)
+    L, prob, a = _stage_args(d)
+    lib, nc, B, L_, N = L.load(), 2, 2, 128, 64
+    f = lambda *s: torch.zeros(s, device="cuda")
+    dy = d["dy"].cuda()
+    a.dout[0] = L.tensor_desc(dy)
+    t = [f(B, L_, H, N), f(B, L_, G, N), f(B, L_, G, N), f(B * nc, H, N), f(B * nc, H, N)]
+    a.ddt, a.dB[0], a.dC[0] = (L.tensor_desc(q) for q in t[:3])
+    redo = torch.full((lib.issm_bwd_chunk_redo_ints(C.byref(a)),), -1, dtype=torch.int32, device="cuda")
+    states, dst, dm = f(B, nc + 1, H, P, N), f(B, nc, H, P, N), f(B, nc, H, 64, 64)
+    L.check(lib.issm_stage_bwd_chunk(C.byref(a), 0, None, states.data_ptr(), dst.data_ptr(), dm.data_ptr(), None, t[3].data_ptr(),
+                                     t[4].data_ptr(), redo.data_ptr()), "bwd_chunk")
+    torch.cuda.synchronize()
+    assert bool((redo == (0 if tile else -1)).all())
+    _, _, ref = _oracle(d, GRAD_NAMES)
+    _, _, g, _ = _run_operator(d, torch.float32)
+    for k, v in ref.items():
+        _check("d" + k, g[k], v, BWD32)
+
+
 @pytest.mark.parametrize("P", [128, 96, 67])
 def test_head_dimension_above_the_tile_limit(P):
     """Heads wider than the kernels' 64 run as several narrower heads that share dt, A, dt_bias and the group's B, C
@@ -954,7 +979,7 @@ def test_tiles_that_decay_as_far_as_the_tile_base_form_reaches(dtype, L_, N, P, 
 @pytest.mark.parametrize("far", [False, True], ids=["", "a head out of range"])
 @pytest.mark.parametrize("L_,N,P,H,G,gated", [(128, 64, 36, 2, 1, False), (192, 128, 48, 4, 2, False), (128, 64, 52, 3, 1, False),
                                               (128, 64, 64, 5, 1, False), (100, 70, 64, 2, 1, False), (67, 5, 40, 2, 1, False),
-                                              (128, 64, 64, 2, 2, True)])
+                                              (128, 64, 64, 2, 2, True), (128, 64, 64, 4, 2, True)])
 def test_chunk_backward_of_wide_fp32_heads(L_, N, P, H, G, gated, far):
     """Heads of three and four tiles, fp32: x with dS and dy with H take turns in one place of the workgroup's memory, also where a
     head in between is left to the level form.  Operands hold 16 bits or more (1.5e-5, less in the mean; four times that and the
