@@ -115,6 +115,7 @@ CASES = [
     # leave a last batch of five steps with one row per thread, of three with two rows per thread
     (1, 64 * 35, 1, 32, 32, 1, dict(softplus=False)),
     (1, 64 * 35 - 9, 1, 40, 32, 1, dict(D="h")),
+    (1, 1186, 2, 36, 70, 1, dict()),                     # the same with columns that are no multiple of four
 ]
 
 
@@ -886,6 +887,13 @@ def test_stage_entry_points_match_oracle_intermediates(shape):
     (1, 192, 2, 20, 512, 1, 2, True, True),      # eight slices, a head tile partly filled
     (2, 256, 2, 36, 128, 1, 2, False, True),
     (2, 256, 2, 36, 128, 1, 2, True, True),
+    # the recurrence with chunks in four and eight slots, several rounds and a rest, columns in fours and not, and fewer than four columns
+    (1, 573, 2, 36, 70, 1, 2, False, True),      # four slots (nine chunks), threads of a row that overlap
+    (1, 1186, 2, 20, 70, 1, 2, False, True),     # eight slots (19 chunks)
+    (1, 1216, 2, 20, 67, 1, 1, True, True),
+    (1, 1100, 2, 16, 64, 1, 1, False, False),    # eight slots, whole columns
+    (1, 640, 2, 8, 3, 1, 2, False, True),
+    (2, 1100, 2, 12, 2, 1, 2, True, False),
 ])
 def test_states_of_the_backward_in_one_kernel(Bsz, L_, H, P, N, G, nd, bf, dfinal):
     """issm_stage_bwd_states against the two stages it stands for: the same products in the same order, sums of the recurrence and
@@ -994,6 +1002,25 @@ def test_chunk_backward_of_wide_fp32_heads(L_, N, P, H, G, gated, far):
     _check("final", fg, fin, 1e-3 if far else 1e-4)
     for k, v in ref.items():
         _check("d" + k, g[k], v, (5e-2 if k == "A" else 1e-2) if far else 1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,P", [(128, 64, 32), (100, 70, 32)])
+@pytest.mark.parametrize("spans", [(95, 95, 95, 95), (10, 10, 95, 95), (95, 0.1, 0.1, 95)], ids=str)
+def test_small_gradients_beside_tiles_that_decay_far(dtype, L_, N, P, spans):
+    """Upstream gradients of 2^-27: what crosses the middle of a chunk is held at up to 2^-96 of its size on its way, 2^-123, where 2^-149
+    is a unit: 2^-26 of the largest entry, below the operands' 16 bits.  So the bounds are those of gradients of size one."""
+    _say(f"small gradients, tiles of 2^-{spans} L={L_} N={N} P={P} {dtype}")
+    d = _problem(2, L_, 2, P, N, 1, seed=19, softplus=False)
+    d["A"] = -torch.linspace(0.5, 1.0, N).repeat(2, 1)
+    rows = torch.tensor(spans, dtype=torch.float32).repeat_interleave(16).repeat(L_ // 64 + 1)[:L_] / (16 * 1.4427)
+    d["dt"] = rows[None, :, None, None].expand(2, L_, 2, N).contiguous()
+    for k in ("x", "dt", "B", "C", "dy"):
+        d[k] = d[k].to(dtype).float()
+    _, _, ref = _oracle(d, GRAD_NAMES)
+    _, _, g, _ = _run_operator(dict(d, dy=d["dy"] * 2.0 ** -27, dfinal=d["dfinal"] * 2.0 ** -27), dtype)
+    for k, v in ref.items():
+        _check("d" + k, g[k].float() * 2.0 ** 27, v, 4e-4 if dtype == torch.float32 else (5e-2 if k == "A" else 2e-2))
 
 
 def test_inplace_edit_between_forward_and_backward_raises():
