@@ -67,8 +67,8 @@ struct BwdTileSmem {
   // bf16 inputs: the group's B and C values of every lane, packed in pairs, [i][tid] (i < 8: B, then C).
   // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
   // streams have been through it in between) and were a third of the kernel's reads; of three and four head tiles, 8 x 1024 tokens,
-  // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 250 states, three 98 and 107:
-  // 93 and 103).
+  // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 1000
+  // tokens, 250 states, by the kernel trace, three 95 and 102: 85 and 92, four 107 and 118: 99 and 106).
   static constexpr bool BCL = !SPLIT;
   unsigned bc[BCL ? 16 * NTHREADS : 0];
   // fp32 inputs of up to three head tiles: the B values, [k][tid]; C has no room (8 x 1024 tokens, 8 heads x 32, 256 states, both
@@ -174,8 +174,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
   // Everything a head reads from global memory is requested one head ahead, at the point of the previous head where
   // few registers are live (after its matrix products), so that the requests are in flight while that head's suffix
-  // sums and stores run.  (B and C of the lane's rows are the same for every head of the group; they are fetched again
-  // per head -- from the cache -- rather than held in 32 registers across the loop.)
+  // sums and stores run.  (B and C of the lane's rows are the same for every head of the group.  They come out of the workgroup's LDS
+  // copy; what has no room there -- C of fp32 inputs, B too for heads of four tiles -- is fetched again per head, from the cache,
+  // rather than held in 16 or 32 registers across the loop.)
   // What one head reads: the thread's share of the tiles the four waves stage in LDS (T: rows tid >> 3 and
   // 32 + (tid >> 3), columns 8 (tid & 7) .. + 7 of the hi -- and lo -- matrix; x, dy: group i of the thread is row
   // e4 / 4PT, columns 4 (e4 % 4PT) .. + 3 with e4 = tid + 256 i) and the lane's column operands.  Requested in the order
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     float dtp[16], dfac[16], pc[16], tt[4];
     lane_dt<true>(p, cf, vn, g4, rm, l_raw, dtp, dfac);
     float half0, half1;
-    lane_half_sums<IOB>(An * LOG2E, cm, g4, rm, dtp, pc, tt, half0, half1);
+    lane_half_sums<IOB>(An * LOG2E, cm, g4, dtp, pc, tt, half0, half1);
     {
       const float worst = fmaxf(fmaxf(fabsf(tt[0]), fabsf(tt[1])), fmaxf(fabsf(tt[2]), fabsf(tt[3])));
       const bool bad = !(worst <= SPAN_LIMIT);  // also true for NaN
@@ -439,12 +440,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
           bvp[i] = s.bc[i * NTHREADS + tid];
           cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
         }
-      } else if constexpr (!SPLIT) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          bvp[i] = pack_bf16(l_Bv[2 * i], l_Bv[2 * i + 1]);
-          cvp[i] = pack_bf16(l_Cv[2 * i], l_Cv[2 * i + 1]);
-        }
       } else {
 #pragma unroll
         for (int k = 0; k < (BL ? 0 : 16); ++k) bvf[k] = l_Bv[k];
@@ -514,12 +509,11 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
         f4 df = {0, 0, 0, 0}, dg = {0, 0, 0, 0};  // DIAG32: those of the diagonal block
         float cd[4], bd[4];                       // DIAG32: the operands of rows 16 R + 4 g4 + j
         if constexpr (DIAG32) {
-          if constexpr (BCL)
 #pragma unroll
-            for (int i = 2 * R; i < 2 * R + 2; ++i) {
-              bvp[i] = s.bc[i * NTHREADS + tid];
-              cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
-            }
+          for (int i = 2 * R; i < 2 * R + 2; ++i) {
+            bvp[i] = s.bc[i * NTHREADS + tid];
+            cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
+          }
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int k = 4 * R + j;

@@ -832,34 +832,20 @@ __device__ __forceinline__ float lane_prep(const KP& p, const Coef& cf, bool vn,
 // (these the same on the four lanes of a column).  Used by the kernel that writes a decay exp2(cs[l] - cs[s]) as
 // exp2(pc[l]) . exp2(-pc[s]) for rows of one half and with exp2(half0 + half1) between the two for rows of both: two exponentials
 // per element and two per column serve every pair of rows of the chunk.
-// LDS: the cross-lane steps through LDS (see group_sums).
+// LDS: the cross-lane steps through LDS (see group_sums).  (No packed sequences: that kernel does not take them.)
 template <bool LDS>
-__device__ __forceinline__ void lane_half_sums(float A2, int cm, int g4, const RowMap& rm, const float (&dtp)[16],
-                                               float (&pc)[16], float (&tt)[4], float& half0, float& half1) {
+__device__ __forceinline__ void lane_half_sums(float A2, int cm, int g4, const float (&dtp)[16], float (&pc)[16], float (&tt)[4],
+                                               float& half0, float& half1) {
   float c[4];
-  if (rm.full || rm.cut == 0) {
 #pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      float a = 0.0f;
+  for (int J = 0; J < 4; ++J) {
+    float a = 0.0f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        a += dtp[4 * J + j] * A2;
-        pc[4 * J + j] = a;
-      }
-      c[J] = a;
+    for (int j = 0; j < 4; ++j) {
+      a += dtp[4 * J + j] * A2;
+      pc[4 * J + j] = a;
     }
-  } else {  // packed sequences: the sum drops by SEQ_CUT at every row where the sequence id changes
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      const unsigned bits = (unsigned)(rm.cut >> (16 * J + 4 * g4)) & 15u;
-      float a = 0.0f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        a += dtp[4 * J + j] * A2 - (((bits >> j) & 1u) ? SEQ_CUT : 0.0f);
-        pc[4 * J + j] = a;
-      }
-      c[J] = a;
-    }
+    c[J] = a;
   }
   float add[4];
   if constexpr (LDS) {

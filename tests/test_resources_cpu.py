@@ -53,6 +53,9 @@ def kernels():
 @pytest.mark.parametrize("name,variants,registers", [
     # rows' gradient, one set a workgroup of 16 waves: two workgroups a CU
     (r"k_interp_rows_grad<[124], (true|false), false>", 4, 64),
+    # chunk backward in tile-base form, incomplete tiles: two of four waves
+    (r"k_bwd_tile<[234], true, false, (true|false), (true|false), false, (true|false)>", 24, 256),
+    (r"k_bwd_tile<[234], false, false, (true|false), false, false, (true|false)>", 12, 256),
 ])
 def test_registers_leave_room_for_the_workgroups(kernels, name, variants, registers):
     hit = {k: v for k, v in kernels.items() if re.fullmatch(name, k)}
