@@ -221,7 +221,7 @@ class Runner:
         return {"p10": pick(0.10), "p50": pick(0.50), "p90": pick(0.90)}
 
     def stage_times(self, reps=20):
-        """Average duration of each kernel, HIP events on the launch stream around `reps`
+        """Average duration of each kernel of the step, HIP events on the launch stream around `reps`
         back-to-back launches of that kernel."""
         torch, lib, a = self.torch, self.lib, self.a
         nd = self.ndir
@@ -238,8 +238,10 @@ class Runner:
             ("chunk_local", lambda: lib.issm_stage_chunk_local(C.byref(a), p(st), p(csl), p(cabt))),
             ("state_passing_fwd", lambda: lib.issm_stage_state_passing_fwd(C.byref(a), p(st), p(csl))),
             ("chunk_scan", lambda: lib.issm_stage_chunk_scan(C.byref(a), p(st), p(cabt), None)),
-            ("bwd_dstates", lambda: lib.issm_stage_bwd_dstates(C.byref(a), None, p(dst), p(dm))),
-            ("state_passing_bwd", lambda: lib.issm_stage_state_passing_bwd(C.byref(a), None, p(csl), p(dst), None, p(dh0d))),
+            *([("bwd_states", lambda: lib.issm_stage_bwd_states(C.byref(a), None, None, p(dst), p(dm), None, p(dh0d)))]
+              if lib.issm_bwd_walks(C.byref(a)) else
+              [("bwd_dstates", lambda: lib.issm_stage_bwd_dstates(C.byref(a), None, p(dst), p(dm))),
+               ("state_passing_bwd", lambda: lib.issm_stage_state_passing_bwd(C.byref(a), None, p(csl), p(dst), None, p(dh0d)))]),
             ("bwd_chunk", lambda: [lib.issm_stage_bwd_chunk(C.byref(a), d, None, p(st), p(dst), p(dm), None, p(pa), p(pb), p(redo))
                                    for d in range(nd)][-1]),
             ("bwd_dx", lambda: lib.issm_stage_bwd_dx(C.byref(a), None, p(dst), p(cabt), p(pd))),
@@ -269,9 +271,10 @@ class Runner:
         return res
 
 
-KERNEL_OF_STAGE = {"chunk_local": "k_local_tile", "state_passing_fwd": "k_state_pass", "chunk_scan": "k_chunk_scan",
-                   "bwd_dstates": "k_bwd_dstates", "state_passing_bwd": "k_state_pass", "bwd_chunk": "k_bwd_tile",
-                   "bwd_dx": "k_bwd_dx", "bwd_reduce": "k_bwd_reduce"}
+# (k_state_pass: its last template argument tells the two recurrences apart)
+KERNEL_OF_STAGE = {"chunk_local": r"k_local_tile\b", "state_passing_fwd": r"k_state_pass<\d+, \w+, false>", "chunk_scan": r"k_chunk_scan\b",
+                   "bwd_states": r"k_bwd_walk\b", "bwd_dstates": r"k_bwd_dstates\b", "state_passing_bwd": r"k_state_pass<\d+, \w+, true>",
+                   "bwd_chunk": r"k_bwd_tile\b", "bwd_dx": r"k_bwd_dx\b", "bwd_reduce": r"k_bwd_reduce\b"}
 
 
 def measured_traffic(stage):
@@ -282,7 +285,7 @@ def measured_traffic(stage):
     has no such row."""
     import re
     path = os.path.join(ROOT, "profiles", "issm_fwd_bwd_bidir_fp32_hbm_traffic.md")
-    pat = re.compile(KERNEL_OF_STAGE.get(stage, stage) + r"\b")
+    pat = re.compile(KERNEL_OF_STAGE.get(stage, stage))
     total = None
     try:
         for row in open(path):
@@ -313,7 +316,9 @@ def stage_work(ndir, shape=None, elt=4):
         "chunk_local": (2 * U * (cs * P * N + tri * N), s * (E_dt + E_x + 2 * E_bc) + 4 * (E_cs + E_m + E_v)),
         # reads dt, C, x, states H, M; writes y
         "chunk_scan": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m)),
-        # reads dt, C, dy, x; writes dH, dM
+        # reads dt, C, dy, x, the final states' gradients; writes dS, dM, the initial states' gradients
+        "bwd_states": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m + 2 * E_st)),
+        # the same in two launches: reads dt, C, dy, x; writes dH, dM; and the recurrence
         "bwd_dstates": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m)),
         # all launches: read dt, x, dy, B, C, H, dS, dM; write ddt, dB, dC, the dA / ddt_bias partials
         "bwd_chunk": (2 * U * (2 * cs * P * N + 2 * tri * N),
@@ -329,7 +334,7 @@ def stage_work(ndir, shape=None, elt=4):
     fwd_rd = s * (E_x + 2 * E_bc + E_dtd + E_st)
     fwd = fwd_rd + s * E_x + 4 * E_st
     bwd = fwd_rd + s * E_x + 4 * E_st + s * (E_x + 2 * E_bc + E_dtd + E_st)
-    w["step"] = (sum(f for f, _ in w.values()), fwd + bwd)
+    w["step"] = (sum(f for k, (f, _) in w.items() if k != "bwd_states"), fwd + bwd)   # (bwd_dstates has its FLOPs)
     return w
 
 
@@ -354,7 +359,7 @@ def workload_report(run, step_us, reps=20):
     work = stage_work(run.ndir, run.shape, run.elt)
     per_stage = {}
     for k, (fl, nb) in work.items():
-        if k == "step":
+        if k not in stages:
             continue
         b, _, fr, both = stage_bound(fl, nb, stages[k], run.elt)
         per_stage[k] = {"us": round(stages[k], 2), "bound": b, "frac": round(fr, 4), **both}
