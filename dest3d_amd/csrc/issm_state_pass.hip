@@ -7,9 +7,9 @@
 // through all chunks, and a wave's accesses are whole rows (1 KB at 256 columns).  (The backward pass once also read the forward's
 // states, half as much again, for the column sums g = sum_p dS_c H_(c+1) that d/d(cs) needs, in slices of 32 or 64 columns by all
 // rows with the rows' sums through LDS.  The chunk backward now takes g from what it has in registers, see k_bwd_tile.
-// 2 x 16384 tokens, 8 heads x 32, 256
-// states: 109 -> 47 us, 5.8 TB/s; 8 x 1024, both directions: 32 -> 26; 16 x 2048, 16 heads x 64, 512 states, both directions: 0.93
-// ms forward, 4.6 TB/s.)
+// Launched over and over on the same buffers, backward, 2 x 16384 tokens, 8 heads x 32, 256 states: 109 -> 47 us, 5.8 TB/s (inside a
+// training step, where the buffers come from HBM, 67, 4 TB/s); 8 x 1024, both directions: 32 -> 26; forward, inside a step, 16 x 2048, 16 heads
+// x 64, 512 states, both directions: 0.93 ms, 4.6 TB/s.)
 #include "issm_dev.h"
 
 namespace issm {

@@ -106,13 +106,12 @@ CASES = [
     (1, 128, 2, 36, 64, 1, dict(D="hp", z=True)),        # complete chunks / slices, ragged head dimension
     (2, 64, 2, 20, 128, 2, dict(softplus=False)),
     (1, 192, 1, 64, 64, 1, dict()),                       # complete tiles, widest head dimension
-    # state passing: 32-column slices with stand-in rows, 37 chunks (six register slots, a last batch of one step)
+    # many chunks of one or two heads: the recurrences walk 37 of them eight ahead, a last batch of five
     (1, 64 * 37, 2, 20, 64, 1, dict()),
-    (1, 64 * 7 - 5, 1, 40, 96, 1, dict(D="hp")),          # two rows per thread, four slots, ragged last chunk
-    (4, 64 * 5, 8, 36, 256, 1, dict(softplus=False)),    # 64-column slices, three slots, 5 chunks, P = 36
+    (1, 64 * 7 - 5, 1, 40, 96, 1, dict(D="hp")),          # four ahead, ragged last chunk
+    (4, 64 * 5, 8, 36, 256, 1, dict(softplus=False)),    # 128 walks of 5 chunks, P = 36
     (16, 70, 8, 16, 96, 1, dict()),                      # many workgroups, N a multiple of 32 but not of 64
-    # state passing, few workgroups and many chunks (column sums of several steps added up together): 35 chunks
-    # leave a last batch of five steps with one row per thread, of three with two rows per thread
+    # the same with half a slice of states, 35 chunks, a last batch of three
     (1, 64 * 35, 1, 32, 32, 1, dict(softplus=False)),
     (1, 64 * 35 - 9, 1, 40, 32, 1, dict(D="h")),
     (1, 1186, 2, 36, 70, 1, dict()),                     # the same with columns that are no multiple of four
@@ -805,8 +804,7 @@ def _stage_args(d, ndir=1):
 
 @pytest.mark.parametrize("shape", [
     (2, 150, 4, 32, 96, 2),
-    # head dimensions that leave threads of the state-passing kernels without a row of their own (stand-ins that only
-    # load): 20 of 32 rows and 40 of 64 with 32-column slices, 36 of 48 with 64-column slices and many workgroups
+    # head dimensions that fill no tile: 20 of 32 rows, 40 and 36 of 48, in one, two and eight column slices
     (1, 150, 2, 20, 64, 1), (1, 150, 2, 40, 96, 1), (4, 130, 8, 36, 512, 1),
     # complete 64 x 64 tiles only: the kernels written for them (row-lane chunk_local, tile-base bwd_chunk)
     (2, 192, 4, 32, 128, 2), (1, 128, 2, 36, 64, 1), (1, 128, 2, 64, 192, 1),
@@ -887,7 +885,7 @@ def test_stage_entry_points_match_oracle_intermediates(shape):
     (1, 192, 2, 20, 512, 1, 2, True, True),      # eight slices, a head tile partly filled
     (2, 256, 2, 36, 128, 1, 2, False, True),
     (2, 256, 2, 36, 128, 1, 2, True, True),
-    # the recurrence with chunks in four and eight slots, several rounds and a rest, columns in fours and not, and fewer than four columns
+    # the recurrence with chunks in four and eight slots, several batches and a rest, columns in fours and not, and fewer than four columns
     (1, 573, 2, 36, 70, 1, 2, False, True),      # four slots (nine chunks), threads of a row that overlap
     (1, 1186, 2, 20, 70, 1, 2, False, True),     # eight slots (19 chunks)
     (1, 1216, 2, 20, 67, 1, 1, True, True),
@@ -941,7 +939,8 @@ def test_states_of_the_backward_in_one_kernel(Bsz, L_, H, P, N, G, nd, bf, dfina
 @pytest.mark.parametrize("L_,H,P,N,G,scale", [
     (256, 2, 32, 64, 1, 1.0),     # tile-base form, complete tiles
     (200, 2, 36, 70, 1, 1.0),     # incomplete tiles, rows past the head dimension
-    (128, 2, 64, 64, 1, 1.0),     # level form
+    (128, 2, 64, 64, 1, 1.0),     # four head tiles: fp32 products
+    (128, 2, 64, 64, 2, 1.0),     # level form, complete tiles (one wide head a group)
     (130, 2, 6, 20, 2, 1.0),      # level form, a head that is no multiple of four wide
     (130, 2, 8, 3, 1, 1.0),       # fewer than four states
     (256, 2, 32, 64, 1, 100.0),   # tiles out of the tile-base form's range
