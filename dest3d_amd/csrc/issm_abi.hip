@@ -15,6 +15,7 @@
 namespace issm {
 int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, bool any, hipStream_t st);
 bool bwd_tile_available(const KP& p, const float* dy_ws);
+bool bwd_tile_dual(const KP& p, const float* dy_ws, int parts);
 int launch_state_fwd(const KP& p, float* states, const float* cs_last, hipStream_t st);
 int launch_chunk_scan(const KP& p, const float* states, const float* cabt, float* out_x, hipStream_t st);
 int launch_bwd_gate(const KP& p, const float* out_x, float* dy_ws, hipStream_t st);
@@ -22,7 +23,7 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
 int launch_state_bwd(const KP& p, const float* cs_last, float* dstates, float* dh0_dir, hipStream_t st);
 int launch_state_sums(const KP& p, const float* states, const float* dstates, float* g_last, hipStream_t st);
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st);
+                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, bool dual, hipStream_t st);
 int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st);
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
                           const float* dm, float* partA, float* partBias, const int* redo,
@@ -430,7 +431,7 @@ int issm_stage_bwd_chunk(const issm_scan_args* a, int dir, const float* dy_gated
   KP p = make_kp(a);
   p.dir0 = dir;
   int pending = 0;
-  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1,
+  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1, false,
                                       (hipStream_t)a->stream),
                      "bwd_chunk")))
     return rc;
@@ -500,23 +501,24 @@ int issm_scan_bwd(const issm_scan_args* a) {
   int* redo = reinterpret_cast<int*>(ws + bw.redo);
   int pending = 0;
   KP pc = p;
-  if (wants_ddt_part(a) && bwd_tile_available(p, dy)) {
+  int parts = 1;
+  if (bwd_tile_available(p, dy)) {
+    parts = bwd_head_parts(a->dims);
+    if (parts > 1 || (p.io_dt && !p.full_tiles)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
+  }
+  const bool dual = bwd_tile_dual(p, dy, parts);
+  if (wants_ddt_part(a) && !dual && bwd_tile_available(p, dy)) {
     // both directions go through the tile-base kernel: the first one's share of the bf16 ddt travels in fp32
     pc.ddt_part.ptr = ws + bw.ddt_part;
     pc.ddt_part.s2 = p.N;
     pc.ddt_part.s1 = (long)p.H * p.N;
     pc.ddt_part.s0 = (long)p.L * p.H * p.N;
   }
-  int parts = 1;
-  if (bwd_tile_available(p, dy)) {
-    parts = bwd_head_parts(a->dims);
-    if (parts > 1 || (p.io_dt && !p.full_tiles)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
-  }
-  for (int dir = 0; dir < p.ndir; ++dir) {
+  for (int dir = 0; dir < (dual ? 1 : p.ndir); ++dir) {
     KP pd = pc;
     pd.dir0 = dir;
     if ((rc = launched(launch_bwd_chunk(pd, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm,
-                                        ws + bw.partA, ws + bw.partBias, redo, &pending, parts, st),
+                                        ws + bw.partA, ws + bw.partBias, redo, &pending, parts, dual, st),
                        "bwd_chunk")))
       return rc;
   }

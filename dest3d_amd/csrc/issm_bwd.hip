@@ -1563,20 +1563,21 @@ static int launch_bwd_chunk_t(const KP& p, int blocks, const float* dy_ws, const
 
 bool bwd_tile_available(const KP& p, const float* dy_ws);
 int launch_bwd_tile(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                    float* partA, float* partBias, int* redo, int parts, hipStream_t st);
+                    float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st);
 
 // Chunk backward of direction p.dir0.  With a `redo` buffer (issm_bwd_chunk_redo_ints words) the tile-base kernel
 // (issm_bwd_tile.hip) does the work and marks the heads outside its range; launch_bwd_chunk_redo then evaluates those
 // with the level-hierarchy kernel.  Without one, or for calls the tile-base kernel is not built for (bwd_tile_available:
 // packed sequences, a gate beside bf16 inputs, mixed input types, no ddt, one fp32 head of more than 48 a group and direction, heads or
 // rows of x and dout that are no multiple of four elements), the level-hierarchy kernel evaluates everything and *redo_pending stays 0.
-// parts: workgroups of the tile-base kernel that share a group's heads (1 without p.dbc_part).
+// parts: workgroups of the tile-base kernel that share a group's heads (1 without p.dbc_part).  dual: that kernel takes both directions
+// in this launch (bwd_tile_dual).
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, hipStream_t st) {
+                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, bool dual, hipStream_t st) {
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
   if (redo && bwd_tile_available(p, dy_ws)) {
     if (redo_pending) *redo_pending = 1;
-    return launch_bwd_tile(p, dy_ws, states, dstates, dm, partA, partBias, redo, parts, st);
+    return launch_bwd_tile(p, dy_ws, states, dstates, dm, partA, partBias, redo, parts, dual, st);
   }
   ISSM_DISPATCH(p, {
     if (int e = launch_bwd_chunk_t<PT_, IOB_, DTB_, FULL_>(p, blocks, dy_ws, states, dstates, dm, partA,

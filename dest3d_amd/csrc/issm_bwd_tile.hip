@@ -80,6 +80,13 @@ struct BwdTileSmem {
   int shared[4];             // per wave: some head was left to the level form
 };
 
+// Both directions in one workgroup: what a half hands to the other lies behind the two or, without room, in the place of x / dy.
+constexpr int DUAL_EX_BYTES = 8 * NTHREADS * sizeof(float);
+template <typename SM>
+constexpr bool dual_ex_in_tiles() { return 2 * (sizeof(SM) + DUAL_EX_BYTES) > 160 * 1024; }
+template <typename SM>
+constexpr size_t dual_lds() { return 2 * sizeof(SM) + (dual_ex_in_tiles<SM>() ? 0 : 2 * DUAL_EX_BYTES); }
+
 // An fp32 value rounded to 17 significand bits; a NaN may come out as zero.  (Where it stands below the conversion alone gives
 // the same number but for ties; without it the kernel spills 200 bytes a lane instead of 20.)
 __device__ __forceinline__ float round17(float v) { return __uint_as_float((__float_as_uint(v) + 0x40u) & 0xffffff80u); }
@@ -102,11 +109,16 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
+// DUAL: both directions in one launch, four waves each of a workgroup of eight, on the same tokens, head by head: dt comes from memory
+// once and their ddt is added up through LDS instead of being stored, read back and stored again (711 -> 510 MB at 8 x 1024 tokens, 8
+// heads x 32, 256 states, fp32).  What it gives is less than that, for eight waves now meet where four did: the two launches 88 + 96 us,
+// this one 172; heads of 36, bf16, 71 + 75 and 134.  (The second direction a barrier or two behind the first, so that they use LDS and
+// the vector ALU at different times: 169, for a barrier then waits for the longer of two different phases.)
 // FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).  PARTS: gridDim.y workgroups
 // share the group's heads, heads_each each (a variant of its own: the two loop bounds more cost the others 25 - 50 scalar
 // registers spilled and 1 - 2 % of a training step).
-template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
+template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS, bool DUAL>
+__global__ __launch_bounds__(DUAL ? 2 * NTHREADS : NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
                                                           const float* __restrict__ dstates,
                                                           const float* __restrict__ dm, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
@@ -117,28 +129,35 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
   constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && (!FULL || PT >= 4);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdTileSmem<PT, SPLIT> SM;
-  SM& s = *reinterpret_cast<SM*>(smem_raw);
+  const int half = DUAL ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS) : 0;
+  SM& s = *reinterpret_cast<SM*>(smem_raw + half * sizeof(SM));
   constexpr int LDP = SM::LDP, LDM = SM::LDM, KT = (PT + 1) / 2;
-  constexpr bool BCL = SM::BCL, BL = SM::BL;
+  constexpr bool BCL = SM::BCL, BL = SM::BL, EX_IN_TILES = dual_ex_in_tiles<SM>();
+  static_assert(!EX_IN_TILES || sizeof(s.xs) >= DUAL_EX_BYTES, "it fits");
   // fp32 inputs take turns: x and dS make Q, then dy and H, which are requested at the head's start and not a head
   // ahead, make R in the same place: two barriers a head more.  With all four at once the prefetch spills 76 bytes a lane at three
   // head tiles, each reload waiting for every request before it, and at four the tiles leave one workgroup a CU.  8 x 1024 tokens, 8
   // heads, 256 states, both directions, per direction: heads of 48 128 and 137 -> 104 and 112 us; of 64, which took the level form, 135
   // -> 114 and 121; of 32 the same as before, but it makes room for B (SM::BL).
   constexpr int KP_ = PT * 4;  // dS / H values per lane
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = DUAL ? threadIdx.x % NTHREADS : threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
   const int nsl = (p.N + NS - 1) / NS;
   Unit u;
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  int wg = xcd_remap(blockIdx.x, gridDim.x);
   int id = wg;
   const int ns = id % nsl;
   id /= nsl;
   u.g = id % p.G;
   id /= p.G;
-  u.c = p.c_lo + id % p.ncl;
+  u.dir = DUAL ? half : p.dir0;
+  u.c = id % p.ncl;
   u.b = id / p.ncl;
-  u.dir = p.dir0;
+  if (DUAL && half) {   // the same tokens: the mirrored chunk, marked where a launch of this direction alone would
+    u.c = p.ncl - 1 - u.c;
+    wg = ((u.b * p.ncl + u.c) * p.G + u.g) * nsl + ns;
+  }
+  u.c += p.c_lo;
   u.bt = u.b * p.ndir + u.dir;
   u.h = u.g * p.hpg;
   const int n = ns * NS + wave * 16 + cm;
@@ -170,7 +189,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 
   // the reversed direction's launch follows the forward one's and shares dt, x, B, C and ddt with it: it walks the
   // heads backwards, so what the first launch touched last (and the last-level cache still holds) is read first
-  auto head_of = [&](int hh) { return u.g * p.hpg + (p.dir0 ? p.hpg - 1 - hh : hh); };
+  auto head_of = [&](int hh) { return u.g * p.hpg + (!DUAL && p.dir0 ? p.hpg - 1 - hh : hh); };
 
   // Everything a head reads from global memory is requested one head ahead, at the point of the previous head where
   // few registers are live (after its matrix products), so that the requests are in flight while that head's suffix
@@ -325,8 +344,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     }
     __syncthreads();
     const int4 bd = *(const int4*)s.bad;
-    const bool skip = (bd.x | bd.y | bd.z | bd.w) != 0;  // uniform: the whole head is left to the level-hierarchy kernel
-    if (tid == 0) redo[(p.dir0 * (int)gridDim.x + wg) * p.hpg + hh] = skip ? 1 : 0;
+    int any_bad = bd.x | bd.y | bd.z | bd.w;
+    if constexpr (DUAL) {
+      const int4 be = *(const int4*)reinterpret_cast<SM*>(smem_raw + (1 - half) * sizeof(SM))->bad;
+      any_bad |= be.x | be.y | be.z | be.w;
+    }
+    const bool skip = any_bad != 0;  // uniform: the whole head is left to the level-hierarchy kernel
+    if (tid == 0) redo[(u.dir * (int)gridDim.x + wg) * p.hpg + (DUAL && half ? p.hpg - 1 - hh : hh)] = skip ? 1 : 0;
     if (DIAG32 && skip) s.shared[wave] = 1;
     const uint16_t* xs_ = s.xs;
     const uint16_t* dys_ = s.dys();
@@ -627,7 +651,25 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
     }
     request(head_of(min(hh + 1, (PARTS ? min(p.hpg, hh0 + heads_each) : p.hpg) - 1)));  // (unconditional: the last head is requested again and not used)
     __builtin_amdgcn_sched_barrier(0);
+    // DUAL: the two halves of the workgroup have one column's rows in opposite order (row k of a lane of the one is row 15 - k of
+    // lane ^ 48 of the other); each hands its first eight over and stores the sums of its last eight.
+    auto store_late = [&](const float (&v)[16]) {
+      typedef typename std::conditional<IOB, uint16_t, float>::type T;
+      T* q = (T*)const_cast<void*>(p.ddt.ptr) + ((long)u.b * p.ddt.s0 + (long)u.h * p.ddt.s2);
+      const unsigned lo = (unsigned)(rm.base * (int)p.ddt.s1 + n) * (unsigned)sizeof(T);
+      unsigned ks = (unsigned)(rm.step * (int)p.ddt.s1) * (unsigned)sizeof(T);
+      ISSM_OPAQUE_S(ks);
+#pragma unroll
+      for (int k = 8; k < 16; ++k) {
+        T* d = (T*)((char*)q + (lo + (unsigned)(16 * (k >> 2) + (k & 3)) * ks));
+        if (IOB) *d = (T)f_to_bf16(v[k]); else *d = (T)v[k];
+      }
+    };
     if (skip) {
+      if constexpr (DUAL) {
+        store_late(val);
+        continue;
+      }
       // the level-hierarchy kernel adds this head's share to ddt later: it must find the other direction's, or zero
       if constexpr (!ACC) {  // (val is all zero here)
         if constexpr (P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
@@ -698,7 +740,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __r
 #pragma unroll
       for (int k = 0; k < 16; ++k) val[k] += old[k];
     }
-    if constexpr (!ACC && P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
+    if constexpr (DUAL) {
+      if constexpr (EX_IN_TILES) __syncthreads();
+      float* ex = reinterpret_cast<float*>(EX_IN_TILES ? (unsigned char*)s.xs : smem_raw + 2 * sizeof(SM) + half * DUAL_EX_BYTES);
+      const float* ey = reinterpret_cast<const float*>(EX_IN_TILES ? (const unsigned char*)reinterpret_cast<SM*>(smem_raw + (1 - half) * sizeof(SM))->xs
+                                                                       : smem_raw + 2 * sizeof(SM) + (1 - half) * DUAL_EX_BYTES);
+      int tq = tid;
+      asm volatile("" : "+v"(tq));
+#pragma unroll
+      for (int k = 0; k < 8; ++k) ex[k * NTHREADS + tq] = val[k];
+      __syncthreads();
+#pragma unroll
+      for (int k = 8; k < 16; ++k) val[k] += ey[(15 - k) * NTHREADS + (tq ^ 48)];
+      store_late(val);
+    } else if constexpr (!ACC && P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
     else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, val);
     sumA = scan_g_incl(sumA, g4);
     sumB = scan_g_incl(sumB, g4);
@@ -746,30 +801,45 @@ bool bwd_tile_available(const KP& p, const float* dy_ws) {
   return true;
 }
 
+// Whether one launch takes both directions (DUAL).  Complete tiles: only then do the two directions' chunks cover the same tokens.
+// bf16, or fp32 heads of 32: others of up to 31 and of 33 to 48 spill 48 - 92 bytes a lane (8 x 1024 tokens, 8 heads x 36, 256 states,
+// training step 526 us in two launches, 535 in one), and of more than 48 lose at five barriers a head what the traffic saves (16 x 2048
+// tokens, 16 heads x 64, 512 states: the kernel 3.60 and 3.59 ms).  From 321 workgroups on: a workgroup fills a CU, so up to 256 leave CUs
+// idle and a few more need another round (320 of them, fp32: 333 against 335 us; 384: 371 and 369; 576: 583 and 562).
+bool bwd_tile_dual(const KP& p, const float* dy_ws, int parts) {
+  const long blocks = (long)p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
+  return p.ndir == 2 && p.full_tiles && !dy_ws && parts == 1 && blocks > 320 && (p.io_dt || p.P == 32) && bwd_tile_available(p, dy_ws);
+}
+
 template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
-                             float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
-  const size_t sm = sizeof(BwdTileSmem<PT, !IOB>);
+                             float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st) {
   static_assert(sizeof(BwdTileSmem<PT, !IOB>) <= 80 * 1024, "two workgroups a CU");
   const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0;
-  auto go = [&](auto kern) -> int {
+  auto go = [&](auto kern, int dirs = 1) -> int {
+    typedef BwdTileSmem<PT, !IOB> SM;
+    const size_t sm = dirs == 1 ? sizeof(SM) : dual_lds<SM>();
     if (sm > 64 * 1024)
       if (int e = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm))
         return e;
-    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
+    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(dirs * NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
                        (p.hpg + parts - 1) / parts);
     return 0;
   };
+  if constexpr (IOB)
+    if (dual && !pnf) return go(&k_bwd_tile<PT, IOB, false, false, false, true, false, true>, 2);
+  if constexpr (IOB || PT == 2)
+    if (dual) return go(&k_bwd_tile<PT, IOB, true, false, false, true, false, true>, 2);
   auto pick = [&](auto p32) -> int {
     constexpr bool P32 = decltype(p32)::value;
     if (parts > 1) {
-      if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, true>);
-      return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, true>);
+      if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, true, false>);
+      return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, true, false>);
     }
-    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, false>);
-    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true, false>);
-    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, false>);
+    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, false, false>);
+    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true, false, false>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true, false, false>);
+    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, false, false>);
   };
   if constexpr (IOB)
     if (p.ddt_part.ptr) return pick(std::true_type{});
@@ -777,7 +847,7 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
 }
 
 int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                    float* partA, float* partBias, int* redo, int parts, hipStream_t st) {
+                    float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st) {
   KP p = p_;
   if (dy_ws) {  // a gated dy: fp32 (Bt, L, H, P) contiguous, batch * direction outermost
     TensorD& t = p.dout[p.dir0];
@@ -791,13 +861,13 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
   const int pt = (p.P + 15) / 16;
   int e = 0;
   if (p.io_dt) {
-    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
-    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
   } else {
-    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
-    else e = launch_bwd_tile_t<4, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    else e = launch_bwd_tile_t<4, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
   }
   if (e) return e;
   return (int)hipGetLastError();

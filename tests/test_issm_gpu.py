@@ -1530,3 +1530,41 @@ def test_dt_of_another_dtype_than_x(io_dtype, dt_dtype, L_):
     for k in ("x", "dt", "A", "B", "C", "D", "dt_bias", "h0"):
         # a bf16 ddt is rounded to 8 bits whatever the arithmetic behind it
         _check("d" + k, ins[k].grad, g_ref[k], BWD16 if (k == "dt" and dt_dtype == torch.bfloat16) else bt)
+
+
+@pytest.mark.parametrize("dtype,P,H,G,far", [("fp32", 32, 2, 1, False), ("fp32", 32, 4, 2, True), ("fp32", 32, 1, 1, False),
+                                             ("bf16", 32, 2, 1, True), ("bf16", 20, 2, 2, False), ("bf16", 36, 2, 1, False),
+                                             ("bf16", 48, 2, 1, True), ("bf16", 64, 2, 1, True), ("bf16", 52, 1, 1, False)])
+def test_both_directions_of_the_chunk_backward_in_one_launch(dtype, P, H, G, far):
+    """3 x 960 tokens, 512 states: 360 workgroups a direction, from 321 of which on one launch takes both.  Against two calls of one
+    direction each on the same tokens, whose sums differ in order, and in the kernel that the states take: fp32 a few 10^-7 of the
+    norm (5e-6 allowed); bf16 ddt is rounded once here and three times there, 2^-9 / sqrt(3) each (the two shares about as
+    large as their sum), 2.5e-3 allowed.  far: a head with tiles that decay out
+    of the form's range, whose ddt and dA are sums in which terms 200 times as large cancel (5e-5)."""
+    from dest3d_amd import ISSM_biscan_combined, ISSM_chunk_scan_combined
+    io = torch.float32 if dtype == "fp32" else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(5)
+    b, l, n = 3, 960, 512
+    rnd = lambda *s, sc=1.0, dt=io: (torch.randn(*s, generator=g, device="cuda") * sc).to(dt)
+    x, B, C, dy = ([rnd(b, l, *s, sc=sc) for _ in range(2)] for s, sc in (((H, P), 1), ((G, n), n ** -0.5), ((G, n), n ** -0.5), ((H, P), 1)))
+    dt = (torch.rand(b, l, H, n, generator=g, device="cuda") * 0.1 + 0.01).to(io)
+    A = -torch.exp(torch.rand(H, 1, generator=g, device="cuda") * math.log(16.0)).repeat(1, n)
+    if far:
+        A[H - 1, 70:80] = -200.0   # about 16 * 0.06 * 200 / ln 2 = 277 a tile
+    D, h0, df = rnd(H, dt=torch.float32), rnd(b, H, P, n, dt=torch.float32), [rnd(b, H, P, n, dt=torch.float32) for _ in range(2)]
+    leaf = lambda t: t.detach().clone().requires_grad_()
+    v = [leaf(t) for t in (*x, dt, A, *B, *C, D, h0)]
+    yf, yb, lf, lb = ISSM_biscan_combined(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], 64, D=v[8], initial_states=v[9])
+    both = torch.autograd.grad((yf, yb, lf, lb), v, (*dy, *df))
+    one = []
+    for d in range(2):
+        t = (lambda q: torch.flip(q, [1])) if d else (lambda q: q)
+        w = [leaf(q) for q in (t(x[d]).contiguous(), t(dt).contiguous(), A, t(B[d]).contiguous(), t(C[d]).contiguous(), D, h0)]
+        y, last = ISSM_chunk_scan_combined(*w[:5], 64, D=w[5], initial_states=w[6], return_final_states=True)
+        gr = torch.autograd.grad((y, last), w, (t(dy[d]).contiguous(), df[d]))
+        one.append([t(gr[0]), t(gr[1]), gr[2], t(gr[3]), t(gr[4]), gr[5], gr[6]])
+    ref = [one[0][0], one[1][0], one[0][1].double() + one[1][1].double(), one[0][2] + one[1][2], one[0][3], one[1][3], one[0][4], one[1][4],
+           one[0][5] + one[1][5], one[0][6] + one[1][6]]
+    for k, (got, want) in enumerate(zip(both, ref)):
+        err = ((got.double() - want.double()).norm() / want.double().norm()).item()
+        assert err <= (2.5e-3 if dtype == "bf16" else 5e-6 if k not in (2, 3) or not far else 5e-5), (k, err)
