@@ -118,10 +118,9 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
 // share the group's heads, heads_each each (a variant of its own: the two loop bounds more cost the others 25 - 50 scalar
 // registers spilled and 1 - 2 % of a training step).
 template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS, bool DUAL>
-__global__ __launch_bounds__(DUAL ? 2 * NTHREADS : NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
-                                                          const float* __restrict__ dstates,
-                                                          const float* __restrict__ dm, float* __restrict__ partA,
-                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+__device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __restrict__ states, const float* __restrict__ dstates,
+                                                const float* __restrict__ dm, float* __restrict__ partA,
+                                                float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
   constexpr bool SPLIT = !IOB;
   // fp32 products in the diagonal blocks / in all blocks.  (Four head tiles, complete: as the level form, which took these calls
   // before, has the closest pairs in fp32.  Operand pairs would leave ddt, dB, dC 5.0 -> 5.4e-6 of their norm from float64, fp32 products
@@ -784,6 +783,19 @@ __global__ __launch_bounds__(DUAL ? 2 * NTHREADS : NTHREADS, 2) void k_bwd_tile(
   }
 }
 
+template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
+__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states, const float* __restrict__ dstates,
+                                                          const float* __restrict__ dm, float* __restrict__ partA,
+                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+  k_bwd_tile_body<PT, IOB, PNF, ACC, P32, FULL, PARTS, false>(p, states, dstates, dm, partA, partBias, redo, heads_each);
+}
+template <int PT, bool IOB, bool PNF>
+__global__ __launch_bounds__(2 * NTHREADS, 2) void k_bwd_tile_dual(KP p, const float* __restrict__ states, const float* __restrict__ dstates,
+                                                                   const float* __restrict__ dm, float* __restrict__ partA,
+                                                                   float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+  k_bwd_tile_body<PT, IOB, PNF, false, false, true, false, true>(p, states, dstates, dm, partA, partBias, redo, heads_each);
+}
+
 // Whether the tile-base kernel is built for this call (otherwise the level-hierarchy kernel does all the work): no packed
 // sequences (their cuts are outside the form's range), x / B / C and dt of one type, x and dout rows that allow vector
 // accesses, ddt wanted, a gated dy (which is fp32) only beside fp32 inputs.  Four fp32 head tiles, one head a group and one
@@ -828,18 +840,18 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
     return 0;
   };
   if constexpr (IOB)
-    if (dual && !pnf) return go(&k_bwd_tile<PT, IOB, false, false, false, true, false, true>, 2);
+    if (dual && !pnf) return go(&k_bwd_tile_dual<PT, IOB, false>, 2);
   if constexpr (IOB || PT == 2)
-    if (dual) return go(&k_bwd_tile<PT, IOB, true, false, false, true, false, true>, 2);
+    if (dual) return go(&k_bwd_tile_dual<PT, IOB, true>, 2);
   auto pick = [&](auto p32) -> int {
     constexpr bool P32 = decltype(p32)::value;
     if (parts > 1) {
-      if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, true, false>);
-      return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, true, false>);
+      if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, true>);
+      return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, true>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, true>);
     }
-    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, false, false>);
-    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true, false, false>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true, false, false>);
-    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, false, false>);
+    if (!p.full_tiles) return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, false, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, false, false>);
+    if (pnf) return acc ? go(&k_bwd_tile<PT, IOB, true, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, true, false, P32, true, false>);
+    return acc ? go(&k_bwd_tile<PT, IOB, false, true, P32, true, false>) : go(&k_bwd_tile<PT, IOB, false, false, P32, true, false>);
   };
   if constexpr (IOB)
     if (p.ddt_part.ptr) return pick(std::true_type{});
