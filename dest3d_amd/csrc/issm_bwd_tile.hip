@@ -52,14 +52,18 @@ constexpr float SPAN_LIMIT = 96.0f;
 template <int PT, bool SPLIT>
 struct BwdTileSmem {
   static constexpr int KW = 16 * PT, LDP = KW + 8;  // x / dy tiles [l][p]
-  static constexpr int LDM = CS + 8;                // T[i][j] = dM[max(i,j)][min(i,j)]
+  // T[i][j] = dM[max(i,j)][min(i,j)]; fp32 inputs: hi and lo of four columns side by side, the operand (hi | lo) of a K = 32 instruction as
+  // one 16-byte read.  (With the two in matrices of their own every second operand took moves, as the heads a set of zeros for the
+  // case that nothing is evaluated: 100 of 1500 vector instructions a head.  8 x 1024 tokens, 8 heads x 48, 256 states, both directions, by
+  // direction 105 and 114 -> 101 and 111 us.)
+  static constexpr int LDM = CS + (SPLIT ? 4 : 8);
   static constexpr int NH = SPLIT ? 2 : 1;          // hi (and lo) copies
   // fp32 inputs: x and dy one after the other in one place.  (The last rows of the arrays go without
   // padding, and three head tiles then take exactly half of a CU's 160 KB.)
   uint16_t xs[NH * CS * LDP - (SPLIT ? 8 : 0)];
   uint16_t dys_own[SPLIT ? 0 : NH * CS * LDP];
   __device__ __forceinline__ uint16_t* dys() { return SPLIT ? xs : dys_own; }
-  alignas(16) uint16_t tm[NH * CS * LDM - (SPLIT ? 8 : 0)];
+  alignas(16) uint16_t tm[NH * CS * LDM];
   static constexpr int LDF = CS + 4;                // the same matrix in fp32 (fp32 inputs, incomplete tiles)
   static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
   __device__ __forceinline__ float* tf() { return reinterpret_cast<float*>(tm); }
@@ -106,10 +110,11 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
   return r;
 }
 
+constexpr int DUAL_TILES = 8;
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
-// DUAL: both directions in one launch, four waves each of a workgroup of eight, on the same tokens, head by head: dt comes from memory
+// TILES: head tiles, DUAL_TILES more (DUAL) for both directions in one launch, four waves each of a workgroup of eight, on the same tokens, head by head: dt comes from memory
 // once and their ddt is added up through LDS instead of being stored, read back and stored again (711 -> 510 MB at 8 x 1024 tokens, 8
 // heads x 32, 256 states, fp32).  What it gives is less than that, for eight waves now meet where four did: the two launches 88 + 96 us,
 // this one 172; heads of 36, bf16, 71 + 75 and 134.  (The second direction a barrier or two behind the first, so that they use LDS and
@@ -117,10 +122,13 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
 // FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).  PARTS: gridDim.y workgroups
 // share the group's heads, heads_each each (a variant of its own: the two loop bounds more cost the others 25 - 50 scalar
 // registers spilled and 1 - 2 % of a training step).
-template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS, bool DUAL>
-__device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __restrict__ states, const float* __restrict__ dstates,
-                                                const float* __restrict__ dm, float* __restrict__ partA,
-                                                float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+template <int TILES, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
+__global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
+                                                          const float* __restrict__ dstates,
+                                                          const float* __restrict__ dm, float* __restrict__ partA,
+                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+  constexpr bool DUAL = TILES >= DUAL_TILES;
+  constexpr int PT = TILES % DUAL_TILES;
   constexpr bool SPLIT = !IOB;
   // fp32 products in the diagonal blocks / in all blocks.  (Four head tiles, complete: as the level form, which took these calls
   // before, has the closest pairs in fp32.  Operand pairs would leave ddt, dB, dC 5.0 -> 5.4e-6 of their norm from float64, fp32 products
@@ -309,11 +317,16 @@ __device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __rest
         put(mrow, l_th0, l_tl0);
         put(32 + mrow, l_th1, l_tl1);
       } else {
-        *(uint4*)(s.tm + mrow * LDM + mcol) = l_th0;
-        *(uint4*)(s.tm + (32 + mrow) * LDM + mcol) = l_th1;
         if constexpr (SPLIT) {
-          *(uint4*)(s.tm + CS * LDM + mrow * LDM + mcol) = l_tl0;
-          *(uint4*)(s.tm + CS * LDM + (32 + mrow) * LDM + mcol) = l_tl1;
+          uint2* d0 = (uint2*)(s.tm + 2 * (mrow * LDM + mcol));
+          uint2* d1 = (uint2*)(s.tm + 2 * ((32 + mrow) * LDM + mcol));
+          d0[0] = make_uint2(l_th0.x, l_th0.y); d0[1] = make_uint2(l_tl0.x, l_tl0.y);
+          d0[2] = make_uint2(l_th0.z, l_th0.w); d0[3] = make_uint2(l_tl0.z, l_tl0.w);
+          d1[0] = make_uint2(l_th1.x, l_th1.y); d1[1] = make_uint2(l_tl1.x, l_tl1.y);
+          d1[2] = make_uint2(l_th1.z, l_th1.w); d1[3] = make_uint2(l_tl1.z, l_tl1.w);
+        } else {
+          *(uint4*)(s.tm + mrow * LDM + mcol) = l_th0;
+          *(uint4*)(s.tm + (32 + mrow) * LDM + mcol) = l_th1;
         }
       }
       if constexpr (SPLIT) {
@@ -356,9 +369,10 @@ __device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __rest
     const uint16_t* tm_ = s.tm;
 
     float dcs[16], val[16], gsum = 0.0f;   // gsum: the lane's share of the states' gradient to the chunk's total, see below
+    if (skip) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) dcs[k] = val[k] = 0.0f;
-    if (!skip) {
+      for (int k = 0; k < 16; ++k) asm volatile("v_mov_b32 %0, 0\nv_mov_b32 %1, 0" : "=v"(dcs[k]), "=v"(val[k]));  // (opaque: zeros set in advance are set for every head)
+    } else {
       // dS and H of the lane's column as (hi, lo) bf16 pairs: the B operands of Q = x . dS and R = dy . H (products over
       // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states, whose rounding to
       // 8 bits would be far above that of the inputs.
@@ -582,12 +596,17 @@ __device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __rest
           xg = block32(from(t[R]), cf32 + 4 * R, xg);
         } else {
           uint2 th[4], tl[4];
-          const uint16_t* row = tm_ + (16 * R + cq) * LDM + 4 * gq;
+          const uint16_t* row = tm_ + (SPLIT ? 2 : 1) * ((16 * R + cq) * LDM + 4 * gq);
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            th[c] = *(const uint2*)(row + 16 * c);
-            if (SPLIT) tl[c] = *(const uint2*)(row + CS * LDM + 16 * c);
-            else tl[c] = make_uint2(0u, 0u);
+            if constexpr (SPLIT) {
+              const uint4 t = *(const uint4*)(row + 32 * c);
+              th[c] = make_uint2(t.x, t.y);
+              tl[c] = make_uint2(t.z, t.w);
+            } else {
+              th[c] = *(const uint2*)(row + 16 * c);
+              tl[c] = make_uint2(0u, 0u);
+            }
           }
           // the other half's blocks first: their sum decays across the middles; then those of the rows' own half
           if (R >= 2) xf = scaled_twice(block2(th, tl, Bh, Bl, 0, xf), e0, e1);
@@ -783,19 +802,6 @@ __device__ __forceinline__ void k_bwd_tile_body(const KP& p, const float* __rest
   }
 }
 
-template <int PT, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PARTS>
-__global__ __launch_bounds__(NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states, const float* __restrict__ dstates,
-                                                          const float* __restrict__ dm, float* __restrict__ partA,
-                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
-  k_bwd_tile_body<PT, IOB, PNF, ACC, P32, FULL, PARTS, false>(p, states, dstates, dm, partA, partBias, redo, heads_each);
-}
-template <int PT, bool IOB, bool PNF>
-__global__ __launch_bounds__(2 * NTHREADS, 2) void k_bwd_tile_dual(KP p, const float* __restrict__ states, const float* __restrict__ dstates,
-                                                                   const float* __restrict__ dm, float* __restrict__ partA,
-                                                                   float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
-  k_bwd_tile_body<PT, IOB, PNF, false, false, true, false, true>(p, states, dstates, dm, partA, partBias, redo, heads_each);
-}
-
 // Whether the tile-base kernel is built for this call (otherwise the level-hierarchy kernel does all the work): no packed
 // sequences (their cuts are outside the form's range), x / B / C and dt of one type, x and dout rows that allow vector
 // accesses, ddt wanted, a gated dy (which is fp32) only beside fp32 inputs.  Four fp32 head tiles, one head a group and one
@@ -840,9 +846,9 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
     return 0;
   };
   if constexpr (IOB)
-    if (dual && !pnf) return go(&k_bwd_tile_dual<PT, IOB, false>, 2);
+    if (dual && !pnf) return go(&k_bwd_tile<DUAL_TILES + PT, IOB, false, false, false, true, false>, 2);
   if constexpr (IOB || PT == 2)
-    if (dual) return go(&k_bwd_tile_dual<PT, IOB, true>, 2);
+    if (dual) return go(&k_bwd_tile<DUAL_TILES + PT, IOB, true, false, false, true, false>, 2);
   auto pick = [&](auto p32) -> int {
     constexpr bool P32 = decltype(p32)::value;
     if (parts > 1) {
