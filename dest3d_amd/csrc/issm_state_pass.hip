@@ -8,7 +8,7 @@
 // states, half as much again, for the column sums g = sum_p dS_c H_(c+1) that d/d(cs) needs, in slices of 32 or 64 columns by all
 // rows with the rows' sums through LDS.  The chunk backward now takes g from what it has in registers, see k_bwd_tile.
 // Launched over and over on the same buffers, backward, 2 x 16384 tokens, 8 heads x 32, 256 states: 109 -> 47 us, 5.8 TB/s (inside a
-// training step, where the buffers come from HBM, 67, 4 TB/s); 8 x 1024, both directions: 32 -> 26; forward, inside a step, 16 x 2048, 16 heads
+// training step, where the buffers come from HBM, 62, 4.3 TB/s); 8 x 1024, both directions: 32 -> 26; forward, inside a step, 16 x 2048, 16 heads
 // x 64, 512 states, both directions: 0.93 ms, 4.6 TB/s.)
 #include "issm_dev.h"
 
@@ -56,7 +56,7 @@ __global__ __launch_bounds__(NTHREADS) void k_state_pass(KP p, float* __restrict
                                                          float* __restrict__ dh0_dir) {
   const int nq = (p.N + 3) >> 2;
   const long total = (long)p.B * p.ndir * p.H * p.P * nq;
-  const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
+  const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= total) return;
   const int q = id % nq;
   long r = id / nq;
@@ -172,8 +172,12 @@ __global__ __launch_bounds__(NTHREADS) void k_state_sums(KP p, const float* __re
 template <bool BACK>
 static int launch_state_pass(const KP& p, float* states, const float* cs_last, float* dh0_dir, hipStream_t st) {
   const long rows = (long)p.B * p.ndir * p.H * p.P, total = rows * (p.N < 4 ? p.N : (p.N + 3) / 4);
-  const int blocks = (int)((total + NTHREADS - 1) / NTHREADS);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), 0, st, p, states, cs_last, dh0_dir); };
+  // Where workgroups of four waves would leave a third of the CUs without one, each wave is one: 2 x 16384 tokens, 8 heads x 32, 256 states,
+  // inside a training step, 64 and 67 us -> 55 and 62 (4.6 TB/s, what a copy reaches; 16 or 24 chunks requested ahead: the same); 2 x 1024,
+  // forward 7.2 -> 6.7.  With 225 of them, 4 x 1000 tokens, 8 heads x 36, 200 states, 9.5 and 9.2 -> 9.8 and 9.6.
+  const int threads = p.N >= 4 && total < 160L * NTHREADS ? 64 : NTHREADS;
+  const int blocks = (int)((total + threads - 1) / threads);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads), 0, st, p, states, cs_last, dh0_dir); };
   const bool few = total < (1L << 17) && p.nc >= 16;
   if (p.N < 4) go(&k_state_pass_narrow<BACK>);
   else if (p.N & 3) few ? go(&k_state_pass<8, true, BACK>) : go(&k_state_pass<4, true, BACK>);
