@@ -286,7 +286,8 @@ static KP make_kp(const issm_scan_args* a) {
   if (a->flags & ISSM_FLAG_SEQ_IDX) {
     p.seq_idx = a->seq_idx; p.seq_s0 = a->seq_idx_stride[0]; p.seq_s1 = a->seq_idx_stride[1];
   }
-  p.c_lo = 0; p.ncl = p.nc;
+  p.by_H = div_by(p.H); p.by_nc = div_by(p.nc); p.by_hpg = div_by(p.hpg); p.by_slices = div_by((p.N + NS - 1) / NS); p.by_G = div_by(p.G);
+  p.by_quads = div_by((p.N + 3) / 4); p.by_P = div_by(p.P);
   p.full_tiles = p.N % 64 == 0 && p.L % ISSM_CHUNK == 0 && !p.seq_idx;
   return p;
 }

@@ -383,17 +383,15 @@ __device__ __forceinline__ void k_bwd_chunk_body(const KP& p, const float* __res
   // `mirror` (complete chunks only): the workgroup's chunk index counts from the other end -- the chunk of this direction
   // that covers the same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions'
   // shares to those tokens' ddt one after the other, and no two workgroups ever update one address).
-  int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int ns = id % nsl;
-  id /= nsl;
-  u.g = id % p.G;
-  id /= p.G;
-  const int cj = id % p.ncl;
-  u.c = p.c_lo + (mirror ? p.ncl - 1 - cj : cj);
-  u.b = id / p.ncl;
+  unsigned id = xcd_remap(blockIdx.x, gridDim.x);
+  const int ns = (int)p.by_slices(id);
+  u.g = (int)p.by_G(id);
+  const int cj = (int)p.by_nc(id);
+  u.c = (mirror ? p.nc - 1 - cj : cj);
+  u.b = (int)id;
   if (redo) {
-    const int nblk = p.B * p.ncl * p.G * nsl;
-    const int wg = ((u.b * p.ncl + (u.c - p.c_lo)) * p.G + u.g) * nsl + ns;  // as the tile-base kernel counts them
+    const int nblk = p.B * p.nc * p.G * nsl;
+    const int wg = ((u.b * p.nc + u.c) * p.G + u.g) * nsl + ns;  // as the tile-base kernel counts them
     redo += (dir_here * nblk + wg) * p.hpg;
     int any = 0;
     for (int hh = 0; hh < p.hpg; ++hh) any |= redo[hh];
@@ -869,18 +867,16 @@ __device__ __forceinline__ void k_bwd_chunk_bf_body(const KP& p, const float* __
   // `mirror` (complete chunks only): the workgroup's chunk index counts from the other end -- the chunk of this direction
   // that covers the same tokens as the un-mirrored chunk of the other direction (one workgroup then adds both directions'
   // shares to those tokens' ddt one after the other, and no two workgroups ever update one address).
-  int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int ns = id % nsl;
-  id /= nsl;
-  u.g = id % p.G;
-  id /= p.G;
-  const int cj = id % p.ncl;
-  u.c = p.c_lo + (mirror ? p.ncl - 1 - cj : cj);
-  u.b = id / p.ncl;
+  unsigned id = xcd_remap(blockIdx.x, gridDim.x);
+  const int ns = (int)p.by_slices(id);
+  u.g = (int)p.by_G(id);
+  const int cj = (int)p.by_nc(id);
+  u.c = (mirror ? p.nc - 1 - cj : cj);
+  u.b = (int)id;
   const float* before = nullptr;   // the sums over the heads the tile-base kernel evaluated
   if (redo) {
-    const int nblk = p.B * p.ncl * p.G * nsl;
-    const int wg = ((u.b * p.ncl + (u.c - p.c_lo)) * p.G + u.g) * nsl + ns;  // as the tile-base kernel counts them
+    const int nblk = p.B * p.nc * p.G * nsl;
+    const int wg = ((u.b * p.nc + u.c) * p.G + u.g) * nsl + ns;  // as the tile-base kernel counts them
     redo += (dir_here * nblk + wg) * p.hpg;
     int any = 0;
     for (int hh = 0; hh < p.hpg; ++hh) any |= redo[hh];
@@ -1476,13 +1472,11 @@ __global__ __launch_bounds__(NTHREADS) void k_bwd_parts_sum(KP p, const int* __r
   const int nsl = (p.N + NS - 1) / NS, wg = blockIdx.x, q = blockIdx.y;
   Unit u;
   u.dir = blockIdx.z;
-  int id = wg;
-  const int ns = id % nsl;
-  id /= nsl;
-  u.g = id % p.G;
-  id /= p.G;
-  u.c = p.c_lo + id % p.ncl;
-  u.b = id / p.ncl;
+  unsigned id = wg;
+  const int ns = (int)p.by_slices(id);
+  u.g = (int)p.by_G(id);
+  u.c = (int)p.by_nc(id);
+  u.b = (int)id;
   u.bt = u.b * p.ndir + u.dir;
   u.h = u.g * p.hpg;
   const long at = (long)u.dir * gridDim.x + wg;

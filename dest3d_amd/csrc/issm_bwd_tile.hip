@@ -152,19 +152,16 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   const int nsl = (p.N + NS - 1) / NS;
   Unit u;
   int wg = xcd_remap(blockIdx.x, gridDim.x);
-  int id = wg;
-  const int ns = id % nsl;
-  id /= nsl;
-  u.g = id % p.G;
-  id /= p.G;
+  unsigned id = wg;
+  const int ns = (int)p.by_slices(id);
+  u.g = (int)p.by_G(id);
   u.dir = DUAL ? half : p.dir0;
-  u.c = id % p.ncl;
-  u.b = id / p.ncl;
+  u.c = (int)p.by_nc(id);
+  u.b = (int)id;
   if (DUAL && half) {   // the same tokens: the mirrored chunk, marked where a launch of this direction alone would
-    u.c = p.ncl - 1 - u.c;
-    wg = ((u.b * p.ncl + u.c) * p.G + u.g) * nsl + ns;
+    u.c = p.nc - 1 - u.c;
+    wg = ((u.b * p.nc + u.c) * p.G + u.g) * nsl + ns;
   }
-  u.c += p.c_lo;
   u.bt = u.b * p.ndir + u.dir;
   u.h = u.g * p.hpg;
   const int n = ns * NS + wave * 16 + cm;

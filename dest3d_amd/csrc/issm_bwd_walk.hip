@@ -152,15 +152,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
   const int cm = lane & 15, g4 = lane >> 4;
   const int nsl = (p.N + NS - 1) / NS;
   // heads fastest: they share C's slice; then the slices, which share the head's dy and x
-  int id = xcd_remap(blockIdx.x, walks);
+  unsigned id = xcd_remap(blockIdx.x, walks);
   Unit u;
-  u.h = id % p.H;
-  id /= p.H;
-  const int ns = id % nsl;
-  u.bt = id / nsl;
-  u.b = u.bt / p.ndir;
-  u.dir = u.bt % p.ndir;
-  u.g = u.h / p.hpg;
+  u.h = (int)p.by_H(id);
+  const int ns = (int)p.by_slices(id);
+  u.bt = (int)id;
+  u.dir = u.bt & (p.ndir - 1);
+  u.b = u.bt >> (p.ndir - 1);
+  unsigned g = (unsigned)u.h;
+  p.by_hpg(g);
+  u.g = (int)g;
   const int n = ns * NS + wave * 16 + cm;
   const bool vn = FULL || n < p.N;
   const Coef cf = lane_coef(p, u.h, n, vn);

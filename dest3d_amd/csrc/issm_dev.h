@@ -46,13 +46,34 @@ struct TensorD {
   long s0, s1, s2;  // element strides of dims 0,1,2 (innermost contiguous)
 };
 
-// Kernel parameter block (passed by value).
+// Division of a number below 2^31 by a fixed one in four instructions: m = (2^32 - 1) / d, the quotient one short at most.
+struct Div {
+  unsigned d, m;
+  // n becomes the quotient; returns the remainder
+  __device__ __forceinline__ unsigned operator()(unsigned& n) const {
+    unsigned q = __umulhi(n, m), r = n - q * d;
+    const bool more = r >= d;
+    q += more ? 1u : 0u;
+    r -= more ? d : 0u;
+    n = q;
+    return r;
+  }
+};
+static inline Div div_by(unsigned d) { return Div{d, 0xffffffffu / d}; }
+
+// Kernel parameter block (passed by value).  What a kernel needs before its first request -- sizes and divisors to find its unit, the inputs'
+// addresses -- lies in front, in few cache lines.
 struct KP {
   int B, L, H, P, N, G, ndir, nc, hpg;
   int dir0;  // direction handled by this launch (kernels launched per direction)
   int io_dt, dt_dt, h0_dt;  // 0 = f32, 1 = bf16
   unsigned flags;
   float dt_min, dt_max;
+  // full_tiles picks the kernel variants: 1 = every chunk has 64 rows and every column slice 64 columns (complete-tile code); 0 = the
+  // "edge" variants (FULL = false), the same code with clamped addresses, dt' = 0 where a row or column is absent and
+  // guarded stores in the workgroups and steps that have such rows or columns.
+  int full_tiles;
+  Div by_H, by_nc, by_hpg, by_slices, by_G, by_quads, by_P;   // slices, quads: of 64 and 4 state columns
   TensorD x[2], Bm[2], Cm[2], z[2], out[2], dout[2], dx[2], dB[2], dC[2], dz[2];
   TensorD dt, ddt, h0;
   // Two directions with a bf16 ddt: the first direction's share of ddt travels in fp32 through this (B, L, H, N) buffer
@@ -72,11 +93,6 @@ struct KP {
   const float* dfinal[2];
   const int* seq_idx;   // (B, L) sequence ids of packed rows, or null
   long seq_s0, seq_s1;
-  // Chunks [c_lo, c_lo + ncl) are the ones a launch of a per-chunk kernel covers (all nc of them).  full_tiles picks
-  // the kernel variants: 1 = every chunk has 64 rows and every column slice 64 columns (complete-tile code); 0 = the
-  // "edge" variants (FULL = false), the same code with clamped addresses, dt' = 0 where a row or column is absent and
-  // guarded stores in the workgroups and steps that have such rows or columns.
-  int c_lo, ncl, full_tiles;
 };
 
 enum : unsigned { F_SOFTPLUS = 1u, F_D_HDIM = 2u, F_NOCLAMP = 4u };
@@ -509,24 +525,21 @@ struct Unit {
 // forward direction is paired with chunk nc - 1 - j of the reversed one: the same block of tokens, so the two
 // workgroups that read one head's dt tile (the largest operand, shared by the directions) run side by side on one
 // XCD and the second read is served by its L2.
-__device__ __forceinline__ Unit decode_unit(const KP& p, int u) {
+// Bound by the latency of what it does, in front of everything: with divisions and a branch on ndir 1300 - 2000 cycles of the 8700
+// until k_local_tile's first step began, one workgroup a CU.
+__device__ __forceinline__ Unit decode_unit(const KP& p, unsigned u) {
   Unit r;
-  r.h = u % p.H;
-  u /= p.H;
-  if (p.ndir == 2) {
-    r.dir = u & 1;
-    u >>= 1;
-    const int j = u % p.ncl;
-    r.b = u / p.ncl;
-    r.c = p.c_lo + (r.dir ? p.ncl - 1 - j : j);
-    r.bt = r.b * 2 + r.dir;
-  } else {
-    r.c = p.c_lo + u % p.ncl;
-    r.bt = u / p.ncl;
-    r.dir = r.bt % p.ndir;
-    r.b = r.bt / p.ndir;
-  }
-  r.g = r.h / p.hpg;
+  r.h = (int)p.by_H(u);
+  const unsigned two = (unsigned)p.ndir - 1;
+  r.dir = (int)(u & two);
+  u >>= two;
+  const int j = (int)p.by_nc(u);
+  r.b = (int)u;
+  r.c = r.dir ? p.nc - 1 - j : j;
+  r.bt = r.b * p.ndir + r.dir;
+  unsigned g = (unsigned)r.h;
+  p.by_hpg(g);
+  r.g = (int)g;
   return r;
 }
 // physical row of logical time t for a direction

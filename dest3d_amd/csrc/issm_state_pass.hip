@@ -58,12 +58,20 @@ __global__ __launch_bounds__(NTHREADS) void k_state_pass(KP p, float* __restrict
   const long total = (long)p.B * p.ndir * p.H * p.P * nq;
   const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= total) return;
-  const int q = id % nq;
-  long r = id / nq;
-  const int pp = r % p.P;
-  r /= p.P;
-  const int h = r % p.H;
-  const int bt = r / p.H;
+  int q, pp, h, bt;
+  if (total < (1L << 31)) {
+    unsigned r = (unsigned)id;
+    q = (int)p.by_quads(r);
+    pp = (int)p.by_P(r);
+    h = (int)p.by_H(r);
+    bt = (int)r;
+  } else {
+    q = id % nq;
+    const long r = id / nq;
+    pp = r % p.P;
+    h = r / p.P % p.H;
+    bt = r / p.P / p.H;
+  }
   const int n = TAIL ? min(q * 4, p.N - 4) : q * 4, skip = q * 4 - n;   // skip: columns of the thread that are its neighbour's
   auto ld = [](const float* a) -> f4 {
     if constexpr (TAIL) return ld_f4_any(a);
