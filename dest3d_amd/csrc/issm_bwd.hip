@@ -74,6 +74,7 @@ __device__ __forceinline__ void k_bwd_dstates_body(const KP& p, const float* __r
   constexpr int LDP = SM::LDP, LDT = SM::LDT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
+  warm_args();
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
 
   int n = wave * 16 + cm;
@@ -1187,6 +1188,7 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   constexpr int LDY = YT::LD, LDK = SM::LDK, LDPR = SM::LDPROD;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
+  warm_args();
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
   const float* ds = dstates + dst_off(p, u.bt, u.c, u.h);
 

@@ -143,6 +143,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_walk(KP p, const float* __r
   constexpr int LDT = SM::LDT, G4 = 4 * PT, ROWS = 4 * PT;
   typedef typename std::conditional<BF, uint16_t, float>::type T;
   typedef typename std::conditional<BF, uint2, f4>::type V;   // four elements of a row
+  warm_args();
   if ((int)blockIdx.x >= walks) {
     dm_unit<PT, BF, FULL>(p, dy_ws, dm, (int)blockIdx.x - walks);
     return;

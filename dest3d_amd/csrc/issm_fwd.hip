@@ -90,6 +90,7 @@ __device__ __forceinline__ void col_store_bf(const float (&v)[16], uint16_t* dst
 
 template <int PT, bool IOB, bool DTB, bool FULL>
 __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
+  warm_args();
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef FwdScanSmem<PT, IOB> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);

@@ -148,6 +148,7 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
 template <int PT, bool IOB, bool DTB, bool FULLP, bool EDGE, bool ANY>
 __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restrict__ states, float* __restrict__ cs_last,
                                                             float* __restrict__ cabt) {
+  warm_args();
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr bool SPLIT = !IOB;
   typedef FwdTileSmem<PT, SPLIT> SM;

@@ -54,6 +54,7 @@ struct Pass {
 template <int D, bool TAIL, bool BACK>
 __global__ __launch_bounds__(NTHREADS) void k_state_pass(KP p, float* __restrict__ states, const float* __restrict__ cs_last,
                                                          float* __restrict__ dh0_dir) {
+  warm_args();
   const int nq = (p.N + 3) >> 2;
   const long total = (long)p.B * p.ndir * p.H * p.P * nq;
   const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;
