@@ -28,13 +28,13 @@
 //   tile raises a flag that all look at once a step, and the rest of the steps is left out (a quarter of the chunks of a freshly
 //   initialised decoder, 8 x 1024 tokens, 256 queries: 195 -> 179 us a layer, 118 without a device-wide fence).  fp32 inputs, whose operand pairs leave no
 //   registers to spare, pay for the look: 1505 -> 1575 us at 16 x 2048 tokens, 16 heads x 64, 512 states, nothing out of range.
-//   ANY, bf16 inputs of calls that nothing is differentiated through: a step with such a tile is left by the loop over the steps
-//   and evaluated, by its wave alone, with the diagonal blocks in parts whose factors are all <= 1 (far_diagonal) and V from its
-//   own exponential; the loop then goes on.  Outside the loop, for what the usual step keeps in flight leaves that form no
-//   registers.  A freshly initialised decoder has such tiles in 16 % of its chunks and heads, there mostly in all steps, and those
-//   workgroups decide when the launch ends: 1024 tokens, 256 queries 27 us a layer (36 with the chunk computed once more, 19 where
-//   no tile is out of range).  As accurate as the level form, but rounded elsewhere, and through six layers the gradients move by
-//   up to 0.8 of their mean square between the two: training keeps the level form (8 x 1024 tokens: 155 us, 110 with this one).
+//   ANY, bf16 inputs of calls that nothing is differentiated through: the first step with such a tile is left by the loop over the steps,
+// and it and all that follow are evaluated, by its wave alone, in a loop of their own, with the diagonal blocks in parts whose factors are all
+// <= 1 (far_diagonal) and V from its own exponential.  A freshly initialised decoder has such tiles in 16 % of its chunks and heads, there
+// mostly in all steps, and those workgroups decide when the launch ends: 1024 tokens, 256 queries 22.7 us a layer (28.1 with every step first in
+// the usual form, and its operands requested anew each time; 36 with the chunk computed once more, 18 where no tile is out of range).  As
+// accurate as the level form, but rounded elsewhere, and through six layers the gradients move by up to 0.8 of their mean square between the
+// two: training keeps the level form (8 x 1024 tokens: 155 us, 110 with this one).
 // bf16 inputs: a tile's whole decay reaches the tile's 16 lanes by DPP, not through LDS (both directions, 8 x 1024 tokens, 8 heads
 // x 36, 256 states 93 -> 91 us; fp32 1 to 2 % slower so).
 #include "issm_dev.h"
@@ -320,23 +320,20 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #include "issm_fwd_tile_step.h"
     }
   } else {
-    for (int n0 = 0;;) {
+    int n0 = 0;
+#pragma unroll 1
+    for (; n0 < p.N; n0 += NS) {
+      constexpr bool DEEP = false;
+#include "issm_fwd_tile_step.h"
+    }
+    if (n0 < p.N) {
       asm volatile("");   // keeps the two loops apart
+      ISSM_REQUEST(n0);
 #pragma unroll 1
       for (; n0 < p.N; n0 += NS) {
-        constexpr bool DEEP = false;
-#include "issm_fwd_tile_step.h"
-      }
-      if (n0 >= p.N) break;
-      ISSM_REQUEST(n0);
-      do {
         constexpr bool DEEP = true;
 #include "issm_fwd_tile_step.h"
-      } while (false);
-      etmin = 1.0f;
-      n0 += NS;
-      if (n0 >= p.N) break;
-      ISSM_REQUEST(n0);
+      }
     }
   }
 #undef ISSM_REQUEST

@@ -27,7 +27,7 @@
       }
     };
     if constexpr (LATE_C) ISSM_REQUEST_C(c)
-    if (!DEEP) {  // branch-free: the last step asks for its own columns once more
+    {  // branch-free: the last step asks for its own columns once more
       const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
       ISSM_REQUEST(nn);
     }

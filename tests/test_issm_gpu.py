@@ -1568,3 +1568,30 @@ def test_both_directions_of_the_chunk_backward_in_one_launch(dtype, P, H, G, far
     for k, (got, want) in enumerate(zip(both, ref)):
         err = ((got.double() - want.double()).norm() / want.double().norm()).item()
         assert err <= (2.5e-3 if dtype == "bf16" else 5e-6 if k not in (2, 3) or not far else 5e-5), (k, err)
+
+
+@pytest.mark.parametrize("L_,P,N,far", [(128, 36, 256, 0), (128, 64, 256, 1), (64, 32, 128, 1), (90, 20, 200, 0), (70, 48, 68, 1)])
+def test_bf16_forward_of_the_steps_behind_a_far_tile(L_, P, N, far):
+    """issm_scan_fwd_only: 16 columns of the step `far` decay beyond 2^100 a tile, so their wave takes that step and those behind it, whose
+    columns do not, in the form without a range, and the other waves none.  Bound as in test_bf16_forward_of_any_decay."""
+    H = 2
+    d = _problem(2, L_, H, P, N, 1, seed=L_ + N, softplus=False, D=None)
+    d["A"] = torch.full((H, N), -1.0)
+    d["A"][1, 64 * far:64 * far + 16] = -60.0
+    d["dt"] = 0.5 * torch.rand(2, L_, H, N, generator=torch.Generator().manual_seed(7))
+    q = {k: d[k].bfloat16() for k in ("x", "dt", "B", "C")}
+    ref = [R.issm_scan_sequential(f(q["x"].double()), q["dt"].double(), d["A"].double(), f(q["B"].double()), f(q["C"].double()),
+                                  initial_states=f(d["h0"].double())) for f in (lambda t: t, torch.abs)]
+    c = {k: v.cuda() for k, v in q.items()}
+    L, prob, a = _stage_args(dict(c, A=d["A"], h0=d["h0"], D=None, z=None, dt_bias=None, softplus=False, dt_limit=(0.0, float("inf"))))
+    lib = L.load()
+    y, last = torch.empty_like(c["x"]), torch.empty(2, H, P, N, device="cuda")
+    a.out[0], a.final_states[0] = L.tensor_desc(y), last.data_ptr()
+    n = C.c_size_t()
+    L.check(lib.issm_fwd_workspace_bytes(C.byref(a), C.byref(n)), "workspace")
+    ws = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n.value
+    L.check(lib.issm_scan_fwd_only(C.byref(a)), "scan")
+    torch.cuda.synchronize()
+    for name, got, want, size in (("y", y, ref[0][0], ref[1][0]), ("last", last, ref[0][1], ref[1][1])):
+        assert ((got.double().cpu() - want).abs() <= 4 * 2.0 ** -9 * 1.125 * size + 1e-30).all(), name
