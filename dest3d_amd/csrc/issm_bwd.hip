@@ -1131,7 +1131,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_bwd_chunk_bf(KP p, const float*
 #ifndef DX_SPLIT_FROM
 #define DX_SPLIT_FROM 2
 #endif
-template <int PT, bool BF>
+template <int PT, bool BF, int NG>
 struct BwdDxSmem {
   static constexpr int LDK = NS + 8;
   // fp32 inputs: the product over the state index on (hi, lo) bf16 tiles, hi.hi + hi.lo + lo.hi, instead of fp32
@@ -1141,8 +1141,11 @@ struct BwdDxSmem {
   static constexpr bool B16 = BF || SPL;
   static constexpr int NH = SPL ? 2 : 1;
   float dys[RowTile<PT>::SIZE];
-  typename std::conditional<B16, uint16_t, float>::type bt[NH * CS * (B16 ? LDK : LDN)];        // B dt' exp2(last - cs) [m][n]
-  typename std::conditional<B16, uint16_t, float>::type dss[NH * PT * 16 * (B16 ? LDK : LDN)];  // dS [p][n]
+  static constexpr int BT = NH * CS * (B16 ? LDK : LDN), DS = NH * PT * 16 * (B16 ? LDK : LDN);
+  typedef typename std::conditional<B16, uint16_t, float>::type Op;
+  alignas(16) Op bt[NG * BT];  // B dt' exp2(last - cs) [m][n], a tile a group of waves
+  Op dss[NG * DS];             // dS [p][n]
+  static_assert(NG == 1 || NG * BT * sizeof(Op) >= PT * NTHREADS * sizeof(f4), "the second group's sums take the place of the tiles");
   // dy * x, in the place of `bt` and `dss` once their product is done
   static constexpr int LDPROD = B16 ? PT * 16 + 4 : LDN;
   __device__ __forceinline__ float* prod() { return reinterpret_cast<float*>(bt); }
@@ -1179,41 +1182,47 @@ __device__ __forceinline__ bf8 frag8(const uint16_t* tile, int row, int g4, int 
 }
 
 // partD: (Bt*nc*H, P) per-unit sums over rows of dy*x
-template <int PT, bool IOB, bool DTB, bool FULL>
+// NG: groups of four waves, as in k_chunk_scan.
+template <int PT, bool IOB, bool DTB, bool FULL, int NG>
 __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  typedef BwdDxSmem<PT, IOB> SM;
+  typedef BwdDxSmem<PT, IOB, NG> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
   typedef RowTile<PT> YT;
   constexpr int LDY = YT::LD, LDK = SM::LDK, LDPR = SM::LDPROD;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int STEP = NG * NS;
+  const int tid = NG > 1 ? threadIdx.x & (NTHREADS - 1) : threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NTHREADS) : 0;
+  typename SM::Op *bt = s.bt + grp * SM::BT, *dss = s.dss + grp * SM::DS;
   const int cm = lane & 15, g4 = lane >> 4;
   warm_args();
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
   const float* ds = dstates + dst_off(p, u.bt, u.c, u.h);
 
-  int n = wave * 16 + cm;
+  int n = grp * NS + wave * 16 + cm;
   bool vn = FULL || n < p.N;
   RowMap rm;
   Coef cf;
-  rm = make_rowmap<FULL>(p, u, g4, 0);
+  rm = make_rowmap<FULL>(p, u, g4, grp * NS);
   float raw[16], bv[16];
   PnRegs<PT> sv;
   lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, bv);
-  pn_load<PT, FULL>(p, ds, 0, sv);
-  {
+  pn_load<PT, FULL>(p, ds, grp * NS, sv, tid);
+  if (grp == NG - 1) {
     float dv[CS * PT * 16 / NTHREADS];
-    dy_load<IOB, PT, FULL>(p, u, dy_ws, dv);
-    lp_store<PT>(dv, s.dys);
+    dy_load<IOB, PT, FULL>(p, u, dy_ws, dv, tid);
+    lp_store<PT>(dv, s.dys, tid);
   }
   f4 acc[PT];
 #pragma unroll
   for (int pt = 0; pt < PT; ++pt) acc[pt] = (f4){0, 0, 0, 0};
 
-  for (int n0 = 0; n0 < p.N; n0 += NS) {
-    {
+  for (int m0 = 0; m0 < p.N; m0 += STEP) {
+    const int n0 = m0 + grp * NS;
+    const bool mine = NG == 1 || n0 < p.N;   // uniform
+    if (mine) {
       float dtp[16], cs[16], dummy[16];
       const float last = lane_prep<false>(p, cf, vn, cm, g4, rm, raw, dtp, cs, dummy);
       if constexpr (IOB) {
@@ -1223,8 +1232,8 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
           btv[k] = bv[k] * dtp[k] * ex2(last - cs[k]);
           btv[k + 1] = bv[k + 1] * dtp[k + 1] * ex2(last - cs[k + 1]);
           const unsigned h2 = pack_bf16(btv[k], btv[k + 1]);
-          s.bt[lane_row(k, g4) * LDK + wave * 16 + cm] = (uint16_t)h2;
-          s.bt[lane_row(k + 1, g4) * LDK + wave * 16 + cm] = (uint16_t)(h2 >> 16);
+          bt[lane_row(k, g4) * LDK + wave * 16 + cm] = (uint16_t)h2;
+          bt[lane_row(k + 1, g4) * LDK + wave * 16 + cm] = (uint16_t)(h2 >> 16);
         }
       } else if constexpr (SM::SPL) {
 #pragma unroll
@@ -1233,52 +1242,53 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
           const unsigned h2 = pack_bf16(b0, b1);
           const unsigned l2 = pack_bf16(b0 - __uint_as_float(h2 << 16), b1 - __uint_as_float(h2 & 0xffff0000u));
           const int o0 = lane_row(k, g4) * LDK + wave * 16 + cm, o1 = lane_row(k + 1, g4) * LDK + wave * 16 + cm;
-          s.bt[o0] = (uint16_t)h2;
-          s.bt[o1] = (uint16_t)(h2 >> 16);
-          s.bt[CS * LDK + o0] = (uint16_t)l2;
-          s.bt[CS * LDK + o1] = (uint16_t)(l2 >> 16);
+          bt[o0] = (uint16_t)h2;
+          bt[o1] = (uint16_t)(h2 >> 16);
+          bt[CS * LDK + o0] = (uint16_t)l2;
+          bt[CS * LDK + o1] = (uint16_t)(l2 >> 16);
         }
       } else {
 #pragma unroll
         for (int k = 0; k < 16; ++k)
-          s.bt[lane_row(k, g4) * LDN + wave * 16 + cm] = bv[k] * dtp[k] * ex2(last - cs[k]);
+          bt[lane_row(k, g4) * LDN + wave * 16 + cm] = bv[k] * dtp[k] * ex2(last - cs[k]);
       }
+      if constexpr (!FULL) pn_edge<PT>(p, n0, sv, tid);
+      if constexpr (IOB) pn_store_bf16<PT, LDK>(sv, dss, tid);
+      else if constexpr (SM::SPL) pn_store_hl<PT, LDK>(sv, dss, dss + PT * 16 * LDK, tid);
+      else pn_store<PT>(sv, dss, tid);
     }
-    if constexpr (!FULL) pn_edge<PT>(p, n0, sv);
-    if constexpr (IOB) pn_store_bf16<PT, LDK>(sv, s.dss);
-    else if constexpr (SM::SPL) pn_store_hl<PT, LDK>(sv, s.dss, s.dss + PT * 16 * LDK);
-    else pn_store<PT>(sv, s.dss);
-    if (n0 + NS < p.N) {
-      n = n0 + NS + wave * 16 + cm;
+    if (n0 + STEP < p.N) {
+      n = n0 + STEP + wave * 16 + cm;
       vn = FULL || n < p.N;
-      rm = make_rowmap<FULL>(p, u, g4, n0 + NS);
+      rm = make_rowmap<FULL>(p, u, g4, n0 + STEP);
       lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
       cf = lane_coef(p, u.h, n, vn);
       lane_load_ln<IOB>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, bv);
-      pn_load<PT, FULL>(p, ds, n0 + NS, sv);
+      pn_load<PT, FULL>(p, ds, n0 + STEP, sv, tid);
     }
     __syncthreads();
-    if constexpr (IOB) {
+    if (!mine) {
+    } else if constexpr (IOB) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const bf8 a = frag8<LDK>(s.bt, wave * 16 + cm, g4, t);
+        const bf8 a = frag8<LDK>(bt, wave * 16 + cm, g4, t);
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) acc[pt] = mfma_bf(a, frag8<LDK>(s.dss, pt * 16 + cm, g4, t), acc[pt]);
+        for (int pt = 0; pt < PT; ++pt) acc[pt] = mfma_bf(a, frag8<LDK>(dss, pt * 16 + cm, g4, t), acc[pt]);
       }
     } else if constexpr (SM::SPL) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const bf8 ah = frag8<LDK>(s.bt, wave * 16 + cm, g4, t), al = frag8<LDK>(s.bt + CS * LDK, wave * 16 + cm, g4, t);
+        const bf8 ah = frag8<LDK>(bt, wave * 16 + cm, g4, t), al = frag8<LDK>(bt + CS * LDK, wave * 16 + cm, g4, t);
 #pragma unroll
         for (int pt = 0; pt < PT; ++pt)
-          acc[pt] = mfma_split(ah, al, frag8<LDK>(s.dss, pt * 16 + cm, g4, t),
-                               frag8<LDK>(s.dss + PT * 16 * LDK, pt * 16 + cm, g4, t), acc[pt]);
+          acc[pt] = mfma_split(ah, al, frag8<LDK>(dss, pt * 16 + cm, g4, t),
+                               frag8<LDK>(dss + PT * 16 * LDK, pt * 16 + cm, g4, t), acc[pt]);
       }
     } else {
 #pragma unroll
       for (int kb = 0; kb < NS; kb += 16)
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) mma16_mm(acc[pt], s.bt, LDN, wave * 16, s.dss, LDN, pt * 16, kb, lane);
+        for (int pt = 0; pt < PT; ++pt) mma16_mm(acc[pt], bt, LDN, wave * 16, dss, LDN, pt * 16, kb, lane);
     }
     __syncthreads();
   }
@@ -1288,38 +1298,52 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
   // M^T of this wave's 16 columns goes straight into matrix-operand registers (lane (column cm, group g4) holds
   // rows 16 kb + 4 g4 .. + 3 of the blocks kb >= wave, the upper triangle of the diagonal block zeroed): no LDS tile,
   // which lets a fourth workgroup live on the CU
-  float mf[4][4];
-  {
-    const float* mcol = cabt + sq_off(p, u.bt, u.c, u.h) + (4 * g4) * CS + wave * 16 + cm;
+  if (grp == NG - 1) {
+    float mf[4][4];
+    {
+      const float* mcol = cabt + sq_off(p, u.bt, u.c, u.h) + (4 * g4) * CS + wave * 16 + cm;
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) mf[kb][j] = mcol[(16 * max(kb, wave) + j) * CS];  // no branch between the loads
+        for (int j = 0; j < 4; ++j) mf[kb][j] = mcol[(16 * max(kb, wave) + j) * CS];  // no branch between the loads
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (kb < wave || (kb == wave && cm > 4 * g4 + j)) mf[kb][j] = 0.0f;
-  }
-  // dx[m][p] += sum_{l>=m} M[l][m] dy[l][p]
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb)
-    if (kb >= wave) {  // uniform
-      // the lane's four M values and four dy values are the operands of one K = 16 bf16 instruction as they stand
-      // (k-slot j of lane group g4 <-> row 16 kb + 4 g4 + j), both as (hi, lo) pairs
-      bf4 ah, al;
-      split4(mf[kb], ah, al);
-#pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        const float* bp = s.dys + YT::at(16 * kb + 4 * g4, pt * 16 + cm);
-        const float yw[4] = {bp[0], bp[LDY], bp[2 * LDY], bp[3 * LDY]};
-        bf4 bh, bl;
-        split4(yw, bh, bl);
-        acc[pt] = mfma_bf16k(al, bh, acc[pt]);
-        acc[pt] = mfma_bf16k(ah, bl, acc[pt]);  // (also for bf16 inputs: a gated dy is an fp32 product)
-        acc[pt] = mfma_bf16k(ah, bh, acc[pt]);
-      }
+        for (int j = 0; j < 4; ++j)
+          if (kb < wave || (kb == wave && cm > 4 * g4 + j)) mf[kb][j] = 0.0f;
     }
+    // dx[m][p] += sum_{l>=m} M[l][m] dy[l][p]
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+      if (kb >= wave) {  // uniform
+        // the lane's four M values and four dy values are the operands of one K = 16 bf16 instruction as they stand
+        // (k-slot j of lane group g4 <-> row 16 kb + 4 g4 + j), both as (hi, lo) pairs
+        bf4 ah, al;
+        split4(mf[kb], ah, al);
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt) {
+          const float* bp = s.dys + YT::at(16 * kb + 4 * g4, pt * 16 + cm);
+          const float yw[4] = {bp[0], bp[LDY], bp[2 * LDY], bp[3 * LDY]};
+          bf4 bh, bl;
+          split4(yw, bh, bl);
+          acc[pt] = mfma_bf16k(al, bh, acc[pt]);
+          acc[pt] = mfma_bf16k(ah, bl, acc[pt]);  // (also for bf16 inputs: a gated dy is an fp32 product)
+          acc[pt] = mfma_bf16k(ah, bh, acc[pt]);
+        }
+      }
+  }
+  if constexpr (NG > 1) {
+    f4* part = (f4*)s.bt;
+    if (grp) {
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt) part[pt * NTHREADS + tid] = acc[pt];
+    }
+    __syncthreads();
+    if (grp) return;
+#pragma unroll
+    for (int pt = 0; pt < PT; ++pt) acc[pt] += part[pt * NTHREADS + tid];
+    __syncthreads();   // dy * x goes where these were
+  }
 
   const TensorD& tx = p.x[u.dir];
   const TensorD& tdx = p.dx[u.dir];
@@ -1357,9 +1381,9 @@ __device__ __forceinline__ void k_bwd_dx_body(const KP& p, const float* __restri
     }
   }
 }
-template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, PT <= 2 ? 4 : 1) void k_bwd_dx(KP p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
-  k_bwd_dx_body<PT, IOB, DTB, FULL>(p, dy_ws, dstates, cabt, partD);
+template <int PT, bool IOB, bool DTB, bool FULL, int NG>
+__global__ __launch_bounds__(NG * NTHREADS, PT <= 2 && NG == 1 ? 4 : 1) void k_bwd_dx(KP p, const float* __restrict__ dy_ws, const float* __restrict__ dstates, const float* __restrict__ cabt, float* __restrict__ partD) {
+  k_bwd_dx_body<PT, IOB, DTB, FULL, NG>(p, dy_ws, dstates, cabt, partD);
 }
 
 // ------------------------------------------------------------------- reductions
@@ -1609,10 +1633,17 @@ int launch_bwd_dx(const KP& p, const float* dy_ws, const float* dstates, const f
                   hipStream_t st) {
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
-    const size_t sm = sizeof(BwdDxSmem<PT_, IOB_>);
-    constexpr auto kern = &k_bwd_dx<PT_, IOB_, DTB_, FULL_>;
-    if (int e = set_lds(kern, sm)) return e;
-    hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, dy_ws, dstates, cabt, partD);
+    if (two_groups(units, p.N)) {
+      const size_t sm = sizeof(BwdDxSmem<PT_, IOB_, 2>);
+      constexpr auto kern = &k_bwd_dx<PT_, IOB_, DTB_, FULL_, 2>;
+      if (int e = set_lds(kern, sm)) return e;
+      hipLaunchKernelGGL(kern, dim3(units), dim3(2 * NTHREADS), sm, st, p, dy_ws, dstates, cabt, partD);
+    } else {
+      const size_t sm = sizeof(BwdDxSmem<PT_, IOB_, 1>);
+      constexpr auto kern = &k_bwd_dx<PT_, IOB_, DTB_, FULL_, 1>;
+      if (int e = set_lds(kern, sm)) return e;
+      hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, dy_ws, dstates, cabt, partD);
+    }
   });
   return (int)hipGetLastError();
 }

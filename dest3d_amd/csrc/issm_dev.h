@@ -36,8 +36,16 @@ constexpr int LDN = NS + 4;    // leading dimension of [*][NS] tiles
 constexpr int LDC = CS + 4;    // leading dimension of [*][CS] tiles
 constexpr int MAXP = 64;       // largest head dimension built
 constexpr int NTHREADS = 256;
+constexpr int NCU = 256;       // compute units of the card
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
+
+// Whether k_chunk_scan and k_bwd_dx take two groups of four waves a workgroup, each with every second slice of the states: where no CU
+// gets a second workgroup.  A lone wave on a SIMD issues a vector instruction every 5.3 cycles, two together every 2.7 to 4.5.  256 units
+// of four slices: k_chunk_scan 13.2 -> 11.4 us (fp32, heads of 32), 14.3 -> 10.8 (bf16, 36), k_bwd_dx 15.6 -> 12.7 (128 units) and 17.4 ->
+// 13.9; 512 units, which share the CUs either way: 16.5 with one group, 18.8 with two.  (k_local_tile, bound by issue in its steps, the same
+// way: 17.6 -> 17.4 us, bf16 without a gradient 22.7 -> 23.9.)
+inline bool two_groups(int units, int N) { return units <= NCU && N > NS; }
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 

@@ -36,7 +36,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_chunk_local(KP p, float* __rest
 #ifndef SCAN_SPLIT_FROM
 #define SCAN_SPLIT_FROM 2
 #endif
-template <int PT, bool BF>
+template <int PT, bool BF, int NG>
 struct FwdScanSmem {
   static constexpr int LDK = NS + 8;  // row stride of the bf16 tiles
   // fp32 inputs: the product over the state index on (hi, lo) bf16 tiles, hi.hi + hi.lo + lo.hi, instead of fp32
@@ -48,8 +48,11 @@ struct FwdScanSmem {
   static constexpr bool B16 = BF || SPL;
   static constexpr int NH = SPL ? 2 : 1;
   float xs[RowTile<PT>::SIZE];                                  // x [s][p]
-  typename std::conditional<B16, uint16_t, float>::type ct[NH * CS * (B16 ? LDK : LDN)];       // C * exp2(cs) [l][n]
-  typename std::conditional<B16, uint16_t, float>::type hs[NH * PT * 16 * (B16 ? LDK : LDN)];  // H [p][n]
+  static constexpr int CT = NH * CS * (B16 ? LDK : LDN), HS = NH * PT * 16 * (B16 ? LDK : LDN);
+  typedef typename std::conditional<B16, uint16_t, float>::type Op;
+  alignas(16) Op ct[NG * CT];  // C * exp2(cs) [l][n], a tile a group of waves
+  Op hs[NG * HS];              // H [p][n]
+  static_assert(NG == 1 || NG * CT * sizeof(Op) >= PT * NTHREADS * sizeof(f4), "the second group's sums take the place of the tiles");
 };
 // a (16 PT x 64) slab of fp32 values (layout of pn_load) rounded to bf16 into LDS dst[p][col], row stride LD
 template <int PT, int LD>
@@ -88,96 +91,104 @@ __device__ __forceinline__ void col_store_bf(const float (&v)[16], uint16_t* dst
   }
 }
 
-template <int PT, bool IOB, bool DTB, bool FULL>
+// NG: groups of four waves.  Two take every second slice of the states each where the grid gives a CU no second workgroup to run
+// beside this one; the second adds M x.
+template <int PT, bool IOB, bool DTB, bool FULL, int NG>
 __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
   warm_args();
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  typedef FwdScanSmem<PT, IOB> SM;
+  typedef FwdScanSmem<PT, IOB, NG> SM;
   SM& s = *reinterpret_cast<SM*>(smem_raw);
   typedef RowTile<PT> XT;
   constexpr int LDX = XT::LD, LDK = SM::LDK;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int STEP = NG * NS;
+  const int tid = NG > 1 ? threadIdx.x & (NTHREADS - 1) : threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NTHREADS) : 0;
+  typename SM::Op *ct = s.ct + grp * SM::CT, *hs = s.hs + grp * SM::HS;
   const int cm = lane & 15, g4 = lane >> 4;
   const Unit u = decode_unit(p, xcd_remap(blockIdx.x, gridDim.x));
   const float* hsrc = states + st_off(p, u.bt, u.c, u.h);
 
-  int n = wave * 16 + cm;
+  int n = grp * NS + wave * 16 + cm;
   bool vn = FULL || n < p.N;
   RowMap rm;
   Coef cf;
-  rm = make_rowmap<FULL>(p, u, g4, 0);
+  rm = make_rowmap<FULL>(p, u, g4, grp * NS);
   float raw[16], cv[16];
   PnRegs<PT> hv;
   lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
   cf = lane_coef(p, u.h, n, vn);
   lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, cv);
-  pn_load<PT, FULL>(p, hsrc, 0, hv);
-  {
+  pn_load<PT, FULL>(p, hsrc, grp * NS, hv, tid);
+  if (grp == NG - 1) {
     float xv[CS * PT * 16 / NTHREADS];
-    lp_load<IOB, PT, FULL>(p, u, p.x[u.dir], xv);
-    lp_store<PT>(xv, s.xs);
+    lp_load<IOB, PT, FULL>(p, u, p.x[u.dir], xv, tid);
+    lp_store<PT>(xv, s.xs, tid);
   }
   f4 acc[PT];
 #pragma unroll
   for (int pt = 0; pt < PT; ++pt) acc[pt] = (f4){0, 0, 0, 0};
 
-  for (int n0 = 0; n0 < p.N; n0 += NS) {
-    {
+  for (int m0 = 0; m0 < p.N; m0 += STEP) {
+    const int n0 = m0 + grp * NS;
+    const bool mine = NG == 1 || n0 < p.N;   // uniform
+    if (mine) {
       float dtp[16], cs[16], dummy[16];
       lane_prep<false>(p, cf, vn, cm, g4, rm, raw, dtp, cs, dummy);
       if constexpr (IOB) {
         float ctv[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) ctv[k] = cv[k] * ex2(cs[k]);
-        col_store_bf<LDK>(ctv, s.ct, g4, wave * 16 + cm);
+        col_store_bf<LDK>(ctv, ct, g4, wave * 16 + cm);
       } else if constexpr (SM::SPL) {
         float ctv[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) ctv[k] = cv[k] * ex2(cs[k]);
-        op_store<LDK, true>(ctv, s.ct, s.ct + CS * LDK, g4, wave * 16 + cm);
+        op_store<LDK, true>(ctv, ct, ct + CS * LDK, g4, wave * 16 + cm);
       } else {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) s.ct[lane_row(k, g4) * LDN + wave * 16 + cm] = cv[k] * ex2(cs[k]);
+        for (int k = 0; k < 16; ++k) ct[lane_row(k, g4) * LDN + wave * 16 + cm] = cv[k] * ex2(cs[k]);
       }
+      if constexpr (!FULL) pn_edge<PT>(p, n0, hv, tid);
+      if constexpr (IOB) pn_store_bf<PT, LDK>(hv, hs, tid);
+      else if constexpr (SM::SPL) pn_store_split<PT, LDK>(hv, hs, hs + PT * 16 * LDK, tid);
+      else pn_store<PT>(hv, hs, tid);
     }
-    if constexpr (!FULL) pn_edge<PT>(p, n0, hv);
-    if constexpr (IOB) pn_store_bf<PT, LDK>(hv, s.hs);
-    else if constexpr (SM::SPL) pn_store_split<PT, LDK>(hv, s.hs, s.hs + PT * 16 * LDK);
-    else pn_store<PT>(hv, s.hs);
-    if (n0 + NS < p.N) {
-      n = n0 + NS + wave * 16 + cm;
+    if (n0 + STEP < p.N) {
+      n = n0 + STEP + wave * 16 + cm;
       vn = FULL || n < p.N;
-      rm = make_rowmap<FULL>(p, u, g4, n0 + NS);
+      rm = make_rowmap<FULL>(p, u, g4, n0 + STEP);
       lane_load_ln<DTB>(p.dt, u.b, u.h, n, vn, g4, rm, raw);
       cf = lane_coef(p, u.h, n, vn);
       lane_load_ln<IOB>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, cv);
-      pn_load<PT, FULL>(p, hsrc, n0 + NS, hv);
+      pn_load<PT, FULL>(p, hsrc, n0 + STEP, hv, tid);
     }
     __syncthreads();
     // y[l][p] += sum_n Ct[l][n] H[p][n]; wave owns 16 rows
-    if constexpr (IOB) {
+    if (!mine) {
+    } else if constexpr (IOB) {
       // bf16 inputs: one rounding of C exp(cs) and of the entry state to bf16 (the reference stores the entry states
       // in the input dtype and casts its dot operands, issm_combined.py:87, issm_chunk_scan.py:149-190)
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const bf8 a = op_frag<LDK>(s.ct, wave * 16 + cm, g4, t);
+        const bf8 a = op_frag<LDK>(ct, wave * 16 + cm, g4, t);
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) acc[pt] = mfma_bf(a, op_frag<LDK>(s.hs, pt * 16 + cm, g4, t), acc[pt]);
+        for (int pt = 0; pt < PT; ++pt) acc[pt] = mfma_bf(a, op_frag<LDK>(hs, pt * 16 + cm, g4, t), acc[pt]);
       }
     } else if constexpr (SM::SPL) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        const bf8 ah = op_frag<LDK>(s.ct, wave * 16 + cm, g4, t), al = op_frag<LDK>(s.ct + CS * LDK, wave * 16 + cm, g4, t);
+        const bf8 ah = op_frag<LDK>(ct, wave * 16 + cm, g4, t), al = op_frag<LDK>(ct + CS * LDK, wave * 16 + cm, g4, t);
 #pragma unroll
         for (int pt = 0; pt < PT; ++pt)
-          acc[pt] = mfma_split(ah, al, op_frag<LDK>(s.hs, pt * 16 + cm, g4, t),
-                               op_frag<LDK>(s.hs + PT * 16 * LDK, pt * 16 + cm, g4, t), acc[pt]);
+          acc[pt] = mfma_split(ah, al, op_frag<LDK>(hs, pt * 16 + cm, g4, t),
+                               op_frag<LDK>(hs + PT * 16 * LDK, pt * 16 + cm, g4, t), acc[pt]);
       }
     } else {
 #pragma unroll
       for (int kb = 0; kb < NS; kb += 16)
 #pragma unroll
-        for (int pt = 0; pt < PT; ++pt) mma16_mm(acc[pt], s.ct, LDN, wave * 16, s.hs, LDN, pt * 16, kb, lane);
+        for (int pt = 0; pt < PT; ++pt) mma16_mm(acc[pt], ct, LDN, wave * 16, hs, LDN, pt * 16, kb, lane);
     }
     __syncthreads();
   }
@@ -186,37 +197,50 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   // M of this wave's 16 rows goes straight into matrix-operand registers (lane (row cm, group g4) holds columns
   // 16 kb + 4 g4 .. + 3 of the blocks kb <= wave, the upper triangle of the diagonal block zeroed): no LDS tile, which
   // lets a fourth workgroup live on the CU
-  f4 mf[4];
-  {
-    const float* mrow = cabt + sq_off(p, u.bt, u.c, u.h) + (wave * 16 + cm) * CS + 4 * g4;
+  if (grp == NG - 1) {
+    f4 mf[4];
+    {
+      const float* mrow = cabt + sq_off(p, u.bt, u.c, u.h) + (wave * 16 + cm) * CS + 4 * g4;
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) mf[kb] = *(const f4*)(mrow + 16 * min(kb, wave));  // no branch between the loads
+      for (int kb = 0; kb < 4; ++kb) mf[kb] = *(const f4*)(mrow + 16 * min(kb, wave));  // no branch between the loads
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (kb > wave || (kb == wave && 4 * g4 + j > cm)) mf[kb][j] = 0.0f;
+    }
+    // y[l][p] += sum_{s<=l} M[l][s] x[s][p]; rows of this wave only need s < 16(wave+1)
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
+      if (kb <= wave) {  // uniform
+        // the lane's four M values and four x values are the operands of one K = 16 bf16 instruction as they stand
+        // (k-slot j of lane group g4 <-> row 16 kb + 4 g4 + j), M as a (hi, lo) pair and, for fp32 inputs, x too
+        const float mw[4] = {mf[kb][0], mf[kb][1], mf[kb][2], mf[kb][3]};
+        bf4 ah, al;
+        split4(mw, ah, al);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (kb > wave || (kb == wave && 4 * g4 + j > cm)) mf[kb][j] = 0.0f;
-  }
-  // y[l][p] += sum_{s<=l} M[l][s] x[s][p]; rows of this wave only need s < 16(wave+1)
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb)
-    if (kb <= wave) {  // uniform
-      // the lane's four M values and four x values are the operands of one K = 16 bf16 instruction as they stand
-      // (k-slot j of lane group g4 <-> row 16 kb + 4 g4 + j), M as a (hi, lo) pair and, for fp32 inputs, x too
-      const float mw[4] = {mf[kb][0], mf[kb][1], mf[kb][2], mf[kb][3]};
-      bf4 ah, al;
-      split4(mw, ah, al);
-#pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        const float* bp = s.xs + XT::at(16 * kb + 4 * g4, pt * 16 + cm);
-        const float xw[4] = {bp[0], bp[LDX], bp[2 * LDX], bp[3 * LDX]};
-        bf4 bh, bl;
-        split4(xw, bh, bl);
-        acc[pt] = mfma_bf16k(al, bh, acc[pt]);
-        if constexpr (!IOB) acc[pt] = mfma_bf16k(ah, bl, acc[pt]);  // (bf16 inputs: x is exact, its lo part zero)
-        acc[pt] = mfma_bf16k(ah, bh, acc[pt]);
+        for (int pt = 0; pt < PT; ++pt) {
+          const float* bp = s.xs + XT::at(16 * kb + 4 * g4, pt * 16 + cm);
+          const float xw[4] = {bp[0], bp[LDX], bp[2 * LDX], bp[3 * LDX]};
+          bf4 bh, bl;
+          split4(xw, bh, bl);
+          acc[pt] = mfma_bf16k(al, bh, acc[pt]);
+          if constexpr (!IOB) acc[pt] = mfma_bf16k(ah, bl, acc[pt]);  // (bf16 inputs: x is exact, its lo part zero)
+          acc[pt] = mfma_bf16k(ah, bh, acc[pt]);
+        }
       }
+  }
+  if constexpr (NG > 1) {
+    f4* part = (f4*)s.ct;
+    if (grp) {
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt) part[pt * NTHREADS + tid] = acc[pt];
     }
+    __syncthreads();
+    if (grp) return;
+#pragma unroll
+    for (int pt = 0; pt < PT; ++pt) acc[pt] += part[pt * NTHREADS + tid];
+  }
 
   const TensorD& to = p.out[u.dir];
   const TensorD& tz = p.z[u.dir];
@@ -246,9 +270,9 @@ __device__ __forceinline__ void k_chunk_scan_body(const KP& p, const float* __re
   }
 }
 // two head tiles, fp32 inputs or edges: 128 registers, so that a fourth workgroup lives on the CU (52 -> 48.5 us)
-template <int PT, bool IOB, bool DTB, bool FULL>
-__global__ __launch_bounds__(NTHREADS, (PT <= 2 && (!IOB || !FULL)) ? 4 : 1) void k_chunk_scan(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
-  k_chunk_scan_body<PT, IOB, DTB, FULL>(p, states, cabt, out_x);
+template <int PT, bool IOB, bool DTB, bool FULL, int NG>
+__global__ __launch_bounds__(NG * NTHREADS, (PT <= 2 && NG == 1 && (!IOB || !FULL)) ? 4 : 1) void k_chunk_scan(KP p, const float* __restrict__ states, const float* __restrict__ cabt, float* __restrict__ out_x) {
+  k_chunk_scan_body<PT, IOB, DTB, FULL, NG>(p, states, cabt, out_x);
 }
 
 // ------------------------------------------------------------------- launchers
@@ -277,10 +301,17 @@ int launch_chunk_local(const KP& p, float* states, float* cs_last, float* cabt, 
 int launch_chunk_scan(const KP& p, const float* states, const float* cabt, float* out_x, hipStream_t st) {
   const int units = p.B * p.ndir * p.nc * p.H;
   ISSM_DISPATCH(p, {
-    const size_t sm = sizeof(FwdScanSmem<PT_, IOB_>);
-    constexpr auto kern = &k_chunk_scan<PT_, IOB_, DTB_, FULL_>;
-    if (int e = set_lds(kern, sm)) return e;
-    hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cabt, out_x);
+    if (two_groups(units, p.N)) {
+      const size_t sm = sizeof(FwdScanSmem<PT_, IOB_, 2>);
+      constexpr auto kern = &k_chunk_scan<PT_, IOB_, DTB_, FULL_, 2>;
+      if (int e = set_lds(kern, sm)) return e;
+      hipLaunchKernelGGL(kern, dim3(units), dim3(2 * NTHREADS), sm, st, p, states, cabt, out_x);
+    } else {
+      const size_t sm = sizeof(FwdScanSmem<PT_, IOB_, 1>);
+      constexpr auto kern = &k_chunk_scan<PT_, IOB_, DTB_, FULL_, 1>;
+      if (int e = set_lds(kern, sm)) return e;
+      hipLaunchKernelGGL(kern, dim3(units), dim3(NTHREADS), sm, st, p, states, cabt, out_x);
+    }
   });
   return (int)hipGetLastError();
 }

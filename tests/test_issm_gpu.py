@@ -1595,3 +1595,24 @@ def test_bf16_forward_of_the_steps_behind_a_far_tile(L_, P, N, far):
     torch.cuda.synchronize()
     for name, got, want, size in (("y", y, ref[0][0], ref[1][0]), ("last", last, ref[0][1], ref[1][1])):
         assert ((got.double().cpu() - want).abs() <= 4 * 2.0 ** -9 * 1.125 * size + 1e-30).all(), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,P,gated", [(256, 128, 32, False), (256, 192, 36, False), (250, 130, 64, True), (200, 65, 16, True), (70, 330, 48, False)])
+def test_outputs_by_one_and_by_two_groups_of_waves(dtype, L_, N, P, gated):
+    """y and dx of scenes few enough for two groups of waves a workgroup, with an even and an odd number of slices of the states, against
+    the same scenes in a batch too large for that.  They differ in the order in which the slices' sums are added: a rounding of a
+    partial sum a slice, and one of the result in bf16."""
+    H = 4
+    few, copies = 2, -(-260 // (2 * H * (-(-L_ // 64))))
+    d = _problem(few, L_, H, P, N, 1, seed=L_ + N + P, D="hp", z=gated)
+    big = {k: v.repeat(copies, *([1] * (v.dim() - 1))) if torch.is_tensor(v) and k not in ("A", "D", "dt_bias") else v for k, v in d.items()}
+    assert few * H * (-(-L_ // 64)) <= 256 < few * copies * H * (-(-L_ // 64))
+    y, _, g, _ = _run_operator(d, dtype)
+    yb, _, gb, _ = _run_operator(big, dtype)
+    slices = -(-N // 64)
+    for got, want in ((y, yb[:few]), (g["x"], gb["x"][:few])):
+        got, want = got.detach().double(), want.detach().double()
+        bound = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24 * 4 * (slices + 2)
+        assert (got - want).norm() <= bound * want.norm()
+        assert torch.isfinite(got).all()
