@@ -15,43 +15,20 @@
 //   dw[s][c][j] = sum_{b,l} dpre[s][b][l][c] u[b][l + j - 3][c],   dbias[s][c] = sum_{b,l} dpre[s][b][l][c],
 // the last two as per-thread partials (one per (b, token tile)) summed in fixed order by a second kernel.
 // Everything is memory bound; arithmetic is fp32.
-#include "issm_dev.h"
+#include "dwconv_dev.h"
 
 namespace issm {
 
-constexpr int DW_TAPS = 7;
 // Tokens per thread, DW_TL.  Backward: 16, but 8 for the chained one, which holds 61 values of its rows and halo per 8 tokens and
 // at 16 needed 272 registers, one wave a SIMD: 8 x 1024 tokens, 290 channels, bf16: 39 us with 16, 25 with 8, 32 with 4 (more
 // halo read twice).  Forward: the most of 16, 8 and 4 that makes two waves a SIMD: one scene of 1024 tokens makes 290 waves of 16
 // (9.4, 7.7 and 5.5 us with 16, 8 and 4), 16 x 4096 tokens pay for the halo (73 us chained with 16, 102 with 4).
 constexpr int DW_BWD = 16, DW_CHAIN_BWD = 8;
 
-template <bool BF>
-__device__ __forceinline__ float dw_ld(const void* p, long i) {
-  return BF ? bf16_to_f(((const uint16_t*)p)[i]) : ((const float*)p)[i];
-}
-template <bool BF>
-__device__ __forceinline__ void dw_st(void* p, long i, float v) {
-  if (BF) ((uint16_t*)p)[i] = f_to_bf16(v); else ((float*)p)[i] = v;
-}
-
-// thread -> (b, tile, c), c fastest
-template <int DW_TL>
-__device__ __forceinline__ bool dw_item(const DwConvP& p, int& b, int& l0, int& c) {
-  const long id = (long)blockIdx.x * NTHREADS + threadIdx.x;
-  const int ntile = (p.L + DW_TL - 1) / DW_TL;
-  if (id >= (long)p.B * ntile * p.C) return false;
-  c = (int)(id % p.C);
-  const long r = id / p.C;
-  l0 = (int)(r % ntile) * DW_TL;
-  b = (int)(r / ntile);
-  return true;
-}
-
 template <bool BF, int S, int DW_TL>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_fwd(DwConvP p) {
   int b, l0, c;
-  if (!dw_item<DW_TL>(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, (long)blockIdx.x * NTHREADS + threadIdx.x, p.C, b, l0, c)) return;
   float w[S][DW_TAPS], bias[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
@@ -98,7 +75,7 @@ template <bool BF, int S>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_bwd(DwConvP p) {
   constexpr int DW_TL = DW_BWD;
   int b, l0, c;
-  if (!dw_item<DW_TL>(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, (long)blockIdx.x * NTHREADS + threadIdx.x, p.C, b, l0, c)) return;
   float w[S][DW_TAPS];
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -177,73 +154,16 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_bwd(DwConvP p) {
 }
 
 // ---- chained pair: set 1 convolves set 0's output (rounded to the I/O dtype, as it is stored)
-template <bool BF>
-__device__ __forceinline__ float dw_round(float v) { return BF ? bf16_to_f(f_to_bf16(v)) : v; }
-
-// output / gradient address of (set s, row, channel c) with or without the channel split
-__device__ __forceinline__ long dw_out_off(const DwConvP& p, long row, int c, bool& head) {
-  head = p.split <= 0 || c < p.split;
-  if (p.split <= 0) return row * p.C + c;
-  return head ? row * p.split + c : row * (p.C - p.split) + (c - p.split);
-}
-
 template <bool BF, int DW_TL>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd(DwConvP p) {
-  int b, l0, c;
-  if (!dw_item<DW_TL>(p, b, l0, c)) return;
-  float w[2][DW_TAPS], bias[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-#pragma unroll
-    for (int j = 0; j < DW_TAPS; ++j) w[s][j] = p.w[((long)s * p.C + c) * DW_TAPS + j];
-    bias[s] = p.bias[(long)s * p.C + c];
-  }
-  const long ub = (long)b * p.u_bs + c;
-  constexpr int W1 = DW_TL + DW_TAPS - 1, W2 = W1 + DW_TAPS - 1;
-  float ub_[W2];  // u[l0 - 6 .. l0 + DW_TL + 5]
-#pragma unroll
-  for (int j = 0; j < W2; ++j) {
-    const int l = l0 + j - 6;
-    const float v = dw_ld<BF>(p.u, ub + (long)min(max(l, 0), p.L - 1) * p.u_ls);
-    ub_[j] = (l >= 0 && l < p.L) ? v : 0.0f;
-  }
-  float pre0[W1], y0[W1];  // rows l0 - 3 .. l0 + DW_TL + 2
-#pragma unroll
-  for (int j = 0; j < W1; ++j) {
-    const int l = l0 + j - 3;
-    float a = bias[0];
-#pragma unroll
-    for (int t = 0; t < DW_TAPS; ++t) a = fmaf(w[0][t], ub_[j + t], a);
-    a = dw_round<BF>(a);
-    pre0[j] = a;
-    y0[j] = (l >= 0 && l < p.L) ? dw_round<BF>(a * sigmoidf_(a)) : 0.0f;
-  }
-#pragma unroll
-  for (int i = 0; i < DW_TL; ++i) {
-    const int l = l0 + i;
-    if (l < p.L) {
-      float a = bias[1];
-#pragma unroll
-      for (int t = 0; t < DW_TAPS; ++t) a = fmaf(w[1][t], y0[i + t], a);
-      a = dw_round<BF>(a);
-      const float y1 = a * sigmoidf_(a);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const long row = ((long)s * p.B + b) * p.L + l;
-        dw_st<BF>(p.pre, row * p.C + c, s ? a : pre0[i + 3]);
-        bool head;
-        const long o = dw_out_off(p, row, c, head);
-        dw_st<BF>(head ? p.y : p.y_tail, o, s ? y1 : y0[i + 3]);
-      }
-    }
-  }
+  dw_chain_fwd<BF, DW_TL, true>(p, (long)blockIdx.x * NTHREADS + threadIdx.x);
 }
 
 template <bool BF>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_bwd(DwConvP p) {
   constexpr int DW_TL = DW_CHAIN_BWD;
   int b, l0, c;
-  if (!dw_item<DW_TL>(p, b, l0, c)) return;
+  if (!dw_item<DW_TL>(p, (long)blockIdx.x * NTHREADS + threadIdx.x, p.C, b, l0, c)) return;
   float w[2][DW_TAPS];
 #pragma unroll
   for (int s = 0; s < 2; ++s)

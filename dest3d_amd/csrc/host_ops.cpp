@@ -1011,10 +1011,10 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                                            &A_log, &D};
     const int64_t nflat = CoreFn::offsets(arrays, off);
     const Tensor d = cast(dist, at::kBFloat16).contiguous(), wt = f32c(wts);
-    enum { ZX, H0, FLAT, A1, X, TAIL, PRE, DT, BC, Y, LAST, KEY, QUERY, WS, PARTS };
-    const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di, 8 * B * Ln * G, 4 * B * Ln * Cc,
-                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di,
-                                  8 * B * di * K, 2 * B * Ln * di, 2 * B * K * di, (int64_t)ws_bytes};
+    enum { ZX, H0, FLAT, A1, X, DT, BC, Y, LAST, KEY, QUERY, WS, PARTS };
+    const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di,
+                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di, 8 * B * di * K,
+                                  2 * B * Ln * di, 2 * B * K * di, (int64_t)ws_bytes};
     int64_t at_[PARTS + 1] = {0};
     for (int i = 0; i < PARTS; ++i) at_[i + 1] = at_[i] + (bytes[i] + 255) / 256 * 256;
     const Tensor arena = fresh({at_[PARTS]}, in_key, at::kByte);
@@ -1032,42 +1032,36 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     lin.job[0] = product(in_key, data(in_key), key_proj, part(ZX), 0);
     lin.job[1] = product(in_query, data(in_query), query_proj, part(H0), K);
     CoreFn::small_parameters(arrays, K, par, (float*)part(A1), stream, &lin);
-    {
-      issm_dwconv_args a{};
-      a.batch = (int32_t)B;
-      a.seqlen = (int32_t)Ln;
-      a.channels = (int32_t)Cc;
-      a.nsets = 2;
-      a.taps = TAPS;
-      a.dtype = ISSM_BF16;
-      a.u = part(ZX, 2 * di);
-      a.u_batch_stride = Ln * W;
-      a.u_token_stride = W;
-      a.chain = 1;
-      a.stream = stream;
-      a.w = par;
-      a.bias = par + off[CoreFn::CB_F];
-      a.y = part(X);
-      a.pre = part(PRE);
-      a.split = (int32_t)di;
-      a.y_tail = part(TAIL);
-      check(issm_dwconv_silu_fwd(&a), "issm_dwconv_silu_fwd");
-    }
     void* bc[4];
     for (int i = 0; i < 4; ++i) bc[i] = part(BC, i * 2 * B * Ln * G * K);
     {
+      issm_dwconv_args c{};
+      c.batch = (int32_t)B;
+      c.seqlen = (int32_t)Ln;
+      c.channels = (int32_t)Cc;
+      c.nsets = 2;
+      c.taps = TAPS;
+      c.dtype = ISSM_BF16;
+      c.u = part(ZX, 2 * di);
+      c.u_batch_stride = Ln * W;
+      c.u_token_stride = W;
+      c.chain = 1;
+      c.stream = stream;
+      c.w = par;
+      c.bias = par + off[CoreFn::CB_F];
+      c.y = part(X);
+      c.split = (int32_t)di;
       issm_pgen_args a = pgen_args(d, par + off[CoreFn::DT_W], H, G);
       a.tok = part(ZX, 2 * (di + Cc));
       a.tok_stride = W;
       a.tok_add = par + off[CoreFn::DT_BIAS];
-      a.tail = part(TAIL);
       a.dt = part(DT);
       a.Bm = bc[0];
       a.Cm = bc[1];
       a.Bm_back = bc[2];
       a.Cm_back = bc[3];
       a.weights = data<const float>(wt);
-      check(issm_param_gen_fwd_only(&a), "issm_param_gen_fwd_only");
+      check(issm_conv_param_gen_fwd(&c, &a), "issm_conv_param_gen_fwd");
     }
     s.flags = (wt.defined() ? 0u : ISSM_FLAG_DT_SOFTPLUS) | (D.dim() == 2 ? ISSM_FLAG_D_HAS_HDIM : 0u);
     s.dt_min = (float)lo;

@@ -79,6 +79,7 @@ int launch_box_dist_fwd(const BoxDistP& p, hipStream_t st);
 int launch_box_dist_bwd(const BoxDistP& p, hipStream_t st);
 int dwconv_partial_rows(int B, int L);
 int launch_dwconv_fwd(const DwConvP& p, hipStream_t st);
+int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st);
 int launch_dwconv_bwd(const DwConvP& p, hipStream_t st);
 int pgen_bwd_blocks(long tokens);
 int launch_pgen_fwd(const PGenP& p, hipStream_t st);
@@ -675,7 +676,7 @@ int issm_gated_rmsnorm_bwd_noalloc(const issm_norm_args* a) {
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_noalloc");
 }
 
-static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward_only = false) {
+static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward_only = false, bool conv = false) {
   if (!a) return fail(ISSM_E_NULL, "param_gen: args is NULL");
   if (a->tokens < 0 || a->K < 0 || a->H < 1 || a->G < 1) return fail(ISSM_E_SHAPE, "param_gen: bad shape");
   if (a->M != 16) return fail(ISSM_E_UNSUPPORTED, "param_gen: M = %d (only 16 is built)", a->M);
@@ -686,7 +687,7 @@ static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward
   if (a->weights && !a->dt_raw && !forward_only) return fail(ISSM_E_NULL, "param_gen: weights given but dt_raw is NULL");
   if (!bwd) {
     if (!a->dt || !a->Bm || !a->Cm) return fail(ISSM_E_NULL, "param_gen: dt/Bm/Cm is NULL");
-    if (!a->bias && (!a->tok || !a->tok_add || !a->tail)) return fail(ISSM_E_NULL, "param_gen: neither bias nor tok/tok_add/tail");
+    if (!a->bias && (!a->tok || !a->tok_add || (!a->tail && !conv))) return fail(ISSM_E_NULL, "param_gen: neither bias nor tok/tok_add/tail");
     if (!a->bias && a->tok_stride < a->H) return fail(ISSM_E_STRIDE, "param_gen: tok_stride %lld", (long long)a->tok_stride);
     if (a->has_back && (!a->Bm_back || !a->Cm_back)) return fail(ISSM_E_NULL, "param_gen: Bm_back/Cm_back is NULL");
   } else {
@@ -732,14 +733,14 @@ int issm_param_gen_bwd(const issm_pgen_args* a) {
   return launched(launch_pgen_bwd(p, (hipStream_t)a->stream), "param_gen_bwd");
 }
 
-static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd) {
+static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool heads_only = false) {
   if (!a) return fail(ISSM_E_NULL, "dwconv: args is NULL");
   if (a->batch < 0 || a->seqlen < 0 || a->channels < 1) return fail(ISSM_E_SHAPE, "dwconv: bad shape");
   if (a->taps != 7) return fail(ISSM_E_UNSUPPORTED, "dwconv: %d taps (only 7 is built)", a->taps);
   if (a->nsets < 1 || a->nsets > 2) return fail(ISSM_E_UNSUPPORTED, "dwconv: nsets = %d (1 or 2)", a->nsets);
   if (a->chain && a->nsets != 2) return fail(ISSM_E_SHAPE, "dwconv: chain needs nsets = 2, got %d", a->nsets);
   if (a->dtype != ISSM_F32 && a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "dwconv: dtype %d", a->dtype);
-  if (!a->u || !a->w || !a->pre) return fail(ISSM_E_NULL, "dwconv: u/w/pre is NULL");
+  if (!a->u || !a->w || (!a->pre && !heads_only)) return fail(ISSM_E_NULL, "dwconv: u/w/pre is NULL");
   if (a->u_token_stride < a->channels || a->u_batch_stride < 0)
     return fail(ISSM_E_STRIDE, "dwconv: u strides (%lld, %lld)", (long long)a->u_batch_stride, (long long)a->u_token_stride);
   if (!bwd && (!a->bias || !a->y)) return fail(ISSM_E_NULL, "dwconv: bias/y is NULL");
@@ -748,7 +749,7 @@ static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd) {
   p->chain = a->chain ? 1 : 0;
   p->u = a->u; p->u_bs = a->u_batch_stride; p->u_ls = a->u_token_stride;
   if (a->split < 0 || a->split >= a->channels) return fail(ISSM_E_SHAPE, "dwconv: split %d outside [0, channels)", a->split);
-  if (a->split > 0 && !bwd && !a->y_tail) return fail(ISSM_E_NULL, "dwconv: y_tail is NULL");
+  if (a->split > 0 && !bwd && !a->y_tail && !heads_only) return fail(ISSM_E_NULL, "dwconv: y_tail is NULL");
   p->split = a->split; p->y_tail = a->y_tail;
   p->dy_tail[0] = a->dy_tail[0]; p->dy_tail[1] = a->nsets > 1 ? a->dy_tail[1] : nullptr;
   p->w = a->w; p->bias = a->bias; p->y = a->y; p->pre = a->pre;
@@ -772,6 +773,22 @@ int issm_dwconv_silu_fwd(const issm_dwconv_args* a) {
   if (rc) return rc;
   if (p.B == 0 || p.L == 0) return ISSM_OK;
   return launched(launch_dwconv_fwd(p, (hipStream_t)a->stream), "dwconv_silu_fwd");
+}
+
+int issm_conv_param_gen_fwd(const issm_dwconv_args* a, const issm_pgen_args* b) {
+  DwConvP c;
+  PGenP p;
+  int rc = dwconv_params(a, &c, false, true);
+  if (rc || (rc = pgen_params(b, &p, false, true, true))) return rc;
+  if (c.dtype != ISSM_BF16 || p.dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "conv_param_gen: dtypes %d, %d (bf16 only)", c.dtype, p.dtype);
+  if (!c.chain || p.bias || !p.has_back || c.split < 1 || c.C - c.split != 2 * p.G || p.tokens != (long)c.B * c.L)
+    return fail(ISSM_E_SHAPE, "conv_param_gen: the two do not belong together (chain %d, split %d of %d, G %d, %lld and %d x %d tokens)",
+                c.chain, c.split, c.C, p.G, (long long)p.tokens, c.B, c.L);
+  if (p.tokens > 0x7fffffff) return fail(ISSM_E_SHAPE, "conv_param_gen: too large");
+  if (p.tokens == 0) return ISSM_OK;
+  if (p.K == 0) return fail(ISSM_E_SHAPE, "conv_param_gen: K = 0");
+  p.dt_raw = nullptr;
+  return launched(launch_conv_pgen(c, p, (hipStream_t)a->stream), "conv_param_gen_fwd");
 }
 
 int issm_dwconv_silu_bwd(const issm_dwconv_args* a) {

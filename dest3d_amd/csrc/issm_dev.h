@@ -524,6 +524,26 @@ __device__ __forceinline__ void lp_store_bf(const float (&v)[CS * PT * 16 / NTHR
   }
 }
 
+// The same (see warm_args) for a kernel whose first BYTES bytes of arguments are other blocks.
+template <int BYTES>
+__device__ __forceinline__ void warm_first() {
+  static_assert(BYTES > 3 * 64 && BYTES <= 9 * 64, "four to nine lines");
+  unsigned t;
+  const auto args = __builtin_amdgcn_kernarg_segment_ptr();
+#define ISSM_WARM_4 "s_load_dword %0, %1, 0x0\ns_load_dword %0, %1, 0x40\ns_load_dword %0, %1, 0x80\ns_load_dword %0, %1, 0xc0\n"
+#define ISSM_WARM(lines_) asm volatile(ISSM_WARM_4 lines_ "s_waitcnt lgkmcnt(0)" : "=&s"(t) : "s"(args))
+#define ISSM_WARM_AT(at_) "s_load_dword %0, %1, " at_ "\n"
+  if constexpr (BYTES <= 4 * 64) ISSM_WARM("");
+  else if constexpr (BYTES <= 5 * 64) ISSM_WARM(ISSM_WARM_AT("0x100"));
+  else if constexpr (BYTES <= 6 * 64) ISSM_WARM(ISSM_WARM_AT("0x100") ISSM_WARM_AT("0x140"));
+  else if constexpr (BYTES <= 7 * 64) ISSM_WARM(ISSM_WARM_AT("0x100") ISSM_WARM_AT("0x140") ISSM_WARM_AT("0x180"));
+  else if constexpr (BYTES <= 8 * 64) ISSM_WARM(ISSM_WARM_AT("0x100") ISSM_WARM_AT("0x140") ISSM_WARM_AT("0x180") ISSM_WARM_AT("0x1c0"));
+  else ISSM_WARM(ISSM_WARM_AT("0x100") ISSM_WARM_AT("0x140") ISSM_WARM_AT("0x180") ISSM_WARM_AT("0x1c0") ISSM_WARM_AT("0x200"));
+#undef ISSM_WARM_AT
+#undef ISSM_WARM
+#undef ISSM_WARM_4
+}
+
 // Every line of a kernel's KP into the scalar cache at once.  Left to itself a kernel waits for one part of it after the other, six or
 // seven times in front of its first request, and on a CU that has not run it just before each wait is a trip to the L2.  2 x 1024
 // tokens, 8 heads x 32, 256 states, forward, one workgroup a CU: k_local_tile 18.4 -> 17.6 us, k_chunk_scan 13.5 -> 13.2, k_state_pass 6.9 -> 6.5;

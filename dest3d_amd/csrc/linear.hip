@@ -90,6 +90,7 @@ __global__ __launch_bounds__(NTHREADS) void k_linear(LinearP p) {
 // (Compiled without -ffast-math for its exp.)
 template <int N>
 __global__ __launch_bounds__(NTHREADS) void k_layer_in(LinearP p, LayerParamsP q) {
+  warm_first<sizeof(LinearP) + sizeof(LayerParamsP)>();
   if ((int)blockIdx.x >= p.blocks1) return layer_params_entry(q, ((int)blockIdx.x - p.blocks1) * NTHREADS + threadIdx.x);
   const bool second = (int)blockIdx.x >= p.blocks0;
   const LinearJob& j = p.job[second ? 1 : 0];

@@ -8,7 +8,7 @@
 // M = 16: launch- and layout-bound.  Here one pass reads `dist` once and writes every output; the backward is
 // one pass as well (ddist, per-token bias gradients, per-workgroup partials of dW) plus a fixed-order
 // reduction of the partials.  Everything is memory bound; arithmetic is fp32.
-#include "issm_dev.h"
+#include "dwconv_dev.h"
 
 namespace issm {
 
@@ -102,32 +102,44 @@ __device__ __forceinline__ void stv(void* p, long i, const float (&v)[KV]) {
 // reading the gathered copy 35.
 // RAW: dt before softplus and weight is kept for the backward where there are weights (a scene of 1024 tokens x 256: 10.4 us,
 // 9.5 without).
-template <bool BF, int KV, bool TOK, bool RAW>
-__global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
+// CONV: B and C's biases are the convolutions' outputs for the last 2G channels, computed here from their inputs.
+template <bool BF, int KV, bool TOK, bool RAW, bool CONV>
+__device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, int block) {
   const int R0 = p.H + 2 * p.G, R = R0 + (p.has_back ? 2 * p.G : 0);
   const int per_tok = (p.K + KV - 1) / KV;  // threads per token
-  const long gid = (long)blockIdx.x * NTHREADS + threadIdx.x;
+  const long gid = (long)block * NTHREADS + threadIdx.x;
   const long t = gid / per_tok;
   const int k = (int)(gid % per_tok) * KV;
   extern __shared__ float tok_bias[];   // TOK: (tokens of the workgroup, R), rows as in p.bias
-  const long t0 = (long)blockIdx.x * NTHREADS / per_tok;
+  const long t0 = (long)block * NTHREADS / per_tok;
+  float d[KV][PG_M], wk[KV];
+  auto request = [&](long tt) {
+#pragma unroll
+    for (int j = 0; j < KV; ++j) load_row16<BF>(p.dist, (tt * p.K + k + j) * PG_M, d[j]);
+#pragma unroll
+    for (int j = 0; j < KV; ++j) wk[j] = p.weights ? p.weights[tt * p.K + k + j] : 1.0f;
+  };
+  if constexpr (CONV) request(min(t, p.tokens - 1));   // (under way while the first wave convolves)
   if constexpr (TOK) {
-    const long t1 = min(((long)(blockIdx.x + 1) * NTHREADS - 1) / per_tok, p.tokens - 1);
+    const long t1 = min(((long)(block + 1) * NTHREADS - 1) / per_tok, p.tokens - 1);
     const int n = (int)(t1 - t0 + 1) * R;
     for (int e = threadIdx.x; e < n; e += NTHREADS) {
       const int tl = e / R, r = e - tl * R, i = r - p.H, set = i >= 2 * p.G ? 1 : 0;
-      tok_bias[e] = r < p.H ? ld1<BF>(p.tok, (t0 + tl) * p.tok_stride + r) + p.tok_add[r]
-                            : ld1<BF>(p.tail, (set * p.tokens + t0 + tl) * (2 * p.G) + i - set * 2 * p.G);
+      if (r < p.H) {
+        tok_bias[e] = ld1<BF>(p.tok, (t0 + tl) * p.tok_stride + r) + p.tok_add[r];
+      } else if constexpr (CONV) {
+        if (set == 0) {   // (its lane has the second set's value too)
+          const int at = (int)(t0 + tl);
+          dw_chain_at<BF>(conv, at / conv.L, at % conv.L, conv.split + i, tok_bias[e], tok_bias[e + 2 * p.G]);
+        }
+      } else {
+        tok_bias[e] = ld1<BF>(p.tail, (set * p.tokens + t0 + tl) * (2 * p.G) + i - set * 2 * p.G);
+      }
     }
     __syncthreads();
   }
   if (t >= p.tokens) return;
-  float d[KV][PG_M];
-#pragma unroll
-  for (int j = 0; j < KV; ++j) load_row16<BF>(p.dist, (t * p.K + k + j) * PG_M, d[j]);
-  float wk[KV];
-#pragma unroll
-  for (int j = 0; j < KV; ++j) wk[j] = p.weights ? p.weights[t * p.K + k + j] : 1.0f;
+  if constexpr (!CONV) request(t);
   // the token's biases, all requested before the row loop (a load per row inside it would be waited for row by
   // row); bb: the reversed-order pair's bias of a B / C row
   float bv[PG_MAXR0], bb[PG_MAXR0];
@@ -172,6 +184,22 @@ __global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
       }
     }
   }
+}
+
+template <bool BF, int KV, bool TOK, bool RAW>
+__global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
+  pgen_fwd<BF, KV, TOK, RAW, false>(p, DwConvP{}, blockIdx.x);
+}
+
+// What lies between a layer's first projections and its scan where no gradient is asked for, one launch: the generation above and,
+// in the workgroups behind it, the convolutions of x.  The two took 9.5 and 5.6 us one after the other at a scene of 1024 tokens,
+// 256 queries, 288 channels, each bound by its launch and a trip or two to memory; each token's 2G channels that the generation
+// needs of the convolutions are computed by its own workgroup (13 inputs and 56 multiply-adds a channel).
+template <int KV, int TL>
+__global__ __launch_bounds__(NTHREADS) void k_conv_pgen(PGenP p, DwConvP c, int pgen_blocks) {
+  warm_first<sizeof(PGenP) + sizeof(DwConvP)>();
+  if ((int)blockIdx.x >= pgen_blocks) dw_chain_fwd<true, TL, false>(c, (long)((int)blockIdx.x - pgen_blocks) * NTHREADS + threadIdx.x);
+  else pgen_fwd<true, KV, true, false, true>(p, c, blockIdx.x);
 }
 
 // Gradient row r of token t: dt heads, then B groups, then C groups (`back`: the reversed-order pair, which
@@ -530,19 +558,25 @@ __global__ __launch_bounds__(NTHREADS) void k_pgen_dw(PGenP p) {
 
 int pgen_bwd_blocks(long tokens) { return (int)((tokens + PG_TOK - 1) / PG_TOK); }
 
-int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
-  // adjacent outputs go out as one store: K a multiple of the group and every output 16-byte aligned
+// adjacent outputs go out as one store: K a multiple of the group and every output 16-byte aligned
+static int pgen_group(const PGenP& p) {
   uintptr_t bits = 0;
   for (const void* q : {(const void*)p.dt, (const void*)p.dt_raw, (const void*)p.Bm, (const void*)p.Cm, (const void*)p.Bb,
                         (const void*)p.Cb})
     bits |= (uintptr_t)q;
   const bool al = (bits & 15) == 0;
   // (four adjacent k per thread, 8-byte bf16 stores, measured slower: 42 us against 39 at 8192 tokens x 256)
-  const int kv = (p.K % 2 == 0 && al) ? 2 : 1;
-  const long threads = p.tokens * ((p.K + kv - 1) / kv);
-  const unsigned blocks = (unsigned)((threads + NTHREADS - 1) / NTHREADS);
-  const int per_tok = (p.K + kv - 1) / kv, R = p.H + (p.has_back ? 4 : 2) * p.G;
-  const size_t lds = p.bias ? 0 : ((NTHREADS - 1) / per_tok + 2) * (size_t)R * sizeof(float);   // at most 23 KB
+  return (p.K % 2 == 0 && al) ? 2 : 1;
+}
+static size_t pgen_lds(const PGenP& p, int per_tok) {
+  const int R = p.H + (p.has_back ? 4 : 2) * p.G;
+  return p.bias ? 0 : ((NTHREADS - 1) / per_tok + 2) * (size_t)R * sizeof(float);   // at most 23 KB
+}
+
+int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
+  const int kv = pgen_group(p), per_tok = (p.K + kv - 1) / kv;
+  const unsigned blocks = (unsigned)((p.tokens * per_tok + NTHREADS - 1) / NTHREADS);
+  const size_t lds = pgen_lds(p, per_tok);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), lds, st, p); };
   const bool raw = !p.weights || p.dt_raw;
   auto forms = [&](auto two, auto one, auto two_only, auto one_only) { raw ? go(kv == 2 ? two : one) : go(kv == 2 ? two_only : one_only); };
@@ -553,6 +587,22 @@ int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
     if (p.dtype) forms(&k_pgen_fwd<true, 2, true, true>, &k_pgen_fwd<true, 1, true, true>, &k_pgen_fwd<true, 2, true, false>, &k_pgen_fwd<true, 1, true, false>);
     else forms(&k_pgen_fwd<false, 2, true, true>, &k_pgen_fwd<false, 1, true, true>, &k_pgen_fwd<false, 2, true, false>, &k_pgen_fwd<false, 1, true, false>);
   }
+  return (int)hipGetLastError();
+}
+
+int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st) {
+  const int kv = pgen_group(p), per_tok = (p.K + kv - 1) / kv;
+  const long gen = (p.tokens * per_tok + NTHREADS - 1) / NTHREADS;
+  // tokens a thread of the convolutions: as few as leave two waves a SIMD (see there)
+  auto items = [&](int tokens) { return (long)c.B * ((c.L + tokens - 1) / tokens) * c.split; };
+  const int tl = items(16) >= 2048 * 64 ? 16 : items(8) >= 2048 * 64 ? 8 : 4;
+  const long conv = (items(tl) + NTHREADS - 1) / NTHREADS;
+  if (gen + conv > 0x7fffffff) return (int)hipErrorInvalidValue;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(gen + conv)), dim3(NTHREADS), pgen_lds(p, per_tok), st, p, c, (int)gen); };
+  auto form = [&](auto two, auto one) { kv == 2 ? go(two) : go(one); };
+  if (tl == 16) form(&k_conv_pgen<2, 16>, &k_conv_pgen<1, 16>);
+  else if (tl == 8) form(&k_conv_pgen<2, 8>, &k_conv_pgen<1, 8>);
+  else form(&k_conv_pgen<2, 4>, &k_conv_pgen<1, 4>);
   return (int)hipGetLastError();
 }
 

@@ -420,6 +420,11 @@ typedef struct issm_dwconv_args {
 int issm_dwconv_partial_rows(int32_t batch, int32_t seqlen);
 int issm_dwconv_silu_fwd(const issm_dwconv_args* args);
 int issm_dwconv_silu_bwd(const issm_dwconv_args* args);
+/* issm_dwconv_silu_fwd of a chained pair and issm_param_gen_fwd_only behind it, in one launch on the convolutions' stream,
+ * ISSM_BF16, for a call that no backward follows: what the second would read from the first's y_tail is computed within (pre,
+ * y_tail and the generation's tail are neither read nor written).  channels - split has to be 2G, tokens batch * seqlen, and the
+ * reversed pair asked for (ISSM_E_SHAPE otherwise). */
+int issm_conv_param_gen_fwd(const issm_dwconv_args* convolutions, const issm_pgen_args* generation);
 
 /* ---- projections of a scene or two of tokens -------------------------------------------------
  * y = x w^T (the layer's nn.Linear without bias, models/dest_module.py:471-503) for one or two independent products in one

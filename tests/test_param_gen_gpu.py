@@ -122,3 +122,47 @@ def test_scan_params_rejects_unbuilt_shapes():
     assert lib.issm_param_gen_fwd(C.byref(a)) == -5
     a.H = 2
     assert lib.issm_param_gen_fwd(C.byref(a)) == -1
+
+
+@pytest.mark.parametrize("B,L,K,H,G,di,weighted", [(1, 1, 1, 1, 1, 2, True), (2, 9, 50, 8, 1, 288, True), (1, 37, 77, 3, 2, 36, False),
+                                                   (2, 1030, 6, 2, 1, 512, True), (1, 2051, 3, 2, 1, 520, False), (3, 5, 700, 4, 4, 64, True)])
+def test_generation_and_convolutions_in_one_launch(B, L, K, H, G, di, weighted):
+    """issm_conv_param_gen_fwd against the two launches it stands for: the same operations in the same order, so the same bits.
+    Tokens that fill no thread, workgroups of several tokens and of a part of one, 4, 8 and 16 tokens a thread of the convolutions."""
+    import ctypes as C
+    from dest3d_amd import _lib as LB
+    lib, dev, bf = LB.load(), "cuda", torch.bfloat16
+    g = torch.Generator(device=dev).manual_seed(L + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    Cc, W = di + 2 * G, 2 * di + 2 * G + H
+    zx, w, bias = rnd(B, L, W).to(bf), rnd(2, Cc, 7), rnd(2, Cc)
+    dist, pw, add, wts = rnd(B, L, K, 16).to(bf), 0.3 * rnd(H + 2 * G, 16), rnd(H), torch.rand(B, L, K, generator=g, device=dev)
+    stream = LB.current_stream_ptr(torch.device("cuda", 0))
+
+    def run(joined):
+        o = [torch.full(s, 7.0, device=dev, dtype=bf) for s in ((2, B, L, di), (2, B, L, 2 * G), (2, B, L, Cc), (B, L, H, K),
+                                                                *[(B, L, G, K)] * 4)]
+        c = LB.DwConvArgs(batch=B, seqlen=L, channels=Cc, nsets=2, taps=7, dtype=LB.ISSM_BF16, u=zx.data_ptr() + 2 * di,
+                          u_batch_stride=L * W, u_token_stride=W, w=w.data_ptr(), bias=bias.data_ptr(), y=o[0].data_ptr(),
+                          pre=None if joined else o[2].data_ptr(), stream=stream, split=di,
+                          y_tail=None if joined else o[1].data_ptr(), chain=1)
+        p = LB.PGenArgs(tokens=B * L, K=K, M=16, H=H, G=G, dtype=LB.ISSM_BF16, has_back=1, dist=dist.data_ptr(), W=pw.data_ptr(),
+                        dt=o[3].data_ptr(), Bm=o[4].data_ptr(), Cm=o[5].data_ptr(), Bm_back=o[6].data_ptr(),
+                        Cm_back=o[7].data_ptr(), weights=wts.data_ptr() if weighted else None, stream=stream,
+                        tok=zx.data_ptr() + 2 * (di + Cc), tok_stride=W, tok_add=add.data_ptr(),
+                        tail=None if joined else o[1].data_ptr())
+        if joined:
+            LB.check(lib.issm_conv_param_gen_fwd(C.byref(c), C.byref(p)), "joined")
+            for who, field, bad in ((c, "chain", 0), (c, "split", di - 1), (c, "dtype", LB.ISSM_F32), (p, "tokens", B * L + 1), (p, "has_back", 0)):
+                was = getattr(who, field)
+                setattr(who, field, bad)
+                assert lib.issm_conv_param_gen_fwd(C.byref(c), C.byref(p)) != 0, field
+                setattr(who, field, was)
+        else:
+            LB.check(lib.issm_dwconv_silu_fwd(C.byref(c)), "conv")
+            LB.check(lib.issm_param_gen_fwd_only(C.byref(p)), "generation")
+        torch.cuda.synchronize()
+        return [o[i] for i in (0, 3, 4, 5, 6, 7)]
+
+    for got, want in zip(run(True), run(False)):
+        assert torch.equal(got, want)
