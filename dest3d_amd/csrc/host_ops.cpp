@@ -1011,10 +1011,9 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                                            &A_log, &D};
     const int64_t nflat = CoreFn::offsets(arrays, off);
     const Tensor d = cast(dist, at::kBFloat16).contiguous(), wt = f32c(wts);
-    enum { ZX, H0, FLAT, A1, X, DT, BC, Y, LAST, KEY, QUERY, WS, PARTS };
+    enum { ZX, H0, FLAT, A1, X, DT, BC, Y, LAST, WS, PARTS };
     const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di,
-                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di, 8 * B * di * K,
-                                  2 * B * Ln * di, 2 * B * K * di, (int64_t)ws_bytes};
+                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di, 8 * B * di * K, (int64_t)ws_bytes};
     int64_t at_[PARTS + 1] = {0};
     for (int i = 0; i < PARTS; ++i) at_[i + 1] = at_[i] + (bytes[i] + 255) / 256 * 256;
     const Tensor arena = fresh({at_[PARTS]}, in_key, at::kByte);
@@ -1081,6 +1080,10 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     s.workspace_bytes = ws_bytes;
     s.stream = stream;
     check(issm_scan_fwd_only(&s), "issm_scan_fwd_only");
+    const Tensor out_key = fresh({B, Ln, out_key_proj.size(0)}, in_key, at::kBFloat16),
+                 out_query = fresh({B, K, out_query_proj.size(0)}, in_key, at::kBFloat16);
+    lin.job[0] = product(in_key, nullptr, out_key_proj, data(out_key), 0);
+    lin.job[1] = product(in_query, nullptr, out_query_proj, data(out_query), 0);
     {
       issm_layer_out_args a{};
       a.batch = (int32_t)B;
@@ -1096,19 +1099,12 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
       a.z_row_stride = W;
       a.key_weight = data(key_norm);
       a.key_eps = (float)(4.0 * key_eps);
-      a.key = part(KEY);
       a.query_weight = data(query_wt);
       a.query_bias = data(query_bt);
       a.query_eps = (float)query_eps;
-      a.query = part(QUERY);
       a.stream = stream;
-      check(issm_layer_out(&a), "issm_layer_out");
+      check(issm_layer_end(&a, &lin), "issm_layer_end");
     }
-    const Tensor out_key = fresh({B, Ln, out_key_proj.size(0)}, in_key, at::kBFloat16),
-                 out_query = fresh({B, K, out_query_proj.size(0)}, in_key, at::kBFloat16);
-    lin.job[0] = product(in_key, part(KEY), out_key_proj, data(out_key), 0);
-    lin.job[1] = product(in_query, part(QUERY), out_query_proj, data(out_query), 0);
-    check(issm_linear_fwd(&lin), "issm_linear_fwd");
     return {out_key, out_query};
   }
   const Tensor zx = linear_tokens(in_key, key_proj), h0 = linear_tokens(in_query, query_proj);

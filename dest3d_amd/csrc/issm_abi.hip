@@ -52,6 +52,7 @@ int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwP& p, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
+int launch_layer_end(LayerOutP& p, LinearP& q, hipStream_t st);
 int launch_box_table(const BoxTableP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
@@ -948,26 +949,54 @@ int issm_linear_dw(const issm_linear_dw_args* a) {
   return launched(launch_linear_dw(p, (hipStream_t)a->stream), "linear_dw");
 }
 
-int issm_layer_out(const issm_layer_out_args* a) {
+static int layer_out_params(const issm_layer_out_args* a, LayerOutP& p, bool norms_out) {
   if (!a) return fail(ISSM_E_NULL, "layer_out: args is NULL");
   if (a->batch < 0 || a->seqlen < 0 || a->queries < 0 || a->d_inner < 1) return fail(ISSM_E_SHAPE, "layer_out: bad shape");
   if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "layer_out: dtype %d (bf16 only)", a->dtype);
   if (a->d_inner % 4 || a->d_inner > 1024)
     return fail(ISSM_E_UNSUPPORTED, "layer_out: %d features (a multiple of 4, at most 1024)", a->d_inner);
-  LayerOutP p{};
   p.rows = (long)a->batch * a->seqlen;
   p.B = a->queries ? a->batch : 0;
   p.K = a->queries ? a->queries : 1;
-  if (p.rows == 0 && p.B == 0) return ISSM_OK;
-  if (p.rows && (!a->y[0] || !a->y[1] || !a->z || !a->key_weight || !a->key)) return fail(ISSM_E_NULL, "layer_out: y/z/key_weight/key is NULL");
+  if (p.rows && (!a->y[0] || !a->y[1] || !a->z || !a->key_weight || (norms_out && !a->key)))
+    return fail(ISSM_E_NULL, "layer_out: y/z/key_weight/key is NULL");
   if (p.rows && a->z_row_stride < a->d_inner) return fail(ISSM_E_STRIDE, "layer_out: z_row_stride %lld", (long long)a->z_row_stride);
-  if (p.B && (!a->last[0] || !a->last[1] || !a->query)) return fail(ISSM_E_NULL, "layer_out: last/query is NULL");
+  if (p.B && (!a->last[0] || !a->last[1] || (norms_out && !a->query))) return fail(ISSM_E_NULL, "layer_out: last/query is NULL");
   p.y0 = (const uint16_t*)a->y[0]; p.y1 = (const uint16_t*)a->y[1]; p.z = (const uint16_t*)a->z; p.zs = a->z_row_stride;
   p.kw = (const uint16_t*)a->key_weight; p.qw = (const uint16_t*)a->query_weight; p.qb = (const uint16_t*)a->query_bias;
   p.key = (uint16_t*)a->key; p.query = (uint16_t*)a->query;
   p.last0 = a->last[0]; p.last1 = a->last[1];
   p.di = a->d_inner; p.keps = a->key_eps; p.qeps = a->query_eps;
+  return ISSM_OK;
+}
+
+int issm_layer_out(const issm_layer_out_args* a) {
+  LayerOutP p{};
+  const int rc = layer_out_params(a, p, true);
+  if (rc || (p.rows == 0 && p.B == 0)) return rc;
   return launched(launch_layer_out(p, (hipStream_t)a->stream), "layer_out");
+}
+
+int issm_layer_end(const issm_layer_out_args* a, const issm_linear_args* b) {
+  LayerOutP p{};
+  LinearP q{};
+  const int rc = layer_out_params(a, p, false);
+  if (rc) return rc;
+  if (!b) return fail(ISSM_E_NULL, "layer_end: products is NULL");
+  if (b->njobs != 2) return fail(ISSM_E_SHAPE, "layer_end: %d products (2)", b->njobs);
+  if (b->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "layer_end: dtype %d (bf16 only)", b->dtype);
+  if (p.di % 32) return fail(ISSM_E_UNSUPPORTED, "layer_end: %d features (a multiple of 32)", p.di);
+  for (int i = 0; i < 2; ++i) {
+    const issm_linear_job& j = b->job[i];
+    const long rows = i ? (long)p.B * p.K : p.rows;
+    if (j.tokens != rows || j.in != p.di || j.out < 0 || j.out > 0x7fffffff - 128 || j.turn || rows > 0x7fffffff - 64)
+      return fail(ISSM_E_SHAPE, "layer_end: product %d of (%lld, %d) -> %d, turned by %d", i, (long long)j.tokens, j.in, j.out, j.turn);
+    const int out = rows ? j.out : 0;
+    if (out && (!j.w || !j.y)) return fail(ISSM_E_NULL, "layer_end: w/y is NULL");
+    if (out && (((uintptr_t)j.w & 15) || ((uintptr_t)j.y & 1))) return fail(ISSM_E_STRIDE, "layer_end: w must be aligned to 16 bytes, y to its elements");
+    q.job[i] = LinearJob{nullptr, (const uint16_t*)j.w, (uint16_t*)j.y, (int)rows, out, p.di / 32, 0, 0};
+  }
+  return launched(launch_layer_end(p, q, (hipStream_t)a->stream), "layer_end");
 }
 
 int issm_transpose_states(const issm_transpose_args* a) {

@@ -6,6 +6,8 @@
 // at one scene (1024 tokens, 256 queries, 288 features) the four took 15 us, this takes 6.  Bound by the launch and
 // one trip to memory; 8 queries a workgroup for 32-byte pieces of a state row and still 32 workgroups at one scene.
 // The sums and averages are rounded to bf16 as the separate kernels stored them.
+#include <algorithm>
+
 #include "issm_dev.h"
 
 namespace issm {
@@ -101,6 +103,156 @@ __global__ __launch_bounds__(NTHREADS) void k_layer_out(LayerOutP p) {
       }
     }
   }
+}
+
+// The same and the output projections behind it, one launch: a workgroup of sixteen waves takes 16 rows (or queries) through the
+// norm into LDS, a wave a row, and multiplies them with the weights of up to 256 outputs, 16 a wave, whose fragments it has asked for
+// before the rows.  The two launches took 6.0 and 5.1 us at one scene, each a trip to memory and a little arithmetic.  A few hundred
+// instructions a wave decide here: with four waves a workgroup and four rows a wave it took 10.2 us.  (The norm of a row is
+// computed once for each workgroup that shares its outputs.)  NC: 64 features each; N: fragments in flight.
+template <int NC, int N>
+__global__ __launch_bounds__(1024) void k_layer_end(LayerOutP p, LinearP q, int per_block0, int per_block1) {
+  warm_first<sizeof(LayerOutP) + sizeof(LinearP) + 8>();
+  constexpr int NV = (NC + 3) / 4, LD = NC * 64 + 8;
+  __shared__ __align__(16) uint16_t tile[16 * LD];
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4, di = p.di;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool second = (int)blockIdx.x >= p.key_blocks;
+  const int out = second ? q.job[1].out : q.job[0].out, nblk = second ? q.job[1].oblocks : q.job[0].oblocks;
+  const int per = second ? per_block1 : per_block0, steps = di / 32;   // per: 16 outputs each, of a workgroup
+  const uint16_t* wt = second ? q.job[1].w : q.job[0].w;
+  const int bid = (int)blockIdx.x - (second ? p.key_blocks : 0), tb = bid / nblk, o0 = ((bid % nblk) * per + w) * 16;
+  const bool mine = w < per && o0 < out;   // uniform
+  const bf8* wa = (const bf8*)(wt + (long)min(o0 + i, out - 1) * di) + g;
+  bf8 fa[N];
+  auto request = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) fa[u] = wa[4 * min(s0 + u, steps - 1)];
+  };
+  request(0);
+  uint16_t* row_of = tile + w * LD;
+  long out_row, rows_left;   // the workgroup's first row of the product, how many of its 16 exist
+  if (!second) {
+    out_row = (long)tb * 16;
+    rows_left = p.rows - out_row;
+    const long row = min(out_row + w, p.rows - 1);
+    f4 x[NV], z[NV], kw[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = min(4 * (lane + 64 * v), di - 4);   // (past the end: the last vector again, not counted)
+      x[v] = ld_bf4(p.y0 + row * di + c) + ld_bf4(p.y1 + row * di + c);
+      z[v] = ld_bf4(p.z + row * p.zs + c);
+      kw[v] = ld_bf4(p.kw + c);
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      x[v] = round_bf4(x[v]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[v][r] *= z[v][r] * sigmoidf_(z[v][r]);
+      if (4 * (lane + 64 * v) < di) ss += sum4(x[v] * x[v]);
+    }
+    const float rstd = 1.0f / sqrtf(wave_total(ss) / (float)di + p.keps);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = 4 * (lane + 64 * v);
+      if (c < di) st_bf4(row_of + c, x[v] * rstd * kw[v]);
+    }
+  } else {
+    const int perb = (p.K + 15) / 16, b = tb / perb, k0 = (tb % perb) * 16;
+    out_row = (long)b * p.K + k0;
+    rows_left = p.K - k0;
+    {
+      const int qi = threadIdx.x & 15, c0 = threadIdx.x >> 4;
+      const long at = (long)b * di * p.K + min(k0 + qi, p.K - 1);   // (queries past the end repeat the last and are not stored)
+      float a0[NC], a1[NC];
+#pragma unroll
+      for (int m = 0; m < NC; ++m) {
+        const long o = at + (long)min(c0 + 64 * m, di - 1) * p.K;
+        a0[m] = p.last0[o];
+        a1[m] = p.last1[o];
+      }
+#pragma unroll
+      for (int m = 0; m < NC; ++m)
+        if (c0 + 64 * m < di) tile[qi * LD + c0 + 64 * m] = f_to_bf16((a0[m] + a1[m]) * 0.5f);
+    }
+    f4 qw[NV], qb[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = min(4 * (lane + 64 * v), di - 4);
+      qw[v] = (f4){1.0f, 1.0f, 1.0f, 1.0f};
+      qb[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+      if (p.qw) qw[v] = ld_bf4(p.qw + c);   // uniform
+      if (p.qb) qb[v] = ld_bf4(p.qb + c);
+    }
+    __syncthreads();
+    f4 x[NV];
+    float s = 0.0f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = 4 * (lane + 64 * v);
+      x[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+      if (c < di) x[v] = ld_bf4(row_of + c);
+      s += sum4(x[v]);
+    }
+    const float mean = wave_total(s) / (float)di;
+    s = 0.0f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      if (4 * (lane + 64 * v) < di) {
+        x[v] -= mean;
+        s += sum4(x[v] * x[v]);
+      }
+    const float rstd = 1.0f / sqrtf(wave_total(s) / (float)di + p.qeps);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = 4 * (lane + 64 * v);
+      if (c < di) st_bf4(row_of + c, x[v] * rstd * qw[v] + qb[v]);
+    }
+  }
+  __syncthreads();
+  if (!mine) return;
+  f4 y4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s0 = 0; s0 < steps; s0 += N) {
+    if (s0) request(s0);
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (s0 + u < steps) y4 = mfma_bf(fa[u], *(const bf8*)(tile + i * LD + 32 * (s0 + u) + 8 * g), y4);   // uniform
+  }
+  if (i >= rows_left) return;
+  const int o = o0 + 4 * g;
+  uint16_t* y = (second ? q.job[1].y : q.job[0].y) + (out_row + i) * out + o;
+  if (o + 4 <= out) {
+    st_bf4(y, y4);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (o + r < out) y[r] = f_to_bf16(y4[r]);
+  }
+}
+
+int launch_layer_end(LayerOutP& p, LinearP& q, hipStream_t st) {
+  const long tiles[2] = {(p.rows + 15) / 16, (long)p.B * ((p.K + 15) / 16)}, all = tiles[0] + tiles[1];
+  long blocks[2];
+  int per[2];
+  for (int k = 0; k < 2; ++k) {
+    // the outputs of a tile of rows shared by as many workgroups as give no CU a second one, 16 outputs a wave
+    const int groups = (q.job[k].out + 15) / 16, least = (groups + 15) / 16;
+    const int want = std::max(least, (int)std::min((long)groups, all ? NCU / all : 1));
+    per[k] = want ? (groups + want - 1) / want : 1;
+    q.job[k].oblocks = (groups + per[k] - 1) / per[k];
+    blocks[k] = tiles[k] * q.job[k].oblocks;
+  }
+  if (blocks[0] + blocks[1] > 0x7fffffff) return (int)hipErrorInvalidValue;
+  if (blocks[0] + blocks[1] == 0) return 0;
+  p.key_blocks = (int)blocks[0];
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(blocks[0] + blocks[1])), dim3(1024), 0, st, p, q, per[0], per[1]); };
+  const bool nine = p.di / 32 % 9 == 0;   // nine fragments where they come out even (288 features), eight otherwise
+  if (p.di <= 256) go(&k_layer_end<4, 8>);
+  else if (p.di <= 320) nine ? go(&k_layer_end<5, 9>) : go(&k_layer_end<5, 8>);
+  else if (p.di <= 512) go(&k_layer_end<8, 8>);
+  else go(&k_layer_end<16, 4>);
+  return (int)hipGetLastError();
 }
 
 int launch_layer_out(LayerOutP& p, hipStream_t st) {

@@ -491,6 +491,10 @@ typedef struct issm_layer_out_args {
 } issm_layer_out_args;
 
 int issm_layer_out(const issm_layer_out_args* args);
+/* issm_layer_out and the two products of its results, products->job[0] of key and job[1] of query, in one launch on the stream
+ * of `args`: y = key w^T and query w^T as issm_linear_fwd computes them.  key, query and the jobs' x are neither read nor
+ * written; the jobs' tokens and in have to be those of key and query, turn 0, and d_inner a multiple of 32 (ISSM_E_UNSUPPORTED). */
+int issm_layer_end(const issm_layer_out_args* args, const issm_linear_args* products);
 
 /* ---- queries <-> scan states -----------------------------------------------------------------
  * The rearrangements around the scan in MultiHeadISSMScan.forward: queries become initial states

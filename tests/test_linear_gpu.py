@@ -250,6 +250,44 @@ def test_behind_the_scan(B, Ln, K, di, affine):
         setattr(a, field, was)
 
 
+@pytest.mark.parametrize("B,Ln,K,di,outs", [(1, 1, 1, 32, (1, 1)), (2, 9, 19, 288, (288, 288)), (1, 40, 33, 320, (130, 97)),
+                                            (3, 7, 16, 512, (33, 129)), (1, 20, 17, 1024, (128, 5)), (1, 3, 2, 576, (260, 260)),
+                                            (2, 0, 3, 288, (9, 9)), (2, 6, 0, 64, (70, 70)), (1, 17, 5, 96, (0, 31))])
+def test_norms_and_projections_behind_the_scan(B, Ln, K, di, outs):
+    """issm_layer_end against fp64 on the sums and averages rounded to bf16: rows that fill no tile, outputs that fill no wave or
+    vector, one set of fragments and several.  Bound: the norm's rounding to 8 bits in each term, and the result's own."""
+    g = torch.Generator().manual_seed(di + K)
+    r = lambda *s: torch.randn(*s, generator=g)
+    bf = lambda t: t.bfloat16().cuda()
+    y, zx, kw = [bf(r(B, Ln, di)) for _ in range(2)], bf(r(B, Ln, di + 3)), bf(r(di))
+    last, qw, qb = [r(B, di, K).cuda() for _ in range(2)], bf(r(di)), bf(r(di))
+    w, rows = [bf(r(o, di)) for o in outs], (B * Ln, B * K)
+    got = [bf(torch.full((n + 1, o), 3.0)) for n, o in zip(rows, outs)]
+    ptr = lambda t: t.data_ptr() if t.numel() else None
+    a = OutArgs(B, Ln, K, di, L.ISSM_BF16, (C.c_void_p * 2)(*map(ptr, y)), ptr(zx), di + 3, kw.data_ptr(), 4e-5, None,
+                (C.c_void_p * 2)(*map(ptr, last)), qw.data_ptr(), qb.data_ptr(), 1e-5, None,
+                L.current_stream_ptr(torch.device("cuda", 0)))
+    q = Args((Job * 2)(*[Job(None, ptr(w[i]), ptr(got[i]), rows[i], di, outs[i], 0) for i in range(2)]), 2, L.ISSM_BF16, None)
+    lib = L.load()
+    assert lib.issm_layer_end(C.byref(a), C.byref(q)) == 0
+    torch.cuda.synchronize()
+    c = lambda t: t.double().cpu()
+    z = c(zx)[..., :di]
+    v = c((y[0].float() + y[1].float()).bfloat16()) * z * torch.sigmoid(z)
+    v = (v * (v.pow(2).mean(-1, keepdim=True) + 4e-5).rsqrt() * c(kw)).reshape(-1, di)
+    s = c(((last[0] + last[1]) * 0.5).bfloat16()).transpose(1, 2).reshape(-1, di)
+    s = (s - s.mean(-1, keepdim=True)) * (s.var(-1, unbiased=False, keepdim=True) + 1e-5).rsqrt() * c(qw) + c(qb)
+    for t, x, m in zip(got, (v, s), w):
+        ref, mag = x @ c(m).t(), x.abs() @ c(m).abs().t()
+        assert ((c(t[:-1]) - ref).abs() <= 2.0 ** -8 * (ref.abs() + mag) + 2.0 ** -18 * (1 + mag)).all() and (t[-1] == 3.0).all()
+    for who, field, bad in ((a, "dtype", L.ISSM_F32), (a, "d_inner", di + 4), (q, "njobs", 1), (q.job[0], "tokens", rows[0] + 1),
+                            (q.job[1], "turn", 1), (q.job[1], "nin", di + 32)):
+        was = getattr(who, field)
+        setattr(who, field, bad)
+        assert lib.issm_layer_end(C.byref(a), C.byref(q)) != 0, field
+        setattr(who, field, was)
+
+
 @pytest.mark.parametrize("B,Ln,K", [(1, 130, 40), (2, 64, 256), (3, 1, 1)])
 @pytest.mark.parametrize("mask", [None, "weights", "drop"])
 def test_layer_without_a_gradient(B, Ln, K, mask):
