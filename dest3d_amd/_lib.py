@@ -32,7 +32,7 @@ EXPORTS = [
     "issm_dwconv_partial_rows", "issm_dwconv_silu_fwd", "issm_dwconv_silu_bwd",
     "issm_box_dist_bwd_scratch_bytes", "issm_box_dist_fwd", "issm_box_dist_bwd",
     "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states", "issm_layer_params", "issm_linear_fwd", "issm_linear_dw", "issm_linear_dw_scratch_bytes", "issm_layer_out", "issm_layer_in",
-    "issm_param_gen_fwd_only", "issm_conv_param_gen_fwd", "issm_layer_end",
+    "issm_param_gen_fwd_only", "issm_conv_param_gen_fwd", "issm_layer_end", "issm_box_dist_fwd_only",
     "issm_box_table",
     "issm_pn2_furthest_point_sampling", "issm_pn2_ball_query", "issm_pn2_group_points", "issm_pn2_group_points_grad",
     "issm_pn2_gather_points", "issm_pn2_gather_points_grad", "issm_pn2_three_nn", "issm_pn2_three_interpolate",
@@ -230,6 +230,7 @@ def load() -> C.CDLL:
     lib.issm_pn2_group_points_grad_cl.argtypes = [i32, i32, i32, i32, i32, vp, vp, vp, vp]
     lib.issm_pn2_three_interpolate_grad_cl.argtypes = [i32, i32, i32, i32, vp, vp, vp, vp, vp]
     lib.issm_box_dist_fwd.argtypes = [P(BoxDistArgs)]
+    lib.issm_box_dist_fwd_only.argtypes = [P(BoxDistArgs)]
     lib.issm_box_dist_bwd.argtypes = [P(BoxDistArgs)]
     lib.issm_dwconv_partial_rows.argtypes = [C.c_int32, C.c_int32]
     lib.issm_dwconv_silu_fwd.argtypes = [P(DwConvArgs)]

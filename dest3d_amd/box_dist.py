@@ -64,7 +64,7 @@ def _watched() -> bool:
 class BoxDistFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, table, key_xyz, corners, angle, qcenter, radius, weight_dist, log_scale, max_value, out_dtype,
-                want_dist, want_weights):
+                want_dist, want_weights, only=False):
         L.require_gpu(key_xyz, "key_xyz")
         lib = L.load()
         Bsz, nP = key_xyz.shape[:2]
@@ -108,7 +108,8 @@ class BoxDistFn(torch.autograd.Function):
                 else:
                     assert as_boxes, "weights need (qcenter, radius) or boxes"
                 a.weights = weights.data_ptr()
-            L.check(lib.issm_box_dist_fwd(C.byref(a)), "issm_box_dist_fwd")
+            run = lib.issm_box_dist_fwd_only if only else lib.issm_box_dist_fwd   # only: no backward follows
+            L.check(run(C.byref(a)), "issm_box_dist_fwd")
         ctx.save_for_backward(key, cor, ang)
         ctx.meta = (None if table is None else (tuple(table.shape), table.dtype), log_scale, max_value, out_dtype)
         ctx.mark_non_differentiable(*[t for t in (weights,) if t is not None])
@@ -143,7 +144,7 @@ class BoxDistFn(torch.autograd.Function):
                 a.stream = L.current_stream_ptr(key.device)
                 L.check(lib.issm_box_dist_bwd(C.byref(a)), "issm_box_dist_bwd")
             dtable = out.to(tdt)
-        return (dtable,) + (None,) * 11
+        return (dtable,) + (None,) * 12
 
 
 def box_dist(table, key_xyz, corners, angle=None, log_scale=512.0, max_value=4.0, out_dtype=None):
@@ -234,7 +235,7 @@ class BoxDistFun(nn.Module):
         out_dtype = self.cpb_mlps[0].weight.dtype if plain else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
         if weight_query_pos is None:
             return BoxDistFn.apply(table, key_xyz, boxes, query_angle, None, None, 0.0, self.log_scale, self.max_value,
-                                   out_dtype, True, False)[0]
+                                   out_dtype, True, False, plain)[0]
         same_boxes = (weight_query_pos.shape[-1] == 6 and query_xyz.data_ptr() == weight_query_pos.data_ptr()
                       and query_size.data_ptr() == weight_query_pos[..., 3:].data_ptr()
                       and query_xyz.stride() == weight_query_pos[..., :3].stride())
@@ -244,4 +245,4 @@ class BoxDistFun(nn.Module):
             qc = weight_query_pos[..., :3]
             rad = weight_query_pos[..., 3:].float().square().sum(-1).sqrt().clamp_min(0.64)
         return BoxDistFn.apply(table, key_xyz, boxes, query_angle, qc, rad, float(weight_dist), self.log_scale,
-                               self.max_value, out_dtype, True, True)
+                               self.max_value, out_dtype, True, True, plain)

@@ -78,20 +78,72 @@ __device__ __forceinline__ float wave_uniform(float v) {
 // The table lies node-major in LDS with 20 floats from node to node: a lane reads its node's 16 channels as four
 // 16-byte pieces, and with 16 floats per node the lanes of one read would meet in the 16 banks that (node mod 4)
 // selects; 20 n mod 64 runs through all sixteen 4-bank groups as n does.
+//
+// AXES, calls that nothing is differentiated through: boxes that stand along the axes, under no rotation.  The eight corners are
+// two positions per axis, so the sum of their trilinear weights is a product of three sums over an axis' positions: at most four nodes
+// an axis, 6 logarithms a pair instead of 24, no queue (all pairs, whether the box is next to the point or around it).  Taken by a
+// wave whose box is such a one, for finite points and a finite table (weights of zero are multiplied too).  1024 points in the order
+// of a Hilbert curve, 256 boxes, bf16: one scene 39.6 -> 24.3 us, eight 171 -> 97; boxes that are turned 39.6 and 170 either way.
+// As accurate, but rounded elsewhere, and an encoding that differs in the last bit of one value in ten thousand moves entries of a
+// gradient behind six bf16 layers by up to 0.48 of their mean square: training keeps the sums it had.
 constexpr int BD_SEG = 512;     // points per wave at most
 constexpr int BD_FWD_T = 1024;  // 16 waves = 8 adjacent boxes x 2 segments per workgroup, one workgroup (96 KB of LDS) per CU
 constexpr int BD_NS = 20;      // floats from node to node
-template <bool BF>
+
+// An axis of a box along the axes: the nodes its two positions lie between and their summed weights; nodes outside the table
+// and those the other position has already have weight zero.
+struct AxisNodes {
+  int node[4];
+  float w[4];
+};
+__device__ __forceinline__ AxisNodes axis_nodes(float p0, float p1, int n, int stride) {
+  const float g0 = floorf(p0), g1 = floorf(p1), a0 = p0 - g0, a1 = p1 - g1;
+  const int i0 = (int)g0, i1 = (int)g1;
+  const bool same = i1 == i0, up = i1 == i0 + 1, down = i1 + 1 == i0;
+  AxisNodes a;
+  a.node[0] = i0;
+  a.w[0] = (1.0f - a0) + (same ? 1.0f - a1 : down ? a1 : 0.0f);
+  a.node[1] = i0 + 1;
+  a.w[1] = a0 + (same ? a1 : up ? 1.0f - a1 : 0.0f);
+  a.node[2] = up ? i1 + 1 : i1;
+  a.w[2] = same ? 0.0f : up ? a1 : 1.0f - a1;
+  a.node[3] = i1 + 1;
+  a.w[3] = same || up || down ? 0.0f : a1;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool in = a.node[e] >= 0 && a.node[e] < n;
+    a.node[e] = in ? a.node[e] * stride : 0;
+    a.w[e] = in ? a.w[e] : 0.0f;
+  }
+  return a;
+}
+__device__ __forceinline__ bool finite_(float v) { return fabsf(v) <= 3.402823466e38f; }
+// Whether the box's corners (order of box_corner) are two positions per axis, unrotated, all finite.
+__device__ __forceinline__ bool along_axes(const BoxLane& bx) {
+  bool ok = finite_(bx.cx[0]) && finite_(bx.cx[2]) && finite_(bx.cy[0]) && finite_(bx.cy[1]) && finite_(bx.cz[0]) && finite_(bx.cz[4]);
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    ok = ok && bx.cx[c] == bx.cx[c & 2] && bx.cy[c] == bx.cy[(c ^ (c >> 1)) & 1] && bx.cz[c] == bx.cz[c & 4] && bx.cs[c] == 1.0f &&
+         bx.sn[c] == 0.0f;
+  return ok;
+}
+
+template <bool BF, bool AXES>
 __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_points) {
   __shared__ __attribute__((aligned(16))) float tab[BD_MAXCELLS * BD_NS];
   __shared__ unsigned short queue[BD_FWD_T / 64][BD_SEG];
   __shared__ int queue_len[BD_FWD_T / 64];
   const int cells = p.D * p.H * p.W;
+  bool odd = false;   // AXES: some value of the table is not finite
   for (int e = threadIdx.x; e < cells * BD_C; e += BD_FWD_T) {
     const int ch = e / cells, cell = e - ch * cells;
-    tab[cell * BD_NS + ch] = p.table[e];
+    const float v = p.table[e];
+    tab[cell * BD_NS + ch] = v;
+    if constexpr (AXES) odd = odd || !finite_(v);
   }
-  __syncthreads();
+  bool plain_table = false;
+  if constexpr (AXES) plain_table = !__syncthreads_or(odd);
+  else __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int kgroups = (p.K + 7) / 8, npair = (p.L + 2 * seg_points - 1) / (2 * seg_points);
   const int kgroup = blockIdx.x % kgroups, bs = blockIdx.x / kgroups;
@@ -108,7 +160,47 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       bx.cx[c] = wave_uniform(bx.cx[c]); bx.cy[c] = wave_uniform(bx.cy[c]); bx.cz[c] = wave_uniform(bx.cz[c]);
       bx.cs[c] = wave_uniform(bx.cs[c]); bx.sn[c] = wave_uniform(bx.sn[c]);
     }
-    for (int base = 0; base < n; base += 64) {
+    int base = 0;
+    if (AXES && plain_table && along_axes(bx)) {   // uniform
+      const float x0 = bx.cx[0], x1 = bx.cx[2], y0 = bx.cy[0], y1 = bx.cy[1], z0 = bx.cz[0], z1 = bx.cz[4];
+#pragma unroll 1
+      for (; base < n; base += 64) {
+        const int li = base + lane;
+        const float* key = p.key + ((long)b * p.L + l0 + min(li, n - 1)) * 3;
+        const float kx = key[0], ky = key[1], kz = key[2];
+        if (__ballot(!(finite_(kx) && finite_(ky) && finite_(kz))) != 0ull) break;   // (this and what follows: below)
+        const AxisNodes ax = axis_nodes(node_pos(x0 - kx, p.log_scale, scale, p.W), node_pos(x1 - kx, p.log_scale, scale, p.W), p.W, BD_NS),
+                        ay = axis_nodes(node_pos(y0 - ky, p.log_scale, scale, p.H), node_pos(y1 - ky, p.log_scale, scale, p.H), p.H, p.W * BD_NS);
+        AxisNodes az = axis_nodes(node_pos(z0 - kz, p.log_scale, scale, p.D), node_pos(z1 - kz, p.log_scale, scale, p.D), p.D, p.H * p.W * BD_NS);
+        f4 acc[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+        const bool x2 = __ballot(ax.w[2] != 0.0f) != 0ull, x3 = __ballot(ax.w[3] != 0.0f) != 0ull;
+#pragma unroll 1
+        for (int k3 = 0; k3 < 4; ++k3) {   // (always entry 0 of az, whose entries move up: registers are not indexed)
+#pragma unroll
+          for (int i3 = 0; i3 < 4; ++i3) {
+            const float zy = az.w[0] * ay.w[i3];
+            if (__ballot(zy != 0.0f) == 0ull) continue;
+            const float* row = tab + az.node[0] + ay.node[i3];
+            auto node = [&](int j3) {
+              const f4* src = (const f4*)(row + ax.node[j3]);
+              const float w = zy * ax.w[j3];
+#pragma unroll
+              for (int j = 0; j < 4; ++j) acc[j] += w * src[j];
+            };
+            node(0);
+            node(1);
+            if (x2) node(2);
+            if (x3) node(3);
+          }
+#pragma unroll
+          for (int e = 0; e < 3; ++e) az.node[e] = az.node[e + 1], az.w[e] = az.w[e + 1];
+        }
+        if (li < n) store_dist<BF>(p, ((long)b * p.L + l0 + li) * p.K + k, acc);
+      }
+    }
+    for (; base < n; base += 64) {
       const int li = base + lane;
       const bool valid = li < n;
       const float* key = p.key + ((long)b * p.L + l0 + (valid ? li : n - 1)) * 3;
@@ -349,15 +441,16 @@ int box_dist_bwd_workgroups(int B, int L, int K) {
   return (int)(items < 256 ? items : 256);  // backward: one 128 KB workgroup per CU
 }
 
-int launch_box_dist_fwd(const BoxDistP& p, hipStream_t st) {
+int launch_box_dist_fwd(const BoxDistP& p, bool only, hipStream_t st) {
   const dim3 b(NTHREADS);
   if (p.dist) {
     // segments of whole waves, as long as the queue allows but no longer than leaves every CU (256) a workgroup
     const long rows = (long)p.B * ((p.K + 7) / 8), want = (256 + rows - 1) / rows;
     const int half = (int)((p.L + 2 * want - 1) / (2 * want)), seg = half >= BD_SEG ? BD_SEG : (half + 63) / 64 * 64;
     const dim3 g((unsigned)(rows * ((p.L + 2 * seg - 1) / (2 * seg))));
-    if (p.dtype) hipLaunchKernelGGL(k_box_dist_fwd<true>, g, dim3(BD_FWD_T), 0, st, p, seg);
-    else hipLaunchKernelGGL(k_box_dist_fwd<false>, g, dim3(BD_FWD_T), 0, st, p, seg);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(BD_FWD_T), 0, st, p, seg); };
+    if (p.dtype) only ? go(&k_box_dist_fwd<true, true>) : go(&k_box_dist_fwd<true, false>);
+    else only ? go(&k_box_dist_fwd<false, true>) : go(&k_box_dist_fwd<false, false>);
   }
   if (p.weights) hipLaunchKernelGGL(k_box_dist_weights, dim3(p.nwg), b, 0, st, p);
   return (int)hipGetLastError();

@@ -76,7 +76,7 @@ int launch_scatter_channel_last(bool k3, int b, int c, int n, int ne, const floa
 int box_dist_workgroups(int B, int L, int K);
 int box_dist_bwd_workgroups(int B, int L, int K);
 long box_dist_bwd_scratch_bytes(int B, int L, int K, int D, int H, int W);
-int launch_box_dist_fwd(const BoxDistP& p, hipStream_t st);
+int launch_box_dist_fwd(const BoxDistP& p, bool only, hipStream_t st);
 int launch_box_dist_bwd(const BoxDistP& p, hipStream_t st);
 int dwconv_partial_rows(int B, int L);
 int launch_dwconv_fwd(const DwConvP& p, hipStream_t st);
@@ -843,13 +843,15 @@ int issm_box_table(const issm_box_table_args* a) {
   return launched(launch_box_table(p, (hipStream_t)a->stream), "box_table");
 }
 
-int issm_box_dist_fwd(const issm_box_dist_args* a) {
+static int box_dist_fwd(const issm_box_dist_args* a, bool only) {
   BoxDistP p;
   int rc = box_dist_params(a, &p, false);
   if (rc) return rc;
   if (p.nwg == 0 || (!p.dist && !p.weights)) return ISSM_OK;
-  return launched(launch_box_dist_fwd(p, (hipStream_t)a->stream), "box_dist_fwd");
+  return launched(launch_box_dist_fwd(p, only, (hipStream_t)a->stream), "box_dist_fwd");
 }
+int issm_box_dist_fwd(const issm_box_dist_args* a) { return box_dist_fwd(a, false); }
+int issm_box_dist_fwd_only(const issm_box_dist_args* a) { return box_dist_fwd(a, true); }
 
 int issm_box_dist_bwd(const issm_box_dist_args* a) {
   BoxDistP p;

@@ -558,6 +558,8 @@ typedef struct issm_box_dist_args {
 
 int64_t issm_box_dist_bwd_scratch_bytes(int32_t batch, int32_t seqlen, int32_t nquery, int32_t D, int32_t H, int32_t W);
 int issm_box_dist_fwd(const issm_box_dist_args* args);
+/* The same for a call that no backward follows: boxes along the axes are summed axis by axis (another order of the same sums). */
+int issm_box_dist_fwd_only(const issm_box_dist_args* args);
 
 /* The encoding's table (dest_module.py:160-166,191): table[16][nodes] fp32 = W2 relu(W1 coords + b1) at every node, coords
  * (nodes, 3) of coords_dtype, w1 (hidden, 3), b1 (hidden), w2 (16, hidden) of dtype, all contiguous; coords, hidden values and

@@ -72,6 +72,39 @@ def test_box_dist_forward_and_table_gradient(case):
     assert _rel(dist_bf.float().cpu().numpy(), ref) <= 1e-2
 
 
+@pytest.mark.parametrize("nP,nQ,dims,spread", [(65, 9, (10, 10, 10), 4.0), (1100, 64, (4, 6, 7), 4.0), (3, 300, (5, 4, 3), 0.2), (200, 16, (1, 30, 30), 2.0),
+                                               (130, 8, (10, 10, 10), 200.0), (1, 1, (2, 2, 2), 0.0)])
+def test_boxes_along_the_axes_without_a_gradient(nP, nQ, dims, spread):
+    """Calls that no backward follows: boxes along the axes are summed axis by axis.  Positions of an axis in the same cell, in
+    neighbouring ones, apart and outside the table, a quarter of the boxes turned, against the fp64 oracle (bound as above)."""
+    from dest3d_amd.box_dist import BoxDistFn, box_parametrization_to_corners
+    run = lambda t, k, c, only: BoxDistFn.apply(t, k, c, None, None, None, 0.0, 512.0, 4.0, torch.float32, True, False, only)[0]
+    key, qxyz, qsize, ang = _inputs(2, nP, nQ, 5 + nP + nQ, True)
+    key, qxyz = (key * np.float32(spread / 4) for key in (key, qxyz))
+    qsize[:, ::3] *= np.float32(1e-3)
+    heading = ang * (np.arange(nQ) % 4 == 1)
+    table = np.random.default_rng(4).standard_normal((16, *dims)).astype(np.float32)
+    t, tk, tq, ts, th = (torch.from_numpy(np.ascontiguousarray(x, np.float32)).cuda() for x in (table, key, qxyz, qsize, heading))
+    corners = box_parametrization_to_corners(tq, ts, th)
+    whole, dist = run(t, tk, corners, False), run(t, tk, corners, True)
+    # the oracle takes one angle for the corners and the rotation: the boxes that are not turned
+    plain = np.arange(nQ) % 4 != 1
+    ref = R.box_dist(key, qxyz, qsize, np.zeros_like(ang), table)
+    assert _rel(dist.cpu().numpy()[:, :, plain], ref[:, :, plain]) <= 2e-5
+    assert torch.equal(dist[:, :, ~plain], whole[:, :, ~plain])
+    assert (dist - whole).norm() <= 2e-5 * whole.norm()
+    # values that are not finite: of the table, of a point, of a box
+    odd = t.clone()
+    odd[3, 0, 0, 0], odd[5, -1, -1, -1] = float("nan"), float("inf")
+    kodd, codd = tk.clone(), corners.clone()
+    kodd[0, nP // 2, 1], codd[1, nQ // 2, 2, 0] = float("inf"), float("nan")
+    for tt, kk, cc in ((odd, tk, corners), (t, kodd, codd)):
+        got, want = run(tt, kk, cc, True), run(tt, kk, cc, False)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        ok = want.isfinite()
+        assert (got[ok] - want[ok]).norm() <= 2e-5 * want[ok].norm() + 1e-30
+
+
 def test_local_weight_and_fused_module_call():
     from dest3d_amd.box_dist import BoxDistFun, local_weight
     B, nP, nQ = 2, 50, 256
