@@ -142,6 +142,7 @@ static FwdWs fwd_layout(const issm_dims& d, bool has_z) {
 static int bwd_head_parts(const issm_dims& d) {
   const long blocks = (long)d.batch * nchunks(d) * d.ngroups * ((d.dstate + ISSM_CHUNK - 1) / ISSM_CHUNK);
   const long heads = d.nheads / d.ngroups, most = std::max<long>(1, std::min<long>(heads, 512 / blocks));
+  if (d.ndir == 1 && heads % 2 == 0 && blocks <= NCU && most <= 3) return 1;   // (a workgroup takes two heads at a time: bwd_tile_pair)
   const long each = (heads + most - 1) / most;
   return (heads - each) * d.ndir < 4 ? 1 : (int)((heads + each - 1) / each);   // (no part without a head)
 }

@@ -110,7 +110,7 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
   return r;
 }
 
-constexpr int DUAL_TILES = 8;
+constexpr int DUAL_TILES = 8, PAIR_TILES = 16;
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
@@ -119,6 +119,9 @@ constexpr int DUAL_TILES = 8;
 // heads x 32, 256 states, fp32).  What it gives is less than that, for eight waves now meet where four did: the two launches 88 + 96 us,
 // this one 172; heads of 36, bf16, 71 + 75 and 134.  (The second direction a barrier or two behind the first, so that they use LDS and
 // the vector ALU at different times: 169, for a barrier then waits for the longer of two different phases.)
+// PAIR_TILES more (PAIR): two heads of the group side by side, four waves each of a workgroup of eight, and their sums of dB and dC added up through
+// LDS at the end.  For grids that give no CU a second workgroup, where a lone wave a SIMD waits for itself: 2 x 160 tokens, 4 heads x 32, 128
+// states, fp32 34.2 -> 24.9 us; 2 x 1000, 4 x 36, 200 states 40.7 -> 31.1; 4 x 1000, 4 x 32, 256 states, bf16 33.1 -> 26.3.
 // FULL: complete chunks and column slices; otherwise rows and columns may be absent (see RowMap).  PARTS: gridDim.y workgroups
 // share the group's heads, heads_each each (a variant of its own: the two loop bounds more cost the others 25 - 50 scalar
 // registers spilled and 1 - 2 % of a training step).
@@ -127,7 +130,8 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
                                                           const float* __restrict__ dstates,
                                                           const float* __restrict__ dm, float* __restrict__ partA,
                                                           float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
-  constexpr bool DUAL = TILES >= DUAL_TILES;
+  constexpr bool DUAL = TILES / DUAL_TILES == 1, PAIR = TILES / PAIR_TILES == 1, TWO = DUAL || PAIR;
+  static_assert(!PAIR || !PARTS, "one or the other");
   constexpr int PT = TILES % DUAL_TILES;
   constexpr bool SPLIT = !IOB;
   // fp32 products in the diagonal blocks / in all blocks.  (Four head tiles, complete: as the level form, which took these calls
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   constexpr bool DIAG32 = IOB && !FULL, ALL32 = SPLIT && (!FULL || PT >= 4);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typedef BwdTileSmem<PT, SPLIT> SM;
-  const int half = DUAL ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS) : 0;
+  const int half = TWO ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS) : 0;
   SM& s = *reinterpret_cast<SM*>(smem_raw + half * sizeof(SM));
   constexpr int LDP = SM::LDP, LDM = SM::LDM, KT = (PT + 1) / 2;
   constexpr bool BCL = SM::BCL, BL = SM::BL, EX_IN_TILES = dual_ex_in_tiles<SM>();
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   // heads, 256 states, both directions, per direction: heads of 48 128 and 137 -> 104 and 112 us; of 64, which took the level form, 135
   // -> 114 and 121; of 32 the same as before, but it makes room for B (SM::BL).
   constexpr int KP_ = PT * 4;  // dS / H values per lane
-  const int tid = DUAL ? threadIdx.x % NTHREADS : threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = TWO ? threadIdx.x % NTHREADS : threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int cm = lane & 15, g4 = lane >> 4;
   const int nsl = (p.N + NS - 1) / NS;
   Unit u;
@@ -287,10 +291,11 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
       }
     }
   };
-  const int hh0 = PARTS ? (int)blockIdx.y * heads_each : 0;
+  // (PAIR: heads_each is half of an even number, so that both halves of the workgroup meet at the same barriers)
+  const int hh0 = PARTS ? (int)blockIdx.y * heads_each : PAIR ? half * heads_each : 0;
   request(head_of(hh0));
 
-  for (int hh = hh0; hh < (PARTS ? min(p.hpg, hh0 + heads_each) : p.hpg); ++hh) {
+  for (int hh = hh0; hh < (PARTS ? min(p.hpg, hh0 + heads_each) : PAIR ? hh0 + heads_each : p.hpg); ++hh) {
     u.h = head_of(hh);
     __syncthreads();  // the previous head no longer reads the tiles
     {
@@ -369,6 +374,10 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     if (skip) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) asm volatile("v_mov_b32 %0, 0\nv_mov_b32 %1, 0" : "=v"(dcs[k]), "=v"(val[k]));  // (opaque: zeros set in advance are set for every head)
+      if constexpr (PAIR && SPLIT) {   // the other half's head may stand at these
+        __syncthreads();
+        __syncthreads();
+      }
     } else {
       // dS and H of the lane's column as (hi, lo) bf16 pairs: the B operands of Q = x . dS and R = dy . H (products over
       // the head dimension, K = 32 per step; k-slot s of step t <-> lane value 8 t + s).  They are fp32 states, whose rounding to
@@ -406,7 +415,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
         bf8 hi[KT], lo[KT];
         state_pairs(l_dsv, hi, lo);
         rows_times(hi, lo, qs);
-        __syncthreads();   // (skip is the workgroup's)
+        __syncthreads();   // (skip is the workgroup's or, PAIR, its half's)
         put_split(l_dv, s.dys(), tq);
         gsum = lane_dot_pn<KP_>(l_dsv, l_hv, p.P, g4, PNF);
         state_pairs(l_hv, hi, lo);
@@ -664,7 +673,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
       if constexpr (P32) lane_load_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, old);
       else lane_load_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, old);
     }
-    request(head_of(min(hh + 1, (PARTS ? min(p.hpg, hh0 + heads_each) : p.hpg) - 1)));  // (unconditional: the last head is requested again and not used)
+    request(head_of(min(hh + 1, (PARTS ? min(p.hpg, hh0 + heads_each) : PAIR ? hh0 + heads_each : p.hpg) - 1)));  // (unconditional: the last head is requested again and not used)
     __builtin_amdgcn_sched_barrier(0);
     // DUAL: the two halves of the workgroup have one column's rows in opposite order (row k of a lane of the one is row 15 - k of
     // lane ^ 48 of the other); each hands its first eight over and stores the sums of its last eight.
@@ -782,6 +791,22 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     }
   }
 
+  if constexpr (PAIR) {   // each half adds up one of the two sums, and stores it
+    __syncthreads();
+    const SM &s0 = *reinterpret_cast<const SM*>(smem_raw), &s1 = *reinterpret_cast<const SM*>(smem_raw + sizeof(SM));
+    float v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = s0.dbc[(16 * half + k) * NTHREADS + tid] + s1.dbc[(16 * half + k) * NTHREADS + tid];
+    if (DIAG32 && p.dbc_part && (s0.shared[wave] | s1.shared[wave])) {
+      float* q = p.dbc_part + ((long)p.dir0 * gridDim.x + wg) * (32 * NTHREADS) + 16 * half * NTHREADS + tid;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) q[k * NTHREADS] = v[k];
+    } else {
+      const TensorD& d = half ? p.dC[u.dir] : p.dB[u.dir];
+      if (d.ptr) lane_store_ln<IOB>(d, u.b, u.g, n, vn, g4, rm, v);
+    }
+    return;
+  }
   if (PARTS || (DIAG32 && p.dbc_part && s.shared[wave])) {  // (the wave's own word)
     const long at = (long)p.dir0 * gridDim.x + wg;
     float* q = p.dbc_part + (PARTS ? (long)blockIdx.y * p.ndir * gridDim.x + at : at) * (32 * NTHREADS) + tid;
@@ -826,26 +851,37 @@ bool bwd_tile_dual(const KP& p, const float* dy_ws, int parts) {
   return p.ndir == 2 && p.full_tiles && !dy_ws && parts == 1 && blocks > 320 && (p.io_dt || p.P == 32) && bwd_tile_available(p, dy_ws);
 }
 
+// Whether two heads of a group share a workgroup (PAIR): an even number of them, in calls of one direction, where no CU gets a second
+// workgroup: two waves a SIMD then take half as many heads each.  Against two workgroups that share the heads (PARTS) it saves
+// the launch that adds up their sums: 4 x 1024 tokens, 8 heads x 32, 256 states, fp32 45.2 + 6.9 us -> 44.0, bf16 35.6 + 7.2 -> 34.0; heads of 64
+// 58.2 + 6.8 -> 60.0; three parts, 3 x 1024, fp32 42.6 + 6.3 -> 42.0, heads of 36, bf16 36.4 + 6.2 -> 37.0.
+static bool bwd_tile_pair(const KP& p, int blocks, int parts) { return p.ndir == 1 && parts == 1 && blocks <= NCU && p.hpg % 2 == 0; }
+
 template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
                              float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st) {
   static_assert(sizeof(BwdTileSmem<PT, !IOB>) <= 80 * 1024, "two workgroups a CU");
-  const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0;
+  const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0, pair = bwd_tile_pair(p, blocks, parts);
   auto go = [&](auto kern, int dirs = 1) -> int {
     typedef BwdTileSmem<PT, !IOB> SM;
-    const size_t sm = dirs == 1 ? sizeof(SM) : dual_lds<SM>();
+    const size_t sm = pair ? 2 * sizeof(SM) : dirs == 1 ? sizeof(SM) : dual_lds<SM>();
     if (sm > 64 * 1024)
       if (int e = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm))
         return e;
     hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(dirs * NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
-                       (p.hpg + parts - 1) / parts);
+                       pair ? p.hpg / 2 : (p.hpg + parts - 1) / parts);
     return 0;
   };
   if constexpr (IOB)
     if (dual && !pnf) return go(&k_bwd_tile<DUAL_TILES + PT, IOB, false, false, false, true, false>, 2);
   if constexpr (IOB || PT == 2)
     if (dual) return go(&k_bwd_tile<DUAL_TILES + PT, IOB, true, false, false, true, false>, 2);
+  if (pair) {
+    if (!p.full_tiles) return go(&k_bwd_tile<PAIR_TILES + PT, IOB, false, false, false, false, false>, 2);
+    if (pnf) return go(&k_bwd_tile<PAIR_TILES + PT, IOB, true, false, false, true, false>, 2);
+    return go(&k_bwd_tile<PAIR_TILES + PT, IOB, false, false, false, true, false>, 2);
+  }
   auto pick = [&](auto p32) -> int {
     constexpr bool P32 = decltype(p32)::value;
     if (parts > 1) {

@@ -1616,3 +1616,11 @@ def test_outputs_by_one_and_by_two_groups_of_waves(dtype, L_, N, P, gated):
         bound = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24 * 4 * (slices + 2)
         assert (got - want).norm() <= bound * want.norm()
         assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("L_,N,H,marked", [(128, 128, 4, True), (100, 70, 4, True), (100, 70, 4, False), (64, 64, 2, False), (1600, 320, 8, True)])
+def test_heads_two_at_a_time(dtype, L_, N, H, marked):
+    """Calls of one direction with an even number of heads a group and few chunks: two heads side by side in a workgroup of the chunk backward,
+    heads out of range in either half of it.  As above, against calls of one head each."""
+    test_heads_shared_by_several_workgroups(dtype, L_, N, H, 1, marked)
