@@ -23,7 +23,8 @@ int launch_bwd_dstates(const KP& p, const float* dy_ws, float* dstates, float* d
 int launch_state_bwd(const KP& p, const float* cs_last, float* dstates, float* dh0_dir, hipStream_t st);
 int launch_state_sums(const KP& p, const float* states, const float* dstates, float* g_last, hipStream_t st);
 int launch_bwd_chunk(const KP& p, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, bool dual, hipStream_t st);
+                     float* partA, float* partBias, int* redo, int* redo_pending, int parts, bool dual, const float* cabt, float* partD,
+                     bool* with_dx, hipStream_t st);
 int launch_bwd_parts_sum(const KP& p, const int* redo, int parts, hipStream_t st);
 int launch_bwd_chunk_redo(const KP& p, int ndirs, const float* dy_ws, const float* states, const float* dstates,
                           const float* dm, float* partA, float* partBias, const int* redo,
@@ -436,7 +437,7 @@ int issm_stage_bwd_chunk(const issm_scan_args* a, int dir, const float* dy_gated
   p.dir0 = dir;
   int pending = 0;
   if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1, false,
-                                      (hipStream_t)a->stream),
+                                      nullptr, nullptr, nullptr, (hipStream_t)a->stream),
                      "bwd_chunk")))
     return rc;
   if (!pending) return ISSM_OK;
@@ -511,6 +512,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
     if (parts > 1 || (p.io_dt && !p.full_tiles)) p.dbc_part = pc.dbc_part = ws + bw.dbc_part;
   }
   const bool dual = bwd_tile_dual(p, dy, parts);
+  bool with_dx = false;   // the chunk backward's launch has dx
   if (wants_ddt_part(a) && !dual && bwd_tile_available(p, dy)) {
     // both directions go through the tile-base kernel: the first one's share of the bf16 ddt travels in fp32
     pc.ddt_part.ptr = ws + bw.ddt_part;
@@ -522,7 +524,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
     KP pd = pc;
     pd.dir0 = dir;
     if ((rc = launched(launch_bwd_chunk(pd, dy, sv + fw.states, ws + bw.dstates, ws + bw.dm,
-                                        ws + bw.partA, ws + bw.partBias, redo, &pending, parts, dual, st),
+                                        ws + bw.partA, ws + bw.partBias, redo, &pending, parts, dual, sv + fw.cabt, ws + bw.partD, &with_dx, st),
                        "bwd_chunk")))
       return rc;
   }
@@ -536,7 +538,7 @@ int issm_scan_bwd(const issm_scan_args* a) {
                        "bwd_chunk (redo)")))
       return rc;
   }
-  if ((rc = launched(launch_bwd_dx(p, dy, ws + bw.dstates, sv + fw.cabt, ws + bw.partD, st), "bwd_dx"))) return rc;
+  if (!with_dx && (rc = launched(launch_bwd_dx(p, dy, ws + bw.dstates, sv + fw.cabt, ws + bw.partD, st), "bwd_dx"))) return rc;
   return launched(launch_bwd_reduce(p, ws + bw.partA, ws + bw.partBias, ws + bw.partD, ws + bw.dh0_dir, a->dA,
                                     a->dt_bias ? a->ddt_bias : nullptr, a->D ? a->dD : nullptr, a->dh0, st),
                   "bwd_reduce");

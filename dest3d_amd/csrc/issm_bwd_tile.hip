@@ -43,7 +43,9 @@
 // products: the recurrences need not read the states for it (33 - 60 % of their bytes), and what cancels does so exactly: ddt_bias
 // and dA of 2 x 512 tokens, 8 heads x 32, 256 states, fp32, 1.7e-4 and 8e-5 -> 6e-6 of their norm from float64; with A a hundred
 // times larger 9e-2 and 0.4 -> 2e-4 and 8e-4.
-#include "issm_dev.h"
+#include <algorithm>
+
+#include "issm_bwd_dx.h"
 
 namespace issm {
 
@@ -111,6 +113,14 @@ __device__ __forceinline__ f4 scaled_twice(f4 v, float a, float b) {
 }
 
 constexpr int DUAL_TILES = 8, PAIR_TILES = 16;
+// PAIR: the workgroups from `blocks` on compute dx (k_bwd_dx_body) of a unit each.  The two do not depend on each other, and where they
+// fit the CUs side by side dx costs nothing: kernels of a training step, fp32, 2 x 160 tokens, 4 heads x 32, 128 states 75.7 -> 64.4 us, 2 x 1000,
+// 4 x 36, 200 states 115 -> 101; and a launch less to issue.
+struct DxPart {
+  const float* cabt;
+  float* partD;
+  int blocks;
+};
 // PNF: the head dimension fills its 16-row tiles (P == 16 PT); ACC: ddt holds the other direction's share already and
 // this launch adds to it; P32 (bf16 only): that share travels in fp32 through p.ddt_part -- the first direction's launch
 // writes it there, the second reads it from there and writes the once-rounded sum to ddt.
@@ -129,10 +139,15 @@ template <int TILES, bool IOB, bool PNF, bool ACC, bool P32, bool FULL, bool PAR
 __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) void k_bwd_tile(KP p, const float* __restrict__ states,
                                                           const float* __restrict__ dstates,
                                                           const float* __restrict__ dm, float* __restrict__ partA,
-                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each) {
+                                                          float* __restrict__ partBias, int* __restrict__ redo, int heads_each, DxPart dx) {
   constexpr bool DUAL = TILES / DUAL_TILES == 1, PAIR = TILES / PAIR_TILES == 1, TWO = DUAL || PAIR;
   static_assert(!PAIR || !PARTS, "one or the other");
   constexpr int PT = TILES % DUAL_TILES;
+  if constexpr (PAIR) {
+    if ((int)blockIdx.x >= dx.blocks)
+      return k_bwd_dx_body<PT, IOB, IOB, FULL, 2>(p, (int)blockIdx.x - dx.blocks, (int)gridDim.x - dx.blocks, nullptr, dstates, dx.cabt, dx.partD);
+  }
+  const int nblocks = PAIR ? dx.blocks : (int)gridDim.x;
   constexpr bool SPLIT = !IOB;
   // fp32 products in the diagonal blocks / in all blocks.  (Four head tiles, complete: as the level form, which took these calls
   // before, has the closest pairs in fp32.  Operand pairs would leave ddt, dB, dC 5.0 -> 5.4e-6 of their norm from float64, fp32 products
@@ -155,7 +170,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   const int cm = lane & 15, g4 = lane >> 4;
   const int nsl = (p.N + NS - 1) / NS;
   Unit u;
-  int wg = xcd_remap(blockIdx.x, gridDim.x);
+  int wg = xcd_remap(blockIdx.x, nblocks);
   unsigned id = wg;
   const int ns = (int)p.by_slices(id);
   u.g = (int)p.by_G(id);
@@ -364,7 +379,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
       any_bad |= be.x | be.y | be.z | be.w;
     }
     const bool skip = any_bad != 0;  // uniform: the whole head is left to the level-hierarchy kernel
-    if (tid == 0) redo[(u.dir * (int)gridDim.x + wg) * p.hpg + (DUAL && half ? p.hpg - 1 - hh : hh)] = skip ? 1 : 0;
+    if (tid == 0) redo[(u.dir * nblocks + wg) * p.hpg + (DUAL && half ? p.hpg - 1 - hh : hh)] = skip ? 1 : 0;
     if (DIAG32 && skip) s.shared[wave] = 1;
     const uint16_t* xs_ = s.xs;
     const uint16_t* dys_ = s.dys();
@@ -798,7 +813,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
 #pragma unroll
     for (int k = 0; k < 16; ++k) v[k] = s0.dbc[(16 * half + k) * NTHREADS + tid] + s1.dbc[(16 * half + k) * NTHREADS + tid];
     if (DIAG32 && p.dbc_part && (s0.shared[wave] | s1.shared[wave])) {
-      float* q = p.dbc_part + ((long)p.dir0 * gridDim.x + wg) * (32 * NTHREADS) + 16 * half * NTHREADS + tid;
+      float* q = p.dbc_part + (long)wg * (32 * NTHREADS) + 16 * half * NTHREADS + tid;
 #pragma unroll
       for (int k = 0; k < 16; ++k) q[k * NTHREADS] = v[k];
     } else {
@@ -859,18 +874,18 @@ static bool bwd_tile_pair(const KP& p, int blocks, int parts) { return p.ndir ==
 
 template <int PT, bool IOB>
 static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const float* dstates, const float* dm,
-                             float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st) {
+                             float* partA, float* partBias, int* redo, int parts, bool dual, DxPart dx, int dx_blocks, hipStream_t st) {
   static_assert(sizeof(BwdTileSmem<PT, !IOB>) <= 80 * 1024, "two workgroups a CU");
   const bool pnf = p.P == 16 * PT, acc = p.dir0 > 0, pair = bwd_tile_pair(p, blocks, parts);
   auto go = [&](auto kern, int dirs = 1) -> int {
     typedef BwdTileSmem<PT, !IOB> SM;
-    const size_t sm = pair ? 2 * sizeof(SM) : dirs == 1 ? sizeof(SM) : dual_lds<SM>();
+    const size_t sm = pair ? std::max(2 * sizeof(SM), sizeof(BwdDxSmem<PT, IOB, 2>)) : dirs == 1 ? sizeof(SM) : dual_lds<SM>();
     if (sm > 64 * 1024)
       if (int e = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm))
         return e;
-    hipLaunchKernelGGL(kern, dim3(blocks, parts), dim3(dirs * NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
-                       pair ? p.hpg / 2 : (p.hpg + parts - 1) / parts);
+    hipLaunchKernelGGL(kern, dim3(blocks + dx_blocks, parts), dim3(dirs * NTHREADS), sm, st, p, states, dstates, dm, partA, partBias, redo,
+                       pair ? p.hpg / 2 : (p.hpg + parts - 1) / parts, dx);
     return 0;
   };
   if constexpr (IOB)
@@ -898,7 +913,8 @@ static int launch_bwd_tile_t(const KP& p, int blocks, const float* states, const
 }
 
 int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const float* dstates, const float* dm,
-                    float* partA, float* partBias, int* redo, int parts, bool dual, hipStream_t st) {
+                    float* partA, float* partBias, int* redo, int parts, bool dual, const float* cabt, float* partD, bool* with_dx,
+                    hipStream_t st) {
   KP p = p_;
   if (dy_ws) {  // a gated dy: fp32 (Bt, L, H, P) contiguous, batch * direction outermost
     TensorD& t = p.dout[p.dir0];
@@ -909,16 +925,21 @@ int launch_bwd_tile(const KP& p_, const float* dy_ws, const float* states, const
     p.full_tiles = 0;   // the variants with fp32 products, see the head of this file
   }
   const int blocks = p.B * p.nc * p.G * ((p.N + NS - 1) / NS);
-  const int pt = (p.P + 15) / 16;
+  const int pt = (p.P + 15) / 16, units = p.B * p.nc * p.H;
+  // dx beside it: a CU for each workgroup of either (and two slices of the states, which dx's two groups of waves share)
+  const bool dx = with_dx && !dy_ws && bwd_tile_pair(p, blocks, parts) && two_groups(units, p.N) && blocks + units <= NCU;
+  const DxPart dxp{cabt, partD, blocks};
+  const int dxb = dx ? units : 0;
+  if (with_dx) *with_dx = dx;
   int e = 0;
   if (p.io_dt) {
-    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
-    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
+    else e = launch_bwd_tile_t<4, true>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
   } else {
-    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
-    else if (pt == 3) e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
-    else e = launch_bwd_tile_t<4, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, st);
+    if (pt <= 2) e = launch_bwd_tile_t<2, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
+    else if (pt == 3) e = launch_bwd_tile_t<3, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
+    else e = launch_bwd_tile_t<4, false>(p, blocks, states, dstates, dm, partA, partBias, redo, parts, dual, dxp, dxb, st);
   }
   if (e) return e;
   return (int)hipGetLastError();

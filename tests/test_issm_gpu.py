@@ -1624,3 +1624,26 @@ def test_heads_two_at_a_time(dtype, L_, N, H, marked):
     """Calls of one direction with an even number of heads a group and few chunks: two heads side by side in a workgroup of the chunk backward,
     heads out of range in either half of it.  As above, against calls of one head each."""
     test_heads_shared_by_several_workgroups(dtype, L_, N, H, 1, marked)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("B,L_,N,P,H,G", [(1, 128, 128, 32, 2, 1), (2, 160, 130, 36, 4, 1), (3, 70, 192, 64, 4, 2), (1, 1280, 256, 16, 4, 1), (1, 64, 65, 48, 2, 1)])
+def test_dx_in_the_launch_of_the_chunk_backward(dtype, B, L_, N, P, H, G):
+    """Few enough chunks for dx beside the chunk backward, against the same scenes in a batch too large for that: every gradient of a scene,
+    in the order of sums that the two batches have (as in test_outputs_by_one_and_by_two_groups_of_waves; a head's sums of dA, dD
+    and the bias run over the batch and are compared there as means)."""
+    copies = -(-700 // (B * (-(-L_ // 64)) * H))
+    d = _problem(B, L_, H, P, N, G, seed=L_ + N + P, D="hp")
+    big = {k: v.repeat(copies, *([1] * (v.dim() - 1))) if torch.is_tensor(v) and k not in ("A", "D", "dt_bias") else v for k, v in d.items()}
+    blocks, units = B * (-(-L_ // 64)) * G * (-(-N // 64)), B * (-(-L_ // 64)) * H
+    assert blocks + units <= 256 < units * copies
+    _, _, g, _ = _run_operator(d, dtype)
+    _, _, gb, _ = _run_operator(big, dtype)
+    for name, got in g.items():
+        want = gb[name]
+        if got is None:
+            continue
+        got, want = got.detach().double(), want.detach().double()
+        want = want[:B] if want.shape[0] != got.shape[0] else want / copies
+        bound = 2.0 ** -7 if dtype == torch.bfloat16 else 2e-5
+        assert torch.isfinite(got).all() and (got - want).norm() <= bound * want.norm() + 1e-30, name
