@@ -783,9 +783,12 @@ __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int 
 // whatever else lies within its third distance (which shrinks on the way; rows beyond it are skipped).  The answer is that of
 // the pass over all points: distances are evaluated the same way, ordered by (distance, index), and cells are left out only
 // if their distance, shortened by far more than the rounding of cell numbers and distances, is above the third one.  Coordinates that
-// are not finite (or above 1e18) send the workgroup to the pass over all points.  20000 x 2048 points, 8 samples:
-// 258 us looking at all, 50 us here.
-constexpr int NN_T = 512, NN_CELLS = 4096;
+// are not finite (or above 1e18) send the workgroup to the pass over all points.  A workgroup's share of the targets is
+// what leaves every CU one workgroup, up to one a thread; the known points stay in registers (R a thread) from the bounds over their
+// cells to the sorted list, and their places in the cells are what the counting's additions return.  20000 x 2048 points, 8 samples: 258 us
+// looking at all, 47 us with a workgroup to 512 targets (320 of them, two on every fourth CU) that read the points three times, 42 like this, 38 with the
+// places of a block's rows read together and a point requested while the one before is looked at.
+constexpr int NN_T = 1024, NN_CELLS = 4096;
 struct Nearest3 {
   float d1, d2, d3;
   int i1, i2, i3;
@@ -797,7 +800,8 @@ struct Nearest3 {
     else if (z) { d3 = d; i3 = k; }
   }
 };
-__global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const float* __restrict__ unknown,
+template <int R>
+__global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, int share, const float* __restrict__ unknown,
                                                         const float* __restrict__ known, float* __restrict__ dist2,
                                                         int* __restrict__ idx) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -809,10 +813,20 @@ __global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const floa
   const float INFV = __builtin_huge_valf();
   const float* kp = known + (long)b * m * 3;
   float lo[3] = {INFV, INFV, INFV}, hi[3] = {-INFV, -INFV, -INFV}, odd = 0.0f;
-  for (int k = tid; k < m; k += NN_T)
+  float pt[R][3];   // points tid, tid + NN_T, .. (past the end: the last one again, not counted)
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int a = 0; a < 3; ++a) pt[r][a] = kp[min(tid + r * NN_T, m - 1) * 3 + a];
+  const int j = blockIdx.x * share + tid;
+  const bool live = tid < share && j < n;
+  const float* u = unknown + ((long)b * n + min(j, n - 1)) * 3;
+  const float ux = u[0], uy = u[1], uz = u[2];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const float v = kp[k * 3 + a];
+      const float v = pt[r][a];
       if (!(fabsf(v) < 1e18f)) odd = 1.0f;
       lo[a] = fminf(lo[a], v);
       hi[a] = fmaxf(hi[a], v);
@@ -849,17 +863,14 @@ __global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const floa
   const float inv = 1.0f / side;
   auto cell1 = [&](float v, int a) { return min(max((int)((v - lo[a]) * inv), 0), g[a] - 1); };
 
-  const int j = blockIdx.x * NN_T + tid;
-  const bool live = j < n;
-  float ux = 0.0f, uy = 0.0f, uz = 0.0f;
-  if (live) {
-    const float* u = unknown + ((long)b * n + j) * 3;
-    ux = u[0]; uy = u[1]; uz = u[2];
-  }
   Nearest3 best = {INFV, INFV, INFV, 0, 0, 0};
   if (odd == 0.0f && longest < INFV) {   // uniform
-    for (int k = tid; k < m; k += NN_T)
-      atomicAdd(&end[1 + (cell1(kp[k * 3 + 2], 2) * g[1] + cell1(kp[k * 3 + 1], 1)) * g[0] + cell1(kp[k * 3], 0)], 1);
+    int cell[R], place[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      cell[r] = (cell1(pt[r][2], 2) * g[1] + cell1(pt[r][1], 1)) * g[0] + cell1(pt[r][0], 0);
+      if (tid + r * NN_T < m) place[r] = atomicAdd(&end[1 + cell[r]], 1);
+    }
     __syncthreads();
     {  // exclusive prefix sum: NN_CELLS / NN_T neighbours per thread
       constexpr int E = NN_CELLS / NN_T;
@@ -875,23 +886,23 @@ __global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const floa
       __syncthreads();
       int at = incl - own;
       for (int w = 0; w < wave; ++w) at += wsum[w];
-      for (int e = 0; e < E; ++e) { const int v = end[1 + tid * E + e]; end[1 + tid * E + e] = at; at += v; }
+      for (int e = 0; e < E; ++e) { at += end[1 + tid * E + e]; end[1 + tid * E + e] = at; }
     }
     __syncthreads();
-    for (int k = tid; k < m; k += NN_T) {
-      const float x = kp[k * 3], y = kp[k * 3 + 1], z = kp[k * 3 + 2];
-      const int at = atomicAdd(&end[1 + (cell1(z, 2) * g[1] + cell1(y, 1)) * g[0] + cell1(x, 0)], 1);
-      pts[at] = make_float4(x, y, z, __builtin_bit_cast(float, k));
-    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (tid + r * NN_T < m) pts[end[cell[r]] + place[r]] = make_float4(pt[r][0], pt[r][1], pt[r][2], __builtin_bit_cast(float, tid + r * NN_T));
     __syncthreads();
     if (live) {
       const int cx = cell1(ux, 0), cy = cell1(uy, 1), cz = cell1(uz, 2);
-      auto cells = [&](int x0, int x1, int y, int z) {   // cells x0 .. x1 of a row
-        const int c = (z * g[1] + y) * g[0];
-        const int e1 = end[c + x1 + 1];
-        for (int e = end[c + x0]; e < e1; ++e) {
-          const float4 p = pts[e];
+      auto points = [&](int e, int e1) {   // of the sorted list; the next one is on its way while this one is looked at
+        if (e >= e1) return;
+        float4 p = pts[e];
+        for (;;) {
+          const float4 next = pts[min(e + 1, m - 1)];
           best.take(sqdist(ux, uy, uz, p.x, p.y, p.z), __builtin_bit_cast(int, p.w));
+          if (++e >= e1) break;
+          p = next;
         }
       };
       // how near a point of cell row (y, z) can be, squared (0 if it may be nearer than the margin for rounding)
@@ -903,15 +914,28 @@ __global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, const floa
       };
       // cells x0 .. x1 of row (y, z), unless every point of it is farther than the third one
       auto row = [&](int x0, int x1, int y, int z) {
-        if (x0 <= x1 && !(gap(du[1], y) + gap(du[2], z) > best.d3)) cells(x0, x1, y, z);
+        const int c = (z * g[1] + y) * g[0];
+        if (x0 <= x1 && !(gap(du[1], y) + gap(du[2], z) > best.d3)) points(end[c + x0], end[c + x1 + 1]);
       };
       int a0[3], a1[3];   // the cells visited so far: first the block around the point's own, its row first
       const int cc[3] = {cx, cy, cz};
 #pragma unroll
       for (int a = 0; a < 3; ++a) { a0[a] = max(cc[a] - 1, 0); a1[a] = min(cc[a] + 1, g[a] - 1); }
-      for (int t = 0; t < 9; ++t) {
-        const int y = cy + (t == 0 || t == 3 || t == 6 ? 0 : t == 1 || t == 4 || t == 7 ? -1 : 1), z = cz + (t < 3 ? 0 : t < 6 ? -1 : 1);
-        if (y >= a0[1] && y <= a1[1] && z >= a0[2] && z <= a1[2]) row(a0[0], a1[0], y, z);
+      {
+        int from[9], to[9];   // the block's rows, their places read together
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const int y = cy + (t % 3 == 0 ? 0 : t % 3 == 1 ? -1 : 1), z = cz + (t < 3 ? 0 : t < 6 ? -1 : 1);
+          const bool in = y >= a0[1] && y <= a1[1] && z >= a0[2] && z <= a1[2];
+          const int c = in ? (z * g[1] + y) * g[0] : 0;
+          from[t] = end[c + a0[0]];
+          to[t] = in ? end[c + a1[0] + 1] : 0;
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const int y = cy + (t % 3 == 0 ? 0 : t % 3 == 1 ? -1 : 1), z = cz + (t < 3 ? 0 : t < 6 ? -1 : 1);
+          if (!(gap(du[1], y) + gap(du[2], z) > best.d3)) points(from[t], to[t]);
+        }
       }
       for (int r = 2;; r *= 2) {
         // everything within the third distance, if there is one: after that nothing is left to see.  Else a larger block.
@@ -1489,8 +1513,13 @@ int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out,
 int launch_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2, int* idx, hipStream_t st) {
   if (m >= 256 && m <= 8192) {   // fewer: building the grid costs as much as looking at all; more: they do not fit in LDS
     const size_t sm = m * sizeof(float4) + (NN_CELLS + 1) * sizeof(int);
-    if (int e = set_lds_rows(&k_three_nn_grid, sm)) return e;
-    hipLaunchKernelGGL(k_three_nn_grid, dim3((n + NN_T - 1) / NN_T, b), dim3(NN_T), sm, st, n, m, unknown, known, dist2, idx);
+    const int groups = std::max((n + NN_T - 1) / NN_T, std::min(std::max(256 / b, 1), (n + 127) / 128)), share = (n + groups - 1) / groups;
+    auto go = [&](auto kern) -> int {
+      if (int e = set_lds_rows(kern, sm)) return e;
+      hipLaunchKernelGGL(kern, dim3((n + share - 1) / share, b), dim3(NN_T), sm, st, n, m, share, unknown, known, dist2, idx);
+      return 0;
+    };
+    if (int e = m <= 2 * NN_T ? go(&k_three_nn_grid<2>) : m <= 4 * NN_T ? go(&k_three_nn_grid<4>) : go(&k_three_nn_grid<8>)) return e;
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(k_three_nn, dim3((n + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, unknown, known, dist2,

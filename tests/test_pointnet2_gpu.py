@@ -409,6 +409,22 @@ def test_interpolation_rows_keep_a_target_without_a_number_to_its_points(c, m, n
     assert np.abs(g[..., :m - 1] - ref).max() <= 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("b,n,m", [(1, 1, 256), (1, 129, 2048), (2, 1025, 2049), (3, 700, 4096), (1, 33000, 4097), (300, 3, 300), (2, 1024, 8192), (1, 262145, 257)])
+def test_three_nn_shares(b, n, m):
+    """Targets shared by workgroups at the edges of their shares, known points at those of a thread's: the pass over all points by index."""
+    from dest3d_amd.pointnet2_utils import three_nn
+    g = torch.Generator().manual_seed(n + m)
+    u, k = torch.rand(b, n, 3, generator=g).cuda(), torch.rand(b, m, 3, generator=g).cuda()
+    k[:, 1::7] = k[:, :1]     # some in one place: ties go to the smaller index
+    dist, idx = three_nn(u, k)
+    at = torch.unique(torch.tensor([0, n // 3, n // 2, n - 1] + [min(x, n - 1) for x in range(0, n, 127)])).cuda()
+    d = (u[:, at, None].cpu().double() - k[:, None].cpu().double()).pow(2).sum(-1)
+    near = torch.sort(d, dim=-1, stable=True).values[..., :3]
+    got = torch.gather(d, 2, idx[:, at].cpu().long())
+    assert ((got - near).abs() <= 1e-6 * near + 1e-12).all() and ((dist[:, at].cpu().double().pow(2) - near).abs() <= 1e-5 * near + 1e-12).all()
+    assert (idx[:, at, 0] != idx[:, at, 1]).all() and (idx[:, at, 1] != idx[:, at, 2]).all()
+
+
 @pytest.mark.parametrize("m", [255, 256, 257, 2048, 8192, 8193])
 def test_three_nn_grid(m):
     """Both sides of the grid's range; sample 1: a flat sheet with duplicates (ties go to the smaller index), clusters and far
