@@ -280,8 +280,8 @@ KERNEL_OF_STAGE = {"chunk_local": r"k_local_tile\b", "state_passing_fwd": r"k_st
 def measured_traffic(stage):
     """HBM bytes of a stage's kernel launches at the headline workload, as the committed profile summary holds them
     (profiles/issm_fwd_bwd_bidir_fp32_hbm_traffic.md: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this script, scaled by
-    the same counters on a plain copy; last column of the kernel's rows, added up over the stage's launches -- the chunk
-    backward is launched once per direction, and its algorithmic bytes are counted the same way); None if the summary
+    the same counters on a plain copy; last column of the kernel's rows, added up over the launches a step makes -- the chunk
+    backward takes both directions in one); None if the summary
     has no such row."""
     import re
     path = os.path.join(ROOT, "profiles", "issm_fwd_bwd_bidir_fp32_hbm_traffic.md")
