@@ -969,9 +969,8 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
   check_core(in_key, in_query, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
-  // Nothing to differentiate, bf16 and few tokens: the projections in pairs and what follows the scan in one launch, eight
-  // launches a layer where the separate steps take fifteen, and no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us ->
-  // 571; two scenes 768).  The chain's products are issm_linear_fwd's, so it ends where those do (FEW_PRODUCTS: between two and
+  // Nothing to differentiate, bf16 and few tokens: six launches a layer where the separate steps take fifteen, and no autograd nodes (six
+  // layers, 1024 tokens, 256 queries: 871 us -> 571 with eight launches; 497 -> 474 with six for eight behind faster kernels).  The chain's products are issm_linear_fwd's, so it ends where those do (FEW_PRODUCTS: between two and
   // three such scenes) and the separate steps take over -- not because they are faster there: three, four and eight scenes take
   // 1252, 1494 and 2486 us with them, and 980, 1175 and 1942 with the chain and issm_linear_fwd at those sizes too.
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);

@@ -3,8 +3,8 @@
 //
 // At these sizes a product is a few microseconds whoever computes it, and what counts is what it costs to launch: a library
 // product takes 19 us of host time to issue, 4.6 here; a decoder layer has four, and six layers on one scene (1024 tokens, 256
-// queries) ran at the pace of the host: 1180 - 1350 us from process to process, 885 with this.  Without a gradient a layer needs
-// two such launches, the queries turned into the layout of the scan's states on the way.  Both operands have the contraction index contiguous, which is the operand layout of
+// queries) ran at the pace of the host: 1180 - 1350 us from process to process, 885 with this.  Without a gradient a layer's first
+// two are one such launch, the queries turned into the layout of the scan's states on the way (the last two: layer_out.hip).  Both operands have the contraction index contiguous, which is the operand layout of
 // v_mfma_f32_16x16x32_bf16 as it lies in memory: a wave asks for all fragments of its 16 tokens and 32 outputs at once (27 loads
 // of 16 bytes a lane at 288 features) and multiplies as they arrive; there is nothing to share through LDS that L1 does not
 // share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens or features the fragments' 64-byte pieces
