@@ -514,6 +514,10 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
 // equally long up to about this many multiply-adds (2048 x 288 -> 586: 8.5 us against 7.4; 4096: 12.3 against 9.3, 512 -> 512:
 // 24 against 9; above, and where training keeps the GPU busy, the kernel counts).
 constexpr double FEW_PRODUCTS = 3.5e8;
+// A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save: a layer of 288
+// features, 4 and 8 scenes of 1024 tokens and 256 queries 160 -> 137 and 269 -> 244 us (16: 501 and 508), of 192, 8 scenes 231 -> 204; of 384, 2
+// and 4 scenes 133 -> 112, 175 and 179; of 512, 1, 2 and 4 scenes 120 -> 79, 139 -> 126, 201 and 215; of 640, 1 and 2 scenes 137 -> 104, 164 and 167.
+constexpr double CHAIN_PRODUCTS = 1.1e9, CHAIN_PRODUCTS_NARROW = 1.4e9;   // up to 288 features
 // (tensors that stand for something else than their memory, under vmap, functionalization, a tensor subclass or a lazy
 // negation, go to the library's product, which knows them)
 bool own_memory(const Tensor& t) {
@@ -526,11 +530,11 @@ bool own_memory(const Tensor& t) {
 bool watched() {
   return c10::impl::TorchDispatchModeTLS::any_modes_set() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
-bool few_tokens(const Tensor& x, const Tensor& w) {
+bool few_tokens(const Tensor& x, const Tensor& w, double most = FEW_PRODUCTS) {
   if (watched() || !own_memory(x) || !own_memory(w)) return false;
   if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
   if (w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || w.size(1) == 0 || w.size(1) % 32 || x.numel() == 0) return false;
-  return (double)x.numel() * (double)w.size(0) <= FEW_PRODUCTS && x.is_contiguous() && w.is_contiguous() &&
+  return (double)x.numel() * (double)w.size(0) <= most && x.is_contiguous() && w.is_contiguous() &&
          (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
 }
 Tensor linear_few(const Tensor& x, const Tensor& w) {
@@ -969,19 +973,20 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
   check_core(in_key, in_query, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
-  // Nothing to differentiate, bf16 and few tokens: six launches a layer where the separate steps take fifteen, and no autograd nodes (six
-  // layers, 1024 tokens, 256 queries: 871 us -> 571 with eight launches; 497 -> 474 with six for eight behind faster kernels).  The chain's products are issm_linear_fwd's, so it ends where those do (FEW_PRODUCTS: between two and
-  // three such scenes) and the separate steps take over -- not because they are faster there: three, four and eight scenes take
-  // 1252, 1494 and 2486 us with them, and 980, 1175 and 1942 with the chain and issm_linear_fwd at those sizes too.
+  // Nothing to differentiate, bf16 and not too many tokens (CHAIN_PRODUCTS): six launches a layer where the separate steps take fifteen, and
+  // no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us -> 571 with eight launches; 524 -> 474 with six for eight behind faster
+  // kernels; 3, 4 and 8 such scenes, which took the separate steps, 1047 -> 869, 1209 -> 1034 and 1990 -> 1788).
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
   auto plain_bf16 = [&](const Tensor& t) {
     return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.device() == in_key.device() &&
                             t.dim() == 1 && t.size(0) == d_inner && own_memory(t));
   };
+  const double most = d_inner <= 288 ? CHAIN_PRODUCTS_NARROW : CHAIN_PRODUCTS;
   // (functorch's transforms refuse autograd functions, and so this path too)
   bool plain = !at::autocast::is_autocast_enabled(at::kCUDA) &&
-               !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) && few_tokens(in_key, key_proj) && few_tokens(in_query, query_proj) &&
-               few_tokens(in_key, out_key_proj) && few_tokens(in_query, out_query_proj) && in_query.device() == in_key.device() &&
+               !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) && few_tokens(in_key, key_proj, most) &&
+               few_tokens(in_query, query_proj, most) && few_tokens(in_key, out_key_proj, most) &&
+               few_tokens(in_query, out_query_proj, most) && in_query.device() == in_key.device() &&
                in_key.size(-1) == d_inner && in_query.size(-1) == d_inner && query_proj.size(0) == d_inner && d_inner % 4 == 0 &&
                d_inner <= 1024 && plain_bf16(key_norm) && plain_bf16(query_wt) && plain_bf16(query_bt);
   for (const Tensor* t : std::initializer_list<const Tensor*>{&in_key, &in_query, &dist, &key_proj, &query_proj, &out_key_proj,

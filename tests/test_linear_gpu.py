@@ -407,3 +407,14 @@ def test_checkpointed_layers(reentrant):
     want = step(lambda layer, k, q: layer(k, q, dist, None))
     got = step(lambda layer, k, q: checkpoint(layer, k, q, dist, None, use_reentrant=reentrant))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("B,Ln,K", [(3, 1000, 40), (8, 1024, 64)])
+def test_layer_without_a_gradient_of_several_scenes(B, Ln, K):
+    """Beyond the sizes whose single products the layer's own kernel takes, up to the chain's limit; bounds as above."""
+    test_layer_without_a_gradient(B, Ln, K, "weights")
+
+
+@pytest.mark.parametrize("D,H,Ln", [(512, 8, 1000), (640, 10, 300)])
+def test_wide_layer_without_a_gradient_against_fp64(D, H, Ln):
+    test_layer_without_a_gradient_against_fp64(D, H, 1, True, 1, Ln, 33, "weights")
