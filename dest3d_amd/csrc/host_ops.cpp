@@ -6,10 +6,12 @@
 // kernels (and, for the layer's four projections, in the tensor library's matrix products).
 #include <Python.h>
 
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/extension.h>
 
 #include "../../include/issm.h"
@@ -530,6 +532,15 @@ bool own_memory(const Tensor& t) {
 bool watched() {
   return c10::impl::TorchDispatchModeTLS::any_modes_set() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer);
 }
+// Whether this may be one of the two runs of a checkpointed segment, which are to give the same bits although the first of them (reentrant
+// checkpointing) or the second records no gradient here.  A reentrant segment runs first in the forward of an autograd function --
+// there, and in inference mode, forward-mode derivatives are off -- and again in a backward pass; one of the other kind with hooks on
+// saved tensors both times.
+bool runs_twice() {
+  const c10::AutogradState& s = c10::AutogradState::get_tls_state();
+  return (!s.get_fw_grad_mode() && !s.get_inference_mode()) || torch::autograd::get_current_graph_task_id() >= 0 ||
+         (s.get_grad_mode() && !at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
+}
 bool few_tokens(const Tensor& x, const Tensor& w, double most = FEW_PRODUCTS) {
   if (watched() || !own_memory(x) || !own_memory(w)) return false;
   if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
@@ -995,9 +1006,8 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     if (!plain) break;
     plain = !t->defined() || (own_memory(*t) && !(at::GradMode::is_enabled() && t->requires_grad()) && !t->_fw_grad(0).defined());
   }
-  // Activations that want a gradient while none is recorded: the first run of a checkpointed segment (reentrant checkpointing),
-  // which a second one with gradients is to repeat.  Both take the same kernels.
-  plain = plain && !(in_key.requires_grad() || in_query.requires_grad() || dist.requires_grad());
+  // A run that another is to repeat takes the kernels of one with gradients.
+  plain = plain && !runs_twice() && !(in_key.requires_grad() || in_query.requires_grad() || dist.requires_grad());
   if (plain) {
     const c10::DeviceGuard guard(in_key.device());
     const int64_t B = in_key.size(0), Ln = in_key.size(1), H = nheads, G = ngroups, di = d_inner, P = di / H, Cc = di + 2 * G,

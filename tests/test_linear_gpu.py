@@ -409,6 +409,63 @@ def test_checkpointed_layers(reentrant):
     assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("B,Ln,K", [(2, 130, 40), (4, 1000, 40)])
+def test_checkpointed_segments_of_several_layers(B, Ln, K):
+    """Segments of two layers under reentrant checkpointing, one scene's products and several scenes': only a segment's own inputs want a
+    gradient in its first run, and the layers behind the first take training's kernels in it all the same."""
+    from torch.utils.checkpoint import checkpoint
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(9)
+    layers = [MultiHeadISSMScan(d_model=288, d_state=K, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16() for _ in range(4)]
+    for layer in layers:
+        layer.dt_bias.data += 6.0   # steps long enough for chunks out of a tile's range
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    key, query, dist, dkey, dquery = bf(B, Ln, 288), bf(B, K, 288), bf(B, Ln, K, 16), bf(B, Ln, 288), bf(B, K, 288)
+
+    def segment(first):
+        def run(k, q):
+            for layer in layers[first:first + 2]:
+                ok, oq = layer(k, q, dist, None)
+                k, q = k + ok, q + oq
+            return k, q
+        return run
+
+    def step(wrap):
+        k, q = key.clone().requires_grad_(), query.clone().requires_grad_()
+        for layer in layers:
+            layer.zero_grad(set_to_none=True)
+        out = wrap(segment(2), *wrap(segment(0), k, q))
+        torch.autograd.backward(out, (dkey, dquery))
+        return *out, k.grad, q.grad, *(p.grad for layer in layers for p in layer.parameters())
+
+    want = step(lambda f, *x: f(*x))
+    got = step(lambda f, *x: checkpoint(f, *x, use_reentrant=True))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with torch.no_grad():
+        plain = segment(0)(key, query)
+    with torch.inference_mode():   # no backward can follow there, although forward-mode derivatives are off as in an autograd function
+        assert all(torch.equal(a, b) for a, b in zip(segment(0)(key, query), plain))
+
+
+@pytest.mark.parametrize("reentrant", [True, False])
+def test_both_runs_of_a_segment_with_a_frozen_layer(reentrant):
+    """A layer that nothing is differentiated through, in a segment that is run twice."""
+    from torch.utils.checkpoint import checkpoint
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(9)
+    layer = MultiHeadISSMScan(d_model=288, d_state=40, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16().requires_grad_(False)
+    layer.dt_bias.data += 6.0
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    key, query, dist, scale, seen = bf(2, 130, 288), bf(2, 40, 288), bf(2, 130, 40, 16), bf(2, 130, 288).requires_grad_(), []
+
+    def segment(s):
+        seen.append(layer(key, query, dist, None))
+        return seen[-1][0] * s
+
+    checkpoint(segment, scale, use_reentrant=reentrant).sum().backward()
+    assert len(seen) == 2 and all(torch.equal(a, b) for a, b in zip(*seen)) and torch.equal(scale.grad, seen[0][0])
+
+
 @pytest.mark.parametrize("B,Ln,K", [(3, 1000, 40), (8, 1024, 64)])
 def test_layer_without_a_gradient_of_several_scenes(B, Ln, K):
     """Beyond the sizes whose single products the layer's own kernel takes, up to the chain's limit; bounds as above."""
