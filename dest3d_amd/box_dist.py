@@ -208,7 +208,8 @@ class BoxDistFun(nn.Module):
                 ps[2].shape != (CHANNELS, w.shape[0]) or not coords.is_contiguous() or coords.device != w.device or \
                 (torch.is_grad_enabled() and (coords.requires_grad or any(p.requires_grad for p in ps))) or \
                 any(p.dtype != w.dtype or p.device != w.device or not p.is_contiguous() or
-                    type(p) not in (nn.Parameter, torch.Tensor) for p in ps):
+                    type(p) not in (nn.Parameter, torch.Tensor) for p in ps) or \
+                L.host().runs_twice():     # a checkpointed segment's run: both of them take the sums of one with gradients
             return None
         n = _lattice(coords)
         if n is None:

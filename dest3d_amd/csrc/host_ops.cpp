@@ -1144,6 +1144,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::gil_scoped_release release;
     return linear_tokens(x, w);
   });
+  m.def("runs_twice", &runs_twice);
   m.def("scan_core", &scan_core);
   m.def("scan_layer", &scan_layer);
 }

@@ -251,6 +251,32 @@ def test_table_of_a_replaced_lattice(shape):
     assert want is None and got is None or torch.equal(got, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_encoding_in_a_checkpointed_segment(dtype):
+    """Reentrant checkpointing runs a segment without gradients first: the encoding's sums and its table are training's in that run too, so
+    that outputs and gradients are those of the segment that is not checkpointed."""
+    from torch.utils.checkpoint import checkpoint
+    from dest3d_amd.box_dist import BoxDistFun
+    torch.manual_seed(2)
+    m = BoxDistFun(out_dim=16).cuda().to(dtype)
+    key, qxyz, qsize, ang = (torch.from_numpy(x).cuda() for x in _inputs(2, 300, 64, 8, False))
+    boxes, scale, dout = torch.cat([qxyz, qsize], dim=-1), torch.rand(2, 300, 64, 16).cuda().to(dtype), torch.randn(2, 300, 64, 16).cuda().to(dtype)
+
+    def segment(s):
+        dist, weights = m(key, boxes[..., :3], boxes[..., 3:], ang, weight_query_pos=boxes)
+        return dist * s, weights
+
+    def step(run):
+        s = scale.clone().requires_grad_()
+        m.zero_grad(set_to_none=True)
+        out, weights = run(s)
+        out.backward(dout)
+        return out, weights, s.grad, *(p.grad for p in m.parameters())
+
+    want, got = step(segment), step(lambda s: checkpoint(segment, s, use_reentrant=True))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_operands_of_another_size_or_device_are_refused():
     """Refused before a kernel is given their address."""
     from dest3d_amd.box_dist import box_dist, box_parametrization_to_corners, local_weight
