@@ -177,7 +177,7 @@ class Runner:
         return (time.perf_counter() - t0) / steps * 1e6
 
     def capture(self):
-        """Record one step (forward + backward, 9 kernel launches, no allocation, no memset) into a HIP graph on a side
+        """Record one step (forward + backward, no allocation, no memset) into a HIP graph on a side
         stream of default priority and return the graph."""
         torch = self.torch
         side = torch.cuda.Stream()
@@ -242,8 +242,7 @@ class Runner:
               if lib.issm_bwd_walks(C.byref(a)) else
               [("bwd_dstates", lambda: lib.issm_stage_bwd_dstates(C.byref(a), None, p(dst), p(dm))),
                ("state_passing_bwd", lambda: lib.issm_stage_state_passing_bwd(C.byref(a), None, p(csl), p(dst), None, p(dh0d)))]),
-            ("bwd_chunk", lambda: [lib.issm_stage_bwd_chunk(C.byref(a), d, None, p(st), p(dst), p(dm), None, p(pa), p(pb), p(redo))
-                                   for d in range(nd)][-1]),
+            ("bwd_chunk", lambda: lib.issm_stage_bwd_chunk(C.byref(a), -1, None, p(st), p(dst), p(dm), None, p(pa), p(pb), p(redo))),
             ("bwd_dx", lambda: lib.issm_stage_bwd_dx(C.byref(a), None, p(dst), p(cabt), p(pd))),
             ("bwd_reduce", lambda: lib.issm_stage_bwd_reduce(C.byref(a), p(pa), p(pb), p(pd), p(dh0d))),
         ]
@@ -320,7 +319,7 @@ def stage_work(ndir, shape=None, elt=4):
         "bwd_states": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m + 2 * E_st)),
         # the same in two launches: reads dt, C, dy, x; writes dH, dM; and the recurrence
         "bwd_dstates": (2 * U * (cs * P * N + tri * P), s * (E_dt + E_bc + 2 * E_x) + 4 * (E_cs + E_m)),
-        # all launches: read dt, x, dy, B, C, H, dS, dM; write ddt, dB, dC, the dA / ddt_bias partials
+        # both directions in one launch or one after the other: read dt, x, dy, B, C, H, dS, dM; write ddt, dB, dC, the dA / ddt_bias partials
         "bwd_chunk": (2 * U * (2 * cs * P * N + 2 * tri * N),
                       s * (2 * E_dt + 2 * E_x + 4 * E_bc) + 4 * (2 * E_cs + E_m + 2 * E_v)),
         # reads dt, B, dy, x, dS, M; writes dx

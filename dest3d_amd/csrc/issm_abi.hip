@@ -431,19 +431,24 @@ int issm_stage_bwd_chunk(const issm_scan_args* a, int dir, const float* dy_gated
   int rc = check_common(a);
   if (rc) return rc;
   if ((rc = check_dout(a, dy_gated))) return rc;
-  if (dir < 0 || dir >= a->dims.ndir) return fail(ISSM_E_SHAPE, "dir %d out of range", dir);
+  if (dir < -1 || dir >= a->dims.ndir) return fail(ISSM_E_SHAPE, "dir %d out of range", dir);
   if (!states || !dstates || !dm || !part_a || !part_bias) return fail(ISSM_E_NULL, "bwd_chunk: NULL buffer");
   KP p = make_kp(a);
-  p.dir0 = dir;
+  hipStream_t st = (hipStream_t)a->stream;
+  const bool dual = dir < 0 && redo && bwd_tile_dual(p, dy_gated, bwd_head_parts(a->dims));
+  const int first = std::max(dir, 0), last = dir < 0 && !dual ? p.ndir - 1 : first;
   int pending = 0;
-  if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1, false,
-                                      nullptr, nullptr, nullptr, (hipStream_t)a->stream),
-                     "bwd_chunk")))
-    return rc;
-  if (!pending) return ISSM_OK;
-  return launched(launch_bwd_chunk_redo(p, 1, dy_gated, states, dstates, dm, part_a, part_bias, redo,
-                                        (hipStream_t)a->stream),
-                  "bwd_chunk (redo)");
+  for (int d = first; d <= last; ++d) {
+    p.dir0 = d;
+    if ((rc = launched(launch_bwd_chunk(p, dy_gated, states, dstates, dm, part_a, part_bias, redo, &pending, 1, dual,
+                                        nullptr, nullptr, nullptr, st),
+                       "bwd_chunk")))
+      return rc;
+    if (pending && (rc = launched(launch_bwd_chunk_redo(p, dual ? 2 : 1, dy_gated, states, dstates, dm, part_a, part_bias, redo, st),
+                                  "bwd_chunk (redo)")))
+      return rc;
+  }
+  return ISSM_OK;
 }
 
 int issm_stage_bwd_dx(const issm_scan_args* a, const float* dy_gated, const float* dstates, const float* cabt,

@@ -221,7 +221,7 @@ int issm_bwd_walks(const issm_scan_args* args);
 /* issm_stage_bwd_chunk: ddt, dB, dC of direction `dir` and the per-unit partial sums
  *   part_a / part_bias (Bt*nc,H,N) of dA / ddt_bias.  g_last is not read (the kernels form it from states, dstates and
  *   their own products) and may be NULL.  ddt accumulates into args->ddt when
- *   dir > 0.  Replaces _chunk_state_bwd_db (issm_chunk_state.py:493-652), _chunk_scan_bwd_dc
+ *   dir > 0.  dir = -1: every direction, in one launch where issm_scan_bwd takes them in one.  Replaces _chunk_state_bwd_db (issm_chunk_state.py:493-652), _chunk_scan_bwd_dc
  *   (issm_chunk_scan.py:515-657), _chunk_scan_chunk_state_bwd_dt (issm_combined.py:398-557),
  *   _bmm_CABT_dbc_chunk_bwd (issm_cabt_bmm.py:454-673), _chunk_scan_bwd_ddAcs_stable
  *   (issm_chunk_scan.py:903-1031) and the elementwise part of _chunk_cumsum_bwd

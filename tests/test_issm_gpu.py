@@ -1570,6 +1570,46 @@ def test_both_directions_of_the_chunk_backward_in_one_launch(dtype, P, H, G, far
         assert err <= (2.5e-3 if dtype == "bf16" else 5e-6 if k not in (2, 3) or not far else 5e-5), (k, err)
 
 
+@pytest.mark.parametrize("B,L_,P,N,one", [(3, 960, 32, 512, True), (3, 960, 24, 512, False), (1, 100, 32, 70, False)])
+def test_stage_of_the_chunk_backward_in_every_direction(B, L_, P, N, one):
+    """Direction -1 of the stage entry point, as issm_scan_bwd launches the directions (one launch for both or one each), against the two
+    directions by number: a head a group, so that no order of heads is in the sums; fp32 sums of two shares, added in either order."""
+    H = G = 2
+    d = _problem(B, L_, H, P, N, G, seed=N + P, softplus=False)
+    d["dt"], d["A"] = 0.1 * torch.rand(d["dt"].shape, generator=torch.Generator().manual_seed(N)), 0.25 * d["A"]
+    L, prob, a = _stage_args(d)
+    lib, nc = L.load(), math.ceil(L_ / 64)
+    a.dims.ndir = 2
+    assert (L_ % 64 == 0 and N % 64 == 0 and P == 32 and B * nc * G * math.ceil(N / 64) > 320) == one
+    g = torch.Generator(device="cuda").manual_seed(P)
+    r = lambda *s, scale=1.0: scale * torch.randn(*s, generator=g, device="cuda")
+    back = [r(B, L_, H, P), r(B, L_, G, N), r(B, L_, G, N)]
+    a.x[1], a.Bm[1], a.Cm[1] = (L.tensor_desc(t) for t in back)
+    dy, states, dst = [r(B, L_, H, P) for _ in range(2)], r(2 * B, nc + 1, H, P, N), r(2 * B, nc, H, P, N)
+    w = torch.tril(r(2 * B, nc, H, 64, 64))
+    w = w + torch.tril(w, -1).transpose(-1, -2)
+    hi = w.bfloat16()
+    dm = torch.stack([hi, (w - hi.float()).bfloat16()], dim=3).contiguous()
+    for i in range(2):
+        a.dout[i] = L.tensor_desc(dy[i])
+    out = []
+    for dirs in ((0, 1), (-1,)):
+        f = lambda *s: torch.full(s, float("nan"), device="cuda")
+        t = [f(B, L_, H, N), *(f(B, L_, G, N) for _ in range(4)), f(2 * B * nc, H, N), f(2 * B * nc, H, N)]
+        a.ddt, a.dB[0], a.dB[1], a.dC[0], a.dC[1] = (L.tensor_desc(q) for q in t[:5])
+        redo = torch.full((lib.issm_bwd_chunk_redo_ints(C.byref(a)),), -1, dtype=torch.int32, device="cuda")
+        for i in dirs:
+            L.check(lib.issm_stage_bwd_chunk(C.byref(a), i, None, states.data_ptr(), dst.data_ptr(), dm.data_ptr(), None, t[5].data_ptr(),
+                                             t[6].data_ptr(), redo.data_ptr()), "bwd_chunk")
+        torch.cuda.synchronize()
+        out.append((t, redo))
+    assert torch.equal(out[0][1], out[1][1]) and bool((out[0][1] == 0).all())
+    for x, y in zip(out[1][0], out[0][0]):
+        assert ((x.double() - y.double()).norm() / y.double().norm()).item() <= (1e-6 if one else 0.0)
+    assert lib.issm_stage_bwd_chunk(C.byref(a), -2, None, states.data_ptr(), dst.data_ptr(), dm.data_ptr(), None, t[5].data_ptr(),
+                                    t[6].data_ptr(), None) != 0
+
+
 @pytest.mark.parametrize("L_,P,N,far", [(128, 36, 256, 0), (128, 64, 256, 1), (64, 32, 128, 1), (90, 20, 200, 0), (70, 48, 68, 1)])
 def test_bf16_forward_of_the_steps_behind_a_far_tile(L_, P, N, far):
     """issm_scan_fwd_only: 16 columns of the step `far` decay beyond 2^100 a tile, so their wave takes that step and those behind it, whose
