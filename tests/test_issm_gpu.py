@@ -700,11 +700,11 @@ def test_bf16_forward_of_any_decay(L_, P, N, only):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("L_,N,H,ndir", [(128, 128, 6, 1), (100, 70, 5, 2), (256, 64, 3, 2), (1600, 256, 7, 1), (130, 8, 5, 1)])
+@pytest.mark.parametrize("L_,N,H,ndir", [(128, 128, 6, 1), (100, 70, 5, 2), (256, 64, 3, 2), (1600, 256, 7, 1), (130, 8, 5, 1), (1600, 320, 8, 1)])
 @pytest.mark.parametrize("marked", [False, True])
 def test_heads_shared_by_several_workgroups(dtype, L_, N, H, ndir, marked):
     """Few chunks and states: several workgroups of the chunk backward share the heads of a group (7 heads at 1600 tokens and
-    256 states: parts of 2, 2, 2 and 1), some heads with decays that the level-hierarchy kernel adds afterwards.  Against calls
+    256 states: parts of 2, 2, 2 and 1), some heads (1 and the last, or those of `marked`) with decays that the level-hierarchy kernel adds afterwards.  Against calls
     of one head each: a head's own gradients bit for bit, those of B and C to the rounding of the sum (and, bf16, of the single
     heads' results)."""
     from dest3d_amd import ISSM_biscan_combined, ISSM_chunk_scan_combined
@@ -712,8 +712,8 @@ def test_heads_shared_by_several_workgroups(dtype, L_, N, H, ndir, marked):
     d = _problem(2 if L_ < 1000 else 1, L_, H, 24, N, 1, seed=L_ + H, softplus=False)
     d["dt"] = d["dt"].abs()
     if marked:
-        d["A"][1] = -80.0 * (1.0 + torch.rand(N, generator=torch.Generator().manual_seed(1)))
-        d["A"][H - 1] = d["A"][1]
+        for h in (1, H - 1) if marked is True else marked:
+            d["A"][h] = -80.0 * (1.0 + torch.rand(N, generator=torch.Generator().manual_seed(1)))
     io = ("x", "dt", "B", "C")
     q = {k: d[k].cuda().to(dtype if k in io else torch.float32) for k in ("x", "dt", "B", "C", "A", "D", "h0")}
     dy, dl = d["dy"].cuda(), d["dfinal"].cuda()
@@ -1659,10 +1659,18 @@ def test_outputs_by_one_and_by_two_groups_of_waves(dtype, L_, N, P, gated):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("L_,N,H,marked", [(128, 128, 4, True), (100, 70, 4, True), (100, 70, 4, False), (64, 64, 2, False), (1600, 320, 8, True)])
+@pytest.mark.parametrize("L_,N,H,marked", [(128, 128, 4, True), (100, 70, 4, True), (100, 70, 4, False), (64, 64, 2, False),
+                                           (128, 128, 4, (1,)), (100, 70, 4, (1,)), (128, 128, 4, (0, 3)), (100, 70, 4, (0, 3)),
+                                           (1600, 512, 8, (1, 6)), (1590, 512, 8, (2, 4, 7))])
 def test_heads_two_at_a_time(dtype, L_, N, H, marked):
     """Calls of one direction with an even number of heads a group and few chunks: two heads side by side in a workgroup of the chunk backward,
-    heads out of range in either half of it.  As above, against calls of one head each."""
+    heads 0 .. H / 2 - 1 in the one half of it and the others in the other.  Heads out of range in both halves at once, in one at a time (the other
+    half's head stands at its barriers), in neither.  As above, against calls of one head each."""
+    blocks = (2 if L_ < 1000 else 1) * math.ceil(L_ / 64) * math.ceil(N / 64)
+    most = min(H, 512 // blocks)
+    assert blocks <= 256 and (most <= 3 or H - math.ceil(H / most) < 4)   # heads are not shared between workgroups instead
+    if isinstance(marked, tuple):
+        assert any((h in marked) != (h + H // 2 in marked) for h in range(H // 2))
     test_heads_shared_by_several_workgroups(dtype, L_, N, H, 1, marked)
 
 

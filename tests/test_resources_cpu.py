@@ -50,15 +50,24 @@ def kernels():
     return {re.sub(r"^void |issm::|\(.*", "", p): found[n] for n, p in zip(found, plain)}
 
 
-@pytest.mark.parametrize("name,variants,registers", [
+@pytest.mark.parametrize("name,variants,registers,spilled", [
     # rows' gradient, one set a workgroup of 16 waves: two workgroups a CU
-    (r"k_interp_rows_grad<[124], (true|false), false>", 4, 64),
+    (r"k_interp_rows_grad<[124], (true|false), false>", 4, 64, 0),
     # chunk backward in tile-base form, incomplete tiles: two of four waves
-    (r"k_bwd_tile<[234], true, false, (true|false), (true|false), false, (true|false)>", 24, 256),
-    (r"k_bwd_tile<[234], false, false, (true|false), false, false, (true|false)>", 12, 256),
+    (r"k_bwd_tile<[234], true, false, (true|false), (true|false), false, (true|false)>", 24, 256, 0),
+    (r"k_bwd_tile<[234], false, false, (true|false), false, false, (true|false)>", 12, 256, 0),
+    # both directions, and two heads side by side: one workgroup of eight waves
+    (r"k_bwd_tile<1[012], (true|false), (true|false), false, false, true, false>", 7, 256, 0),
+    (r"k_bwd_tile<(18|19|20), (true|false), (true|false), false, false, (true|false), false>", 18, 256, 8),   # (fp32 heads of 33 to 47, complete tiles)
+    # two groups of four waves: with up to two head tiles two workgroups a CU
+    (r"(k_chunk_scan|k_bwd_dx)<2, (true|false), (true|false), (true|false), 2>", 16, 128, 0),
+    (r"(k_chunk_scan|k_bwd_dx)<[34], (true|false), (true|false), (true|false), 2>", 32, 256, 0),
+    # workgroups of sixteen waves
+    (r"(k_layer_end|k_three_nn_grid|k_box_dist_fwd)<.*>", 12, 128, 0),
 ])
-def test_registers_leave_room_for_the_workgroups(kernels, name, variants, registers):
+def test_registers_leave_room_for_the_workgroups(kernels, name, variants, registers, spilled):
     hit = {k: v for k, v in kernels.items() if re.fullmatch(name, k)}
     assert len(hit) == variants
     for k, (r, scratch) in hit.items():
-        assert r <= registers and scratch == 0, (k, r, scratch)
+        assert r <= registers and scratch <= spilled, (k, r, scratch)
+    assert sum(scratch for _, scratch in hit.values()) == spilled
