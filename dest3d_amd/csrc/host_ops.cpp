@@ -520,6 +520,12 @@ constexpr double FEW_PRODUCTS = 3.5e8;
 // features, 4 and 8 scenes of 1024 tokens and 256 queries 160 -> 137 and 269 -> 244 us (16: 501 and 508), of 192, 8 scenes 231 -> 204; of 384, 2
 // and 4 scenes 133 -> 112, 175 and 179; of 512, 1, 2 and 4 scenes 120 -> 79, 139 -> 126, 201 and 215; of 640, 1 and 2 scenes 137 -> 104, 164 and 167.
 constexpr double CHAIN_PRODUCTS = 1.1e9, CHAIN_PRODUCTS_NARROW = 1.4e9;   // up to 288 features
+// The chain's convolutions and generation of dt, B and C are one launch up to this many threads of the generation, two queries each where their
+// number is even: the first wave of a workgroup convolves while the others wait, and from 0.6 million threads on that costs more than the
+// launch and what lies between the two.  8 heads, 64 features, 256 queries, scenes of 1024 tokens: 2 64 us in one launch and 67 in two, 5 121
+// and 121, 10 207 and 199, 31 624 and 580; 288 features 86 and 89, 166 and 165, 308 and 301, 970 and 923; 51 queries, 64 features, 12, 24 and 98
+// scenes 130 and 129, 230 and 220, 922 and 850.
+constexpr int64_t JOINED_THREADS = 600000;
 // (tensors that stand for something else than their memory, under vmap, functionalization, a tensor subclass or a lazy
 // negation, go to the library's product, which knows them)
 bool own_memory(const Tensor& t) {
@@ -984,7 +990,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
   check_core(in_key, in_query, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
-  // Nothing to differentiate, bf16 and not too many tokens (CHAIN_PRODUCTS): six launches a layer where the separate steps take fifteen, and
+  // Nothing to differentiate, bf16 and not too many tokens (CHAIN_PRODUCTS): six or seven launches a layer where the separate steps take fifteen, and
   // no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us -> 571 with eight launches; 524 -> 474 with six for eight behind faster
   // kernels; 3, 4 and 8 such scenes, which took the separate steps, 1047 -> 869, 1209 -> 1034 and 1990 -> 1788).
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
@@ -1025,9 +1031,11 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
                                                            &A_log, &D};
     const int64_t nflat = CoreFn::offsets(arrays, off);
     const Tensor d = cast(dist, at::kBFloat16).contiguous(), wt = f32c(wts);
-    enum { ZX, H0, FLAT, A1, X, DT, BC, Y, LAST, WS, PARTS };
-    const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di,
-                                  2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di, 8 * B * di * K, (int64_t)ws_bytes};
+    const bool joined = B * Ln * (K % 2 ? K : K / 2) <= JOINED_THREADS;
+    enum { ZX, H0, FLAT, A1, X, TAIL, PRE, DT, BC, Y, LAST, WS, PARTS };
+    const int64_t bytes[PARTS] = {2 * B * Ln * W, 2 * B * di * K, 4 * nflat, 4 * H * K, 4 * B * Ln * di, joined ? 0 : 8 * B * Ln * G,
+                                  joined ? 0 : 4 * B * Ln * Cc, 2 * B * Ln * H * K, 8 * B * Ln * G * K, 4 * B * Ln * di, 8 * B * di * K,
+                                  (int64_t)ws_bytes};
     int64_t at_[PARTS + 1] = {0};
     for (int i = 0; i < PARTS; ++i) at_[i + 1] = at_[i] + (bytes[i] + 255) / 256 * 256;
     const Tensor arena = fresh({at_[PARTS]}, in_key, at::kByte);
@@ -1074,7 +1082,14 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
       a.Bm_back = bc[2];
       a.Cm_back = bc[3];
       a.weights = data<const float>(wt);
-      check(issm_conv_param_gen_fwd(&c, &a), "issm_conv_param_gen_fwd");
+      if (joined) {
+        check(issm_conv_param_gen_fwd(&c, &a), "issm_conv_param_gen_fwd");
+      } else {
+        c.pre = part(PRE);
+        a.tail = c.y_tail = part(TAIL);
+        check(issm_dwconv_silu_fwd(&c), "issm_dwconv_silu_fwd");
+        check(issm_param_gen_fwd_only(&a), "issm_param_gen_fwd_only");
+      }
     }
     s.flags = (wt.defined() ? 0u : ISSM_FLAG_DT_SOFTPLUS) | (D.dim() == 2 ? ISSM_FLAG_D_HAS_HDIM : 0u);
     s.dt_min = (float)lo;

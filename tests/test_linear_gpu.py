@@ -466,9 +466,10 @@ def test_both_runs_of_a_segment_with_a_frozen_layer(reentrant):
     assert len(seen) == 2 and all(torch.equal(a, b) for a, b in zip(*seen)) and torch.equal(scale.grad, seen[0][0])
 
 
-@pytest.mark.parametrize("B,Ln,K", [(3, 1000, 40), (8, 1024, 64)])
+@pytest.mark.parametrize("B,Ln,K", [(3, 1000, 40), (8, 1024, 64), (8, 1024, 160), (8, 1024, 77)])
 def test_layer_without_a_gradient_of_several_scenes(B, Ln, K):
-    """Beyond the sizes whose single products the layer's own kernel takes, up to the chain's limit; bounds as above."""
+    """Beyond the sizes whose single products the layer's own kernel takes, up to the chain's limit, the convolutions and the generation in
+    one launch and, with an even and an odd number of queries, in two; bounds as above."""
     test_layer_without_a_gradient(B, Ln, K, "weights")
 
 
