@@ -516,10 +516,17 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
 // equally long up to about this many multiply-adds (2048 x 288 -> 586: 8.5 us against 7.4; 4096: 12.3 against 9.3, 512 -> 512:
 // 24 against 9; above, and where training keeps the GPU busy, the kernel counts).
 constexpr double FEW_PRODUCTS = 3.5e8;
-// A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save: a layer of 288
-// features, 4 and 8 scenes of 1024 tokens and 256 queries 160 -> 137 and 269 -> 244 us (16: 501 and 508), of 192, 8 scenes 231 -> 204; of 384, 2
-// and 4 scenes 133 -> 112, 175 and 179; of 512, 1, 2 and 4 scenes 120 -> 79, 139 -> 126, 201 and 215; of 640, 1 and 2 scenes 137 -> 104, 164 and 167.
-constexpr double CHAIN_PRODUCTS = 1.1e9, CHAIN_PRODUCTS_NARROW = 1.4e9;   // up to 288 features
+// A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save, as long as
+// it is ahead for 16 to 512 queries (multiples of 32 up to 640 features; separate steps and chain in us, scenes of 1024 tokens and 256
+// queries unless said).  288 features, 4, 8, 11 and 16 scenes: 159 and 138, 269 and 242, 347 and 327, 504 and 492; 192, 16 scenes: 432 and 400; 96, 62:
+// 1229 and 1152.  Rows of 128 bytes and multiples of them suit its products least: 64 features, 64 queries, 59, 89 and 135 scenes 527 and 505, 751
+// and 749, 1093 and 1112, 16 queries, 31 and 47 scenes of 2048 449 and 447, 649 and 677; 128, 16 queries, 12 and 20 scenes of 2048 221 and 216, 329 and
+// 341; 320, whose ten fragments take two requests of eight, 3, 4, 5 and 6 scenes 153 and 134, 170 and 169, 200 and 212, 222 and 233; 384, 3 and 4
+// scenes 153 and 145, 175 and 180; 512, 2, 3 and 4 scenes 140 and 126, 166 and 160, 202 and 217; 640, 1 and 2 scenes 132 and 106, 165 and 168.  (Wider odd
+// multiples of 32 would stay ahead for longer: 352, 7 scenes, 268 and 251, 480, 5 scenes, 232 and 218.)
+double chain_products(int64_t features) {
+  return features <= 64 ? 5.5e8 : features == 320 ? 8.6e8 : features == 128 || features > 288 ? 1.1e9 : 1.4e9;
+}
 // The chain's convolutions and generation of dt, B and C are one launch up to this many threads of the generation, two queries each where their
 // number is even: the first wave of a workgroup convolves while the others wait, and from 0.6 million threads on that costs more than the
 // launch and what lies between the two.  8 heads, 64 features, 256 queries, scenes of 1024 tokens: 2 64 us in one launch and 67 in two, 5 121
@@ -990,7 +997,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
   check_core(in_key, in_query, dist, opt(weights_), d_inner, nheads, ngroups,
              {&conv_w_f, &conv_b_f, &conv_w_b, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D, &key_norm});
   py::gil_scoped_release release;
-  // Nothing to differentiate, bf16 and not too many tokens (CHAIN_PRODUCTS): six or seven launches a layer where the separate steps take fifteen, and
+  // Nothing to differentiate, bf16 and not too many tokens (chain_products): six or seven launches a layer where the separate steps take fifteen, and
   // no autograd nodes (six layers, 1024 tokens, 256 queries: 871 us -> 571 with eight launches; 524 -> 474 with six for eight behind faster
   // kernels; 3, 4 and 8 such scenes, which took the separate steps, 1047 -> 869, 1209 -> 1034 and 1990 -> 1788).
   const Tensor query_wt = opt(query_w), query_bt = opt(query_b), wts = opt(weights_);
@@ -998,7 +1005,7 @@ std::vector<Tensor> scan_layer(const Tensor& in_key, const Tensor& in_query, con
     return !t.defined() || (t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.device() == in_key.device() &&
                             t.dim() == 1 && t.size(0) == d_inner && own_memory(t));
   };
-  const double most = d_inner <= 288 ? CHAIN_PRODUCTS_NARROW : CHAIN_PRODUCTS;
+  const double most = chain_products(d_inner);
   // (functorch's transforms refuse autograd functions, and so this path too)
   bool plain = !at::autocast::is_autocast_enabled(at::kCUDA) &&
                !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) && few_tokens(in_key, key_proj, most) &&

@@ -473,6 +473,20 @@ def test_layer_without_a_gradient_of_several_scenes(B, Ln, K):
     test_layer_without_a_gradient(B, Ln, K, "weights")
 
 
+@pytest.mark.parametrize("D,B,short", [(32, 110, True), (64, 60, True), (64, 61, False), (128, 31, True), (128, 32, False), (288, 8, True), (288, 9, False), (320, 4, True), (320, 5, False),
+                                       (384, 3, True), (384, 4, False)])
+def test_layer_without_a_gradient_takes_the_shorter_chain_where_it_is_the_faster(D, B, short):
+    """Scenes of 1024 tokens, told by the number of allocations."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    layer = MultiHeadISSMScan(d_model=D, d_state=8, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    x = [torch.zeros(s, device="cuda", dtype=torch.bfloat16) for s in ((B, 1024, D), (B, 8, D), (B, 1024, 8, 16))]
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    with torch.no_grad():
+        before = count()
+        layer(*x, None, None)
+        assert (count() - before <= 3) == short
+
+
 @pytest.mark.parametrize("D,H,Ln", [(512, 8, 1000), (640, 10, 300)])
 def test_wide_layer_without_a_gradient_against_fp64(D, H, Ln):
     test_layer_without_a_gradient_against_fp64(D, H, 1, True, 1, Ln, 33, "weights")
