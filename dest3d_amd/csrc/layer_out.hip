@@ -1,11 +1,11 @@
-// What lies between a decoder layer's scan and its output projections where no gradient is asked for (gfx950), bf16, one launch:
+// What lies behind a decoder layer's scan where no gradient is asked for (gfx950), bf16:
 //   key    = RMSNorm(bf16(y0 + y1) * silu(z)) * w          a wave a row of the (batch x seqlen, d_inner) scan outputs
-//   query  = LayerNorm(bf16((last0 + last1) / 2)^T)         8 queries a workgroup: their d_inner values, fp32 and one per state
-//                                                           row, meet in LDS as bf16 (issm_transpose_states' result)
-// Each was a launch or two of its own (add, norm, transpose, LayerNorm), 3 to 4 us whatever its size and as much again to issue;
-// at one scene (1024 tokens, 256 queries, 288 features) the four took 15 us, this takes 6.  Bound by the launch and
-// one trip to memory; 8 queries a workgroup for 32-byte pieces of a state row and still 32 workgroups at one scene.
-// The sums and averages are rounded to bf16 as the separate kernels stored them.
+//   query  = LayerNorm(bf16((last0 + last1) / 2)^T)         the d_inner values of a few queries, fp32 and one per state row, meet in LDS as
+//                                                           bf16 (issm_transpose_states' result)
+// and their output projections: k_layer_end, which is what the layer takes, and k_layer_out, the same without the projections, for
+// callers that have something else behind the norms.  Each line was a launch or two of its own (add, norm, transpose, LayerNorm), 3 to
+// 4 us whatever its size and as much again to issue; at one scene (1024 tokens, 256 queries, 288 features) the four took 15 us, k_layer_out 6.
+// Bound by the launch and one trip to memory.  The sums and averages are rounded to bf16 as the separate kernels stored them.
 #include <algorithm>
 
 #include "issm_dev.h"
@@ -25,61 +25,57 @@ __device__ __forceinline__ float wave_total(float v) {
   return v;
 }
 
-constexpr int LO_Q = 8;   // queries a workgroup
-
+// The gated norm of row `row`, by a wave: four features a lane and vector.
 template <int NV>
-__global__ __launch_bounds__(NTHREADS) void k_layer_out(LayerOutP p) {
-  __shared__ uint16_t tile[LO_Q * (NV * 256 + 4)];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, di = p.di;
-  if ((int)blockIdx.x < p.key_blocks) {
-    const long row = (long)blockIdx.x * 4 + w;
-    if (row >= p.rows) return;
-    f4 x[NV], z[NV], g[NV];
+__device__ __forceinline__ void key_norm(const LayerOutP& p, long row, int lane, uint16_t* to) {
+  const int di = p.di;
+  f4 x[NV], z[NV], kw[NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * (lane + 64 * v);
-      const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-      x[v] = z[v] = g[v] = zero;
-      if (c < di) {
-        x[v] = ld_bf4(p.y0 + row * di + c) + ld_bf4(p.y1 + row * di + c);
-        z[v] = ld_bf4(p.z + row * p.zs + c);
-        g[v] = ld_bf4(p.kw + c);
-      }
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      x[v] = round_bf4(x[v]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[v][r] *= z[v][r] * sigmoidf_(z[v][r]);
-      ss += sum4(x[v] * x[v]);
-    }
-    const float rstd = 1.0f / sqrtf(wave_total(ss) / (float)di + p.keps);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * (lane + 64 * v);
-      if (c < di) st_bf4(p.key + row * di + c, x[v] * rstd * g[v]);
-    }
-    return;
+  for (int v = 0; v < NV; ++v) {
+    const int c = min(4 * (lane + 64 * v), di - 4);   // (past the end: the last vector again, not counted)
+    x[v] = ld_bf4(p.y0 + row * di + c) + ld_bf4(p.y1 + row * di + c);
+    z[v] = ld_bf4(p.z + row * p.zs + c);
+    kw[v] = ld_bf4(p.kw + c);
   }
-  const int qb = (int)blockIdx.x - p.key_blocks, per = (p.K + LO_Q - 1) / LO_Q, b = qb / per, k0 = (qb % per) * LO_Q;
-  const int ld = NV * 256 + 4;
-  {
-    const int q = threadIdx.x % LO_Q, k = min(k0 + q, p.K - 1);   // (queries past the end repeat the last and are not stored)
-    const long at = (long)b * di * p.K + k;
-#pragma unroll 4
-    for (int c = threadIdx.x / LO_Q; c < di; c += NTHREADS / LO_Q)
-      tile[q * ld + c] = f_to_bf16((p.last0[at + (long)c * p.K] + p.last1[at + (long)c * p.K]) * 0.5f);
+  float ss = 0.0f;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    x[v] = round_bf4(x[v]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[v][r] *= z[v][r] * sigmoidf_(z[v][r]);
+    if (4 * (lane + 64 * v) < di) ss += sum4(x[v] * x[v]);
   }
-  __syncthreads();
-  for (int q = w; q < LO_Q && k0 + q < p.K; q += 4) {
+  const float rstd = 1.0f / sqrtf(wave_total(ss) / (float)di + p.keps);
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int c = 4 * (lane + 64 * v);
+    if (c < di) st_bf4(to + c, x[v] * rstd * kw[v]);
+  }
+}
+
+// The LayerNorm of a query whose values lie in LDS, by a wave.
+template <int NV>
+struct QueryNorm {
+  f4 w[NV], b[NV];
+  __device__ __forceinline__ QueryNorm(const LayerOutP& p, int lane) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int c = min(4 * (lane + 64 * v), p.di - 4);
+      w[v] = (f4){1.0f, 1.0f, 1.0f, 1.0f};
+      b[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+      if (p.qw) w[v] = ld_bf4(p.qw + c);   // uniform
+      if (p.qb) b[v] = ld_bf4(p.qb + c);
+    }
+  }
+  __device__ __forceinline__ void operator()(const LayerOutP& p, int lane, const uint16_t* from, uint16_t* to) const {
+    const int di = p.di;
     f4 x[NV];
     float s = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int c = 4 * (lane + 64 * v);
       x[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-      if (c < di) x[v] = ld_bf4(tile + q * ld + c);
+      if (c < di) x[v] = ld_bf4(from + c);
       s += sum4(x[v]);
     }
     const float mean = wave_total(s) / (float)di;
@@ -91,21 +87,40 @@ __global__ __launch_bounds__(NTHREADS) void k_layer_out(LayerOutP p) {
         s += sum4(x[v] * x[v]);
       }
     const float rstd = 1.0f / sqrtf(wave_total(s) / (float)di + p.qeps);
-    uint16_t* o = p.query + ((long)b * p.K + k0 + q) * di;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int c = 4 * (lane + 64 * v);
-      if (c < di) {
-        f4 y = x[v] * rstd;
-        if (p.qw) y *= ld_bf4(p.qw + c);
-        if (p.qb) y += ld_bf4(p.qb + c);
-        st_bf4(o + c, y);
-      }
+      if (c < di) st_bf4(to + c, x[v] * rstd * w[v] + b[v]);
     }
   }
+};
+
+constexpr int LO_Q = 8;   // queries a workgroup: 32-byte pieces of a state row and still 32 workgroups at one scene
+
+template <int NV>
+__global__ __launch_bounds__(NTHREADS) void k_layer_out(LayerOutP p) {
+  __shared__ uint16_t tile[LO_Q * (NV * 256 + 4)];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, di = p.di;
+  if ((int)blockIdx.x < p.key_blocks) {
+    const long row = (long)blockIdx.x * 4 + w;
+    if (row < p.rows) key_norm<NV>(p, row, lane, p.key + row * di);
+    return;
+  }
+  const int qb = (int)blockIdx.x - p.key_blocks, per = (p.K + LO_Q - 1) / LO_Q, b = qb / per, k0 = (qb % per) * LO_Q;
+  const int ld = NV * 256 + 4;
+  {
+    const int q = threadIdx.x % LO_Q, k = min(k0 + q, p.K - 1);   // (queries past the end repeat the last and are not stored)
+    const long at = (long)b * di * p.K + k;
+#pragma unroll 4
+    for (int c = threadIdx.x / LO_Q; c < di; c += NTHREADS / LO_Q)
+      tile[q * ld + c] = f_to_bf16((p.last0[at + (long)c * p.K] + p.last1[at + (long)c * p.K]) * 0.5f);
+  }
+  const QueryNorm<NV> norm(p, lane);
+  __syncthreads();
+  for (int q = w; q < LO_Q && k0 + q < p.K; q += 4) norm(p, lane, tile + q * ld, p.query + ((long)b * p.K + k0 + q) * di);
 }
 
-// The same and the output projections behind it, one launch: a workgroup of sixteen waves takes 16 rows (or queries) through the
+// The norms and the output projections, one launch: a workgroup of sixteen waves takes 16 rows (or queries) through the
 // norm into LDS, a wave a row, and multiplies them with the weights of up to 256 outputs, 16 a wave, whose fragments it has asked for
 // before the rows.  The two launches took 6.0 and 5.1 us at one scene, each a trip to memory and a little arithmetic.  A few hundred
 // instructions a wave decide here: with four waves a workgroup and four rows a wave it took 10.2 us.  (The norm of a row is
@@ -135,29 +150,7 @@ __global__ __launch_bounds__(1024) void k_layer_end(LayerOutP p, LinearP q, int 
   if (!second) {
     out_row = (long)tb * 16;
     rows_left = p.rows - out_row;
-    const long row = min(out_row + w, p.rows - 1);
-    f4 x[NV], z[NV], kw[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = min(4 * (lane + 64 * v), di - 4);   // (past the end: the last vector again, not counted)
-      x[v] = ld_bf4(p.y0 + row * di + c) + ld_bf4(p.y1 + row * di + c);
-      z[v] = ld_bf4(p.z + row * p.zs + c);
-      kw[v] = ld_bf4(p.kw + c);
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      x[v] = round_bf4(x[v]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) x[v][r] *= z[v][r] * sigmoidf_(z[v][r]);
-      if (4 * (lane + 64 * v) < di) ss += sum4(x[v] * x[v]);
-    }
-    const float rstd = 1.0f / sqrtf(wave_total(ss) / (float)di + p.keps);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * (lane + 64 * v);
-      if (c < di) st_bf4(row_of + c, x[v] * rstd * kw[v]);
-    }
+    key_norm<NV>(p, min(out_row + w, p.rows - 1), lane, row_of);
   } else {
     const int perb = (p.K + 15) / 16, b = tb / perb, k0 = (tb % perb) * 16;
     out_row = (long)b * p.K + k0;
@@ -176,39 +169,9 @@ __global__ __launch_bounds__(1024) void k_layer_end(LayerOutP p, LinearP q, int 
       for (int m = 0; m < NC; ++m)
         if (c0 + 64 * m < di) tile[qi * LD + c0 + 64 * m] = f_to_bf16((a0[m] + a1[m]) * 0.5f);
     }
-    f4 qw[NV], qb[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = min(4 * (lane + 64 * v), di - 4);
-      qw[v] = (f4){1.0f, 1.0f, 1.0f, 1.0f};
-      qb[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-      if (p.qw) qw[v] = ld_bf4(p.qw + c);   // uniform
-      if (p.qb) qb[v] = ld_bf4(p.qb + c);
-    }
+    const QueryNorm<NV> norm(p, lane);
     __syncthreads();
-    f4 x[NV];
-    float s = 0.0f;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * (lane + 64 * v);
-      x[v] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-      if (c < di) x[v] = ld_bf4(row_of + c);
-      s += sum4(x[v]);
-    }
-    const float mean = wave_total(s) / (float)di;
-    s = 0.0f;
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-      if (4 * (lane + 64 * v) < di) {
-        x[v] -= mean;
-        s += sum4(x[v] * x[v]);
-      }
-    const float rstd = 1.0f / sqrtf(wave_total(s) / (float)di + p.qeps);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * (lane + 64 * v);
-      if (c < di) st_bf4(row_of + c, x[v] * rstd * qw[v] + qb[v]);
-    }
+    norm(p, lane, row_of, row_of);
   }
   __syncthreads();
   if (!mine) return;
