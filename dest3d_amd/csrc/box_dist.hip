@@ -82,8 +82,11 @@ __device__ __forceinline__ float wave_uniform(float v) {
 // AXES, calls that nothing is differentiated through: boxes that stand along the axes, under no rotation.  The eight corners are
 // two positions per axis, so the sum of their trilinear weights is a product of three sums over an axis' positions: at most four nodes
 // an axis, 6 logarithms a pair instead of 24, no queue (all pairs, whether the box is next to the point or around it).  Taken by a
-// wave whose box is such a one, for finite points and a finite table (weights of zero are multiplied too).  1024 points in the order
-// of a Hilbert curve, 256 boxes, bf16: one scene 39.6 -> 24.3 us, eight 171 -> 97; boxes that are turned 39.6 and 170 either way.
+// wave whose box is such a one, for finite points and a finite table.  Bound by the LDS reads, 64 bytes a node and lane; a lane
+// leaves out the nodes of weight zero (outside the table, or the other position's): with all of them read, points in random order lost
+// to the form by corners.  A call of the encoding, 256 boxes, 1024 points a scene, bf16, by corners, with every node read and like this: one scene, in the
+// order of a Hilbert curve 49.7, 37.2 and 34.9 us, in random order 50.5, 44.4 and 36.1; eight 171, 103 and 90, 184, 190 and 113.  Boxes that are
+// turned pay 0.6 us a launch for the look at them (47 and 201 us).
 // As accurate, but rounded elsewhere, and an encoding that differs in the last bit of one value in ten thousand moves entries of a
 // gradient behind six bf16 layers by up to 0.48 of their mean square: training keeps the sums it had.
 constexpr int BD_SEG = 512;     // points per wave at most
@@ -132,18 +135,17 @@ template <bool BF, bool AXES>
 __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_points) {
   __shared__ __attribute__((aligned(16))) float tab[BD_MAXCELLS * BD_NS];
   __shared__ unsigned short queue[BD_FWD_T / 64][BD_SEG];
-  __shared__ int queue_len[BD_FWD_T / 64];
+  __shared__ int queue_len[BD_FWD_T / 64], odd_of[BD_FWD_T / 64];
   const int cells = p.D * p.H * p.W;
-  bool odd = false;   // AXES: some value of the table is not finite
+  bool odd = false;   // AXES: some value of the table is not finite (odd_of: of a wave's share of it)
   for (int e = threadIdx.x; e < cells * BD_C; e += BD_FWD_T) {
     const int ch = e / cells, cell = e - ch * cells;
     const float v = p.table[e];
     tab[cell * BD_NS + ch] = v;
-    if constexpr (AXES) odd = odd || !finite_(v);
+    if constexpr (AXES) odd |= !finite_(v);
   }
-  bool plain_table = false;
-  if constexpr (AXES) plain_table = !__syncthreads_or(odd);
-  else __syncthreads();
+  if constexpr (AXES) odd_of[threadIdx.x >> 6] = __ballot(odd) != 0ull;
+  __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int kgroups = (p.K + 7) / 8, npair = (p.L + 2 * seg_points - 1) / (2 * seg_points);
   const int kgroup = blockIdx.x % kgroups, bs = blockIdx.x / kgroups;
@@ -161,7 +163,12 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       bx.cs[c] = wave_uniform(bx.cs[c]); bx.sn[c] = wave_uniform(bx.sn[c]);
     }
     int base = 0;
-    if (AXES && plain_table && along_axes(bx)) {   // uniform
+    bool axes = AXES && along_axes(bx);   // uniform
+    if (axes) {
+#pragma unroll
+      for (int w = 0; w < BD_FWD_T / 64; ++w) axes = axes && __builtin_amdgcn_readfirstlane(odd_of[w]) == 0;
+    }
+    if (axes) {   // uniform
       const float x0 = bx.cx[0], x1 = bx.cx[2], y0 = bx.cy[0], y1 = bx.cy[1], z0 = bx.cz[0], z1 = bx.cz[4];
 #pragma unroll 1
       for (; base < n; base += 64) {
@@ -186,8 +193,10 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
             auto node = [&](int j3) {
               const f4* src = (const f4*)(row + ax.node[j3]);
               const float w = zy * ax.w[j3];
+              if (w != 0.0f) {
 #pragma unroll
-              for (int j = 0; j < 4; ++j) acc[j] += w * src[j];
+                for (int j = 0; j < 4; ++j) acc[j] += w * src[j];
+              }
             };
             node(0);
             node(1);
