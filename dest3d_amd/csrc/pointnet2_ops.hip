@@ -788,6 +788,9 @@ __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int 
 // cells to the sorted list, and their places in the cells are what the counting's additions return.  20000 x 2048 points, 8 samples: 258 us
 // looking at all, 47 us with a workgroup to 512 targets (320 of them, two on every fourth CU) that read the points three times, 42 like this, 38 with the
 // places of a block's rows read together and a point requested while the one before is looked at.
+// More targets than that: two workgroups a CU while their points fit (up to 4063 of them), at 64 registers a lane, and where all of them
+// then fit at once the targets are shared by as many as there is room for.  At 70 and 82 registers, one a CU, 16 samples of 20000 x 1000 points
+// took 71 us (55 now; 59 with 512 threads a workgroup, three or four a CU), 64 of 40000 x 1000 311 (230; 244), 16 of 20000 x 3000 77 (60; 79).
 constexpr int NN_T = 1024, NN_CELLS = 4096;
 struct Nearest3 {
   float d1, d2, d3;
@@ -801,7 +804,7 @@ struct Nearest3 {
   }
 };
 template <int R>
-__global__ __launch_bounds__(NN_T) void k_three_nn_grid(int n, int m, int share, const float* __restrict__ unknown,
+__global__ __launch_bounds__(NN_T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, int m, int share, const float* __restrict__ unknown,
                                                         const float* __restrict__ known, float* __restrict__ dist2,
                                                         int* __restrict__ idx) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1513,7 +1516,10 @@ int launch_group_points_grad(int b, int c, int n, int ms, const float* grad_out,
 int launch_three_nn(int b, int n, int m, const float* unknown, const float* known, float* dist2, int* idx, hipStream_t st) {
   if (m >= 256 && m <= 8192) {   // fewer: building the grid costs as much as looking at all; more: they do not fit in LDS
     const size_t sm = m * sizeof(float4) + (NN_CELLS + 1) * sizeof(int);
-    const int groups = std::max((n + NN_T - 1) / NN_T, std::min(std::max(256 / b, 1), (n + 127) / 128)), share = (n + groups - 1) / groups;
+    const int room = 2 * (sm + 512) <= 160 * 1024 ? 2 * NCU : NCU;   // workgroups at once; 512: the kernel's own LDS
+    int groups = std::max((n + NN_T - 1) / NN_T, std::min(std::max(NCU / b, 1), (n + 127) / 128));
+    if ((long)groups * b > NCU && (long)groups * b <= room) groups = room / b;
+    const int share = (n + groups - 1) / groups;
     auto go = [&](auto kern) -> int {
       if (int e = set_lds_rows(kern, sm)) return e;
       hipLaunchKernelGGL(kern, dim3((n + share - 1) / share, b), dim3(NN_T), sm, st, n, m, share, unknown, known, dist2, idx);
