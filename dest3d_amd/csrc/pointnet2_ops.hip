@@ -790,7 +790,10 @@ __global__ __launch_bounds__(NTHREADS) void k_group_points_grad(long total, int 
 // places of a block's rows read together and a point requested while the one before is looked at.
 // More targets than that: two workgroups a CU while their points fit (up to 4063 of them), at 64 registers a lane, and where all of them
 // then fit at once the targets are shared by as many as there is room for.  At 70 and 82 registers, one a CU, 16 samples of 20000 x 1000 points
-// took 71 us (55 now; 59 with 512 threads a workgroup, three or four a CU), 64 of 40000 x 1000 311 (230; 244), 16 of 20000 x 3000 77 (60; 79).
+// took 71 us (54 now; 59 with 512 threads a workgroup, three or four a CU, reading the points three times), 16 of 20000 x 3000 77 (60; 79).  Where
+// they do not fit at once and four of half the size fit a CU (up to 1519 points), those: a CU then waits for the slowest of eight waves and
+// not of sixteen.  12 of 50000 x 1024 86 us with 1024 threads, 79 with 512, 64 of 40000 x 1000 229 and 226; targets outside the known points 197 and 185, 494 and
+// 485 (186 and 477 with those that read three times).
 constexpr int NN_T = 1024, NN_CELLS = 4096;
 struct Nearest3 {
   float d1, d2, d3;
@@ -803,24 +806,24 @@ struct Nearest3 {
     else if (z) { d3 = d; i3 = k; }
   }
 };
-template <int R>
-__global__ __launch_bounds__(NN_T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, int m, int share, const float* __restrict__ unknown,
+template <int T, int R>
+__global__ __launch_bounds__(T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, int m, int share, const float* __restrict__ unknown,
                                                         const float* __restrict__ known, float* __restrict__ dist2,
                                                         int* __restrict__ idx) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   float4* pts = (float4*)smem_raw;           // [m] x, y, z, index
   int* end = (int*)(pts + m);                // [NN_CELLS + 1]: end[c + 1] = end of cell c's points, end[0] = 0
-  __shared__ float red[7][NN_T / 64];
-  __shared__ int wsum[NN_T / 64];
+  __shared__ float red[7][T / 64];
+  __shared__ int wsum[T / 64];
   const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const float INFV = __builtin_huge_valf();
   const float* kp = known + (long)b * m * 3;
   float lo[3] = {INFV, INFV, INFV}, hi[3] = {-INFV, -INFV, -INFV}, odd = 0.0f;
-  float pt[R][3];   // points tid, tid + NN_T, .. (past the end: the last one again, not counted)
+  float pt[R][3];   // points tid, tid + T, .. (past the end: the last one again, not counted)
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int a = 0; a < 3; ++a) pt[r][a] = kp[min(tid + r * NN_T, m - 1) * 3 + a];
+    for (int a = 0; a < 3; ++a) pt[r][a] = kp[min(tid + r * T, m - 1) * 3 + a];
   const int j = blockIdx.x * share + tid;
   const bool live = tid < share && j < n;
   const float* u = unknown + ((long)b * n + min(j, n - 1)) * 3;
@@ -841,13 +844,13 @@ __global__ __launch_bounds__(NN_T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, in
     const float l = -wave_fmax(-lo[a]), h = wave_fmax(hi[a]);
     if (lane == 0) { red[a][wave] = l; red[3 + a][wave] = h; }
   }
-  for (int c = tid; c <= NN_CELLS; c += NN_T) end[c] = 0;
+  for (int c = tid; c <= NN_CELLS; c += T) end[c] = 0;
   __syncthreads();
   odd = red[6][0];
 #pragma unroll
   for (int a = 0; a < 3; ++a) { lo[a] = red[a][0]; hi[a] = red[3 + a][0]; }
 #pragma unroll
-  for (int w = 1; w < NN_T / 64; ++w) {
+  for (int w = 1; w < T / 64; ++w) {
     odd = fmaxf(odd, red[6][w]);
 #pragma unroll
     for (int a = 0; a < 3; ++a) { lo[a] = fminf(lo[a], red[a][w]); hi[a] = fmaxf(hi[a], red[3 + a][w]); }
@@ -872,11 +875,11 @@ __global__ __launch_bounds__(NN_T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, in
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       cell[r] = (cell1(pt[r][2], 2) * g[1] + cell1(pt[r][1], 1)) * g[0] + cell1(pt[r][0], 0);
-      if (tid + r * NN_T < m) place[r] = atomicAdd(&end[1 + cell[r]], 1);
+      if (tid + r * T < m) place[r] = atomicAdd(&end[1 + cell[r]], 1);
     }
     __syncthreads();
-    {  // exclusive prefix sum: NN_CELLS / NN_T neighbours per thread
-      constexpr int E = NN_CELLS / NN_T;
+    {  // exclusive prefix sum: NN_CELLS / T neighbours per thread
+      constexpr int E = NN_CELLS / T;
       int own = 0;
       for (int e = 0; e < E; ++e) own += end[1 + tid * E + e];
       int incl = own;
@@ -894,7 +897,7 @@ __global__ __launch_bounds__(NN_T, R > 4 ? 4 : 8) void k_three_nn_grid(int n, in
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < R; ++r)
-      if (tid + r * NN_T < m) pts[end[cell[r]] + place[r]] = make_float4(pt[r][0], pt[r][1], pt[r][2], __builtin_bit_cast(float, tid + r * NN_T));
+      if (tid + r * T < m) pts[end[cell[r]] + place[r]] = make_float4(pt[r][0], pt[r][1], pt[r][2], __builtin_bit_cast(float, tid + r * T));
     __syncthreads();
     if (live) {
       const int cx = cell1(ux, 0), cy = cell1(uy, 1), cz = cell1(uz, 2);
@@ -1519,13 +1522,15 @@ int launch_three_nn(int b, int n, int m, const float* unknown, const float* know
     const int room = 2 * (sm + 512) <= 160 * 1024 ? 2 * NCU : NCU;   // workgroups at once; 512: the kernel's own LDS
     int groups = std::max((n + NN_T - 1) / NN_T, std::min(std::max(NCU / b, 1), (n + 127) / 128));
     if ((long)groups * b > NCU && (long)groups * b <= room) groups = room / b;
-    const int share = (n + groups - 1) / groups;
-    auto go = [&](auto kern) -> int {
+    const bool halves = (long)groups * b > 2 * NCU && m <= 3 * NN_T / 2 && 4 * (sm + 256) <= 160 * 1024;
+    const int share = halves ? NN_T / 2 : (n + groups - 1) / groups;
+    auto go = [&](auto kern, int threads = NN_T) -> int {
       if (int e = set_lds_rows(kern, sm)) return e;
-      hipLaunchKernelGGL(kern, dim3((n + share - 1) / share, b), dim3(NN_T), sm, st, n, m, share, unknown, known, dist2, idx);
+      hipLaunchKernelGGL(kern, dim3((n + share - 1) / share, b), dim3(threads), sm, st, n, m, share, unknown, known, dist2, idx);
       return 0;
     };
-    if (int e = m <= 2 * NN_T ? go(&k_three_nn_grid<2>) : m <= 4 * NN_T ? go(&k_three_nn_grid<4>) : go(&k_three_nn_grid<8>)) return e;
+    if (int e = halves ? go(&k_three_nn_grid<NN_T / 2, 3>, NN_T / 2) : m <= 2 * NN_T ? go(&k_three_nn_grid<NN_T, 2>)
+                : m <= 4 * NN_T ? go(&k_three_nn_grid<NN_T, 4>) : go(&k_three_nn_grid<NN_T, 8>)) return e;
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(k_three_nn, dim3((n + NTHREADS - 1) / NTHREADS, b), dim3(NTHREADS), 0, st, n, m, unknown, known, dist2,

@@ -410,7 +410,8 @@ def test_interpolation_rows_keep_a_target_without_a_number_to_its_points(c, m, n
 
 
 @pytest.mark.parametrize("b,n,m", [(1, 1, 256), (1, 129, 2048), (2, 1025, 2049), (3, 700, 4096), (1, 33000, 4097), (300, 3, 300), (2, 1024, 8192), (1, 262145, 257),
-                                   (86, 2049, 256), (129, 1025, 2047), (17, 16385, 4063), (17, 16385, 4064), (257, 1024, 300), (257, 1025, 300)])
+                                   (86, 2049, 256), (129, 1025, 2047), (17, 16385, 4063), (17, 16385, 4064), (257, 1024, 300), (257, 1025, 300),
+                                   (257, 1537, 1519), (257, 1536, 1520), (171, 2561, 256), (513, 3, 1025)])
 def test_three_nn_shares(b, n, m):
     """Targets shared by workgroups at the edges of their shares, known points at those of a thread's: the pass over all points by index."""
     from dest3d_amd.pointnet2_utils import three_nn
