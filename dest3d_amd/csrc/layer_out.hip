@@ -210,9 +210,9 @@ int launch_layer_end(LayerOutP& p, LinearP& q, hipStream_t st) {
   if (blocks[0] + blocks[1] == 0) return 0;
   p.key_blocks = (int)blocks[0];
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(blocks[0] + blocks[1])), dim3(1024), 0, st, p, q, per[0], per[1]); };
-  const bool nine = p.di / 32 % 9 == 0;   // nine fragments where they come out even (288 features), eight otherwise
+  // (fragments in flight: all there are, up to 320 features; 320, four scenes of 1024 tokens, a layer 172 us with eight of ten, 168 so)
   if (p.di <= 256) go(&k_layer_end<4, 8>);
-  else if (p.di <= 320) nine ? go(&k_layer_end<5, 9>) : go(&k_layer_end<5, 8>);
+  else if (p.di <= 320) go(&k_layer_end<5, 10>);
   else if (p.di <= 512) go(&k_layer_end<8, 8>);
   else go(&k_layer_end<16, 4>);
   return (int)hipGetLastError();

@@ -63,7 +63,7 @@ def kernels():
     (r"(k_chunk_scan|k_bwd_dx)<2, (true|false), (true|false), (true|false), 2>", 16, 128, 0),
     (r"(k_chunk_scan|k_bwd_dx)<[34], (true|false), (true|false), (true|false), 2>", 32, 256, 0),
     # workgroups of sixteen waves
-    (r"(k_layer_end<.*>|k_three_nn_grid<1024, .*>|k_box_dist_fwd<.*>)", 12, 128, 0),
+    (r"(k_layer_end<.*>|k_three_nn_grid<1024, .*>|k_box_dist_fwd<.*>)", 11, 128, 0),
     # two of them a CU, and four of eight
     (r"k_three_nn_grid<(1024, [24]|512, 3)>", 3, 64, 0),
 ])
