@@ -521,7 +521,8 @@ constexpr double FEW_PRODUCTS = 3.5e8;
 // queries unless said).  288 features, 4, 8, 11 and 16 scenes: 159 and 138, 269 and 242, 347 and 327, 504 and 492; 192, 16 scenes: 432 and 400; 96, 62:
 // 1229 and 1152.  Rows of 128 bytes and multiples of them suit its products least: 64 features, 64 queries, 59, 89 and 135 scenes 527 and 505, 751
 // and 749, 1093 and 1112, 16 queries, 31 and 47 scenes of 2048 449 and 447, 649 and 677; 128, 16 queries, 12 and 20 scenes of 2048 221 and 216, 329 and
-// 341; 320, whose ten fragments take two requests of eight, 3, 4, 5 and 6 scenes 153 and 134, 170 and 169, 200 and 212, 222 and 233; 384, 3 and 4
+// 341; 320, whose ten fragments take two requests of eight (the first products; the last ones', asked for at once, take 2 % off the layer since), 3, 4, 5 and 6
+// scenes 153 and 134, 170 and 169, 200 and 212, 222 and 233; 384, 3 and 4
 // scenes 153 and 145, 175 and 180; 512, 2, 3 and 4 scenes 140 and 126, 166 and 160, 202 and 217; 640, 1 and 2 scenes 132 and 106, 165 and 168.  (Wider odd
 // multiples of 32 would stay ahead for longer: 352, 7 scenes, 268 and 251, 480, 5 scenes, 232 and 218.)
 double chain_products(int64_t features) {
