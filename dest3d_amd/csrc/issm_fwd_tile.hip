@@ -3,8 +3,12 @@
 //
 // Lane (i, kg) of a wave owns row i of every 16-row tile of the chunk and four adjacent state columns
 // n = n0 + 4 kg .. + 3: exactly the operand layout of v_mfma_f32_16x16x16_bf16 for a contraction over the state
-// columns, and a 16-byte (fp32) or 8-byte (bf16) load per tensor and tile.  The four waves of a workgroup take the
-// four 16-column quarters of each 64-column step.
+// columns, and 16 bytes (fp32) or 8 (bf16) per tensor and tile.  Four lanes that follow one another in a wave request one row's 16 columns, and
+// the wave hands the pieces over to the lanes that work on them (row_pieces_to_lanes).  The four waves of a workgroup take the
+// four 16-column quarters of each 64-column step.  A step's operands are requested when the step before has used its own, in
+// one stretch of code without branches, so that a wait is for the request it needs and not for the stores behind it.
+//   Requests by row pieces, those waits, and no copies of what was requested: 8 x 1024 tokens, both directions, 8 heads x 32, 256 states, fp32 91
+// -> 82 us; heads of 36, bf16 84 -> 66; 2 x 16384, one direction, bf16 188 -> 150; 16 x 2048, both, 16 heads x 64, 512 states, fp32 1463 -> 1303.
 //
 //   running sums   down the 16 rows of a tile = across the 16 lanes of a DPP row: four shifted adds per value.
 //                  pc[l] = sum of a = dt' A log2(e) over the rows of l's tile up to and including l.
@@ -31,12 +35,10 @@
 //   ANY, bf16 inputs of calls that nothing is differentiated through: the first step with such a tile is left by the loop over the steps,
 // and it and all that follow are evaluated, by its wave alone, in a loop of their own, with the diagonal blocks in parts whose factors are all
 // <= 1 (far_diagonal) and V from its own exponential.  A freshly initialised decoder has such tiles in 16 % of its chunks and heads, there
-// mostly in all steps, and those workgroups decide when the launch ends: 1024 tokens, 256 queries 22.7 us a layer (28.1 with every step first in
-// the usual form, and its operands requested anew each time; 36 with the chunk computed once more, 18 where no tile is out of range).  As
+// mostly in all steps, and those workgroups decide when the launch ends: 1024 tokens, 256 queries 20.9 us a layer (36 with the chunk computed once
+// more; 22.1 with the loop over the steps left at a step's end, its operands masked so that it adds nothing).  As
 // accurate as the level form, but rounded elsewhere, and through six layers the gradients move by up to 0.8 of their mean square between the
 // two: training keeps the level form (8 x 1024 tokens: 155 us, 110 with this one).
-// bf16 inputs: a tile's whole decay reaches the tile's 16 lanes by DPP, not through LDS (both directions, 8 x 1024 tokens, 8 heads
-// x 36, 256 states 93 -> 91 us; fp32 1 to 2 % slower so).
 #include "issm_dev.h"
 #include "issm_fwd_local.h"
 
@@ -49,7 +51,7 @@ struct FwdTileSmem {
   static constexpr int LDT = CS + 8;   // row stride of the transposed x tile
   uint16_t xt_hi[PT * 16 * LDT];       // x tile transposed, [p][l]
   uint16_t xt_lo[SPLIT ? PT * 16 * LDT : 8];
-  f4 red[4 * 10 * 64];                 // the four waves' partial sums of the ten blocks of M
+  f4 red[4 * 10 * 64];                 // the four waves' partial sums of the ten blocks of M; before, each wave's part serves row_pieces_to_lanes
   int bad;                             // not ANY: some tile is out of range
 };
 template <int PT, bool SPLIT, bool ANY>
@@ -58,16 +60,19 @@ constexpr size_t fwd_tile_lds() {     // not ANY: the level-hierarchy body lays 
                                                                                    : sizeof(FwdTileSmem<PT, SPLIT>);
 }
 
-// inclusive running sum over the 16 lanes of a DPP row (lanes sharing lane >> 4)
-__device__ __forceinline__ float row_scan16(float v) {
-#define ISSM_DPP_SHR(ctrl) \
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true))
-  ISSM_DPP_SHR(0x111);  // row_shr:1, lanes without a source add 0
-  ISSM_DPP_SHR(0x112);
-  ISSM_DPP_SHR(0x114);
-  ISSM_DPP_SHR(0x118);
-#undef ISSM_DPP_SHR
-  return v;
+// inclusive running sums over the 16 lanes of a DPP row (lanes sharing lane >> 4) of 16 values, step by step for all of them: an instruction
+// that reads another lane's value waits for two others behind the one that wrote it
+template <int CTRL>
+__device__ __forceinline__ void row_add(float (&v)[16]) {   // lanes without a source add 0
+#pragma unroll
+  for (int k = 0; k < 16; ++k)
+    v[k] += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v[k]), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ void row_scans(float (&v)[16]) {
+  row_add<0x111>(v);  // row_shr:1
+  row_add<0x112>(v);
+  row_add<0x114>(v);
+  row_add<0x118>(v);
 }
 
 // the value of lane J of a DPP row, on its 16 lanes
@@ -137,6 +142,25 @@ __device__ __forceinline__ void unpack4(const typename RawVec<BF>::type& r, floa
   }
 }
 
+// What the lanes of a wave have requested -- lane 4 r + q the columns 4 q .. + 3 of row r, so that four neighbours' accesses are one
+// piece of memory -- to those that work on it, through LDS that no other wave uses.  Piece 4 r + q lies in slot 4 r + (q ^ turn): those of one q,
+// read together, are in different banks.  (Requested by the lanes that work on it, an instruction's 64 lanes were 64 look-ups in the L1
+// instead of 16: 148 thousand of them a CU, which the kernel waited for in its 165 thousand cycles, at the first size above, vector issue 59 % of
+// the cycles; 57 thousand now, and vector issue 71 %.  By itself the change gave 91 -> 83 us fp32 and 84 -> 70 bf16, heads of 36.)
+template <typename Raw>
+__device__ __forceinline__ void row_pieces_to_lanes(const Raw (&raw)[4], void* area, int lane, float (&v)[16]) {
+  constexpr bool BF = sizeof(Raw) == 8;
+  typedef typename std::conditional<BF, uint2, f4>::type Plain;
+  typedef Plain __attribute__((may_alias)) Slot;
+  Slot* q = (Slot*)area;
+  auto slot = [](int r, int c) { return 4 * r + (c ^ (BF ? (r >> 3) * 2 : r >> 2)); };
+  const int from = slot(lane >> 2, lane & 3), to = slot(lane & 15, lane >> 4);
+#pragma unroll
+  for (int J = 0; J < 4; ++J) q[64 * J + from] = __builtin_bit_cast(Plain, raw[J]);
+#pragma unroll
+  for (int J = 0; J < 4; ++J) unpack4<BF>(__builtin_bit_cast(Raw, (Plain)q[64 * J + to]), v + 4 * J);
+}
+
 // FULLP: the head dimension fills its tiles.  EDGE: chunks with fewer than 64 rows and steps with fewer than 64 columns
 // may exist (N >= 4).  A lane's rows past the end read the chunk's last one and get dt' = 0, as do whole lanes past the last
 // column; a lane whose four columns cross it works on columns N - 4 .. N - 1 instead, those its neighbour owns with dt' = 0
@@ -163,15 +187,16 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, kg = lane >> 4;
+  const int ri = lane >> 2, rkg = lane & 3;   // the row and the columns that the lane requests
   const int uidx = xcd_remap(blockIdx.x, gridDim.x);
   const Unit u = decode_unit(p, uidx);
 
   // addresses: uniform base + per-lane 32-bit element offset (the host checks that seqlen * stride fits in 31 bits);
   // tile J lies 16 J rows further along the scan, the step's columns 64 further along the row
-  const int tl = u.dir ? p.L - 1 - u.c * CS - i : u.c * CS + i;   // the lane's token of tile 0
+  const int tl = u.dir ? p.L - 1 - u.c * CS - ri : u.c * CS + ri;   // the token of tile 0 whose operands the lane requests
   const int sgn = u.dir ? -1 : 1;
   const int nvalid = EDGE ? min(CS, p.L - u.c * CS) : CS;
-  const int ncol = 16 * w + 4 * kg;                                // the lane's first column within a step
+  const int ncol = 16 * w + 4 * kg, rcol = 16 * w + 4 * rkg;       // the lane's first column within a step, and of what it requests
   const TDt* qdt = (const TDt*)p.dt.ptr + ((long)u.b * p.dt.s0 + (long)u.h * p.dt.s2);
   const TIo* qB = (const TIo*)p.Bm[u.dir].ptr + ((long)u.b * p.Bm[u.dir].s0 + (long)u.g * p.Bm[u.dir].s2);
   const TIo* qC = (const TIo*)p.Cm[u.dir].ptr + ((long)u.b * p.Cm[u.dir].s0 + (long)u.g * p.Cm[u.dir].s2);
@@ -182,38 +207,45 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   unsigned odt[NO], oB[NO], oC[NO];
 #pragma unroll
   for (int J = 0; J < NO; ++J) {
-    const int t = EDGE ? tl + sgn * (min(16 * J + i, nvalid - 1) - i) : tl;
-    odt[J] = (unsigned)(t * sdt + (EDGE ? 0 : ncol));
-    oB[J] = (unsigned)(t * sB + (EDGE ? 0 : ncol));
-    oC[J] = (unsigned)(t * sC + (EDGE ? 0 : ncol));
+    const int t = EDGE ? tl + sgn * (min(16 * J + ri, nvalid - 1) - ri) : tl;
+    odt[J] = (unsigned)(t * sdt + (EDGE ? 0 : rcol));
+    oB[J] = (unsigned)(t * sB + (EDGE ? 0 : rcol));
+    oC[J] = (unsigned)(t * sC + (EDGE ? 0 : rcol));
   }
   const int jdt = EDGE ? 0 : sgn * 16 * sdt, jB = EDGE ? 0 : sgn * 16 * sB, jC = EDGE ? 0 : sgn * 16 * sC;
   const float* qA = p.A + u.h * p.N;
   const float* qbias = (p.dt_bias ? p.dt_bias : p.A) + u.h * p.N;  // without a bias: any valid address, scaled by 0
   const float bias_on = p.dt_bias ? 1.0f : 0.0f;
 
-  // fp32 inputs, incomplete tiles, two head tiles: C is requested at the step's start and not a step ahead (it is used last, and its 16
-  // registers made the kernel spill 56 bytes a lane: 8 x 1000 tokens, 8 heads x 32, 250 states 60.6 -> 54.3 us, 2 x 160, 4 heads, 128 states
-  // 14.5 -> 13.7; three and four head tiles have the registers)
-  constexpr bool LATE_C = EDGE && !IOB && PT <= 2;
   RawDt rdt[4];
   RawIo rB[4], rC[4];
   F4Any rA, rbias;
-#define ISSM_REQUEST_C(c_)                                                             \
+#define ISSM_REQUEST_DT(n0_)                                                           \
   {                                                                                    \
+    const int c_ = EDGE ? min((n0_) + rcol, p.N - 4) : (n0_);                          \
+    const int a_ = EDGE ? min((n0_) + ncol, p.N - 4) : (n0_) + ncol;                   \
     _Pragma("unroll") for (int J = 0; J < 4; ++J)                                      \
-      rC[J] = *(const RawIo*)(qC + (int)(oC[J % NO] + (unsigned)(J * jC + (c_))));     \
+      rdt[J] = *(const RawDt*)(qdt + (int)(odt[J % NO] + (unsigned)(J * jdt + c_)));   \
+    rA = *(const F4Any*)(qA + a_);                                                     \
+    rbias = *(const F4Any*)(qbias + a_);                                               \
+  }
+#define ISSM_REQUEST_B(n0_)                                                            \
+  {                                                                                    \
+    const int c_ = EDGE ? min((n0_) + rcol, p.N - 4) : (n0_);                          \
+    _Pragma("unroll") for (int J = 0; J < 4; ++J)                                      \
+      rB[J] = *(const RawIo*)(qB + (int)(oB[J % NO] + (unsigned)(J * jB + c_)));       \
+  }
+#define ISSM_REQUEST_C(n0_)                                                            \
+  {                                                                                    \
+    const int c_ = EDGE ? min((n0_) + rcol, p.N - 4) : (n0_);                          \
+    _Pragma("unroll") for (int J = 0; J < 4; ++J)                                      \
+      rC[J] = *(const RawIo*)(qC + (int)(oC[J % NO] + (unsigned)(J * jC + c_)));       \
   }
 #define ISSM_REQUEST(n0_)                                                              \
   {                                                                                    \
-    const int c_ = EDGE ? min((n0_) + ncol, p.N - 4) : (n0_);                          \
-    _Pragma("unroll") for (int J = 0; J < 4; ++J) {                                    \
-      rdt[J] = *(const RawDt*)(qdt + (int)(odt[J % NO] + (unsigned)(J * jdt + c_)));   \
-      rB[J] = *(const RawIo*)(qB + (int)(oB[J % NO] + (unsigned)(J * jB + c_)));       \
-    }                                                                                  \
-    if constexpr (!LATE_C) ISSM_REQUEST_C(c_)                                          \
-    rA = *(const F4Any*)(qA + (EDGE ? c_ : c_ + ncol));                                \
-    rbias = *(const F4Any*)(qbias + (EDGE ? c_ : c_ + ncol));                          \
+    ISSM_REQUEST_DT(n0_)                                                               \
+    ISSM_REQUEST_C(n0_)                                                                \
+    ISSM_REQUEST_B(n0_)                                                                \
   }
   ISSM_REQUEST(0);
 
@@ -225,6 +257,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   }
 
 
+  auto hand_over = [&](const auto& raw, float (&v)[16]) __attribute__((always_inline)) { row_pieces_to_lanes(raw, s.red + w * 640, lane, v); };
+
   // identity operand of the exchange of lane and register roles: B[k = 4 kg + r][j = i] = (k == j)
   bf4 ident;
   {
@@ -233,8 +267,6 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
     const uint2 idr = make_uint2((r1 == 0 ? one : 0u) | (r1 == 1 ? one << 16 : 0u), (r1 == 2 ? one : 0u) | (r1 == 3 ? one << 16 : 0u));
     ident = __builtin_bit_cast(bf4, idr);
   }
-  const int last_lane = lane | 15;
-  const float thr = ex2(-FWD_SPAN_LIMIT);
 
   // Diagonal block of a tile whose decays may be out of range: pairs of rows in different halves, then in different quarters
   // of a half, each with the row between the two as the reference -- both factors of every pair are <= 1 -- and in fp32 those
@@ -307,16 +339,24 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
 #pragma unroll
   for (int q = 0; q < 10; ++q) macc[q] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
   float etmin = 1.0f;  // smallest whole-tile decay seen by the lane
+  const float thr = ex2(-FWD_SPAN_LIMIT);
 
   if (tid == 0) s.bad = 0;
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0).  (What is under way here the waits in the loop would count with their own, as the compiler
+                                        // merges the two: the one at its head then waited for everything, the stores of the step before among it.)
   __syncthreads();  // x tile complete
   float* sdst = states + st_off(p, u.bt, u.c, u.h);
+  const __amdgpu_buffer_rsrc_t slab = __builtin_amdgcn_make_buffer_rsrc(sdst, 0, (unsigned)(p.P * p.N) * 4u, 0x00027000);
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
   float* cdst = cs_last + vec_off(p, u.bt, u.c, u.h);
 
+  // not ANY, a tile was out of range: the loop ends with the step.  (With a second way out of it, in the middle of a step, every wait at its
+  // head counts on a step broken off there and waits for all that is under way, the step's own stores among it.)
+  bool stop = false;
   if constexpr (!ANY) {
     constexpr bool DEEP = false;
 #pragma unroll 1
-    for (int n0 = 0; n0 < p.N; n0 += NS) {
+    for (int n0 = 0; (n0 < p.N) & !stop; n0 += NS) {
 #include "issm_fwd_tile_step.h"
     }
   } else {
@@ -338,6 +378,8 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_local_tile(KP p, float* __restr
   }
 #undef ISSM_REQUEST
 #undef ISSM_REQUEST_C
+#undef ISSM_REQUEST_B
+#undef ISSM_REQUEST_DT
 
   // ---- M: the waves' partial sums meet in LDS; wave w then finishes blocks w, w + 4, w + 8
 #pragma unroll

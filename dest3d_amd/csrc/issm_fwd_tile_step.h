@@ -1,18 +1,12 @@
 // One step of k_local_tile (issm_fwd_tile.hip): 64 state columns, 16 of them the wave's.  Included where it runs, inside a loop
-// over n0 and with DEEP defined: the usual form (false), which breaks off with nothing stored where some tile of the wave's
-// columns is out of range (bf16 inputs), and, ANY only, the form that has no range (true).  (Text and not a function: as an inlined lambda
+// over n0 and with DEEP defined: the usual form (false), which, where some tile of the wave's columns is out of range (bf16 inputs), breaks
+// off with nothing stored (ANY) or ends the loop with the step, and, ANY only, the form that has no range (true).  (Text and not a function: as an inlined lambda
 // the usual form is allocated differently, fp32 1 to 4 % slower.)
     const int bad_seen = IOB && !ANY ? __hip_atomic_load(&s.bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0;
-    // ---- this step's values out of the request registers; the next step's request follows at once
-    float dtv[16], bv[16], cv[16];
-#pragma unroll
-    for (int J = 0; J < 4; ++J) {
-      unpack4<DTB>(rdt[J], dtv + 4 * J);
-      unpack4<IOB>(rB[J], bv + 4 * J);
-      if constexpr (!LATE_C) unpack4<IOB>(rC[J], cv + 4 * J);
-    }
     const float A2[4] = {rA.x * LOG2E, rA.y * LOG2E, rA.z * LOG2E, rA.w * LOG2E};
-    const float bias[4] = {rbias.x * bias_on, rbias.y * bias_on, rbias.z * bias_on, rbias.w * bias_on};
+    float bias[4] = {rbias.x * bias_on, rbias.y * bias_on, rbias.z * bias_on, rbias.w * bias_on};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(bias[r]));   // (multiplied and added at once, every sum would begin as a copy of its dt)
     // the lane's columns this step: c .. c + 3, of which the first `skip` are not its own
     const int c = EDGE ? min(n0 + ncol, p.N - 4) : n0 + ncol, skip = EDGE ? n0 + ncol - c : 0;
     auto put = [&](float* q, f4 v) {   // q: where column c goes
@@ -26,45 +20,46 @@
           if (j >= skip) q[j] = v[j];
       }
     };
-    if constexpr (LATE_C) ISSM_REQUEST_C(c)
-    {  // branch-free: the last step asks for its own columns once more
-      const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
-      ISSM_REQUEST(nn);
-    }
+    // the next step, whose operands are requested once this one's have been used (the last one asks for its own once more: no branch)
+    const int nn = EDGE ? (n0 + NS < p.N ? n0 + NS : n0) : min(n0 + NS, p.N - NS);
 
     // ---- dt transform and the running sums of the tiles
     float dtp[16], dummy[16];
     {
       float pre[16];
+      hand_over(rdt, pre);
 #pragma unroll
-      for (int k = 0; k < 16; ++k) pre[k] = dtv[k] + bias[k & 3];
+      for (int k = 0; k < 16; ++k) pre[k] += bias[k & 3];
+      ISSM_REQUEST_DT(nn)
       dt_transform<false, 16>(p, pre, dtp, dummy);
       if constexpr (EDGE) {
         if (nvalid < CS || n0 + NS > p.N) {  // uniform
 #pragma unroll
-          for (int k = 0; k < 16; ++k) {
-            const bool past = 16 * (k >> 2) + i >= nvalid;
-            if (past || (k & 3) < skip) dtp[k] = 0.0f;
-            if (!LATE_C && past) cv[k] = 0.0f;   // (rows of M past the end come out as zero)
-          }
+          for (int k = 0; k < 16; ++k)
+            if (16 * (k >> 2) + i >= nvalid || (k & 3) < skip) dtp[k] = 0.0f;
         }
       }
     }
     float pc[16], up[16], et[16];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) pc[k] = row_scan16(dtp[k] * A2[k & 3]);
+    for (int k = 0; k < 16; ++k) pc[k] = dtp[k] * A2[k & 3];
+    row_scans(pc);
 #pragma unroll
     for (int k = 0; k < 16; ++k) up[k] = ex2(pc[k]);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) et[k] = IOB ? row_lane<15>(up[k]) : __shfl(up[k], last_lane, 64);  // whole-tile decay of the lane's columns
+    for (int k = 0; k < 16; ++k) et[k] = row_lane<15>(up[k]);  // whole-tile decay of the lane's columns
     if (!DEEP) {
 #pragma unroll
       for (int k = 0; k < 16; k += 2) etmin = fminf(etmin, fminf(et[k], et[k + 1]));
     }
     if constexpr (IOB && !DEEP) {
-      const bool out = __ballot(!(etmin >= thr)) != 0ull;
-      if (!ANY && out) s.bad = 1;
-      if (out || (!ANY && __builtin_amdgcn_readfirstlane(bad_seen))) break;  // wave-uniform; no barrier in the loop
+      const bool out = __ballot(!(etmin >= thr)) != 0ull;   // wave-uniform; no barrier in the loop
+      if constexpr (ANY) {
+        if (out) break;
+      } else {
+        if (out) s.bad = 1;
+        stop = out | (__builtin_amdgcn_readfirstlane(bad_seen) != 0);
+      }
     }
     {  // the chunk's total decay (natural logarithm), four adjacent columns per lane group.  All 16 lanes of a group
        // store the same values to the same place: a store under a lane condition sits behind a branch, and the waits
@@ -73,14 +68,24 @@
       f4 tot;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float t = (((pc[r] + pc[4 + r]) + pc[8 + r]) + pc[12 + r]) * LN2;
-        tot[r] = IOB ? row_lane<15>(t) : __shfl(t, last_lane, 64);
+        tot[r] = row_lane<15>((((pc[r] + pc[4 + r]) + pc[8 + r]) + pc[12 + r]) * LN2);
       }
       put(cdst + c, tot);
     }
 
     // ---- operands
-    float w16[EDGE || DEEP ? 16 : 1];
+    float bv[16], cv[16], w16[EDGE || DEEP ? 16 : 1];
+    hand_over(rC, cv);
+    ISSM_REQUEST_C(nn)
+    if constexpr (EDGE) {
+      if (nvalid < CS) {  // uniform
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+          if (16 * (k >> 2) + i >= nvalid) cv[k] = 0.0f;   // (rows of M past the end come out as zero)
+      }
+    }
+    hand_over(rB, bv);
+    ISSM_REQUEST_B(nn)
     if constexpr (DEEP) {
 #pragma unroll
       for (int J = 0; J < 4; ++J) {
@@ -91,15 +96,6 @@
         for (int k = 4 * J; k < 4 * J + 4; ++k) cv[k] *= up[k];
       }
     } else if constexpr (EDGE) {
-      if constexpr (LATE_C) {
-#pragma unroll
-        for (int J = 0; J < 4; ++J) unpack4<IOB>(rC[J], cv + 4 * J);
-        if (nvalid < CS) {  // uniform
-#pragma unroll
-          for (int k = 0; k < 16; ++k)
-            if (16 * (k >> 2) + i >= nvalid) cv[k] = 0.0f;
-        }
-      }
       // diagonal blocks, before anything else needs registers: W takes the place of B and dt', C up that of C.  fp32 matrix
       // instructions: k-slot kg of instruction r <-> the lane's column r; the blocks' chains are interleaved.
 #pragma unroll
@@ -183,6 +179,10 @@
     if (FULLP) {  // every state row exists: plain stores (see the note at the chunk's total decay)
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt) put(sdst + (16 * pt + i) * p.N + c, sacc[pt]);
+    } else if constexpr (!EDGE) {   // (rows past the last lie behind the slab's end, where a store is dropped: no branch either)
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, sacc[pt]), slab, (unsigned)((16 * pt + i) * p.N + c) * 4u, 0, 0);
     } else {
 #pragma unroll
       for (int pt = 0; pt < PT; ++pt)
