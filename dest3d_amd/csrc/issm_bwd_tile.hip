@@ -38,6 +38,9 @@
 // workgroups that have such rows or columns.  8 x 1024 tokens, 8 heads x 32, one direction: N = 250 104 us fp32, 83 us bf16
 // (107 and 86 with operand pairs, 147 and 111 in the level form; N = 256: 88 and 59 us); N = 256 with a gated dy, fp32: 99 us
 // (88 with operand pairs, 122 in the level form).
+// The lane's own LDS values in 16-byte accesses, rows of x and dy through buffers (their addresses took branches, 64-bit products and, in
+// them, waits for the kernel's arguments) and marks that no lane condition holds up: both directions, 8 x 1024 tokens, 8 heads x 32, 256
+// states, fp32 172 -> 161 us; heads of 36, bf16 134 -> 131; the training steps of 16 x 2048 tokens, 16 heads x 64, 512 states 8993 -> 8948.
 //
 // What reaches the chunk's total decay through the states is formed here as well (see `gsum`), from dS, H and the state terms'
 // products: the recurrences need not read the states for it (33 - 60 % of their bytes), and what cancels does so exactly: ddt_bias
@@ -54,6 +57,23 @@ constexpr float SPAN_LIMIT = 96.0f;
 template <int PT, bool SPLIT>
 struct BwdTileSmem {
   static constexpr int KW = 16 * PT, LDP = KW + 8;  // x / dy tiles [l][p]
+  // Per-lane values in pieces of four, [k / 4][tid][k % 4]: one 16-byte access each.  In front: an access carries up to 64 KB of its address,
+  // and what lies behind costs another register.
+  f4 dbc[8 * NTHREADS];      // dB / dC accumulators, k < 16: dB, then dC
+  __device__ __forceinline__ float dbc_at(int k, int tid) const { return dbc[(k >> 2) * NTHREADS + tid][k & 3]; }
+  // bf16 inputs: the group's B and C values of every lane, packed in pairs (i < 8: B, then C).
+  // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
+  // streams have been through it in between) and were a third of the kernel's reads; of three and four head tiles, 8 x 1024 tokens,
+  // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 1000
+  // tokens, 250 states, by the kernel trace, three 95 and 102: 85 and 92, four 107 and 118: 99 and 106).
+  static constexpr bool BCL = !SPLIT;
+  uint4 bc[BCL ? 4 * NTHREADS : 0];
+  __device__ __forceinline__ uint2 bc_of(int q, int tid) const { return reinterpret_cast<const uint2*>(bc + (q >> 1) * NTHREADS + tid)[q & 1]; }   // pairs 2 q, 2 q + 1
+  // fp32 inputs of up to three head tiles: the B values; C has no room (8 x 1024 tokens, 8 heads x 32, 256 states, both
+  // directions, training step 480 -> 466 us, per direction 90 and 100 -> 85 and 94; heads of 48 105 and 112 -> 94 and 104.  It is the
+  // 32 registers that B takes neither ahead of a head nor through it, and the loads).
+  static constexpr bool BL = SPLIT && PT <= 3;
+  f4 bl[BL ? 4 * NTHREADS : 0];
   // T[i][j] = dM[max(i,j)][min(i,j)]; fp32 inputs: hi and lo of four columns side by side, the operand (hi | lo) of a K = 32 instruction as
   // one 16-byte read.  (With the two in matrices of their own every second operand took moves, as the heads a set of zeros for the
   // case that nothing is evaluated: 100 of 1500 vector instructions a head.  8 x 1024 tokens, 8 heads x 48, 256 states, both directions, by
@@ -69,19 +89,6 @@ struct BwdTileSmem {
   static constexpr int LDF = CS + 4;                // the same matrix in fp32 (fp32 inputs, incomplete tiles)
   static_assert(!SPLIT || CS * LDF * sizeof(float) <= sizeof(tm), "it takes the pairs' place");
   __device__ __forceinline__ float* tf() { return reinterpret_cast<float*>(tm); }
-  float dbc[32 * NTHREADS];  // per-lane dB / dC accumulators [k][tid]
-  // bf16 inputs: the group's B and C values of every lane, packed in pairs, [i][tid] (i < 8: B, then C).
-  // They are the same for every head of the group; read from global memory again per head they miss the L2 (the heads'
-  // streams have been through it in between) and were a third of the kernel's reads; of three and four head tiles, 8 x 1024 tokens,
-  // both directions, they cost 76 and 84 us where this takes 71 and 75 (four tiles 84 and 91: 78 and 84; 1000
-  // tokens, 250 states, by the kernel trace, three 95 and 102: 85 and 92, four 107 and 118: 99 and 106).
-  static constexpr bool BCL = !SPLIT;
-  unsigned bc[BCL ? 16 * NTHREADS : 0];
-  // fp32 inputs of up to three head tiles: the B values, [k][tid]; C has no room (8 x 1024 tokens, 8 heads x 32, 256 states, both
-  // directions, training step 480 -> 466 us, per direction 90 and 100 -> 85 and 94; heads of 48 105 and 112 -> 94 and 104.  It is the
-  // 32 registers that B takes neither ahead of a head nor through it, and the loads).
-  static constexpr bool BL = SPLIT && PT <= 3;
-  float bl[BL ? 16 * NTHREADS : 0];
   int bad[4];                // per wave: some column of the head exceeds SPAN_LIMIT
   int shared[4];             // per wave: some head was left to the level form
 };
@@ -189,7 +196,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   const RowMap rm = make_rowmap<FULL>(p, u, g4, ns * NS);
 
 #pragma unroll
-  for (int k = 0; k < 16; ++k) s.dbc[k * NTHREADS + tid] = s.dbc[(16 + k) * NTHREADS + tid] = 0.0f;
+  for (int q = 0; q < 8; ++q) s.dbc[q * NTHREADS + tid] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
 
   if (DIAG32) s.shared[wave] = 0;
 
@@ -197,16 +204,20 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     float tb[16];
     lane_load_ln<false>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, tb);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) s.bl[k * NTHREADS + tid] = tb[k];
+    for (int q = 0; q < 4; ++q) s.bl[q * NTHREADS + tid] = (f4){tb[4 * q], tb[4 * q + 1], tb[4 * q + 2], tb[4 * q + 3]};
   }
   if constexpr (BCL) {
     float tb[16], tc[16];
     lane_load_ln<true>(p.Bm[u.dir], u.b, u.g, n, vn, g4, rm, tb);
     lane_load_ln<true>(p.Cm[u.dir], u.b, u.g, n, vn, g4, rm, tc);
+    auto packed = [&](const float (&v)[16], int q) {   // exact: the values are bf16 numbers
+      return make_uint4(pack_bf16(v[8 * q], v[8 * q + 1]), pack_bf16(v[8 * q + 2], v[8 * q + 3]), pack_bf16(v[8 * q + 4], v[8 * q + 5]),
+                        pack_bf16(v[8 * q + 6], v[8 * q + 7]));
+    };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      s.bc[i * NTHREADS + tid] = pack_bf16(tb[2 * i], tb[2 * i + 1]);  // exact: the values are bf16 numbers
-      s.bc[(8 + i) * NTHREADS + tid] = pack_bf16(tc[2 * i], tc[2 * i + 1]);
+    for (int q = 0; q < 2; ++q) {
+      s.bc[q * NTHREADS + tid] = packed(tb, q);
+      s.bc[(2 + q) * NTHREADS + tid] = packed(tc, q);
     }
   }
 
@@ -228,53 +239,53 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
   f4 l_xv[SPLIT ? PT : 1], l_dv[SPLIT ? PT : 1];
   uint2 l_nx[SPLIT ? 1 : PT], l_ny[SPLIT ? 1 : PT];
   float l_raw[16], l_A, l_bias, l_dsv[KP_], l_hv[KP_], l_Bv[BCL || BL ? 1 : 16], l_Cv[BCL ? 1 : 16];
-  auto request_dy_h = [&](int h) {   // fp32 inputs: the operands of R
+  // x and dy: the chunk's rows of a head behind a buffer's base, the first in memory first; pieces that do not exist read zero
+  auto rows = [&](const TensorD& t, int h) {
+    const int first = u.dir ? p.L - u.c * CS - (FULL ? CS : rm.nvalid) : u.c * CS;
+    const char* q = (const char*)t.ptr + ((long)u.b * t.s0 + (long)h * t.s2 + (long)first * t.s1) * (IOB ? 2 : 4);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(q), 0, 0xfffffffcu, 0x00027000);
+  };
+  auto row_piece = [&](int e4, int s1) -> unsigned {   // four elements, where the thread's group e4 of a tile is
     constexpr int G4 = 4 * PT;
+    const int l = e4 / G4, p4 = (e4 % G4) * 4, r = u.dir ? (FULL ? CS : rm.nvalid) - 1 - l : l;
+    const bool ok = (PNF || p4 < p.P) && (FULL || l < rm.nvalid);
+    return ok ? (unsigned)(r * s1 + p4) * (IOB ? 2u : 4u) : 0xfffffffcu;
+  };
+  auto request_dy_h = [&](int h) {   // fp32 inputs: the operands of R
     int tq = tid;
     asm volatile("" : "+v"(tq));
-    const TensorD& ty = p.dout[u.dir];
-    const float* qy = (const float*)ty.ptr + ((long)u.b * ty.s0 + (long)h * ty.s2);
-    const long t0 = u.dir ? p.L - 1 - u.c * CS : u.c * CS, sgn = u.dir ? -1 : 1;
+    const __amdgpu_buffer_rsrc_t rs = rows(p.dout[u.dir], h);
+    const int sy = (int)p.dout[u.dir].s1;
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-      const int e4 = tq + i * NTHREADS, l = e4 / G4, p4 = (e4 % G4) * 4;
-      const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
-      const f4 a = *(const f4*)(qy + (ok ? (t0 + sgn * l) * ty.s1 + p4 : 0));
-      l_dv[i] = ok ? a : (f4){0, 0, 0, 0};
-    }
+    for (int i = 0; i < PT; ++i)
+      l_dv[i] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, row_piece(tq + i * NTHREADS, sy), 0, 0));
     lane_load_pn<KP_>(states + st_off(p, u.bt, u.c, h), p.P, p.N, n, vn, g4, PNF, l_hv);
   };
   auto request = [&](int hnext) {
-    constexpr int G4 = 4 * PT;
     int tq = tid;
     asm volatile("" : "+v"(tq));
-    const int mrow = tq >> 3, mcol = (tq & 7) * 8;
-    const uint16_t* dmb = reinterpret_cast<const uint16_t*>(dm + sq_off(p, u.bt, u.c, hnext));
-    l_th0 = *(const uint4*)(dmb + mrow * CS + mcol);
-    l_th1 = *(const uint4*)(dmb + (32 + mrow) * CS + mcol);
+    const char* dmb = reinterpret_cast<const char*>(dm + sq_off(p, u.bt, u.c, hnext));
+    const unsigned mo = (unsigned)tq * 16u;
+    l_th0 = *(const uint4*)(dmb + mo);
+    l_th1 = *(const uint4*)(dmb + (mo + 32u * CS * 2u));
     if constexpr (SPLIT) {
-      l_tl0 = *(const uint4*)(dmb + CS * CS + mrow * CS + mcol);
-      l_tl1 = *(const uint4*)(dmb + CS * CS + (32 + mrow) * CS + mcol);
+      l_tl0 = *(const uint4*)(dmb + (mo + CS * CS * 2u));
+      l_tl1 = *(const uint4*)(dmb + (mo + (CS * CS + 32u * CS) * 2u));
     }
     {
-      typedef typename std::conditional<IOB, uint16_t, float>::type T;
-      const TensorD& tx = p.x[u.dir];
-      const TensorD& ty = p.dout[u.dir];
-      const T* qx = (const T*)tx.ptr + ((long)u.b * tx.s0 + (long)hnext * tx.s2);
-      const T* qy = (const T*)ty.ptr + ((long)u.b * ty.s0 + (long)hnext * ty.s2);
-      const long t0 = u.dir ? p.L - 1 - u.c * CS : u.c * CS, sgn = u.dir ? -1 : 1;
+      const __amdgpu_buffer_rsrc_t rx = rows(p.x[u.dir], hnext);
+      const int sx = (int)p.x[u.dir].s1;
+      if constexpr (SPLIT) {
 #pragma unroll
-      for (int i = 0; i < PT; ++i) {
-        const int e4 = tq + i * NTHREADS, l = e4 / G4, p4 = (e4 % G4) * 4;
-        const bool ok = p4 < p.P && (FULL || l < rm.nvalid);
-        const long ox = ok ? (t0 + sgn * l) * tx.s1 + p4 : 0, oy = ok ? (t0 + sgn * l) * ty.s1 + p4 : 0;
-        if constexpr (SPLIT) {
-          const f4 b = *(const f4*)(qx + ox);
-          l_xv[i] = ok ? b : (f4){0, 0, 0, 0};
-        } else {
-          const uint2 a = *(const uint2*)(qy + oy), b = *(const uint2*)(qx + ox);
-          l_ny[i] = ok ? a : make_uint2(0u, 0u);
-          l_nx[i] = ok ? b : make_uint2(0u, 0u);
+        for (int i = 0; i < PT; ++i)
+          l_xv[i] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rx, row_piece(tq + i * NTHREADS, sx), 0, 0));
+      } else {
+        const __amdgpu_buffer_rsrc_t ry = rows(p.dout[u.dir], hnext);
+        const int sy = (int)p.dout[u.dir].s1;
+#pragma unroll
+        for (int i = 0; i < PT; ++i) {
+          l_ny[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(ry, row_piece(tq + i * NTHREADS, sy), 0, 0));
+          l_nx[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rx, row_piece(tq + i * NTHREADS, sx), 0, 0));
         }
       }
     }
@@ -368,8 +379,9 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     {
       const float worst = fmaxf(fmaxf(fabsf(tt[0]), fabsf(tt[1])), fmaxf(fabsf(tt[2]), fabsf(tt[3])));
       const bool bad = !(worst <= SPAN_LIMIT);  // also true for NaN
-      const int wbad = __any(bad) ? 1 : 0;
-      if (lane == 0) s.bad[wave] = wbad;
+      int wq = wave;
+      asm volatile("" : "+v"(wq));   // (an address formed here, not kept)
+      s.bad[wq] = __any(bad) ? 1 : 0;
     }
     __syncthreads();
     const int4 bd = *(const int4*)s.bad;
@@ -379,7 +391,8 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
       any_bad |= be.x | be.y | be.z | be.w;
     }
     const bool skip = any_bad != 0;  // uniform: the whole head is left to the level-hierarchy kernel
-    if (tid == 0) redo[(u.dir * nblocks + wg) * p.hpg + (DUAL && half ? p.hpg - 1 - hh : hh)] = skip ? 1 : 0;
+    // (all threads store the one value: a store under a lane condition has the waits for the requests before it wait for the store as well)
+    redo[(u.dir * nblocks + wg) * p.hpg + (DUAL && half ? p.hpg - 1 - hh : hh)] = skip ? 1 : 0;
     if (DIAG32 && skip) s.shared[wave] = 1;
     const uint16_t* xs_ = s.xs;
     const uint16_t* dys_ = s.dys();
@@ -457,24 +470,27 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
         return (f4){__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u), __uint_as_float(a.y << 16),
                     __uint_as_float(a.y & 0xffff0000u)};
       };
-      auto b_of = [&](int k) { return BL ? s.bl[k * NTHREADS + tid] : l_Bv[BCL || BL ? 0 : k]; };
-      auto half_of = [](unsigned w, int k) { return __uint_as_float((k & 1) ? (w & 0xffff0000u) : (w << 16)); };
+      auto b_tile = [&](int R) {   // B of the lane's rows of tile R
+        if constexpr (BL) return s.bl[R * NTHREADS + tid];
+        else return (f4){l_Bv[BCL ? 0 : 4 * R], l_Bv[BCL ? 0 : 4 * R + 1], l_Bv[BCL ? 0 : 4 * R + 2], l_Bv[BCL ? 0 : 4 * R + 3]};
+      };
       // Cu = C up (operand of the G blocks), Bi = B dt' iup (operand of the F blocks)
       bf4 Ch[4], Bh[4], Cl[4], Bl[4];
       float cf32[ALL32 ? 16 : 1], bf32[ALL32 ? 16 : 1];
 #pragma unroll
-      for (int J = 0; J < 4; ++J)
+      for (int J = 0; J < 4; ++J) {
+        f4 b4, c4;
+        if constexpr (!BCL) {
+          b4 = b_tile(J);
+          c4 = (f4){l_Cv[4 * J], l_Cv[4 * J + 1], l_Cv[4 * J + 2], l_Cv[4 * J + 3]};
+        } else {  // out of the workgroup's LDS copy of the group's B and C
+          b4 = wide(s.bc_of(J, tid));
+          c4 = wide(s.bc_of(4 + J, tid));
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int k = 4 * J + j;
-          float cu, bi;
-          if constexpr (!BCL) {
-            cu = l_Cv[k] * up[k];
-            bi = b_of(k) * dtp[k] * iup[k];
-          } else {  // out of the workgroup's LDS copy of the group's B and C
-            cu = half_of(s.bc[(8 + (k >> 1)) * NTHREADS + tid], k) * up[k];
-            bi = half_of(s.bc[(k >> 1) * NTHREADS + tid], k) * dtp[k] * iup[k];
-          }
+          const float cu = c4[j] * up[k], bi = b4[j] * dtp[k] * iup[k];
           if constexpr (ALL32) {
             cf32[k] = cu;
             bf32[k] = bi;
@@ -487,6 +503,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
             Bl[J][j] = (__bf16)(bi - (float)Bh[J][j]);
           }
         }
+      }
       // B (and, for bf16 inputs, C) as the column phase needs them: bf16 inputs are bf16 numbers and stay packed, two
       // to a register
       unsigned bvp[8], cvp[8];
@@ -494,9 +511,10 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
       if constexpr (BCL && DIAG32) {  // read tile by tile below
       } else if constexpr (BCL) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          bvp[i] = s.bc[i * NTHREADS + tid];
-          cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
+        for (int q = 0; q < 4; ++q) {
+          const uint2 b2 = s.bc_of(q, tid), c2 = s.bc_of(4 + q, tid);
+          bvp[2 * q] = b2.x; bvp[2 * q + 1] = b2.y;
+          cvp[2 * q] = c2.x; cvp[2 * q + 1] = c2.y;
         }
       } else {
 #pragma unroll
@@ -568,9 +586,10 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
         float cd[4], bd[4];                       // DIAG32: the operands of rows 16 R + 4 g4 + j
         if constexpr (DIAG32) {
 #pragma unroll
-          for (int i = 2 * R; i < 2 * R + 2; ++i) {
-            bvp[i] = s.bc[i * NTHREADS + tid];
-            cvp[i] = s.bc[(8 + i) * NTHREADS + tid];
+          for (int j = 0; j < 2; ++j) {
+            const uint2 b2 = s.bc_of(R, tid), c2 = s.bc_of(4 + R, tid);
+            bvp[2 * R + j] = j ? b2.y : b2.x;
+            cvp[2 * R + j] = j ? c2.y : c2.x;
           }
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
@@ -652,13 +671,15 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
         // matrix instructions took them: a pair of rows then enters both of its rows as one and the same product and
         // cancels in the suffix sums to fp32 rounding.  The state terms take, with bf16 inputs, the unrounded operands (B and
         // C are exact, the decays fp32); with fp32 inputs the operand pairs are as accurate as the split products Q and R.
+        f4 db4 = s.dbc[R * NTHREADS + tid], dc4 = s.dbc[(4 + R) * NTHREADS + tid], b4;
+        if constexpr (BL) b4 = b_tile(R);
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int k = 4 * R + rr;
-          const float bv = SPLIT ? (BL ? b_of(k) : bvf[SPLIT && !BL ? k : 0]) : unpk(bvp, k);
+          const float bv = SPLIT ? (BL ? b4[rr] : bvf[SPLIT && !BL ? k : 0]) : unpk(bvp, k);
           const float E1 = iup[k] * (sg[rr] + xg[rr] + dg[rr]), X2 = up[k] * (sf[rr] + xf[rr] + df[rr]);
-          s.dbc[k * NTHREADS + tid] += dtp[k] * E1;
-          s.dbc[(16 + k) * NTHREADS + tid] += X2;
+          db4[rr] += dtp[k] * E1;
+          dc4[rr] += X2;
           val[k] = bv * E1;
           if constexpr (ALL32) {
             dcs[k] = cf32[k] * (xf[rr] + sf[rr]) - bf32[k] * (xg[rr] + sg[rr]);
@@ -676,6 +697,8 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
             gsum += own;
           }
         }
+        s.dbc[R * NTHREADS + tid] = db4;
+        s.dbc[(4 + R) * NTHREADS + tid] = dc4;
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -781,16 +804,20 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     }
     if constexpr (DUAL) {
       if constexpr (EX_IN_TILES) __syncthreads();
-      float* ex = reinterpret_cast<float*>(EX_IN_TILES ? (unsigned char*)s.xs : smem_raw + 2 * sizeof(SM) + half * DUAL_EX_BYTES);
-      const float* ey = reinterpret_cast<const float*>(EX_IN_TILES ? (const unsigned char*)reinterpret_cast<SM*>(smem_raw + (1 - half) * sizeof(SM))->xs
+      f4* ex = reinterpret_cast<f4*>(EX_IN_TILES ? (unsigned char*)s.xs : smem_raw + 2 * sizeof(SM) + half * DUAL_EX_BYTES);
+      const f4* ey = reinterpret_cast<const f4*>(EX_IN_TILES ? (const unsigned char*)reinterpret_cast<SM*>(smem_raw + (1 - half) * sizeof(SM))->xs
                                                                        : smem_raw + 2 * sizeof(SM) + (1 - half) * DUAL_EX_BYTES);
       int tq = tid;
       asm volatile("" : "+v"(tq));
 #pragma unroll
-      for (int k = 0; k < 8; ++k) ex[k * NTHREADS + tq] = val[k];
+      for (int q = 0; q < 2; ++q) ex[q * NTHREADS + tq] = (f4){val[4 * q], val[4 * q + 1], val[4 * q + 2], val[4 * q + 3]};
       __syncthreads();
 #pragma unroll
-      for (int k = 8; k < 16; ++k) val[k] += ey[(15 - k) * NTHREADS + (tq ^ 48)];
+      for (int q = 0; q < 2; ++q) {
+        const f4 v = ey[q * NTHREADS + (tq ^ 48)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) val[15 - 4 * q - j] += v[j];
+      }
       store_late(val);
     } else if constexpr (!ACC && P32) lane_store_ln<false>(p.ddt_part, u.b, u.h, n, vn, g4, rm, val);
     else lane_store_ln<IOB>(p.ddt, u.b, u.h, n, vn, g4, rm, val);
@@ -811,7 +838,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     const SM &s0 = *reinterpret_cast<const SM*>(smem_raw), &s1 = *reinterpret_cast<const SM*>(smem_raw + sizeof(SM));
     float v[16];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = s0.dbc[(16 * half + k) * NTHREADS + tid] + s1.dbc[(16 * half + k) * NTHREADS + tid];
+    for (int k = 0; k < 16; ++k) v[k] = s0.dbc_at(16 * half + k, tid) + s1.dbc_at(16 * half + k, tid);
     if (DIAG32 && p.dbc_part && (s0.shared[wave] | s1.shared[wave])) {
       float* q = p.dbc_part + (long)wg * (32 * NTHREADS) + 16 * half * NTHREADS + tid;
 #pragma unroll
@@ -826,13 +853,13 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
     const long at = (long)p.dir0 * gridDim.x + wg;
     float* q = p.dbc_part + (PARTS ? (long)blockIdx.y * p.ndir * gridDim.x + at : at) * (32 * NTHREADS) + tid;
 #pragma unroll
-    for (int k = 0; k < 32; ++k) q[k * NTHREADS] = s.dbc[k * NTHREADS + tid];
+    for (int k = 0; k < 32; ++k) q[k * NTHREADS] = s.dbc_at(k, tid);
   } else {
     float vb[16], vc[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      vb[k] = s.dbc[k * NTHREADS + tid];
-      vc[k] = s.dbc[(16 + k) * NTHREADS + tid];
+      vb[k] = s.dbc_at(k, tid);
+      vc[k] = s.dbc_at(16 + k, tid);
     }
     if (p.dB[u.dir].ptr) lane_store_ln<IOB>(p.dB[u.dir], u.b, u.g, n, vn, g4, rm, vb);
     if (p.dC[u.dir].ptr) lane_store_ln<IOB>(p.dC[u.dir], u.b, u.g, n, vn, g4, rm, vc);
