@@ -671,6 +671,7 @@ __global__ __launch_bounds__(TILES >= DUAL_TILES ? 2 * NTHREADS : NTHREADS, 2) v
         // matrix instructions took them: a pair of rows then enters both of its rows as one and the same product and
         // cancels in the suffix sums to fp32 rounding.  The state terms take, with bf16 inputs, the unrounded operands (B and
         // C are exact, the decays fp32); with fp32 inputs the operand pairs are as accurate as the split products Q and R.
+        if constexpr (!SPLIT) __builtin_amdgcn_sched_barrier(0);   // (asked for any earlier, the sums cost 8 to 20 bytes a lane of scratch)
         f4 db4 = s.dbc[R * NTHREADS + tid], dc4 = s.dbc[(4 + R) * NTHREADS + tid], b4;
         if constexpr (BL) b4 = b_tile(R);
 #pragma unroll

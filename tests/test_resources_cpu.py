@@ -58,7 +58,7 @@ def kernels():
     (r"k_bwd_tile<[234], false, false, (true|false), false, false, (true|false)>", 12, 256, 0),
     # both directions, and two heads side by side: one workgroup of eight waves
     (r"k_bwd_tile<1[012], (true|false), (true|false), false, false, true, false>", 7, 256, 0),
-    (r"k_bwd_tile<(18|19|20), (true|false), (true|false), false, false, (true|false), false>", 18, 256, 8),   # (fp32 heads of 33 to 47, complete tiles)
+    (r"k_bwd_tile<(18|19|20), (true|false), (true|false), false, false, (true|false), false>", 18, 256, 0),
     # two groups of four waves: with up to two head tiles two workgroups a CU
     (r"(k_chunk_scan|k_bwd_dx)<2, (true|false), (true|false), (true|false), 2>", 16, 128, 0),
     (r"(k_chunk_scan|k_bwd_dx)<[34], (true|false), (true|false), (true|false), 2>", 32, 256, 0),
