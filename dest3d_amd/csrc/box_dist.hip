@@ -89,6 +89,9 @@ __device__ __forceinline__ float wave_uniform(float v) {
 // turned pay 0.6 us a launch for the look at them (47 and 201 us).
 // As accurate, but rounded elsewhere, and an encoding that differs in the last bit of one value in ten thousand moves entries of a
 // gradient behind six bf16 layers by up to 0.48 of their mean square: training keeps the sums it had.
+// In training such a box's corners still enter one by one, the same operations in the same order, but from the two positions an axis has
+// (corner_window_axes; in the queue too): 6 logarithms and 36 products of two axes a pair instead of 24 and 72.  8 x 1024 points, 256 boxes, bf16 162
+// -> 139 us, the same values.  (Loops of their own: with both forms in one step the kernel spilled 92 bytes a lane.)
 constexpr int BD_SEG = 512;     // points per wave at most
 constexpr int BD_FWD_T = 1024;  // 16 waves = 8 adjacent boxes x 2 segments per workgroup, one workgroup (96 KB of LDS) per CU
 constexpr int BD_NS = 20;      // floats from node to node
@@ -120,17 +123,6 @@ __device__ __forceinline__ AxisNodes axis_nodes(float p0, float p1, int n, int s
   }
   return a;
 }
-__device__ __forceinline__ bool finite_(float v) { return fabsf(v) <= 3.402823466e38f; }
-// Whether the box's corners (order of box_corner) are two positions per axis, unrotated, all finite.
-__device__ __forceinline__ bool along_axes(const BoxLane& bx) {
-  bool ok = finite_(bx.cx[0]) && finite_(bx.cx[2]) && finite_(bx.cy[0]) && finite_(bx.cy[1]) && finite_(bx.cz[0]) && finite_(bx.cz[4]);
-#pragma unroll
-  for (int c = 0; c < 8; ++c)
-    ok = ok && bx.cx[c] == bx.cx[c & 2] && bx.cy[c] == bx.cy[(c ^ (c >> 1)) & 1] && bx.cz[c] == bx.cz[c & 4] && bx.cs[c] == 1.0f &&
-         bx.sn[c] == 0.0f;
-  return ok;
-}
-
 template <bool BF, bool AXES>
 __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_points) {
   __shared__ __attribute__((aligned(16))) float tab[BD_MAXCELLS * BD_NS];
@@ -163,7 +155,8 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       bx.cs[c] = wave_uniform(bx.cs[c]); bx.sn[c] = wave_uniform(bx.sn[c]);
     }
     int base = 0;
-    bool axes = AXES && along_axes(bx);   // uniform
+    const bool aligned = along_axes(bx);   // uniform
+    bool axes = AXES && aligned;
     if (axes) {
 #pragma unroll
       for (int w = 0; w < BD_FWD_T / 64; ++w) axes = axes && __builtin_amdgcn_readfirstlane(odd_of[w]) == 0;
@@ -209,13 +202,15 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
         if (li < n) store_dist<BF>(p, ((long)b * p.L + l0 + li) * p.K + k, acc);
       }
     }
-    for (; base < n; base += 64) {
+    // a step's points: those with a window at once, the others into the queue
+    auto step = [&](auto window) __attribute__((always_inline)) {
       const int li = base + lane;
       const bool valid = li < n;
       const float* key = p.key + ((long)b * p.L + l0 + (valid ? li : n - 1)) * 3;
       const float kx = key[0], ky = key[1], kz = key[2];
       Window win;
-      const bool one_window = corner_window(p, bx, kx, ky, kz, scale, win);
+      const int one_window = window(kx, ky, kz, win);
+      if (one_window < 0) return false;   // uniform
       if (valid && one_window) {
         f4 acc[4];
 #pragma unroll
@@ -230,7 +225,18 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
       const unsigned long long rest = __ballot(valid && !one_window);
       if (valid && !one_window) queue[wave][queued + __popcll(rest & ((1ull << lane) - 1ull))] = (unsigned short)li;
       queued += __popcll(rest);
+      return true;
+    };
+    if (aligned) {
+#pragma unroll 1
+      for (; base < n; base += 64)
+        if (!step([&](float kx, float ky, float kz, Window& win) -> int {
+              if (__ballot(!(finite_(kx) && finite_(ky) && finite_(kz))) != 0ull) return -1;   // (this and what follows: below)
+              return corner_window_axes(p, bx, kx, ky, kz, scale, win);
+            })) break;
     }
+#pragma unroll 1
+    for (; base < n; base += 64) step([&](float kx, float ky, float kz, Window& win) -> int { return corner_window(p, bx, kx, ky, kz, scale, win); });
   }
   if (lane == 0) queue_len[wave] = queued;
   __syncthreads();
@@ -246,22 +252,32 @@ __global__ __launch_bounds__(BD_FWD_T) void k_box_dist_fwd(BoxDistP p, int seg_p
     f4 acc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
-    // A rolled loop that always works on slot 0 and then rotates the box's registers by one corner: fully unrolled,
-    // the compiler issues the LDS reads of all 8 corners first and spills them.
-#pragma unroll 1
-    for (int c = 0; c < 8; ++c) {
-      const float dx = bx.cx[0] - kx, dy = bx.cy[0] - ky, dz = bx.cz[0] - kz;
-      const float rx = dx * bx.cs[0] - dy * bx.sn[0], ry = dx * bx.sn[0] + dy * bx.cs[0];
+    auto corner = [&](float x, float y, float z) __attribute__((always_inline)) {
       Tri t;
-      trilinear(p, node_pos(rx, p.log_scale, scale, p.W), node_pos(ry, p.log_scale, scale, p.H),
-                node_pos(dz, p.log_scale, scale, p.D), t, BD_NS);
+      trilinear(p, x, y, z, t, BD_NS);
 #pragma unroll
       for (int n8 = 0; n8 < 8; ++n8) {
         const f4* src = (const f4*)(tab + t.off[n8]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] += t.w[n8] * src[j];
       }
-      rotate_box(bx);
+    };
+    if (along_axes(bx) && __ballot(!(finite_(kx) && finite_(ky) && finite_(kz))) == 0ull) {   // uniform; the same sums from two positions an axis
+      const float x0 = node_pos(bx.cx[0] - kx, p.log_scale, scale, p.W), x1 = node_pos(bx.cx[2] - kx, p.log_scale, scale, p.W),
+                  y0 = node_pos(bx.cy[0] - ky, p.log_scale, scale, p.H), y1 = node_pos(bx.cy[1] - ky, p.log_scale, scale, p.H),
+                  z0 = node_pos(bx.cz[0] - kz, p.log_scale, scale, p.D), z1 = node_pos(bx.cz[4] - kz, p.log_scale, scale, p.D);
+#pragma unroll 1
+      for (int c = 0; c < 8; ++c) corner(c & 2 ? x1 : x0, (c ^ (c >> 1)) & 1 ? y1 : y0, c & 4 ? z1 : z0);
+    } else {
+      // A rolled loop that always works on slot 0 and then rotates the box's registers by one corner: fully unrolled,
+      // the compiler issues the LDS reads of all 8 corners first and spills them.
+#pragma unroll 1
+      for (int c = 0; c < 8; ++c) {
+        const float dx = bx.cx[0] - kx, dy = bx.cy[0] - ky, dz = bx.cz[0] - kz;
+        const float rx = dx * bx.cs[0] - dy * bx.sn[0], ry = dx * bx.sn[0] + dy * bx.cs[0];
+        corner(node_pos(rx, p.log_scale, scale, p.W), node_pos(ry, p.log_scale, scale, p.H), node_pos(dz, p.log_scale, scale, p.D));
+        rotate_box(bx);
+      }
     }
     store_dist<BF>(p, ((long)b * p.L + l) * p.K + k, acc);
   }

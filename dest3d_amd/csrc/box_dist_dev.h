@@ -71,6 +71,17 @@ __device__ __forceinline__ void rotate_box(BoxLane& bx) {
   bx.cx[7] = x0; bx.cy[7] = y0; bx.cz[7] = z0; bx.cs[7] = c0; bx.sn[7] = s0;
 }
 
+__device__ __forceinline__ bool finite_(float v) { return fabsf(v) <= 3.402823466e38f; }
+// Whether the box's corners (order of box_corner) are two positions per axis, unrotated, all finite.
+__device__ __forceinline__ bool along_axes(const BoxLane& bx) {
+  bool ok = finite_(bx.cx[0]) && finite_(bx.cx[2]) && finite_(bx.cy[0]) && finite_(bx.cy[1]) && finite_(bx.cz[0]) && finite_(bx.cz[4]);
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+    ok = ok && bx.cx[c] == bx.cx[c & 2] && bx.cy[c] == bx.cy[(c ^ (c >> 1)) & 1] && bx.cz[c] == bx.cz[c & 4] && bx.cs[c] == 1.0f &&
+         bx.sn[c] == 0.0f;
+  return ok;
+}
+
 // signed log compression and grid_sample's un-normalisation (align_corners False) in one: position in node units
 __device__ __forceinline__ float node_pos(float v, float log_scale, float scale, int n) {
   const float m = __log2f(fabsf(v) * log_scale + 1.0f) * scale;  // scale = 1 / (log2(8) * max_value)
@@ -147,6 +158,42 @@ __device__ __forceinline__ bool corner_window(const BoxDistP& p, const BoxLane& 
         for (int k = 0; k < 3; ++k) win.w[k * 9 + i * 3 + j] = fmaf(az[k], yx, win.w[k * 9 + i * 3 + j]);
       }
   }
+  return true;
+}
+// The window of a box along the axes (finite point): two positions an axis, 6 logarithms instead of 24, and the corners' weights as above, in
+// the same operations in the same order.
+__device__ __forceinline__ bool corner_window_axes(const BoxDistP& p, const BoxLane& bx, float kx, float ky, float kz, float scale, Window& win) {
+  float ax[2][3], ay[2][3], az[2][3];
+  auto axis = [&](float p0, float p1, int& m, float (&a)[2][3]) {
+    const float g0 = floorf(p0), g1 = floorf(p1), f[2] = {p0 - g0, p1 - g1};
+    const int i[2] = {(int)g0, (int)g1};
+    m = min(i[0], i[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const bool s = i[e] != m;
+      a[e][0] = s ? 0.0f : 1.0f - f[e];
+      a[e][1] = s ? 1.0f - f[e] : f[e];
+      a[e][2] = s ? f[e] : 0.0f;
+    }
+    return max(i[0], i[1]) - m <= 1;
+  };
+  const bool okx = axis(node_pos(bx.cx[0] - kx, p.log_scale, scale, p.W), node_pos(bx.cx[2] - kx, p.log_scale, scale, p.W), win.mx, ax),
+             oky = axis(node_pos(bx.cy[0] - ky, p.log_scale, scale, p.H), node_pos(bx.cy[1] - ky, p.log_scale, scale, p.H), win.my, ay),
+             okz = axis(node_pos(bx.cz[0] - kz, p.log_scale, scale, p.D), node_pos(bx.cz[4] - kz, p.log_scale, scale, p.D), win.mz, az);
+  if (!(okx && oky && okz)) return false;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const float yx[2][2] = {{ay[0][i] * ax[0][j], ay[0][i] * ax[1][j]}, {ay[1][i] * ax[0][j], ay[1][i] * ax[1][j]}};
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        float w = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) w = fmaf(az[c >> 2][k], yx[(c ^ (c >> 1)) & 1][(c >> 1) & 1], w);
+        win.w[k * 9 + i * 3 + j] = w;
+      }
+    }
   return true;
 }
 // visit the window's nodes that lie inside the table and carry weight: f(LDS offset in floats, weight)
@@ -258,6 +305,45 @@ __device__ __forceinline__ void for_entries(const CornerGrid& cg, F f) {
   } else {
 #pragma unroll
     for (int c = 0; c < 8; ++c) f(cg.ix[c], cg.iy[c], cg.iz[c], 1u << c);
+  }
+}
+
+// The same of a box along the axes, whose corners are two positions per axis: base nodes and clusters are an axis', and the corners of a
+// combination those that its three clusters have in common -- the entries that corner_grid finds, from 6 logarithms instead of 24.
+struct AxisClusters {
+  int anchor[2];
+  unsigned corners[2];   // of either cluster; the second may have none
+};
+__device__ __forceinline__ AxisClusters axis_clusters(float p0, float p1, unsigned at0, unsigned at1) {
+  const int i0 = (int)floorf(p0), i1 = (int)floorf(p1), lo = min(i0, i1), hi = max(i0, i1);
+  const bool apart = hi > lo + 1;
+  AxisClusters a;
+  a.anchor[0] = lo;
+  a.anchor[1] = apart ? hi : lo;
+  const unsigned far = !apart ? 0u : i0 == hi ? at0 : at1;
+  a.corners[1] = far;
+  a.corners[0] = 0xffu & ~far;
+  return a;
+}
+// the corners (order of box_corner) at either position of an axis
+constexpr unsigned BOX_X0 = 0x33u, BOX_X1 = 0xccu, BOX_Y0 = 0x99u, BOX_Y1 = 0x66u, BOX_Z0 = 0x0fu, BOX_Z1 = 0xf0u;
+template <class F>
+__device__ __forceinline__ void for_axis_entries(const BoxDistP& p, const BoxLane& bx, float kx, float ky, float kz, float scale, F f) {
+  const AxisClusters x = axis_clusters(node_pos(bx.cx[0] - kx, p.log_scale, scale, p.W), node_pos(bx.cx[2] - kx, p.log_scale, scale, p.W), BOX_X0, BOX_X1),
+                     y = axis_clusters(node_pos(bx.cy[0] - ky, p.log_scale, scale, p.H), node_pos(bx.cy[1] - ky, p.log_scale, scale, p.H), BOX_Y0, BOX_Y1),
+                     z = axis_clusters(node_pos(bx.cz[0] - kz, p.log_scale, scale, p.D), node_pos(bx.cz[4] - kz, p.log_scale, scale, p.D), BOX_Z0, BOX_Z1);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (k && __ballot(z.corners[1] != 0u) == 0ull) continue;   // uniform
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (i && __ballot(y.corners[1] != 0u) == 0ull) continue;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const unsigned mask = x.corners[j] & y.corners[i] & z.corners[k];
+        if (mask) f(x.anchor[j], y.anchor[i], z.anchor[k], mask);
+      }
+    }
   }
 }
 

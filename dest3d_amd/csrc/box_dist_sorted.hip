@@ -30,6 +30,7 @@ constexpr int BDS_MAXBINS = 9280;  // (D + 2)(H + 2)(W + 2) for D*H*W <= 1024 is
 // atomics; without those 53 and 15).
 constexpr int BDS_NWG = 1024;
 constexpr int BDS_OUT = 27 * BD_C; // results per work item
+constexpr int BDS_BOX = 48;        // floats of a box
 
 struct SortP {
   unsigned* scal;               // [0] bits of max|ddist|, [1] number of work items
@@ -39,7 +40,8 @@ struct SortP {
   int* items;                   // [maxitems][3] bin, first entry, one past the last entry
   unsigned long long* records;  // [maxrecords] pair index | corner mask << 32
   long long* item_out;          // [maxitems][BDS_OUT]
-  float* boxtab;                // [B * K][40] corners x, y, z and rotations cos, sin of every box, 8 values each
+  float* boxtab;                // [B * K][BDS_BOX] corners x, y, z and rotations cos, sin of every box, 8 values each; two x, y, z and whether
+                                // they are the box (along_axes)
   long long* dtab;              // [2][cells][16]: sums of the low 32 bits of the items' results, sums of the rest
   int nbins, maxitems, nwg;   // nwg: BDS_NWG or half of it
   long maxrecords;
@@ -73,19 +75,23 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_boxes(BoxDistP p, SortP s) {
   if (i >= p.B * p.K) return;
   BoxLane bx;
   load_box(p, i / p.K, i % p.K, bx);
-  float* o = s.boxtab + (long)i * 40;
+  float* o = s.boxtab + (long)i * BDS_BOX;
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     o[c] = bx.cx[c]; o[8 + c] = bx.cy[c]; o[16 + c] = bx.cz[c]; o[24 + c] = bx.cs[c]; o[32 + c] = bx.sn[c];
   }
+  *(f4*)(o + 40) = (f4){bx.cx[0], bx.cx[2], bx.cy[0], bx.cy[1]};
+  *(f4*)(o + 44) = (f4){bx.cz[0], bx.cz[4], along_axes(bx) ? 1.0f : 0.0f, 0.0f};
 }
 
-// The walk shared by count and fill: thread = (b, l, k) as in the forward, f(bin, pair index, corner mask).
+// The walk shared by count and fill: thread = (b, l, k) as in the forward, f(bin, pair index, corner mask).  A wave whose boxes all stand
+// along the axes finds their entries axis by axis: 8 x 1024 points, 256 boxes, count 52 -> 29 us, fill 62 -> 37.
 template <class F>
 __device__ __forceinline__ void bds_walk(const BoxDistP& p, F f) {
   const Items it = my_items(p);
   const float scale = 1.0f / (3.0f * p.max_value);
   BoxLane bx;
+  bool axes = false;
   long cur = -1;
   for (long item = it.i0; item < it.i1; ++item) {
     const int l = (int)(item % p.L);
@@ -94,16 +100,23 @@ __device__ __forceinline__ void bds_walk(const BoxDistP& p, F f) {
     if (k >= p.K) continue;
     if (bk != cur) {
       load_box(p, b, k, bx);
+      axes = along_axes(bx);
       cur = bk;
     }
     const float* key = p.key + ((long)b * p.L + l) * 3;
-    CornerGrid cg;
-    corner_grid(p, bx, key[0], key[1], key[2], scale, cg);
+    const float kx = key[0], ky = key[1], kz = key[2];
     const unsigned pid = (unsigned)(((long)b * p.L + l) * p.K + k);
-    for_entries(cg, [&](int mx, int my, int mz, unsigned mask) {
+    auto entry = [&](int mx, int my, int mz, unsigned mask) {
       const int bin = bds_bin(p, mx, my, mz);
       if (bin >= 0) f(bin, pid, mask);
-    });
+    };
+    if (__ballot(!(axes && finite_(kx) && finite_(ky) && finite_(kz))) == 0ull) {
+      for_axis_entries(p, bx, kx, ky, kz, scale, entry);
+    } else {
+      CornerGrid cg;
+      corner_grid(p, bx, kx, ky, kz, scale, cg);
+      for_entries(cg, entry);
+    }
   }
 }
 
@@ -308,27 +321,54 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_accum(BoxDistP p, SortP s) {
 #pragma unroll
         for (int j = 0; j < (BF ? 2 : 4); ++j) graw[j] = src[j];
       }
-      f4 bt[10];  // the box: x[8], y[8], z[8], cos[8], sin[8]
+      const float* box = s.boxtab + ((long)b * p.K + k) * BDS_BOX;
+      const f4 two_xy = *(const f4*)(box + 40), two_z = *(const f4*)(box + 44);
+      // A box along the axes: the entry's corners are all that its positions on the three axes have in common, and the sum of their
+      // weights is a product of sums over an axis' positions: 6 logarithms and 36 products an entry instead of 24 and 288 (8 x 1024 points,
+      // 256 boxes, bf16 170 -> 116 us).
+      if (__ballot(!(two_z[2] != 0.0f && finite_(kx) && finite_(ky) && finite_(kz))) == 0ull) {
+        auto hats = [&](float p0, float p1, unsigned at0, unsigned at1, float m, int n, float (&a)[3]) {
+          float a0[3], a1[3];
+          axis3(node_pos(p0, p.log_scale, scale, n), m, a0);
+          axis3(node_pos(p1, p.log_scale, scale, n), m, a1);
 #pragma unroll
-      for (int j = 0; j < 10; ++j) bt[j] = *(const f4*)(s.boxtab + ((long)b * p.K + k) * 40 + 4 * j);
+          for (int j = 0; j < 3; ++j) a[j] = (mask & at0 ? a0[j] : 0.0f) + (mask & at1 ? a1[j] : 0.0f);
+        };
+        float ax[3], ay[3], az[3];
+        hats(two_xy[0] - kx, two_xy[1] - kx, BOX_X0, BOX_X1, fmx, p.W, ax);
+        hats(two_xy[2] - ky, two_xy[3] - ky, BOX_Y0, BOX_Y1, fmy, p.H, ay);
+        hats(two_z[0] - kz, two_z[1] - kz, BOX_Z0, BOX_Z1, fmz, p.D, az);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if (mask & (1u << c)) {
-          float x, y, z;
-          corner_pos(p, bt[c >> 2][c & 3], bt[2 + (c >> 2)][c & 3], bt[4 + (c >> 2)][c & 3], bt[6 + (c >> 2)][c & 3],
-                     bt[8 + (c >> 2)][c & 3], kx, ky, kz, scale, x, y, z);
-          float ax[3], ay[3], az[3];
-          axis3(x, fmx, ax);
-          axis3(y, fmy, ay);
-          axis3(z, fmz, az);
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-          for (int i = 0; i < 3; ++i)
+          for (int j = 0; j < 3; ++j) {
+            const float yx = ay[i] * ax[j];
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-              const float yx = ay[i] * ax[j];
+            for (int kk = 0; kk < 3; ++kk) w[kk * 9 + i * 3 + j] = az[kk] * yx;
+          }
+      } else {
+        f4 bt[10];  // the box: x[8], y[8], z[8], cos[8], sin[8]
 #pragma unroll
-              for (int kk = 0; kk < 3; ++kk) w[kk * 9 + i * 3 + j] = fmaf(az[kk], yx, w[kk * 9 + i * 3 + j]);
-            }
+        for (int j = 0; j < 10; ++j) bt[j] = *(const f4*)(box + 4 * j);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          if (mask & (1u << c)) {
+            float x, y, z;
+            corner_pos(p, bt[c >> 2][c & 3], bt[2 + (c >> 2)][c & 3], bt[4 + (c >> 2)][c & 3], bt[6 + (c >> 2)][c & 3],
+                       bt[8 + (c >> 2)][c & 3], kx, ky, kz, scale, x, y, z);
+            float ax[3], ay[3], az[3];
+            axis3(x, fmx, ax);
+            axis3(y, fmy, ay);
+            axis3(z, fmz, az);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+              for (int j = 0; j < 3; ++j) {
+                const float yx = ay[i] * ax[j];
+#pragma unroll
+                for (int kk = 0; kk < 3; ++kk) w[kk * 9 + i * 3 + j] = fmaf(az[kk], yx, w[kk * 9 + i * 3 + j]);
+              }
+          }
         }
       }
       if (BF) {
@@ -487,7 +527,7 @@ static BdsLayout bds_layout(int B, int L, int K, int D, int H, int W) {
   y.records = o; o = bds_align(o + maxrec * 8);
   y.item_out = o; o = bds_align(o + (long)y.maxitems * BDS_OUT * 8);
   y.dtab = o; o = bds_align(o + (long)D * H * W * BD_C * 16);  // two halves
-  y.boxtab = o; o = bds_align(o + (long)B * K * 40 * 4);
+  y.boxtab = o; o = bds_align(o + (long)B * K * BDS_BOX * 4);
   y.total = o;
   return y;
 }

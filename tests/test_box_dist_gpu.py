@@ -105,6 +105,39 @@ def test_boxes_along_the_axes_without_a_gradient(nP, nQ, dims, spread):
         assert (got[ok] - want[ok]).norm() <= 2e-5 * want[ok].norm() + 1e-30
 
 
+@pytest.mark.parametrize("nP,nQ,dims,spread", [(33, 65, (10, 10, 10), 4.0), (1100, 64, (4, 6, 7), 4.0), (700, 100, (5, 4, 3), 0.2),
+                                               (520, 130, (10, 10, 10), 200.0), (4200, 16, (1, 30, 30), 2.0)])
+def test_boxes_along_the_axes_in_training(nP, nQ, dims, spread):
+    """Encoding and table gradient of boxes along the axes, which find windows and weights axis by axis, against the same boxes with one corner moved
+    by a unit in the last place, which take the form by corners: 3e-7 of a position of up to 4, which the logarithm stretches by at most 300
+    nodes next to a point (1e-4 of a node) and by a few elsewhere; 2e-5 of the norm, as against the oracle.  Small and large calls (the gradient in
+    LDS and by sorted windows); a point and a box that are not finite come out in the same places."""
+    from dest3d_amd.box_dist import box_dist, box_parametrization_to_corners
+    key, qxyz, qsize, ang = _inputs(2, nP, nQ, 3 + nP + nQ, False)
+    key, qxyz = (v * np.float32(spread / 4) for v in (key, qxyz))
+    qsize[:, ::3] *= np.float32(1e-3)
+    tk, tq, ts, ta = (torch.from_numpy(v).cuda() for v in (key, qxyz, qsize, ang))
+    g = torch.Generator().manual_seed(2)
+    table, dout = torch.randn(16, *dims, generator=g).cuda(), torch.randn(2, nP, nQ, 16, generator=g).cuda()
+    corners = box_parametrization_to_corners(tq, ts, ta)
+    moved = corners.clone()
+    moved[:, :, 5, 0] = torch.nextafter(moved[:, :, 5, 0], torch.full_like(moved[:, :, 5, 0], 1e9))
+
+    def run(k, c):
+        t = table.clone().requires_grad_()
+        dist = box_dist(t, k, c)
+        dist.backward(dout)
+        return dist.detach(), t.grad
+
+    for got, want in zip(run(tk, corners), run(tk, moved)):
+        assert (got - want).norm() <= 2e-5 * want.norm()
+    tk[0, nP // 2, 1], corners[1, nQ // 2, 2, 0], moved[1, nQ // 2, 2, 0] = float("inf"), float("nan"), float("nan")
+    got, want = run(tk, corners)[0], run(tk, moved)[0]
+    assert torch.equal(got.isfinite(), want.isfinite())
+    ok = want.isfinite()
+    assert (got[ok] - want[ok]).norm() <= 2e-5 * want[ok].norm()
+
+
 def test_local_weight_and_fused_module_call():
     from dest3d_amd.box_dist import BoxDistFun, local_weight
     B, nP, nQ = 2, 50, 256
