@@ -281,7 +281,7 @@ __device__ __forceinline__ unsigned signed_digits(int v) { return ((unsigned)v +
 // 64 w .. 64 w + 63: it stages their values as Wq[node][entry], Gq[channel][entry] and reads back 16 entries per lane.
 constexpr int BDS_ROW = 64 + 4;  // dwords per staged row: lanes of one 16-lane group start 4 banks apart
 template <bool BF>
-__global__ __launch_bounds__(NTHREADS) void k_bds_accum(BoxDistP p, SortP s) {
+__global__ __launch_bounds__(NTHREADS, 3) void k_bds_accum(BoxDistP p, SortP s) {
   __shared__ __attribute__((aligned(16))) unsigned Wq[4][27][BDS_ROW];
   __shared__ __attribute__((aligned(16))) unsigned Gq[4][BD_C][BDS_ROW];
   const int item = blockIdx.x;
@@ -297,8 +297,11 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_accum(BoxDistP p, SortP s) {
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int c = 0; c < 6; ++c) acc[t][c] = (i4){0, 0, 0, 0};
+  // (an item has entries; the next ones' records are requested a batch ahead)
+  unsigned long long ahead = s.records[min(first + (int)threadIdx.x, last - 1)];
   for (int base = first; base < last; base += NTHREADS) {
     const int e = base + threadIdx.x;
+    const unsigned long long rec = ahead;
     float w[27];
 #pragma unroll
     for (int j = 0; j < 27; ++j) w[j] = 0.0f;
@@ -306,7 +309,6 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_accum(BoxDistP p, SortP s) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) g[j] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
     if (e < last) {
-      const unsigned long long rec = s.records[e];
       unsigned pid = (unsigned)rec, mask = (unsigned)(rec >> 32);
       if (pid >= (unsigned)((long)p.B * p.L * p.K) || mask > 255u) { pid = 0u; mask = 0u; }  // never index with a stray record
       const int k = (int)(pid % (unsigned)p.K);
@@ -385,6 +387,7 @@ __global__ __launch_bounds__(NTHREADS) void k_bds_accum(BoxDistP p, SortP s) {
         for (int j = 0; j < 4; ++j) g[j] = __builtin_bit_cast(f4, graw[j]);
       }
     }
+    ahead = s.records[min(e + NTHREADS, last - 1)];
     // a weight is at most 8 (eight corners on one node): 2^27 as an integer; |ddist * g_scale| <= 2^22 (three digits)
 #pragma unroll
     for (int j = 0; j < 27; ++j) Wq[wave][j][lane] = signed_digits(__float2int_rn(w[j] * BDS_W_SCALE));
