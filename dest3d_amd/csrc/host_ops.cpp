@@ -512,10 +512,18 @@ Tensor norm(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, con
 // 8192 x 288 -> 586 in bf16.  Here the tokens are cut into slices that run as one batched product and the slices' results are
 // summed (24 us).
 //
-// The forward products of few tokens are issm_linear_fwd's: 4.6 us to issue where the library's take 19, and the kernels are
-// equally long up to about this many multiply-adds (2048 x 288 -> 586: 8.5 us against 7.4; 4096: 12.3 against 9.3, 512 -> 512:
-// 24 against 9; above, and where training keeps the GPU busy, the kernel counts).
+// The forward products of few tokens are issm_linear_fwd's: 4.6 us to issue where the library's take 19, and the kernels are no
+// longer up to about this many multiply-adds, whatever the sizes (2048 x 288 -> 586: 5.0 us against 6.7; 448 -> 448 6.0 and 5.8).
 constexpr double FEW_PRODUCTS = 3.5e8;
+// With more tokens they are where a contraction of up to this many features is a few steps of its tiles (8192 tokens, issm_linear_fwd's and the
+// library's in us: 96 -> 202 3.9 and 6.1, 288 -> 288 6.2 and 8.9, 288 -> 586 10.6 and 13.0, 384 -> 778 15.3 and 17.9, but 512 -> 512 12.9 and 10.0), and the
+// gradients dx = dy W to as many features, from contractions of up to DX_CONTRACTION (2048 and 8192 tokens: 288 -> 288 5.1 and 6.2, 6.8 and 10.4; 586 -> 288
+// 8.5 and 9.2, 11.6 and 16.3; 906 -> 448 11.5 and 10.5, 21.6 and 20.9; below 2048 tokens they are up to 1 us longer and 14 us sooner issued).
+constexpr int64_t TILE_RESULTS = 384, DX_CONTRACTION = 640;
+// (with results in whole multiples of 64 the library's larger tiles come out even, and are ahead where tokens fill the GPU with them many times:
+// 16384 tokens, 256 -> 256 8.5 and 8.1, 288 -> 288 9.0 and 13.2; 32768, 320 -> 320 22.6 and 19.4, 288 -> 288 14.9 and 21.6; with other results the two
+// meet at 65536 tokens: 288 -> 586 63.1 and 62.8, 352 -> 352 43.9 and 43.8)
+bool tiled_tokens(int64_t tokens, int64_t results) { return tokens <= (results % 64 ? 32768 : 8192); }
 // A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save, as long as
 // it is ahead for 16 to 512 queries (multiples of 32 up to 640 features; separate steps and chain in us, scenes of 1024 tokens and 256
 // queries unless said).  288 features, 4, 8, 11 and 16 scenes: 159 and 138, 269 and 242, 347 and 327, 504 and 492; 192, 16 scenes: 432 and 400; 96, 62:
@@ -555,14 +563,41 @@ bool runs_twice() {
   return (!s.get_fw_grad_mode() && !s.get_inference_mode()) || torch::autograd::get_current_graph_task_id() >= 0 ||
          (s.get_grad_mode() && !at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
 }
-bool few_tokens(const Tensor& x, const Tensor& w, double most = FEW_PRODUCTS) {
+bool own_product(const Tensor& x, const Tensor& w) {
   if (watched() || !own_memory(x) || !own_memory(w)) return false;
   if (x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !x.is_cuda() || w.device() != x.device()) return false;
   if (w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || w.size(1) == 0 || w.size(1) % 32 || x.numel() == 0) return false;
-  return (double)x.numel() * (double)w.size(0) <= most && x.is_contiguous() && w.is_contiguous() &&
-         (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
+  return x.is_contiguous() && w.is_contiguous() && (((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) & 15) == 0;
 }
-Tensor linear_few(const Tensor& x, const Tensor& w) {
+bool few_tokens(const Tensor& x, const Tensor& w, double most = FEW_PRODUCTS) {
+  return own_product(x, w) && (double)x.numel() * (double)w.size(0) <= most;
+}
+bool many_tokens(const Tensor& x, const Tensor& w) {
+  return own_product(x, w) && w.size(0) >= 96 && w.size(1) <= TILE_RESULTS && tiled_tokens(x.numel() / x.size(-1), w.size(0));
+}
+// dx = dy W (issm_linear_dx)
+bool own_dx(const Tensor& dy, const Tensor& w) {
+  if (at::GradMode::is_enabled() || watched() || !own_memory(dy) || !own_memory(w)) return false;
+  if (dy.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kBFloat16 || !dy.is_cuda() || w.device() != dy.device()) return false;
+  if (w.dim() != 2 || dy.dim() < 1 || dy.numel() == 0 || dy.size(-1) != w.size(0) || !dy.is_contiguous() || !w.is_contiguous()) return false;
+  const int64_t tokens = dy.numel() / dy.size(-1);
+  return w.size(0) % 2 == 0 && w.size(0) <= DX_CONTRACTION && w.size(1) % 2 == 0 && w.size(1) >= 96 && w.size(1) <= TILE_RESULTS && tokens >= 64 &&
+         tiled_tokens(tokens, w.size(1)) && (((uintptr_t)dy.data_ptr() | (uintptr_t)w.data_ptr()) & 3) == 0;
+}
+Tensor linear_dx(const Tensor& dy, const Tensor& w) {
+  const c10::DeviceGuard guard(dy.device());
+  at::DimVector sizes(dy.sizes());
+  sizes.back() = w.size(1);
+  Tensor dx = fresh(sizes, dy, at::kBFloat16);
+  issm_linear_args a{};
+  a.job[0] = issm_linear_job{data(dy), data(w), data(dx), dy.numel() / dy.size(-1), (int32_t)w.size(0), (int32_t)w.size(1), 0};
+  a.njobs = 1;
+  a.dtype = ISSM_BF16;
+  a.stream = stream_of(dy);
+  check(issm_linear_dx(&a), "issm_linear_dx");
+  return dx;
+}
+Tensor linear_own(const Tensor& x, const Tensor& w) {
   const c10::DeviceGuard guard(x.device());
   at::DimVector sizes(x.sizes());
   sizes.back() = w.size(0);
@@ -608,7 +643,7 @@ Tensor linear_dw(const Tensor& x, const Tensor& dy) {
 struct LinearFn : public Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
     ctx->save_for_backward({x, w});
-    if (few_tokens(x, w)) return linear_few(x, w);
+    if (few_tokens(x, w) || many_tokens(x, w)) return linear_own(x, w);
     return at::linear(x, w);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
@@ -618,7 +653,7 @@ struct LinearFn : public Function<LinearFn> {
     const Tensor &x = v[0], &w = v[1];
     const Tensor dy = cast(grads[0], x.scalar_type());
     Tensor dx, dw;
-    if (ctx->needs_input_grad(0)) dx = at::matmul(dy, w);
+    if (ctx->needs_input_grad(0)) dx = own_dx(dy, w) ? linear_dx(dy, w) : at::matmul(dy, w);
     if (ctx->needs_input_grad(1)) {
       const Tensor x2 = x.reshape({-1, x.size(-1)}), dy2 = dy.reshape({-1, dy.size(-1)});
       if (narrow_result(x2, dy2)) return {dx, linear_dw(x2, dy2)};

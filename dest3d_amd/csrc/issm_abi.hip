@@ -49,6 +49,8 @@ struct TrP {
 };
 int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
+bool linear_tile_takes(long tokens, int in, int out, bool nn);
+int launch_linear_tile(LinearTileP& p, int njobs, bool nn, hipStream_t st);
 int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwP& p, hipStream_t st);
@@ -915,12 +917,54 @@ static int linear_params(const issm_linear_args* a, LinearP& p, int& n) {
   return ISSM_OK;
 }
 
+// Whether the products go through LDS in tiles (linear_tile.hip) or straight from memory into the matrix operands (linear.hip): the same sums
+// in the same order.  Tiles from 64 tokens and 96 outputs on (linear.hip and tiles in us: 1024 x 96 -> 202 3.4 and 2.9, 192 -> 394 4.8 and 3.8,
+// 320 -> 650 12.9 and 5.1, 4096 x 288 -> 586 12.0 and 6.4), but for odd multiples of 288 features, nine fragments from rows that
+// lie across the memory channels, which linear.hip has sooner up to some 350000 results: 128 x 288 -> 586 3.7 and 4.4, 1024 x 288 -> 288 3.8 and 4.4,
+// 1024 x 864 -> 288 7.7 and 8.5, 1024 x 288 -> 586 5.7 and 4.5 (576 features: 128 tokens 8.0 and 6.3).
+static bool linear_in_tiles(const LinearP& p, int n) {
+  int64_t results = 0;
+  bool nines = true;
+  for (int i = 0; i < n; ++i) {
+    const LinearJob& j = p.job[i];
+    if (j.turn || !linear_tile_takes(j.tokens, 32 * j.steps, j.out, false)) return false;
+    results += (int64_t)j.tokens * j.out;
+    nines = nines && j.steps % 18 == 9;
+  }
+  return !nines || results > 350000;
+}
+
 int issm_linear_fwd(const issm_linear_args* a) {
   LinearP p{};
   int n;
   const int rc = linear_params(a, p, n);
   if (rc || n == 0) return rc;
+  if (linear_in_tiles(p, n)) {
+    LinearTileP q{};
+    for (int i = 0; i < n; ++i) q.job[i] = LinearTileJob{p.job[i].x, p.job[i].w, p.job[i].y, p.job[i].tokens, 32 * p.job[i].steps, p.job[i].out, 0};
+    return launched(launch_linear_tile(q, n, false, (hipStream_t)a->stream), "linear_fwd");
+  }
   return launched(launch_linear(p, n, nullptr, (hipStream_t)a->stream), "linear_fwd");
+}
+
+int issm_linear_dx(const issm_linear_args* a) {
+  if (!a) return fail(ISSM_E_NULL, "linear_dx: args is NULL");
+  if (a->njobs < 0 || a->njobs > ISSM_LINEAR_JOBS) return fail(ISSM_E_SHAPE, "linear_dx: %d products (0..%d)", a->njobs, ISSM_LINEAR_JOBS);
+  if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "linear_dx: dtype %d (bf16 only)", a->dtype);
+  LinearTileP p{};
+  for (int i = 0; i < a->njobs; ++i) {
+    const issm_linear_job& j = a->job[i];
+    if (j.tokens < 0 || j.in < 0 || j.out < 0 || j.turn || j.tokens > 0x7fffffff - 64)
+      return fail(ISSM_E_SHAPE, "linear_dx: (%lld, %d) -> %d, turned by %d", (long long)j.tokens, j.in, j.out, j.turn);
+    if (!linear_tile_takes(j.tokens, j.in, j.out, true))
+      return fail(ISSM_E_UNSUPPORTED, "linear_dx: (%lld, %d) -> %d (from 64 tokens and 96 results on, even sizes)", (long long)j.tokens, j.in, j.out);
+    if (!j.x || !j.w || !j.y) return fail(ISSM_E_NULL, "linear_dx: x/w/y is NULL");
+    if (((uintptr_t)j.x | (uintptr_t)j.w) & 3) return fail(ISSM_E_STRIDE, "linear_dx: x and w must be aligned to 4 bytes");
+    if ((uintptr_t)j.y & 1) return fail(ISSM_E_STRIDE, "linear_dx: y must be aligned to its elements");
+    p.job[i] = LinearTileJob{(const uint16_t*)j.x, (const uint16_t*)j.w, (uint16_t*)j.y, (int)j.tokens, j.in, j.out, 0};
+  }
+  if (a->njobs == 0) return ISSM_OK;
+  return launched(launch_linear_tile(p, a->njobs, true, (hipStream_t)a->stream), "linear_dx");
 }
 
 int issm_layer_in(const issm_linear_args* a, const issm_layer_params_args* b) {

@@ -213,6 +213,16 @@ struct LinearP {
   LinearJob job[2];
   int blocks0, blocks1;   // of the first, of both
 };
+// parameters of the products of many tokens (linear_tile.hip)
+struct LinearTileJob {
+  const uint16_t *x, *w;
+  uint16_t* y;
+  int tokens, in, out, otiles;
+};
+struct LinearTileP {
+  LinearTileJob job[2];
+  int blocks0;
+};
 // parameters of the projections' weight gradient (linear_dw.hip)
 struct LinearDwP {
   const uint16_t *dy, *x;   // (tokens, out), (tokens, in)

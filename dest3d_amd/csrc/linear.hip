@@ -7,8 +7,8 @@
 // two are one such launch, the queries turned into the layout of the scan's states on the way (the last two: layer_out.hip).  Both operands have the contraction index contiguous, which is the operand layout of
 // v_mfma_f32_16x16x32_bf16 as it lies in memory: a wave asks for all fragments of its 16 tokens and 32 outputs at once (27 loads
 // of 16 bytes a lane at 288 features) and multiplies as they arrive; there is nothing to share through LDS that L1 does not
-// share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens or features the fragments' 64-byte pieces
-// of 16 rows a load are what it pays for, and staging tiles through LDS wins: 8192 x 288 -> 586 21 us (13.5).
+// share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens the fragments' 64-byte pieces
+// of 16 rows a load are what it pays for, and staging tiles through LDS wins (linear_tile.hip): 8192 x 288 -> 586 21 us, in tiles 10.6.
 #include "layer_params.h"
 
 namespace issm {

@@ -447,6 +447,9 @@ typedef struct issm_linear_args {
 } issm_linear_args;
 
 int issm_linear_fwd(const issm_linear_args* args);
+/* The products' gradient to x, y (tokens, out) = x (tokens, in) w with w (in, out): `in` the outputs and `out` the features of the product it
+ * belongs to.  From 64 tokens and 96 results on, in and out even, turn 0 (ISSM_E_UNSUPPORTED otherwise); x and w aligned to 4 bytes. */
+int issm_linear_dx(const issm_linear_args* args);
 /* issm_linear_fwd and issm_layer_params in one launch, on the products' stream; neither may read what the other writes. */
 int issm_layer_in(const issm_linear_args* products, const issm_layer_params_args* params);
 

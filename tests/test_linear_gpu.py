@@ -59,6 +59,41 @@ def test_linear_at_its_remainders(shapes):
         assert (y[-1] == 3.0).all()
 
 
+@pytest.mark.parametrize("shapes", [[(8192, 288, 586), (2048, 288, 288)], [(16400, 96, 200)], [(11000, 288, 97)], [(4097, 320, 289), (8193, 64, 610)],
+                                    [(64, 32, 160000)], [(64, 96, 96)], [(3700, 288, 96), (65, 864, 100)]])
+def test_many_tokens_at_their_remainders(shapes):
+    """Products in tiles (from 64 tokens and 96 outputs on, 350000 results for odd multiples of 288): tokens, outputs and contractions that fill
+    no tile or step, rows of odd length."""
+    test_linear_at_its_remainders(shapes)
+
+
+@pytest.mark.parametrize("shapes", [[(64, 2, 96)], [(65, 586, 288), (64, 288, 288)], [(1000, 98, 130)], [(130, 94, 98), (4099, 610, 320)]])
+def test_gradient_to_the_tokens_at_its_remainders(shapes):
+    """issm_linear_dx: y = x w with w (in, out); contractions that end within a piece of eight, a row of which the next begins with what is
+    no number."""
+    lib = L.load()
+    a, kept = Args(), []
+    for i, (t, nin, nout) in enumerate(shapes):
+        g = torch.Generator().manual_seed(3 * i + t)
+        x, w = torch.randn(t, nin, generator=g).bfloat16(), (torch.randn(nin, nout, generator=g) * nin ** -0.5).bfloat16()
+        x[t // 2 :: 7, 0] = float("nan")
+        xd, wd = x.cuda(), w.cuda()
+        y = torch.full((t + 1, nout), 3.0, dtype=torch.bfloat16, device="cuda")
+        a.job[i] = Job(xd.data_ptr(), wd.data_ptr(), y.data_ptr(), t, nin, nout, 0)
+        kept.append((x, w, xd, wd, y))
+    a.njobs, a.dtype, a.stream = len(shapes), L.ISSM_BF16, L.current_stream_ptr(torch.device("cuda", 0))
+    assert lib.issm_linear_dx(C.byref(a)) == 0
+    torch.cuda.synchronize()
+    for x, w, _, _, y in kept:
+        ok = ~x[:, 0].isnan()
+        assert y[:-1].cpu()[~ok].isnan().all()
+        _close(y[:-1][ok.cuda()], x[ok], w.t(), x[ok].double() @ w.double())
+        assert (y[-1] == 3.0).all()
+    for t, nin, nout in ((63, 96, 96), (64, 96, 95), (64, 97, 96), (64, 96, 97)):
+        a.njobs, a.job[0].tokens, a.job[0].nin, a.job[0].nout = 1, t, nin, nout
+        assert lib.issm_linear_dx(C.byref(a)) != 0
+
+
 def test_linear_refuses_what_it_does_not_take():
     lib = L.load()
     x = torch.zeros(64, 64, dtype=torch.bfloat16, device="cuda")
@@ -192,6 +227,31 @@ def test_weight_gradient_of_every_form(form):
     ref, mag = dy.t() @ x, dy.abs().t() @ x.abs()
     # (the library may add in bf16 pieces: a rounding of the result each, four at most)
     assert ((w.grad.double().cpu() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -9 * mag.sqrt() + 300 * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("form", ["few", "many", "odd", "expanded gradient", "unaligned gradient", "wide", "again"])
+def test_gradient_to_the_tokens_of_every_form(form):
+    """Both routes of the projections and of their gradients to the tokens, and the forms that stay the library's."""
+    from dest3d_amd.scan_module import _LinearTokens
+    t, nin, nout = {"many": (2049, 288, 610), "odd": (130, 96, 51), "wide": (100, 96, 1300)}.get(form, (130, 96, 202))
+    x, w, ref = _operands(t, nin, nout, 9)
+    x, w = x.cuda().requires_grad_(), w.cuda()
+    dy = torch.randn(t, nout).cuda().bfloat16()
+    if form == "expanded gradient":
+        dy = dy[:1].expand(t, nout)
+    elif form == "unaligned gradient":
+        dy = torch.cat([dy.new_zeros(1), dy.flatten()])[1:].view(t, nout)
+    y = _LinearTokens.apply(x, w)
+    _close(y.detach(), x.detach().cpu(), w.cpu(), ref)
+    if form == "again":
+        dy.requires_grad_()
+        dx, = torch.autograd.grad(y, x, dy, create_graph=True)
+        got, = torch.autograd.grad(dx, dy, x.detach())
+        _close(got, x.detach().cpu(), w.cpu(), ref)
+    else:
+        y.backward(dy)
+        dx = x.grad
+    _close(dx.detach(), dy.detach().cpu(), w.cpu().t(), dy.detach().double().cpu() @ w.double().cpu())
 
 
 def test_weight_gradient_differentiated_again():
