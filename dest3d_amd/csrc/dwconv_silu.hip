@@ -328,7 +328,7 @@ int launch_dwconv_bwd(const DwConvP& p_, hipStream_t st) {
     else hipLaunchKernelGGL((k_dwconv_bwd<false, 2>), g, b, 0, st, p);
   }
   int e = (int)hipGetLastError();
-  if (e) return e;
+  if (e || !p.dw) return e;
   hipLaunchKernelGGL(k_dwconv_dw, dim3((p.nsets * 8 * p.C + 31) / 32), b, 0, st, p);
   return (int)hipGetLastError();
 }

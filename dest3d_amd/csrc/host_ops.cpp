@@ -14,6 +14,8 @@
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/extension.h>
 
+#include <numeric>
+
 #include "../../include/issm.h"
 
 namespace {
@@ -896,7 +898,7 @@ struct CoreFn : public Function<CoreFn> {
     const Kind* in = r->in;
     const c10::DeviceGuard guard(key.device());
     const int64_t H = r->H, G = r->G, di = r->di, P = di / H, Cc = di + 2 * G, Bsz = d.size(0), Ln = d.size(1),
-                  K = d.size(2), R0 = H + 2 * G, R = H + 4 * G, Wd = di + Cc + H;
+                  K = d.size(2), R0 = H + 2 * G, Wd = di + Cc + H;
     const Scan s = Scan::pop(v, 12, 2, !wt.defined(), r->lo, r->hi);
     const at::ScalarType k = key.scalar_type(), hdt = in[1].type;
     float* const par = data<float>(flat);
@@ -906,7 +908,7 @@ struct CoreFn : public Function<CoreFn> {
     Tensor dkey = fresh(key.sizes(), key, k);
     Tensor dzx = fresh({Bsz, Ln, Wd}, key, k);   // row of d zxbcdt: [dz | d xbc | d dt]; each producer writes its part
     const int64_t nb = issm_rmsnorm_bwd_blocks(Bsz * Ln);
-    Tensor dwp = fresh({nb, di}, key, at::kFloat), dnw = fresh({di}, key, at::kFloat);
+    Tensor dwp = fresh({nb, di}, key, at::kFloat);
     {
       issm_norm_args a = norm_args(key, z2, nw, Tensor(), r->eps, 0, false, false);
       a.rstd = data<float>(rstd);
@@ -917,18 +919,16 @@ struct CoreFn : public Function<CoreFn> {
       a.dz = data(dzx);
       a.dz_row_stride = Wd;
       a.dw_partial = data<float>(dwp);
-      a.dw = data<float>(dnw);
-      check(issm_gated_rmsnorm_bwd(&a), "issm_gated_rmsnorm_bwd");
+      check(issm_gated_rmsnorm_bwd_part(&a), "issm_gated_rmsnorm_bwd_part");
     }
     // 3'. the scan: both directions receive the gradient of their sum, and half of the averaged final states'
     const Tensor dyh = dkey.view({Bsz, Ln, H, P});
     const Tensor dfin = transpose_states(grads[1].reshape({Bsz, K, di}), Tensor(), 0.5, at::kFloat).view({Bsz, H, P, K});
     const Tensor dys[2] = {dyh, dyh}, dlast[2] = {dfin, dfin};
     const Scan::Grad g = s.backward(ws, dys, dlast);
-    // 2'. parameter generation
-    Tensor ddist, dbias = fresh({Bsz, Ln, R}, key, at::kFloat), dW = fresh({R0, WIDTH}, key, at::kFloat),
-                  dbias_sum = fresh({R}, key, at::kFloat);
-    Tensor dwpart = fresh({std::max(issm_param_gen_bwd_blocks(Bsz * Ln), 1), R0, WIDTH}, key, at::kFloat);
+    // 2'. parameter generation; the gradients of its biases go to the convolutions' backward and to dzx
+    const int gen_rows = issm_param_gen_bwd_blocks(Bsz * Ln);
+    Tensor ddist, dwpart = fresh({std::max(gen_rows, 1), R0, WIDTH + 1}, key, at::kFloat), dtail = fresh({2, Bsz, Ln, 2 * G}, key, k);
     if (ctx->needs_input_grad(2)) ddist = fresh(d.sizes(), d, k);
     {
       issm_pgen_args a = pgen_args(d, par + off_w, H, G);
@@ -938,21 +938,17 @@ struct CoreFn : public Function<CoreFn> {
       a.dBm_back = data(g.dB[1]);
       a.dCm_back = data(g.dC[1]);
       a.ddist = data(ddist);
-      a.dbias = data<float>(dbias);
       a.dw_partial = data<float>(dwpart);
-      a.dW = data<float>(dW);
-      a.dbias_sum = data<float>(dbias_sum);
       if (wt.defined()) {
         a.weights = data<const float>(wt);
         a.dt_raw = data(raw);
       }
-      check(issm_param_gen_bwd(&a), "issm_param_gen_bwd");
+      const issm_pgen_producers to{(char*)data(dzx) + (di + Cc) * dzx.element_size(), Wd, data(dtail)};
+      check(issm_param_gen_bwd_part(&a, &to), "issm_param_gen_bwd_part");
     }
     // 1'. the convolutions: gradients of (x, b-bias, c-bias) per branch
-    Tensor dtail = fresh({2, Bsz, Ln, 2 * G}, key, k);
-    dtail.copy_(dbias.narrow(2, H, 4 * G).unflatten(-1, {2, 2 * G}).permute({2, 0, 1, 3}));
-    Tensor part = fresh({std::max(issm_dwconv_partial_rows((int)Bsz, (int)Ln), 1), 2, 8, Cc}, key, at::kFloat);
-    Tensor dcw = fresh({2, Cc, TAPS}, key, at::kFloat), dcb = fresh({2, Cc}, key, at::kFloat);
+    const int conv_rows = issm_dwconv_partial_rows((int)Bsz, (int)Ln);
+    Tensor part = fresh({std::max(conv_rows, 1), 2, 8, Cc}, key, at::kFloat);
     {
       issm_dwconv_args a = conv_args(xbc);
       a.w = par;
@@ -966,26 +962,46 @@ struct CoreFn : public Function<CoreFn> {
       a.du_batch_stride = Ln * Wd;
       a.du_token_stride = Wd;
       a.partial = data<float>(part);
-      a.dw = data<float>(dcw);
-      a.dbias = data<float>(dcb);
-      check(issm_dwconv_silu_bwd(&a), "issm_dwconv_silu_bwd");
+      check(issm_dwconv_silu_bwd_part(&a), "issm_dwconv_silu_bwd_part");
     }
-    dzx.narrow(2, di + Cc, H).copy_(dbias.narrow(2, 0, H));
-    const Tensor dA_log = g.dA.sum(-1).mul_(A1.select(1, 0));
-    const Tensor dh0 = transpose_states(g.dh0.view({Bsz, di, K}), Tensor(), 1.0, kernel_type(hdt));
-    // parameter gradients, inputs 4 .. 13: one buffer, one conversion to the parameters' type when they share one
-    std::vector<Tensor> pg{dcw.select(0, 0), dcb.select(0, 0), dcw.select(0, 1), dcb.select(0, 1), dW.narrow(0, 0, H),
-                           dW.narrow(0, H, 2 * G), dbias_sum.narrow(0, 0, H), dA_log, g.dD, dnw};
-    bool shared = in[4].type != at::kFloat;
-    for (int i = 4; i < NIN; ++i) shared = shared && in[i].type == in[4].type;
-    if (shared) {
-      std::vector<int64_t> n;
-      for (Tensor& t : pg) {
-        n.push_back(t.numel());
-        t = t.reshape({-1});
-      }
-      pg = at::split_with_sizes(at::cat(pg).to(in[4].type), n);
+    // the sums of all the parts, inputs 4 .. 13, in the parameters' type when they share one, and the queries' gradient
+    bool bf16 = true;
+    for (int i = 4; i < NIN; ++i) bf16 = bf16 && in[i].type == at::kBFloat16;
+    const std::vector<int64_t> n{Cc * TAPS, Cc, Cc * TAPS, Cc, H * WIDTH, 2 * G * WIDTH, H, H, g.dD.numel(), di};
+    Tensor dh0 = fresh({Bsz, K, di}, key, kernel_type(hdt)),
+           sums = fresh({std::accumulate(n.begin(), n.end(), (int64_t)0)}, key, bf16 ? at::kBFloat16 : at::kFloat);
+    {
+      issm_layer_grads_args a{};
+      a.conv = data<const float>(part);
+      a.gen = data<const float>(dwpart);
+      a.norm = data<const float>(dwp);
+      a.conv_rows = conv_rows;
+      a.gen_rows = gen_rows;
+      a.norm_rows = (int32_t)nb;
+      a.C = (int32_t)Cc;
+      a.H = (int32_t)H;
+      a.G = (int32_t)G;
+      a.d_inner = (int32_t)di;
+      a.K = (int32_t)K;
+      a.dA = data<const float>(g.dA);
+      a.A = data<const float>(A1);
+      a.dD = data<const float>(g.dD);
+      a.nD = (int32_t)g.dD.numel();
+      a.dtype = code(sums.scalar_type());
+      a.out = data(sums);
+      a.stream = stream_of(key);
+      issm_transpose_args t{};
+      t.batch = (int)Bsz;
+      t.rows = (int)di;
+      t.cols = (int)K;
+      t.in_dtype = ISSM_F32;
+      t.out_dtype = code(dh0.scalar_type());
+      t.in0 = data(g.dh0);
+      t.out = data(dh0);
+      t.alpha = 1.0f;
+      check(issm_layer_grads(&a, &t), "issm_layer_grads");
     }
+    const std::vector<Tensor> pg = at::split_with_sizes(sums, n);
     variable_list out(NIN + 6);
     out[0] = cast(dzx, in[0].type);
     out[1] = cast(dh0, hdt);

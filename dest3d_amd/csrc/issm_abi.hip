@@ -40,14 +40,8 @@ int launch_rmsnorm_fwd(const NormP& p, hipStream_t st);
 int launch_rmsnorm_bwd(const NormP& p, hipStream_t st);
 int launch_hilbert_codes(const HilbertP& p, hipStream_t st);
 int launch_hilbert_order(const HilbertOrderP& p, hipStream_t st);
-struct TrP {
-  int B, R, C, in_dt, out_dt;
-  const void* in0;
-  const void* in1;
-  void* out;
-  float alpha;
-};
 int launch_transpose_states(const TrP& p, hipStream_t st);
+int launch_layer_grads(LayerGradsP& p, const TrP& t, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 bool linear_tile_takes(long tokens, int in, int out, bool nn);
 int launch_linear_tile(LinearTileP& p, int njobs, bool nn, hipStream_t st);
@@ -557,7 +551,7 @@ int issm_rmsnorm_bwd_blocks(int64_t rows) {
   return (int)(rows < 2048 ? rows : 2048);
 }
 
-static int norm_params(const issm_norm_args* a, NormP* p, bool bwd) {
+static int norm_params(const issm_norm_args* a, NormP* p, bool bwd, bool part = false) {
   if (!a) return fail(ISSM_E_NULL, "args is NULL");
   if (a->rows <= 0 || a->ncols <= 0) return fail(ISSM_E_SHAPE, "rmsnorm: rows=%lld ncols=%d", (long long)a->rows, a->ncols);
   const int gs = a->group_size > 0 ? a->group_size : a->ncols;
@@ -566,7 +560,7 @@ static int norm_params(const issm_norm_args* a, NormP* p, bool bwd) {
   if (!a->x || !a->w || !a->rstd) return fail(ISSM_E_NULL, "rmsnorm: x/w/rstd is NULL");
   if (a->ncols > 16384) return fail(ISSM_E_UNSUPPORTED, "rmsnorm: ncols %d > 16384", a->ncols);
   if (!bwd && !a->y) return fail(ISSM_E_NULL, "rmsnorm: y is NULL");
-  if (bwd && (!a->dy || !a->dx || !a->dw_partial || !a->dw)) return fail(ISSM_E_NULL, "rmsnorm bwd: NULL buffer");
+  if (bwd && (!a->dy || !a->dx || !a->dw_partial || (!a->dw && !part))) return fail(ISSM_E_NULL, "rmsnorm bwd: NULL buffer");
   if (bwd && a->z && !a->dz) return fail(ISSM_E_NULL, "rmsnorm bwd: dz is NULL");
   if (a->layer_norm && !a->mean) return fail(ISSM_E_NULL, "layernorm: mean is NULL");
   if (bwd && a->bias && (!a->db_partial || !a->db)) return fail(ISSM_E_NULL, "norm bwd with bias: db_partial/db is NULL");
@@ -598,6 +592,16 @@ int issm_gated_rmsnorm_bwd(const issm_norm_args* a) {
   if (rc) return rc;
   norm_scratch_warm((hipStream_t)a->stream);
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd");
+}
+
+int issm_gated_rmsnorm_bwd_part(const issm_norm_args* a) {
+  NormP p;
+  int rc = norm_params(a, &p, true, true);
+  if (rc) return rc;
+  if (p.b) return fail(ISSM_E_UNSUPPORTED, "rmsnorm_bwd_part: no bias");
+  norm_scratch_warm((hipStream_t)a->stream);
+  p.dw = nullptr;
+  return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_part");
 }
 
 }  // extern "C"
@@ -687,7 +691,7 @@ int issm_gated_rmsnorm_bwd_noalloc(const issm_norm_args* a) {
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_noalloc");
 }
 
-static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward_only = false, bool conv = false) {
+static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward_only = false, bool conv = false, bool part = false) {
   if (!a) return fail(ISSM_E_NULL, "param_gen: args is NULL");
   if (a->tokens < 0 || a->K < 0 || a->H < 1 || a->G < 1) return fail(ISSM_E_SHAPE, "param_gen: bad shape");
   if (a->M != 16) return fail(ISSM_E_UNSUPPORTED, "param_gen: M = %d (only 16 is built)", a->M);
@@ -702,7 +706,7 @@ static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward
     if (!a->bias && a->tok_stride < a->H) return fail(ISSM_E_STRIDE, "param_gen: tok_stride %lld", (long long)a->tok_stride);
     if (a->has_back && (!a->Bm_back || !a->Cm_back)) return fail(ISSM_E_NULL, "param_gen: Bm_back/Cm_back is NULL");
   } else {
-    if (!a->dw_partial || !a->dW) return fail(ISSM_E_NULL, "param_gen bwd: dw_partial/dW is NULL");
+    if (!a->dw_partial || (!a->dW && !part)) return fail(ISSM_E_NULL, "param_gen bwd: dw_partial/dW is NULL");
   }
   p->tokens = a->tokens; p->K = a->K; p->H = a->H; p->G = a->G; p->dtype = a->dtype; p->has_back = a->has_back ? 1 : 0;
   p->dist = a->dist; p->W = a->W; p->bias = a->bias;
@@ -714,6 +718,9 @@ static int pgen_params(const issm_pgen_args* a, PGenP* p, bool bwd, bool forward
   p->dbias_sum = a->dbias_sum;
   p->ddist = a->ddist; p->dbias = a->dbias; p->dw_partial = a->dw_partial; p->dW = a->dW;
   p->nblocks = pgen_bwd_blocks(a->tokens);
+  p->dtok = p->dtail = nullptr;
+  p->dtok_stride = 0;
+  p->bias_partial = nullptr;
   return ISSM_OK;
 }
 
@@ -744,7 +751,20 @@ int issm_param_gen_bwd(const issm_pgen_args* a) {
   return launched(launch_pgen_bwd(p, (hipStream_t)a->stream), "param_gen_bwd");
 }
 
-static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool heads_only = false) {
+int issm_param_gen_bwd_part(const issm_pgen_args* a, const issm_pgen_producers* b) {
+  PGenP p;
+  int rc = pgen_params(a, &p, true, false, false, true);
+  if (rc) return rc;
+  if (!b || !b->dtok || !b->dtail || !a->has_back) return fail(ISSM_E_NULL, "param_gen bwd: dtok/dtail is NULL, or has_back is 0");
+  if (b->dtok_stride < a->H) return fail(ISSM_E_STRIDE, "param_gen bwd: dtok_stride %lld", (long long)b->dtok_stride);
+  if (p.tokens == 0) return ISSM_OK;
+  p.dW = p.dbias_sum = nullptr;
+  p.dtok = b->dtok; p.dtok_stride = b->dtok_stride; p.dtail = b->dtail;
+  p.bias_partial = p.dw_partial + (long)p.nblocks * (p.H + 2 * p.G) * 16;
+  return launched(launch_pgen_bwd(p, (hipStream_t)a->stream), "param_gen_bwd_part");
+}
+
+static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool heads_only = false, bool part = false) {
   if (!a) return fail(ISSM_E_NULL, "dwconv: args is NULL");
   if (a->batch < 0 || a->seqlen < 0 || a->channels < 1) return fail(ISSM_E_SHAPE, "dwconv: bad shape");
   if (a->taps != 7) return fail(ISSM_E_UNSUPPORTED, "dwconv: %d taps (only 7 is built)", a->taps);
@@ -755,7 +775,7 @@ static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool h
   if (a->u_token_stride < a->channels || a->u_batch_stride < 0)
     return fail(ISSM_E_STRIDE, "dwconv: u strides (%lld, %lld)", (long long)a->u_batch_stride, (long long)a->u_token_stride);
   if (!bwd && (!a->bias || !a->y)) return fail(ISSM_E_NULL, "dwconv: bias/y is NULL");
-  if (bwd && (!a->partial || !a->dw || !a->dbias)) return fail(ISSM_E_NULL, "dwconv bwd: partial/dw/dbias is NULL");
+  if (bwd && (!a->partial || (!part && (!a->dw || !a->dbias)))) return fail(ISSM_E_NULL, "dwconv bwd: partial/dw/dbias is NULL");
   p->B = a->batch; p->L = a->seqlen; p->C = a->channels; p->nsets = a->nsets; p->dtype = a->dtype;
   p->chain = a->chain ? 1 : 0;
   p->u = a->u; p->u_bs = a->u_batch_stride; p->u_ls = a->u_token_stride;
@@ -807,6 +827,16 @@ int issm_dwconv_silu_bwd(const issm_dwconv_args* a) {
   int rc = dwconv_params(a, &p, true);
   if (rc) return rc;
   return launched(launch_dwconv_bwd(p, (hipStream_t)a->stream), "dwconv_silu_bwd");
+}
+
+int issm_dwconv_silu_bwd_part(const issm_dwconv_args* a) {
+  DwConvP p;
+  int rc = dwconv_params(a, &p, true, false, true);
+  if (rc) return rc;
+  if (!p.chain) return fail(ISSM_E_UNSUPPORTED, "dwconv_bwd_part: a chained pair only");
+  if (p.B == 0 || p.L == 0) return ISSM_OK;
+  p.dw = p.dbias = nullptr;
+  return launched(launch_dwconv_bwd(p, (hipStream_t)a->stream), "dwconv_silu_bwd_part");
 }
 
 static int box_dist_params(const issm_box_dist_args* a, BoxDistP* p, bool bwd) {
@@ -1053,18 +1083,48 @@ int issm_layer_end(const issm_layer_out_args* a, const issm_linear_args* b) {
   return launched(launch_layer_end(p, q, (hipStream_t)a->stream), "layer_end");
 }
 
-int issm_transpose_states(const issm_transpose_args* a) {
+static int transpose_params(const issm_transpose_args* a, TrP& p) {
   if (!a) return fail(ISSM_E_NULL, "transpose: args is NULL");
   if (a->batch < 0 || a->rows < 0 || a->cols < 0) return fail(ISSM_E_SHAPE, "transpose: bad shape");
   if ((a->in_dtype != ISSM_F32 && a->in_dtype != ISSM_BF16) || (a->out_dtype != ISSM_F32 && a->out_dtype != ISSM_BF16))
     return fail(ISSM_E_DTYPE, "transpose: dtypes %d -> %d", a->in_dtype, a->out_dtype);
+  p.B = 0;
   if (a->batch == 0 || a->rows == 0 || a->cols == 0) return ISSM_OK;
   if (!a->in0 || !a->out) return fail(ISSM_E_NULL, "transpose: in0/out is NULL");
   if (a->batch > 65535 || (a->rows + 63) / 64 > 65535) return fail(ISSM_E_SHAPE, "transpose: batch / rows too large for one launch");
-  TrP p;
   p.B = a->batch; p.R = a->rows; p.C = a->cols; p.in_dt = a->in_dtype; p.out_dt = a->out_dtype;
   p.in0 = a->in0; p.in1 = a->in1; p.out = a->out; p.alpha = a->alpha;
+  return ISSM_OK;
+}
+
+int issm_transpose_states(const issm_transpose_args* a) {
+  TrP p;
+  const int rc = transpose_params(a, p);
+  if (rc || p.B == 0) return rc;
   return launched(launch_transpose_states(p, (hipStream_t)a->stream), "transpose_states");
+}
+
+int issm_layer_grads(const issm_layer_grads_args* a, const issm_transpose_args* b) {
+  if (!a) return fail(ISSM_E_NULL, "layer_grads: args is NULL");
+  if (a->conv_rows < 0 || a->gen_rows < 0 || a->norm_rows < 0 || a->C < 1 || a->H < 1 || a->G < 1 || a->d_inner < 1 || a->K < 0 || a->nD < 0)
+    return fail(ISSM_E_SHAPE, "layer_grads: bad shape");
+  if (a->dtype != ISSM_F32 && a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "layer_grads: dtype %d", a->dtype);
+  if (((int64_t)a->C + a->H + a->G) * 64 + (int64_t)a->H * a->K + a->d_inner + a->nD > ((int64_t)1 << 30)) return fail(ISSM_E_SHAPE, "layer_grads: too large");
+  if ((a->conv_rows && !a->conv) || (a->gen_rows && !a->gen) || (a->norm_rows && !a->norm) || (a->K && (!a->dA || !a->A)) || (a->nD && !a->dD) || !a->out)
+    return fail(ISSM_E_NULL, "layer_grads: a part or out is NULL");
+  TrP t{};
+  if (b) {
+    const int rc = transpose_params(b, t);
+    if (rc) return rc;
+    if (b->in_dtype != ISSM_F32 || b->in1) return fail(ISSM_E_UNSUPPORTED, "layer_grads: states are one fp32 tensor");
+  }
+  const long R0 = a->H + 2 * a->G;
+  LayerGradsP p{};
+  p.conv = a->conv; p.gen = a->gen; p.gen_bias = a->gen ? a->gen + a->gen_rows * R0 * 16 : nullptr; p.norm = a->norm;
+  p.conv_rows = a->conv_rows; p.gen_rows = a->gen_rows; p.norm_rows = a->norm_rows;
+  p.C = a->C; p.H = a->H; p.R0 = (int)R0; p.di = a->d_inner; p.K = a->K; p.nD = a->nD;
+  p.dA = a->dA; p.A = a->A; p.dD = a->dD; p.out = a->out; p.bf16 = a->dtype == ISSM_BF16;
+  return launched(launch_layer_grads(p, t, (hipStream_t)a->stream), "layer_grads");
 }
 
 int issm_hilbert_codes(const issm_hilbert_args* a) {

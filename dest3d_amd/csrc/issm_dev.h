@@ -200,6 +200,24 @@ struct DwConvP {
   float* dbias;        // (nsets, C) fp32
 };
 
+// parameters of the kernels of transpose_states.hip
+struct TrP {
+  int B, R, C, in_dt, out_dt;
+  const void* in0;
+  const void* in1;
+  void* out;
+  float alpha;
+};
+struct LayerGradsP {
+  const float *conv, *gen, *gen_bias, *norm;   // (conv_rows, 2, 8, C), (gen_rows, R0, 16), (gen_rows, R0), (norm_rows, di)
+  int conv_rows, gen_rows, norm_rows;
+  int C, H, R0, di, K, nD;
+  const float *dA, *A, *dD;                    // (H, K), (H, K), (nD)
+  void* out;
+  int bf16;
+  int b_gen, b_bias, b_norm, b_A, b_D, b_tr;   // first workgroup of each kind
+};
+
 // parameters of the dt / B / C generation kernels (param_gen.hip)
 // parameters of the layer-parameter kernel (layer_params.hip)
 constexpr int LAYER_ARRAYS = 9;
@@ -266,7 +284,10 @@ struct PGenP {
   float* dbias;          // (tokens, R) fp32
   float* dbias_sum;      // (R) fp32 or NULL: dbias summed over the tokens
   float* dw_partial;     // (nblocks, R0, M) fp32
-  float* dW;             // (R0, M) fp32
+  float* dW;             // (R0, M) fp32 or NULL: dw_partial is what the caller wants, and
+  void *dtok, *dtail;    // the bias gradients in io dtype, (tokens, H) rows dtok_stride apart, (2, tokens, 2G), or NULL,
+  long dtok_stride;
+  float* bias_partial;   // and the first R0 summed over a workgroup's tokens, (nblocks, R0)
   int nblocks;
 };
 

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
   constexpr int KS = 128 / (BF ? 2 : 4);   // columns of a step: 128 bytes of a gradient row
   typedef typename std::conditional<BF, uint16_t, float>::type T;
   typedef typename std::conditional<BF, uint2, f4>::type T4;
-  __shared__ float wred[4][16 * PG_M];
+  __shared__ float wred[4][16 * PG_M], bred[4][16];
   // FULLK, each wave's own: a step's gradient rows and what goes with them (raw dt, reversed-order gradients; a row more for the lanes that have
   // none), its block of dist, the weights, and two tiles of effective gradients [row][k] in turn.
   __shared__ __align__(16) unsigned char srow[FULLK ? 4 : 1][2][FULLK ? (PG_MAXR0 + 1) * PG_LDR : 16];
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
   };
   // one block of 16 k, operands already in registers (a / ab / rw2 / ww2: layout 2; x*, raw1, w1: layout 1)
   f4 accW = zero4;
-  float bs = 0.0f, bsb = 0.0f;
+  float bs = 0.0f, bsb = 0.0f, bsum = 0.0f;
   auto block = [&](f4 a, f4 ab, f4 rw2, f4 ww2, const float (&dv)[4], const float (&x)[3], const float (&xb)[3],
                    const float (&raw1)[3], float w1, T* ddst, float* dwdst, bool in_k) {
     if constexpr (HASW) {
@@ -531,13 +531,29 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
       p.dbias[t * R + i] = bs;
       if (p.has_back && i >= p.H) p.dbias[t * R + R0 + (i - p.H)] = bsb;
     }
+    if (p.dtail) {   // uniform
+      bsum += bs;
+      auto io = [](float v) -> T {
+        if constexpr (BF) return f_to_bf16(v);
+        else return v;
+      };
+      if (q == 0 && i < p.H) ((T*)p.dtok)[t * p.dtok_stride + i] = io(bs);
+      if (q == 0 && i >= p.H && i < R0) {
+        T* to = (T*)p.dtail + t * (2 * p.G) + (i - p.H);
+        to[0] = io(bs);
+        to[p.tokens * (2 * p.G)] = io(bsb);
+      }
+    }
   }
   // dW partial of the workgroup: the four waves in order.  Lane (m, q) holds rows 4q .. 4q + 3 of column m.
 #pragma unroll
   for (int v = 0; v < 4; ++v) wred[wave][(4 * q + v) * PG_M + i] = accW[v];
+  if (q == 0) bred[wave][i] = bsum;
   __syncthreads();
   for (int e = threadIdx.x; e < R0 * PG_M; e += NTHREADS)
     p.dw_partial[(long)blockIdx.x * R0 * PG_M + e] = (wred[0][e] + wred[1][e]) + (wred[2][e] + wred[3][e]);
+  const int r = threadIdx.x;
+  if (p.dtail && r < R0) p.bias_partial[(long)blockIdx.x * R0 + r] = (bred[0][r] + bred[1][r]) + (bred[2][r] + bred[3][r]);
 }
 
 // dW = fixed-order sum of the per-workgroup partials: one workgroup per entry of dW; the workgroups after those sum
@@ -646,7 +662,7 @@ int launch_pgen_bwd(const PGenP& p, hipStream_t st) {
     else pgen_bwd_launch<false, false>(p, st);
   }
   int e = (int)hipGetLastError();
-  if (e) return e;
+  if (e || !p.dW) return e;
   const int R = R0 + (p.has_back ? 2 * p.G : 0);
   hipLaunchKernelGGL(k_pgen_dw, dim3(R0 * PG_M + (p.dbias_sum ? R : 0)), dim3(NTHREADS), 0, st, p);
   return (int)hipGetLastError();

@@ -407,7 +407,7 @@ int launch_rmsnorm_bwd(const NormP& p, hipStream_t st) {
   if (norm_fast_ok(p)) NORM_FAST(k_rmsnorm_bwd_fast, dim3(p.nblocks), dim3(64));
   else hipLaunchKernelGGL(k_rmsnorm_bwd, dim3(p.nblocks), dim3(64), (size_t)(p.b ? 2 : 1) * p.ncols * sizeof(float), st, p);
   int e = (int)hipGetLastError();
-  if (e) return e;
+  if (e || !p.dw) return e;
   hipLaunchKernelGGL(k_rmsnorm_dw, dim3((p.ncols + 7) / 8), dim3(NTHREADS), 0, st, p, p.dw_partial, p.dw);
   if (p.b) hipLaunchKernelGGL(k_rmsnorm_dw, dim3((p.ncols + 7) / 8), dim3(NTHREADS), 0, st, p, p.db_partial, p.db);
   return (int)hipGetLastError();

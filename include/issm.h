@@ -290,6 +290,8 @@ typedef struct issm_norm_args {
 int issm_rmsnorm_bwd_blocks(int64_t rows);
 int issm_gated_rmsnorm_fwd(const issm_norm_args* args);
 int issm_gated_rmsnorm_bwd(const issm_norm_args* args);
+/* issm_gated_rmsnorm_bwd without its last sum: dw_partial keeps (issm_rmsnorm_bwd_blocks, ncols), dw is not written (no bias). */
+int issm_gated_rmsnorm_bwd_part(const issm_norm_args* args);
 
 /* issm_gated_rmsnorm_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and the same
@@ -353,6 +355,18 @@ typedef struct issm_pgen_args {
   const float* tok_add; /* (H) fp32 */
   const void* tail;     /* (has_back ? 2 : 1, tokens, 2G) */
 } issm_pgen_args;
+
+/* The backward for a caller that takes the sums over the tokens with other sums later (issm_layer_grads): dw_partial has room for
+ * issm_param_gen_bwd_blocks(tokens) * R0 * (M + 1) floats and keeps the workgroups' parts, (blocks, R0, M) of dW and then (blocks, R0) of the
+ * forward-order pair's bias gradients; dW and dbias_sum are not written and may be NULL.  The bias gradients go to where the producers'
+ * backwards read them, in `dtype`: of dt to dtok[t * dtok_stride + h], of B and C to dtail[0][t][0 .. 2G), of the reversed pair to dtail[1][t]
+ * (has_back is required). */
+typedef struct issm_pgen_producers {
+  void* dtok;
+  int64_t dtok_stride;
+  void* dtail; /* (2, tokens, 2G) */
+} issm_pgen_producers;
+int issm_param_gen_bwd_part(const issm_pgen_args* args, const issm_pgen_producers* producers);
 
 /* The small parameters of a layer as its kernels read them: ISSM_LAYER_ARRAYS arrays src[i] of n[i] values of dtype[i]
  * (issm_dtype), converted to fp32 and laid one behind the other in out, and A[h][k] = -exp(src[a_log][h]) for h < n[a_log],
@@ -418,6 +432,8 @@ typedef struct issm_dwconv_args {
 } issm_dwconv_args;
 
 int issm_dwconv_partial_rows(int32_t batch, int32_t seqlen);
+/* issm_dwconv_silu_bwd without its last sums: a chained pair's partial keeps (issm_dwconv_partial_rows, 2, 8, C); dw and dbias are not written. */
+int issm_dwconv_silu_bwd_part(const issm_dwconv_args* args);
 int issm_dwconv_silu_fwd(const issm_dwconv_args* args);
 int issm_dwconv_silu_bwd(const issm_dwconv_args* args);
 /* issm_dwconv_silu_fwd of a chained pair and issm_param_gen_fwd_only behind it, in one launch on the convolutions' stream,
@@ -517,6 +533,25 @@ typedef struct issm_transpose_args {
 } issm_transpose_args;
 
 int issm_transpose_states(const issm_transpose_args* args);
+
+/* The gradients of a layer's small parameters in one launch, each a sum over the parts that the backwards left, one behind the other in `dtype`:
+ * for either convolution its weight (C, 7) and bias (C); the rows of dt_proj (H, 16) and bc_proj (2 G, 16); dt_bias (H); A_log (H), A[h][0] *
+ * sum_k dA[h][k]; D (nD); the norm's weight (d_inner).  No rows of a part: zero.  The order of each sum depends on the sizes alone.
+ * states, if not NULL: issm_transpose_states in the same launch, on this call's stream (in_dtype ISSM_F32, in1 NULL). */
+typedef struct issm_layer_grads_args {
+  const float* conv; /* issm_dwconv_silu_bwd_part's */
+  const float* gen;  /* issm_param_gen_bwd_part's */
+  const float* norm; /* issm_gated_rmsnorm_bwd_part's */
+  int32_t conv_rows, gen_rows, norm_rows;
+  int32_t C, H, G, d_inner, K;
+  const float *dA, *A; /* (H, K) */
+  const float* dD;
+  int32_t nD;
+  int32_t dtype;
+  void* out;
+  void* stream;
+} issm_layer_grads_args;
+int issm_layer_grads(const issm_layer_grads_args* args, const issm_transpose_args* states);
 
 /* ---- box-to-point distance encoding and locality weight ----------------------------------
  * BoxDistFun.forward (models/dest_module.py:174-195) and ISSMDecoderLayer.local_weight (:240-249), the two
