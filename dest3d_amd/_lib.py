@@ -31,7 +31,7 @@ EXPORTS = [
     "issm_param_gen_bwd_blocks", "issm_param_gen_fwd", "issm_param_gen_bwd",
     "issm_dwconv_partial_rows", "issm_dwconv_silu_fwd", "issm_dwconv_silu_bwd",
     "issm_box_dist_bwd_scratch_bytes", "issm_box_dist_fwd", "issm_box_dist_bwd",
-    "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states", "issm_layer_params", "issm_linear_fwd", "issm_linear_dx", "issm_linear_dw", "issm_linear_dw_scratch_bytes", "issm_layer_out", "issm_layer_in",
+    "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states", "issm_layer_params", "issm_linear_fwd", "issm_linear_dx", "issm_linear_dw", "issm_linear_dw_pair", "issm_linear_dw_scratch_bytes", "issm_layer_out", "issm_layer_in",
     "issm_param_gen_fwd_only", "issm_conv_param_gen_fwd", "issm_layer_end", "issm_box_dist_fwd_only",
     "issm_box_table",
     "issm_pn2_furthest_point_sampling", "issm_pn2_ball_query", "issm_pn2_group_points", "issm_pn2_group_points_grad",

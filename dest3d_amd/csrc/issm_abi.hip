@@ -47,7 +47,7 @@ bool linear_tile_takes(long tokens, int in, int out, bool nn);
 int launch_linear_tile(LinearTileP& p, int njobs, bool nn, hipStream_t st);
 int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
-int launch_linear_dw(LinearDwP& p, hipStream_t st);
+int launch_linear_dw(LinearDwJobs& j, int njobs, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
 int launch_layer_end(LayerOutP& p, LinearP& q, hipStream_t st);
 int launch_box_table(const BoxTableP& p, hipStream_t st);
@@ -1017,7 +1017,7 @@ size_t issm_linear_dw_scratch_bytes(int64_t tokens, int32_t in, int32_t out) {
   return linear_dw_sizes(tokens, in, out) ? (size_t)linear_dw_splits(tokens, in, out) * in * out * sizeof(float) : 0;
 }
 
-int issm_linear_dw(const issm_linear_dw_args* a) {
+static int linear_dw_params(const issm_linear_dw_args* a, LinearDwP& p) {
   if (!a) return fail(ISSM_E_NULL, "linear_dw: args is NULL");
   if (a->dtype != ISSM_BF16) return fail(ISSM_E_DTYPE, "linear_dw: dtype %d (bf16 only)", a->dtype);
   if (!linear_dw_sizes(a->tokens, a->in, a->out)) return fail(ISSM_E_SHAPE, "linear_dw: %lld tokens, (%d, %d)", (long long)a->tokens, a->out, a->in);
@@ -1026,11 +1026,23 @@ int issm_linear_dw(const issm_linear_dw_args* a) {
   if (a->scratch_bytes < issm_linear_dw_scratch_bytes(a->tokens, a->in, a->out)) return fail(ISSM_E_WORKSPACE, "linear_dw: scratch too small");
   if ((uintptr_t)a->scratch & 15) return fail(ISSM_E_STRIDE, "linear_dw: scratch must be aligned to 16 bytes");
   if (((uintptr_t)a->dy | (uintptr_t)a->x | (uintptr_t)a->dw) & 1) return fail(ISSM_E_STRIDE, "linear_dw: operands must be aligned to their elements");
-  LinearDwP p{};
   p.dy = (const uint16_t*)a->dy; p.x = (const uint16_t*)a->x; p.dw = (uint16_t*)a->dw; p.partial = (float*)a->scratch;
   p.tokens = (int)a->tokens; p.in = a->in; p.out = a->out;
   p.splits = linear_dw_splits(a->tokens, a->in, a->out);
-  return launched(launch_linear_dw(p, (hipStream_t)a->stream), "linear_dw");
+  return ISSM_OK;
+}
+
+int issm_linear_dw(const issm_linear_dw_args* a) {
+  LinearDwJobs j{};
+  if (const int rc = linear_dw_params(a, j.job[0])) return rc;
+  return launched(launch_linear_dw(j, 1, (hipStream_t)a->stream), "linear_dw");
+}
+
+int issm_linear_dw_pair(const issm_linear_dw_args* a, const issm_linear_dw_args* b) {
+  LinearDwJobs j{};
+  int rc = linear_dw_params(a, j.job[0]);
+  if (rc || (rc = linear_dw_params(b, j.job[1]))) return rc;
+  return launched(launch_linear_dw(j, 2, (hipStream_t)a->stream), "linear_dw_pair");
 }
 
 static int layer_out_params(const issm_layer_out_args* a, LayerOutP& p, bool norms_out) {

@@ -248,6 +248,10 @@ struct LinearDwP {
   uint16_t* dw;             // (out, in)
   int tokens, in, out, splits, btiles, per;
 };
+struct LinearDwJobs {
+  LinearDwP job[2];
+  int blocks0, sums0;       // workgroups of the first, of its sums
+};
 // parameters of the kernel behind the scan (layer_out.hip)
 struct LayerOutP {
   const uint16_t *y0, *y1, *z, *kw, *qw, *qb;   // qw, qb may be NULL

@@ -37,10 +37,13 @@ __device__ __forceinline__ void pair_rows(const unsigned (&w)[8], bf8& lo, bf8& 
   hi = __builtin_bit_cast(bf8, b);
 }
 
-__global__ __launch_bounds__(NTHREADS, 2) void k_linear_dw(LinearDwP p) {
+__global__ __launch_bounds__(NTHREADS, 2) void k_linear_dw(LinearDwJobs jobs) {
   __shared__ f4 red[2][DW_FA * DW_FB][64];
+  const bool second = (int)blockIdx.x >= jobs.blocks0;
+  const LinearDwP& p = jobs.job[second ? 1 : 0];
+  const int bid = (int)blockIdx.x - (second ? jobs.blocks0 : 0);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
-  const int part = (int)blockIdx.x % p.splits, tile = (int)blockIdx.x / p.splits;
+  const int part = bid % p.splits, tile = bid / p.splits;
   const int a0 = (tile / p.btiles) * DW_TA, b0 = (tile % p.btiles) * DW_TB;
   const int ca = min(a0 + DW_FA * i, p.out - DW_FA), cb = min(b0 + DW_FB * i, p.in - DW_FB);
   const int per = p.per, t0 = min((part * 4 + w) * per, p.tokens), t1 = min(t0 + per, p.tokens);
@@ -136,8 +139,10 @@ __global__ __launch_bounds__(NTHREADS, 2) void k_linear_dw(LinearDwP p) {
     }
 }
 
-__global__ __launch_bounds__(NTHREADS) void k_linear_dw_sum(LinearDwP p) {
-  const long n = (long)p.out * p.in, e = ((long)blockIdx.x * NTHREADS + threadIdx.x) * 2;
+__global__ __launch_bounds__(NTHREADS) void k_linear_dw_sum(LinearDwJobs jobs) {
+  const bool second = (int)blockIdx.x >= jobs.sums0;
+  const LinearDwP& p = jobs.job[second ? 1 : 0];
+  const long n = (long)p.out * p.in, e = ((long)((int)blockIdx.x - (second ? jobs.sums0 : 0)) * NTHREADS + threadIdx.x) * 2;
   if (e >= n) return;
   const bool two = e + 1 < n;
   float x = 0.0f, y = 0.0f;
@@ -160,15 +165,21 @@ int linear_dw_splits(long tokens, int in, int out) {
   return (int)(n >= 8 ? n & ~7L : n);
 }
 
-int launch_linear_dw(LinearDwP& p, hipStream_t st) {
-  const int atiles = (p.out + DW_TA - 1) / DW_TA;
-  p.btiles = (p.in + DW_TB - 1) / DW_TB;
-  p.per = (int)((((long)p.tokens + p.splits * 4 - 1) / (p.splits * 4) + 31) / 32 * 32);
-  const long blocks = (long)atiles * p.btiles * p.splits, sums = ((long)p.out * p.in + 2 * NTHREADS - 1) / (2 * NTHREADS);
-  if (blocks > 0x7fffffff || sums > 0x7fffffff) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_linear_dw, dim3((unsigned)blocks), dim3(NTHREADS), 0, st, p);
+int launch_linear_dw(LinearDwJobs& j, int njobs, hipStream_t st) {
+  long blocks[2] = {0, 0}, sums[2] = {0, 0};
+  for (int k = 0; k < njobs; ++k) {
+    LinearDwP& p = j.job[k];
+    p.btiles = (p.in + DW_TB - 1) / DW_TB;
+    p.per = (int)((((long)p.tokens + p.splits * 4 - 1) / (p.splits * 4) + 31) / 32 * 32);
+    blocks[k] = (long)((p.out + DW_TA - 1) / DW_TA) * p.btiles * p.splits;
+    sums[k] = ((long)p.out * p.in + 2 * NTHREADS - 1) / (2 * NTHREADS);
+  }
+  if (blocks[0] + blocks[1] > 0x7fffffff || sums[0] + sums[1] > 0x7fffffff) return (int)hipErrorInvalidValue;
+  j.blocks0 = (int)blocks[0];
+  j.sums0 = (int)sums[0];
+  hipLaunchKernelGGL(k_linear_dw, dim3((unsigned)(blocks[0] + blocks[1])), dim3(NTHREADS), 0, st, j);
   if (hipError_t e = hipGetLastError()) return (int)e;
-  hipLaunchKernelGGL(k_linear_dw_sum, dim3((unsigned)sums), dim3(NTHREADS), 0, st, p);
+  hipLaunchKernelGGL(k_linear_dw_sum, dim3((unsigned)(sums[0] + sums[1])), dim3(NTHREADS), 0, st, j);
   return (int)hipGetLastError();
 }
 

@@ -485,6 +485,8 @@ typedef struct issm_linear_dw_args {
 
 size_t issm_linear_dw_scratch_bytes(int64_t tokens, int32_t in, int32_t out);
 int issm_linear_dw(const issm_linear_dw_args* args);
+/* Two of them in one launch and its sums in another, on a's stream; neither may read what the other writes. */
+int issm_linear_dw_pair(const issm_linear_dw_args* a, const issm_linear_dw_args* b);
 
 /* ---- behind the scan of a layer, without a gradient ------------------------------------------
  * models/dest_module.py:574-585 up to the output projections, ISSM_BF16, one launch:

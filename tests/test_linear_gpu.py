@@ -211,6 +211,58 @@ def test_weight_gradient_at_its_remainders(tokens, nin, nout):
         setattr(a, field, was)
 
 
+@pytest.mark.parametrize("shapes", [[(1000, 288, 586), (64, 288, 288)], [(33, 7, 5), (8200, 97, 130)]])
+def test_two_weight_gradients_in_a_launch(shapes):
+    """The same bits as one at a time."""
+    lib = L.load()
+    args, kept = [], []
+    for t, nin, nout in shapes:
+        x, dy = torch.randn(t, nin).bfloat16().cuda(), torch.randn(t, nout).bfloat16().cuda()
+        alone, pair = (torch.full((nout, nin), 3.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        size = lib.issm_linear_dw_scratch_bytes(t, nin, nout)
+        scratch = torch.full((size // 4,), float("nan"), device="cuda")
+        a = DwArgs(dy.data_ptr(), x.data_ptr(), alone.data_ptr(), t, nin, nout, L.ISSM_BF16, scratch.data_ptr(), size,
+                   L.current_stream_ptr(torch.device("cuda", 0)))
+        assert lib.issm_linear_dw(C.byref(a)) == 0
+        a.dw = pair.data_ptr()
+        args.append(a)
+        kept.append((x, dy, scratch, alone, pair))
+    assert lib.issm_linear_dw_pair(C.byref(args[0]), C.byref(args[1])) == 0
+    torch.cuda.synchronize()
+    for *_, alone, pair in kept:
+        assert torch.equal(alone, pair)
+    args[1].bytes -= 1
+    assert lib.issm_linear_dw_pair(C.byref(args[0]), C.byref(args[1])) != 0
+    assert lib.issm_linear_dw_pair(C.byref(args[0]), None) != 0
+
+
+@pytest.mark.parametrize("K", [40, 130])
+def test_projections_beside_each_other(K):
+    """An output that no loss reads gives its projection no gradient and leaves the others' as they are; frozen sides stay without one."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(7)
+    B, Ln, D = 2, 70, 288
+    layer = MultiHeadISSMScan(d_model=D, d_state=K, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    key, query, dist, dkey, dquery = bf(B, Ln, D), bf(B, K, D), bf(B, Ln, K, 16), bf(B, Ln, D), bf(B, K, D)
+    grads = lambda: {n: p.grad for n, p in layer.named_parameters() if p.grad is not None}
+    out = layer(key, query, dist, None, None)
+    torch.autograd.backward(out[:1], [dkey])
+    alone = grads()
+    assert "out_key_proj.weight" in alone and "out_query_proj.weight" not in alone and "query_norm.weight" not in alone
+    layer.zero_grad(set_to_none=True)
+    out = layer(key, query, dist, None, None)
+    torch.autograd.backward(out, [dkey, torch.zeros_like(dquery)])
+    both = grads()
+    for n, g in alone.items():
+        assert torch.equal(g, both[n]), n
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    layer.out_query_proj.weight.requires_grad_()
+    out = layer(key, query, dist, None, None)
+    assert not out[0].requires_grad and out[1].requires_grad
+
+
 @pytest.mark.parametrize("form", ["plain", "rows apart", "expanded gradient", "wide"])
 def test_weight_gradient_of_every_form(form):
     from dest3d_amd.scan_module import _LinearTokens
