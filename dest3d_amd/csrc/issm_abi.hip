@@ -46,6 +46,7 @@ int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 bool linear_tile_takes(long tokens, int in, int out, bool nn);
 int launch_linear_tile(LinearTileP& p, int njobs, bool nn, hipStream_t st);
 int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st);
+int launch_layer_in_tile(LinearTileP& t, LinearP& p, const LayerParamsP& q, hipStream_t st);
 int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwJobs& j, int njobs, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
@@ -1005,6 +1006,11 @@ int issm_layer_in(const issm_linear_args* a, const issm_layer_params_args* b) {
   if (n == 0 || q.total == 0) {   // (nothing to join)
     if (n && (rc = issm_linear_fwd(a))) return rc;
     return q.total ? issm_layer_params(b) : ISSM_OK;
+  }
+  if (linear_in_tiles(p, 1)) {
+    LinearTileP t{};
+    t.job[0] = LinearTileJob{p.job[0].x, p.job[0].w, p.job[0].y, p.job[0].tokens, 32 * p.job[0].steps, p.job[0].out, 0};
+    return launched(launch_layer_in_tile(t, p, q, (hipStream_t)a->stream), "layer_in");
   }
   return launched(launch_linear(p, n, &q, (hipStream_t)a->stream), "layer_in");
 }

@@ -10,6 +10,7 @@
 // share.  1024 x 288 -> 586: 6.3 us (library 6.1), 288: 4.5 (5.1).  With more tokens the fragments' 64-byte pieces
 // of 16 rows a load are what it pays for, and staging tiles through LDS wins (linear_tile.hip): 8192 x 288 -> 586 21 us, in tiles 10.6.
 #include "layer_params.h"
+#include "linear_tile_dev.h"
 
 namespace issm {
 
@@ -97,6 +98,33 @@ __global__ __launch_bounds__(NTHREADS) void k_layer_in(LinearP p, LayerParamsP q
   const int bid = (int)blockIdx.x - (second ? p.blocks0 : 0);
   if (j.turn) linear_block<N, true>(j, bid);
   else linear_block<N, false>(j, bid);
+}
+
+// The same with the first product in tiles, where issm_linear_fwd takes them.  A layer without a gradient, us, scenes of 1024 tokens and 256
+// queries: 288 features, 1, 4 and 8 scenes 58.2 -> 57.8, 135 -> 129, 232 -> 223; 96, 16: 293 -> 288; 320, 3: 131 -> 113; 512, 2: 126 -> 107.
+template <int N>
+__global__ __launch_bounds__(NTHREADS) void k_layer_in_tile(LinearTileP t, LinearP p, LayerParamsP q) {
+  warm_first<sizeof(LinearTileP) + sizeof(LinearP) + sizeof(LayerParamsP)>();
+  const int wg = blockIdx.x;
+  if (wg >= p.blocks1) return layer_params_entry(q, (wg - p.blocks1) * NTHREADS + threadIdx.x);
+  if (wg < t.blocks0) return linear_tile<false>(t.job[0], xcd_remap(wg, t.blocks0));
+  const LinearJob& j = p.job[1];
+  if (j.turn) linear_block<N, true>(j, wg - t.blocks0);
+  else linear_block<N, false>(j, wg - t.blocks0);
+}
+
+int launch_layer_in_tile(LinearTileP& t, LinearP& p, const LayerParamsP& q, hipStream_t st) {
+  t.job[0].otiles = (t.job[0].out + LT_O - 1) / LT_O;
+  p.job[1].oblocks = (p.job[1].out + 31) / 32;
+  const long tiles = (long)((t.job[0].tokens + LT_T - 1) / LT_T) * t.job[0].otiles,
+             blocks = tiles + (long)((p.job[1].tokens + 63) / 64) * p.job[1].oblocks, params = ((long)q.total + q.H * q.K + NTHREADS - 1) / NTHREADS;
+  if (blocks + params > 0x7fffffff) return (int)hipErrorInvalidValue;
+  t.blocks0 = (int)tiles;
+  p.blocks1 = (int)blocks;
+  const dim3 grid((unsigned)(blocks + params)), block(NTHREADS);
+  if (p.job[1].steps % 9 == 0) hipLaunchKernelGGL(k_layer_in_tile<9>, grid, block, 0, st, t, p, q);
+  else hipLaunchKernelGGL(k_layer_in_tile<8>, grid, block, 0, st, t, p, q);
+  return (int)hipGetLastError();
 }
 
 int launch_linear(LinearP& p, int njobs, const LayerParamsP* q, hipStream_t st) {
