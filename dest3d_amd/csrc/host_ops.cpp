@@ -465,7 +465,9 @@ struct NormFn : public Function<NormFn> {
     Tensor dx = fresh(x2.sizes(), x2, x2.scalar_type()), dz;
     if (z2.defined()) dz = fresh(z2.sizes(), z2, z2.scalar_type());
     const int64_t cols = x2.size(1), nb = issm_rmsnorm_bwd_blocks(x2.size(0)), np = b.defined() ? 2 : 1;
-    Tensor part = fresh({np, nb, cols}, x2, at::kFloat), dwb = fresh({np, cols}, x2, at::kFloat);
+    // the gradients in the parameters' type where that is one that the kernels write
+    const at::ScalarType wt = in->weight.type, type = is_kernel_type(wt) && (np == 1 || in->bias.type == wt) ? wt : at::kFloat;
+    Tensor part = fresh({np, nb, cols}, x2, at::kFloat), dwb = fresh({np, cols}, x2, type);
     issm_norm_args a = norm_args(x2, z2, w, b, in->eps, in->group, in->before_gate, !rms);
     a.rstd = data<float>(stats);
     if (!rms) a.mean = data<float>(stats) + stats.size(1);
@@ -478,12 +480,12 @@ struct NormFn : public Function<NormFn> {
       a.dz_row_stride = dz.stride(0);
     }
     a.dw_partial = data<float>(part);
-    a.dw = data<float>(dwb);
+    a.dw = (float*)data(dwb);
     if (np == 2) {
       a.db_partial = data<float>(part) + nb * cols;
-      a.db = data<float>(dwb) + cols;
+      a.db = (float*)(data<char>(dwb) + cols * dwb.element_size());
     }
-    check(issm_gated_rmsnorm_bwd(&a), "issm_gated_rmsnorm_bwd");
+    check(issm_gated_rmsnorm_bwd_as(&a, code(type)), "issm_gated_rmsnorm_bwd_as");
     variable_list out(8);
     out[0] = cast(dx.view(in->x.sizes), in->x.type);
     out[1] = cast(dwb.select(0, 0), in->weight.type);

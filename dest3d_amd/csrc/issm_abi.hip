@@ -573,7 +573,7 @@ static int norm_params(const issm_norm_args* a, NormP* p, bool bwd, bool part = 
   p->x = a->x; p->z = a->z; p->w = a->w; p->xs = a->x_row_stride; p->zs = a->z_row_stride;
   p->y = a->y; p->ys = a->y_row_stride; p->rstd = a->rstd;
   p->dy = a->dy; p->dys = a->dy_row_stride; p->dx = a->dx; p->dz = a->dz; p->dxs = a->dx_row_stride;
-  p->dzs = a->dz_row_stride; p->dw_partial = a->dw_partial; p->dw = a->dw;
+  p->dzs = a->dz_row_stride; p->dw_partial = a->dw_partial; p->dw = a->dw; p->dw_dt = ISSM_F32;
   p->nblocks = issm_rmsnorm_bwd_blocks(a->rows);
   p->ln = a->layer_norm ? 1 : 0; p->b = a->bias; p->mean = a->mean; p->db_partial = a->db_partial; p->db = a->db;
   return ISSM_OK;
@@ -593,6 +593,16 @@ int issm_gated_rmsnorm_bwd(const issm_norm_args* a) {
   if (rc) return rc;
   norm_scratch_warm((hipStream_t)a->stream);
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd");
+}
+
+int issm_gated_rmsnorm_bwd_as(const issm_norm_args* a, int32_t grad_dtype) {
+  NormP p;
+  int rc = norm_params(a, &p, true);
+  if (rc) return rc;
+  if ((unsigned)grad_dtype > 1u) return fail(ISSM_E_DTYPE, "rmsnorm: unknown dtype");
+  norm_scratch_warm((hipStream_t)a->stream);
+  p.dw_dt = grad_dtype;
+  return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_as");
 }
 
 int issm_gated_rmsnorm_bwd_part(const issm_norm_args* a) {

@@ -123,13 +123,14 @@ struct NormP {
   void *dx, *dz;
   long dxs, dzs;
   float* dw_partial;
-  float* dw;
+  void* dw;         // (ncols) of dw_dt, as db
+  int dw_dt;
   int nblocks;
   int ln;           // LayerNorm statistics (mean subtracted) instead of RMS
   const void* b;    // bias in the weight's dtype, or null
   float* mean;
   float* db_partial;
-  float* db;
+  void* db;
 };
 
 // parameters of the serialization-code kernel (hilbert.hip)

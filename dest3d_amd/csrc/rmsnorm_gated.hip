@@ -348,10 +348,12 @@ __global__ __launch_bounds__(64) void k_rmsnorm_bwd(NormP p) {
 
 // dw[c] = sum over the per-block partials, in a fixed order: block = 8 columns x 32 row groups, row group g adds
 // partials g, g+32, ... with two independent accumulators, then the 32 group sums are combined in order.
-__global__ __launch_bounds__(NTHREADS) void k_rmsnorm_dw(NormP p, const float* __restrict__ partial,
-                                                         float* __restrict__ out) {
+// db behind dw, in the same launch; both in the type that the caller wants of them (bf16 weights: their conversion was a launch of its own).
+__global__ __launch_bounds__(NTHREADS) void k_rmsnorm_dw(NormP p) {
   __shared__ float red[NTHREADS];
-  const int c = blockIdx.x * 8 + (threadIdx.x & 7), g = threadIdx.x >> 3;
+  const int per = (p.ncols + 7) / 8, of_bias = (int)blockIdx.x >= per;
+  const float* __restrict__ partial = of_bias ? p.db_partial : p.dw_partial;
+  const int c = ((int)blockIdx.x - (of_bias ? per : 0)) * 8 + (threadIdx.x & 7), g = threadIdx.x >> 3;
   float a0 = 0.0f, a1 = 0.0f;
   if (c < p.ncols) {
     int b = g;
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsnorm_dw(NormP p, const float* _
     float t = 0.0f;
 #pragma unroll
     for (int k = 0; k < 32; ++k) t += red[k * 8 + (threadIdx.x & 7)];
-    out[c] = t;
+    stv(of_bias ? p.db : p.dw, c, p.dw_dt, t);
   }
 }
 
@@ -408,8 +410,7 @@ int launch_rmsnorm_bwd(const NormP& p, hipStream_t st) {
   else hipLaunchKernelGGL(k_rmsnorm_bwd, dim3(p.nblocks), dim3(64), (size_t)(p.b ? 2 : 1) * p.ncols * sizeof(float), st, p);
   int e = (int)hipGetLastError();
   if (e || !p.dw) return e;
-  hipLaunchKernelGGL(k_rmsnorm_dw, dim3((p.ncols + 7) / 8), dim3(NTHREADS), 0, st, p, p.dw_partial, p.dw);
-  if (p.b) hipLaunchKernelGGL(k_rmsnorm_dw, dim3((p.ncols + 7) / 8), dim3(NTHREADS), 0, st, p, p.db_partial, p.db);
+  hipLaunchKernelGGL(k_rmsnorm_dw, dim3((p.ncols + 7) / 8 * (p.b ? 2 : 1)), dim3(NTHREADS), 0, st, p);
   return (int)hipGetLastError();
 }
 

@@ -290,6 +290,8 @@ typedef struct issm_norm_args {
 int issm_rmsnorm_bwd_blocks(int64_t rows);
 int issm_gated_rmsnorm_fwd(const issm_norm_args* args);
 int issm_gated_rmsnorm_bwd(const issm_norm_args* args);
+/* issm_gated_rmsnorm_bwd with dw and db in grad_dtype (issm_dtype): one rounding of the fp32 sums. */
+int issm_gated_rmsnorm_bwd_as(const issm_norm_args* args, int32_t grad_dtype);
 /* issm_gated_rmsnorm_bwd without its last sum: dw_partial keeps (issm_rmsnorm_bwd_blocks, ncols), dw is not written (no bias). */
 int issm_gated_rmsnorm_bwd_part(const issm_norm_args* args);
 

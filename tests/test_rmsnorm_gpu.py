@@ -193,3 +193,24 @@ def test_inputs_the_kernels_read_copies_of_may_change_before_the_backward():
             t.mul_(2.0)
     for a, c in zip(torch.autograd.grad(y, (x, w, b, z), dy), want):
         assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,use_b", [(1, 4, False), (70, 292, True), (2100, 37, True)])
+def test_parameter_gradients_in_the_parameters_type(rows, cols, use_b, wdtype):
+    """The sums over the rows, rounded once to the parameters' type."""
+    g = torch.Generator().manual_seed(rows)
+    x, dy = (torch.randn(rows, cols, generator=g).cuda() for _ in range(2))
+    w, b = (torch.randn(cols, generator=g).to(wdtype).cuda().requires_grad_() for _ in range(2))
+    from dest3d_amd.layernorm_gated import layernorm_fn, rmsnorm_fn
+    y = layernorm_fn(x, w, b, eps=1e-5) if use_b else rmsnorm_fn(x, w, None, eps=1e-5)
+    y.backward(dy)
+    xd, dyd = x.double(), dy.double()
+    if use_b:
+        xd = xd - xd.mean(-1, keepdim=True)
+    xhat = xd * (xd.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+    for grad, terms in ((w.grad, dyd * xhat), (b.grad, dyd)) if use_b else ((w.grad, dyd * xhat),):
+        assert grad.dtype == wdtype
+        # fp32 sums of terms that are right to a few 2^-22, one rounding
+        bound = torch.finfo(wdtype).eps / 2 * terms.sum(0).abs() + (rows + 16) * 2.0 ** -22 * terms.abs().sum(0) + 1e-7
+        assert ((grad.double() - terms.sum(0)).abs() <= bound).all()
