@@ -1024,7 +1024,7 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_param_gen_bwd_part(&a, &to), "issm_param_gen_bwd_part");
     }
     // 1'. the convolutions: gradients of (x, b-bias, c-bias) per branch
-    const int conv_rows = issm_dwconv_partial_rows((int)Bsz, (int)Ln);
+    const int conv_rows = issm_dwconv_part_rows((int)Bsz, (int)Ln);
     Tensor part = fresh({std::max(conv_rows, 1), 2, 8, Cc}, key, at::kFloat);
     {
       issm_dwconv_args a = conv_args(xbc);

@@ -76,7 +76,7 @@ int box_dist_bwd_workgroups(int B, int L, int K);
 long box_dist_bwd_scratch_bytes(int B, int L, int K, int D, int H, int W);
 int launch_box_dist_fwd(const BoxDistP& p, bool only, hipStream_t st);
 int launch_box_dist_bwd(const BoxDistP& p, hipStream_t st);
-int dwconv_partial_rows(int B, int L);
+int dwconv_partial_rows(int B, int L, bool chain);
 int launch_dwconv_fwd(const DwConvP& p, hipStream_t st);
 int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st);
 int launch_dwconv_bwd(const DwConvP& p, hipStream_t st);
@@ -798,7 +798,7 @@ static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool h
   p->dy[0] = a->dy[0]; p->dy[1] = a->nsets > 1 ? a->dy[1] : nullptr;
   if ((a->du_batch_stride || a->du_token_stride) && (a->du_token_stride < a->channels || a->du_batch_stride < 0))
     return fail(ISSM_E_STRIDE, "dwconv: du strides (%lld, %lld)", (long long)a->du_batch_stride, (long long)a->du_token_stride);
-  p->du = a->du; p->partial = a->partial; p->nrows = dwconv_partial_rows(a->batch, a->seqlen);
+  p->du = a->du; p->partial = a->partial; p->nrows = 0;
   p->du_ls = a->du_token_stride ? a->du_token_stride : a->channels;
   p->du_bs = a->du_token_stride ? a->du_batch_stride : (long)a->seqlen * a->channels;
   p->dw = a->dw; p->dbias = a->dbias;
@@ -806,7 +806,11 @@ static int dwconv_params(const issm_dwconv_args* a, DwConvP* p, bool bwd, bool h
 }
 
 int issm_dwconv_partial_rows(int32_t batch, int32_t seqlen) {
-  return (batch > 0 && seqlen > 0) ? dwconv_partial_rows(batch, seqlen) : 0;
+  return (batch > 0 && seqlen > 0) ? dwconv_partial_rows(batch, seqlen, false) : 0;   // (a chained pair's are no more)
+}
+
+int issm_dwconv_part_rows(int32_t batch, int32_t seqlen) {
+  return (batch > 0 && seqlen > 0) ? dwconv_partial_rows(batch, seqlen, true) : 0;
 }
 
 int issm_dwconv_silu_fwd(const issm_dwconv_args* a) {

@@ -55,8 +55,8 @@ __global__ __launch_bounds__(NTHREADS) void k_transpose_states(TrP p) {
 }
 
 // The gradients of a layer's small parameters from what the backwards left of them (issm_layer_grads), and the queries' gradient turned, in
-// one launch.  A few thousand results from 23 MB at most: each kind's workgroups are a few round trips to memory, and together they take the time of
-// the longest: 12.3 us at 8 x 1024 tokens, 288 features and 256 queries, where the three sums (5.3, 7.1 and 7.4 us), A_log's sum and product, the
+// one launch.  A few thousand results from 10 MB at most: each kind's workgroups are a few round trips to memory, and together they take the time of
+// the longest: 8.7 us at 8 x 1024 tokens, 288 features and 256 queries, where the three sums (5.3, 7.1 and 7.4 us), A_log's sum and product, the
 // concatenation, the conversion and the transposition were eight launches and 43 us.
 //
 // Column `col` of src (rows, ncol), summed by NTHREADS / COLS threads that take every NTHREADS / COLS-th row; the sum in those of row 0.  The

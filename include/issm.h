@@ -434,7 +434,8 @@ typedef struct issm_dwconv_args {
 } issm_dwconv_args;
 
 int issm_dwconv_partial_rows(int32_t batch, int32_t seqlen);
-/* issm_dwconv_silu_bwd without its last sums: a chained pair's partial keeps (issm_dwconv_partial_rows, 2, 8, C); dw and dbias are not written. */
+/* issm_dwconv_silu_bwd without its last sums: a chained pair's partial keeps (issm_dwconv_part_rows, 2, 8, C); dw and dbias are not written. */
+int issm_dwconv_part_rows(int32_t batch, int32_t seqlen);
 int issm_dwconv_silu_bwd_part(const issm_dwconv_args* args);
 int issm_dwconv_silu_fwd(const issm_dwconv_args* args);
 int issm_dwconv_silu_bwd(const issm_dwconv_args* args);

@@ -198,3 +198,105 @@ def test_dwconv_split_outputs_equal_the_slices():
     y1, t1, du1, dw1, db1 = run(split)
     assert torch.equal(y1, y0[..., :split]) and torch.equal(t1, y0[..., split:])
     assert torch.equal(du1, du0) and torch.equal(dw1, dw0) and torch.equal(db1, db0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Ln,Cn,split,absent,far", [(2, 64, 34, 32, None, False), (1, 65, 97, 33, None, False), (2, 129, 32, 0, 0, False),
+                                                      (1, 63, 7, 5, 1, False), (3, 192, 70, 64, None, False), (1, 3, 40, 38, None, True)])
+def test_chain_backward_in_its_tiles(dtype, B, Ln, Cn, split, absent, far):
+    """Tiles of 64 tokens and of 32 channels on either side of the split, a set without a gradient, tokens 2^22 elements apart, NaN around
+    every tensor; the parts that issm_dwconv_silu_bwd_part leaves add up to the sums."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    from dest3d_amd import dwconv as D
+    lib = L.load()
+    g = torch.Generator().manual_seed(Ln + Cn)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    nan = lambda n: torch.full((n,), float("nan"), dtype=dtype, device="cuda")
+
+    def framed(t):   # the same values between NaN
+        t = t.to(dtype).cuda().contiguous()
+        return torch.cat([nan(640), t.flatten(), nan(640)])[640:-640].view(t.shape)
+    rows = (1 << 22) + 64 if far else Cn + 6
+    u = nan(B * Ln * rows).view(B, Ln, rows)[..., :Cn]
+    u.copy_(rnd(B, Ln, Cn))
+    w, b = (0.4 * rnd(2, Cn, 7)).cuda(), rnd(2, Cn).cuda()
+    pre, dy = framed(rnd(2, B, Ln, Cn)), [None if s == absent else rnd(B, Ln, Cn).to(dtype) for s in range(2)]
+    pieces = [[] if t is None else [framed(p) for p in ((t[..., :split], t[..., split:]) if split else (t,))] for t in dy]
+    du = torch.full((B, Ln, rows), 3.0, dtype=dtype, device="cuda")
+    nr = lib.issm_dwconv_part_rows(B, Ln)
+    assert 0 < nr <= lib.issm_dwconv_partial_rows(B, Ln)
+    part, dw, db = torch.full((nr + 1, 2, 8, Cn), 3.0, device="cuda"), torch.zeros(2, Cn, 7, device="cuda"), torch.zeros(2, Cn, device="cuda")
+    a = D._args(u, 2)
+    a.w, a.bias, a.pre, a.chain, a.split, a.partial = w.data_ptr(), b.data_ptr(), pre.data_ptr(), 1, split, part.data_ptr()
+    a.du, a.du_batch_stride, a.du_token_stride = du.data_ptr(), Ln * rows, rows
+    for s in range(2):
+        for field, t in zip((a.dy, a.dy_tail), pieces[s]):
+            field[s] = t.data_ptr()
+    L.check(lib.issm_dwconv_silu_bwd_part(C.byref(a)), "part")
+    torch.cuda.synchronize()
+    assert (part[nr] == 3.0).all() and (du[..., Cn:] == 3.0).all()
+    first = du.clone()
+    a.dw, a.dbias = dw.data_ptr(), db.data_ptr()
+    L.check(lib.issm_dwconv_silu_bwd(C.byref(a)), "bwd")
+    torch.cuda.synchronize()
+    assert torch.equal(first, du)
+    sums = part[:nr].double().sum(0)
+    close = lambda got, want, tol: ((got.double().cpu() - want.double().cpu()).norm() <= tol * want.double().norm().cpu() + 1e-30)
+    assert close(dw, sums[:, :7].transpose(1, 2), 1e-6) and close(db, sums[:, 7], 1e-6)
+    # fp64: dpre[1], what flows back through the second convolution, dpre[0]
+    p64, u64, w64 = pre.double().cpu(), u.double().cpu(), w.double().cpu()
+    silu_grad = lambda x: torch.sigmoid(x) * (1 + x * (1 - torch.sigmoid(x)))
+    d64 = [torch.zeros(B, Ln, Cn, dtype=torch.double) if t is None else t.double() for t in dy]
+    y0 = F.silu(p64[0]).to(dtype).double()
+
+    def back(d, wt, x):   # input and weight gradient of a depthwise convolution
+        x = x.clone().requires_grad_()
+        wt = wt.reshape(Cn, 1, 7).clone().requires_grad_()
+        F.conv1d(x.transpose(1, 2), wt, padding=3, groups=Cn).backward(d.transpose(1, 2))
+        return x.grad, wt.grad.reshape(Cn, 7)
+    e1 = d64[1] * silu_grad(p64[1])
+    through, gw1 = back(e1, w64[1], y0)
+    e0 = (d64[0] + through) * silu_grad(p64[0])
+    want, gw0 = back(e0, w64[0], u64)
+    assert close(du[..., :Cn], want, 1e-5 if dtype == torch.float32 else 3e-3)
+    assert close(dw, torch.stack([gw0, gw1]), 1e-5) and close(db, torch.stack([e0.sum((0, 1)), e1.sum((0, 1))]), 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,Ln,Cn,split", [(1, 16, 34, 32), (2, 17, 33, 0), (1, 35, 7, 5), (1, 3, 40, 38), (40, 65, 770, 768)])
+def test_chain_forward_in_its_tiles(dtype, B, Ln, Cn, split):
+    """Tiles of 16 and of 64 tokens and the rows too far apart for either (2^22 elements): the same bits, and nothing written beside them."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    from dest3d_amd import dwconv as D
+    lib = L.load()
+    g = torch.Generator().manual_seed(Ln + Cn)
+    near = torch.full((B, Ln, Cn + 6), float("nan"), dtype=dtype, device="cuda")[..., :Cn]
+    near.copy_(torch.randn(B, Ln, Cn, generator=g))
+    w, b = (0.4 * torch.randn(2, Cn, 7, generator=g)).cuda(), torch.randn(2, Cn, generator=g).cuda()
+
+    def run(u, seqs):
+        y = torch.full((2 * seqs * Ln * Cn + 1,), 3.0, dtype=dtype, device="cuda")
+        pre = torch.full((2 * seqs * Ln * Cn + 1,), 3.0, dtype=dtype, device="cuda")
+        a = D._args(u, 2)
+        a.w, a.bias, a.pre, a.chain, a.split = w.data_ptr(), b.data_ptr(), pre.data_ptr(), 1, split
+        a.y, a.y_tail = y.data_ptr(), y.data_ptr() + 2 * seqs * Ln * split * y.element_size()
+        L.check(lib.issm_dwconv_silu_fwd(C.byref(a)), "fwd")
+        torch.cuda.synchronize()
+        assert y[-1] == 3.0 and pre[-1] == 3.0
+        pieces = y[:-1].split([2 * seqs * Ln * split, 2 * seqs * Ln * (Cn - split)])
+        return torch.cat([t.view(2, seqs, Ln, -1) for t in pieces if t.numel()], -1), pre[:-1].view(2, seqs, Ln, Cn)
+    y, pre = run(near, B)
+    ref = _ref(near.double().cpu(), [w[0].double().cpu()], [b[0].double().cpu()])[0]
+    assert _rel(y[0], ref) <= (1e-5 if dtype == torch.float32 else 1e-2)
+    ref = _ref(y[0].double().cpu(), [w[1].double().cpu()], [b[1].double().cpu()])[0]
+    assert _rel(y[1], ref) <= (1e-5 if dtype == torch.float32 else 1e-2)
+    rows = 1 << 22
+    apart = torch.full((min(Ln, 36) * rows,), float("nan"), dtype=dtype, device="cuda").view(1, -1, rows)[..., :Cn]
+    apart.copy_(near[:1, :36])
+    if Ln <= 36:
+        far_y, far_pre = run(apart, 1)
+        assert torch.equal(far_y[:, 0], y[:, 0]) and torch.equal(far_pre[:, 0], pre[:, 0])
+    one_y, one_pre = run(near[-1:], 1)   # (of many sequences 64 tokens a tile, of one 16)
+    assert torch.equal(one_y[:, 0], y[:, -1]) and torch.equal(one_pre[:, 0], pre[:, -1])
