@@ -27,7 +27,7 @@ EXPORTS = [
     "issm_stage_state_passing_bwd", "issm_stage_bwd_states", "issm_bwd_walks", "issm_stage_bwd_chunk", "issm_bwd_chunk_redo_ints", "issm_stage_bwd_dx",
     "issm_stage_bwd_reduce",
     "issm_rmsnorm_bwd_blocks", "issm_gated_rmsnorm_fwd", "issm_gated_rmsnorm_bwd",
-    "issm_gated_rmsnorm_bwd_noalloc", "issm_gated_rmsnorm_bwd_part", "issm_gated_rmsnorm_bwd_as", "issm_param_gen_bwd_part", "issm_dwconv_silu_bwd_part", "issm_dwconv_part_rows", "issm_layer_grads",
+    "issm_gated_rmsnorm_bwd_noalloc", "issm_gated_rmsnorm_bwd_part", "issm_gated_rmsnorm_bwd_as", "issm_param_gen_bwd_part", "issm_dwconv_silu_bwd_part", "issm_dwconv_part_rows", "issm_layer_grads", "issm_layer_begin", "issm_layer_behind",
     "issm_param_gen_bwd_blocks", "issm_param_gen_fwd", "issm_param_gen_bwd",
     "issm_dwconv_partial_rows", "issm_dwconv_silu_fwd", "issm_dwconv_silu_bwd",
     "issm_box_dist_bwd_scratch_bytes", "issm_box_dist_fwd", "issm_box_dist_bwd",

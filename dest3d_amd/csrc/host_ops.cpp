@@ -762,11 +762,16 @@ variable_list linear_pair(Tensor x0, Tensor w0, Tensor x1, Tensor w1) {
 
 // ------------------------------------------------------------------------------- the chain between a layer's projections
 // (B, R, C) -> (B, C, R): alpha * (in0 + in1) in `type`; in1 may be undefined (issm_transpose_states)
-Tensor transpose_states(const Tensor& in0_, const Tensor& in1_, double alpha, at::ScalarType type) {
-  const at::ScalarType k = kernel_type(in0_.scalar_type());
-  const Tensor in0 = cast(in0_, k).contiguous(), in1 = in1_.defined() ? cast(in1_, k).contiguous() : in1_;
-  Tensor out = fresh({in0.size(0), in0.size(2), in0.size(1)}, in0, type);
+struct Turn {   // (its tensors kept while the arguments point to them)
+  Tensor in0, in1, out;
   issm_transpose_args a{};
+  Turn(const Tensor& in0_, const Tensor& in1_, double alpha, at::ScalarType type);
+};
+Turn::Turn(const Tensor& in0_, const Tensor& in1_, double alpha, at::ScalarType type) {
+  const at::ScalarType k = kernel_type(in0_.scalar_type());
+  in0 = cast(in0_, k).contiguous();
+  in1 = in1_.defined() ? cast(in1_, k).contiguous() : in1_;
+  out = fresh({in0.size(0), in0.size(2), in0.size(1)}, in0, type);
   a.batch = (int)in0.size(0);
   a.rows = (int)in0.size(1);
   a.cols = (int)in0.size(2);
@@ -777,8 +782,11 @@ Tensor transpose_states(const Tensor& in0_, const Tensor& in1_, double alpha, at
   a.out = data(out);
   a.alpha = (float)alpha;
   a.stream = stream_of(in0);
-  check(issm_transpose_states(&a), "issm_transpose_states");
-  return out;
+}
+Tensor transpose_states(const Tensor& in0, const Tensor& in1, double alpha, at::ScalarType type) {
+  const Turn t(in0, in1, alpha, type);
+  check(issm_transpose_states(&t.a), "issm_transpose_states");
+  return t.out;
 }
 
 constexpr int TAPS = 7;   // of the depthwise convolutions
@@ -849,7 +857,7 @@ struct CoreFn : public Function<CoreFn> {
     return off[NSMALL];
   }
   static void small_parameters(const std::array<const Tensor*, NSMALL>& arrays, int64_t K, float* flat, float* A, void* stream,
-                               const issm_linear_args* with = nullptr) {   // with: in the products' launch
+                               const issm_linear_args* with = nullptr, const issm_transpose_args* turn = nullptr) {   // with, turn: in their launch
     static_assert(NSMALL == ISSM_LAYER_ARRAYS, "one array per parameter");
     issm_layer_params_args a{};
     Tensor kept[NSMALL];
@@ -864,7 +872,7 @@ struct CoreFn : public Function<CoreFn> {
     a.out = flat;
     a.A = A;
     a.stream = stream;
-    check(with ? issm_layer_in(with, &a) : issm_layer_params(&a), "issm_layer_params");
+    check(with ? issm_layer_in(with, &a) : turn ? issm_layer_begin(&a, turn) : issm_layer_params(&a), "issm_layer_params");
   }
 
   // tensor inputs: zxbcdt, h0_lin, dist, weights, conv_w_f, conv_b_f, conv_w_b, conv_b_b, dt_w, bc_w, dt_bias, A_log, D, norm_w
@@ -893,7 +901,9 @@ struct CoreFn : public Function<CoreFn> {
     int64_t off[NSMALL + 1];
     const std::array<const Tensor*, NSMALL> arrays{&conv_w_f, &conv_w_b, &conv_b_f, &conv_b_b, &dt_w, &bc_w, &dt_bias, &A_log, &D};
     Tensor flat = fresh({offsets(arrays, off)}, zx, at::kFloat), A1 = fresh({H, K}, zx, at::kFloat);
-    small_parameters(arrays, K, data<float>(flat), data<float>(A1), stream_of(zx));
+    // (and the queries in the layout of the scan's initial states)
+    const Turn states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()));
+    small_parameters(arrays, K, data<float>(flat), data<float>(A1), stream_of(zx), nullptr, &states.a);
     float* const par = data<float>(flat);
     // 1. both depthwise convolutions + SiLU; the conv writes x and the B / C biases apart
     Tensor x = fresh({2, Bsz, Ln, H, P}, zx, k), tail = fresh({2, Bsz, Ln, 2 * G}, zx, k), pre = fresh({2, Bsz, Ln, Cc}, zx, k);
@@ -927,8 +937,7 @@ struct CoreFn : public Function<CoreFn> {
       check(issm_param_gen_fwd(&a), "issm_param_gen_fwd");
     }
     // 3. the bidirectional scan, queries as initial state
-    const Tensor h0 = transpose_states(h0_lin.reshape({Bsz, K, di}), Tensor(), 1.0, kernel_type(h0_lin.scalar_type()))
-                          .view({Bsz, H, P, K});
+    const Tensor h0 = states.out.view({Bsz, H, P, K});
     const Tensor xs[2] = {x.select(0, 0), x.select(0, 1)}, Bs[2] = {bc.select(0, 0), bc.select(0, 2)},
                  Cs[2] = {bc.select(0, 1), bc.select(0, 3)}, none[2];
     const Scan s = Scan::make(2, xs, dt, A1, Bs, Cs, D.dim() == 1 ? flat.narrow(0, off[D_], H) : D, none, Tensor(), h0,
@@ -936,19 +945,26 @@ struct CoreFn : public Function<CoreFn> {
     Scan::Out o = s.forward(true);
     // 4. gated RMSNorm (norm(x * silu(z))) of the two directions' average: the norm of s / 2 with eps is the norm of s with
     // 4 eps, so the sum goes in as it is and the halving never runs (nor its backward)
-    const Tensor key = at::add(o.y[0], o.y[1]).view({Bsz * Ln, di});
+    const bool together = di % 4 == 0 && di <= 1024;   // in one launch with the average of the final states
+    const Tensor key = together ? fresh({Bsz * Ln, di}, zx, k) : at::add(o.y[0], o.y[1]).view({Bsz * Ln, di});
     const Tensor z2 = z.as_strided({Bsz * Ln, di}, {zx.stride(1), 1});
     const Tensor nw = cast(norm_w, kernel_type(norm_w.scalar_type())).contiguous();
     Tensor key_n = fresh(key.sizes(), key, k), rstd = fresh({Bsz * Ln}, key, at::kFloat);
+    const Turn final(o.last[0].view({Bsz, di, K}), o.last[1].view({Bsz, di, K}), 0.5, kernel_type(h0_lin.scalar_type()));
     {
       issm_norm_args a = norm_args(key, z2, nw, Tensor(), 4.0 * eps, 0, false, false);
       a.y = data(key_n);
       a.y_row_stride = key_n.stride(0);
       a.rstd = data<float>(rstd);
-      check(issm_gated_rmsnorm_fwd(&a), "issm_gated_rmsnorm_fwd");
+      if (together) {
+        a.x = data(o.y[0]);
+        check(issm_layer_behind(&a, data(o.y[1]), data(key), &final.a), "issm_layer_behind");
+      } else {
+        check(issm_gated_rmsnorm_fwd(&a), "issm_gated_rmsnorm_fwd");
+        check(issm_transpose_states(&final.a), "issm_transpose_states");
+      }
     }
-    const Tensor last = transpose_states(o.last[0].view({Bsz, di, K}), o.last[1].view({Bsz, di, K}), 0.5,
-                                         kernel_type(h0_lin.scalar_type()));
+    const Tensor last = final.out;
     variable_list saved{xbc, pre, flat, d, wt, raw, key, z2, nw, rstd, A1, o.ws};
     s.push(saved);
     ctx->save_for_backward(std::move(saved));

@@ -41,6 +41,9 @@ int launch_rmsnorm_bwd(const NormP& p, hipStream_t st);
 int launch_hilbert_codes(const HilbertP& p, hipStream_t st);
 int launch_hilbert_order(const HilbertOrderP& p, hipStream_t st);
 int launch_transpose_states(const TrP& p, hipStream_t st);
+int launch_layer_begin(const LayerParamsP& p, const TrP& t, hipStream_t st);
+bool layer_behind_takes(const NormP& p);
+int launch_layer_behind(const NormP& p, const void* x2, void* sum, const TrP& t, hipStream_t st);
 int launch_layer_grads(LayerGradsP& p, const TrP& t, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 bool linear_tile_takes(long tokens, int in, int out, bool nn);
@@ -1134,6 +1137,28 @@ int issm_transpose_states(const issm_transpose_args* a) {
   const int rc = transpose_params(a, p);
   if (rc || p.B == 0) return rc;
   return launched(launch_transpose_states(p, (hipStream_t)a->stream), "transpose_states");
+}
+
+int issm_layer_begin(const issm_layer_params_args* a, const issm_transpose_args* b) {
+  LayerParamsP p;
+  TrP t{};
+  int rc = layer_params(a, p);
+  if (rc || (rc = transpose_params(b, t))) return rc;
+  if (b->in_dtype != b->out_dtype) return fail(ISSM_E_UNSUPPORTED, "layer_begin: states of one type");
+  if (p.total == 0 && t.B == 0) return ISSM_OK;
+  return launched(launch_layer_begin(p, t, (hipStream_t)a->stream), "layer_begin");
+}
+
+int issm_layer_behind(const issm_norm_args* a, const void* x2, void* sum, const issm_transpose_args* b) {
+  NormP p;
+  TrP t{};
+  int rc = norm_params(a, &p, false);
+  if (rc || (rc = transpose_params(b, t))) return rc;
+  if (!x2 || !sum) return fail(ISSM_E_NULL, "layer_behind: x2/sum is NULL");
+  if (b->in_dtype != ISSM_F32 || !layer_behind_takes(p) || p.xs != p.ncols)
+    return fail(ISSM_E_UNSUPPORTED, "layer_behind: one group of up to 1024 columns, a multiple of 4, in contiguous rows, no bias, fp32 states");
+  norm_scratch_warm((hipStream_t)a->stream);
+  return launched(launch_layer_behind(p, x2, sum, t, (hipStream_t)a->stream), "layer_behind");
 }
 
 int issm_layer_grads(const issm_layer_grads_args* a, const issm_transpose_args* b) {

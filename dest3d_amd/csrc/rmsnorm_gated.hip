@@ -8,7 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "issm_dev.h"
+#include "transpose_dev.h"
 
 namespace issm {
 
@@ -132,10 +132,11 @@ __device__ __forceinline__ f4 silu4(f4 z, f4& sg) {
 }
 
 // EXT: LayerNorm statistics and / or a bias (p.ln, p.b); the plain RMS form compiles without either.
-template <bool BF, int NV, bool EXT>
-__global__ __launch_bounds__(NTHREADS) void k_rmsnorm_fwd_fast(NormP p) {
+// x2: x is the sum of two, rounded as it is stored for the backward.
+template <bool BF, int NV, bool EXT, bool SUM>
+__device__ __forceinline__ void rmsnorm_fwd_rows(const NormP& p, int four, const void* x2, void* sum) {   // four: of the rows, a wave each
   const int lane = threadIdx.x & 63;
-  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long row = (long)four * 4 + (threadIdx.x >> 6);
   if (row >= p.rows) return;
   const int nvec = p.ncols >> 2;
   const int ax = al_of(p.x, p.xs, BF), az = al_of(p.z, p.zs, BF), ay = al_of(p.y, p.ys, BF);
@@ -149,6 +150,19 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsnorm_fwd_fast(NormP p) {
     const bool ok = vi < nvec;
     x[v] = ld4<BF>(p.x, row * p.xs + 4 * vi, ok, ax);
     gate[v] = ld4<BF>(zp, row * zs + 4 * vi, ok, az);
+  }
+  if constexpr (SUM) {
+    f4 other[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) other[v] = ld4<BF>(x2, row * p.xs + 4 * (lane + 64 * v), lane + 64 * v < nvec, ax);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      x[v] += other[v];
+      if constexpr (BF)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[v][i] = bf16_round(x[v][i]);
+      if (lane + 64 * v < nvec) st4<BF>(sum, row * p.xs + 4 * (lane + 64 * v), x[v], ax);
+    }
   }
   ldw<NV>(p.w, lane, nvec, p.wdt, wv);
   f4 bv[EXT ? NV : 1];
@@ -187,6 +201,18 @@ __global__ __launch_bounds__(NTHREADS) void k_rmsnorm_fwd_fast(NormP p) {
       st4<BF>(p.y, row * p.ys + 4 * vi, y, ay);
     }
   }
+}
+
+template <bool BF, int NV, bool EXT>
+__global__ __launch_bounds__(NTHREADS) void k_rmsnorm_fwd_fast(NormP p) { rmsnorm_fwd_rows<BF, NV, EXT, false>(p, blockIdx.x, nullptr, nullptr); }
+
+// What lies behind a layer's scan with gradients (issm_layer_behind): the norm of the two directions' sum and the average of their final states,
+// turned.  8 x 1024 tokens, 288 features, 256 queries, bf16: 10.3 us, as sum, norm and transposition 5.2 + 6.7 + 4.8.
+template <bool BF, int NV, bool OUT_BF>
+__global__ __launch_bounds__(NTHREADS) void k_layer_behind(NormP p, const void* x2, void* sum, TrP t, int tiles) {
+  __shared__ float tile[64][65];
+  if ((int)blockIdx.x >= tiles) return rmsnorm_fwd_rows<BF, NV, false, true>(p, blockIdx.x - tiles, x2, sum);
+  transpose_nth<false, OUT_BF>(t, blockIdx.x, tile);   // (first: a tile takes longer than four rows)
 }
 
 template <bool BF, int NV, bool EXT>
@@ -402,6 +428,20 @@ int launch_rmsnorm_fwd(const NormP& p, hipStream_t st) {
   }
   const long items = p.rows * p.ngroups;
   hipLaunchKernelGGL(k_rmsnorm_fwd, dim3((unsigned)((items + 3) / 4)), dim3(NTHREADS), 0, st, p);
+  return (int)hipGetLastError();
+}
+
+bool layer_behind_takes(const NormP& p) { return norm_fast_ok(p) && !p.ln && !p.b; }
+int launch_layer_behind(const NormP& p, const void* x2, void* sum, const TrP& t, hipStream_t st) {
+  const long tiles = transpose_tiles(t), blocks = tiles + (p.rows + 3) / 4;
+  if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NTHREADS), 0, st, p, x2, sum, t, (int)tiles); };
+  const int nv = (p.ncols / 4 + 63) / 64;
+  auto form = [&](auto one, auto two, auto four) { nv <= 1 ? go(one) : nv == 2 ? go(two) : go(four); };
+  if (p.dt && t.out_dt) form(&k_layer_behind<true, 1, true>, &k_layer_behind<true, 2, true>, &k_layer_behind<true, 4, true>);
+  else if (p.dt) form(&k_layer_behind<true, 1, false>, &k_layer_behind<true, 2, false>, &k_layer_behind<true, 4, false>);
+  else if (t.out_dt) form(&k_layer_behind<false, 1, true>, &k_layer_behind<false, 2, true>, &k_layer_behind<false, 4, true>);
+  else form(&k_layer_behind<false, 1, false>, &k_layer_behind<false, 2, false>, &k_layer_behind<false, 4, false>);
   return (int)hipGetLastError();
 }
 

@@ -5,48 +5,9 @@
 //   out[b][c][r] = alpha * (in0[b][r][c] + in1[b][r][c])        in (B, R, C), out (B, C, R), in1 optional.
 // As tensor ops each is a strided copy (uncoalesced on one side) plus separate add / scale / cast kernels; here a
 // 64 x 64 tile goes through LDS so that both sides move 64 consecutive elements per wave row.
-#include "issm_dev.h"
+#include "transpose_dev.h"
 
 namespace issm {
-
-template <bool IN_BF, bool OUT_BF>
-__device__ __forceinline__ void transpose_tile(const TrP& p, int c0, int r0, int b, float (&tile)[64][65]) {
-  const int lx = threadIdx.x & 63, ly = threadIdx.x >> 6;
-  const long base = (long)b * p.R * p.C;
-  // absent elements read the slab's first element and are not stored: no branch around the loads
-  float v[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = r0 + ly + 4 * i, c = c0 + lx;
-    const bool ok = r < p.R && c < p.C;
-    const long o = base + (ok ? (long)r * p.C + c : 0);
-    v[i] = IN_BF ? bf16_to_f(((const uint16_t*)p.in0)[o]) : ((const float*)p.in0)[o];
-  }
-  if (p.in1) {  // uniform; one branch around all sixteen loads
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = r0 + ly + 4 * i, c = c0 + lx;
-      const bool ok = r < p.R && c < p.C;
-      const long o = base + (ok ? (long)r * p.C + c : 0);
-      v[i] += IN_BF ? bf16_to_f(((const uint16_t*)p.in1)[o]) : ((const float*)p.in1)[o];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) v[i] *= p.alpha;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) tile[ly + 4 * i][lx] = v[i];
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int c = c0 + ly + 4 * i, r = r0 + lx;
-    if (c < p.C && r < p.R) {
-      const float a = tile[lx][ly + 4 * i];
-      const long o = base + (long)c * p.R + r;
-      if (OUT_BF) ((uint16_t*)p.out)[o] = f_to_bf16(a);
-      else ((float*)p.out)[o] = a;
-    }
-  }
-}
 
 template <bool IN_BF, bool OUT_BF>
 __global__ __launch_bounds__(NTHREADS) void k_transpose_states(TrP p) {
@@ -89,10 +50,7 @@ __global__ __launch_bounds__(NTHREADS) void k_layer_grads(LayerGradsP p, TrP t) 
   __shared__ float tile[64][65];
   float* const red = &tile[0][0];
   const int b = blockIdx.x, lane = threadIdx.x & 63;
-  if (b >= p.b_tr) {
-    const int cs = (t.C + 63) / 64, rs = (t.R + 63) / 64, u = b - p.b_tr;
-    return transpose_tile<false, OUT_BF>(t, u % cs * 64, u / cs % rs * 64, u / (cs * rs), tile);
-  }
+  if (b >= p.b_tr) return transpose_nth<false, OUT_BF>(t, b - p.b_tr, tile);
   const int conv = 16 * p.C, gen = 16 * p.R0;   // results of the convolutions and of the generation
   auto put = [&](int e, float v) { stv(p.out, e, p.bf16, v); };
   if (b < p.b_gen) {
@@ -133,7 +91,7 @@ int launch_layer_grads(LayerGradsP& p, const TrP& t, hipStream_t st) {
   p.b_A = p.b_norm + (p.di + 7) / 8;
   p.b_D = p.b_A + (p.H + 3) / 4;
   p.b_tr = p.b_D + (p.nD + NTHREADS - 1) / NTHREADS;
-  const long blocks = p.b_tr + (long)((t.C + 63) / 64) * ((t.R + 63) / 64) * t.B;
+  const long blocks = p.b_tr + transpose_tiles(t);
   if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
   if (t.out_dt) hipLaunchKernelGGL(k_layer_grads<true>, dim3((unsigned)blocks), dim3(NTHREADS), 0, st, p, t);
   else hipLaunchKernelGGL(k_layer_grads<false>, dim3((unsigned)blocks), dim3(NTHREADS), 0, st, p, t);

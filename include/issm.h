@@ -539,6 +539,15 @@ typedef struct issm_transpose_args {
 
 int issm_transpose_states(const issm_transpose_args* args);
 
+/* issm_layer_params and issm_transpose_states (in_dtype = out_dtype) in one launch, on the parameters' stream; neither may read what the other
+ * writes. */
+int issm_layer_begin(const issm_layer_params_args* params, const issm_transpose_args* states);
+
+/* The norm of a sum and the average of two states in one launch, on the norm's stream: issm_gated_rmsnorm_fwd of sum = x + x2 rounded to `dtype`
+ * (x, x2 and sum contiguous rows; no bias, no layer_norm, one group, ncols a multiple of 4 up to 1024), and issm_transpose_states (in_dtype
+ * ISSM_F32). */
+int issm_layer_behind(const issm_norm_args* norm, const void* x2, void* sum, const issm_transpose_args* states);
+
 /* The gradients of a layer's small parameters in one launch, each a sum over the parts that the backwards left, one behind the other in `dtype`:
  * for either convolution its weight (C, 7) and bias (C); the rows of dt_proj (H, 16) and bc_proj (2 G, 16); dt_bias (H); A_log (H), A[h][0] *
  * sum_k dA[h][k]; D (nD); the norm's weight (d_inner).  No rows of a part: zero.  The order of each sum depends on the sizes alone.

@@ -103,3 +103,66 @@ def test_parts_of_the_generation(dtype, tokens, K, H, G, weighted):
     to.stride = H - 1
     assert lib.issm_param_gen_bwd_part(C.byref(b), C.byref(to)) != 0
     assert lib.issm_param_gen_bwd_part(C.byref(b), None) != 0
+
+
+def _turn(src, other, alpha, out):
+    code = lambda t: L.ISSM_BF16 if t.dtype == torch.bfloat16 else L.ISSM_F32
+    t = L.TransposeArgs()
+    t.batch, t.rows, t.cols, t.in_dtype, t.out_dtype, t.alpha = *src.shape, code(src), code(out), alpha
+    t.in0, t.in1, t.out, t.stream = src.data_ptr(), None if other is None else other.data_ptr(), out.data_ptr(), L.current_stream_ptr(src.device)
+    return t
+
+
+@pytest.mark.parametrize("dtype,to", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("rows,cols,B,R,Cc", [(1, 4, 1, 1, 1), (5, 256, 2, 65, 64), (130, 288, 0, 3, 5), (7, 260, 1, 64, 130), (33, 1024, 3, 70, 33)])
+def test_behind_the_scan_with_gradients(dtype, to, rows, cols, B, R, Cc):
+    """The norm of a sum and the turned average in one launch: the bits of the sum, the norm and the transposition on their own."""
+    lib = L.load()
+    g = torch.Generator().manual_seed(rows + cols)
+    x, x2, z = (torch.randn(rows, cols, generator=g).to(dtype).cuda() for _ in range(3))
+    w = torch.randn(cols, generator=g).to(dtype).cuda()
+    s0, s1 = (torch.randn(B, R, Cc, generator=g).cuda() for _ in range(2))
+    full = lambda *s, dt=dtype: torch.full(s, 3.0, dtype=dt, device="cuda")
+    from dest3d_amd.layernorm_gated import _norm_args
+    want, y, ssum = full(rows, cols), full(rows + 1, cols), full(rows + 1, cols)
+    rstd, rstd2, turned, alone = full(rows, dt=torch.float32), full(rows, dt=torch.float32), full(B, Cc, R, dt=to), full(B, Cc, R, dt=to)
+    total = x + x2
+    a = _norm_args(total, z, w, 1e-5, None, False)
+    a.y, a.y_row_stride, a.rstd = want.data_ptr(), cols, rstd.data_ptr()
+    assert lib.issm_gated_rmsnorm_fwd(C.byref(a)) == 0
+    assert lib.issm_transpose_states(C.byref(_turn(s0, s1, 0.5, alone))) == 0
+    a.x, a.y, a.rstd = x.data_ptr(), y.data_ptr(), rstd2.data_ptr()
+    t = _turn(s0, s1, 0.5, turned)
+    assert lib.issm_layer_behind(C.byref(a), C.c_void_p(x2.data_ptr()), C.c_void_p(ssum.data_ptr()), C.byref(t)) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(ssum[:rows], total) and torch.equal(y[:rows], want) and torch.equal(rstd, rstd2) and torch.equal(turned, alone)
+    assert (ssum[rows] == 3.0).all() and (y[rows] == 3.0).all()
+    assert lib.issm_layer_behind(C.byref(a), None, C.c_void_p(ssum.data_ptr()), C.byref(t)) != 0
+    a.layer_norm, a.mean = 1, rstd.data_ptr()
+    assert lib.issm_layer_behind(C.byref(a), C.c_void_p(x2.data_ptr()), C.c_void_p(ssum.data_ptr()), C.byref(t)) != 0
+
+
+class LayerParams(C.Structure):
+    _fields_ = [("src", C.c_void_p * 9), ("n", C.c_int32 * 9), ("dtype", C.c_int32 * 9), ("a_log", C.c_int32), ("K", C.c_int32),
+                ("out", C.c_void_p), ("A", C.c_void_p), ("stream", C.c_void_p)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sizes,K,B,R,Cc", [((3, 0, 1, 500, 2, 7, 8, 8, 1), 33, 2, 65, 70), ((0,) * 9, 4, 1, 64, 64), ((9,) * 9, 0, 0, 1, 1)])
+def test_begin_of_a_layer(dtype, sizes, K, B, R, Cc):
+    """The small parameters and the turned queries in one launch: the bits of either on its own."""
+    lib = L.load()
+    g = torch.Generator().manual_seed(K)
+    arrays, q = [torch.randn(n, generator=g).to(dtype).cuda() for n in sizes], torch.randn(B, R, Cc, generator=g).to(dtype).cuda()
+    out, A, out2, A2 = (torch.full((n + 1,), 3.0, device="cuda") for n in 2 * (sum(sizes), sizes[7] * K))
+    turned = torch.full((B, Cc, R), 3.0, dtype=dtype, device="cuda")
+    p = LayerParams()
+    for i, t in enumerate(arrays):
+        p.src[i], p.n[i], p.dtype[i] = t.data_ptr(), t.numel(), L.ISSM_BF16 if dtype == torch.bfloat16 else L.ISSM_F32
+    p.a_log, p.K, p.out, p.A, p.stream = 7, K, out.data_ptr(), A.data_ptr(), L.current_stream_ptr(q.device)
+    assert lib.issm_layer_params(C.byref(p)) == 0
+    p.out, p.A = out2.data_ptr(), A2.data_ptr()
+    assert lib.issm_layer_begin(C.byref(p), C.byref(_turn(q, None, 1.0, turned))) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, out2) and torch.equal(A, A2) and torch.equal(turned, q.transpose(1, 2))
+    assert lib.issm_layer_begin(C.byref(p), None) != 0
