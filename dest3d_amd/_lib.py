@@ -33,7 +33,7 @@ EXPORTS = [
     "issm_box_dist_bwd_scratch_bytes", "issm_box_dist_fwd", "issm_box_dist_bwd",
     "issm_hilbert_codes", "issm_hilbert_order", "issm_transpose_states", "issm_layer_params", "issm_linear_fwd", "issm_linear_dx", "issm_linear_dw", "issm_linear_dw_pair", "issm_linear_dw_scratch_bytes", "issm_layer_out", "issm_layer_in",
     "issm_param_gen_fwd_only", "issm_conv_param_gen_fwd", "issm_layer_end", "issm_box_dist_fwd_only",
-    "issm_box_table",
+    "issm_box_table", "issm_box_table_bwd",
     "issm_pn2_furthest_point_sampling", "issm_pn2_ball_query", "issm_pn2_group_points", "issm_pn2_group_points_grad",
     "issm_pn2_gather_points", "issm_pn2_gather_points_grad", "issm_pn2_three_nn", "issm_pn2_three_interpolate",
     "issm_pn2_three_interpolate_grad", "issm_pn2_group_xyz_points", "issm_pn2_group_points_grad_rows",
@@ -247,6 +247,7 @@ def load() -> C.CDLL:
     lib.issm_param_gen_fwd_only.argtypes = [P(PGenArgs)]
     lib.issm_conv_param_gen_fwd.argtypes = [P(DwConvArgs), P(PGenArgs)]
     lib.issm_box_table.argtypes = [P(BoxTableArgs)]
+    lib.issm_box_table_bwd.argtypes = [P(BoxTableArgs), vp, vp, vp, vp]   # (without: addresses arrive as 32-bit integers)
     lib.issm_linear_dw_scratch_bytes.argtypes = [C.c_int64, C.c_int32, C.c_int32]
     lib.issm_linear_dw_scratch_bytes.restype = C.c_size_t
     _lib = lib

@@ -10,7 +10,6 @@ There is no fallback path."""
 from __future__ import annotations
 
 import ctypes as C
-import math
 from typing import Optional
 
 import torch
@@ -59,6 +58,38 @@ def _watched() -> bool:
     is a function mode as well, and asks for nothing but new tensors.)"""
     return bool(torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack()
                 or any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+
+
+class BoxTableFn(torch.autograd.Function):
+    """The table of ``BoxDistFun`` with gradients: its modules' products forward, one kernel backward."""
+
+    @staticmethod
+    def forward(ctx, module, w1, b1, w2, coords):
+        ctx.save_for_backward(w1, b1, w2, coords)
+        return module.rpe_table().float().contiguous()
+
+    @staticmethod
+    def backward(ctx, dtable):
+        w1, b1, w2, coords = ctx.saved_tensors
+        if torch.is_grad_enabled():   # to be differentiated again: as operations that autograd records
+            x, g = coords.reshape(-1, 3).to(w1.dtype), dtable.reshape(CHANNELS, -1).to(w1.dtype)
+            h = torch.relu(nn.functional.linear(x, w1, b1))
+            dh = (g.t() @ w2) * (h > 0)
+            return None, dh.t() @ x, dh.sum(0), g @ h, None
+        a, g = _table_args(w1, b1, w2, coords), _f32c(dtable)
+        grads = [torch.empty_like(t) for t in (w1, b1, w2)]
+        with torch.cuda.device(w1.device):
+            L.check(L.load().issm_box_table_bwd(C.byref(a), g.data_ptr(), *(t.data_ptr() for t in grads)), "issm_box_table_bwd")
+        return None, *grads, None
+
+
+def _table_args(w1, b1, w2, coords):
+    a = L.BoxTableArgs()
+    a.nodes, a.hidden = coords.numel() // 3, w1.shape[0]
+    a.dtype, a.coords_dtype = L.dtype_code(w1.dtype), L.dtype_code(coords.dtype)
+    a.coords, a.w1, a.b1, a.w2 = coords.data_ptr(), w1.data_ptr(), b1.data_ptr(), w2.data_ptr()
+    a.stream = L.current_stream_ptr(w1.device)
+    return a
 
 
 class BoxDistFn(torch.autograd.Function):
@@ -186,9 +217,9 @@ class BoxDistFun(nn.Module):
         """(out_dim, n, n, n): the MLP evaluated on the coordinate lattice (dest_module.py:191)."""
         return self.cpb_mlps(self.relative_coords_table.to(self.cpb_mlps[0].weight.dtype))[0].permute(3, 0, 1, 2)
 
-    def _plain_table(self):
-        """The same table, (out_dim, n, n, n) fp32, from one kernel where nothing is to be differentiated and the modules are
-        what this class made them (calling them would do nothing else, and nobody watches); None otherwise."""
+    def _plain_mlp(self):
+        """(w1, b1, w2, coords) of the table where the kernels take them and the modules are what this class made them (calling them would
+        do nothing else, and nobody watches); None otherwise."""
         if _watched():
             return None
         if type(self.cpb_mlps) is not nn.Sequential or len(self.cpb_mlps) != 3:
@@ -206,20 +237,22 @@ class BoxDistFun(nn.Module):
                 coords.dtype not in (torch.float32, torch.bfloat16) or \
                 w.shape[0] > 256 or w.shape != (w.shape[0], 3) or ps[1].shape != w.shape[:1] or \
                 ps[2].shape != (CHANNELS, w.shape[0]) or not coords.is_contiguous() or coords.device != w.device or \
-                (torch.is_grad_enabled() and (coords.requires_grad or any(p.requires_grad for p in ps))) or \
+                (torch.is_grad_enabled() and coords.requires_grad) or \
                 any(p.dtype != w.dtype or p.device != w.device or not p.is_contiguous() or
-                    type(p) not in (nn.Parameter, torch.Tensor) for p in ps) or \
-                L.host().runs_twice():     # a checkpointed segment's run: both of them take the sums of one with gradients
+                    type(p) not in (nn.Parameter, torch.Tensor) for p in ps) or _lattice(coords) is None:
             return None
-        n = _lattice(coords)
-        if n is None:
+        return (*ps, coords)
+
+    def _plain_table(self):
+        """The same table, (out_dim, n, n, n) fp32, from one kernel where nothing is to be differentiated; None otherwise."""
+        mlp = self._plain_mlp()
+        # (a checkpointed segment's run: both of them take the sums of one with gradients)
+        if mlp is None or (torch.is_grad_enabled() and any(p.requires_grad for p in mlp)) or L.host().runs_twice():
             return None
-        a = L.BoxTableArgs()
-        a.nodes, a.hidden = math.prod(n), w.shape[0]
-        a.dtype, a.coords_dtype = L.dtype_code(w.dtype), L.dtype_code(coords.dtype)
-        a.coords, a.w1, a.b1, a.w2 = coords.data_ptr(), w.data_ptr(), ps[1].data_ptr(), ps[2].data_ptr()
-        table = torch.empty((CHANNELS, *n), dtype=torch.float32, device=w.device)
-        a.table, a.stream = table.data_ptr(), L.current_stream_ptr(w.device)
+        w = mlp[0]
+        table = torch.empty((CHANNELS, *_lattice(mlp[3])), dtype=torch.float32, device=w.device)
+        a = _table_args(*mlp)
+        a.table = table.data_ptr()
         with torch.cuda.device(w.device):
             L.check(L.load().issm_box_table(C.byref(a)), "issm_box_table")
         return table
@@ -231,9 +264,12 @@ class BoxDistFun(nn.Module):
         boxes = torch.cat([query_xyz, query_size, query_angle.unsqueeze(-1)], dim=-1).detach()
         table = self._plain_table()
         plain = table is not None
-        if not plain:
-            table = self.rpe_table()
-        out_dtype = self.cpb_mlps[0].weight.dtype if plain else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
+        mlp = None if plain else self._plain_mlp()
+        if mlp is not None and torch.is_grad_enabled() and any(p.requires_grad for p in mlp):
+            table = BoxTableFn.apply(self, *mlp)
+        elif not plain:
+            mlp, table = None, self.rpe_table()
+        out_dtype = self.cpb_mlps[0].weight.dtype if plain or mlp is not None else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
         if weight_query_pos is None:
             return BoxDistFn.apply(table, key_xyz, boxes, query_angle, None, None, 0.0, self.log_scale, self.max_value,
                                    out_dtype, True, False, plain)[0]

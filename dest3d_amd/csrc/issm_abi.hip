@@ -55,6 +55,7 @@ int linear_dw_splits(long tokens, int in, int out);
 int launch_linear_dw(LinearDwJobs& j, int njobs, hipStream_t st);
 int launch_layer_out(LayerOutP& p, hipStream_t st);
 int launch_layer_end(LayerOutP& p, LinearP& q, hipStream_t st);
+int launch_box_table_bwd(const BoxTableP& p, const float* dtable, void* dw1, void* db1, void* dw2, hipStream_t st);
 int launch_box_table(const BoxTableP& p, hipStream_t st);
 int launch_fps(int b, int n, int npoint, const float* xyz, float* temp, int* idxs, hipStream_t st);
 int launch_ball_query(int b, int n, int m, float radius, int nsample, const float* new_xyz, const float* xyz, int* idx,
@@ -909,14 +910,28 @@ int64_t issm_box_dist_bwd_scratch_bytes(int32_t batch, int32_t seqlen, int32_t n
   return box_dist_bwd_scratch_bytes(batch, seqlen, nquery, D, H, W);
 }
 
-int issm_box_table(const issm_box_table_args* a) {
+static int box_table_params(const issm_box_table_args* a, BoxTableP& p) {
   if (!a) return fail(ISSM_E_NULL, "box_table: args is NULL");
   if (a->nodes < 1 || a->hidden < 1 || a->nodes > (1 << 26)) return fail(ISSM_E_SHAPE, "box_table: %d nodes, %d hidden", a->nodes, a->hidden);
   if (a->hidden > 256) return fail(ISSM_E_UNSUPPORTED, "box_table: %d hidden values (at most 256)", a->hidden);
   for (int t : {a->dtype, a->coords_dtype})
     if (t != ISSM_F32 && t != ISSM_BF16) return fail(ISSM_E_DTYPE, "box_table: dtype %d", t);
-  if (!a->coords || !a->w1 || !a->b1 || !a->w2 || !a->table) return fail(ISSM_E_NULL, "box_table: coords/w1/b1/w2/table is NULL");
-  const BoxTableP p{a->nodes, a->hidden, a->dtype, a->coords_dtype, a->coords, a->w1, a->b1, a->w2, a->table};
+  if (!a->coords || !a->w1 || !a->b1 || !a->w2) return fail(ISSM_E_NULL, "box_table: coords/w1/b1/w2 is NULL");
+  p = BoxTableP{a->nodes, a->hidden, a->dtype, a->coords_dtype, a->coords, a->w1, a->b1, a->w2, a->table};
+  return ISSM_OK;
+}
+
+int issm_box_table_bwd(const issm_box_table_args* a, const float* dtable, void* dw1, void* db1, void* dw2) {
+  BoxTableP p;
+  if (const int rc = box_table_params(a, p)) return rc;
+  if (!dtable || !dw1 || !db1 || !dw2) return fail(ISSM_E_NULL, "box_table_bwd: dtable/dw1/db1/dw2 is NULL");
+  return launched(launch_box_table_bwd(p, dtable, dw1, db1, dw2, (hipStream_t)a->stream), "box_table_bwd");
+}
+
+int issm_box_table(const issm_box_table_args* a) {
+  BoxTableP p;
+  if (const int rc = box_table_params(a, p)) return rc;
+  if (!p.table) return fail(ISSM_E_NULL, "box_table: table is NULL");
   return launched(launch_box_table(p, (hipStream_t)a->stream), "box_table");
 }
 

@@ -630,6 +630,9 @@ typedef struct issm_box_table_args {
 } issm_box_table_args;
 
 int issm_box_table(const issm_box_table_args* args);
+/* Its backward (args->table is not used): dtable (16, nodes) fp32 -> dw1 (hidden, 3), db1 (hidden), dw2 (16, hidden) of dtype, sums in fp32 in an
+ * order that depends on the sizes alone. */
+int issm_box_table_bwd(const issm_box_table_args* args, const float* dtable, void* dw1, void* db1, void* dw2);
 int issm_box_dist_bwd(const issm_box_dist_args* args);
 
 /* ---- serialization codes of the key points ------------------------------------------------

@@ -196,3 +196,16 @@ def test_operands_of_another_size_or_device_are_refused():
             L.require_operand(x, "x", x, *sizes)
     with pytest.raises(RuntimeError):
         L.require_operand(x.to("meta"), "x", x)
+
+
+def test_entry_points_that_python_hands_addresses_declare_them(lib):
+    """Without argument types ctypes passes an integer as 32 bits, and half of an address reaches the kernel: every call in the package with
+    more than argument blocks (byref) goes to an entry point that has declared its types."""
+    calls = set()
+    for name in os.listdir(os.path.join(ROOT, "dest3d_amd")):
+        if name.endswith(".py"):
+            src = open(os.path.join(ROOT, "dest3d_amd", name)).read()
+            calls |= {m.group(1) for m in re.finditer(r"\.(issm_[a-z0-9_]+)\(([^\n]*)", src) if "data_ptr()" in m.group(2)}
+    assert "issm_box_table_bwd" in calls
+    for name in calls:
+        assert getattr(lib, name).argtypes, name

@@ -228,6 +228,37 @@ def test_table_without_a_gradient(quant, rpe_dim, dtype):
     assert ((got.double().cpu() - ref).abs() <= u * (mag + ref.abs())).all()
 
 
+@pytest.mark.parametrize("quant,rpe_dim", [("bilinear_4_10", 128), ("bilinear_4_3", 7), ("bilinear_2_1", 256)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("again", [False, True])
+def test_gradients_of_the_tables_mlp(quant, rpe_dim, dtype, again):
+    """One kernel for the MLP's backward, against fp64 from hidden values rounded as the modules round them (each may round the other way,
+    2^-8 of it); the forward is the modules'.  A backward that is to be differentiated again goes through operations."""
+    from dest3d_amd.box_dist import BoxDistFun, BoxTableFn
+    torch.manual_seed(rpe_dim)
+    m = BoxDistFun(out_dim=16, rpe_quant=quant, rpe_dim=rpe_dim).cuda().to(dtype)
+    mlp = m._plain_mlp()
+    table = BoxTableFn.apply(m, *mlp)
+    assert table.dtype == torch.float32 and torch.equal(table, m.rpe_table().float())
+    g = torch.randn(table.shape, device="cuda").to(dtype).float()
+    grads = torch.autograd.grad(table, mlp[:3], g, create_graph=again)
+    w1, b1, w2, x = (t.detach().double() for t in mlp)
+    x = m.relative_coords_table.to(dtype).double().reshape(-1, 3)
+    h = (x @ w1.t() + b1).to(dtype).double().relu()
+    gd = g.double().reshape(16, -1)
+    dh = (gd.t() @ w2) * (h > 0)
+    near = (gd.t() @ w2).abs() * ((x @ w1.t() + b1).abs() <= 2.0 ** -18 * ((x.abs() @ w1.abs().t()) + b1.abs()))   # either side of zero
+    u = (2.0 ** -5 if again else 2.0 ** -8) if dtype == torch.bfloat16 else 2.0 ** -18
+    for got, want, mag, edge in ((grads[0], dh.t() @ x, dh.abs().t() @ x.abs(), near.t() @ x.abs()), (grads[1], dh.sum(0), dh.abs().sum(0), near.sum(0)),
+                                 (grads[2], gd @ h, gd.abs() @ h, 0.0)):
+        assert got.dtype == dtype and ((got.double() - want).abs() <= u * (mag + want.abs()) + edge + 1e-12).all()
+    if again:
+        torch.autograd.grad(grads[2].float().square().sum(), mlp[0])
+    hook = m.cpb_mlps[1].register_forward_hook(lambda *_: None)
+    assert m._plain_mlp() is None
+    hook.remove()
+
+
 def test_modes_see_the_tables_mlp():
     """Who counts or records operations or functions sees the two products of the table's MLP; a default device does not ask."""
     from torch.overrides import TorchFunctionMode
