@@ -783,6 +783,12 @@ Turn::Turn(const Tensor& in0_, const Tensor& in1_, double alpha, at::ScalarType 
   a.alpha = (float)alpha;
   a.stream = stream_of(in0);
 }
+Tensor transpose_states(const Tensor& in0, const Tensor& in1, double alpha, at::ScalarType type) {
+  const Turn t(in0, in1, alpha, type);
+  check(issm_transpose_states(&t.a), "issm_transpose_states");
+  return t.out;
+}
+
 constexpr int TAPS = 7;   // of the depthwise convolutions
 constexpr int WIDTH = 16; // of the distance encoding
 
@@ -990,8 +996,7 @@ struct CoreFn : public Function<CoreFn> {
     const at::ScalarType k = key.scalar_type(), hdt = in[1].type;
     float* const par = data<float>(flat);
     const int64_t off_w = 2 * Cc * TAPS + 2 * Cc;
-    // 4'. gated RMSNorm, and half of the averaged final states' gradient in the layout of the states
-    const Turn turned(grads[1].reshape({Bsz, K, di}), Tensor(), 0.5, at::kFloat);
+    // 4'. gated RMSNorm
     const Tensor dy = cast(grads[0], k).reshape({Bsz * Ln, di}).contiguous();
     Tensor dkey = fresh(key.sizes(), key, k);
     Tensor dzx = fresh({Bsz, Ln, Wd}, key, k);   // row of d zxbcdt: [dz | d xbc | d dt]; each producer writes its part
@@ -1007,11 +1012,11 @@ struct CoreFn : public Function<CoreFn> {
       a.dz = data(dzx);
       a.dz_row_stride = Wd;
       a.dw_partial = data<float>(dwp);
-      check(issm_gated_rmsnorm_bwd_part(&a, &turned.a), "issm_gated_rmsnorm_bwd_part");
+      check(issm_gated_rmsnorm_bwd_part(&a), "issm_gated_rmsnorm_bwd_part");
     }
     // 3'. the scan: both directions receive the gradient of their sum, and half of the averaged final states'
     const Tensor dyh = dkey.view({Bsz, Ln, H, P});
-    const Tensor dfin = turned.out.view({Bsz, H, P, K});
+    const Tensor dfin = transpose_states(grads[1].reshape({Bsz, K, di}), Tensor(), 0.5, at::kFloat).view({Bsz, H, P, K});
     const Tensor dys[2] = {dyh, dyh}, dlast[2] = {dfin, dfin};
     const Scan::Grad g = s.backward(ws, dys, dlast);
     // 2'. parameter generation; the gradients of its biases go to the convolutions' backward and to dzx

@@ -44,7 +44,6 @@ int launch_transpose_states(const TrP& p, hipStream_t st);
 int launch_layer_begin(const LayerParamsP& p, const TrP& t, hipStream_t st);
 bool layer_behind_takes(const NormP& p);
 int launch_layer_behind(const NormP& p, const void* x2, void* sum, const TrP& t, hipStream_t st);
-int launch_layer_ahead(const NormP& p, const TrP& t, hipStream_t st);
 int launch_layer_grads(LayerGradsP& p, const TrP& t, hipStream_t st);
 int launch_layer_params(const LayerParamsP& p, hipStream_t st);
 bool linear_tile_takes(long tokens, int in, int out, bool nn);
@@ -600,20 +599,6 @@ int issm_gated_rmsnorm_bwd(const issm_norm_args* a) {
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd");
 }
 
-static int transpose_params(const issm_transpose_args* a, TrP& p) {
-  if (!a) return fail(ISSM_E_NULL, "transpose: args is NULL");
-  if (a->batch < 0 || a->rows < 0 || a->cols < 0) return fail(ISSM_E_SHAPE, "transpose: bad shape");
-  if ((a->in_dtype != ISSM_F32 && a->in_dtype != ISSM_BF16) || (a->out_dtype != ISSM_F32 && a->out_dtype != ISSM_BF16))
-    return fail(ISSM_E_DTYPE, "transpose: dtypes %d -> %d", a->in_dtype, a->out_dtype);
-  p.B = 0;
-  if (a->batch == 0 || a->rows == 0 || a->cols == 0) return ISSM_OK;
-  if (!a->in0 || !a->out) return fail(ISSM_E_NULL, "transpose: in0/out is NULL");
-  if (a->batch > 65535 || (a->rows + 63) / 64 > 65535) return fail(ISSM_E_SHAPE, "transpose: batch / rows too large for one launch");
-  p.B = a->batch; p.R = a->rows; p.C = a->cols; p.in_dt = a->in_dtype; p.out_dt = a->out_dtype;
-  p.in0 = a->in0; p.in1 = a->in1; p.out = a->out; p.alpha = a->alpha;
-  return ISSM_OK;
-}
-
 int issm_gated_rmsnorm_bwd_as(const issm_norm_args* a, int32_t grad_dtype) {
   NormP p;
   int rc = norm_params(a, &p, true);
@@ -624,17 +609,13 @@ int issm_gated_rmsnorm_bwd_as(const issm_norm_args* a, int32_t grad_dtype) {
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_as");
 }
 
-int issm_gated_rmsnorm_bwd_part(const issm_norm_args* a, const issm_transpose_args* b) {
+int issm_gated_rmsnorm_bwd_part(const issm_norm_args* a) {
   NormP p;
-  TrP t{};
   int rc = norm_params(a, &p, true, true);
-  if (rc || (b && (rc = transpose_params(b, t)))) return rc;
+  if (rc) return rc;
   if (p.b) return fail(ISSM_E_UNSUPPORTED, "rmsnorm_bwd_part: no bias");
-  if (b && (b->out_dtype != ISSM_F32 || b->in1)) return fail(ISSM_E_UNSUPPORTED, "rmsnorm_bwd_part: states are one tensor, turned into fp32");
   norm_scratch_warm((hipStream_t)a->stream);
   p.dw = nullptr;
-  if (t.B && layer_behind_takes(p)) return launched(launch_layer_ahead(p, t, (hipStream_t)a->stream), "rmsnorm_bwd_part");
-  if (t.B && (rc = launched(launch_transpose_states(t, (hipStream_t)a->stream), "transpose_states"))) return rc;
   return launched(launch_rmsnorm_bwd(p, (hipStream_t)a->stream), "rmsnorm_bwd_part");
 }
 
@@ -1150,6 +1131,20 @@ int issm_layer_end(const issm_layer_out_args* a, const issm_linear_args* b) {
     q.job[i] = LinearJob{nullptr, (const uint16_t*)j.w, (uint16_t*)j.y, (int)rows, out, p.di / 32, 0, 0};
   }
   return launched(launch_layer_end(p, q, (hipStream_t)a->stream), "layer_end");
+}
+
+static int transpose_params(const issm_transpose_args* a, TrP& p) {
+  if (!a) return fail(ISSM_E_NULL, "transpose: args is NULL");
+  if (a->batch < 0 || a->rows < 0 || a->cols < 0) return fail(ISSM_E_SHAPE, "transpose: bad shape");
+  if ((a->in_dtype != ISSM_F32 && a->in_dtype != ISSM_BF16) || (a->out_dtype != ISSM_F32 && a->out_dtype != ISSM_BF16))
+    return fail(ISSM_E_DTYPE, "transpose: dtypes %d -> %d", a->in_dtype, a->out_dtype);
+  p.B = 0;
+  if (a->batch == 0 || a->rows == 0 || a->cols == 0) return ISSM_OK;
+  if (!a->in0 || !a->out) return fail(ISSM_E_NULL, "transpose: in0/out is NULL");
+  if (a->batch > 65535 || (a->rows + 63) / 64 > 65535) return fail(ISSM_E_SHAPE, "transpose: batch / rows too large for one launch");
+  p.B = a->batch; p.R = a->rows; p.C = a->cols; p.in_dt = a->in_dtype; p.out_dt = a->out_dtype;
+  p.in0 = a->in0; p.in1 = a->in1; p.out = a->out; p.alpha = a->alpha;
+  return ISSM_OK;
 }
 
 int issm_transpose_states(const issm_transpose_args* a) {

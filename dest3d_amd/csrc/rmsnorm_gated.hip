@@ -215,22 +215,9 @@ __global__ __launch_bounds__(NTHREADS) void k_layer_behind(NormP p, const void* 
   transpose_nth<false, OUT_BF>(t, blockIdx.x, tile);   // (first: a tile takes longer than four rows)
 }
 
-// the sum of all lanes, in each, without a trip through LDS per step
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-#define ISSM_ADD_STEP(ctrl, rows) v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, rows, 0xf, false))
-  ISSM_ADD_STEP(0x111, 0xf);   // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
-  ISSM_ADD_STEP(0x112, 0xf);
-  ISSM_ADD_STEP(0x114, 0xf);
-  ISSM_ADD_STEP(0x118, 0xf);
-  ISSM_ADD_STEP(0x142, 0xa);   // row 0 -> 1, 2 -> 3
-  ISSM_ADD_STEP(0x143, 0xc);   // row 1 -> 2, 3
-#undef ISSM_ADD_STEP
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
 template <bool BF, int NV, bool EXT>
-__device__ __forceinline__ void rmsnorm_bwd_rows(const NormP& p, int block) {   // by a wave
-  const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(64) void k_rmsnorm_bwd_fast(NormP p) {
+  const int lane = threadIdx.x;
   const int nvec = p.ncols >> 2;
   const int ax = al_of(p.x, p.xs, BF), az = al_of(p.z, p.zs, BF), ady = al_of(p.dy, p.dys, BF);
   const int adx = al_of(p.dx, p.dxs, BF), adz = al_of(p.dz, p.dzs, BF);
@@ -261,8 +248,8 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const NormP& p, int block) {   
       zn[v] = ld4<BF>(zp, row * zs + 4 * vi, ok, az);
     }
   };
-  if ((long)block < p.rows) fetch(block);
-  for (long row = block; row < p.rows; row += p.nblocks) {
+  if ((long)blockIdx.x < p.rows) fetch(blockIdx.x);
+  for (long row = blockIdx.x; row < p.rows; row += p.nblocks) {
     const float rstd = rstd_n, mean = mean_n;  // mean stays 0 for RMS statistics
     f4 xo[NV], dyo[NV], z[NV], sg[NV], gate[NV];
 #pragma unroll
@@ -282,8 +269,8 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const NormP& p, int block) {   
       c1 += (t.x + t.y) + (t.z + t.w);
       if (EXT) c2 += (wd.x + wd.y) + (wd.z + wd.w);
     }
-    c1 = wave_sum_dpp(c1) / (float)p.ncols;
-    c2 = (EXT && p.ln) ? wave_sum_dpp(c2) / (float)p.ncols : 0.0f;
+    c1 = wave_sum(c1) / (float)p.ncols;
+    c2 = (EXT && p.ln) ? wave_sum(c2) / (float)p.ncols : 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int vi = lane + 64 * v;
@@ -315,27 +302,10 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const NormP& p, int block) {   
   for (int v = 0; v < NV; ++v) {
     const int vi = lane + 64 * v;
     if (vi < nvec) {
-      *(f4*)(p.dw_partial + (long)block * p.ncols + 4 * vi) = dwacc[v];
-      if constexpr (EXT) { if (p.b) *(f4*)(p.db_partial + (long)block * p.ncols + 4 * vi) = dbacc[v]; }
+      *(f4*)(p.dw_partial + (long)blockIdx.x * p.ncols + 4 * vi) = dwacc[v];
+      if constexpr (EXT) { if (p.b) *(f4*)(p.db_partial + (long)blockIdx.x * p.ncols + 4 * vi) = dbacc[v]; }
     }
   }
-}
-
-// Four waves a workgroup, sums over a row without LDS: 8192 x 288, bf16, 12.3 us -> 11.3.
-template <bool BF, int NV, bool EXT>
-__global__ __launch_bounds__(NTHREADS) void k_rmsnorm_bwd_fast(NormP p) {
-  const int block = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (block < p.nblocks) rmsnorm_bwd_rows<BF, NV, EXT>(p, block);
-}
-
-// The norm's backward and, in the workgroups in front, the gradient of a layer's final states turned (issm_gated_rmsnorm_bwd_part).  8 x 1024 tokens, 288
-// features, 256 queries, bf16: 11.9 us, 13.5 + 4.9 as two launches.
-template <bool BF, int NV, bool IN_BF>
-__global__ __launch_bounds__(NTHREADS) void k_layer_ahead(NormP p, TrP t, int tiles) {
-  __shared__ float tile[64][65];
-  if ((int)blockIdx.x < tiles) return transpose_nth<IN_BF, false>(t, blockIdx.x, tile);
-  const int block = ((int)blockIdx.x - tiles) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (block < p.nblocks) rmsnorm_bwd_rows<BF, NV, false>(p, block);
 }
 
 static bool norm_fast_ok(const NormP& p) { return p.ngroups == 1 && (p.ncols & 3) == 0 && p.ncols <= 1024; }
@@ -475,21 +445,8 @@ int launch_layer_behind(const NormP& p, const void* x2, void* sum, const TrP& t,
   return (int)hipGetLastError();
 }
 
-int launch_layer_ahead(const NormP& p, const TrP& t, hipStream_t st) {   // where layer_behind_takes
-  const long tiles = transpose_tiles(t), blocks = tiles + (p.nblocks + 3) / 4;
-  if (blocks > 0x7fffffff) return (int)hipErrorInvalidValue;
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NTHREADS), 0, st, p, t, (int)tiles); };
-  const int nv = (p.ncols / 4 + 63) / 64;
-  auto form = [&](auto one, auto two, auto four) { nv <= 1 ? go(one) : nv == 2 ? go(two) : go(four); };
-  if (p.dt && t.in_dt) form(&k_layer_ahead<true, 1, true>, &k_layer_ahead<true, 2, true>, &k_layer_ahead<true, 4, true>);
-  else if (p.dt) form(&k_layer_ahead<true, 1, false>, &k_layer_ahead<true, 2, false>, &k_layer_ahead<true, 4, false>);
-  else if (t.in_dt) form(&k_layer_ahead<false, 1, true>, &k_layer_ahead<false, 2, true>, &k_layer_ahead<false, 4, true>);
-  else form(&k_layer_ahead<false, 1, false>, &k_layer_ahead<false, 2, false>, &k_layer_ahead<false, 4, false>);
-  return (int)hipGetLastError();
-}
-
 int launch_rmsnorm_bwd(const NormP& p, hipStream_t st) {
-  if (norm_fast_ok(p)) NORM_FAST(k_rmsnorm_bwd_fast, dim3((p.nblocks + 3) / 4), dim3(NTHREADS));
+  if (norm_fast_ok(p)) NORM_FAST(k_rmsnorm_bwd_fast, dim3(p.nblocks), dim3(64));
   else hipLaunchKernelGGL(k_rmsnorm_bwd, dim3(p.nblocks), dim3(64), (size_t)(p.b ? 2 : 1) * p.ncols * sizeof(float), st, p);
   int e = (int)hipGetLastError();
   if (e || !p.dw) return e;

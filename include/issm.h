@@ -292,11 +292,8 @@ int issm_gated_rmsnorm_fwd(const issm_norm_args* args);
 int issm_gated_rmsnorm_bwd(const issm_norm_args* args);
 /* issm_gated_rmsnorm_bwd with dw and db in grad_dtype (issm_dtype): one rounding of the fp32 sums. */
 int issm_gated_rmsnorm_bwd_as(const issm_norm_args* args, int32_t grad_dtype);
-/* issm_gated_rmsnorm_bwd without its last sum: dw_partial keeps (issm_rmsnorm_bwd_blocks, ncols), dw is not written (no bias).  states, if not
- * NULL: issm_transpose_states (out_dtype ISSM_F32, in1 NULL) on this call's stream, in the same launch where rows are of up to 1024 columns, a
- * multiple of 4. */
-struct issm_transpose_args;
-int issm_gated_rmsnorm_bwd_part(const issm_norm_args* args, const struct issm_transpose_args* states);
+/* issm_gated_rmsnorm_bwd without its last sum: dw_partial keeps (issm_rmsnorm_bwd_blocks, ncols), dw is not written (no bias). */
+int issm_gated_rmsnorm_bwd_part(const issm_norm_args* args);
 
 /* issm_gated_rmsnorm_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and the same

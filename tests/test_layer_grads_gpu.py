@@ -166,37 +166,3 @@ def test_begin_of_a_layer(dtype, sizes, K, B, R, Cc):
     torch.cuda.synchronize()
     assert torch.equal(out, out2) and torch.equal(A, A2) and torch.equal(turned, q.transpose(1, 2))
     assert lib.issm_layer_begin(C.byref(p), None) != 0
-
-
-@pytest.mark.parametrize("dtype,sdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
-@pytest.mark.parametrize("rows,cols,B,R,Cc", [(1, 4, 1, 1, 1), (2051, 256, 2, 65, 64), (130, 288, 0, 3, 5), (7, 30, 1, 64, 130), (33, 1024, 3, 70, 33)])
-def test_ahead_of_the_scans_backward(dtype, sdt, rows, cols, B, R, Cc):
-    """The norm's backward without its last sum and the turned gradient: what issm_gated_rmsnorm_bwd and the transposition give."""
-    lib = L.load()
-    g = torch.Generator().manual_seed(rows + cols)
-    x, z, dy = (torch.randn(rows, cols, generator=g).to(dtype).cuda() for _ in range(3))
-    w, rstd = torch.randn(cols, generator=g).to(dtype).cuda(), (0.5 + torch.rand(rows, generator=g)).cuda()
-    s = torch.randn(B, R, Cc, generator=g).to(sdt).cuda()
-    from dest3d_amd.layernorm_gated import _norm_args
-    nb = lib.issm_rmsnorm_bwd_blocks(rows)
-    out = []
-    for part in (False, True):
-        dx, dz = (torch.full((rows + 1, cols), 3.0, dtype=dtype, device="cuda") for _ in range(2))
-        parts, dw = torch.full((nb + 1, cols), 3.0, device="cuda"), torch.full((cols,), 3.0, device="cuda")
-        a = _norm_args(x, z, w, 1e-5, None, False)
-        a.rstd, a.dy, a.dy_row_stride, a.dx, a.dx_row_stride = rstd.data_ptr(), dy.data_ptr(), cols, dx.data_ptr(), cols
-        a.dz, a.dz_row_stride, a.dw_partial = dz.data_ptr(), cols, parts.data_ptr()
-        turned = torch.full((B, Cc, R), 3.0, device="cuda")
-        if part:
-            assert lib.issm_gated_rmsnorm_bwd_part(C.byref(a), C.byref(_turn(s, None, 0.5, turned))) == 0
-        else:
-            a.dw = dw.data_ptr()
-            assert lib.issm_gated_rmsnorm_bwd(C.byref(a)) == 0
-        torch.cuda.synchronize()
-        assert (parts[nb] == 3.0).all() and (dx[rows] == 3.0).all() and (dz[rows] == 3.0).all()
-        out.append((dx, dz, parts, dw, turned))
-    for i in range(3):
-        assert torch.equal(out[0][i], out[1][i])
-    total = out[1][2][:nb].double()
-    assert ((out[0][3].double() - total.sum(0)).abs() <= nb * 2.0 ** -24 * total.abs().sum(0)).all()
-    assert torch.equal(out[1][4], 0.5 * s.float().transpose(1, 2))
