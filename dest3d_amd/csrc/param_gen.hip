@@ -85,7 +85,8 @@ __device__ __forceinline__ void st1(void* p, long i, float v) {
 // RAW: dt before softplus and weight is kept for the backward where there are weights (a scene of 1024 tokens x 256: 10.4 us,
 // 9.5 without).
 // CONV: B and C's biases are the convolutions' outputs for the last 2G channels, computed here from their inputs.
-template <bool BF, int KV, bool TOK, bool RAW, bool CONV>
+// FAR: two tokens' rows are not within 31-bit byte offsets (KV = 1).
+template <bool BF, int KV, bool TOK, bool RAW, bool CONV, bool FAR>
 __device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, int block) {
   const int R0 = p.H + 2 * p.G, R = R0 + (p.has_back ? 2 * p.G : 0);
   const int per_tok = (p.K + KV - 1) / KV;  // threads per token
@@ -127,13 +128,22 @@ __device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, in
   // product a store, 109 v_mul_lo and 102 v_mad_u64, a quarter of the rate each, stood beside 360 multiply-adds: 8192 tokens x 256, bf16,
   // weights, 36.1 us -> 33.4; a layer without a gradient of 4 scenes 129.0 -> 125.1, of one 57.7 -> 57.1.)
   constexpr int SZ = BF ? 2 : 4;
-  const unsigned at_h = (unsigned)((int)tl * p.H * p.K + k) * SZ, at_g = (unsigned)((int)tl * p.G * p.K + k) * SZ;
-  auto rows = [&](void* q, int per) __attribute__((always_inline)) {
-    return __builtin_amdgcn_make_buffer_rsrc((char*)q + t0 * per * p.K * SZ, 0, (unsigned)(wg_tokens * per * p.K) * SZ, 0x00027000);
+  const unsigned at_h = tl * (unsigned)(p.H * p.K) * SZ + (unsigned)k * SZ, at_g = tl * (unsigned)(p.G * p.K) * SZ + (unsigned)k * SZ;
+  struct Rows {
+    __amdgpu_buffer_rsrc_t buf;
+    char* first;   // FAR: the thread's place in row 0 of its token
   };
-  auto put = [&](const __amdgpu_buffer_rsrc_t& q, unsigned at, int row, const float (&v)[KV]) __attribute__((always_inline)) {
+  auto rows = [&](void* q, int per) __attribute__((always_inline)) {
+    char* base = (char*)q + t0 * per * p.K * SZ;
+    return Rows{__builtin_amdgcn_make_buffer_rsrc(base, 0, FAR ? 0u : (unsigned)(wg_tokens * per * p.K) * SZ, 0x00027000),
+                FAR ? base + ((long)tl * per * p.K + k) * SZ : nullptr};
+  };
+  auto put = [&](const Rows& to, unsigned at, int row, const float (&v)[KV]) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t& q = to.buf;
     const int s = row * p.K * SZ;   // uniform
-    if constexpr (BF && KV == 2) {
+    if constexpr (FAR) {
+      st1<BF>(to.first, (long)row * p.K, v[0]);
+    } else if constexpr (BF && KV == 2) {
       __builtin_amdgcn_raw_buffer_store_b32((unsigned)f_to_bf16(v[0]) | ((unsigned)f_to_bf16(v[1]) << 16), q, at, s, 0);
     } else if constexpr (BF) {
       __builtin_amdgcn_raw_buffer_store_b16(f_to_bf16(v[0]), q, at, s, 0);
@@ -144,8 +154,8 @@ __device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, in
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), q, at, s, 0);
     }
   };
-  const __amdgpu_buffer_rsrc_t dt_rows = rows(p.dt, p.H), raw_rows = rows(RAW && p.dt_raw ? p.dt_raw : p.dt, p.H);
-  const __amdgpu_buffer_rsrc_t bc_rows[4] = {rows(p.Bm, p.G), rows(p.Cm, p.G), rows(p.has_back ? p.Bb : p.Bm, p.G), rows(p.has_back ? p.Cb : p.Cm, p.G)};
+  const Rows dt_rows = rows(p.dt, p.H), raw_rows = rows(RAW && p.dt_raw ? p.dt_raw : p.dt, p.H);
+  const Rows bc_rows[4] = {rows(p.Bm, p.G), rows(p.Cm, p.G), rows(p.has_back ? p.Bb : p.Bm, p.G), rows(p.has_back ? p.Cb : p.Cm, p.G)};
   // the token's biases, all requested before the row loop (a load per row inside it would be waited for row by
   // row); bb: the reversed-order pair's bias of a B / C row
   float bv[PG_MAXR0], bb[PG_MAXR0];
@@ -195,7 +205,12 @@ __device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, in
 
 template <bool BF, int KV, bool TOK, bool RAW>
 __global__ __launch_bounds__(NTHREADS) void k_pgen_fwd(PGenP p) {
-  pgen_fwd<BF, KV, TOK, RAW, false>(p, DwConvP{}, blockIdx.x);
+  pgen_fwd<BF, KV, TOK, RAW, false, false>(p, DwConvP{}, blockIdx.x);
+}
+template <bool BF, bool TOK>
+__global__ __launch_bounds__(NTHREADS) void k_pgen_fwd_far(PGenP p) {
+  if (!p.weights || p.dt_raw) pgen_fwd<BF, 1, TOK, true, false, true>(p, DwConvP{}, blockIdx.x);
+  else pgen_fwd<BF, 1, TOK, false, false, true>(p, DwConvP{}, blockIdx.x);
 }
 
 // What lies between a layer's first projections and its scan where no gradient is asked for, one launch: the generation above and,
@@ -206,7 +221,11 @@ template <int KV, int TL>
 __global__ __launch_bounds__(NTHREADS) void k_conv_pgen(PGenP p, DwConvP c, int pgen_blocks) {
   warm_first<sizeof(PGenP) + sizeof(DwConvP)>();
   if ((int)blockIdx.x >= pgen_blocks) dw_chain_fwd<true, TL, false>(c, (long)((int)blockIdx.x - pgen_blocks) * NTHREADS + threadIdx.x);
-  else pgen_fwd<true, KV, true, false, true>(p, c, blockIdx.x);
+  else pgen_fwd<true, KV, true, false, true, false>(p, c, blockIdx.x);
+}
+__global__ __launch_bounds__(NTHREADS) void k_conv_pgen_far(PGenP p, DwConvP c, int pgen_blocks) {
+  if ((int)blockIdx.x >= pgen_blocks) dw_chain_fwd<true, 4, false>(c, (long)((int)blockIdx.x - pgen_blocks) * NTHREADS + threadIdx.x);
+  else pgen_fwd<true, 1, true, false, true, true>(p, c, blockIdx.x);
 }
 
 // Gradient row r of token t: dt heads, then B groups, then C groups (`back`: the reversed-order pair, which
@@ -613,16 +632,24 @@ static int pgen_group(const PGenP& p) {
   // (four adjacent k per thread, 8-byte bf16 stores, measured slower: 42 us against 39 at 8192 tokens x 256)
   return (p.K % 2 == 0 && al) ? 2 : 1;
 }
+// Whether the rows of the two tokens that a workgroup of so many queries may have reach beyond 31-bit byte offsets
+static bool pgen_far(const PGenP& p) { return 2L * std::max(p.H, p.G) * p.K * (p.dtype ? 2 : 4) >= 1L << 31; }
 static size_t pgen_lds(const PGenP& p, int per_tok) {
   const int R = p.H + (p.has_back ? 4 : 2) * p.G;
   return p.bias ? 0 : ((NTHREADS - 1) / per_tok + 2) * (size_t)R * sizeof(float);   // at most 23 KB
 }
 
 int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
-  const int kv = pgen_group(p), per_tok = (p.K + kv - 1) / kv;
+  const bool far = pgen_far(p);
+  const int kv = far ? 1 : pgen_group(p), per_tok = (p.K + kv - 1) / kv;
   const unsigned blocks = (unsigned)((p.tokens * per_tok + NTHREADS - 1) / NTHREADS);
   const size_t lds = pgen_lds(p, per_tok);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), lds, st, p); };
+  if (far) {
+    if (p.dtype) p.bias ? go(&k_pgen_fwd_far<true, false>) : go(&k_pgen_fwd_far<true, true>);
+    else p.bias ? go(&k_pgen_fwd_far<false, false>) : go(&k_pgen_fwd_far<false, true>);
+    return (int)hipGetLastError();
+  }
   const bool raw = !p.weights || p.dt_raw;
   auto forms = [&](auto two, auto one, auto two_only, auto one_only) { raw ? go(kv == 2 ? two : one) : go(kv == 2 ? two_only : one_only); };
   if (p.bias) {
@@ -636,16 +663,18 @@ int launch_pgen_fwd(const PGenP& p, hipStream_t st) {
 }
 
 int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st) {
-  const int kv = pgen_group(p), per_tok = (p.K + kv - 1) / kv;
+  const bool far = pgen_far(p);
+  const int kv = far ? 1 : pgen_group(p), per_tok = (p.K + kv - 1) / kv;
   const long gen = (p.tokens * per_tok + NTHREADS - 1) / NTHREADS;
   // tokens a thread of the convolutions: as few as leave two waves a SIMD (see there)
   auto items = [&](int tokens) { return (long)c.B * ((c.L + tokens - 1) / tokens) * c.split; };
-  const int tl = items(16) >= 2048 * 64 ? 16 : items(8) >= 2048 * 64 ? 8 : 4;
+  const int tl = far ? 4 : items(16) >= 2048 * 64 ? 16 : items(8) >= 2048 * 64 ? 8 : 4;
   const long conv = (items(tl) + NTHREADS - 1) / NTHREADS;
   if (gen + conv > 0x7fffffff) return (int)hipErrorInvalidValue;
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(gen + conv)), dim3(NTHREADS), pgen_lds(p, per_tok), st, p, c, (int)gen); };
   auto form = [&](auto two, auto one) { kv == 2 ? go(two) : go(one); };
-  if (tl == 16) form(&k_conv_pgen<2, 16>, &k_conv_pgen<1, 16>);
+  if (far) go(&k_conv_pgen_far);
+  else if (tl == 16) form(&k_conv_pgen<2, 16>, &k_conv_pgen<1, 16>);
   else if (tl == 8) form(&k_conv_pgen<2, 8>, &k_conv_pgen<1, 8>);
   else form(&k_conv_pgen<2, 4>, &k_conv_pgen<1, 4>);
   return (int)hipGetLastError();
@@ -654,7 +683,7 @@ int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st) {
 template <bool BF, bool HASW>
 static void pgen_bwd_launch(const PGenP& p, hipStream_t st) {
   const dim3 g((unsigned)p.nblocks), b(NTHREADS);
-  if (p.K % 64 == 0) hipLaunchKernelGGL((k_pgen_bwd<BF, true, HASW>), g, b, 0, st, p);
+  if (p.K % 64 == 0 && p.K < 1 << 24) hipLaunchKernelGGL((k_pgen_bwd<BF, true, HASW>), g, b, 0, st, p);
   else hipLaunchKernelGGL((k_pgen_bwd<BF, false, HASW>), g, b, 0, st, p);
 }
 

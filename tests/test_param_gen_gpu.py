@@ -166,3 +166,29 @@ def test_generation_and_convolutions_in_one_launch(B, L, K, H, G, di, weighted):
 
     for got, want in zip(run(True), run(False)):
         assert torch.equal(got, want)
+
+
+def test_rows_beyond_32_bit_offsets():
+    """A token with so many queries that its rows are not within 31-bit byte offsets: the kernels with 64-bit places, against the same
+    queries in a call of their own."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib = L.load()
+    K, H, G, few = 53_700_001, 10, 1, 777
+    W, bias = torch.randn(H + 2 * G, 16).cuda(), torch.randn(1, H + 2 * G).cuda()
+    dist = torch.zeros(1, K, 16, dtype=torch.bfloat16, device="cuda")
+    dist[:, -few:] = torch.randn(1, few, 16).bfloat16().cuda()
+
+    def run(d):
+        k = d.shape[1]
+        dt, Bm, Cm = (torch.full((1, n, k), 3.0, dtype=torch.bfloat16, device="cuda") for n in (H, G, G))
+        a = L.PGenArgs()
+        a.tokens, a.K, a.M, a.H, a.G, a.dtype, a.has_back = 1, k, 16, H, G, L.ISSM_BF16, 0
+        a.dist, a.W, a.bias, a.dt, a.Bm, a.Cm = (t.data_ptr() for t in (d, W, bias, dt, Bm, Cm))
+        a.stream = L.current_stream_ptr(d.device)
+        assert lib.issm_param_gen_fwd(C.byref(a)) == 0
+        torch.cuda.synchronize()
+        return dt, Bm, Cm
+    for far, near in zip(run(dist), run(dist[:, -few:].contiguous())):
+        assert torch.equal(far[..., -few:], near)
+        assert torch.equal(far[..., :5], far[..., K // 2:K // 2 + 5]) and (far[..., 0] != 3.0).all()
