@@ -694,9 +694,19 @@ struct LinearFn : public Function<LinearFn> {
 // The projections of keys and queries that stand beside each other in the layer, as one node: where both are products of the kernels here, forward, input
 // and weight gradients take one launch for the two (and the weight gradients' sums another) instead of two each, the shorter one beside the other:
 // 8 x 1024 keys and 8 x 256 queries, 288 features, us a pair: forward 15.1 -> 10.2, dx 16.6 -> 11.4, dW 19.5 -> 13.3 and its sums 9.1 -> 4.6.
+// What a side saves is its own: a backward pass that wants the one neither looks at the other's tensors (which may have been changed in place) nor frees
+// them, so that a second pass may want those.
+struct PairRecord : torch::CustomClassHolder {
+  torch::autograd::SavedVariable saved[2][2];   // of either side x, w
+  void save(int side, const Tensor& x, const Tensor& w) {
+    saved[side][0] = torch::autograd::SavedVariable(x, false);
+    saved[side][1] = torch::autograd::SavedVariable(w, false);
+  }
+};
 struct LinearPairFn : public Function<LinearPairFn> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x0, const Tensor& w0, const Tensor& x1, const Tensor& w1) {
-    ctx->save_for_backward({x0, w0, x1, w1});
+  static variable_list forward(AutogradContext* ctx, const Tensor& x0, const Tensor& w0, const Tensor& x1, const Tensor& w1,
+                               const c10::intrusive_ptr<PairRecord>& record) {
+    keep(ctx, record);
     ctx->set_materialize_grads(false);   // an output that nothing was made of gives its weight no gradient
     if (own_linear(x0, w0) && own_linear(x1, w1) && x0.device() == x1.device()) {
       Product p[2] = {{&x0, &w0, {}}, {&x1, &w1, {}}};
@@ -707,28 +717,31 @@ struct LinearPairFn : public Function<LinearPairFn> {
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
-    const variable_list v = ctx->get_saved_variables();
-    Tensor dy[2], out[4];
-    bool want_x[2], want_w[2];
+    const auto record = kept<PairRecord>(ctx);
+    Tensor x[2], w[2], dy[2], out[4];
+    bool want_x[2], want_w[2], want[2];
     for (int i = 0; i < 2; ++i) {
-      if (grads[i].defined()) dy[i] = cast(grads[i], v[2 * i].scalar_type());
-      want_x[i] = dy[i].defined() && ctx->needs_input_grad(2 * i);
-      want_w[i] = dy[i].defined() && ctx->needs_input_grad(2 * i + 1);
+      want_x[i] = grads[i].defined() && ctx->needs_input_grad(2 * i);
+      want_w[i] = grads[i].defined() && ctx->needs_input_grad(2 * i + 1);
+      want[i] = want_x[i] || want_w[i];
+      if (!want[i]) continue;
+      x[i] = record->saved[i][0].unpack();
+      w[i] = record->saved[i][1].unpack();
+      dy[i] = cast(grads[i], x[i].scalar_type());
     }
-    const bool together = v[0].device() == v[2].device();
-    if (together && want_x[0] && want_x[1] && own_dx(dy[0], v[1]) && own_dx(dy[1], v[3])) {
-      Product p[2] = {{&dy[0], &v[1], {}}, {&dy[1], &v[3], {}}};
+    if (want_x[0] && want_x[1] && x[0].device() == x[1].device() && own_dx(dy[0], w[0]) && own_dx(dy[1], w[1])) {
+      Product p[2] = {{&dy[0], &w[0], {}}, {&dy[1], &w[1], {}}};
       launch_products(&issm_linear_dx, true, p);
       out[0] = p[0].y;
       out[2] = p[1].y;
     } else {
       for (int i = 0; i < 2; ++i)
-        if (want_x[i]) out[2 * i] = own_dx(dy[i], v[2 * i + 1]) ? linear_dx(dy[i], v[2 * i + 1]) : at::matmul(dy[i], v[2 * i + 1]);
+        if (want_x[i]) out[2 * i] = own_dx(dy[i], w[i]) ? linear_dx(dy[i], w[i]) : at::matmul(dy[i], w[i]);
     }
     WeightGradient g[2];
     for (int i = 0; i < 2; ++i)
-      if (want_w[i]) g[i] = {v[2 * i].reshape({-1, v[2 * i].size(-1)}), dy[i].reshape({-1, dy[i].size(-1)}), {}};
-    if (together && want_w[0] && want_w[1] && narrow_result(g[0].x, g[0].dy) && narrow_result(g[1].x, g[1].dy)) {
+      if (want_w[i]) g[i] = {x[i].reshape({-1, x[i].size(-1)}), dy[i].reshape({-1, dy[i].size(-1)}), {}};
+    if (want_w[0] && want_w[1] && x[0].device() == x[1].device() && narrow_result(g[0].x, g[0].dy) && narrow_result(g[1].x, g[1].dy)) {
       launch_weight_gradients(g);
       out[1] = g[0].dw;
       out[3] = g[1].dw;
@@ -736,7 +749,12 @@ struct LinearPairFn : public Function<LinearPairFn> {
       for (int i = 0; i < 2; ++i)
         if (want_w[i]) out[2 * i + 1] = weight_gradient(g[i].x, g[i].dy);
     }
-    return {out[0], out[1], out[2], out[3]};
+    // (as a node's own saved tensors; what has been freed says so when it is asked for again)
+    if (!torch::autograd::get_current_graph_task_keep_graph())
+      for (int i = 0; i < 2; ++i)
+        for (auto& s : record->saved[i])
+          if (want[i]) s.reset_data();
+    return {out[0], out[1], out[2], out[3], Tensor()};
   }
 };
 
@@ -757,7 +775,13 @@ variable_list linear_pair(Tensor x0, Tensor w0, Tensor x1, Tensor w1) {
   if ((x0.requires_grad() || w0.requires_grad()) != (x1.requires_grad() || w1.requires_grad())) return {linear_tokens(x0, w0), linear_tokens(x1, w1)};
   autocast_types({&x0, &w0, &x1, &w1});
   const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::DispatchKey::AutocastCUDA);
-  return LinearPairFn::apply(x0, w0, x1, w1);
+  const auto record = c10::make_intrusive<PairRecord>();
+  variable_list y = LinearPairFn::apply(x0, w0, x1, w1, record);
+  if (y[0].requires_grad()) {
+    record->save(0, x0, w0);
+    record->save(1, x1, w1);
+  }
+  return y;
 }
 
 // ------------------------------------------------------------------------------- the chain between a layer's projections
@@ -1310,6 +1334,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_tokens", [](const Tensor& x, const Tensor& w) {
     py::gil_scoped_release release;
     return linear_tokens(x, w);
+  });
+  m.def("linear_pair", [](const Tensor& x0, const Tensor& w0, const Tensor& x1, const Tensor& w1) {
+    py::gil_scoped_release release;
+    return linear_pair(x0, w0, x1, w1);
   });
   m.def("runs_twice", &runs_twice);
   m.def("scan_core", &scan_core);

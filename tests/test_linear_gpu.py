@@ -281,6 +281,32 @@ def test_weight_gradient_of_every_form(form):
     assert ((w.grad.double().cpu() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -9 * mag.sqrt() + 300 * 2.0 ** -24 * mag).all()
 
 
+def test_backward_passes_of_either_output():
+    """One pass after the other through a layer's two outputs, without retain_graph, to what only that output was made with: the gradients of one
+    pass for both."""
+    from dest3d_amd.scan_module import MultiHeadISSMScan
+    torch.manual_seed(8)
+    B, Ln, K, D = 2, 70, 40, 288
+    layer = MultiHeadISSMScan(d_model=D, d_state=K, d_dist=16, chunk_size=256, nheads=8, expand=1).cuda().bfloat16()
+    bf = lambda *s: torch.randn(*s).cuda().bfloat16()
+    key, query, dist, dkey, dquery = bf(B, Ln, D), bf(B, K, D), bf(B, Ln, K, 16), bf(B, Ln, D), bf(B, K, D)
+    of_key, of_query = [layer.out_key_proj.weight], [layer.out_query_proj.weight, layer.query_norm.weight, layer.query_norm.bias]
+    want = torch.autograd.grad(layer(key, query, dist, None, None), of_key + of_query, (dkey, dquery))
+    out = layer(key, query, dist, None, None)
+    got = torch.autograd.grad(out[0], of_key, dkey) + torch.autograd.grad(out[1], of_query, dquery)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    # (and where nothing else has a gradient)
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    layer.out_key_proj.weight.requires_grad_()
+    layer.out_query_proj.weight.requires_grad_()
+    out = layer(key, query, dist, None, None)
+    out[1].backward(dquery)
+    out[0].backward(dkey)
+    assert torch.equal(layer.out_key_proj.weight.grad, want[0]) and torch.equal(layer.out_query_proj.weight.grad, want[1])
+
+
 @pytest.mark.parametrize("form", ["few", "many", "odd", "expanded gradient", "unaligned gradient", "wide", "again"])
 def test_gradient_to_the_tokens_of_every_form(form):
     """Both routes of the projections and of their gradients to the tokens, and the forms that stay the library's."""

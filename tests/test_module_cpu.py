@@ -1,4 +1,5 @@
 """Host-side checks of the MultiHeadISSMScan mirror that need no GPU."""
+import pytest
 
 
 def test_reference_state_dict_names():
@@ -80,3 +81,44 @@ def test_lattice_of_the_distance_table_is_checked_before_a_kernel_writes_it():
     assert _lattice(torch.zeros(1, 4, 5, 6, 3)) == (4, 5, 6)
     for shape in ((10, 10, 10, 3), (2, 4, 5, 6, 3), (1, 4, 5, 6, 6), (1, 1, 4, 5, 6, 3), (1, 4, 5, 3), (8, 3), (3,)):
         assert _lattice(torch.zeros(shape)) is None, shape
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_projections_in_a_pair_keep_their_tensors_to_themselves(first):
+    """Two products in one autograd node are two as far as a backward pass can tell: one that wants a side neither frees the other's tensors nor
+    looks at what was done to them, and a side asked for again says that it has been freed."""
+    import torch
+    from dest3d_amd import _lib as L
+    g = torch.Generator().manual_seed(first)
+    sides = [[torch.randn(*s, generator=g, dtype=torch.float64).requires_grad_() for s in shapes] for shapes in (((3, 5, 6), (4, 6)), ((7, 2), (3, 2)))]
+    dy = [torch.randn(*x.shape[:-1], w.shape[0], generator=g, dtype=torch.float64) for x, w in sides]
+    want = [torch.autograd.grad(torch.nn.functional.linear(x, w), (x, w), d) for (x, w), d in zip(sides, dy)]
+    pair = lambda: L.host().linear_pair(*sides[0], *sides[1])
+
+    def check(got, side):
+        assert all(torch.allclose(a, b, rtol=1e-12) for a, b in zip(got, want[side]))
+    second = 1 - first
+    y, unpacked = None, []
+
+    def unpack(t):
+        unpacked.append(t)
+        return t
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = pair()
+    check(torch.autograd.grad(y[first], sides[first], dy[first]), first)
+    assert len(unpacked) == 2
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(y[first], sides[first], dy[first])
+    check(torch.autograd.grad(y[second], sides[second], dy[second]), second)
+    # kept for another pass where that is asked for; both at once; one side's operand changed
+    y = pair()
+    check(torch.autograd.grad(y[first], sides[first], dy[first], retain_graph=True), first)
+    got = torch.autograd.grad(y, (*sides[0], *sides[1]), dy)
+    check(got[:2], 0)
+    check(got[2:], 1)
+    y = pair()
+    with torch.no_grad():
+        sides[second][1].add_(1.0)
+    check(torch.autograd.grad(y, sides[first], dy), first)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y[second], sides[second], dy[second])
