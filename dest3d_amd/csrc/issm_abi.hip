@@ -980,31 +980,41 @@ static int linear_params(const issm_linear_args* a, LinearP& p, int& n) {
   return ISSM_OK;
 }
 
-// Whether the products go through LDS in tiles (linear_tile.hip) or straight from memory into the matrix operands (linear.hip): the same sums
-// in the same order.  Tiles from 64 tokens and 96 outputs on (linear.hip and tiles in us: 1024 x 96 -> 202 3.4 and 2.9, 192 -> 394 4.8 and 3.8,
-// 320 -> 650 12.9 and 5.1, 4096 x 288 -> 586 12.0 and 6.4), but for odd multiples of 288 features, nine fragments from rows that
-// lie across the memory channels, which linear.hip has sooner up to some 350000 results: 128 x 288 -> 586 3.7 and 4.4, 1024 x 288 -> 288 3.8 and 4.4,
-// 1024 x 864 -> 288 7.7 and 8.5, 1024 x 288 -> 586 5.7 and 4.5 (576 features: 128 tokens 8.0 and 6.3).
-static bool linear_in_tiles(const LinearP& p, int n) {
-  int64_t results = 0;
+// Which products of a launch go through LDS in tiles (linear_tile.hip), the others straight from memory into the matrix operands (linear.hip): the
+// same sums in the same order.  Tiles from 64 tokens and 96 outputs on, each product for itself (linear.hip and tiles in us: 1024 x 96 -> 202 3.4 and 2.9,
+// 192 -> 394 4.8 and 3.8, 320 -> 650 12.9 and 5.1, 4096 x 288 -> 586 11.4 and 6.0; beside 32 x 288 -> 288, 8192 x 288 -> 586 20.7 and 10.2, beside 63 x 192 -> 192,
+// 512 x 192 -> 192 4.7 and 4.7), but for odd multiples of 288 features, nine fragments from rows that lie across the memory channels, which linear.hip
+// has sooner as long as a launch's workgroups there have a CU each: 288 -> 288 of 1024, 1536 and 2048 tokens (144, 216 and 288 workgroups) 3.8 and 4.4,
+// 3.8 and 4.4, 5.4 and 4.5; 768 and 1024 x 288 -> 586 (228 and 304) 3.9 and 4.5, 5.6 and 4.5; 1024 x 288 -> 288 beside 512 and 1024 tokens (216 and 288) 3.9 and
+// 4.4, 5.5 and 4.4; 864 -> 288 of 1536 and 2048 tokens 7.7 and 8.4, 13.1 and 8.5 (of 576 features tiles are ahead from 64 tokens on, 8.0 and 6.3).
+static void linear_forms(const LinearP& p, int n, bool (&tiles)[2]) {
+  int64_t workgroups = 0;
   bool nines = true;
   for (int i = 0; i < n; ++i) {
     const LinearJob& j = p.job[i];
-    if (j.turn || !linear_tile_takes(j.tokens, 32 * j.steps, j.out, false)) return false;
-    results += (int64_t)j.tokens * j.out;
+    tiles[i] = !j.turn && linear_tile_takes(j.tokens, 32 * j.steps, j.out, false);
+    workgroups += ((int64_t)j.tokens + 63) / 64 * (((int64_t)j.out + 31) / 32);
     nines = nines && j.steps % 18 == 9;
   }
-  return !nines || results > 350000;
+  if (nines && workgroups <= NCU) tiles[0] = tiles[1] = false;
 }
+static LinearTileJob linear_tile_job(const LinearJob& j) { return LinearTileJob{j.x, j.w, j.y, j.tokens, 32 * j.steps, j.out, 0}; }
 
 int issm_linear_fwd(const issm_linear_args* a) {
   LinearP p{};
   int n;
   const int rc = linear_params(a, p, n);
   if (rc || n == 0) return rc;
-  if (linear_in_tiles(p, n)) {
-    LinearTileP q{};
-    for (int i = 0; i < n; ++i) q.job[i] = LinearTileJob{p.job[i].x, p.job[i].w, p.job[i].y, p.job[i].tokens, 32 * p.job[i].steps, p.job[i].out, 0};
+  bool tiles[2] = {false, false};
+  linear_forms(p, n, tiles);
+  LinearTileP q{};
+  if (n == 2 && tiles[0] != tiles[1]) {   // the tiles first
+    if (tiles[1]) std::swap(p.job[0], p.job[1]);
+    q.job[0] = linear_tile_job(p.job[0]);
+    return launched(launch_layer_in_tile(q, p, LayerParamsP{}, (hipStream_t)a->stream), "linear_fwd");
+  }
+  if (tiles[0]) {
+    for (int i = 0; i < n; ++i) q.job[i] = linear_tile_job(p.job[i]);
     return launched(launch_linear_tile(q, n, false, (hipStream_t)a->stream), "linear_fwd");
   }
   return launched(launch_linear(p, n, nullptr, (hipStream_t)a->stream), "linear_fwd");
@@ -1039,9 +1049,11 @@ int issm_layer_in(const issm_linear_args* a, const issm_layer_params_args* b) {
     if (n && (rc = issm_linear_fwd(a))) return rc;
     return q.total ? issm_layer_params(b) : ISSM_OK;
   }
-  if (linear_in_tiles(p, 1)) {
+  bool tiles[2];
+  linear_forms(p, n, tiles);
+  if (tiles[0]) {
     LinearTileP t{};
-    t.job[0] = LinearTileJob{p.job[0].x, p.job[0].w, p.job[0].y, p.job[0].tokens, 32 * p.job[0].steps, p.job[0].out, 0};
+    t.job[0] = linear_tile_job(p.job[0]);
     return launched(launch_layer_in_tile(t, p, q, (hipStream_t)a->stream), "layer_in");
   }
   return launched(launch_linear(p, n, &q, (hipStream_t)a->stream), "layer_in");

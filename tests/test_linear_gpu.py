@@ -62,9 +62,34 @@ def test_linear_at_its_remainders(shapes):
 @pytest.mark.parametrize("shapes", [[(8192, 288, 586), (2048, 288, 288)], [(16400, 96, 200)], [(11000, 288, 97)], [(4097, 320, 289), (8193, 64, 610)],
                                     [(64, 32, 160000)], [(64, 96, 96)], [(3700, 288, 96), (65, 864, 100)]])
 def test_many_tokens_at_their_remainders(shapes):
-    """Products in tiles (from 64 tokens and 96 outputs on, 350000 results for odd multiples of 288): tokens, outputs and contractions that fill
-    no tile or step, rows of odd length."""
+    """Products in tiles (from 64 tokens and 96 outputs on, for odd multiples of 288 from more than 256 workgroups of linear.hip on): tokens, outputs
+    and contractions that fill no tile or step, rows of odd length."""
     test_linear_at_its_remainders(shapes)
+
+
+@pytest.mark.parametrize("shapes", [[(8192, 288, 586), (33, 288, 288)], [(63, 320, 320), (300, 320, 650)], [(1000, 192, 95), (70, 192, 200)],
+                                    [(700, 320, 161), (66, 320, 97, 33)], [(1024, 288, 512), (1, 288, 5)], [(1024, 288, 480), (64, 288, 1024)],
+                                    [(2048, 288, 257), (0, 288, 288)]])
+def test_products_of_a_launch_in_a_form_each(shapes):
+    """One product in tiles beside one that is not (few tokens, few outputs, turned), in either order, and both sides of the 256 workgroups up to which
+    odd multiples of 288 features go without; every product as by itself."""
+    test_linear_at_its_remainders(shapes)
+    lib = L.load()
+    a, kept = Args(), []
+    for i, (t, nin, nout, *turn) in enumerate(shapes):
+        x, w, _ = _operands(max(t, 1), nin, nout, i)
+        y, alone = (torch.full((max(t, 1), nout), 3.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        kept.append((x.cuda(), w.cuda(), y, alone))
+        a.job[0], a.njobs, a.dtype = Job(kept[i][0].data_ptr(), kept[i][1].data_ptr(), alone.data_ptr(), t, nin, nout, *turn), 1, L.ISSM_BF16
+        a.stream = L.current_stream_ptr(alone.device)
+        assert lib.issm_linear_fwd(C.byref(a)) == 0
+    for i, (t, nin, nout, *turn) in enumerate(shapes):
+        a.job[i] = Job(*(v.data_ptr() for v in kept[i][:3]), t, nin, nout, *turn)
+    a.njobs = 2
+    assert lib.issm_linear_fwd(C.byref(a)) == 0
+    torch.cuda.synchronize()
+    for *_, y, alone in kept:
+        assert torch.equal(y, alone)
 
 
 @pytest.mark.parametrize("shapes", [[(64, 2, 96)], [(65, 586, 288), (64, 288, 288)], [(1000, 98, 130)], [(130, 94, 98), (4099, 610, 320)]])
