@@ -60,23 +60,42 @@ def _watched() -> bool:
                 or any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
 
 
+class _HiddenFn(torch.autograd.Function):
+    """The hidden values of the table's MLP, from copies of their weights, as values that w1 and b1 get a gradient through."""
+
+    @staticmethod
+    def forward(ctx, w1, b1, x, first):
+        h = torch.relu(nn.functional.linear(x, first[:w1.numel()].view(w1.shape), first[w1.numel():]))
+        ctx.save_for_backward(x, h)
+        return h
+
+    @staticmethod
+    def backward(ctx, dh):
+        x, h = ctx.saved_tensors
+        dh = dh * (h > 0)
+        return dh.t() @ x, dh.sum(0), None, None
+
+
 class BoxTableFn(torch.autograd.Function):
-    """The table of ``BoxDistFun`` with gradients: its modules' products forward, one kernel backward."""
+    """The table of ``BoxDistFun`` with gradients: its modules' products forward, one kernel backward.  The modules keep neither w1 nor b1 for
+    their backward, and both may be changed in place before it: what the kernel computes the hidden values from again are copies."""
 
     @staticmethod
     def forward(ctx, module, w1, b1, w2, coords):
-        ctx.save_for_backward(w1, b1, w2, coords)
+        ctx.first = (w1, b1)   # (whose gradient it is; not their values)
+        ctx.save_for_backward(torch.cat((w1.reshape(-1), b1)), w2, coords.to(w1.dtype))
         return module.rpe_table().float().contiguous()
 
     @staticmethod
     def backward(ctx, dtable):
-        w1, b1, w2, coords = ctx.saved_tensors
+        first, w2, coords = ctx.saved_tensors
+        w1, b1 = ctx.first
         if torch.is_grad_enabled():   # to be differentiated again: as operations that autograd records
-            x, g = coords.reshape(-1, 3).to(w1.dtype), dtable.reshape(CHANNELS, -1).to(w1.dtype)
-            h = torch.relu(nn.functional.linear(x, w1, b1))
+            x, g = coords.reshape(-1, 3), dtable.reshape(CHANNELS, -1).to(w1.dtype)
+            h = _HiddenFn.apply(w1, b1, x, first)
             dh = (g.t() @ w2) * (h > 0)
             return None, dh.t() @ x, dh.sum(0), g @ h, None
-        a, g = _table_args(w1, b1, w2, coords), _f32c(dtable)
+        a, g = _table_args(first[:w1.numel()].view(w1.shape), first[w1.numel():], w2, coords), _f32c(dtable)
         grads = [torch.empty_like(t) for t in (w1, b1, w2)]
         with torch.cuda.device(w1.device):
             L.check(L.load().issm_box_table_bwd(C.byref(a), g.data_ptr(), *(t.data_ptr() for t in grads)), "issm_box_table_bwd")

@@ -259,6 +259,41 @@ def test_gradients_of_the_tables_mlp(quant, rpe_dim, dtype, again):
     hook.remove()
 
 
+@pytest.mark.parametrize("again", [False, True])
+def test_tables_mlp_after_its_first_layer_has_changed(again):
+    """The encoding's first weights and its bias changed in place between forward and backward: the gradients of the values that the forward used,
+    as from the modules, which do not keep them; the second weights are kept, and say so."""
+    from dest3d_amd.box_dist import BoxDistFun, BoxTableFn
+    torch.manual_seed(5)
+    m = BoxDistFun(out_dim=16).cuda()
+    mlp = m._plain_mlp()
+    g = torch.randn(16, 10, 10, 10, device="cuda")
+    run = lambda t: torch.autograd.grad(t, mlp[:3], g, create_graph=again)
+    of_modules = lambda: m.rpe_table().float().contiguous()
+    want, kept = run(of_modules()), run(BoxTableFn.apply(m, *mlp))
+    for make in (of_modules, lambda: BoxTableFn.apply(m, *mlp)):
+        table = make()
+        before = [p.detach().clone() for p in mlp[:3]]
+        with torch.no_grad():
+            mlp[0].neg_()
+            mlp[1].add_(1.0)
+        for a, b, c in zip(run(table), want, kept):
+            assert (a - b).norm() <= 1e-5 * b.norm() and (torch.equal(a, c) or make is of_modules)
+        with torch.no_grad():
+            mlp[0].copy_(before[0])
+            mlp[1].copy_(before[1])
+    if again:   # differentiated twice: d / dw1 of a function of dw2
+        a, = torch.autograd.grad(want[2].square().sum(), mlp[0])
+        b, = torch.autograd.grad(kept[2].square().sum(), mlp[0])
+        assert (a - b).norm() <= 1e-5 * a.norm()
+    table = BoxTableFn.apply(m, *mlp)
+    with torch.no_grad():
+        mlp[2].add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        run(table)
+
+
+
 def test_modes_see_the_tables_mlp():
     """Who counts or records operations or functions sees the two products of the table's MLP; a default device does not ask."""
     from torch.overrides import TorchFunctionMode
