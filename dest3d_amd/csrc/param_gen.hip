@@ -291,8 +291,7 @@ __device__ __forceinline__ float dsoftplus_(float x) { return x <= 20.0f ? sigmo
 // g of a B / C row is the sum of its forward-order and reversed-order gradients wherever the shared base row is
 // differentiated; the two bias gradients stay apart.  HASW (dt = softplus(raw) * weight): g of a dt row is
 // ddt * weight * softplus'(raw), and dweight[k] = sum_h ddt[h][k] softplus(raw[h][k]).
-// FULLK: K is a multiple of 64, so no load or store needs a bound on k, and every per-lane address is a
-// pointer advanced once per trip plus a compile-time offset.
+// FULLK: K is a multiple of 64, so no load or store needs a bound on k (pgen_pieces).
 template <bool BF, bool FULLK, bool HASW>
 __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_pgen_bwd(PGenP p) {
   constexpr int KS = 128 / (BF ? 2 : 4);   // columns of a step: 128 bytes of a gradient row
@@ -412,6 +411,8 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
       // step before has put its own into LDS; ddist takes dist's place there and leaves in the same pieces.  The rows read in the layout of
       // the products, 8 bytes a lane and 64 look-ups in the L1 an instruction, kept the look-ups busy 82 % of the time:
       // 8192 tokens x 256 queries, bf16, with weights, 53.4 -> 50.1 us, 234 MB at the rate of a copy.
+      // (The pieces' type promises the elements' alignment and no more: one wide access all the same.)
+      typedef unsigned Piece __attribute__((ext_vector_type(4), aligned(2)));
       const T* nil = (const T*)p.dist;  // what a lane with no row reads (at least 64 * 16 elements long)
       const int piece = (lane & 7) * (16 / (int)sizeof(T));
       const T *pa[2], *px[2];
@@ -446,9 +447,9 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
       auto request = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          ra[j] = *(const u4*)(pa[j] + (oka[j] ? k0 : 0));
-          rx[j] = *(const u4*)(px[j] + (okx[j] ? k0 : 0));
-          rd[j] = *(const u4*)(pd + (long)k0 * (PG_M * sizeof(T)) + 1024 * j);
+          ra[j] = *(const Piece*)(pa[j] + (oka[j] ? k0 : 0));
+          rx[j] = *(const Piece*)(px[j] + (okx[j] ? k0 : 0));
+          rd[j] = *(const Piece*)(pd + (long)k0 * (PG_M * sizeof(T)) + 1024 * j);
         }
         if constexpr (HASW) rw = pw[k0];
       };
@@ -680,10 +681,12 @@ int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// Whether the backward goes by whole steps of 64 queries, a token's ddist behind a buffer: 32-bit offsets, and whole dwords to store
+static bool pgen_pieces(const PGenP& p) { return p.K % 64 == 0 && p.K < 1 << 24 && ((uintptr_t)p.ddist & 3) == 0; }
 template <bool BF, bool HASW>
 static void pgen_bwd_launch(const PGenP& p, hipStream_t st) {
   const dim3 g((unsigned)p.nblocks), b(NTHREADS);
-  if (p.K % 64 == 0 && p.K < 1 << 24) hipLaunchKernelGGL((k_pgen_bwd<BF, true, HASW>), g, b, 0, st, p);
+  if (pgen_pieces(p)) hipLaunchKernelGGL((k_pgen_bwd<BF, true, HASW>), g, b, 0, st, p);
   else hipLaunchKernelGGL((k_pgen_bwd<BF, false, HASW>), g, b, 0, st, p);
 }
 

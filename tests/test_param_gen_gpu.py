@@ -192,3 +192,43 @@ def test_rows_beyond_32_bit_offsets():
     for far, near in zip(run(dist), run(dist[:, -few:].contiguous())):
         assert torch.equal(far[..., -few:], near)
         assert torch.equal(far[..., :5], far[..., K // 2:K // 2 + 5]) and (far[..., 0] != 3.0).all()
+
+
+@pytest.mark.parametrize("operands,ddist", [(1, 0), (2, 2), (4, 8), (0, 1), (3, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_backward_of_operands_at_any_element(dtype, operands, ddist):
+    """Gradients, dt and dist that begin `operands` elements behind an aligned address, ddist `ddist` elements: as from aligned ones.  (A ddist at
+    an odd bf16 element takes the form with a bound on k: the same rows' sums in blocks of 16, another order of the sums over k.)"""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib = L.load()
+    tokens, K, H, G = 21, 128, 8, 1
+    R0, R = H + 2 * G, H + 4 * G
+    gen = torch.Generator().manual_seed(3)
+    W, w = torch.randn(R0, 16, generator=gen).cuda(), torch.rand(tokens, K, generator=gen).cuda()
+    tensors = [torch.randn(tokens, *s, generator=gen).to(dtype) for s in ((K, 16), (H, K), (G, K), (G, K), (G, K), (G, K), (H, K))]
+
+    def run(shift, dshift):
+        behind = lambda t, n: torch.cat([t.new_zeros(n), t.flatten()]).cuda()
+        kept = [behind(t, shift) for t in tensors]
+        dd = torch.full((dshift + tokens * K * 16 + 1,), 3.0, dtype=dtype, device="cuda")
+        f32 = lambda *s: torch.empty(*s, device="cuda")
+        sums = f32(tokens, K), f32(tokens, R), f32(R), f32(R0, 16)
+        scratch = f32(lib.issm_param_gen_bwd_blocks(tokens), R0, 16)
+        a = L.PGenArgs()
+        a.tokens, a.K, a.M, a.H, a.G, a.dtype, a.has_back = tokens, K, 16, H, G, L.dtype_code(dtype), 1
+        a.W, a.weights, a.dw_partial = W.data_ptr(), w.data_ptr(), scratch.data_ptr()
+        a.dist, a.ddt, a.dBm, a.dCm, a.dBm_back, a.dCm_back, a.dt_raw = (t[shift:].data_ptr() for t in kept)
+        a.ddist = dd[dshift:].data_ptr()
+        a.dweights, a.dbias, a.dbias_sum, a.dW = (t.data_ptr() for t in sums)
+        a.stream = L.current_stream_ptr(dd.device)
+        assert lib.issm_param_gen_bwd(C.byref(a)) == 0
+        torch.cuda.synchronize()
+        assert (dd[:dshift] == 3.0).all() and dd[-1] == 3.0
+        return dd[dshift:-1], *sums
+    same = dtype == torch.float32 or ddist % 2 == 0
+    for got, want in zip(run(operands, ddist), run(0, 0)):
+        if same:
+            assert torch.equal(got, want)
+        else:   # fp32 sums in another order; ddist and bf16 roundings of it
+            assert _rel(got, want) <= (2.0 ** -8 if got.dtype == torch.bfloat16 else 1e-5)
