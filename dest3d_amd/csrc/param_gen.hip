@@ -681,8 +681,9 @@ int launch_conv_pgen(const DwConvP& c, const PGenP& p, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// Whether the backward goes by whole steps of 64 queries, a token's ddist behind a buffer: 32-bit offsets, and whole dwords to store
-static bool pgen_pieces(const PGenP& p) { return p.K % 64 == 0 && p.K < 1 << 24 && ((uintptr_t)p.ddist & 3) == 0; }
+// Whether the backward goes by whole steps of 64 queries, of which it requests the first unasked, a token's ddist behind a buffer: 32-bit offsets, and
+// whole dwords to store
+static bool pgen_pieces(const PGenP& p) { return p.K > 0 && p.K % 64 == 0 && p.K < 1 << 24 && ((uintptr_t)p.ddist & 3) == 0; }
 template <bool BF, bool HASW>
 static void pgen_bwd_launch(const PGenP& p, hipStream_t st) {
   const dim3 g((unsigned)p.nblocks), b(NTHREADS);

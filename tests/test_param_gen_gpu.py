@@ -232,3 +232,24 @@ def test_backward_of_operands_at_any_element(dtype, operands, ddist):
             assert torch.equal(got, want)
         else:   # fp32 sums in another order; ddist and bf16 roundings of it
             assert _rel(got, want) <= (2.0 ** -8 if got.dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_backward_without_queries(dtype):
+    """No query: sums of nothing, and nothing read or written where a query would be."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib = L.load()
+    tokens, H, G = 9, 4, 1
+    R0, R = H + 2 * G, H + 4 * G
+    W, buf = torch.randn(R0, 16).cuda(), torch.full((64,), 3.0, dtype=dtype, device="cuda")
+    out = [torch.full(s, 3.0, device="cuda") for s in ((tokens, R), (R,), (R0, 16), (lib.issm_param_gen_bwd_blocks(tokens), R0, 16))]
+    a = L.PGenArgs()
+    a.tokens, a.K, a.M, a.H, a.G, a.dtype, a.has_back = tokens, 0, 16, H, G, L.dtype_code(dtype), 1
+    a.W = W.data_ptr()
+    a.dist = a.ddt = a.dBm = a.dCm = a.dBm_back = a.dCm_back = a.ddist = buf.data_ptr()
+    a.dbias, a.dbias_sum, a.dW, a.dw_partial = (t.data_ptr() for t in out)
+    a.stream = L.current_stream_ptr(buf.device)
+    assert lib.issm_param_gen_bwd(C.byref(a)) == 0
+    torch.cuda.synchronize()
+    assert all((t == 0.0).all() for t in out[:3]) and (buf == 3.0).all()
