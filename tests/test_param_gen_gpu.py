@@ -175,6 +175,7 @@ def test_rows_beyond_32_bit_offsets():
     from dest3d_amd import _lib as L
     lib = L.load()
     K, H, G, few = 53_700_001, 10, 1, 777
+    torch.manual_seed(4)
     W, bias = torch.randn(H + 2 * G, 16).cuda(), torch.randn(1, H + 2 * G).cuda()
     dist = torch.zeros(1, K, 16, dtype=torch.bfloat16, device="cuda")
     dist[:, -few:] = torch.randn(1, few, 16).bfloat16().cuda()
@@ -192,6 +193,90 @@ def test_rows_beyond_32_bit_offsets():
     for far, near in zip(run(dist), run(dist[:, -few:].contiguous())):
         assert torch.equal(far[..., -few:], near)
         assert torch.equal(far[..., :5], far[..., K // 2:K // 2 + 5]) and (far[..., 0] != 3.0).all()
+
+
+@pytest.mark.parametrize("form,K", [("bias", 26_900_001), ("bias weights raw", 53_700_002), ("tok", 53_700_002), ("tok weights raw", 26_900_001),
+                                    ("tok weights", 53_700_001), ("joined", 53_700_002)])
+def test_forms_beyond_32_bit_offsets(form, K):
+    """The other forms of the kernels with 64-bit places -- fp32 and bf16, gathered biases and the producers' own, with a reversed pair, weights with and
+    without raw dt, and the one with the convolutions in its launch -- against the last queries in a call of their own: the same bits."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib, H, G, few, di = L.load(), 10, 1, 777, 34
+    dtype = torch.float32 if K < 50_000_000 else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    R0, Cc = H + 2 * G, di + 2 * G
+    W, add, bias = 0.3 * rnd(R0, 16), rnd(H), rnd(1, H + 4 * G)
+    row, tail = rnd(1, 2 * di + 2 * G + H).to(dtype), rnd(2, 1, 2 * G).to(dtype)
+    cw, cb = rnd(2, Cc, 7), rnd(2, Cc)
+    dist = torch.zeros(1, K, 16, dtype=dtype, device="cuda")
+    dist[:, -few:] = rnd(1, few, 16).to(dtype)
+    weights = torch.ones(1, K, device="cuda")
+    weights[:, -few:] = torch.rand(1, few, generator=g, device="cuda")
+    stream = L.current_stream_ptr(torch.device("cuda", 0))
+
+    def run(d, w):
+        k = d.shape[1]
+        out = [torch.full((1, n, k), 3.0, dtype=dtype, device="cuda") for n in (H, G, G, G, G) + ((H,) if "raw" in form else ())]
+        a = L.PGenArgs(tokens=1, K=k, M=16, H=H, G=G, dtype=L.dtype_code(dtype), has_back=1, dist=d.data_ptr(), W=W.data_ptr(), stream=stream)
+        a.dt, a.Bm, a.Cm, a.Bm_back, a.Cm_back = (t.data_ptr() for t in out[:5])
+        if "raw" in form:
+            a.dt_raw = out[5].data_ptr()
+        if "weights" in form or form == "joined":
+            a.weights = w.data_ptr()
+        if "bias" in form:
+            a.bias = bias.data_ptr()
+        else:
+            a.tok, a.tok_stride, a.tok_add = row[:, di + Cc:].data_ptr(), row.shape[1], add.data_ptr()
+            if form != "joined":
+                a.tail = tail.data_ptr()
+        if form == "joined":
+            y = torch.full((2, 1, 1, di), 3.0, dtype=dtype, device="cuda")
+            c = L.DwConvArgs(batch=1, seqlen=1, channels=Cc, nsets=2, taps=7, dtype=L.ISSM_BF16, u=row[:, di:].data_ptr(), u_batch_stride=row.shape[1],
+                             u_token_stride=row.shape[1], w=cw.data_ptr(), bias=cb.data_ptr(), y=y.data_ptr(), stream=stream, split=di, chain=1)
+            L.check(lib.issm_conv_param_gen_fwd(C.byref(c), C.byref(a)), "joined")
+            out.append(y)
+        else:
+            # (raw dt is the training form's: without it, and with weights, only the form that no backward follows takes the call)
+            L.check((lib.issm_param_gen_fwd if "raw" in form or "weights" not in form else lib.issm_param_gen_fwd_only)(C.byref(a)), form)
+        torch.cuda.synchronize()
+        return out
+    far, near = run(dist, weights), run(dist[:, -few:].contiguous(), weights[:, -few:].contiguous())
+    for f, n in zip(far, near):
+        assert torch.equal(f[..., -n.shape[-1]:], n)
+        if n.shape[-1] == few:
+            assert torch.equal(f[..., :5], f[..., K // 2:K // 2 + 5]) and (f[..., 0] != 3.0).all()
+
+
+@pytest.mark.parametrize("K", [(1 << 24) - 64, 1 << 24])
+def test_backward_at_the_last_offsets_of_its_pieces(K):
+    """Both sides of the number of queries up to which a token's ddist lies behind a buffer, against the queries that have a gradient in a call of
+    their own: fp32 sums of the same values, in other blocks."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib, H, G, few, dtype = L.load(), 1, 1, 128, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(1)
+    W = torch.randn(H + 2 * G, 16, generator=g, device="cuda")
+    full = [torch.zeros(1, *s, dtype=dtype, device="cuda") for s in ((K, 16), (H, K), (G, K), (G, K))]
+    full[0][:, -few:] = torch.randn(1, few, 16, generator=g, device="cuda").to(dtype)
+    for t in full[1:]:
+        t[..., -few:] = torch.randn(*t.shape[:2], few, generator=g, device="cuda").to(dtype)
+
+    def run(d, *grads):
+        dd, dbias, dW = torch.full_like(d, 3.0), torch.empty(1, H + 2 * G, device="cuda"), torch.empty(H + 2 * G, 16, device="cuda")
+        scratch = torch.empty(lib.issm_param_gen_bwd_blocks(1), H + 2 * G, 16, device="cuda")
+        a = L.PGenArgs(tokens=1, K=d.shape[1], M=16, H=H, G=G, dtype=L.ISSM_BF16, has_back=0, dist=d.data_ptr(), W=W.data_ptr(),
+                       dw_partial=scratch.data_ptr(), dW=dW.data_ptr(), dbias=dbias.data_ptr(), ddist=dd.data_ptr(),
+                       stream=L.current_stream_ptr(d.device))
+        a.ddt, a.dBm, a.dCm = (t.data_ptr() for t in grads)
+        assert lib.issm_param_gen_bwd(C.byref(a)) == 0
+        torch.cuda.synchronize()
+        return dd, dbias, dW
+    want = run(full[0][:, -few:].contiguous(), *(t[..., -few:].contiguous() for t in full[1:]))
+    dd, dbias, dW = run(*full)
+    assert _rel(dd[:, -few:], want[0]) <= 2.0 ** -8 and (dd[:, :-few] == 0).all()
+    assert _rel(dbias, want[1]) <= 1e-5 and _rel(dW, want[2]) <= 1e-5
 
 
 @pytest.mark.parametrize("operands,ddist", [(1, 0), (2, 2), (4, 8), (0, 1), (3, 5)])
