@@ -528,24 +528,22 @@ constexpr int64_t TILE_RESULTS = 384, DX_CONTRACTION = 640;
 // 16384 tokens, 256 -> 256 8.5 and 8.1, 288 -> 288 9.0 and 13.2; 32768, 320 -> 320 22.6 and 19.4, 288 -> 288 14.9 and 21.6; with other results the two
 // meet at 65536 tokens: 288 -> 586 63.1 and 62.8, 352 -> 352 43.9 and 43.8)
 bool tiled_tokens(int64_t tokens, int64_t results) { return tokens <= (results % 64 ? 32768 : 8192); }
-// A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save, as long as
-// it is ahead for 16 to 512 queries (multiples of 32 up to 640 features; separate steps and chain in us, scenes of 1024 tokens and 256
-// queries unless said).  288 features, 4, 8, 11 and 16 scenes: 159 and 138, 269 and 242, 347 and 327, 504 and 492; 192, 16 scenes: 432 and 400; 96, 62:
-// 1229 and 1152.  Rows of 128 bytes and multiples of them suit its products least: 64 features, 64 queries, 59, 89 and 135 scenes 527 and 505, 751
-// and 749, 1093 and 1112, 16 queries, 31 and 47 scenes of 2048 449 and 447, 649 and 677; 128, 16 queries, 12 and 20 scenes of 2048 221 and 216, 329 and
-// 341; 320, whose ten fragments take two requests of eight (the first products; the last ones', asked for at once, take 2 % off the layer since), 3, 4, 5 and 6
-// scenes 153 and 134, 170 and 169, 200 and 212, 222 and 233; 384, 3 and 4
-// scenes 153 and 145, 175 and 180; 512, 2, 3 and 4 scenes 140 and 126, 166 and 160, 202 and 217; 640, 1 and 2 scenes 132 and 106, 165 and 168.  (Wider odd
-// multiples of 32 would stay ahead for longer: 352, 7 scenes, 268 and 251, 480, 5 scenes, 232 and 218.)
+// A layer without a gradient (scan_layer's chain) goes on taking them beyond that, for what the launches between them save, up to where it
+// was ahead for 16 to 512 queries while its first products were linear.hip's (multiples of 32 up to 640 features).  Separate steps and chain now, both with
+// tiles, in us, scenes of 1024 tokens and 256 queries unless said.  At the line, 64 features, 50 and 66 scenes 822 and 767, 1070 and 1004; 128, 32 587 and 568;
+// 288, 6, 8 and 12 scenes 160 and 160, 205 and 203, 306 and 307, with 64 queries 97 and 95, 110 and 118, 145 and 157; 320, 3 and 4 103 and 103, 123 and 131, 16 queries
+// and 2 scenes of 2048 81 and 79; 384, 2 and 3 90 and 94, 109 and 115; 512, 2 and 3 122 and 104, 145 and 127.  So it lies within 8 % of where either is ahead
+// for 288 to 384 features, whose separate products are in tiles and in one launch; to both sides of those the chain stays ahead beyond it: 64, 287 scenes
+// 4518 and 4284; 192, 34 716 and 680; 256, 19 458 and 439; 448, 5 195 and 189; 512, 4 171 and 170.
 double chain_products(int64_t features) {
   return features <= 64 ? 5.5e8 : features == 320 ? 8.6e8 : features == 128 || features > 288 ? 1.1e9 : 1.4e9;
 }
 // The chain's convolutions and generation of dt, B and C are one launch up to this many threads of the generation, two queries each where their
-// number is even: the first wave of a workgroup convolves while the others wait, and from 0.6 million threads on that costs more than the
-// launch and what lies between the two.  8 heads, 64 features, 256 queries, scenes of 1024 tokens: 2 64 us in one launch and 67 in two, 5 121
-// and 121, 10 207 and 199, 31 624 and 580; 288 features 86 and 89, 166 and 165, 308 and 301, 970 and 923; 51 queries, 64 features, 12, 24 and 98
-// scenes 130 and 129, 230 and 220, 922 and 850.
-constexpr int64_t JOINED_THREADS = 600000;
+// number is even: the first wave of a workgroup convolves while the others wait, and from 0.4 million threads on that costs more than the
+// launch and what lies between the two.  8 heads, 64 features, 256 queries, scenes of 1024 tokens: 1, 2, 3, 5 and 12 47.6 us in two launches and 46.6 in one, 58.7
+// and 57.8, 70.9 and 71.4, 98.8 and 99.6, 191 and 196; 288 features 57.3 and 55.2, 79.1 and 79.6, 95.0 and 94.1, 140 and 142, 305 and 320; 51 queries, 64
+// features, 5, 8 and 31 scenes 65.6 and 63.6, 85.2 and 85.1, 237 and 241.
+constexpr int64_t JOINED_THREADS = 400000;
 // (tensors that stand for something else than their memory, under vmap, functionalization, a tensor subclass or a lazy
 // negation, go to the library's product, which knows them)
 bool own_memory(const Tensor& t) {
