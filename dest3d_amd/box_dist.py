@@ -111,6 +111,10 @@ def _table_args(w1, b1, w2, coords):
     return a
 
 
+def _wants_gradient(mlp) -> bool:
+    return torch.is_grad_enabled() and any(p.requires_grad for p in mlp)
+
+
 class BoxDistFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, table, key_xyz, corners, angle, qcenter, radius, weight_dist, log_scale, max_value, out_dtype,
@@ -262,11 +266,11 @@ class BoxDistFun(nn.Module):
             return None
         return (*ps, coords)
 
-    def _plain_table(self):
+    def _plain_table(self, mlp=None):
         """The same table, (out_dim, n, n, n) fp32, from one kernel where nothing is to be differentiated; None otherwise."""
-        mlp = self._plain_mlp()
+        mlp = self._plain_mlp() if mlp is None else mlp
         # (a checkpointed segment's run: both of them take the sums of one with gradients)
-        if mlp is None or (torch.is_grad_enabled() and any(p.requires_grad for p in mlp)) or L.host().runs_twice():
+        if mlp is None or _wants_gradient(mlp) or L.host().runs_twice():
             return None
         w = mlp[0]
         table = torch.empty((CHANNELS, *_lattice(mlp[3])), dtype=torch.float32, device=w.device)
@@ -281,14 +285,14 @@ class BoxDistFun(nn.Module):
         of ``local_weight`` are computed in the same pass and returned as a second value."""
         # the kernel derives the corners (and, for the weights, centre and radius) from the boxes themselves
         boxes = torch.cat([query_xyz, query_size, query_angle.unsqueeze(-1)], dim=-1).detach()
-        table = self._plain_table()
+        mlp = self._plain_mlp()
+        table = None if mlp is None else self._plain_table(mlp)
         plain = table is not None
-        mlp = None if plain else self._plain_mlp()
-        if mlp is not None and torch.is_grad_enabled() and any(p.requires_grad for p in mlp):
+        if mlp is not None and _wants_gradient(mlp):
             table = BoxTableFn.apply(self, *mlp)
         elif not plain:
             mlp, table = None, self.rpe_table()
-        out_dtype = self.cpb_mlps[0].weight.dtype if plain or mlp is not None else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
+        out_dtype = self.cpb_mlps[0].weight.dtype if mlp is not None else table.dtype if table.dtype in (torch.float32, torch.bfloat16) else torch.float32
         if weight_query_pos is None:
             return BoxDistFn.apply(table, key_xyz, boxes, query_angle, None, None, 0.0, self.log_scale, self.max_value,
                                    out_dtype, True, False, plain)[0]
