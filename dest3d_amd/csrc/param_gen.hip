@@ -410,7 +410,8 @@ __global__ __launch_bounds__(NTHREADS, (BF || !HASW || !FULLK) ? 4 : 3) void k_p
       // (LDS instructions of one wave are carried out in order: a read sees the writes before it.)  A step's pieces are requested when the
       // step before has put its own into LDS; ddist takes dist's place there and leaves in the same pieces.  The rows read in the layout of
       // the products, 8 bytes a lane and 64 look-ups in the L1 an instruction, kept the look-ups busy 82 % of the time:
-      // 8192 tokens x 256 queries, bf16, with weights, 53.4 -> 50.1 us, 234 MB at the rate of a copy.
+      // 8192 tokens x 256 queries, bf16, with weights, 53.4 -> 50.1 us, 234 MB at the rate of a copy (51.8 since it also leaves the producers their bias
+      // gradients, for which an address goes to scratch before the loops and comes back behind them: 12 bytes a lane).
       // (The pieces' type promises the elements' alignment and no more: one wide access all the same.)
       typedef unsigned Piece __attribute__((ext_vector_type(4), aligned(2)));
       const T* nil = (const T*)p.dist;  // what a lane with no row reads (at least 64 * 16 elements long)
