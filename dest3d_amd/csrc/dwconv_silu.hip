@@ -26,7 +26,7 @@ namespace issm {
 // Tokens per thread of the kernels that are not chained, DW_TL.  Backward: 16.  Forward: the most of 16, 8 and 4 that makes two waves a SIMD: one
 // scene of 1024 tokens makes 290 waves of 16 (9.4, 7.7 and 5.5 us with 16, 8 and 4).
 // Tokens per tile of the chained ones.  Backward: 64 (32: 17.3 us with half more of the sums for the parts; 64: 17.2, of which 2 went with the
-// sums' LDS that left a CU four workgroups of five).  Forward: 64, or 16 where that makes fewer than 1024 workgroups.
+// sums' LDS that left a CU four workgroups of five).  Forward: 64, or 16 where that makes fewer than 1024 workgroups (and more: launch_dwconv_fwd).
 constexpr int DW_BWD = 16, DW_CHAIN_BWD = 64;
 
 template <bool BF, int S, int DW_TL>
@@ -158,10 +158,10 @@ __global__ __launch_bounds__(NTHREADS) void k_dwconv_bwd(DwConvP p) {
 }
 
 // ---- chained pair: set 1 convolves set 0's output (rounded to the I/O dtype, as it is stored)
-// (rows far apart: the tiles below address theirs in 32 bits)
-template <bool BF>
-__global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd_far(DwConvP p) {
-  dw_chain_fwd<BF, 4, true>(p, (long)blockIdx.x * NTHREADS + threadIdx.x);
+// A thread to DW_TL tokens of a channel: rows far apart (the tiles below address theirs in 32 bits), and fp32 whose rows no cache holds (launch_dwconv_fwd)
+template <bool BF, int DW_TL>
+__global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd_threads(DwConvP p) {
+  dw_chain_fwd<BF, DW_TL, true>(p, (long)blockIdx.x * NTHREADS + threadIdx.x);
 }
 
 constexpr int DW_CH = 32, DW_RUNS = NTHREADS / DW_CH, DW_HALO = DW_TAPS - 1;
@@ -192,7 +192,7 @@ static unsigned dw_tiles(const DwConvP& p, int tokens) {
   const int split = p.split > 0 ? p.split : p.C;
   return (unsigned)p.B * ((p.L + tokens - 1) / tokens) * ((split + DW_CH - 1) / DW_CH + (p.C - split + DW_CH - 1) / DW_CH);
 }
-// Whether a tile's rows (76, 4-byte values at most) are within 31-bit byte offsets
+// Whether a tile's rows (76, or 140 of 2-byte values) are within 31-bit byte offsets
 static bool dw_near(const DwConvP& p) { return std::max(std::max(p.u_ls, p.du ? p.du_ls : 0L), (long)p.C) < 1L << 22; }
 
 // Rows from .. to - 1 behind a buffer: what lies outside them or the channels reads zero and is not stored, an addition an access where a pointer, a
@@ -228,7 +228,7 @@ __device__ __forceinline__ const void* dw_at(const void* q, long n) {
 
 // Thread = channel and one of eight runs of rows; u and y[0] go through LDS, so that the halo of 6 + 6 rows is loaded and convolved once a
 // workgroup, not once a thread.  290 channels, bf16, us, with a thread to 16, 8 or 4 tokens and now: 1 x 1024 tokens 4.8 and 3.7, 8 x 1024 14.8 and 8.5,
-// 16 x 4096 67.8 and 41.2 (fp32 104 and 106, the memory's time).
+// 16 x 4096 67.8 and 41.2.
 template <bool BF, int T>
 __global__ __launch_bounds__(NTHREADS) void k_dwconv_chain_fwd(DwConvP p) {
   constexpr int CH = DW_CH, RUNS = DW_RUNS, HALO = DW_HALO, N0 = T + HALO, N1 = N0 + HALO;
@@ -489,7 +489,13 @@ static int launch_dwconv_fwd_t(const DwConvP& p, hipStream_t st) {
 int launch_dwconv_fwd(const DwConvP& p, hipStream_t st) {
   if (p.chain) {
     auto go = [&](auto kern, unsigned blocks) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NTHREADS), 0, st, p); };
-    if (!dw_near(p)) p.dtype ? go(&k_dwconv_chain_fwd_far<true>, dw_blocks(p, 4)) : go(&k_dwconv_chain_fwd_far<false>, dw_blocks(p, 4));
+    // Past what the last cache holds (256 MB of u, y and pre), the pieces of lines that tiles side by side write reach memory: in fp32 a thread's
+    // channel, whose wave writes 256 bytes of a row, is ahead again, in bf16 tiles of 128 tokens (buffers in turn, us, threads of 16 tokens, tiles of 64 and of 128:
+    // fp32 24 x 2048 tokens, 290 channels 86, 94, 101; 16 x 4096 113, 125, 137; 16 x 2048, 514 95, 105, 96; 1026 183, 214, 234; and below, 16 x 2048, 290 59, 58, 57;
+    // 16 x 1000, 514 50, 45, 46; bf16 16 x 2048, 1026 120, 132, 112; 32 x 4096, 288 133, 123, 100; 16 x 4096, 290 74, 75, 65).
+    const bool beyond = 5.0 * p.B * p.L * p.C * (p.dtype ? 2 : 4) > (double)(256 << 20);
+    if (!dw_near(p)) p.dtype ? go(&k_dwconv_chain_fwd_threads<true, 4>, dw_blocks(p, 4)) : go(&k_dwconv_chain_fwd_threads<false, 4>, dw_blocks(p, 4));
+    else if (beyond) p.dtype ? go(&k_dwconv_chain_fwd<true, 128>, dw_tiles(p, 128)) : go(&k_dwconv_chain_fwd_threads<false, 16>, dw_blocks(p, 16));
     else if (dw_tiles(p, 64) >= 1024) p.dtype ? go(&k_dwconv_chain_fwd<true, 64>, dw_tiles(p, 64)) : go(&k_dwconv_chain_fwd<false, 64>, dw_tiles(p, 64));
     else p.dtype ? go(&k_dwconv_chain_fwd<true, 16>, dw_tiles(p, 16)) : go(&k_dwconv_chain_fwd<false, 16>, dw_tiles(p, 16));
     return (int)hipGetLastError();

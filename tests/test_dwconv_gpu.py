@@ -300,3 +300,29 @@ def test_chain_forward_in_its_tiles(dtype, B, Ln, Cn, split):
         assert torch.equal(far_y[:, 0], y[:, 0]) and torch.equal(far_pre[:, 0], pre[:, 0])
     one_y, one_pre = run(near[-1:], 1)   # (of many sequences 64 tokens a tile, of one 16)
     assert torch.equal(one_y[:, 0], y[:, -1]) and torch.equal(one_pre[:, 0], pre[:, -1])
+
+
+@pytest.mark.parametrize("dtype,Ln", [(torch.float32, 15503), (torch.bfloat16, 31001)])
+def test_chain_beyond_the_last_cache(dtype, Ln):
+    """More rows than 256 MB hold: the forms that take them, against the first and the last tokens in calls of their own (their inner edge left out):
+    the same bits of both outputs and what is kept for the backward."""
+    import ctypes as C
+    from dest3d_amd import _lib as L
+    lib, B, Cn, split, few = L.load(), 3, 290, 288, 300
+    g = torch.Generator(device="cuda").manual_seed(Ln)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    u, w, b = rnd(B, Ln, Cn).to(dtype), 0.4 * rnd(2, Cn, 7), 0.2 * rnd(2, Cn)
+
+    def run(u):
+        n = u.shape[1]
+        y, tail, pre = (torch.full((2, B, n, c), 3.0, dtype=dtype, device="cuda") for c in (split, Cn - split, Cn))
+        a = L.DwConvArgs(batch=B, seqlen=n, channels=Cn, nsets=2, taps=7, dtype=L.dtype_code(dtype), u=u.data_ptr(), u_batch_stride=n * Cn,
+                         u_token_stride=Cn, w=w.data_ptr(), bias=b.data_ptr(), y=y.data_ptr(), y_tail=tail.data_ptr(), pre=pre.data_ptr(), split=split,
+                         chain=1, stream=L.current_stream_ptr(u.device))
+        assert lib.issm_dwconv_silu_fwd(C.byref(a)) == 0
+        torch.cuda.synchronize()
+        return y, tail, pre
+    whole, first, last = run(u), run(u[:, :few].contiguous()), run(u[:, -few:].contiguous())
+    for t, f, l in zip(whole, first, last):
+        assert torch.equal(t[:, :, :few - 6], f[:, :, :few - 6]) and torch.equal(t[:, :, 6 - few:], l[:, :, 6:])
+        assert t.isfinite().all() and (t[:, :, few:-few] != 3.0).any(-1).all()
