@@ -65,7 +65,7 @@ def kernels():
     # workgroups of sixteen waves
     (r"(k_layer_end<.*>|k_three_nn_grid<1024, .*>|k_box_dist_fwd<.*>)", 11, 128, 0),
     # generation's backward by whole steps: four workgroups a CU, one form with an address in scratch outside its loops
-    (r"k_pgen_bwd<(true|false), true, (true|false)>", 4, 128, 12),
+    (r"k_pgen_bwd<(true|false), true, (true|false), (true|false)>", 8, 128, 12),
     # sums of the distance table's gradient: three, which cost scratch (40 bytes fp32, 12 bf16) and are faster than two without
     (r"k_bds_accum<(true|false)>", 2, 168, 52),
     # two of them a CU, and four of eight
