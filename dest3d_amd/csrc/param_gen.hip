@@ -124,34 +124,37 @@ __device__ __forceinline__ void pgen_fwd(const PGenP& p, const DwConvP& conv, in
   }
   if (t >= p.tokens) return;
   if constexpr (!CONV) request(t);
-  // Outputs behind buffers that begin with the workgroup's first token: a row is one scalar offset away from the row before.  (With a 64-bit
-  // product a store, 109 v_mul_lo and 102 v_mad_u64, a quarter of the rate each, stood beside 360 multiply-adds: 8192 tokens x 256, bf16,
-  // weights, 36.1 us -> 33.4; a layer without a gradient of 4 scenes 129.0 -> 125.1, of one 57.7 -> 57.1.)
+  // Outputs from the workgroup's first token on: a row is one scalar offset away from the row before, a thread's place one 32-bit offset.  (With a 64-bit
+  // product a store, 109 v_mul_lo and 102 v_mad_u64, a quarter of the rate each, stood beside 360 multiply-adds: 8192 tokens x 256, fp32, 8 heads
+  // 46 -> 38 us.)  Behind buffers; bf16 with gathered biases behind a scalar address, which suits its calls of few heads better, buffers and that, with
+  // weights: 8192 x 256, 8 heads 32.8 and 31.8 us, 4096 x 1000, 2 heads 37.2 and 35.1, 4000 x 77, 3 heads 6.4 and 6.1 (the producers' biases in training, 8192 x 256
+  // 33.4 and 34.4, fp32 62.5 and 64.0, 79.4 and 79.9, 7.8 and 7.9).
   constexpr int SZ = BF ? 2 : 4;
   const unsigned at_h = tl * (unsigned)(p.H * p.K) * SZ + (unsigned)k * SZ, at_g = tl * (unsigned)(p.G * p.K) * SZ + (unsigned)k * SZ;
   struct Rows {
     __amdgpu_buffer_rsrc_t buf;
-    char* first;   // FAR: the thread's place in row 0 of its token
+    char* first;                  // row 0 of the workgroup's first token (FAR: the thread's place in row 0 of its token)
   };
   auto rows = [&](void* q, int per) __attribute__((always_inline)) {
     char* base = (char*)q + t0 * per * p.K * SZ;
     return Rows{__builtin_amdgcn_make_buffer_rsrc(base, 0, FAR ? 0u : (unsigned)(wg_tokens * per * p.K) * SZ, 0x00027000),
-                FAR ? base + ((long)tl * per * p.K + k) * SZ : nullptr};
+                FAR ? base + ((long)tl * per * p.K + k) * SZ : base};
   };
   auto put = [&](const Rows& to, unsigned at, int row, const float (&v)[KV]) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t& q = to.buf;
-    const int s = row * p.K * SZ;   // uniform
     if constexpr (FAR) {
       st1<BF>(to.first, (long)row * p.K, v[0]);
-    } else if constexpr (BF && KV == 2) {
-      __builtin_amdgcn_raw_buffer_store_b32((unsigned)f_to_bf16(v[0]) | ((unsigned)f_to_bf16(v[1]) << 16), q, at, s, 0);
     } else if constexpr (BF) {
-      __builtin_amdgcn_raw_buffer_store_b16(f_to_bf16(v[0]), q, at, s, 0);
+      const unsigned two = KV == 2 ? (unsigned)f_to_bf16(v[0]) | ((unsigned)f_to_bf16(v[KV - 1]) << 16) : f_to_bf16(v[0]);
+      char* q = to.first + (long)row * p.K * SZ + at;   // uniform, and the thread's
+      if constexpr (TOK && KV == 2) __builtin_amdgcn_raw_buffer_store_b32(two, to.buf, at, row * p.K * SZ, 0);
+      else if constexpr (TOK) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)two, to.buf, at, row * p.K * SZ, 0);
+      else if constexpr (KV == 2) *(unsigned*)q = two;
+      else *(uint16_t*)q = (uint16_t)two;
     } else if constexpr (KV == 2) {
       typedef unsigned u2 __attribute__((ext_vector_type(2)));
-      __builtin_amdgcn_raw_buffer_store_b64((u2){__float_as_uint(v[0]), __float_as_uint(v[1])}, q, at, s, 0);
+      __builtin_amdgcn_raw_buffer_store_b64((u2){__float_as_uint(v[0]), __float_as_uint(v[1])}, to.buf, at, row * p.K * SZ, 0);
     } else {
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), q, at, s, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), to.buf, at, row * p.K * SZ, 0);
     }
   };
   const Rows dt_rows = rows(p.dt, p.H), raw_rows = rows(RAW && p.dt_raw ? p.dt_raw : p.dt, p.H);
